@@ -55,6 +55,7 @@ struct GemmParams {
                                     // x[.., t mod ka] with W[.., t mod kw]; with ka = 3 K0, kw = 2 K0 the 6 K0 steps meet
                                     // every (x part, W part) pair once.
   int out32;                        // outputs / residual stream are float32 (PagedKVCache mode), no 16-bit rounding
+  int rnd;                          // .. but for a plain store with logical rounding (layer 0 of that mode: RND_*)
   int epi; void* out; int ldo; void* resid; int pair_offset;
   Glu glu; int silu_cols;
   // 128 x 128 tile only: K split over gridDim.z workgroups when the (M, N) grid alone leaves most CUs idle (a prompt of a
@@ -74,7 +75,7 @@ __device__ __forceinline__ void epi32_swiglu(const GemmParams& p, int m, int n, 
   ((float*)p.out)[(size_t)m * p.ldo + n] = sl * up;
 }
 __device__ __forceinline__ void epi32_plain(const GemmParams& p, int m, int n, float y) {
-  if (p.epi == EPI_STORE) ((float*)p.out)[(size_t)m * p.ldo + n] = y;
+  if (p.epi == EPI_STORE) ((float*)p.out)[(size_t)m * p.ldo + n] = round_rt(y, p.rnd);
   else { float* h = (float*)p.resid; h[(size_t)m * p.ldo + n] = h[(size_t)m * p.ldo + n] + y; }
 }
 
@@ -1074,9 +1075,10 @@ __global__ __launch_bounds__(256) void rmsnorm_row_block_f32_kernel(const float*
 // terms = 2 (round 4, dense bf16 weights): [hi | lo] only, 16+ mantissa bits of x, TWO walks of W instead of three.  What
 // that costs in accuracy was measured on the CPU before it was built (oracle/numerics.py X_SPLIT2): the
 // float32-accumulating variants' deviation from the exact oracle does not move (mean 1.91352e-4 vs 1.91362e-4).
+// rnd: the normed row with the logical rounding of layer 0 (as rmsnorm_row_block_f32_kernel); values of T are one term, exactly.
 template <typename AT>
 __global__ __launch_bounds__(256) void split3_rows_kernel(const float* x, int ldx, const float* norm_w, float eps, AT* out,
-                                                          int K, int terms) {
+                                                          int K, int terms, int rnd) {
   __shared__ float part[4];
   const int row = blockIdx.x, tid = threadIdx.x;
   const float* xr = x + (size_t)row * ldx;
@@ -1100,7 +1102,8 @@ __global__ __launch_bounds__(256) void split3_rows_kernel(const float* x, int ld
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const f32x4 wv = *(const f32x4*)(norm_w + k + 4 * h);
-          v[h].x = (v[h].x * rs) * wv.x; v[h].y = (v[h].y * rs) * wv.y; v[h].z = (v[h].z * rs) * wv.z; v[h].w = (v[h].w * rs) * wv.w;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[h][j] = round_rt(round_rt(v[h][j] * rs, rnd) * wv[j], rnd);
         }
       }
       AT hi[8], mid[8], lo[8];
@@ -1113,7 +1116,7 @@ __global__ __launch_bounds__(256) void split3_rows_kernel(const float* x, int ld
         lo[j] = (AT)(r1 - (float)mid[j]);
       }
       *(uint4*)(o + k) = *(const uint4*)hi;
-      *(uint4*)(o + K + k) = *(const uint4*)mid;
+      if (terms >= 2) *(uint4*)(o + K + k) = *(const uint4*)mid;
       if (terms == 3) *(uint4*)(o + 2 * K + k) = *(const uint4*)lo;      // (uniform)
     }
     return;
@@ -1122,7 +1125,8 @@ __global__ __launch_bounds__(256) void split3_rows_kernel(const float* x, int ld
     f32x4 v = *(const f32x4*)(xr + k);
     if (norm_w != nullptr) {
       const f32x4 wv = *(const f32x4*)(norm_w + k);
-      v.x = (v.x * rs) * wv.x; v.y = (v.y * rs) * wv.y; v.z = (v.z * rs) * wv.z; v.w = (v.w * rs) * wv.w;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = round_rt(round_rt(v[j] * rs, rnd) * wv[j], rnd);
     }
     AT hi[4], mid[4], lo[4];
 #pragma unroll
@@ -1133,7 +1137,7 @@ __global__ __launch_bounds__(256) void split3_rows_kernel(const float* x, int ld
       lo[j] = (AT)(r1 - (float)mid[j]);
     }
     *(uint2*)(o + k) = *(const uint2*)hi;
-    *(uint2*)(o + K + k) = *(const uint2*)mid;
+    if (terms >= 2) *(uint2*)(o + K + k) = *(const uint2*)mid;
     if (terms == 3) *(uint2*)(o + 2 * K + k) = *(const uint2*)lo;      // (uniform)
   }
 }
@@ -1158,7 +1162,9 @@ int launch_rmsnorm_block(const void* x, int ldx, const void* w, void* out, int l
 }  // namespace
 
 bool gemm_prefill_supported(const LinearW& W, const GemvCall& c, size_t rows) {
-  if (c.force_v1 || c.rnd != RND_NONE || W.layout != 1) return false;
+  if (c.force_v1 || W.layout != 1) return false;
+  // logical rounding (layer 0 of the PagedKVCache mode): plain stores of float32 activations
+  if (c.rnd != RND_NONE && (c.act != MI_F32 || c.epi != EPI_STORE || W.lora_b[0] != nullptr || W.lora_b[1] != nullptr)) return false;
   if (rows < 32) return false;
   const bool dense = (W.wk == WK_BF16 && c.act == MI_BF16) || (W.wk == WK_F16 && c.act == MI_F16);
   const bool q4 = ((W.wk == WK_Q4_BF16 && c.act == MI_BF16) || (W.wk == WK_Q4_F16 && c.act == MI_F16)) && W.group == 64 &&
@@ -1206,11 +1212,11 @@ int launch_rmsnorm_rows(const void* x, int ldx, const void* w, void* out, int ld
 size_t split3_bytes(size_t rows, int K) { return rows * 3 * (size_t)K * 2; }
 
 int launch_split3_rows(const void* x, int ldx, const void* norm_w, float eps, void* out, int rows, int K, hipStream_t st,
-                       int terms) {
+                       int terms, int rnd) {
   if (K % 4 != 0 || ldx % 4 != 0) return fail(MI_ERR_UNSUPPORTED, "split3_rows: K and the row stride must be multiples of 4");
-  if (terms != 2 && terms != 3) return fail(MI_ERR_INVALID, "split3_rows: two or three terms");
+  if (terms < 1 || terms > 3) return fail(MI_ERR_INVALID, "split3_rows: one to three terms");
   hipLaunchKernelGGL(split3_rows_kernel<bf16>, dim3(rows), dim3(256), 0, st, (const float*)x, ldx, (const float*)norm_w, eps,
-                     (bf16*)out, K, terms);
+                     (bf16*)out, K, terms, rnd);
   MI_HIP(hipGetLastError());
   return MI_OK;
 }
@@ -1234,10 +1240,10 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
     const int kt = hilo ? c.kx : W.K;      // the true K
     if (hilo && (W.K != 2 * c.kx || W.wk != WK_BF16)) return fail(MI_ERR_INVALID, "gemm_prefill: a [hi | lo] matrix has 2 kx bf16 columns");
     const bool pair = wk_is_quant(W.wk) || hilo;     // W itself is a [hi | lo] pair: 3 x-terms against 2 W-terms meet over 6 kt steps
-    const int terms = c.ldx == 2 * kt ? 2 : 3;
-    if (c.ldx != terms * kt || (pair && terms != 3))
+    const int terms = c.ldx == kt ? 1 : c.ldx == 2 * kt ? 2 : 3;
+    if (c.ldx != terms * kt || (pair && terms == 2))
       return fail(MI_ERR_INVALID, "gemm_prefill: float32 activations must be split first (launch_split3_rows; two terms: dense bf16 weights only)");
-    p.ka = terms * kt; p.K = (pair ? 6 : terms) * kt; p.out32 = 1;
+    p.ka = terms * kt; p.K = terms * (pair ? 2 : 1) * kt; p.out32 = 1; p.rnd = c.rnd;
     if (hilo) p.kw = 2 * kt;
   }
   if (c.out32) p.out32 = 1;

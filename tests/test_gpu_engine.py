@@ -132,6 +132,28 @@ def test_float32_kv_prefill_two_and_three_terms_of_x(tiny_dirs, name):
     eng.close()
 
 
+@pytest.mark.parametrize("B,L0", [(1, 32), (3, 29), (5, 64), (2, 257)])
+@pytest.mark.parametrize("name", ["llama_bf16_gqa", "llama_f16", "qwen3_bf16", "llama_q4_bf16"])
+def test_float32_kv_prefill_first_layer_on_the_tile_gemm(tiny_dirs, name, B, L0):
+    """The rounded q|k|v call of layer 0 in the PagedKVCache mode: one bf16 term of x (f16 models: three) on the tile GEMM, the output
+    rounded in its epilogue.  Both kernel families take the sums in float32 and round them to the model dtype: they may differ by a
+    flip where a sum lies at a rounding boundary, and are held to the tolerances of the oracle comparison above."""
+    if name not in tiny_dirs:
+        pytest.skip(f"no tiny model {name}")
+    model, ref, cfg = _load_pair(tiny_dirs, name)
+    eng = model.engine
+    toks = _left_pad_prompts(cfg, B, L0)
+    want = ref(toks, cache=ref.make_cache(B, paged=True))
+    outs = {}
+    for on in (1, 0):
+        eng.set_option("prefill_gemm", on)
+        kv = eng.new_kv(B, capacity=L0 + 8, kv_dtype="float32")
+        outs[on] = eng.forward(toks, kv, all_positions=True)
+        kv.close()
+        assert np.abs(outs[on] - want).max() <= 4e-3 and np.sqrt(((outs[on] - want) ** 2).mean()) <= 2e-4, (on, np.abs(outs[on] - want).max())
+    eng.close()
+
+
 @pytest.mark.parametrize("name", ["llama_bf16_gqa", "llama_f16", "qwen3_bf16"])
 def test_decode_swiglu_on_the_row_interleaved_gate_up_copy_is_bit_identical(tiny_dirs, name):
     """Decode steps of <= 16 rows stream a row-interleaved copy of the dense gate|up matrix (tile t = gate rows 8t..8t+7 then
