@@ -14,6 +14,7 @@
 // O^T = V^T P, whose A fragments come out of the [16-d tile][key][16 d] image through
 // ds_read_b64_tr_b16.  Lane (c16 = query, g) owns the running max / sum of its query and
 // O[query][16 dt + 4g + r].  Tiles are launched heaviest (latest queries) first.
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -21,7 +22,11 @@
 
 namespace mi {
 
+int gemv_cu_count();      // gemv_mfma.hip
+
 namespace {
+
+constexpr int PREFILL_MAX_SLICES = 16;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -51,6 +56,77 @@ template <typename T>
 __device__ __forceinline__ uint32_t pack2(float a, float b) {
   T v[2] = {(T)a, (T)b};
   return __builtin_bit_cast(uint32_t, v);
+}
+
+__device__ __forceinline__ u32x4 load16_agent(const void* p) {       // (as in gemv_phase.h: past this XCD's L2)
+  const unsigned long long* q = (const unsigned long long*)p;
+  const unsigned long long a = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const unsigned long long b = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return u32x4{(uint32_t)a, (uint32_t)(a >> 32), (uint32_t)b, (uint32_t)(b >> 32)};
+}
+__device__ __forceinline__ void store16_agent(void* p, const f32x4& v) {
+  unsigned long long* q = (unsigned long long*)p;
+  __hip_atomic_store(q, ((unsigned long long)__float_as_uint(v.y) << 32) | __float_as_uint(v.x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(q + 1, ((unsigned long long)__float_as_uint(v.w) << 32) | __float_as_uint(v.z), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Keys split over gridDim.z workgroups: a chunk of a prompt that enters next to decoding sequences has few query tiles (32 tokens x 8
+// kv heads: 16 workgroups for 256 CUs) and walked all its keys in one chain of dependent blocks -- 58 us at 640 keys (Qwen3-14B
+// heads, rocprof) whatever the chip could do.  Slice z takes key blocks [z nb / nz, (z + 1) nb / nz), leaves (m, l, O) and counts itself;
+// the last one of a tile adds the slices in order (no spinning; hand-off as in gemm_skinny.hip).  l: summed over the lanes of a query.
+// false: not the last.  part: [tile][slice][wave][64 lanes][DT + 1] x 16 bytes.
+template <int DT>
+__device__ __forceinline__ bool join_slices(const AttnCall& c, int tile, int waves, int wave, int lane, f32x4 (&acc)[DT], float& m, float& l) {
+  const int nz = gridDim.z, z = blockIdx.z;
+  __shared__ int last_sh;
+  float* base = c.partial + ((size_t)tile * nz * waves + wave) * (64 * (DT + 1) * 4) + lane * 4;
+  const size_t slice = (size_t)waves * (64 * (DT + 1) * 4);
+  float* mine = base + z * slice;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) store16_agent(mine + dt * 256, acc[dt]);
+  store16_agent(mine + DT * 256, f32x4{m, l, 0.f, 0.f});
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int* cp = c.counters + tile;
+    const int old = __hip_atomic_fetch_add(cp, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (old == nz - 1) __hip_atomic_store(cp, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);       // for the next launch
+    last_sh = old == nz - 1;
+  }
+  __syncthreads();
+  if (!last_sh) return false;
+  float mz[PREFILL_MAX_SLICES], lz[PREFILL_MAX_SLICES];
+  m = -1e30f;
+#pragma unroll
+  for (int i = 0; i < PREFILL_MAX_SLICES; ++i) {
+    const u32x4 v = load16_agent(base + (size_t)min(i, nz - 1) * slice + DT * 256);
+    mz[i] = i < nz ? __uint_as_float(v.x) : -INFINITY;
+    lz[i] = __uint_as_float(v.y);
+  }
+#pragma unroll
+  for (int i = 0; i < PREFILL_MAX_SLICES; ++i) m = fmaxf(m, mz[i]);
+  l = 0.f;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i0 = 0; i0 < PREFILL_MAX_SLICES; i0 += 2) {
+    if (i0 >= nz) break;                              // (uniform)
+    u32x4 v[2][DT];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) v[j][dt] = load16_agent(base + (size_t)min(i0 + j, nz - 1) * slice + dt * 256);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const float w = __builtin_amdgcn_exp2f(mz[i0 + j] - m);          // (a slice past the last: exp2(-inf) = 0)
+      l += lz[i0 + j] * w;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[dt][r] += __uint_as_float(v[j][dt][r]) * w;
+    }
+  }
+  return true;
 }
 
 constexpr int QT = 16;      // queries per query group (one MFMA column set)
@@ -277,6 +353,7 @@ __global__ __launch_bounds__(G * 64, G >= 2 ? 2 : 1) void attn_prefill_dma_kerne
   const int t0 = qt * QTT;
   const int nk = off + min(t0 + QTT, s.L);            // keys any query of the tile may see
   const int nb = (nk + KB - 1) / KB;
+  const int j0 = (int)((long)blockIdx.z * nb / gridDim.z), j1 = (int)((long)(blockIdx.z + 1) * nb / gridDim.z);   // this slice's blocks
   const int h = kh * G + wave;
 
   // K / V blocks go global -> LDS by LDS-DMA into a ring of THREE buffers: block j + 2 is issued at the head of
@@ -328,8 +405,8 @@ __global__ __launch_bounds__(G * 64, G >= 2 ? 2 : 1) void attn_prefill_dma_kerne
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) qf[u][kk] = *(const u32x4*)(qp + 32 * kk + 8 * g4);
   }
-  dma_block(0, 0);
-  dma_block(1, 1);                                    // (past the last block: clamped keys, masked)
+  dma_block(j0, 0);
+  dma_block(j0 + 1, 1);                               // (past the last block: clamped keys, masked)
   // the Q fragments count as loaded from here on (hipcc waits for its own loads with vmcnt(0): blocks 0 and 1 have landed too)
 #pragma unroll
   for (int u = 0; u < QG; ++u)
@@ -349,9 +426,9 @@ __global__ __launch_bounds__(G * 64, G >= 2 ? 2 : 1) void attn_prefill_dma_kerne
   }
   const int tq4 = c16 >> 2, tp = c16 & 3;
 
-  int buf = 0;                                        // j mod 3
-  for (int j = 0; j < nb; ++j) {
-    const int bnext2 = buf == 0 ? 2 : buf - 1;        // (j + 2) mod 3
+  int buf = 0;                                        // (j - j0) mod 3
+  for (int j = j0; j < j1; ++j) {
+    const int bnext2 = buf == 0 ? 2 : buf - 1;        // (j - j0 + 2) mod 3
     dma_block(j + 2, bnext2);
     f32x4 sc[QG][2];
 #pragma unroll
@@ -441,6 +518,9 @@ __global__ __launch_bounds__(G * 64, G >= 2 ? 2 : 1) void attn_prefill_dma_kerne
     float l = l_run[u];
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
+    if (gridDim.z > 1) {                              // (launched with one query group only)
+      if (!join_slices<DT>(c, bh * gridDim.x + qt, G, wave, lane, accO[u], m_run[u], l)) return;
+    }
     if (t0 + QT * u + c16 < s.L) {
       const float inv = 1.0f / l;
       T* op = (T*)c.out + ((size_t)b * s.L + tq[u]) * s.Hq * D + (size_t)h * D + 4 * g4;
@@ -459,9 +539,10 @@ int launch_pg(const AttnCall& c, hipStream_t st) {
   // one query group per wave.  Two (32 queries per workgroup, every K / V fragment feeding two MFMAs) was built and
   // measured: prefill 83.3 .. 83.8 k tok/s against 84.0 .. 84.1 k (same box, alternating runs) -- the vector ALU bounds the
   // loop, not the LDS traffic -- and 79 k once the leaner softmax below pushed it past 256 registers.
-  const dim3 grid((s.L + QT - 1) / QT, s.B * s.Hkv), block(G * 64);
+  dim3 grid((s.L + QT - 1) / QT, s.B * s.Hkv), block(G * 64);
   const char* env = getenv("MI_ATTN_PREFILL_DMA");     // A/B and the bit-equality test: 0 = the register-staged kernel (read per call)
   if (env == nullptr || atoi(env) != 0) {
+    grid.z = c.nsplit;
     if (s.btab) hipLaunchKernelGGL((attn_prefill_dma_kernel<T, D, G, true, 1>), grid, block, 0, st, c);
     else hipLaunchKernelGGL((attn_prefill_dma_kernel<T, D, G, false, 1>), grid, block, 0, st, c);
   } else {
@@ -660,6 +741,7 @@ __global__ __launch_bounds__(G * 64, 2) void attn_prefill_f32s_kernel(AttnCall c
   const int t0 = qt * QT;
   const int nk = off + min(t0 + QT, s.L);             // keys any query of the tile may see
   const int nb = (nk + KB - 1) / KB;
+  const int j0 = (int)((long)blockIdx.z * nb / gridDim.z), j1 = (int)((long)(blockIdx.z + 1) * nb / gridDim.z);   // this slice's blocks
   const int h = kh * G + wave;
 
   __shared__ __attribute__((aligned(16))) unsigned char khi[2][IMG];
@@ -709,7 +791,7 @@ __global__ __launch_bounds__(G * 64, 2) void attn_prefill_f32s_kernel(AttnCall c
     }
   };
 
-  load_block(0);
+  load_block(j0);
   // Q^T fragments of this wave's head (B operand: column = query), hi and lo
   u32x4 qh[KK], ql[KK];
   const int tq = min(t0 + c16, s.L - 1);              // this lane's query (clamped; stores are guarded)
@@ -738,8 +820,8 @@ __global__ __launch_bounds__(G * 64, 2) void attn_prefill_f32s_kernel(AttnCall c
   for (int dt = 0; dt < DT; ++dt) accO[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int tq4 = c16 >> 2, tp = c16 & 3;
 
-  for (int j = 0; j < nb; ++j) {
-    const int buf = j & 1;
+  for (int j = j0; j < j1; ++j) {
+    const int buf = (j - j0) & 1;
     load_block(j + 1);                                // straight-line (past the last block: clamped keys, never stored); the loads fly during this block's work
     f32x4 sc[2];
 #pragma unroll
@@ -804,12 +886,15 @@ __global__ __launch_bounds__(G * 64, 2) void attn_prefill_f32s_kernel(AttnCall c
       accO[dt] = mfma16<T>(vfh, pl, accO[dt]);
       accO[dt] = mfma16<T>(vfl, pf, accO[dt]);
     }
-    if (j + 1 < nb) store_block(buf ^ 1);             // the other buffer: nobody reads it during this block
+    if (j + 1 < j1) store_block(buf ^ 1);             // the other buffer: nobody reads it during this block
     __syncthreads();
   }
 
   l_run += __shfl_xor(l_run, 16, 64);
   l_run += __shfl_xor(l_run, 32, 64);
+  if (gridDim.z > 1) {
+    if (!join_slices<DT>(c, bh * gridDim.x + qt, G, wave, lane, accO, m_run, l_run)) return;
+  }
   if (t0 + c16 < s.L) {
     const float inv = 1.0f / l_run;
     float* op = (float*)c.out + ((size_t)b * s.L + tq) * s.Hq * D + (size_t)h * D + 4 * g4;
@@ -825,9 +910,10 @@ __global__ __launch_bounds__(G * 64, 2) void attn_prefill_f32s_kernel(AttnCall c
 template <int D, int G>
 int launch_pg32(const AttnCall& c, hipStream_t st) {
   const AttnShape& s = c.s;
-  const dim3 grid((s.L + QT - 1) / QT, s.B * s.Hkv), block(G * 64);
+  dim3 grid((s.L + QT - 1) / QT, s.B * s.Hkv), block(G * 64);
   const char* env = getenv("MI_ATTN_PREFILL_F32_EXACT");   // A/B and the comparison test (read per call): 1 = exact float32 products
   if (env == nullptr || atoi(env) == 0) {
+    grid.z = c.nsplit;
     if (s.btab) hipLaunchKernelGGL((attn_prefill_f32s_kernel<D, G, true>), grid, block, 0, st, c);
     else hipLaunchKernelGGL((attn_prefill_f32s_kernel<D, G, false>), grid, block, 0, st, c);
   } else if (s.btab) hipLaunchKernelGGL((attn_prefill_f32_kernel<D, G, true>), grid, block, 0, st, c);
@@ -860,9 +946,22 @@ bool attention_prefill_supported(const AttnShape& s) {
   return s.D == 32 || s.D == 64 || s.D == 128;
 }
 
+// Slices of the keys: as many as fill the chip (one workgroup per CU), each with at least two blocks of the longest tile's keys; a call
+// that has a workgroup for most CUs by itself is not cut (its slices would only queue behind each other and pay the join).
+int attention_prefill_slices(const AttnShape& s, int max_keys) {
+  if (!attention_prefill_supported(s)) return 1;
+  const int tiles = (s.L + QT - 1) / QT * s.B * s.Hkv, blocks = (max_keys + KB - 1) / KB;
+  return std::max(1, std::min({gemv_cu_count() / tiles, blocks / 2, PREFILL_MAX_SLICES}));
+}
+size_t attention_prefill_part_floats(const AttnShape& s, int slices) {
+  return (size_t)((s.L + QT - 1) / QT) * s.B * s.Hkv * slices * (s.Hq / s.Hkv) * 64 * (s.D / 16 + 1) * 4;
+}
+int attention_prefill_tiles(const AttnShape& s) { return (s.L + QT - 1) / QT * s.B * s.Hkv; }
+
 int launch_attention_prefill(const AttnCall& c, hipStream_t st) {
   if (!attention_prefill_supported(c.s)) return fail(MI_ERR_UNSUPPORTED, "attention_prefill: shape / dtype not supported");
-  if (c.nsplit != 1) return fail(MI_ERR_INVALID, "attention_prefill: no split-KV");
+  if (c.nsplit < 1 || c.nsplit > PREFILL_MAX_SLICES || (c.nsplit > 1 && (c.partial == nullptr || c.counters == nullptr)))
+    return fail(MI_ERR_INVALID, "attention_prefill: bad split configuration");
   if (c.s.act == MI_F32) return c.s.D == 128 ? launch_pd32<128>(c, st) : launch_pd32<64>(c, st);
   return c.s.act == MI_BF16 ? launch_pt<bf16>(c, st) : launch_pt<f16>(c, st);
 }

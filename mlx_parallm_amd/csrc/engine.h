@@ -187,6 +187,8 @@ struct mi_engine {
   int last_n = 0;                        // rows of the last enqueued step (device-resident token feed)                // value of *d_seam_counter once every enqueued launch has run
   void* xn = nullptr;            // [rows][max(H, I)] normalised activations of the prefill GEMMs
   void* xs = nullptr; size_t xs_cap = 0;   // [rows][3 K] bf16: float32 activations split three ways (float32-KV prefill)
+  float* ap_part = nullptr; size_t ap_part_cap = 0;       // prefill attention with split keys: the slices' partial results ..
+  int* ap_ctr = nullptr; size_t ap_ctr_cap = 0;           // .. and arrival tickets (zero between launches)
   void* gk_ws = nullptr; size_t gk_cap = 0;   // float32 partial tiles of the K-split 128 x 128 tile GEMM
   // ---- layer-list models (engine_layers.hip)
   bool layered = false;

@@ -670,6 +670,31 @@ int choose_nsplit(const mi_kv* kv, int B, int Hkv, int L, const int32_t* rows = 
   return std::max(1, std::min(ns, 16));
 }
 
+// prefill attention (L > 1): the keys split over workgroups where the query tiles alone leave the chip idle
+int split_prefill(mi_engine* e, AttnCall& ac, int max_keys) {
+  ac.nsplit = 1; ac.partial = nullptr;
+  if (ac.variant == 1) return MI_OK;
+  const int n = attention_prefill_slices(ac.s, max_keys);
+  if (n <= 1) return MI_OK;
+  const size_t need = attention_prefill_part_floats(ac.s, n), ctr = attention_prefill_tiles(ac.s);
+  if (need > e->ap_part_cap) {
+    MI_HIP(hipStreamSynchronize(e->stream));
+    hipFree(e->ap_part); e->ap_part = nullptr; e->ap_part_cap = 0;
+    MI_HIP(hipMalloc(&e->ap_part, need * sizeof(float)));
+    e->ap_part_cap = need;
+  }
+  if (ctr > e->ap_ctr_cap) {
+    MI_HIP(hipStreamSynchronize(e->stream));
+    hipFree(e->ap_ctr); e->ap_ctr = nullptr; e->ap_ctr_cap = 0;
+    const size_t cap = std::max<size_t>(ctr, 256);       // (at most one tile per CU where the keys are split)
+    MI_HIP(hipMalloc(&e->ap_ctr, cap * sizeof(int)));
+    MI_HIP(hipMemsetAsync(e->ap_ctr, 0, cap * sizeof(int), e->stream));
+    e->ap_ctr_cap = cap;
+  }
+  ac.nsplit = n; ac.partial = e->ap_part; ac.counters = e->ap_ctr;
+  return MI_OK;
+}
+
 // the model forward for B*L tokens already in e->d_tokens; logits of the requested rows end
 // up in e->logits (float32, [B][V] or [B*L][V]).
 // `rows` (host, B distinct cache rows) = the call covers that subset of kv's rows, batch entry b <-> rows[b]
@@ -773,6 +798,11 @@ int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool wan
         AttnShape sa = s; sa.rnd = RND_NONE;  // SDPA output dtype = promote(q, kv): float32 in quirk mode
         AttnCall ac{sa, e->q, kc, vc, kv->d_off, e->attn, 1.0f / sqrtf((float)D), nsplit, kv->partial,
                     e->opt_attn_mfma ? 0 : 1};
+        if (L > 1) {
+          int mx = 0;
+          for (int b = 0; b < B; ++b) mx = std::max(mx, kv->h_off[row_of(b)] + L);
+          MI_TRY(split_prefill(e, ac, mx));
+        }
         MI_TRY(launch_attention(ac, st)); }
     }
     {
@@ -906,6 +936,7 @@ int forward_mixed(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t* l
       MI_TRY(launch_rope_append(rc, st));
       AttnShape sa = s; sa.rnd = RND_NONE;
       AttnCall ac{sa, q_i, kc, vc, kv->d_off, o_i, 1.0f / sqrtf((float)D), 1, nullptr, e->opt_attn_mfma ? 0 : 1};
+      MI_TRY(split_prefill(e, ac, kv->h_off[rows[i]] + lens[i]));
       MI_TRY(launch_attention(ac, st));
     }
     { GemvCall co; co.x = e->attn; co.ldx = Hq * D; co.act = act; co.rnd = RND_NONE; co.epi = EPI_RESID; co.resid = e->h; co.ldo = H;
@@ -1064,7 +1095,7 @@ void mi_engine_destroy(mi_engine* e) {
   hipFree(e->final_norm); hipFree(e->cos_tab); hipFree(e->sin_tab);
   hipFree(e->h); hipFree(e->qkv); hipFree(e->q); hipFree(e->attn); hipFree(e->act); hipFree(e->logits); hipFree(e->lora_t); hipFree(e->d_forced); hipFree(e->d_gather);
   hipFree(e->d_seam_counter); hipFree(e->d_seam_error); hipHostFree(e->h_seam_err); hipFree(e->d_rowpar); hipFree(e->deq_scratch);
-  hipFree(e->sk_ws); hipFree(e->sk_ctr); hipFree(e->d_sq);
+  hipFree(e->sk_ws); hipFree(e->sk_ctr); hipFree(e->d_sq); hipFree(e->ap_part); hipFree(e->ap_ctr);
   hipFree(e->d_tokens); hipFree(e->d_next); hipFree(e->d_rowstats);
   hipFree(e->d_uniforms); hipFree(e->d_topk_ids); hipFree(e->d_topk_lp); hipFree(e->d_bias_ids); hipFree(e->d_bias_vals);
   for (auto& s : e->slots) {

@@ -235,13 +235,18 @@ struct AttnCall {
   const int32_t* offsets;  // device [B]: tokens in the cache BEFORE this call's L were appended
   void* out;             // [B*L][Hq*D]
   float scale;
-  int nsplit;            // >1 only for L == 1
-  float* partial;        // [B*L*Hq][nsplit][D+2] when nsplit > 1
+  int nsplit;            // > 1: L == 1, or the MFMA prefill kernels (attention_prefill_slices)
+  float* partial;        // nsplit > 1: [B*L*Hq][nsplit][D+2], or attention_prefill_part_floats()
   int variant;           // 0: L > 1 goes to the MFMA prefill kernel where it applies; 1: always the VALU kernel
+  int* counters = nullptr;   // nsplit > 1, L > 1: attention_prefill_tiles() arrival tickets, zero between launches
 };
 int launch_attention(const AttnCall& c, hipStream_t st);
 // causal prefill attention on the matrix cores (attn_prefill.hip); launch_attention dispatches to it
 bool attention_prefill_supported(const AttnShape& s);
+// over how many workgroups the keys of a call that reaches at most max_keys keys are split, and what that needs
+int attention_prefill_slices(const AttnShape& s, int max_keys);
+size_t attention_prefill_part_floats(const AttnShape& s, int slices);
+int attention_prefill_tiles(const AttnShape& s);
 int launch_attention_prefill(const AttnCall& c, hipStream_t st);
 
 // fused decode step (L == 1): q/k norm + RoPE + KV append + split-KV attention + combine

@@ -652,6 +652,34 @@ def test_mixed_steps_chunked_prefill_next_to_decode_rows(tiny_dirs, name, kvd):
     eng.close()
 
 
+@pytest.mark.parametrize("name", ["qwen3_bf16", "llama_f16"])
+@pytest.mark.parametrize("kvd", ["model", "float32"])
+def test_a_chunk_behind_cached_tokens_splits_its_keys(tiny_dirs, name, kvd):
+    """Prefill attention of a few query tiles: the keys are split over workgroups (attention_prefill_slices) and the slices' softmax
+    states joined.  Chunks around the tile edge (16 queries) behind caches around the block and slice edges (32 keys, two blocks a
+    slice), rows of different lengths, contiguous and paged: all positions against the oracle's whole sequence."""
+    model, ref, cfg = _load_pair(tiny_dirs, name)
+    eng = model.engine
+    tol = 4e-3 if kvd == "float32" else 0.1           # (the bounds of the prefill comparisons above)
+    for off, L in [(0, 65), (1, 64), (63, 2), (64, 15), (127, 16), (130, 17), (300, 33), (440, 50)]:
+        toks = RNG.integers(3, cfg["vocab_size"], size=(2, off + L)).astype(np.int32)
+        want = ref(toks, cache=ref.make_cache(2, paged=kvd == "float32"))
+        for paged in (False, True):
+            kv = eng.new_paged_kv(2, block_tokens=16, max_tokens_per_row=512, kv_dtype=kvd) if paged else eng.new_kv(2, capacity=512, kv_dtype=kvd)
+            if off:
+                eng.forward(toks[:, :off], kv, want_logits=False)
+            got = eng.forward(toks[:, off:], kv, all_positions=True)
+            assert np.abs(got - want[:, off:]).max() <= tol, (off, L, paged, np.abs(got - want[:, off:]).max())
+            kv.reset()
+            if off > 40:                              # one row alone, its cache shorter: more slices, another row's blocks untouched
+                short = off - 37
+                eng.step_wait(eng.step_enqueue_rows(kv, [1], toks[1:, :short], SampleArgs(temp=0.0)), 1)
+                got = eng.forward_segments(kv, [1], [toks[1, short:]], [off + L - short - 1])
+                assert np.abs(got[0] - want[1, -1]).max() <= tol, (off, L, paged)
+            kv.close()
+    eng.close()
+
+
 def test_converted_checkpoint_and_lora_hot_swap(tiny_dirs, tmp_path):
     """a directory written by convert(quantize=True) loads and matches the oracle on the same
     files; weight_updater swaps adapters on the live engine (adapters.safetensors + config, then adapter.npz)."""
