@@ -14,6 +14,8 @@
 // wave-instruction, weights go HBM -> VGPR directly, never through LDS); the activations are
 // staged once per workgroup into LDS as fp32 in K-chunks of KC; fp32 accumulate; one
 // butterfly reduction per row at the end.
+#include <algorithm>
+
 #include "kernels.h"
 
 namespace mi {
@@ -110,6 +112,57 @@ __device__ __forceinline__ void load8(const GemvParams& p, int row, int kb, floa
 __device__ __forceinline__ int xs_addr(int m, int kk) {
   const int ks = kk >> 9, ln = (kk & 511) >> 3, half = (kk & 7) >> 2, j = kk & 3;
   return ((((m * (KC / 512) + ks) * 2 + half) * 64 + ln) << 2) + j;
+}
+
+// nn.silu(gate) * up, every op rounded to the activation dtype (llama.py:165), or another unit
+template <typename AT>
+__device__ __forceinline__ void finish_glu(const GemvParams& p, int m, int n, float gate, float up) {
+  AT* out = (AT*)p.out;
+  if (p.glu.kind != GLU_SILU) { out[(size_t)m * p.ldo + n] = store_act<AT>(glu_f(p.glu, gate, up), p.rnd); return; }
+  const float g = to_f32(store_act<AT>(gate, p.rnd));
+  const float u = to_f32(store_act<AT>(up, p.rnd));
+  const float sig = to_f32(store_act<AT>(1.0f / (1.0f + expf(-g)), p.rnd));
+  const float s = to_f32(store_act<AT>(g * sig, p.rnd));
+  out[(size_t)m * p.ldo + n] = store_act<AT>(s * u, p.rnd);
+}
+// the other epilogues of y[m][n] = v
+template <typename AT>
+__device__ __forceinline__ void finish_one(const GemvParams& p, int m, int n, float v) {
+  AT* out = (AT*)p.out;
+  if (p.out32) {
+    if (p.epi == EPI_RESID) { float* h32 = (float*)p.resid + (size_t)m * p.ldo + n; *h32 = *h32 + v; }
+    else ((float*)p.out)[(size_t)m * p.ldo + n] = v;
+    return;
+  }
+  float y = to_f32(store_act<AT>(silu_col(p.silu_cols, n, v), p.rnd));
+  // LoRALinear: y + (scale * ((x A) B)).astype(x.dtype)
+  if (p.lora_t != nullptr) {
+#pragma unroll
+    for (int sl = 0; sl < 2; ++sl) {
+      const int row0 = sl ? p.lora_row0_1 : p.lora_row0_0;
+      const int ln = sl ? p.lora_n_1 : p.lora_n_0;
+      const int rk = sl ? p.lora_rank_1 : p.lora_rank_0;
+      const float* lb = sl ? p.lora_b1 : p.lora_b0;
+      if (lb != nullptr && n >= row0 && n < row0 + ln) {
+        const float* t = p.lora_t + (size_t)m * p.lora_t_ld + sl * (p.lora_t_ld / 2);
+        float z = 0.f;
+        for (int j = 0; j < rk; ++j) z = fmaf(t[j], lb[(size_t)j * ln + (n - row0)], z);
+        z = round_rt(z, p.lora_rnd);
+        z = round_rt((sl ? p.lora_scale_1 : p.lora_scale_0) * z, p.lora_rnd);
+        z = to_f32(store_act<AT>(z, p.rnd));
+        y = to_f32(store_act<AT>(y + z, p.rnd));
+      }
+    }
+  }
+  if (p.epi == EPI_STORE) {
+    out[(size_t)m * p.ldo + n] = from_f32<AT>(y);
+  } else if (p.epi == EPI_STORE_F32) {
+    ((float*)p.out)[(size_t)m * p.ldo + n] = y;
+  } else {  // EPI_RESID
+    AT* h = (AT*)p.resid;
+    const float hv = to_f32(h[(size_t)m * p.ldo + n]);
+    h[(size_t)m * p.ldo + n] = store_act<AT>(hv + y, p.rnd);
+  }
 }
 
 template <typename AT, int WK, int MT>
@@ -230,55 +283,91 @@ __global__ __launch_bounds__(NTHR) void gemv_v1_kernel(GemvParams p) {
       }
     if (!pvalid[a] || lane >= p.M || lane >= MT) continue;
     const int m = lane;
-    AT* out = (AT*)p.out;
     if (p.epi == EPI_SWIGLU) {
-      // nn.silu(gate) * up, every op rounded to the activation dtype (llama.py:165)
-      if (p.glu.kind != GLU_SILU) { out[(size_t)m * p.ldo + rows[a][0]] = store_act<AT>(glu_f(p.glu, mine[0], mine[1]), p.rnd); continue; }
-      const float g = to_f32(store_act<AT>(mine[0], p.rnd));
-      const float u = to_f32(store_act<AT>(mine[1], p.rnd));
-      const float sig = to_f32(store_act<AT>(1.0f / (1.0f + expf(-g)), p.rnd));
-      const float s = to_f32(store_act<AT>(g * sig, p.rnd));
-      out[(size_t)m * p.ldo + rows[a][0]] = store_act<AT>(s * u, p.rnd);
+      finish_glu<AT>(p, m, rows[a][0], mine[0], mine[1]);
       continue;
     }
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
       const int n = rows[a][r];
       if (r == 1 && 2 * ((blockIdx.x * 4 + wave) * PW + a) + 1 >= p.N) continue;
-      if (p.out32) {
-        if (p.epi == EPI_RESID) { float* h32 = (float*)p.resid + (size_t)m * p.ldo + n; *h32 = *h32 + mine[r]; }
-        else ((float*)p.out)[(size_t)m * p.ldo + n] = mine[r];
-        continue;
-      }
-      float y = to_f32(store_act<AT>(silu_col(p.silu_cols, n, mine[r]), p.rnd));
-      // LoRALinear: y + (scale * ((x A) B)).astype(x.dtype)
-      if (p.lora_t != nullptr) {
+      finish_one<AT>(p, m, n, mine[r]);
+    }
+  }
+}
+
+// Rows of at most 512 inputs.  In gemv_v1_kernel a wave spreads one row over its 64 lanes and every workgroup stages (and zero-fills)
+// a 2048-wide image of x: at 64 inputs 8 of 64 lanes have work.  Here LG lanes hold a row (LG = 8, 16, 64), a wave takes 64 / LG of
+// them at a time, and a lane keeps its 8 columns of x for every batch row in registers -- normed there, so nothing goes through LDS
+// and no barrier stands in front of the weights.  int4, 64 inputs, 2 rows, float32 activations: 151936 outputs 74 -> 12 us, 192 outputs
+// 9.8 -> 4.7 us (rocprof; an empty kernel is 4).
+template <typename AT, int WK, int MT, int LG, bool GLU>
+__global__ __launch_bounds__(NTHR) void gemv_short_kernel(GemvParams p) {
+  constexpr int NR = GLU ? 2 : 1, RPW = 64 / LG, U = GLU || MT > 2 ? 2 : 4;
+  const int tid = threadIdx.x, lane = tid & 63, grp = lane / LG, gl = lane % LG, k = gl * 8;
+  const bool on = k < p.K;
+  const AT* x = (const AT*)p.x;
+  float xv[MT][8];
 #pragma unroll
-        for (int sl = 0; sl < 2; ++sl) {
-          const int row0 = sl ? p.lora_row0_1 : p.lora_row0_0;
-          const int ln = sl ? p.lora_n_1 : p.lora_n_0;
-          const int rk = sl ? p.lora_rank_1 : p.lora_rank_0;
-          const float* lb = sl ? p.lora_b1 : p.lora_b0;
-          if (lb != nullptr && n >= row0 && n < row0 + ln) {
-            const float* t = p.lora_t + (size_t)m * p.lora_t_ld + sl * (p.lora_t_ld / 2);
-            float z = 0.f;
-            for (int j = 0; j < rk; ++j) z = fmaf(t[j], lb[(size_t)j * ln + (n - row0)], z);
-            z = round_rt(z, p.lora_rnd);
-            z = round_rt((sl ? p.lora_scale_1 : p.lora_scale_0) * z, p.lora_rnd);
-            z = to_f32(store_act<AT>(z, p.rnd));
-            y = to_f32(store_act<AT>(y + z, p.rnd));
-          }
+  for (int m = 0; m < MT; ++m) {
+    const AT* xr = x + (size_t)min(m, p.M - 1) * p.ldx + (on ? k : 0);
+    alignas(16) AT e[8];
+#pragma unroll
+    for (int j = 0; j < (int)sizeof(AT) / 2; ++j) ((u32x4*)e)[j] = ((const u32x4*)xr)[j];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) xv[m][j] = on ? to_f32(e[j]) : 0.f;
+  }
+  auto group_sum = [&](float v) {                    // all-reduce over the LG lanes of a row
+    if constexpr (LG == 8) return lane8_sum(v);
+    v = row16_sum(v);
+    if constexpr (LG == 64) { v += __shfl_xor(v, 16); v += __shfl_xor(v, 32); }
+    return v;
+  };
+  if (p.pro == PRO_NORM) {
+    alignas(16) AT nw[8];
+#pragma unroll
+    for (int j = 0; j < (int)sizeof(AT) / 2; ++j) ((u32x4*)nw)[j] = ((const u32x4*)((const AT*)p.norm_w + (on ? k : 0)))[j];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ss = fmaf(xv[m][j], xv[m][j], ss);
+      const float rs = 1.0f / sqrtf(group_sum(ss) / (float)p.K + p.eps);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const AT xn = store_act<AT>(xv[m][j] * rs, p.rnd);
+        xv[m][j] = on ? to_f32(store_act<AT>(to_f32(xn) * to_f32(nw[j]), p.rnd)) : 0.f;
+      }
+    }
+  }
+  const int items = GLU ? p.pair_offset : p.N, waves = gridDim.x * (NTHR / 64);
+  for (int it0 = (blockIdx.x * (NTHR / 64) + (tid >> 6)) * RPW; it0 < items; it0 += waves * RPW * U) {      // (uniform per wave)
+    float w8[U][NR][8];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int it = min(it0 + u * waves * RPW + grp, items - 1);
+#pragma unroll
+      for (int r = 0; r < NR; ++r) load8<WK>(p, it + r * p.pair_offset, on ? k : 0, w8[u][r]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int it = it0 + u * waves * RPW + grp;
+      float mine[NR];
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        mine[r] = 0.f;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          float a = 0.f;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) a = fmaf(w8[u][r][j], xv[m][j], a);
+          a = group_sum(a);
+          if (gl == m) mine[r] = a;
         }
       }
-      if (p.epi == EPI_STORE) {
-        out[(size_t)m * p.ldo + n] = from_f32<AT>(y);
-      } else if (p.epi == EPI_STORE_F32) {
-        ((float*)p.out)[(size_t)m * p.ldo + n] = y;
-      } else {  // EPI_RESID
-        AT* h = (AT*)p.resid;
-        const float hv = to_f32(h[(size_t)m * p.ldo + n]);
-        h[(size_t)m * p.ldo + n] = store_act<AT>(hv + y, p.rnd);
-      }
+      if (it >= items || gl >= p.M || gl >= MT) continue;
+      if constexpr (GLU) finish_glu<AT>(p, gl, it, mine[0], mine[1]);
+      else finish_one<AT>(p, gl, it, mine[0]);
     }
   }
 }
@@ -394,8 +483,34 @@ __global__ __launch_bounds__(256) void lora_up_add_kernel(GemvParams p, const fl
   }
 }
 
+template <typename AT, int WK, int MT>
+int launch_short(const GemvParams& p, hipStream_t st) {
+  const bool glu = p.epi == EPI_SWIGLU;
+  const int lg = p.K <= 64 ? 8 : p.K <= 128 ? 16 : 64;
+  const int items = glu ? p.pair_offset : p.N;
+  // (2048 workgroups: eight per CU, what 64-register waves allow; more rows than that are looped over)
+  const int nwg = std::min(2048, (items + 4 * (64 / lg) - 1) / (4 * (64 / lg)));
+  auto go = [&](auto kern) -> int {
+    hipLaunchKernelGGL(kern, dim3(nwg), dim3(NTHR), 0, st, p);
+    MI_HIP(hipGetLastError());
+    return MI_OK;
+  };
+#define GO(LG) return glu ? go(gemv_short_kernel<AT, WK, MT, LG, true>) : go(gemv_short_kernel<AT, WK, MT, LG, false>)
+  if (lg == 8) GO(8);
+  if (lg == 16) GO(16);
+  GO(64);
+#undef GO
+}
+
 template <typename AT, int WK>
 int launch_mt(const GemvParams& p, hipStream_t st) {
+  // short rows: x and the norm weights are read 16 bytes at a time there
+  const bool al = ((uintptr_t)p.x | (uintptr_t)(p.pro == PRO_NORM ? p.norm_w : nullptr)) % 16 == 0 && (size_t)p.ldx * sizeof(AT) % 16 == 0;
+  if (p.K <= 512 && al) {
+    if (p.M <= 2) return launch_short<AT, WK, 2>(p, st);
+    if (p.M <= 4) return launch_short<AT, WK, 4>(p, st);
+    return launch_short<AT, WK, 8>(p, st);
+  }
   const int nwg = (p.npairs + 4 * PW - 1) / (4 * PW);
   auto go = [&](auto kern, int MT) -> int {
     const size_t lds = (size_t)(MT * KC + MT + 4 * MT) * sizeof(float);

@@ -154,6 +154,30 @@ def test_gemv_epilogues(act, kind, force_generic):
     _assert_close(host(out), want, act)
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 8])
+@pytest.mark.parametrize("act,kind,K", [("float32", "f32", 8), ("float32", "f32", 72), ("float32", "q4_f32", 64), ("float32", "q8_f32", 128), ("float32", "f32", 136),
+                                        ("bfloat16", "bf16", 264), ("float16", "q4_f16", 256), ("float32", "f32", 512), ("bfloat16", "q8_bf16", 512), ("float32", "f32", 520)])
+def test_gemv_short_rows(act, kind, K, M):
+    """Rows of at most 512 inputs (gemv_short_kernel: 8, 16 or 64 lanes a row) and one beyond, outputs that do not divide the waves'
+    shares, more outputs than one pass of the grid at 64 lanes a row, SwiGLU pairs, and a row stride that is no multiple of 16 bytes."""
+    for N, pad in ((77, 0), (3, 0), (40000 if K == 512 and M == 2 else 600, 0), (50, 1)):
+        ol, wdense, keep = _make_weight(kind, N, K, act)
+        x = round_to(RNG.standard_normal((M, K)).astype(np.float32), act)
+        nw = round_to(1.0 + 0.1 * RNG.standard_normal(K).astype(np.float32), act)
+        xn, _ = ref_model.rms_norm(x, act, nw, act, 1e-5)
+        xd = dev(np.pad(x, ((0, 0), (0, pad))), act)
+        out = torch.zeros((M, N), dtype=xd.dtype, device="cuda")
+        gemv(ol, xd, M, act, pro=L.PRO_NORM, norm_w=dev(nw, act), eps=1e-5, epi=L.EPI_STORE, out=out, ldo=N, force_generic=1, ldx=K + pad)
+        _assert_close(host(out), round_to(matmul_nt(xn, wdense), act), act)
+    I = 37
+    ol, wdense, keep = _make_weight(kind, 2 * I, K, act)
+    g, u = round_to(matmul_nt(x, wdense[:I]), act), round_to(matmul_nt(x, wdense[I:]), act)
+    sig = round_to(1.0 / (1.0 + np.exp(-g.astype(np.float64))), act)
+    out = torch.zeros((M, I), dtype=xd.dtype, device="cuda")
+    gemv(ol, dev(x, act), M, act, epi=L.EPI_SWIGLU, out=out, ldo=I, pair_offset=I, force_generic=1)
+    _assert_close(host(out), round_to(round_to(g * sig, act) * u, act), act)
+
+
 @pytest.mark.parametrize("M", [9, 16])
 @pytest.mark.parametrize("act,kind", [("bfloat16", "bf16"), ("bfloat16", "q4_bf16"), ("float16", "q4_f16")])
 def test_gemv_mfma_16_rows(act, kind, M):
