@@ -367,16 +367,19 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
       // matrices keep the exact three (their own pair needs the 3 : 2 walk)
       // The rounded call of layer 0: its input is a bf16 value, i.e. one term (8 x 1024 rows of Mistral-7B: 256 launches of the
       // streaming kernel at 32 rows each, 4.6 ms, against 0.4 ms here).
-      const int terms = c.rnd == RND_BF16 ? 1 : (e->opt_prefill_x_terms == 2 && f.W.wk == WK_BF16 && c.kx == 0 && c.rnd == RND_NONE) ? 2 : 3;
+      // (Logits keep the three terms that they had on the streaming kernel.)
+      const int terms = c.rnd == RND_BF16 ? 1 : (e->opt_prefill_x_terms == 2 && f.W.wk == WK_BF16 && c.kx == 0 && c.rnd == RND_NONE && c.epi != EPI_STORE_F32) ? 2 : 3;
       MI_TRY(launch_split3_rows(c.x, c.ldx, c.pro == PRO_NORM ? c.norm_w : nullptr, c.eps, e->xs, (int)rows, KT, e->stream, terms, c.rnd));
       c.x = e->xs; c.ldx = terms * KT; c.pro = PRO_NONE;
     } else if (c.pro == PRO_NORM) {    // (one workgroup per row also here: one L2 round trip per row instead of a wave's 16)
       MI_TRY(launch_rmsnorm_rows(c.x, c.ldx, c.norm_w, e->xn, KT, (int)rows, KT, c.eps, c.act, e->stream, true));
       c.x = e->xn; c.ldx = KT; c.pro = PRO_NONE;
     }
+    // logits of many positions against a quantised matrix: 32768 outputs at a time, so that the copy below stays within 4 x 32768 x K bytes
+    const int ncol = (wk_is_quant(f.W.wk) && c.epi == EPI_STORE_F32) ? std::min(f.W.N, 32768) : f.W.N;
     void* scratch = nullptr;
     if (wk_is_quant(f.W.wk)) {               // int4: the GEMM multiplies by a [hi | lo] 16-bit copy made on the fly
-      const size_t need = dequant_hilo_bytes(f.W.N, KT);
+      const size_t need = dequant_hilo_bytes(ncol, KT);
       if (need > e->deq_cap) {
         MI_HIP(hipStreamSynchronize(e->stream));
         hipFree(e->deq_scratch);
@@ -390,7 +393,16 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
       e->gk_cap = (size_t)128 << 20;
       if (hipMalloc(&e->gk_ws, e->gk_cap) != hipSuccess) { e->gk_ws = nullptr; e->gk_cap = 0; }
     }
-    MI_TRY(launch_gemm_prefill(f.W, c, rows, e->stream, scratch, rows < 4096 ? e->gk_ws : nullptr, e->gk_cap));
+    for (int n0 = 0; n0 < f.W.N; n0 += ncol) {
+      LinearW part = f.W;
+      GemvCall cp = c;
+      if (ncol < f.W.N) {
+        part.N = std::min(ncol, f.W.N - n0);
+        part.w = (const char*)f.W.w + (wk_bits(f.W.wk) == 4 ? tiled_block_q4(n0, 0, f.W.K) : tiled_block_q8(n0, 0, f.W.K));
+        cp.out = (float*)c.out + n0;
+      }
+      MI_TRY(launch_gemm_prefill(part, cp, rows, e->stream, scratch, rows < 4096 ? e->gk_ws : nullptr, e->gk_cap));
+    }
     if (f.W.lora_b[0] != nullptr || f.W.lora_b[1] != nullptr) {   // y = T(y + T(scale (x A) B)) on the adapted columns
       GemvCall cl = c.act == MI_F32 ? c_in : c;
       cl.M = (int)rows;

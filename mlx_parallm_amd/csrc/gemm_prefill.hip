@@ -1176,7 +1176,6 @@ bool gemm_prefill_supported(const LinearW& W, const GemvCall& c, size_t rows) {
                    c.ldx % 4 == 0 && W.K % 4 == 0;
   if (!dense && !q4 && !q8 && !x32) return false;
   if (W.K % BK != 0 || (!x32 && c.ldx % 8 != 0)) return false;
-  if (c.epi == EPI_STORE_F32) return false;
   if (c.out32 && (c.epi == EPI_SWIGLU || W.lora_b[0] || W.lora_b[1])) return false;
   // an adapted matrix: the caller adds the LoRA term to the stored output afterwards (launch_lora_up_add)
   if ((W.lora_b[0] != nullptr || W.lora_b[1] != nullptr) && c.epi != EPI_STORE) return false;
@@ -1248,6 +1247,10 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
   }
   if (c.out32) p.out32 = 1;
   p.epi = c.epi; p.out = c.out; p.ldo = c.ldo; p.resid = c.resid; p.pair_offset = c.pair_offset;
+  if (c.epi == EPI_STORE_F32) {            // logits: float32, rounded to the activation dtype first
+    p.epi = EPI_STORE;
+    if (!x32) { p.out32 = 1; p.rnd = c.act == MI_BF16 ? RND_BF16 : RND_F16; }
+  }
   p.glu = c.glu; p.silu_cols = c.silu_cols;
   const bool sw = c.epi == EPI_SWIGLU;
   const int ncols = sw ? c.pair_offset : W.N;

@@ -154,6 +154,30 @@ def test_float32_kv_prefill_first_layer_on_the_tile_gemm(tiny_dirs, name, B, L0)
     eng.close()
 
 
+@pytest.mark.parametrize("dtype,bits", [("bfloat16", 4), ("float16", 8), ("bfloat16", 0)])
+@pytest.mark.parametrize("kvd", ["model", "float32"])
+def test_logits_of_many_positions_on_the_tile_gemm(tmp_path, dtype, bits, kvd):
+    """Logits of all positions of a call of 32 rows or more: the output matrix on the tile GEMM, a quantised one 32768 outputs at a time
+    (the vocabulary here: two pieces, the second short).  Against the streaming kernels' logits on the same weights."""
+    from mlx_parallm_amd.tiny_model import build_tiny_model
+
+    cfg = build_tiny_model(tmp_path, seed=11, vocab_size=33008, dtype=dtype, quantize_model=bits > 0, q_bits=bits or 4, hidden_size=256, layers=1, heads=4,
+                           kv_heads=2, intermediate_size=256, head_dim=64, tie_word_embeddings=False, with_tokenizer=False)
+    model = utils.load_model(str(tmp_path), max_positions=512)
+    eng = model.engine
+    for B, Lt in ((1, 33), (3, 100)):
+        toks = RNG.integers(3, cfg["vocab_size"], size=(B, Lt)).astype(np.int32)
+        outs = {}
+        for on in (1, 0):
+            eng.set_option("prefill_gemm", on)
+            kv = eng.new_kv(B, capacity=Lt + 8, kv_dtype=kvd)
+            outs[on] = eng.forward(toks, kv, all_positions=True)
+            kv.close()
+        d = np.abs(outs[1] - outs[0])             # 16-bit logits of about 1 and the rounding of one layer's sums in two orders: two ulps; float32: layer 0's flips
+        assert d.max() <= (4e-3 if kvd == "float32" else 0.04) and np.sqrt((d ** 2).mean()) <= (2e-4 if kvd == "float32" else 4e-3), (d.max(), np.sqrt((d ** 2).mean()))
+    eng.close()
+
+
 @pytest.mark.parametrize("name", ["llama_bf16_gqa", "llama_f16", "qwen3_bf16"])
 def test_decode_swiglu_on_the_row_interleaved_gate_up_copy_is_bit_identical(tiny_dirs, name):
     """Decode steps of <= 16 rows stream a row-interleaved copy of the dense gate|up matrix (tile t = gate rows 8t..8t+7 then

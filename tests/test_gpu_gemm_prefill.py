@@ -72,6 +72,10 @@ def test_store_and_residual_match_oracle_and_the_register_staged_tile(act, kind,
     _assert_close(got[1][rows], want, act)
     for m in MODES:
         assert np.array_equal(got[m], got[0]), f"LDS-DMA tile (MI_GEMM_DMA={m}) differs from the register-staged tile"
+    # logits: the same values as float32
+    lg = torch.full((M + 3, N), 7.0, dtype=torch.float32, device="cuda")
+    _run(ol, xd, M, act, 1, epi=L.EPI_STORE_F32, out=lg, ldo=N)
+    assert np.array_equal(host(lg)[:M], got[1]) and np.all(host(lg)[M:] == 7.0)
     # residual epilogue: h += y, in place
     hres = {}
     for dma in MODES + (0,):
