@@ -1761,6 +1761,16 @@ int mi_engine_set_option(mi_engine* e, const char* key, int64_t value) {
   return fail(MI_ERR_NOTFOUND, "unknown option: " + k);
 }
 
+int mi_host_alloc(uint64_t bytes, void** out) {
+  if (!out || bytes == 0) return fail(MI_ERR_INVALID, "mi_host_alloc: null argument or no bytes");
+  if (hipHostMalloc(out, (size_t)bytes, hipHostMallocPortable) != hipSuccess) {
+    (void)hipGetLastError();               // (no error of a later launch)
+    return fail(MI_ERR_RUNTIME, "mi_host_alloc: out of pinned memory");
+  }
+  return MI_OK;
+}
+void mi_host_free(void* p) { if (p) hipHostFree(p); }
+
 int mi_engine_sync(mi_engine* e) {
   if (!e) return fail(MI_ERR_INVALID, "null engine");
   MI_HIP(hipSetDevice(e->device));

@@ -8,6 +8,7 @@ libmi355_decode.so; PyTorch is used only to hold host/device tensors on their wa
 from __future__ import annotations
 
 import ctypes as C
+import threading
 import weakref
 from typing import Dict, Iterable, Optional, Sequence, Tuple
 
@@ -44,6 +45,82 @@ def _tensor_info(t) -> Tuple[int, Tuple[int, ...], int, int, object]:
 
 def _i32(a) -> np.ndarray:
     return np.ascontiguousarray(np.asarray(a), dtype=np.int32)
+
+
+class _ResultPool:
+    """Pinned host memory behind the large arrays that ``forward`` returns: an array owns its block until it is dropped, then the block
+    serves the next one.  At most ``MAX_BYTES`` are out or kept at any time (a caller that collects more gets ordinary memory); what is
+    kept is given back when the last engine is closed.  One pool per process: blocks belong to no device or stream, and a block is
+    handed out again only when nobody can see its array any more."""
+
+    MIN_BYTES, MAX_BYTES = 1 << 18, 256 << 20        # below: a pageable copy is as quick
+
+    def __init__(self):
+        self._lock = threading.RLock()                # (re-entrant: a collection inside may drop an array)
+        self._free: Dict[int, list] = {}
+        self._bytes = 0                               # out and kept
+        self._engines = 0
+
+    def engine_opened(self) -> None:
+        with self._lock:
+            self._engines += 1
+
+    def engine_closed(self) -> None:
+        with self._lock:
+            self._engines -= 1
+            if self._engines == 0:
+                self._drop_free()
+
+    def _drop_free(self) -> None:
+        for size, blocks in self._free.items():
+            for p in blocks:
+                L.lib().mi_host_free(p)
+                self._bytes -= size
+        self._free.clear()
+
+    def empty(self, shape) -> np.ndarray:
+        """float32 array of this shape, contents undefined."""
+        n = 4 * int(np.prod(shape, dtype=np.int64))
+        if n < self.MIN_BYTES or n > self.MAX_BYTES:
+            return np.empty(shape, dtype=np.float32)
+        size = (n + (1 << 18) - 1) >> 18 << 18
+        with self._lock:
+            blocks = self._free.get(size)
+            if blocks:
+                p = blocks.pop()
+            else:
+                if self._bytes + size > self.MAX_BYTES:
+                    self._drop_free()
+                p = C.c_void_p()
+                if self._bytes + size > self.MAX_BYTES or L.lib().mi_host_alloc(size, C.byref(p)) != 0:
+                    return np.empty(shape, dtype=np.float32)
+                self._bytes += size
+        return np.asarray(_ResultBlock(self, p, size, tuple(shape)))
+
+    def give_back(self, p, size: int) -> None:
+        with self._lock:
+            if self._engines > 0:
+                self._free.setdefault(size, []).append(p)
+            else:
+                L.lib().mi_host_free(p)
+                self._bytes -= size
+
+
+class _ResultBlock:
+    """What an array of the pool keeps alive."""
+
+    def __init__(self, pool: _ResultPool, p, size: int, shape):
+        self._pool, self._p, self._size = pool, p, size
+        self.__array_interface__ = {"shape": shape, "typestr": "<f4", "data": (p.value, False), "version": 3}
+
+    def __del__(self):
+        try:
+            self._pool.give_back(self._p, self._size)
+        except Exception:                             # (interpreter shutdown)
+            pass
+
+
+_results = _ResultPool()
 
 
 class SampleArgs:
@@ -251,6 +328,7 @@ class Engine:
         self._h = C.c_void_p()
         self._kvs = weakref.WeakSet()
         L.check(L.lib().mi_engine_create(C.byref(d), device, C.byref(self._h)))
+        _results.engine_opened()
         self._finalized = False
 
     def _create_layers(self, config: dict, model_type: str, device: int, max_positions: Optional[int], act_dtype: str) -> None:
@@ -282,6 +360,7 @@ class Engine:
         self._kvs = weakref.WeakSet()
         self._finalized = False
         L.check(L.lib().mi_engine_create_layers(C.byref(d), arr, len(layers), device, C.byref(self._h)))
+        _results.engine_opened()
 
     def kv_block_bytes(self, block_tokens: int, kv_dtype: str = "model") -> int:
         """Bytes one block of a paged cache takes over all layers."""
@@ -375,7 +454,7 @@ class Engine:
         ptr = None
         if want_logits:
             V = self.desc.vocab_size
-            out = np.empty((B, Lq, V) if all_positions else (B, V), dtype=np.float32)
+            out = _results.empty((B, Lq, V) if all_positions else (B, V))
             ptr = out.ctypes.data_as(C.POINTER(C.c_float))
         L.check(L.lib().mi_forward(self._h, kv._h, tok.ctypes.data_as(C.POINTER(C.c_int32)), B, Lq, ptr,
                                    int(all_positions)))
@@ -451,7 +530,7 @@ class Engine:
         toks = np.ascontiguousarray(np.concatenate([_i32(t).reshape(-1) for t in token_lists]))
         offs = kv.offsets
         kv.ensure(max(offs[int(i)] + int(n) for i, n in zip(r, lens)))
-        out = np.empty((len(w), self.desc.vocab_size), dtype=np.float32)
+        out = _results.empty((len(w), self.desc.vocab_size))
         I32 = C.POINTER(C.c_int32)
         L.check(L.lib().mi_forward_segments(self._h, kv._h, r.ctypes.data_as(I32), lens.ctypes.data_as(I32), len(r),
                                             toks.ctypes.data_as(I32), w.ctypes.data_as(I32), len(w),
@@ -532,6 +611,7 @@ class Engine:
                 kv.close()
             L.lib().mi_engine_destroy(self._h)
             self._h = C.c_void_p()
+            _results.engine_closed()
 
     def __del__(self):
         try:

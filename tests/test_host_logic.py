@@ -153,3 +153,57 @@ def test_lru_caches(tiny):
     memo.put("a", 1); memo.put("b", 2); memo.peek("a"); memo.put("c", 3)
     assert memo.peek("b") is None and memo.peek("a") == 1 and memo.fetch("c", lambda: 9) == 3 and len(memo) == 2
     assert memo.fetch("d", lambda: 4) == 4 and memo.peek("a") is None
+
+
+def test_result_pool_hands_out_only_what_nobody_sees(monkeypatch):
+    """The pinned blocks behind forward()'s arrays: an array's block is not handed out again while the array (or a view of it) lives, the
+    total stays bounded with ordinary memory beyond it, and everything is given back with the last engine -- also what is dropped later."""
+    import ctypes as C
+
+    from mlx_parallm_amd import engine as E
+
+    live = {}
+
+    class Fake:
+        @staticmethod
+        def mi_host_alloc(n, out):
+            if Fake.full:
+                return -4
+            buf = C.create_string_buffer(n)
+            out._obj.value = C.addressof(buf)
+            live[C.addressof(buf)] = buf
+            return 0
+
+        @staticmethod
+        def mi_host_free(p):
+            del live[p.value]
+        full = False
+
+    monkeypatch.setattr(E.L, "lib", lambda: Fake)
+    monkeypatch.setattr(E._ResultPool, "MIN_BYTES", 1 << 10)
+    monkeypatch.setattr(E._ResultPool, "MAX_BYTES", 1 << 20)
+    pool = E._ResultPool()
+    pool.engine_opened()
+    assert len(live) == 0 and pool.empty((2, 100)).shape == (2, 100) and len(live) == 0          # small: ordinary memory
+    a, b = pool.empty((4, 1000)), pool.empty((4, 1000))
+    a[:], b[:] = 1.0, 2.0
+    at = {x.__array_interface__["data"][0] for x in (a, b)}
+    assert len(at) == 2 and len(live) == 2 and a.flags.writeable and a.dtype == np.float32
+    row = b[1]
+    del a, b
+    c = pool.empty((4, 1001))                                                                    # the same size class: a's block, not b's
+    assert c.__array_interface__["data"][0] in at and len(live) == 2
+    c[:] = 3.0
+    assert np.all(row == 2.0)
+    many = [pool.empty((4, 1000)) for _ in range(10)]
+    assert len(live) == 4 and pool._bytes <= 1 << 20                                             # 4 x 256 KiB, the rest ordinary
+    del many
+    big = pool.empty((200, 1000))                                                                # another size: what is kept makes room
+    assert big.shape == (200, 1000) and pool._bytes <= 1 << 20
+    Fake.full = True
+    assert pool.empty((4, 4000)).shape == (4, 4000)
+    del big
+    pool.engine_closed()
+    assert len(live) == 2                                                                        # what c and row still show
+    del c, row
+    assert len(live) == 0 and pool._bytes == 0
