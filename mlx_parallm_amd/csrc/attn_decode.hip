@@ -512,11 +512,13 @@ __device__ __forceinline__ void attn_decode_mfma_body(const AttnDecodeCall& c, u
   // removes a dependent global load from the head of the chain
   const int kb = c.n_host_off > 0 ? c.host_row[b] : (s.rows ? s.rows[b] : b);   // cache row of batch entry b
   const int pos = c.n_host_off > 0 ? c.host_off[b] : c.offsets[kb];
-  // the pos cached keys are cut evenly over the splits (a 1024-key context = 4 x 256 = one round each); the
+  // the pos cached keys are cut evenly over the row's splits (a 1024-key context = 4 x 256 = one round each); the
   // new key is merged by the last split from registers / LDS
-  const int chunk = (pos + c.nsplit - 1) / c.nsplit;
+  const int nsplit = decode_row_splits(c.nsplit, pos);
+  if (split >= nsplit) return;                   // (the whole workgroup: a row shorter than the call's longest)
+  const int chunk = (pos + nsplit - 1) / nsplit;
   const int s0 = split * chunk;
-  const bool owner = split == c.nsplit - 1;
+  const bool owner = split == nsplit - 1;
   const int nq = s.Hq * D;
   const T* row = (const T*)c.qkv + (size_t)b * (nq + 2 * s.Hkv * D);
 
@@ -532,7 +534,6 @@ __device__ __forceinline__ void attn_decode_mfma_body(const AttnDecodeCall& c, u
   T* vc = (T*)c.vcache;
   const int send = min(s0 + chunk, pos);         // cached keys of this split: [s0, send)
 
-  // ---- the K fragments and V rows of the first round go out before anything else
   u32x4 kf[T32 ? 1 : 2][T32 ? 1 : KK], vrow[T32 ? 1 : NV];
   f32x4 kf32[F32 ? NP : 1], vv32[F32 ? 4 : 1][F32 ? NH : 1];
   f32x4 kraw[F32S ? 2 : 1][F32S ? KK : 1][2], vraw[F32S ? NVS : 1];   // F32S: the float32 bits of the 16-bit kernel's fragments / rows
@@ -591,9 +592,6 @@ __device__ __forceinline__ void attn_decode_mfma_body(const AttnDecodeCall& c, u
       }
     }
   };
-  issue_k(s0);
-  issue_v(s0);
-
   // ---- prologue, spread over the workgroup: lane group (wave, gq) = vector vi owns ONE of the G query
   // heads (vi < G), the new key (vi == G) or the new value (vi == G + 1): raw load, RMSNorm, RoPE,
   // result to LDS.  One code path for every group (pointers are selected, nothing branches), so a wave
@@ -614,6 +612,12 @@ __device__ __forceinline__ void attn_decode_mfma_body(const AttnDecodeCall& c, u
   }
   uint32_t r0[NW32];
   if constexpr (NORM) load_raw<NW32>((const T*)(is_k ? c.k_norm_w : c.q_norm_w) + li * EPL, r0);
+  // ---- the K fragments and V rows of the first round behind them: a wave's loads return in the order of their issue, so with the
+  // rows in front (as this kernel had it) q waited for the whole first round to arrive from HBM, and the norm, the rotation and the
+  // barrier stood behind that instead of under it
+  __builtin_amdgcn_sched_barrier(0);
+  issue_k(s0);
+  issue_v(s0);
   __builtin_amdgcn_sched_barrier(0);
   after_loads();                                 // every global load the prologue waits for is in the queue ahead of this
   __builtin_amdgcn_sched_barrier(0);
@@ -724,7 +728,7 @@ __device__ __forceinline__ void attn_decode_mfma_body(const AttnDecodeCall& c, u
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) accO[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   if constexpr (F32) {
-    for (int base = s0; base < send; base += KPW * NWV) {       // uniform trip count; 16 keys per wave and round
+    for (int base = s0; base + KPW * wave < send; base += KPW * NWV) {       // 16 keys per wave and round; a wave leaves when its keys are done
       f32x4 sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < NP; ++i)
@@ -763,7 +767,7 @@ __device__ __forceinline__ void attn_decode_mfma_body(const AttnDecodeCall& c, u
       __builtin_amdgcn_sched_barrier(0);
     }
   } else if constexpr (F32S) {
-    for (int base = s0; base < send; base += 32 * NWV) {      // uniform trip count; 32 keys per wave and round
+    for (int base = s0; base + 32 * wave < send; base += 32 * NWV) {      // 32 keys per wave and round; a wave leaves when its keys are done
       f32x4 sc[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
@@ -841,7 +845,7 @@ __device__ __forceinline__ void attn_decode_mfma_body(const AttnDecodeCall& c, u
       }
     }
   } else {
-  for (int base = s0; base < send; base += 32 * NWV) {        // uniform trip count
+  for (int base = s0; base + 32 * wave < send; base += 32 * NWV) {        // a wave leaves when its keys are done
     // S^T tiles: rows = keys, columns = heads
     f32x4 sc[2];
 #pragma unroll
@@ -939,7 +943,7 @@ __device__ __forceinline__ void attn_decode_mfma_body(const AttnDecodeCall& c, u
       O = fmaf(st_o[(w * G + g) * D + d], cw, O);
     }
     const int h = kh * G + g;
-    if (c.nsplit == 1) {
+    if (nsplit == 1) {
       store_out<T>(&out[(size_t)h * D + d], store_act<T>(O / L, c.rnd_out), WT);
     } else {
       float* pp = c.partial + (((size_t)b * s.Hq + h) * c.nsplit + split) * (D + 2);
@@ -950,12 +954,12 @@ __device__ __forceinline__ void attn_decode_mfma_body(const AttnDecodeCall& c, u
       }
     }
   }
-  if (c.nsplit == 1 || c.counters == nullptr) return;
+  if (nsplit == 1 || c.counters == nullptr) return;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (tid == 0) {
     const int ticket = __hip_atomic_fetch_add(&c.counters[bh], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const int last = ticket == c.nsplit - 1;
+    const int last = ticket == nsplit - 1;
     if (last) __hip_atomic_store(&c.counters[bh], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     is_last_sh = last;
   }
@@ -964,7 +968,7 @@ __device__ __forceinline__ void attn_decode_mfma_body(const AttnDecodeCall& c, u
   for (int idx = tid; idx < G * D; idx += NTH) {
     const int g = idx / D, d = idx % D, h = kh * G + g;
     const float* pp = c.partial + ((size_t)b * s.Hq + h) * c.nsplit * (D + 2);
-    store_out<T>(&out[(size_t)h * D + d], store_act<T>(combine_splits<D>(pp, c.nsplit, d), c.rnd_out), WT);
+    store_out<T>(&out[(size_t)h * D + d], store_act<T>(combine_splits<D>(pp, nsplit, d), c.rnd_out), WT);
   }
 }
 

@@ -14,6 +14,7 @@ static thread_local std::string g_err;
 void set_error(const std::string& m) { g_err = m; }
 int fail(int code, const std::string& m) { g_err = m; return code; }
 
+int gemv_cu_count();      // gemv_mfma.hip
 int launch_gemv_v1(const LinearW& W, const GemvCall& c, hipStream_t st);
 int launch_gemv_mfma(const LinearW& W, const GemvCall& c, hipStream_t st);
 bool gemv_mfma_supported(const LinearW& W, const GemvCall& c);
@@ -659,27 +660,18 @@ size_t kv_layer_elems(const mi_kv* kv, const mi_model_desc& d) {
                    : (size_t)kv->B * d.num_kv_heads * kv->cap * d.head_dim;
 }
 
+// Splits of the decode attention: one workgroup per CU (8 waves, 84 KiB of LDS: a second one does not fit, so a launch of more runs in
+// rounds -- 8 rows x 8 heads, 1024 float32 keys: 4 splits 20 us, 5 splits 30; 8 rows at 8192 16-bit keys: 4 splits 43 us, 5 / 8 / 9 57 /
+// 48 / 58).  Rows shorter than the longest take fewer splits (decode_row_splits), so a call counts as its keys over the longest row's.
 int choose_nsplit(const mi_kv* kv, int B, int Hkv, int L, const int32_t* rows = nullptr) {
   if (L != 1) return 1;
-  int mx = 0;
-  for (int b = 0; b < B; ++b) mx = std::max(mx, kv->h_off[rows ? rows[b] : b] + 1);
-  int ns = (256 + B * Hkv - 1) / (B * Hkv);
-  ns = std::min(ns, std::max(1, mx / 64));
-  // long contexts: at most four 256-key rounds per workgroup -- eight when the batch alone fills the CUs (every extra
-  // workgroup then costs a prologue and a merge on a CU that is already busy)
-  const int per_wg = B * Hkv >= 256 ? 2048 : 1024;
-  ns = std::max(ns, (mx + per_wg - 1) / per_wg);
-  ns = std::max(1, std::min(ns, 16));
-  // a workgroup walks its keys in rounds of 256 (float32 caches: 128): the smallest split count with the SAME number of
-  // rounds has fewer workgroups to start and fewer partials to merge (KV length 1100, B = 8: 4 -> 3 splits, float32-KV
-  // 1968 -> 1995 tok/s, bf16 2238 -> 2252; more splits are slower: 5 / 6 / 8 splits 2175 / 2173 / 2155)
-  const int rk = kv->dtype == MI_F32 ? 128 : 256;
-  auto rounds = [&](int n) { return ((mx - 1 + n - 1) / n + rk - 1) / rk; };     // (the cached keys; the new one is merged from registers)
-  const int r0 = rounds(ns);
-  while (ns > 1 && rounds(ns - 1) == r0) --ns;
+  int mx = 1;
+  long sum = 0;
+  for (int b = 0; b < B; ++b) { const int k = std::max(1, kv->h_off[rows ? rows[b] : b]); mx = std::max(mx, k); sum += k; }
+  const int alike = (int)((sum + mx - 1) / mx);
   static const int ns_env = getenv("MI_ATTN_NSPLIT") ? atoi(getenv("MI_ATTN_NSPLIT")) : 0;   // A/B
-  if (ns_env > 0) ns = std::min(ns_env, std::max(1, mx / 64));
-  return std::max(1, std::min(ns, 16));
+  const int fill = ns_env > 0 ? ns_env : gemv_cu_count() / (Hkv * alike);
+  return decode_row_splits(std::min(fill, 16), mx);
 }
 
 // prefill attention (L > 1): the keys split over workgroups where the query tiles alone leave the chip idle

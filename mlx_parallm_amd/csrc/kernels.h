@@ -249,6 +249,15 @@ size_t attention_prefill_part_floats(const AttnShape& s, int slices);
 int attention_prefill_tiles(const AttnShape& s);
 int launch_attention_prefill(const AttnCall& c, hipStream_t st);
 
+// Decode attention: over how many of at most `most` workgroups a row's `keys` cached keys are split (device: per row; host: the longest
+// row's).  A split costs its publication and its share of the join, so a workgroup gets a full round of 256 keys where four splits
+// do not suffice; below that four splits of 96 keys and more still beat fewer (16-bit caches, rocprof: 330 keys, 1 row x 8 heads
+// 9.3 / 9.1 / 8.6 / 8.3 us in 1 / 2 / 3 / 4 splits, 8.7 in 5; 2048 keys 12.0 / 10.6 / 11.3 in 4 / 8 / 16).
+__host__ __device__ inline int decode_row_splits(int most, int keys) {
+  const int four = (keys + 95) / 96 < 4 ? (keys + 95) / 96 : 4, full = keys / 256;
+  const int want = four > full ? four : full;
+  return want < 1 || most < 1 ? 1 : want < most ? want : most;
+}
 // fused decode step (L == 1): q/k norm + RoPE + KV append + split-KV attention + combine
 struct AttnDecodeCall {
   AttnShape s;             // s.rnd = logical rounding of q / k after norm and RoPE

@@ -427,6 +427,36 @@ def test_fused_decode_attention(act, Hq, Hkv, D, qk_norm, variant):
             assert close_frac(got, want, act, atol=2e-3) <= 0.02, (nsplit, close_frac(got, want, act, atol=2e-3))
 
 
+@pytest.mark.parametrize("act", ["bfloat16", "float32"])
+@pytest.mark.parametrize("Hq,Hkv", [(4, 1), (10, 2)])
+def test_decode_attention_rows_take_their_own_number_of_splits(act, Hq, Hkv):
+    """Rows around the edges of decode_row_splits (96 keys a split up to four, 256 beyond) and of a wave's share of a round, in a call
+    of 16 splits: against the same call in one.  Float32 sums in another order, rounded to the cache's type once at the end: 2^-20
+    relative to the values' scale for float32, one ulp (bfloat16: at most 2^-7 of the value) for the few 16-bit outputs at a rounding boundary."""
+    D, offs = 128, [1, 95, 96, 97, 192, 193, 288, 289, 384, 385, 1023, 1279, 1280, 1281, 2000, 4095]
+    B, cap = len(offs), 4100
+    cos, sin, _, _ = _rope_setup(D, cap + 1)
+    s = attn_shape(B, 1, Hq, Hkv, D, act, act, 0, cap)
+    kc, vc = (dev(RNG.standard_normal((B, Hkv, cap, D)).astype(np.float32), act) for _ in range(2))
+    qkv, off = dev(RNG.standard_normal((B, (Hq + 2 * Hkv) * D)).astype(np.float32), act), dev_i32(offs)
+    got = {}
+    for nsplit in (1, 16):
+        out = torch.zeros((B, Hq * D), dtype=qkv.dtype, device="cuda")
+        part = torch.zeros((B * Hq * nsplit * (D + 2),), dtype=torch.float32, device="cuda")
+        ctr = torch.zeros((B * Hkv,), dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        for _ in range(2):                                 # (the second call finds the tickets that the first gave back)
+            L.check(L.lib().mi_op_attention_decode(C.byref(s), ptr(qkv), ptr(kc), ptr(vc), ptr(off), None, None, 1e-6, ptr(cos), ptr(sin), ptr(out),
+                                                   float(D ** -0.5), 0, nsplit, ptr(part), ptr(ctr), 0, 1, None))
+        assert not ctr.cpu().numpy().any()
+        got[nsplit] = host(out)
+    d = np.abs(got[1] - got[16])
+    if act == "float32":
+        assert d.max() <= 4e-6, d.max()                    # |values| <= 4
+    else:
+        assert (d <= 2.0 ** -7 * np.maximum(np.abs(got[1]), 2.0 ** -7)).all() and (d > 0).mean() <= 0.02, (d.max(), (d > 0).mean())
+
+
 def _run_sampler(lg, temp, top_p, u, k=0):
     B, V = lg.shape
     t = dev(lg)
