@@ -367,7 +367,7 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
       // dense bf16 weights: two terms (16+ mantissa bits of x, two walks of W; option "prefill_x_terms"); int4 / [hi | lo]
       // matrices keep the exact three (their own pair needs the 3 : 2 walk)
       // The rounded call of layer 0: its input is a bf16 value, i.e. one term (8 x 1024 rows of Mistral-7B: 256 launches of the
-      // streaming kernel at 32 rows each, 4.6 ms, against 0.4 ms here).
+      // streaming kernel at 32 rows each, 4.6 ms, against 0.9 ms here).
       // (Logits keep the three terms that they had on the streaming kernel.)
       const int terms = c.rnd == RND_BF16 ? 1 : (e->opt_prefill_x_terms == 2 && f.W.wk == WK_BF16 && c.kx == 0 && c.rnd == RND_NONE && c.epi != EPI_STORE_F32) ? 2 : 3;
       MI_TRY(launch_split3_rows(c.x, c.ldx, c.pro == PRO_NORM ? c.norm_w : nullptr, c.eps, e->xs, (int)rows, KT, e->stream, terms, c.rnd));

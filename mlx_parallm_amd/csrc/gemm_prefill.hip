@@ -96,7 +96,12 @@ __device__ __forceinline__ bool group_of_tile(GemmParams& p, int bm, int n0, int
 }
 
 // GROUPED: blockIdx.x = tile of the device-resident table; every group of rows has its own matrix (GroupedGemm, kernels.h)
-template <typename AT, bool SWIGLU, bool GROUPED = false>
+// FOLD: the accumulators are added to a second set every three K steps, i.e. no float32 chain is longer than six MFMAs + K / 192
+// additions.  For outputs that are ROUNDED to 16 bits where an exact computation rounds too (layer 0 of the float32-cache mode): the
+// longer the chain, the more values round the other way (mean |logprob - exact| of three recorded float32-cache cases: streaming
+// kernel 1.64 / 1.27 / 2.08e-4, the 256 x 256 tile's one chain over K 2.02 / 1.74 / 2.53e-4, here 1.52 / 1.04 / 1.98e-4).  8 x 1024 rows
+// of Mistral-7B's q|k|v: 0.9 ms against 0.4 on the 256 x 256 tile and 4.6 streaming.
+template <typename AT, bool SWIGLU, bool GROUPED = false, bool FOLD = false>
 __global__ __launch_bounds__(256) void gemm_tile_kernel(GemmParams p) {
   __shared__ __attribute__((aligned(16))) AT As[2][BM][LDA];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -197,10 +202,27 @@ __global__ __launch_bounds__(256) void gemm_tile_kernel(GemmParams p) {
       __syncthreads();
     }
   };
+  f32x4 tot[FOLD ? 4 : 1][FOLD ? 4 : 1];
+#pragma unroll
+  for (int i = 0; i < (FOLD ? 4 : 1); ++i)
+#pragma unroll
+    for (int j = 0; j < (FOLD ? 4 : 1); ++j) tot[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int ks = ks0; ks < nk; ks += 3) {
     step(ks, std::integral_constant<int, 0>{});
     if (ks + 1 < nk) step(ks + 1, std::integral_constant<int, 1>{});
     if (ks + 2 < nk) step(ks + 2, std::integral_constant<int, 2>{});
+    if constexpr (FOLD) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) { tot[i][j] += acc[i][j]; acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+    }
+  }
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = tot[i][j];
   }
 
   if constexpr (!SWIGLU) {
@@ -1268,7 +1290,8 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
   int ks256 = 1;
   const char* sk_env = getenv("MI_GEMM_DMA_SPLITK");     // (read per call: the tests switch it)
   const bool splitk256 = sk_env == nullptr || atoi(sk_env) != 0;
-  if (rows >= 256 && !small_only && dma && splitk256 && !sw && splitk_ws != nullptr && W.N % 4 == 0) {
+  const bool fold = x32 && c.rnd != RND_NONE;           // (plain stores: gemm_prefill_supported)
+  if (rows >= 256 && !small_only && !fold && dma && splitk256 && !sw && splitk_ws != nullptr && W.N % 4 == 0) {
     // one 128-KiB workgroup per CU: the launch runs in rounds of n_cu workgroups.  Pick the split whose last round is
     // fullest, charging 2 % per extra slice for its partial tile and its share of the reduce (q|k|v at 1024 rows: 96
     // tiles -> 5 slices = 480 workgroups, 1.9 rounds; o_proj: 64 tiles -> 4 slices = one full round)
@@ -1281,7 +1304,7 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
       if (score > best + 1e-9) { best = score; ks256 = ks; }
     }
   }
-  if (rows >= 256 && !small_only && (blocks256 >= 192 || ks256 > 1)) {  // both operands through LDS (256 x 256 tile)
+  if (rows >= 256 && !small_only && !fold && (blocks256 >= 192 || ks256 > 1)) {  // both operands through LDS (256 x 256 tile)
     const int bn = sw ? 128 : BN2;
     dim3 grid2(((int)rows + BM2 - 1) / BM2, (ncols + bn - 1) / bn), block2(512);
     if (ks256 > 1) { grid2.z = ks256; p.ksplit = ks256; p.ws = (float*)splitk_ws; }
@@ -1333,7 +1356,8 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
     while (ks > 1 && (size_t)ks * rows * W.N * sizeof(float) > splitk_cap) --ks;
     if (ks > 1) { p.ksplit = ks; p.ws = (float*)splitk_ws; grid.z = ks; }
   }
-  if (c.act == MI_BF16 || x32) {
+  if (fold) hipLaunchKernelGGL((gemm_tile_kernel<bf16, false, false, true>), grid, block, 0, st, p);
+  else if (c.act == MI_BF16 || x32) {
     if (sw) hipLaunchKernelGGL((gemm_tile_kernel<bf16, true>), grid, block, 0, st, p);
     else hipLaunchKernelGGL((gemm_tile_kernel<bf16, false>), grid, block, 0, st, p);
   } else {
