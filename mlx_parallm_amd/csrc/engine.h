@@ -164,7 +164,7 @@ struct mi_engine {
   int opt_attn_mfma = 1;                 // decode attention on the matrix cores where the shape allows
   int opt_tile_weights = 1;
   int opt_prefill_gemm = 1;
-  int opt_skinny_gemm = 1;      // decode steps of 9..128 rows (int4 / int8: 1..128): the split-K weight-streaming GEMM (gemm_skinny.hip)
+  int opt_skinny_gemm = 1;      // decode steps of 9..128 rows (int4 / int8: 1..128): the split-K weight-streaming GEMM (gemm_skinny.hip; int4 / int8 up to 8 rows: gemv_reg.hip)
   int cur_L = 0;                // tokens per sequence of the forward pass being enqueued
   // RMSNorm hand-over between gemm_skinny launches (GemvCall::sq_out / sq_in): the residual linear in front of a norm
   // leaves the rows' sums of squares, the normalised linear behind it uses them instead of an rmsnorm launch

@@ -297,6 +297,11 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
   // (Mistral-7B bf16, KV 512: 96 rows 7.18 vs 7.14 ms / step, 128 rows 8.71 vs 7.96)
   static const int decode_max_env = getenv("MI_SKINNY_DECODE_MAX") ? atoi(getenv("MI_SKINNY_DECODE_MAX")) : 0;   // A/B
   const size_t decode_max = decode_max_env > 0 ? (size_t)decode_max_env : (quant ? 128 : 96);
+  if (e->opt_skinny_gemm && gemv_reg_supported(f.W, c, rows)) {
+    // quantised weights, at most 8 rows (gemv_reg.hip): the norm is its own, nothing is handed over
+    Prof pr(e, prof);
+    return launch_gemv_reg(f.W, c, rows, e->stream);
+  }
   if (e->opt_skinny_gemm && ((e->cur_L == 1 && rows <= decode_max) || rows <= short_rows) && gemm_skinny_supported(f.W, c, rows)) {
     // the decode step of a batch of 9..128 sequences (int4 / int8 weights: any batch up to 128): W is streamed once, K split over workgroups (gemm_skinny.hip).
     // Also a prefill of up to 128 rows in all (a short prompt, a few short prompts): at that size the op is a weight

@@ -974,7 +974,7 @@ int launch_k(const SkinnyParams& p, int grid, hipStream_t st) {
 template <typename AT, int QB, bool SWIGLU>
 int launch_mt(const SkinnyParams& p, int mt, int grid, hipStream_t st) {
   switch (mt) {
-    case 1: return launch_k<AT, QB, 1, SWIGLU>(p, grid, st);    // int8: every decode step; 16-bit / int4: 9..16 rows
+    case 1: return launch_k<AT, QB, 1, SWIGLU>(p, grid, st);    // 9..16 rows; below that the quantised calls that gemv_reg.hip does not take
     case 2: return launch_k<AT, QB, 2, SWIGLU>(p, grid, st);
     case 3: return launch_k<AT, QB, 3, SWIGLU>(p, grid, st);
     case 4: return launch_k<AT, QB, 4, SWIGLU>(p, grid, st);
@@ -1017,9 +1017,10 @@ bool gemm_skinny_supported(const LinearW& W, const GemvCall& c, size_t rows) {
   if (c.rnd != RND_NONE) return false;
   if (c.out32 && (wk_is_quant(W.wk) || W.lora_b[0] || W.lora_b[1] || (c.epi != EPI_STORE && c.epi != EPI_RESID))) return false;
   const bool q8 = ((W.wk == WK_Q8_BF16 && c.act == MI_BF16) || (W.wk == WK_Q8_F16 && c.act == MI_F16)) && W.group == 64 &&
-                  W.K % 64 == 0;                         // int8 has no M <= 16 kernel of its own: every decode step runs here
+                  W.K % 64 == 0;                         // (up to 8 rows gemv_reg.hip is asked first)
   // int4: this kernel also wins below 9 rows, on every linear (M = 8, Mistral-7B shapes, us: q|k|v 9.2 vs 12.4, o 9.8 vs
-  // 9.8, gate|up 19.0 vs 24.3, down 14.8 vs 23.7, lm_head 17.7 vs 24.5 -- more than the two RMSNorm launches it adds)
+  // 9.8, gate|up 19.0 vs 24.3, down 14.8 vs 23.7, lm_head 17.7 vs 24.5 -- more than the two RMSNorm launches it adds); it serves
+  // those that gemv_reg.hip does not take (LoRA, K beyond its registers with a norm in front)
   static const bool q4_small = getenv("MI_SKINNY_Q4_MIN_ROWS") == nullptr;   // A/B: set = hand-over at skinny_min_rows() as for 16-bit
   if (rows < 1 || rows > 128) return false;
   if (wk_is_quant(W.wk) && !q8 && rows > (skinny_slabs_on() ? 128u : 96u)) return false;   // (the 128-row int4 SwiGLU instantiation would spill registers; as 32-row slabs it runs)

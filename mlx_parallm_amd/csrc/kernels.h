@@ -118,6 +118,10 @@ int launch_dequant_q4_hilo(const LinearW& src, void* dst, hipStream_t st);
 int launch_rmsnorm_rows(const void* x, int ldx, const void* w, void* out, int ldo, int rows, int H, float eps, int act,
                         hipStream_t st, bool block_per_row = false, int rnd = 0);
 
+// int4 / int8 weights, at most 8 rows, activations in registers (gemv_reg.hip); applies the RMSNorm of c.pro = PRO_NORM itself
+bool gemv_reg_supported(const LinearW& W, const GemvCall& c, size_t rows);
+int launch_gemv_reg(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st);
+
 // 9..64 rows, int8 weights 1..64 (decode steps of larger batches): weight-streaming split-K GEMM (gemm_skinny.hip).
 // c.pro must be PRO_NONE; `ws` >= gemm_skinny_ws_bytes(), `ctr` >= gemm_skinny_groups() words that are zero between
 // launches (the kernel leaves them zero); ksplit = 0 lets the cost model choose.

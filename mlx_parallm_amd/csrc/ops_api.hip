@@ -149,6 +149,15 @@ int mi_op_gemm_prefill(const mi_op_linear* w, const mi_op_gemv_args* a, int iter
   return rc != MI_OK ? rc : rc2;
 }
 
+int mi_op_gemv_reg(const mi_op_linear* w, const mi_op_gemv_args* a) {
+  if (!w || !a) return fail(MI_ERR_INVALID, "null argument");
+  MI_TRY(ready());
+  const GemvCall c = to_call(a);
+  if (c.M < 1) return fail(MI_ERR_INVALID, "mi_op_gemv_reg: M out of range");
+  MI_TRY(launch_gemv_reg(to_linear(w), c, (size_t)c.M, nullptr));
+  return finish();
+}
+
 int mi_op_gemv_uses_mfma(const mi_op_linear* w, const mi_op_gemv_args* a) {
   if (!w || !a) return 0;
   return gemv_mfma_supported(to_linear(w), to_call(a)) ? 1 : 0;

@@ -132,6 +132,14 @@ def gemm_prefill(ol: L.OpLinear, x, M, act, *, epi=0, out=None, ldo=0, resid=Non
     return ms.value if iters >= 1 else None
 
 
+def gemv_reg(ol: L.OpLinear, x, M, act, *, epi=0, out=None, ldo=0, resid=None, pair_offset=0, norm_w=None, eps=1e-5, ldx=None):
+    """gemv_reg.hip on its own (decode linears of at most 8 rows on quantised weights)."""
+    a = gemv_args(x, M, act, epi=epi, out=out, ldo=ldo, resid=resid, pair_offset=pair_offset, ldx=ldx, norm_w=norm_w, eps=eps,
+                  pro=L.PRO_NORM if norm_w is not None else L.PRO_NONE)
+    torch.cuda.synchronize()
+    L.check(L.lib().mi_op_gemv_reg(C.byref(ol), C.byref(a)))
+
+
 def serve_and_compare(model_dir, scheduler, oracle, cfg, greedy):
     """``python -m mlx_parallm_amd.cli`` on a checkpoint of this design: concurrent completions of unequal prompts are the plain
     implementation's greedy tokens, a streamed chat ends."""

@@ -1,0 +1,82 @@
+"""Kernel-level parity (-m gpu) of gemv_reg.hip -- decode linears of at most 8 rows on int4 / int8 weights -- against the oracle's
+matmul, through mi_op_gemv_reg (include/mi355_ops.h).  Tolerances as in test_gpu_kernels.py."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import ref_model
+from oracle.numerics import matmul_nt, round_to
+
+pytestmark = pytest.mark.gpu
+
+from mlx_parallm_amd import _lib as L  # noqa: E402
+from gpu_helpers import dev, gemv_reg, host  # noqa: E402
+from test_gpu_kernels import _assert_close  # noqa: E402
+from test_gpu_skinny import KINDS, _weight  # noqa: E402
+
+QUANT = [k for k in KINDS if k[1].startswith("q")]
+
+
+# K in blocks of 128 (int4): fewer than the 8 waves (two of them, one wave with work), not a multiple of 8, each register size's last
+# K and the first of the next, the register path's last K and the first beyond, the long path's steps, its last K
+@pytest.mark.parametrize("act,kind", QUANT)
+@pytest.mark.parametrize("M,N,K", [(1, 16, 128), (8, 80, 256), (3, 64, 1152), (5, 48, 2048), (8, 32, 2176), (7, 32, 4096), (2, 32, 4224),
+                                   (8, 48, 5120), (8, 32, 5248), (6, 48, 8192), (4, 16, 11264), (8, 16, 14336), (1, 32, 17408),
+                                   (8, 16 * 515, 256)])      # (more tiles than two rounds of workgroups)
+def test_matches_oracle(act, kind, M, N, K):
+    if kind.startswith("q8") and K > 5120:
+        pytest.skip("int8: K in registers only")
+    rng = np.random.default_rng(M * 1000003 + N * 1009 + K)
+    ol, wdense, keep = _weight(kind, N, K, rng)
+    x = round_to(rng.standard_normal((M, K)).astype(np.float32), act)
+    h = round_to(rng.standard_normal((M, N)).astype(np.float32) * 4.0, act)
+    xd, hd = dev(np.concatenate([x, np.full((1, K), np.nan, np.float32)]), act), dev(np.concatenate([h, h[:1]]), act)
+    y = round_to(matmul_nt(x, wdense), act)
+    outs = []
+    for _ in range(2):
+        out = torch.full((M + 1, N), 7.0, dtype=xd.dtype, device="cuda")
+        gemv_reg(ol, xd, M, act, epi=L.EPI_STORE, out=out, ldo=N)
+        outs.append(host(out))
+    assert np.array_equal(outs[0], outs[1]) and np.all(outs[0][M:] == 7.0)
+    _assert_close(outs[0][:M], y, act)
+    out = torch.full((M + 1, N), 7.0, dtype=torch.float32, device="cuda")
+    gemv_reg(ol, xd, M, act, epi=L.EPI_STORE_F32, out=out, ldo=N)
+    assert np.array_equal(host(out), outs[0])
+    gemv_reg(ol, xd, M, act, epi=L.EPI_RESID, resid=hd, ldo=N)
+    got = host(hd)
+    assert np.array_equal(got[:M], round_to(h + outs[0][:M], act)) and np.array_equal(got[M:], h[:1])
+
+
+@pytest.mark.parametrize("act,kind", QUANT)
+@pytest.mark.parametrize("M,N,K", [(1, 16, 128), (8, 80, 1152), (5, 4128, 2048), (3, 32, 4096), (8, 48, 5120)])
+def test_norm_and_swiglu(act, kind, M, N, K):
+    rng = np.random.default_rng(M * 1000003 + N * 1009 + K + 1)
+    ol, wdense, keep = _weight(kind, 2 * N, K, rng)
+    x = round_to(rng.standard_normal((M, K)).astype(np.float32) * 0.5, act)
+    nw = round_to(1.0 + 0.1 * rng.standard_normal(K).astype(np.float32), act)
+    xd, nwd = dev(x, act), dev(nw, act)
+    xn = ref_model.rms_norm(x, act, nw, act, 1e-5)[0]
+    y = round_to(matmul_nt(xn, wdense), act)
+    out = torch.zeros((M, 2 * N), dtype=torch.float32, device="cuda")
+    gemv_reg(ol, xd, M, act, epi=L.EPI_STORE_F32, out=out, ldo=2 * N, norm_w=nwd)
+    _assert_close(host(out), y, act)
+    if kind.startswith("q8"):
+        return                                          # (int8 SwiGLU and normed 16-bit stores: gemm_skinny.hip)
+    out2 = torch.zeros((M, 2 * N), dtype=xd.dtype, device="cuda")
+    gemv_reg(ol, xd, M, act, epi=L.EPI_STORE, out=out2, ldo=2 * N, norm_w=nwd)
+    assert np.array_equal(host(out2), host(out))
+    sig = round_to(1.0 / (1.0 + np.exp(-y[:, :N].astype(np.float64))), act)
+    out = torch.zeros((M, N), dtype=xd.dtype, device="cuda")
+    gemv_reg(ol, xd, M, act, epi=L.EPI_SWIGLU, out=out, ldo=N, pair_offset=N, norm_w=nwd)
+    _assert_close(host(out), round_to(round_to(y[:, :N] * sig, act) * y[:, N:], act), act, scale=4.0)
+
+
+@pytest.mark.parametrize("kind,M,K,epi,norm", [("q4_bf16", 9, 256, L.EPI_STORE, False), ("q4_bf16", 8, 17536, L.EPI_STORE, False),
+                                               ("q4_bf16", 8, 5248, L.EPI_STORE, True), ("q4_bf16", 8, 256, L.EPI_SWIGLU, False),
+                                               ("q8_bf16", 8, 5248, L.EPI_STORE, False), ("q8_bf16", 8, 256, L.EPI_STORE, True)])
+def test_refuses_what_it_does_not_take(kind, M, K, epi, norm):
+    ol, _, keep = _weight(kind, 32, K)
+    xd = torch.zeros((M, K), dtype=torch.bfloat16, device="cuda")
+    out = torch.zeros((M, 32), dtype=torch.bfloat16, device="cuda")
+    with pytest.raises(Exception, match="gemv_reg"):
+        gemv_reg(ol, xd, M, "bfloat16", epi=epi, out=out, ldo=32, pair_offset=16, norm_w=xd[0] if norm else None)
