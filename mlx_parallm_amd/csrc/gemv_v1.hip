@@ -296,11 +296,23 @@ __global__ __launch_bounds__(NTHR) void gemv_v1_kernel(GemvParams p) {
   }
 }
 
+// the value of lane i ^ 4 (inside groups of 8: row_ror:4 for the upper four lanes, row_ror:12 for the lower)
+__device__ __forceinline__ float xor4(float v) {
+  const float up = __builtin_amdgcn_update_dpp(0.f, v, 0x124, 0xf, 0xa, false);
+  return __builtin_amdgcn_update_dpp(up, v, 0x12C, 0xf, 0x5, false);
+}
+__device__ __forceinline__ float xor2_xor1(float v) {
+  v += __builtin_amdgcn_update_dpp(0.f, v, 0x4E, 0xf, 0xf, false);    // quad_perm:[2,3,0,1]
+  v += __builtin_amdgcn_update_dpp(0.f, v, 0xB1, 0xf, 0xf, false);    // quad_perm:[1,0,3,2]
+  return v;
+}
+
 // Rows of at most 512 inputs.  In gemv_v1_kernel a wave spreads one row over its 64 lanes and every workgroup stages (and zero-fills)
 // a 2048-wide image of x: at 64 inputs 8 of 64 lanes have work.  Here LG lanes hold a row (LG = 8, 16, 64), a wave takes 64 / LG of
 // them at a time, and a lane keeps its 8 columns of x for every batch row in registers -- normed there, so nothing goes through LDS
 // and no barrier stands in front of the weights.  int4, 64 inputs, 2 rows, float32 activations: 151936 outputs 74 -> 12 us, 192 outputs
-// 9.8 -> 4.7 us (rocprof; an empty kernel is 4).
+// 9.8 -> 5.1 us (rocprof; an empty kernel is 4).  All sums are taken in gemv_v1_kernel's order: the results are the same bit for bit,
+// whichever of the two an operand's alignment selects.
 template <typename AT, int WK, int MT, int LG, bool GLU>
 __global__ __launch_bounds__(NTHR) void gemv_short_kernel(GemvParams p) {
   constexpr int NR = GLU ? 2 : 1, RPW = 64 / LG, U = GLU || MT > 2 ? 2 : 4;
@@ -318,7 +330,7 @@ __global__ __launch_bounds__(NTHR) void gemv_short_kernel(GemvParams p) {
     for (int j = 0; j < 8; ++j) xv[m][j] = on ? to_f32(e[j]) : 0.f;
   }
   auto group_sum = [&](float v) {                    // all-reduce over the LG lanes of a row
-    if constexpr (LG == 8) return lane8_sum(v);
+    if constexpr (LG == 8) return xor2_xor1(v + xor4(v));
     v = row16_sum(v);
     if constexpr (LG == 64) { v += __shfl_xor(v, 16); v += __shfl_xor(v, 32); }
     return v;
@@ -329,10 +341,31 @@ __global__ __launch_bounds__(NTHR) void gemv_short_kernel(GemvParams p) {
     for (int j = 0; j < (int)sizeof(AT) / 2; ++j) ((u32x4*)nw)[j] = ((const u32x4*)((const AT*)p.norm_w + (on ? k : 0)))[j];
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-      float ss = 0.f;
+#pragma clang fp contract(off)                        // (the squares are rounded before they are added, there as here)
+      // gemv_v1_kernel's order: thread t of 256 holds k = t (and t + 256), its wave_sum pairs k with k + 8, + 4, + 2, + 1 inside 16, the
+      // four sixteens of 64 in pairs, the sixty-fours in sequence.  Here 64 columns are 8 lanes.
+      float s[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) ss = fmaf(xv[m][j], xv[m][j], ss);
-      const float rs = 1.0f / sqrtf(group_sum(ss) / (float)p.K + p.eps);
+      for (int j = 0; j < 8; ++j) s[j] = xv[m][j] * xv[m][j];
+      if constexpr (LG == 64)
+        if (p.K > 256) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const float far = __shfl_xor(xv[m][j], 32);
+            s[j] = lane < 32 ? fmaf(far, far, s[j]) : 0.f;
+          }
+        }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s[j] += __builtin_amdgcn_update_dpp(0.f, s[j], 0xB1, 0xf, 0xf, false);     // quad_perm:[1,0,3,2]
+      float t = ((s[0] + s[4]) + (s[2] + s[6])) + ((s[1] + s[5]) + (s[3] + s[7]));
+      t += __builtin_amdgcn_update_dpp(0.f, t, 0x4E, 0xf, 0xf, false);                                       // quad_perm:[2,3,0,1]
+      t += xor4(t);
+      if constexpr (LG == 16) t += __builtin_amdgcn_update_dpp(0.f, t, 0x128, 0xf, 0xf, false);              // row_ror:8
+      if constexpr (LG == 64) {
+        auto at = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, t), l)); };
+        t = ((at(0) + at(8)) + at(16)) + at(24);
+      }
+      const float rs = 1.0f / sqrtf(t / (float)p.K + p.eps);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const AT xn = store_act<AT>(xv[m][j] * rs, p.rnd);

@@ -169,6 +169,11 @@ def test_gemv_short_rows(act, kind, K, M):
         out = torch.zeros((M, N), dtype=xd.dtype, device="cuda")
         gemv(ol, xd, M, act, pro=L.PRO_NORM, norm_w=dev(nw, act), eps=1e-5, epi=L.EPI_STORE, out=out, ldo=N, force_generic=1, ldx=K + pad)
         _assert_close(host(out), round_to(matmul_nt(xn, wdense), act), act)
+        if not pad:                                     # the same bits from gemv_v1_kernel, which takes any stride
+            out2 = torch.zeros((M, N), dtype=xd.dtype, device="cuda")
+            gemv(ol, dev(np.pad(x, ((0, 0), (0, 1))), act), M, act, pro=L.PRO_NORM, norm_w=dev(nw, act), eps=1e-5, epi=L.EPI_STORE, out=out2, ldo=N,
+                 force_generic=1, ldx=K + 1)
+            assert torch.equal(out, out2)
     I = 37
     ol, wdense, keep = _make_weight(kind, 2 * I, K, act)
     g, u = round_to(matmul_nt(x, wdense[:I]), act), round_to(matmul_nt(x, wdense[I:]), act)
