@@ -95,8 +95,10 @@ int mi_op_gemm_skinny(const mi_op_linear* w, const mi_op_gemv_args* a, int kspli
  * nn.Linear over B x L rows at once).  a->M rows of 16-bit activations, tile-major dense 16-bit weights, a->pro =
  * MI_PRO_NONE; plain / residual / SwiGLU epilogues.  iters >= 1 also times that many back-to-back launches into *avg_ms. */
 int mi_op_gemm_prefill(const mi_op_linear* w, const mi_op_gemv_args* a, int iters, float* avg_ms);
-/* gemv_reg.hip on its own: the decode linears of at most 8 rows on tile-major int4 / int8 (group 64) weights with scales of the
- * activations' type; a->pro MI_PRO_NONE or MI_PRO_NORM; plain / float32 / residual / SwiGLU (with the norm) epilogues. */
+/* gemv_reg.hip on its own: the decode linears of at most 8 rows on tile-major weights -- int4 / int8 (group 64) with scales of the
+ * activations' type (plain / float32 / residual / SwiGLU epilogues, the last with the norm), dense 16-bit ones with activations of
+ * their type or float32 on bf16 (plain / float32 / residual; float32 also MI_EPI 4, SwiGLU on a row-interleaved gate|up matrix:
+ * 8 gate rows, their 8 up rows, ...).  a->pro MI_PRO_NONE or MI_PRO_NORM. */
 int mi_op_gemv_reg(const mi_op_linear* w, const mi_op_gemv_args* a);
 /* tile-major weight layout of the streaming kernels (what mi_engine_finalize applies to eligible
  * matrices): returns the size of the tiled buffer (0 if the matrix is not eligible) / fills `dst`. */

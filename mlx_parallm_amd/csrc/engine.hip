@@ -302,6 +302,20 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
     Prof pr(e, prof);
     return launch_gemv_reg(f.W, c, rows, e->stream);
   }
+  if (e->opt_skinny_gemm && rows <= 8 && !quant) {
+    // dense weights: float32 activations, and the short linears of 16-bit ones (gemv_reg.hip)
+    LinearW wv = f.W;
+    GemvCall cd = c;
+    if (c.epi == EPI_SWIGLU && c.act == MI_F32 && gu8_wanted(e, f0, c.pair_offset) && f.W.w == f0.W.w &&
+        ensure_gu8(e, const_cast<FusedLinear&>(f0), c.pair_offset)) {
+      wv.w = f0.w_gu8;                         // (a view: the copy stays owned by f0)
+      cd.epi = EPI_SWIGLU_GU8;
+    }
+    if (gemv_dense_supported(wv, cd, rows)) {
+      Prof pr(e, prof);
+      return launch_gemv_dense(wv, cd, rows, e->stream);
+    }
+  }
   if (e->opt_skinny_gemm && ((e->cur_L == 1 && rows <= decode_max) || rows <= short_rows) && gemm_skinny_supported(f.W, c, rows)) {
     // the decode step of a batch of 9..128 sequences (int4 / int8 weights: any batch up to 128): W is streamed once, K split over workgroups (gemm_skinny.hip).
     // Also a prefill of up to 128 rows in all (a short prompt, a few short prompts): at that size the op is a weight

@@ -993,7 +993,7 @@ int launch_at(const SkinnyParams& p, int qb, bool swiglu, int mt, int grid, hipS
 
 }  // namespace
 
-// 16-bit / int4 weights: gemv_mfma.hip serves up to 8 rows, this kernel 9..64 (its 16-row instantiation beats the
+// 16-bit / int4 weights: gemv_reg.hip and, where it does not apply, gemv_mfma.hip serve up to 8 rows, this kernel 9..64 (its 16-row instantiation beats the
 // M <= 16 form of gemv_mfma.hip, which stages all of x per workgroup: Mistral-7B bf16 B = 16 3557 -> 3835 tok/s, int4
 // 4181 -> 5973, Qwen3-14B bf16 1401 -> 2386; at 8 rows and below gemv_mfma.hip wins, 3.59 vs 3.95 ms/step).
 // MI_SKINNY_MIN_ROWS moves the hand-over (A/B).

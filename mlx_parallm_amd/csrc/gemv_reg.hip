@@ -1,4 +1,4 @@
-// gemv_reg.hip -- decode linears of at most 8 rows on int4 / int8 weights, activations in registers: y[M][N] = x[M][K] . W[N][K]^T
+// gemv_reg.hip -- decode linears of at most 8 rows, activations in registers: int4 / int8 weights, and (gemv_dense_kernel) 16-bit ones: y[M][N] = x[M][K] . W[N][K]^T
 // (nn.QuantizedLinear call sites llama.py:64-67,93,143,160-165,250-252; qwen3.py:37-40,63,115).
 //
 // The split-K kernel of gemm_skinny.hip spends most of a short launch outside the weight stream: x goes through LDS in chunks with a
@@ -111,13 +111,16 @@ __device__ __forceinline__ void mul_blk(f32x4& acc, const WBlk<QB>& w, const u32
   }
 }
 
+__device__ __forceinline__ float sum_waves(const float* q) {      // the eight waves' partial tiles at one place
+  return ((q[0] + q[256]) + (q[512] + q[768])) + ((q[1024] + q[1280]) + (q[1536] + q[1792]));
+}
+
 // y[m][n] of one tile (gate and up for SwiGLU), m = tid / 16, n = tile's column tid % 16: the waves' partial tiles added pairwise
 template <typename AT, int NW, bool SW>
 __device__ __forceinline__ void finish_tile(const RegParams& p, const float* part, int tile, int tid, float hv) {
   const int m = tid >> 4, n = tile * 16 + (tid & 15), at = ((m >> 2) * 16 + (tid & 15)) * 4 + (m & 3);
-  auto sum = [&](const float* q) { return ((q[0] + q[256]) + (q[512] + q[768])) + ((q[1024] + q[1280]) + (q[1536] + q[1792])); };
   static_assert(NW == 8, "");
-  const float y = sum(part + at), u = SW ? sum(part + NW * 256 + at) : 0.f;
+  const float y = sum_waves(part + at), u = SW ? sum_waves(part + NW * 256 + at) : 0.f;
   AT* out = (AT*)p.out;
   if constexpr (SW) out[(size_t)m * p.ldo + n] = silu16<AT>(y, u);
   else if (p.epi == EPI_STORE) out[(size_t)m * p.ldo + n] = (AT)y;
@@ -299,6 +302,161 @@ __global__ __launch_bounds__(512, 2) void gemv_long_kernel(const RegParams p) {
   if (fin) finish_tile<AT, NW, false>(p, part, tile, tid, (float)hv);
 }
 
+// Dense 16-bit weights, x in float32 (the float32-cache mode; X32) or in the weights' type.  The same split of the work; x is split exactly
+// into three terms of the weights' type in registers (96 of them at 512 k per wave), each weight fragment meets the three, their sums stay
+// apart up to the end.  A tile's 16 fragments are all in flight, the next tile's go out as they are consumed.
+// GU: tiles of the row-interleaved gate|up copy (8 gate, 8 up rows; repack.hip): seven per CU where whole pairs are 3.5.
+// Measured (Mistral-7B shapes, rocprof us; an empty kernel is 4).  float32 x, 8 rows, gemm_skinny.hip -> here: gate|up 50.6 -> 43.0 (235 MB at
+// the card's 5.9 TB/s: 41.7; 224 workgroups there), q|k|v 17.0 -> 15.7, o 13.1 -> 11.3; its rms error against 64 bits is 0.4 of that kernel's.
+// 16-bit x, 1 row, gemv_mfma.hip -> here: q|k|v and o 12.6 on average -> 11.0 and 7.9; K = 2048, 4 rows 18.3 -> 10.3.
+template <typename AT, bool X32>
+struct RawX { u32x4 v[X32 ? 2 : 1]; };
+template <typename AT, bool X32>
+__device__ __forceinline__ void unpack_raw(const RawX<AT, X32>& r, f32x2 (&e)[4]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if constexpr (X32) e[j] = f32x2{__uint_as_float(r.v[j >> 1][2 * (j & 1)]), __uint_as_float(r.v[j >> 1][2 * (j & 1) + 1])};
+    else e[j] = unpack2<AT>(r.v[0][j]);
+  }
+}
+
+template <typename AT, bool X32, bool GU, bool NORM, int KW>
+__global__ __launch_bounds__(512, 2) void gemv_dense_kernel(const RegParams p) {
+  using XT = typename std::conditional<X32, float, AT>::type;
+  constexpr int NW = 8, NP = KW / 32, NQ = NP / 2, T = X32 ? 3 : 1, NC = X32 ? 3 : 2;      // products, pairs of them, terms, chains of sums
+  __shared__ __attribute__((aligned(16))) float part[2][NW * 256];
+  __shared__ float sq[NW][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c16 = lane & 15, g = lane >> 4;
+  const int q0 = wave * p.nblk / NW, nq = (wave + 1) * p.nblk / NW - q0;        // this wave's pairs (64 k each) of every tile
+  const int step = gridDim.x;
+
+  u32x4 wb[NP];
+  auto pair_at = [&](int q) { return q0 + min(q, max(nq - 1, 0)); };            // (past the last: the last one again, times zero)
+  auto issue = [&](int i, int tile) {
+    wb[i] = __builtin_nontemporal_load((const u32x4*)((const char*)p.w + ((size_t)tile * p.nblk * 2 + pair_at(i >> 1) * 2 + (i & 1)) * 1024 + lane * 16));
+  };
+  auto issue_first = [&] {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) issue(i, blockIdx.x);
+  };
+  if constexpr (!NORM) issue_first();
+
+  RawX<AT, X32> raw[NQ], nw[NORM ? NQ : 1];
+  const int koff = (c16 >> 3) * 32 + g * 8;                                     // lanes of columns 8 .. 15: the pair's second fragment
+  const XT* xr = (const XT*)p.x + (size_t)min(c16 & 7, p.M - 1) * p.ldx + koff;
+  auto load_raw = [&](RawX<AT, X32>& r, const XT* s, int q) {
+#pragma unroll
+    for (int h = 0; h < (X32 ? 2 : 1); ++h) r.v[h] = *(const u32x4*)(s + pair_at(q) * 64 + h * 4);
+  };
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) load_raw(raw[q], xr, q);
+  if constexpr (NORM) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) load_raw(nw[q], (const XT*)p.norm_w + koff, q);
+    __builtin_amdgcn_sched_barrier(0);
+    issue_first();
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const bool res = !GU && p.epi == EPI_RESID, fin = tid < 256 && (tid >> 4) < p.M;
+  const XT* hrow = (const XT*)(res ? p.resid : p.x) + (res ? (size_t)min(tid >> 4, p.M - 1) * p.ldo + (tid & 15) : 0);
+
+  float rs = 1.f;
+  if constexpr (NORM) {
+    float ss = 0.f;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      f32x2 e[4];
+      unpack_raw<AT, X32>(raw[q], e);
+      float s1 = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s1 = fmaf(e[j].x, e[j].x, fmaf(e[j].y, e[j].y, s1));
+      ss += q < nq ? s1 : 0.f;
+    }
+    ss += __builtin_amdgcn_update_dpp(0.f, ss, 0x128, 0xf, 0xf, false);      // (columns c and c + 8 hold one row)
+    ss += __shfl_xor(ss, 16);
+    ss += __shfl_xor(ss, 32);
+    if (g == 0) sq[wave][c16] = ss;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    float t = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) t += sq[w][c16];
+    rs = 1.0f / sqrtf(t / (float)p.K + p.eps);
+  }
+  u32x4 xf[T][NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    f32x2 e[4], we[4];
+    unpack_raw<AT, X32>(raw[q], e);
+    if constexpr (NORM) unpack_raw<AT, X32>(nw[q], we);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if constexpr (X32) {
+        f32x2 v = e[j];
+        if constexpr (NORM) v = f32x2{v.x * rs * we[j].x, v.y * rs * we[j].y};
+        const uint32_t hi = pack2<AT>(v);
+        const f32x2 h = unpack2<AT>(hi), r1 = f32x2{v.x - h.x, v.y - h.y};
+        const uint32_t mid = pack2<AT>(r1);
+        const f32x2 m = unpack2<AT>(mid);
+        xf[0][q][j] = hi; xf[1][q][j] = mid; xf[2][q][j] = pack2<AT>(f32x2{r1.x - m.x, r1.y - m.y});
+      } else if constexpr (NORM) {                    // w * cast_T(x32 * rsqrt(..)), rounded to T
+        const f32x2 xn = unpack2<AT>(pack2<AT>(f32x2{e[j].x * rs, e[j].y * rs}));
+        xf[0][q][j] = pack2<AT>(f32x2{xn.x * we[j].x, xn.y * we[j].y});
+      } else {
+        xf[0][q][j] = raw[q].v[0][j];
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+      if (q >= nq) xf[t][q] = u32x4{0u, 0u, 0u, 0u};
+  }
+
+  int buf = 0;
+  auto do_tile = [&](int tile, auto more) {
+    const XT hv = hrow[res ? tile * 16 : 0];
+    f32x4 acc[NC];
+#pragma unroll
+    for (int a = 0; a < NC; ++a) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const u32x4 f = (i & 1) ? ror8(xf[t][i >> 1]) : xf[t][i >> 1];
+        f32x4& a = acc[X32 ? t : i & 1];
+        a = mfma16<AT>(f, wb[i], a);
+      }
+      if constexpr (decltype(more)::value) {
+        __builtin_amdgcn_sched_barrier(0);
+        issue(i, tile + step);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    *(f32x4*)&part[buf][wave * 256 + lane * 4] = X32 ? (acc[NC - 1] + acc[1]) + acc[0] : acc[0] + acc[1];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();                     // (the loads of the next tile stay in flight)
+    asm volatile("" ::: "memory");
+    if constexpr (!X32) {
+      if (fin) finish_tile<AT, NW, false>(p, part[buf], tile, tid, (float)hv);
+    } else if (fin) {
+      const int m = tid >> 4, c = tid & 15, at = ((m >> 2) * 16 + c) * 4 + (m & 3);
+      const float y = sum_waves(part[buf] + at);
+      if constexpr (GU) {
+        const float u = __shfl_down(y, 8);
+        if (c < 8) {
+          const float sig = 1.0f / (1.0f + expf(-y)), sl = y * sig;
+          ((float*)p.out)[(size_t)m * p.ldo + tile * 8 + c] = sl * u;
+        }
+      } else if (res) ((float*)p.resid)[(size_t)m * p.ldo + tile * 16 + c] = hv + y;
+      else ((float*)p.out)[(size_t)m * p.ldo + tile * 16 + c] = y;
+    }
+    buf ^= 1;                                         // the buffer read now is written again two tiles on, behind the next barrier
+  };
+  int tile = blockIdx.x;
+  for (; tile + step < p.ntiles; tile += step) do_tile(tile, std::true_type{});
+  do_tile(tile, std::false_type{});
+}
+
 int quant_bits(const LinearW& W, int act) {           // 4 / 8: codes with scales of the activation type, 0: neither
   if (((W.wk == WK_Q4_BF16 && act == MI_BF16) || (W.wk == WK_Q4_F16 && act == MI_F16)) && W.group == 64) return 4;
   if (((W.wk == WK_Q8_BF16 && act == MI_BF16) || (W.wk == WK_Q8_F16 && act == MI_F16)) && W.group == 64) return 8;
@@ -362,6 +520,49 @@ int launch_gemv_reg(const LinearW& W, const GemvCall& c, size_t rows, hipStream_
   p.nblk = W.K / (qb == 4 ? 128 : 64);
   if (c.act == MI_BF16) return qb == 4 ? launch_reg<bf16, 4>(p, sw, st) : launch_reg<bf16, 8>(p, sw, st);
   return qb == 4 ? launch_reg<f16, 4>(p, sw, st) : launch_reg<f16, 8>(p, sw, st);
+}
+
+bool gemv_dense_supported(const LinearW& W, const GemvCall& c, size_t rows) {
+  static const bool off = getenv("MI_GEMV_DENSE") != nullptr && atoi(getenv("MI_GEMV_DENSE")) == 0;      // (A/B)
+  if (off || c.force_v1 || W.layout != 1 || rows < 1 || rows > 8 || c.rnd != RND_NONE || c.kx != 0) return false;
+  if (W.lora_b[0] != nullptr || W.lora_b[1] != nullptr || c.out32 || c.silu_cols > 0 || c.glu.kind != GLU_SILU) return false;
+  const bool x32 = c.act == MI_F32 && W.wk == WK_BF16;
+  if (!x32 && !(W.wk == WK_BF16 && c.act == MI_BF16) && !(W.wk == WK_F16 && c.act == MI_F16)) return false;
+  if (c.epi == EPI_SWIGLU_GU8 ? !(x32 && c.pro == PRO_NORM && c.pair_offset % 8 == 0 && W.N == 2 * c.pair_offset)
+                              : c.epi != EPI_STORE && c.epi != EPI_STORE_F32 && c.epi != EPI_RESID) return false;
+  if (W.K % 64 != 0 || W.N % 16 != 0 || W.K > REG_K) return false;
+  // 16-byte loads of x and the norm's weights
+  return c.ldx % (x32 ? 4 : 8) == 0 && (uintptr_t)c.x % 16 == 0 && (c.pro != PRO_NORM || (uintptr_t)c.norm_w % 16 == 0);
+}
+
+template <typename AT, bool X32>
+static int launch_dense(const RegParams& p, bool gu, hipStream_t st) {
+  const int kw = (p.nblk + 7) / 8 * 64, grid = std::min(p.ntiles, gemv_cu_count());
+  auto go = [&](auto kern) -> int {
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(512), 0, st, p);
+    MI_HIP(hipGetLastError());
+    return MI_OK;
+  };
+  if constexpr (X32)
+    if (gu) return kw <= 256 ? go(gemv_dense_kernel<AT, X32, true, true, 256>) : kw <= 512 ? go(gemv_dense_kernel<AT, X32, true, true, 512>)
+                             : go(gemv_dense_kernel<AT, X32, true, true, 640>);
+  if (p.norm) return kw <= 256 ? go(gemv_dense_kernel<AT, X32, false, true, 256>) : kw <= 512 ? go(gemv_dense_kernel<AT, X32, false, true, 512>)
+                               : go(gemv_dense_kernel<AT, X32, false, true, 640>);
+  return kw <= 256 ? go(gemv_dense_kernel<AT, X32, false, false, 256>) : kw <= 512 ? go(gemv_dense_kernel<AT, X32, false, false, 512>)
+                   : go(gemv_dense_kernel<AT, X32, false, false, 640>);
+}
+
+int launch_gemv_dense(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st) {
+  if (!gemv_dense_supported(W, c, rows)) return fail(MI_ERR_UNSUPPORTED, "gemv_dense: shape / dtype not supported");
+  RegParams p{};
+  p.x = c.x; p.ldx = c.ldx; p.M = (int)rows;
+  p.norm = c.pro == PRO_NORM; p.norm_w = c.norm_w; p.eps = c.eps;
+  p.w = W.w; p.N = W.N; p.K = W.K;
+  p.epi = c.epi; p.out = c.out; p.ldo = c.ldo; p.resid = c.resid;
+  p.ntiles = W.N / 16; p.nblk = W.K / 64;
+  const bool gu = c.epi == EPI_SWIGLU_GU8;
+  if (c.act == MI_F32) return launch_dense<bf16, true>(p, gu, st);
+  return c.act == MI_BF16 ? launch_dense<bf16, false>(p, gu, st) : launch_dense<f16, false>(p, gu, st);
 }
 
 }  // namespace mi

@@ -122,6 +122,10 @@ int launch_rmsnorm_rows(const void* x, int ldx, const void* w, void* out, int ld
 bool gemv_reg_supported(const LinearW& W, const GemvCall& c, size_t rows);
 int launch_gemv_reg(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st);
 
+// the same on dense 16-bit weights, x of their type or (bf16 weights) float32; EPI_SWIGLU_GU8 with float32 x and the norm
+bool gemv_dense_supported(const LinearW& W, const GemvCall& c, size_t rows);
+int launch_gemv_dense(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st);
+
 // 9..64 rows, int8 weights 1..64 (decode steps of larger batches): weight-streaming split-K GEMM (gemm_skinny.hip).
 // c.pro must be PRO_NONE; `ws` >= gemm_skinny_ws_bytes(), `ctr` >= gemm_skinny_groups() words that are zero between
 // launches (the kernel leaves them zero); ksplit = 0 lets the cost model choose.

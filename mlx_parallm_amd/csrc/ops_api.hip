@@ -154,7 +154,8 @@ int mi_op_gemv_reg(const mi_op_linear* w, const mi_op_gemv_args* a) {
   MI_TRY(ready());
   const GemvCall c = to_call(a);
   if (c.M < 1) return fail(MI_ERR_INVALID, "mi_op_gemv_reg: M out of range");
-  MI_TRY(launch_gemv_reg(to_linear(w), c, (size_t)c.M, nullptr));
+  const LinearW W = to_linear(w);
+  MI_TRY(wk_is_quant(W.wk) ? launch_gemv_reg(W, c, (size_t)c.M, nullptr) : launch_gemv_dense(W, c, (size_t)c.M, nullptr));
   return finish();
 }
 

@@ -10,7 +10,7 @@ from oracle.numerics import matmul_nt, round_to
 pytestmark = pytest.mark.gpu
 
 from mlx_parallm_amd import _lib as L  # noqa: E402
-from gpu_helpers import dev, gemv_reg, host  # noqa: E402
+from gpu_helpers import dev, gemv_reg, host, op_linear, to_tiled  # noqa: E402
 from test_gpu_kernels import _assert_close  # noqa: E402
 from test_gpu_skinny import KINDS, _weight  # noqa: E402
 
@@ -80,3 +80,57 @@ def test_refuses_what_it_does_not_take(kind, M, K, epi, norm):
     out = torch.zeros((M, 32), dtype=torch.bfloat16, device="cuda")
     with pytest.raises(Exception, match="gemv_reg"):
         gemv_reg(ol, xd, M, "bfloat16", epi=epi, out=out, ldo=32, pair_offset=16, norm_w=xd[0] if norm else None)
+
+
+DENSE = [("bfloat16", "bf16"), ("float16", "f16"), ("float32", "bf16")]
+
+
+# K in pairs of 64: one (seven idle waves), not a multiple of 8, each register size's last K and the first of the next
+@pytest.mark.parametrize("act,kind", DENSE)
+@pytest.mark.parametrize("M,N,K", [(1, 16, 64), (8, 80, 576), (3, 48, 2048), (5, 32, 2112), (7, 32, 4096), (2, 32, 4160), (8, 48, 5120),
+                                   (8, 16 * 515, 128)])
+def test_dense_matches_oracle(act, kind, M, N, K):
+    rng = np.random.default_rng(M * 1000003 + N * 1009 + K + 2)
+    ol, w, keep = _weight(kind, N, K, rng)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    h = rng.standard_normal((M, N)).astype(np.float32) * 4.0
+    nw = 1.0 + 0.1 * rng.standard_normal(K).astype(np.float32)
+    if act != "float32":
+        x, h, nw = round_to(x, act), round_to(h, act), round_to(nw, act)
+    xd, hd, nwd = dev(np.concatenate([x, np.full((1, K), np.nan, np.float32)]), act), dev(np.concatenate([h, h[:1]]), act), dev(nw, act)
+    for norm in (None, nwd):
+        xn = x if norm is None else ref_model.rms_norm(x, act, nw, act, 1e-5)[0]
+        want = matmul_nt(xn, w)
+        outs = []
+        for _ in range(2):
+            out = torch.full((M + 1, N), 7.0, dtype=xd.dtype, device="cuda")
+            gemv_reg(ol, xd, M, act, epi=L.EPI_STORE, out=out, ldo=N, norm_w=norm)
+            outs.append(host(out))
+        assert np.array_equal(outs[0], outs[1]) and np.all(outs[0][M:] == 7.0)
+        _assert_close(outs[0][:M], want if act == "float32" else round_to(want, act), act, scale=float(np.sqrt(K)) if act == "float32" else None)
+        out = torch.full((M + 1, N), 7.0, dtype=torch.float32, device="cuda")
+        gemv_reg(ol, xd, M, act, epi=L.EPI_STORE_F32, out=out, ldo=N, norm_w=norm)
+        assert np.array_equal(host(out), outs[0])
+    gemv_reg(ol, xd, M, act, epi=L.EPI_RESID, resid=hd, ldo=N, norm_w=nwd)
+    got = host(hd)
+    want = h + outs[0][:M]
+    assert np.array_equal(got[:M], want if act == "float32" else round_to(want, act)) and np.array_equal(got[M:], h[:1])
+
+
+@pytest.mark.parametrize("M,I,K", [(1, 16, 64), (8, 48, 576), (5, 4128, 2048), (8, 48, 5120)])
+def test_dense_swiglu_on_interleaved_rows(M, I, K):
+    rng = np.random.default_rng(M * 1000003 + I * 1009 + K + 3)
+    w = round_to(rng.standard_normal((2 * I, K)).astype(np.float32) * 0.05, "bfloat16")
+    order = np.concatenate([np.r_[8 * t:8 * t + 8, I + 8 * t:I + 8 * t + 8] for t in range(I // 8)])
+    wd = dev(w[order], "bfloat16")
+    ol, keep = op_linear("bf16", 2 * I, K, wd), [wd]
+    assert to_tiled(ol, keep)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    nw = 1.0 + 0.1 * rng.standard_normal(K).astype(np.float32)
+    xd, nwd = dev(x, "float32"), dev(nw, "float32")
+    y = matmul_nt(ref_model.rms_norm(x, "float32", nw, "float32", 1e-5)[0], w).astype(np.float64)
+    out = torch.full((M + 1, I), 7.0, dtype=torch.float32, device="cuda")
+    gemv_reg(ol, xd, M, "float32", epi=4, out=out, ldo=I, pair_offset=I, norm_w=nwd)
+    want = y[:, :I] / (1.0 + np.exp(-y[:, :I])) * y[:, I:]
+    assert np.all(host(out)[M:] == 7.0)
+    _assert_close(host(out)[:M], want, "float32", scale=float(np.abs(y).max()) ** 2)
