@@ -77,14 +77,12 @@ __device__ __forceinline__ u32x4 unpack_q4(uint32_t v) {
   // fragment element 2p <- nibble p, element 2p+1 <- nibble p+4
   u32x4 r;
   if constexpr (std::is_same<T, bf16>::value) {
-    // (x & mask) | magic as ONE v_and_or_b32 with both constants in registers: hipcc emits v_and + v_or with
-    // literals (a VOP3 cannot carry two), and this kernel is bound by its VALU instruction count
-    const uint32_t mask = 0x00780078u, magic = 0x41804180u;
-    auto and_or = [&](uint32_t x) {
-      uint32_t o;
-      asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(o) : "v"(x), "v"(mask), "v"(magic));
-      return o;
-    };
+    // (x & mask) | magic as ONE v_and_or_b32 with both constants in registers: given literals, hipcc emits v_and + v_or (a VOP3 cannot
+    // carry two), and this kernel is bound by its VALU instruction count.  The constants are made opaque, the instruction is the
+    // compiler's: it keeps the distance a matrix product needs behind a write of its operand, which it cannot do for one in an asm.
+    uint32_t mask = 0x00780078u, magic = 0x41804180u;
+    asm("" : "+v"(mask), "+v"(magic));
+    auto and_or = [&](uint32_t x) { return (x & mask) | magic; };
     r.x = and_or(v << 3);
     r.y = and_or(v >> 1);
     r.z = and_or(v >> 5);
