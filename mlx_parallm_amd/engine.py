@@ -72,11 +72,12 @@ class _ResultPool:
                 self._drop_free()
 
     def _drop_free(self) -> None:
-        for size, blocks in self._free.items():
-            for p in blocks:
-                L.lib().mi_host_free(p)
+        while self._free:                             # (a block is off the lists before it is freed: what a collection in here drops comes back to them)
+            size, blocks = self._free.popitem()
+            while blocks:
+                p = blocks.pop()
                 self._bytes -= size
-        self._free.clear()
+                L.lib().mi_host_free(p)
 
     def empty(self, shape) -> np.ndarray:
         """float32 array of this shape, contents undefined."""

@@ -207,3 +207,54 @@ def test_result_pool_hands_out_only_what_nobody_sees(monkeypatch):
     assert len(live) == 2                                                                        # what c and row still show
     del c, row
     assert len(live) == 0 and pool._bytes == 0
+
+
+def test_result_pool_frees_while_a_collection_drops_arrays(monkeypatch):
+    """A collection inside the pool's own freeing may drop another array: nothing raises, no block is freed twice or handed out behind its
+    free, and the count stays right -- also where the array is of the size class that is being freed."""
+    import ctypes as C
+    import gc
+
+    from mlx_parallm_amd import engine as E
+
+    live = {}
+
+    class Fake:
+        @staticmethod
+        def mi_host_alloc(n, out):
+            buf = C.create_string_buffer(n)
+            out._obj.value = C.addressof(buf)
+            live[C.addressof(buf)] = buf
+            return 0
+
+        @staticmethod
+        def mi_host_free(p):
+            gc.collect()
+            del live[p.value]
+
+    monkeypatch.setattr(E.L, "lib", lambda: Fake)
+    monkeypatch.setattr(E._ResultPool, "MIN_BYTES", 1 << 10)
+    monkeypatch.setattr(E._ResultPool, "MAX_BYTES", 8 << 18)
+
+    class Cycle:
+        def __init__(self, array):
+            self.array, self.me = array, self
+
+    for rows in (1000, 70000, 140000):                 # the array that the collection drops: one, two, three blocks of 256 KiB
+        gc.collect()
+        gc.disable()
+        try:
+            pool = E._ResultPool()
+            pool.engine_opened()
+            kept = [pool.empty((4, 1000)), pool.empty((70000,)), pool.empty((4, 1000))]
+            Cycle(pool.empty((rows,)))                 # unreachable, not yet collected
+            del kept
+            big = pool.empty((500000,))                # eight blocks: all that is kept goes
+            assert len(live) == 1 and pool._bytes == 8 << 18 and not pool._free
+            Cycle(big)
+            del big
+            pool.engine_closed()
+            gc.collect()
+        finally:
+            gc.enable()
+        assert not live and pool._bytes == 0 and not pool._free
