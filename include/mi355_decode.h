@@ -378,8 +378,11 @@ int mi_engine_set_option(mi_engine* e, const char* key, int64_t value);
 int mi_engine_sync(mi_engine* e);
 
 /* Pinned host memory for results (any buffer works; a copy into pinned memory runs at the link's rate, one into fresh pageable
- * memory is staged in pieces and faults every page: 39 MB of logits 5.3 ms against 0.8).  Free it with mi_host_free. */
+ * memory is staged in pieces and faults every page: 39 MB of logits 5.3 ms against 0.8).  Free it with mi_host_free.
+ * mi_engine_host_alloc makes the engine's device the calling thread's first, as every call on an engine does; mi_host_alloc
+ * allocates under whichever device that is (a new thread's: device 0). */
 int mi_host_alloc(uint64_t bytes, void** out);
+int mi_engine_host_alloc(mi_engine* e, uint64_t bytes, void** out);
 void mi_host_free(void* p);
 
 const char* mi_last_error(void);

@@ -134,6 +134,7 @@ SIGNATURES = {
     "mi_engine_set_option": (C.c_int, [_P, C.c_char_p, C.c_int64]),
     "mi_engine_sync": (C.c_int, [_P]),
     "mi_host_alloc": (C.c_int, [C.c_uint64, C.POINTER(_P)]),
+    "mi_engine_host_alloc": (C.c_int, [_P, C.c_uint64, C.POINTER(_P)]),
     "mi_host_free": (None, [_P]),
     "mi_last_error": (C.c_char_p, []),
     "mi_version": (C.c_char_p, []),

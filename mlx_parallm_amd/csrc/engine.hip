@@ -1780,6 +1780,11 @@ int mi_host_alloc(uint64_t bytes, void** out) {
   }
   return MI_OK;
 }
+int mi_engine_host_alloc(mi_engine* e, uint64_t bytes, void** out) {
+  if (!e) return fail(MI_ERR_INVALID, "null engine");
+  MI_HIP(hipSetDevice(e->device));
+  return mi_host_alloc(bytes, out);
+}
 void mi_host_free(void* p) { if (p) hipHostFree(p); }
 
 int mi_engine_sync(mi_engine* e) {

@@ -79,8 +79,9 @@ class _ResultPool:
                 self._bytes -= size
                 L.lib().mi_host_free(p)
 
-    def empty(self, shape) -> np.ndarray:
-        """float32 array of this shape, contents undefined."""
+    def empty(self, shape, engine: Optional[C.c_void_p] = None) -> np.ndarray:
+        """float32 array of this shape, contents undefined.  ``engine``: whose device a new block is made under (a thread that has not
+        used the engine yet is on device 0)."""
         n = 4 * int(np.prod(shape, dtype=np.int64))
         if n < self.MIN_BYTES or n > self.MAX_BYTES:
             return np.empty(shape, dtype=np.float32)
@@ -93,7 +94,9 @@ class _ResultPool:
                 if self._bytes + size > self.MAX_BYTES:
                     self._drop_free()
                 p = C.c_void_p()
-                if self._bytes + size > self.MAX_BYTES or L.lib().mi_host_alloc(size, C.byref(p)) != 0:
+                lib = L.lib()
+                if self._bytes + size > self.MAX_BYTES or (lib.mi_engine_host_alloc(engine, size, C.byref(p)) if engine else
+                                                           lib.mi_host_alloc(size, C.byref(p))) != 0:
                     return np.empty(shape, dtype=np.float32)
                 self._bytes += size
         return np.asarray(_ResultBlock(self, p, size, tuple(shape)))
@@ -455,7 +458,7 @@ class Engine:
         ptr = None
         if want_logits:
             V = self.desc.vocab_size
-            out = _results.empty((B, Lq, V) if all_positions else (B, V))
+            out = _results.empty((B, Lq, V) if all_positions else (B, V), self._h)
             ptr = out.ctypes.data_as(C.POINTER(C.c_float))
         L.check(L.lib().mi_forward(self._h, kv._h, tok.ctypes.data_as(C.POINTER(C.c_int32)), B, Lq, ptr,
                                    int(all_positions)))
@@ -531,7 +534,7 @@ class Engine:
         toks = np.ascontiguousarray(np.concatenate([_i32(t).reshape(-1) for t in token_lists]))
         offs = kv.offsets
         kv.ensure(max(offs[int(i)] + int(n) for i, n in zip(r, lens)))
-        out = _results.empty((len(w), self.desc.vocab_size))
+        out = _results.empty((len(w), self.desc.vocab_size), self._h)
         I32 = C.POINTER(C.c_int32)
         L.check(L.lib().mi_forward_segments(self._h, kv._h, r.ctypes.data_as(I32), lens.ctypes.data_as(I32), len(r),
                                             toks.ctypes.data_as(I32), w.ctypes.data_as(I32), len(w),

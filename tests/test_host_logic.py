@@ -258,3 +258,40 @@ def test_result_pool_frees_while_a_collection_drops_arrays(monkeypatch):
         finally:
             gc.enable()
         assert not live and pool._bytes == 0 and not pool._free
+
+
+def test_result_blocks_are_made_under_the_engine_s_device(monkeypatch):
+    """forward() and forward_segments() ask for their result block before the call that sets the engine's device: in a thread that has not
+    used the engine the block would be made under device 0, whichever device the engine is on."""
+    import ctypes as C
+    import types
+
+    from mlx_parallm_amd import engine as E
+
+    asked, blocks = [], []
+
+    class Fake:
+        @staticmethod
+        def mi_engine_host_alloc(e, n, out):
+            asked.append(e.value)
+            blocks.append(C.create_string_buffer(n))
+            out._obj.value = C.addressof(blocks[-1])
+            return 0
+
+        @staticmethod
+        def mi_host_alloc(n, out):
+            raise AssertionError("a block under the thread's device")
+
+        mi_host_free = mi_engine_destroy = staticmethod(lambda p: None)
+        mi_forward = mi_forward_segments = staticmethod(lambda *a: 0)
+
+    monkeypatch.setattr(E.L, "lib", lambda: Fake)
+    pool = E._ResultPool()
+    monkeypatch.setattr(E, "_results", pool)
+    eng = E.Engine.__new__(E.Engine)
+    eng._h, eng._kvs, eng.desc = C.c_void_p(77), set(), types.SimpleNamespace(vocab_size=70000)
+    pool.engine_opened()
+    kv = types.SimpleNamespace(offsets=[0, 0], ensure=lambda n: None, _h=None)
+    a, b = eng.forward(np.zeros((2, 3), np.int32), kv), eng.forward_segments(kv, [0, 1], [[1], [2, 3]], [0])
+    assert a.shape == (2, 70000) and b.shape == (1, 70000) and asked == [77, 77]
+    eng.close()
