@@ -8,6 +8,8 @@ libmi355_decode.so; PyTorch is used only to hold host/device tensors on their wa
 from __future__ import annotations
 
 import ctypes as C
+import mmap
+import os
 import threading
 import weakref
 from typing import Dict, Iterable, Optional, Sequence, Tuple
@@ -51,15 +53,21 @@ class _ResultPool:
     """Pinned host memory behind the large arrays that ``forward`` returns: an array owns its block until it is dropped, then the block
     serves the next one.  At most ``MAX_BYTES`` are out or kept at any time (a caller that collects more gets ordinary memory); what is
     kept is given back when the last engine is closed.  One pool per process: blocks belong to no device or stream, and a block is
-    handed out again only when nobody can see its array any more."""
+    handed out again only when nobody can see its array any more.
+
+    A forked child does not inherit pinned pages (the driver's mapping is VM_DONTCOPY): it finds the arrays that were alive at the fork in
+    private memory at the same addresses, and an empty pool that never calls the library for the parent's blocks."""
 
     MIN_BYTES, MAX_BYTES = 1 << 18, 256 << 20        # below: a pageable copy is as quick
 
     def __init__(self):
         self._lock = threading.RLock()                # (re-entrant: a collection inside may drop an array)
         self._free: Dict[int, list] = {}
+        self._out: Dict[int, int] = {}                # address -> bytes, of the blocks behind arrays
         self._bytes = 0                               # out and kept
         self._engines = 0
+        self._forks = 0                               # between the process that made a block and this one
+        self._copies: list = []                       # of what is out, during a fork
 
     def engine_opened(self) -> None:
         with self._lock:
@@ -99,32 +107,52 @@ class _ResultPool:
                                                            lib.mi_host_alloc(size, C.byref(p))) != 0:
                     return np.empty(shape, dtype=np.float32)
                 self._bytes += size
+            self._out[p.value] = size
         return np.asarray(_ResultBlock(self, p, size, tuple(shape)))
 
-    def give_back(self, p, size: int) -> None:
+    def give_back(self, p, size: int, forks: int) -> None:
         with self._lock:
+            if forks != self._forks:                  # a parent's block: private memory here, the child's end frees it
+                return
+            del self._out[p.value]
             if self._engines > 0:
                 self._free.setdefault(size, []).append(p)
             else:
                 L.lib().mi_host_free(p)
                 self._bytes -= size
 
+    def before_fork(self) -> None:
+        self._lock.acquire()
+        self._copies = [(at, size, C.string_at(at, size)) for at, size in self._out.items()]
+
+    def after_fork(self, child: bool) -> None:
+        if child:
+            libc = C.CDLL(None)
+            libc.mmap.restype, libc.mmap.argtypes = C.c_void_p, [C.c_void_p, C.c_size_t, C.c_int, C.c_int, C.c_int, C.c_long]
+            for at, size, data in self._copies:       # (MAP_FIXED: nothing else can be where the parent's block was)
+                if libc.mmap(at, size, mmap.PROT_READ | mmap.PROT_WRITE, mmap.MAP_PRIVATE | mmap.MAP_ANONYMOUS | 0x10, -1, 0) == at:
+                    C.memmove(at, data, size)
+            self._free, self._out, self._bytes, self._engines, self._forks = {}, {}, 0, 0, self._forks + 1
+        self._copies = []
+        self._lock.release()
+
 
 class _ResultBlock:
     """What an array of the pool keeps alive."""
 
     def __init__(self, pool: _ResultPool, p, size: int, shape):
-        self._pool, self._p, self._size = pool, p, size
+        self._pool, self._p, self._size, self._forks = pool, p, size, pool._forks
         self.__array_interface__ = {"shape": shape, "typestr": "<f4", "data": (p.value, False), "version": 3}
 
     def __del__(self):
         try:
-            self._pool.give_back(self._p, self._size)
+            self._pool.give_back(self._p, self._size, self._forks)
         except Exception:                             # (interpreter shutdown)
             pass
 
 
 _results = _ResultPool()
+os.register_at_fork(before=lambda: _results.before_fork(), after_in_parent=lambda: _results.after_fork(False), after_in_child=lambda: _results.after_fork(True))
 
 
 class SampleArgs:

@@ -295,3 +295,57 @@ def test_result_blocks_are_made_under_the_engine_s_device(monkeypatch):
     a, b = eng.forward(np.zeros((2, 3), np.int32), kv), eng.forward_segments(kv, [0, 1], [[1], [2, 3]], [0])
     assert a.shape == (2, 70000) and b.shape == (1, 70000) and asked == [77, 77]
     eng.close()
+
+
+def test_results_are_readable_in_a_forked_child(monkeypatch):
+    """Pinned pages are not copied to a forked child (VM_DONTCOPY): an array that is alive at the fork is to hold its values there all the
+    same, writes of the child stay its own, and neither dropping it nor ending the pool there reaches the library."""
+    import ctypes as C
+    import mmap
+    import os
+
+    from mlx_parallm_amd import engine as E
+
+    libc = C.CDLL(None)
+    libc.mmap.restype, libc.mmap.argtypes = C.c_void_p, [C.c_void_p, C.c_size_t, C.c_int, C.c_int, C.c_int, C.c_long]
+    libc.madvise.argtypes, libc.munmap.argtypes = [C.c_void_p, C.c_size_t, C.c_int], [C.c_void_p, C.c_size_t]
+    size, parent, live = {}, os.getpid(), []
+
+    class Fake:
+        @staticmethod
+        def mi_host_alloc(n, out):
+            out._obj.value = libc.mmap(None, n, mmap.PROT_READ | mmap.PROT_WRITE, mmap.MAP_PRIVATE | mmap.MAP_ANONYMOUS, -1, 0)
+            assert libc.madvise(out._obj.value, n, 10) == 0                  # MADV_DONTFORK
+            size[out._obj.value] = n
+            return 0
+
+        @staticmethod
+        def mi_host_free(p):
+            if os.getpid() != parent:
+                os._exit(3)
+            libc.munmap(p.value, size.pop(p.value))
+
+    monkeypatch.setattr(E.L, "lib", lambda: Fake)
+    pool = E._ResultPool()
+    monkeypatch.setattr(E, "_results", pool)
+    pool.engine_opened()
+    live = [pool.empty((300, 1000)), pool.empty((4, 70000))]
+    pool.empty((500, 1000))                                                  # kept, shown by nobody
+    for i, a in enumerate(live):
+        a[:] = np.arange(a.size, dtype=np.float32).reshape(a.shape) + i
+    pid = os.fork()
+    if pid == 0:
+        code = 4
+        try:
+            ok = all(np.array_equal(a.ravel(), np.arange(a.size, dtype=np.float32) + i) for i, a in enumerate(live))
+            live[0][:] = -1.0
+            pool.engine_closed()
+            del a, live[:]
+            code = 0 if ok else 5
+        finally:
+            os._exit(code)
+    assert os.waitpid(pid, 0)[1] == 0
+    assert live[0][0, 1] == 1.0 and len(size) == 3
+    del a, live[:]
+    pool.engine_closed()
+    assert not size and pool._bytes == 0 and not pool._out
