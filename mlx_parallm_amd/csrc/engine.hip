@@ -320,9 +320,9 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
     // the decode step of a batch of 9..128 sequences (int4 / int8 weights: any batch up to 128): W is streamed once, K split over workgroups (gemm_skinny.hip).
     // Also a prefill of up to 128 rows in all (a short prompt, a few short prompts): at that size the op is a weight
     // stream, not a GEMM -- measured on Mistral-7B bf16, one prompt of 64 tokens: 13.0 ms through the 128 x 128 tile GEMM
-    // (32 workgroups for N = 4096) against ~6 ms here.  The price: a sequence's prefill arithmetic (summation order) now
-    // depends on whether the whole call is above or below 128 rows; inside one regime rows stay bit-independent of
-    // their neighbours (tests/test_gpu_fullsize.py).
+    // (32 workgroups for N = 4096) against ~6 ms here.  The price: a sequence's prefill arithmetic (summation order)
+    // depends on the SHAPE of its call (above or below 128 rows; how K, and the attention's keys, are split).  In calls of one
+    // shape a row's bits depend on nothing of its neighbours (tests/test_gpu_fullsize.py, test_gpu_engine.py).
     Prof pr(e, prof);
     // (float32 activations: the split-K kernel neither leaves nor takes the row statistics -- always the norm launch)
     c.M = (int)rows;

@@ -257,6 +257,14 @@ size_t attention_prefill_part_floats(const AttnShape& s, int slices);
 int attention_prefill_tiles(const AttnShape& s);
 int launch_attention_prefill(const AttnCall& c, hipStream_t st);
 
+// Prefill attention: over how many of at most `most` workgroups the keys of a row that reaches `keys` of them are split (device: per row;
+// host: the longest row's): two blocks each at least.
+constexpr int PREFILL_KEY_BLOCK = 32;
+__host__ __device__ inline int prefill_row_slices(int most, int keys) {
+  const int pairs = (keys + PREFILL_KEY_BLOCK - 1) / PREFILL_KEY_BLOCK / 2, n = pairs < most ? pairs : most;
+  return n < 1 ? 1 : n;
+}
+
 // Decode attention: over how many of at most `most` workgroups a row's `keys` cached keys are split (device: per row; host: the longest
 // row's).  A split costs its publication and its share of the join, so a workgroup gets a full round of 256 keys where four splits
 // do not suffice; below that four splits of 96 keys and more still beat fewer (16-bit caches, rocprof: 330 keys, 1 row x 8 heads

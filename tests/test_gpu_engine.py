@@ -704,6 +704,27 @@ def test_a_chunk_behind_cached_tokens_splits_its_keys(tiny_dirs, name, kvd):
     eng.close()
 
 
+@pytest.mark.parametrize("kvd", ["model", "float32"])
+def test_a_chunk_s_bits_do_not_depend_on_its_neighbours_caches(tiny_dirs, kvd):
+    """Prefill attention with split keys: a row's slices follow from the call's shape and its own keys.  The same chunk behind the same
+    cache, next to a neighbour with less and with far more in its cache (one to seven slices of two blocks): the same bits."""
+    model, ref, cfg = _load_pair(tiny_dirs, "qwen3_bf16")
+    eng = model.engine
+    toks = RNG.integers(3, cfg["vocab_size"], size=(2, 480)).astype(np.int32)
+    for off, L in [(20, 16), (130, 17), (300, 2)]:
+        got = []
+        for other in (0, off, 440):
+            kv = eng.new_kv(2, capacity=512, kv_dtype=kvd)
+            for row, n in ((0, off), (1, other)):
+                if n:
+                    eng.step_wait(eng.step_enqueue_rows(kv, [row], toks[row:row + 1, :n], SampleArgs(temp=0.0)), 1)
+            assert list(kv.offsets) == [off, other]
+            got.append(eng.forward(np.stack([toks[0, off:off + L], toks[1, :L]]), kv, all_positions=True)[0].copy())
+            kv.close()
+        assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2]), (off, L)
+    eng.close()
+
+
 def test_converted_checkpoint_and_lora_hot_swap(tiny_dirs, tmp_path):
     """a directory written by convert(quantize=True) loads and matches the oracle on the same
     files; weight_updater swaps adapters on the live engine (adapters.safetensors + config, then adapter.npz)."""
