@@ -111,6 +111,13 @@ int mi_op_rope_append(const mi_op_attn_shape* s, const void* qkv, void* q_out, v
                       const float* cos_tab, const float* sin_tab, int max_pos);
 int mi_op_attention(const mi_op_attn_shape* s, const void* q, const void* kcache, const void* vcache,
                     const int32_t* offsets, void* out, float scale, int nsplit, float* partial);
+/* causal prefill attention on the matrix cores alone (L > 1), its keys split over up to 16 workgroups, `nsplit` for the longest row and
+ * fewer for rows of few keys.  partial: ceil(L / 16) x B x Hkv x nsplit x Hq / Hkv x 64 x (D / 16 + 1) x 4 floats, counters:
+ * ceil(L / 16) x B x Hkv ints, zero before and after (both may be NULL for nsplit 1).  btab: block table of a paged cache
+ * ([row][bt_stride], blocks of 2^bs_shift tokens), NULL: contiguous. */
+int mi_op_attention_prefill(const mi_op_attn_shape* s, const int32_t* btab, int bt_stride, int bs_shift, const void* q,
+                            const void* kcache, const void* vcache, const int32_t* offsets, void* out, float scale,
+                            int nsplit, float* partial, int32_t* counters);
 /* fused decode attention (L == 1): q/k norm + RoPE + append + split-KV attention + combine.
  * counters: [B*Hkv] zero-initialised ints.  variant 0: MFMA kernel where it applies (16-bit caches,
  * head_dim % 32 == 0; float32 caches, head_dim 64 / 128), 1: VALU kernel (2: the MFMA kernel in its twelve-wave form,

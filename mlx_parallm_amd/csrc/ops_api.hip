@@ -209,6 +209,18 @@ int mi_op_attention(const mi_op_attn_shape* s, const void* q, const void* kcache
   return finish();
 }
 
+int mi_op_attention_prefill(const mi_op_attn_shape* s, const int32_t* btab, int bt_stride, int bs_shift, const void* q,
+                            const void* kcache, const void* vcache, const int32_t* offsets, void* out, float scale,
+                            int nsplit, float* partial, int32_t* counters) {
+  if (!s) return fail(MI_ERR_INVALID, "null argument");
+  MI_TRY(ready());
+  AttnCall ac{to_shape(s), q, kcache, vcache, offsets, out, scale, nsplit, partial, 0, (int*)counters};
+  ac.s.btab = btab; ac.s.bt_stride = bt_stride; ac.s.bs_shift = bs_shift;
+  if (s->L < 2) return fail(MI_ERR_INVALID, "mi_op_attention_prefill: L > 1");
+  MI_TRY(launch_attention_prefill(ac, nullptr));
+  return finish();
+}
+
 int mi_op_attention_decode(const mi_op_attn_shape* s, const void* qkv, void* kcache, void* vcache,
                            const int32_t* offsets, const void* q_norm_w, const void* k_norm_w, float eps,
                            const float* cos_tab, const float* sin_tab, void* out, float scale, int rnd_out,

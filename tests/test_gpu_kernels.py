@@ -369,6 +369,64 @@ def test_prefill_attention_many_blocks(act, Hq, Hkv, D):
                 assert close_frac(got[b, t], o[0, :, 0], act, atol=1e-3) <= 0.02, (b, t)
 
 
+@pytest.mark.parametrize("act", ["bfloat16", "float16", "float32"])
+@pytest.mark.parametrize("Hq,Hkv,D", [(8, 2, 128), (4, 4, 64), (5, 1, 32), (8, 1, 128), (10, 2, 128)])
+def test_prefill_attention_with_split_keys(act, Hq, Hkv, D):
+    """join_slices: the keys of a tile over 2 .. 16 workgroups against one, every output, rows with their own number of slices (3, 16 and
+    5 at most), tiles with fewer blocks than slices (the first row's), a call whose last tile is ragged; the tickets come back to
+    zero, a paged cache gives the contiguous one's bits.  Bounds: P and V enter in two 16-bit terms, 2^-16 of a product at most, in
+    either result, so float32 outputs lie within 2^-15 of the largest value; 16-bit ones are one ulp apart where that crosses a
+    rounding boundary."""
+    if act == "float32" and D % 64 != 0:
+        pytest.skip("float32 caches: the matrix-core prefill kernels take head_dim 64 / 128")
+    B, L_, cap, bs = 3, 200, 1104, 16
+    offs = [0, 900, 97]
+    rng = np.random.default_rng(99 + D + Hq)
+    kc, vc = (round_to(rng.standard_normal((B, Hkv, cap, D)).astype(np.float32), act) for _ in range(2))
+    q = round_to(rng.standard_normal((B, L_, Hq, D)).astype(np.float32), act)
+    s = attn_shape(B, L_, Hq, Hkv, D, act, act, 0, cap)
+    q_d, kc_d, vc_d, off_d = dev(q.reshape(B * L_, Hq * D), act), dev(kc, act), dev(vc, act), dev_i32(offs)
+    nblk = B * cap // bs
+    place = rng.permutation(nblk).astype(np.int32)                 # block i of the rows in order -> its place in the arena
+    def arena(x):
+        a = np.empty((nblk, Hkv, bs, D), np.float32)
+        a[place] = x.reshape(B, Hkv, cap // bs, bs, D).transpose(0, 2, 1, 3, 4).reshape(nblk, Hkv, bs, D)
+        return dev(a, act)
+    kp_d, vp_d, btab = arena(kc), arena(vc), dev_i32(place)
+    tiles, G = (L_ + 15) // 16 * B * Hkv, Hq // Hkv
+    part = torch.full((tiles * 16 * G * 64 * (D // 16 + 1) * 4,), float("nan"), dtype=torch.float32, device="cuda")
+    ctr = torch.zeros((tiles,), dtype=torch.int32, device="cuda")
+
+    def run(nsplit, paged):
+        out = torch.full((B * L_ + 1, Hq * D), 7.0, dtype=q_d.dtype, device="cuda")
+        torch.cuda.synchronize()
+        L.check(L.lib().mi_op_attention_prefill(C.byref(s), ptr(btab) if paged else None, cap // bs, 4, ptr(q_d), ptr(kp_d if paged else kc_d),
+                                                ptr(vp_d if paged else vc_d), ptr(off_d), ptr(out), float(D ** -0.5), nsplit, ptr(part), ptr(ctr)))
+        assert not ctr.cpu().numpy().any() and bool((out[-1] == 7.0).all())
+        return out[:-1]
+
+    one = run(1, False)
+    for nsplit in (2, 3, 9, 15, 16):
+        got = run(nsplit, False)
+        assert torch.equal(got, run(nsplit, True))
+        d, v = (got.float() - one.float()).abs(), one.float().abs()
+        assert float(d.max()) > 0.0                                # (another order of sums: the keys are split)
+        if act == "float32":
+            assert float(d.max()) <= 2.0 ** -15 * float(np.abs(vc).max()), (nsplit, float(d.max()))
+        else:
+            ulp = 2.0 ** -7 if act == "bfloat16" else 2.0 ** -10
+            assert bool((d <= ulp * v.clamp_min(ulp)).all()) and float((d > 0).float().mean()) <= 0.02, (nsplit, float(d.max()), float((d > 0).float().mean()))
+    got = host(got).reshape(B, L_, Hq, D)
+    for b in range(B):
+        for t in (0, 15, 16, 33, L_ - 1):
+            n = offs[b] + t + 1
+            o, _ = ref_model.sdpa(q[b:b + 1, t:t + 1].transpose(0, 2, 1, 3), kc[b:b + 1, :, :n], vc[b:b + 1, :, :n], D ** -0.5, None, act, act)
+            if act == "float32":
+                assert np.allclose(got[b, t], o[0, :, 0], rtol=1e-4, atol=2e-5), (b, t)
+            else:
+                assert close_frac(got[b, t], o[0, :, 0], act, atol=1e-3) <= 0.02, (b, t)
+
+
 @pytest.mark.parametrize("variant", [0, 1])
 @pytest.mark.parametrize("act", ["bfloat16", "float16", "float32"])
 @pytest.mark.parametrize("Hq,Hkv,D,qk_norm", [(8, 2, 128, False), (5, 1, 128, True), (4, 4, 64, True), (16, 2, 32, False)])
