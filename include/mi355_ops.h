@@ -126,6 +126,9 @@ int mi_op_attention_decode(const mi_op_attn_shape* s, const void* qkv, void* kca
                            const int32_t* offsets, const void* q_norm_w, const void* k_norm_w, float eps,
                            const float* cos_tab, const float* sin_tab, void* out, float scale, int rnd_out,
                            int nsplit, float* partial, int32_t* counters, int variant, int iters, float* avg_ms);
+/* splits that a decode step's attention is launched with: `groups` (rows x kv heads) whose rows have `keys` cached keys of kv_dtype, on
+ * ncu compute units (no device needed) */
+int mi_op_attention_decode_splits(int ncu, int groups, int keys, int kv_dtype);
 int mi_op_sample(float* logits, int B, int V, float temperature, float top_p, const float* uniforms,
                  int top_logprobs, int32_t* tokens_out, float* logprob_out, float* prob_row0_out,
                  int32_t* topk_ids, float* topk_logprobs, float* row_stats);

@@ -1103,6 +1103,31 @@ bool attention_decode_supported(const AttnShape& s) {
   return s.D == 32 || s.D == 64 || s.D == 128;
 }
 
+// One workgroup per CU (8 waves, 84 KiB of LDS: a second one does not fit), so a launch of more runs in rounds.
+// At most half the CUs have a (row, kv head): as many splits as fill ONE round (16-bit caches, 12 rows x 8 heads x 2047 keys: 2 splits 19.7
+// us, 3 / 4 29.2 / 25.6; 6 rows x 4100: 5 / 6 20.2 / 29.5), but four for five of 16-bit caches: the join takes four at a time, and the
+// fifth's trip costs more than its share saves (4 / 5 splits, 1 row x 1400 keys 9.9 / 10.1, 6 x 2047 13.8 / 14.5; float32 16.3 / 15.2, 21.8 / 21.9).  Above that the cheapest by the rounds of ncu workgroups, in keys of a full
+// round: one that is filled to u costs max(0.49 + 0.2 u, u) of a full one -- a workgroup alone streams about twice as fast as one of 256 --,
+// a round's start and end 180 keys, the join 100 (float32 caches: half, a key is twice the bytes).  33 rows x 8 heads x 4100 keys
+// in 1 / 2 / 3 / 4 splits: 135 / 119 / 114 / 113 us (the last round of one split has 8 workgroups), float32 273 / 230 / 219 / 210; 1000 keys 33.9 /
+// 36.9 / 37.8; 17 rows x 8000 in 1 / 2 / 3: 108 / 135 / 101; 56 rows x 4100 in 1 / 2 / 3: 154 / 169 / 176.
+int attention_decode_splits(int ncu, int groups, int keys, bool f32) {
+  if (2 * groups <= ncu) {
+    const int n = decode_row_splits(std::min(ncu / groups, 16), keys);
+    return n == 5 && !f32 ? 4 : n;
+  }
+  const double round = f32 ? 90 : 180, join = f32 ? 50 : 100;
+  double best = 0;
+  int pick = 1;
+  for (int n = 1; n <= decode_row_splits(16, keys); ++n) {
+    const int full = groups * n / ncu, rest = groups * n % ncu;
+    const double u = (double)rest / ncu, part = rest ? std::max(0.49 + 0.2 * u, u) : 0.0;
+    const double cost = (full + part) * keys / n + (full + (rest > 0)) * round + (n > 1) * join;
+    if (n == 1 || cost < best) { best = cost; pick = n; }
+  }
+  return pick;
+}
+
 int launch_attention_decode(const AttnDecodeCall& c, hipStream_t st) {
   const AttnShape& s = c.s;
   if (!attention_decode_supported(s)) return fail(MI_ERR_UNSUPPORTED, "attention_decode: shape / dtype not supported");

@@ -679,9 +679,8 @@ size_t kv_layer_elems(const mi_kv* kv, const mi_model_desc& d) {
                    : (size_t)kv->B * d.num_kv_heads * kv->cap * d.head_dim;
 }
 
-// Splits of the decode attention: one workgroup per CU (8 waves, 84 KiB of LDS: a second one does not fit, so a launch of more runs in
-// rounds -- 8 rows x 8 heads, 1024 float32 keys: 4 splits 20 us, 5 splits 30; 8 rows at 8192 16-bit keys: 4 splits 43 us, 5 / 8 / 9 57 /
-// 48 / 58).  Rows shorter than the longest take fewer splits (decode_row_splits), so a call counts as its keys over the longest row's.
+// Splits of the decode attention.  Rows shorter than the longest take fewer (decode_row_splits), so a call counts as its keys over the
+// longest row's.
 int choose_nsplit(const mi_kv* kv, int B, int Hkv, int L, const int32_t* rows = nullptr) {
   if (L != 1) return 1;
   int mx = 1;
@@ -689,8 +688,7 @@ int choose_nsplit(const mi_kv* kv, int B, int Hkv, int L, const int32_t* rows = 
   for (int b = 0; b < B; ++b) { const int k = std::max(1, kv->h_off[rows ? rows[b] : b]); mx = std::max(mx, k); sum += k; }
   const int alike = (int)((sum + mx - 1) / mx);
   static const int ns_env = getenv("MI_ATTN_NSPLIT") ? atoi(getenv("MI_ATTN_NSPLIT")) : 0;   // A/B
-  const int fill = ns_env > 0 ? ns_env : gemv_cu_count() / (Hkv * alike);
-  return decode_row_splits(std::min(fill, 16), mx);
+  return ns_env > 0 ? decode_row_splits(std::min(ns_env, 16), mx) : attention_decode_splits(gemv_cu_count(), Hkv * alike, mx, kv->dtype == MI_F32);
 }
 
 // prefill attention (L > 1): the keys split over workgroups where the query tiles alone leave the chip idle

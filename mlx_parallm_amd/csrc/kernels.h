@@ -274,6 +274,8 @@ __host__ __device__ inline int decode_row_splits(int most, int keys) {
   const int want = four > full ? four : full;
   return want < 1 || most < 1 ? 1 : want < most ? want : most;
 }
+// .. and of how many a call is launched, `groups` = rows like the longest x kv heads (attn_decode.hip)
+int attention_decode_splits(int ncu, int groups, int keys, bool f32);
 // fused decode step (L == 1): q/k norm + RoPE + KV append + split-KV attention + combine
 struct AttnDecodeCall {
   AttnShape s;             // s.rnd = logical rounding of q / k after norm and RoPE

@@ -247,6 +247,11 @@ int mi_op_attention_decode(const mi_op_attn_shape* s, const void* qkv, void* kca
   return finish();
 }
 
+int mi_op_attention_decode_splits(int ncu, int groups, int keys, int kv_dtype) {
+  if (ncu < 1 || groups < 1 || keys < 0) return fail(MI_ERR_INVALID, "mi_op_attention_decode_splits: counts");
+  return attention_decode_splits(ncu, groups, keys, kv_dtype == MI_F32);
+}
+
 int mi_op_sample(float* logits, int B, int V, float temperature, float top_p, const float* uniforms,
                  int top_logprobs, int32_t* tokens_out, float* logprob_out, float* prob_row0_out,
                  int32_t* topk_ids, float* topk_logprobs, float* row_stats) {

@@ -349,3 +349,25 @@ def test_results_are_readable_in_a_forked_child(monkeypatch):
     del a, live[:]
     pool.engine_closed()
     assert not size and pool._bytes == 0 and not pool._out
+
+
+@pytest.mark.parametrize("f32", [False, True])
+def test_decode_attention_splits(f32):
+    """How many splits a decode step's attention is launched with: one round of workgroups where the rows leave half the chip idle; above
+    that, the rounds that would otherwise end nearly empty (33 to 40 rows, 17 rows of long contexts) are cut finer and full ones are not."""
+    from mlx_parallm_amd import _lib as L
+
+    def splits(rows, keys):
+        return L.lib().mi_op_attention_decode_splits(256, rows * 8, keys, L.MI_F32 if f32 else L.MI_BF16)
+
+    assert [splits(b, 8000) for b in (1, 2, 4, 6, 8, 10, 12, 16)] == [16, 16, 8, 5 if f32 else 4, 4, 3, 2, 2]
+    assert [splits(1, k) for k in (0, 1, 96, 97, 300, 1279, 1280)] == [1, 1, 1, 2, 4, 4, 5 if f32 else 4]
+    for b in (20, 24, 28, 31, 32, 56, 60, 64, 96, 128):                 # a full last round, or short rows: one split
+        assert splits(b, 1000) == 1 and (b in (20,) or splits(b, 4100) == 1), b
+    assert all(splits(b, 500) == 1 for b in range(17, 129))
+    for b in (33, 34, 36, 40):                                          # 8 to 64 of 256 workgroups in the last round
+        assert 2 <= splits(b, 4100) <= 6 and 2 <= splits(b, 2047) <= 4, b
+    assert splits(17, 8000) >= 3
+    for b in range(1, 129):
+        for keys in (0, 1, 95, 700, 5000, 32000):
+            assert 1 <= splits(b, keys) <= 16
