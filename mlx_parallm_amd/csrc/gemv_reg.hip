@@ -142,8 +142,10 @@ __device__ __forceinline__ u32x4 ror8(u32x4 v) {
   return r;
 }
 
-// KW: k per wave, at most (a wave with less has zero fragments at the end)
-template <typename AT, int QB, bool SW, bool NORM, int KW>
+// KW: k per wave, at most; FULL: every wave has that.  Otherwise a wave with less loads its last block again, and skips it -- zero
+// fragments would do for finite weights, but 0 x inf is NaN.  The skip's branches cost 0.1 to 0.5 us a launch (o of Mistral-7B in bf16 7.9 -> 8.4),
+// so the full shares have none.
+template <typename AT, int QB, bool SW, bool NORM, int KW, bool FULL>
 __global__ __launch_bounds__(512, 2) void gemv_reg_kernel(const RegParams p) {
   using B = Blk<QB>;
   constexpr int NW = 8, NA = SW ? 2 : 1, NB = KW / B::K, NP = KW / 64, PB = B::F / 2;     // pairs of fragments: in all, per block
@@ -217,7 +219,6 @@ __global__ __launch_bounds__(512, 2) void gemv_reg_kernel(const RegParams p) {
   f32x4 sx[NP];
 #pragma unroll
   for (int q = 0; q < NP; ++q) {
-    if (q / PB >= nb) xf[q] = u32x4{0u, 0u, 0u, 0u};
     if constexpr (QB == 4) xf[q] = nibble_order(xf[q]);
     sx[q] = mfma16<AT>(xf[q], ones16<AT>(), f32x4{0.f, 0.f, 0.f, 0.f});
     sx[q] = mfma16<AT>(ror8(xf[q]), ones16<AT>(), sx[q]);
@@ -236,7 +237,7 @@ __global__ __launch_bounds__(512, 2) void gemv_reg_kernel(const RegParams p) {
       for (int q = 0; q < PB; ++q) { f[2 * q] = xf[i * PB + q]; f[2 * q + 1] = ror8(xf[i * PB + q]); }
 #pragma unroll
       for (int a = 0; a < NA; ++a) {
-        mul_blk<AT, QB>(acc[a], wb[a][i], f, sx + i * PB);
+        if (FULL || i < nb) mul_blk<AT, QB>(acc[a], wb[a][i], f, sx + i * PB);      // (uniform)
         if constexpr (decltype(more)::value) {
           __builtin_amdgcn_sched_barrier(0);
           issue(a, i, tile + step);
@@ -325,7 +326,7 @@ __device__ __forceinline__ void unpack_raw(const RawX<AT, X32>& r, f32x2 (&e)[4]
   }
 }
 
-template <typename AT, bool X32, bool GU, bool NORM, int KW>
+template <typename AT, bool X32, bool GU, bool NORM, int KW, bool FULL>       // (KW, FULL: as gemv_reg_kernel)
 __global__ __launch_bounds__(512, 2) void gemv_dense_kernel(const RegParams p) {
   using XT = typename std::conditional<X32, float, AT>::type;
   constexpr int NW = 8, NP = KW / 32, NQ = NP / 2, T = X32 ? 3 : 1, NC = X32 ? 3 : 2;      // products, pairs of them, terms, chains of sums
@@ -336,7 +337,7 @@ __global__ __launch_bounds__(512, 2) void gemv_dense_kernel(const RegParams p) {
   const int step = gridDim.x;
 
   u32x4 wb[NP];
-  auto pair_at = [&](int q) { return q0 + min(q, max(nq - 1, 0)); };            // (past the last: the last one again, times zero)
+  auto pair_at = [&](int q) { return q0 + min(q, max(nq - 1, 0)); };            // (past the last: the last one again, unused)
   auto issue = [&](int i, int tile) {
     wb[i] = __builtin_nontemporal_load((const u32x4*)((const char*)p.w + ((size_t)tile * p.nblk * 2 + pair_at(i >> 1) * 2 + (i & 1)) * 1024 + lane * 16));
   };
@@ -412,9 +413,6 @@ __global__ __launch_bounds__(512, 2) void gemv_dense_kernel(const RegParams p) {
         xf[0][q][j] = raw[q].v[0][j];
       }
     }
-#pragma unroll
-    for (int t = 0; t < T; ++t)
-      if (q >= nq) xf[t][q] = u32x4{0u, 0u, 0u, 0u};
   }
 
   int buf = 0;
@@ -425,11 +423,13 @@ __global__ __launch_bounds__(512, 2) void gemv_dense_kernel(const RegParams p) {
     for (int a = 0; a < NC; ++a) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
+      if (FULL || i < 2 * nq) {                       // (uniform)
 #pragma unroll
-      for (int t = 0; t < T; ++t) {
-        const u32x4 f = (i & 1) ? ror8(xf[t][i >> 1]) : xf[t][i >> 1];
-        f32x4& a = acc[X32 ? t : i & 1];
-        a = mfma16<AT>(f, wb[i], a);
+        for (int t = 0; t < T; ++t) {
+          const u32x4 f = (i & 1) ? ror8(xf[t][i >> 1]) : xf[t][i >> 1];
+          f32x4& a = acc[X32 ? t : i & 1];
+          a = mfma16<AT>(f, wb[i], a);
+        }
       }
       if constexpr (decltype(more)::value) {
         __builtin_amdgcn_sched_barrier(0);
@@ -488,6 +488,14 @@ bool gemv_reg_supported(const LinearW& W, const GemvCall& c, size_t rows) {
   return c.ldx % 8 == 0 && (uintptr_t)c.x % 16 == 0 && (c.pro != PRO_NORM || (uintptr_t)c.norm_w % 16 == 0);
 }
 
+// f(k per wave of the instantiation, every wave has that): the smallest registers that hold a wave's blocks of bk
+template <class F>
+static int by_share(int nblk, int bk, F f) {
+  auto at = [&](auto kw) { return nblk * bk == 8 * kw ? f(kw, std::true_type{}) : f(kw, std::false_type{}); };
+  const int kw = (nblk + 7) / 8 * bk;
+  return kw <= 256 ? at(std::integral_constant<int, 256>{}) : kw <= 512 ? at(std::integral_constant<int, 512>{}) : at(std::integral_constant<int, 640>{});
+}
+
 template <typename AT, int QB>
 static int launch_reg(const RegParams& p, bool sw, hipStream_t st) {
   auto go = [&](auto kern, int grid) -> int {
@@ -495,21 +503,19 @@ static int launch_reg(const RegParams& p, bool sw, hipStream_t st) {
     MI_HIP(hipGetLastError());
     return MI_OK;
   };
-  const int nb = (p.nblk + 7) / 8, kw = nb * Blk<QB>::K, grid = std::min(p.ntiles, gemv_cu_count());
+  const int grid = std::min(p.ntiles, gemv_cu_count());
   if constexpr (QB == 4) {
     if (p.K > REG_K) {
+      const int nb = (p.nblk + 7) / 8;
       if (nb <= 8) return go(gemv_long_kernel<AT, 8>, p.ntiles);
       if (nb <= 11) return go(gemv_long_kernel<AT, 11>, p.ntiles);
       if (nb <= 14) return go(gemv_long_kernel<AT, 14>, p.ntiles);
       return go(gemv_long_kernel<AT, 17>, p.ntiles);
     }
-    if (sw) return kw <= 256 ? go(gemv_reg_kernel<AT, 4, true, true, 256>, grid) : kw <= 512 ? go(gemv_reg_kernel<AT, 4, true, true, 512>, grid)
-                             : go(gemv_reg_kernel<AT, 4, true, true, 640>, grid);
+    if (sw) return by_share(p.nblk, 128, [&](auto kw, auto full) { return go(gemv_reg_kernel<AT, 4, true, true, kw.value, full.value>, grid); });
   }
-  if (p.norm) return kw <= 256 ? go(gemv_reg_kernel<AT, QB, false, true, 256>, grid) : kw <= 512 ? go(gemv_reg_kernel<AT, QB, false, true, 512>, grid)
-                               : go(gemv_reg_kernel<AT, QB, false, true, 640>, grid);
-  return kw <= 256 ? go(gemv_reg_kernel<AT, QB, false, false, 256>, grid) : kw <= 512 ? go(gemv_reg_kernel<AT, QB, false, false, 512>, grid)
-                   : go(gemv_reg_kernel<AT, QB, false, false, 640>, grid);
+  if (p.norm) return by_share(p.nblk, Blk<QB>::K, [&](auto kw, auto full) { return go(gemv_reg_kernel<AT, QB, false, true, kw.value, full.value>, grid); });
+  return by_share(p.nblk, Blk<QB>::K, [&](auto kw, auto full) { return go(gemv_reg_kernel<AT, QB, false, false, kw.value, full.value>, grid); });
 }
 
 int launch_gemv_reg(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st) {
@@ -542,19 +548,16 @@ bool gemv_dense_supported(const LinearW& W, const GemvCall& c, size_t rows) {
 
 template <typename AT, bool X32>
 static int launch_dense(const RegParams& p, bool gu, hipStream_t st) {
-  const int kw = (p.nblk + 7) / 8 * 64, grid = std::min(p.ntiles, gemv_cu_count());
+  const int grid = std::min(p.ntiles, gemv_cu_count());
   auto go = [&](auto kern) -> int {
     hipLaunchKernelGGL(kern, dim3(grid), dim3(512), 0, st, p);
     MI_HIP(hipGetLastError());
     return MI_OK;
   };
   if constexpr (X32)
-    if (gu) return kw <= 256 ? go(gemv_dense_kernel<AT, X32, true, true, 256>) : kw <= 512 ? go(gemv_dense_kernel<AT, X32, true, true, 512>)
-                             : go(gemv_dense_kernel<AT, X32, true, true, 640>);
-  if (p.norm) return kw <= 256 ? go(gemv_dense_kernel<AT, X32, false, true, 256>) : kw <= 512 ? go(gemv_dense_kernel<AT, X32, false, true, 512>)
-                               : go(gemv_dense_kernel<AT, X32, false, true, 640>);
-  return kw <= 256 ? go(gemv_dense_kernel<AT, X32, false, false, 256>) : kw <= 512 ? go(gemv_dense_kernel<AT, X32, false, false, 512>)
-                   : go(gemv_dense_kernel<AT, X32, false, false, 640>);
+    if (gu) return by_share(p.nblk, 64, [&](auto kw, auto full) { return go(gemv_dense_kernel<AT, X32, true, true, kw.value, full.value>); });
+  if (p.norm) return by_share(p.nblk, 64, [&](auto kw, auto full) { return go(gemv_dense_kernel<AT, X32, false, true, kw.value, full.value>); });
+  return by_share(p.nblk, 64, [&](auto kw, auto full) { return go(gemv_dense_kernel<AT, X32, false, false, kw.value, full.value>); });
 }
 
 int launch_gemv_dense(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st) {

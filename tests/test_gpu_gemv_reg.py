@@ -4,13 +4,13 @@ import numpy as np
 import pytest
 import torch
 
-from oracle import ref_model
+from oracle import ref_model, ref_quant
 from oracle.numerics import matmul_nt, round_to
 
 pytestmark = pytest.mark.gpu
 
 from mlx_parallm_amd import _lib as L  # noqa: E402
-from gpu_helpers import dev, gemv_reg, host, op_linear, to_tiled  # noqa: E402
+from gpu_helpers import dev, dev_u32, gemv_reg, host, op_linear, to_tiled  # noqa: E402
 from test_gpu_kernels import _assert_close  # noqa: E402
 from test_gpu_skinny import KINDS, _weight  # noqa: E402
 
@@ -134,3 +134,31 @@ def test_dense_swiglu_on_interleaved_rows(M, I, K):
     want = y[:, :I] / (1.0 + np.exp(-y[:, :I])) * y[:, I:]
     assert np.all(host(out)[M:] == 7.0)
     _assert_close(host(out)[:M], want, "float32", scale=float(np.abs(y).max()) ** 2)
+
+
+@pytest.mark.parametrize("act,kind", [("bfloat16", "bf16"), ("float16", "f16"), ("bfloat16", "q4_bf16"), ("bfloat16", "q8_bf16")])
+@pytest.mark.parametrize("K", [256, 1152, 2048, 2176])      # waves without a block, with one less than others, with fewer than registers, full
+def test_an_infinite_weight_stays_in_its_own_products(act, kind, K):
+    """A wave with fewer blocks than its registers hold loads its last one again: that copy must not enter the sums, where zero times
+    infinity is NaN.  One infinite weight (quantised: bias, i.e. a group of them) in every block of one output row in turn: the row's
+    outputs are infinite with the sign of x there (of the sum of x over the group), the others finite."""
+    rng = np.random.default_rng(K)
+    for at in range(7, K, 64):
+        if kind.startswith("q"):
+            packed, scales, biases = ref_quant.quantize(round_to(rng.standard_normal((32, K)).astype(np.float32), act), 64, int(kind[1]), act)
+            biases[5, at // 64] = np.inf
+            keep = [dev_u32(packed), dev(scales, act), dev(biases, act)]
+        else:
+            w = round_to(rng.standard_normal((32, K)).astype(np.float32), act)
+            w[5, at] = np.inf
+            keep = [dev(w, act)]
+        ol = op_linear(kind, 32, K, *keep)
+        assert to_tiled(ol, keep)
+        x = round_to(np.abs(rng.standard_normal((3, K))).astype(np.float32) + 0.5, act)
+        x[1] *= -1.0
+        xd = dev(x, act)
+        out = torch.zeros((3, 32), dtype=torch.float32, device="cuda")
+        gemv_reg(ol, xd, 3, act, epi=L.EPI_STORE_F32, out=out, ldo=32)
+        got = host(out)
+        assert np.array_equal(got[:, 5], [np.inf, -np.inf, np.inf]), (at, got[:, 5])
+        assert np.isfinite(np.delete(got, 5, 1)).all(), at
