@@ -1253,7 +1253,7 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
     MI_TRY(launch_dequant_q4_hilo(W, scratch, st));
     p.w = scratch; p.K = 2 * W.K; p.kw = 2 * W.K;
   }
-  const bool x32 = c.act == MI_F32;        // c.x is the [hi | mid | lo] bf16 image of launch_split3_rows, c.ldx = 3 K
+  const bool x32 = c.act == MI_F32;        // c.x is the bf16 image of launch_split3_rows, c.ldx its terms x the true K
   if (x32) {
     // c.kx > 0: W is the persistent [hi | lo] bf16 copy of an f16 matrix (2 kx columns, launch_f16_to_hilo) -- the same
     // walk as over an int4 matrix's on-the-fly [hi | lo] copy: x = [hi | mid | lo] (3 kx) against W (2 kx) over 6 kx steps
@@ -1262,7 +1262,8 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
     if (hilo && (W.K != 2 * c.kx || W.wk != WK_BF16)) return fail(MI_ERR_INVALID, "gemm_prefill: a [hi | lo] matrix has 2 kx bf16 columns");
     const bool pair = wk_is_quant(W.wk) || hilo;     // W itself is a [hi | lo] pair: 3 x-terms against 2 W-terms meet over 6 kt steps
     const int terms = c.ldx == kt ? 1 : c.ldx == 2 * kt ? 2 : 3;
-    if (c.ldx != terms * kt || (pair && terms == 2))
+    // (one term: values that are bf16 already, i.e. the rounded call of layer 0 -- any other row of stride K is one nobody has split)
+    if (c.ldx != terms * kt || (pair && terms == 2) || (terms == 1 && c.rnd != RND_BF16))
       return fail(MI_ERR_INVALID, "gemm_prefill: float32 activations must be split first (launch_split3_rows; two terms: dense bf16 weights only)");
     p.ka = terms * kt; p.K = terms * (pair ? 2 : 1) * kt; p.out32 = 1; p.rnd = c.rnd;
     if (hilo) p.kw = 2 * kt;

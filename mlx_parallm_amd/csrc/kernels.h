@@ -103,8 +103,9 @@ struct GroupedGemm {
   Glu glu;
 };
 int launch_gemm_grouped(const GroupedGemm& g, hipStream_t st);
-// float32 activations (PagedKVCache mode) in front of launch_gemm_prefill: rows of [hi | mid | lo] bf16, 3 K wide, with the
-// RMSNorm (norm_w = float32 weights, or null) applied first; then call launch_gemm_prefill with c.x = out, c.ldx = 3 K
+// float32 activations (PagedKVCache mode) in front of launch_gemm_prefill: rows of [hi | mid | lo] bf16, `terms` K wide, with the
+// RMSNorm (norm_w = float32 weights, or null) applied first; then call launch_gemm_prefill with c.x = out, c.ldx = terms x K (one
+// term: c.rnd = RND_BF16 only)
 size_t split3_bytes(size_t rows, int K);
 // rnd: logical rounding of the normed values (layer 0); values of bf16 are then one term
 int launch_split3_rows(const void* x, int ldx, const void* norm_w, float eps, void* out, int rows, int K, hipStream_t st,
