@@ -394,7 +394,7 @@ __global__ __launch_bounds__(NTHR) void gemv_short_kernel(GemvParams p) {
           float a = 0.f;
 #pragma unroll
           for (int j = 0; j < 8; ++j) a = fmaf(w8[u][r][j], xv[m][j], a);
-          a = group_sum(a);
+          a = group_sum(on ? a : 0.f);                // (a lane past K read the row's first weights: 0 x inf is NaN)
           if (gl == m) mine[r] = a;
         }
       }

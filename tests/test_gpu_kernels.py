@@ -183,6 +183,21 @@ def test_gemv_short_rows(act, kind, K, M):
     _assert_close(host(out), round_to(round_to(g * sig, act) * u, act), act)
 
 
+@pytest.mark.parametrize("act,kind,K", [("float32", "f32", 8), ("bfloat16", "bf16", 72), ("float16", "f16", 264)])      # 7 of 8, 7 of 16, 31 of 64 lanes past K
+def test_gemv_short_rows_keep_an_infinite_weight(act, kind, K):
+    """Lanes past the row's end repeat its first weights: an infinite one must not meet their zeros."""
+    w = np.abs(RNG.standard_normal((80, K)).astype(np.float32)) + 0.5
+    w[5, 3], w[46, 0] = np.inf, -np.inf
+    x = np.abs(RNG.standard_normal((3, K)).astype(np.float32)) + 0.5
+    x[1] *= -1.0
+    wd = dev(w, act)
+    out = torch.zeros((3, 80), dtype=torch.float32, device="cuda")
+    gemv(op_linear(kind, 80, K, wd), dev(x, act), 3, act, epi=L.EPI_STORE_F32, out=out, ldo=80, force_generic=1)
+    got, inf = host(out), np.float32(np.inf)
+    assert np.array_equal(got[:, 5], [inf, -inf, inf]) and np.array_equal(got[:, 46], [-inf, inf, -inf])
+    assert np.isfinite(np.delete(got, [5, 46], 1)).all()
+
+
 @pytest.mark.parametrize("M", [9, 16])
 @pytest.mark.parametrize("act,kind", [("bfloat16", "bf16"), ("bfloat16", "q4_bf16"), ("float16", "q4_f16")])
 def test_gemv_mfma_16_rows(act, kind, M):
