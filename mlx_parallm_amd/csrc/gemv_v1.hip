@@ -20,6 +20,8 @@
 
 namespace mi {
 
+int gemv_cu_count();      // gemv_mfma.hip
+
 namespace {
 
 constexpr int KC = 2048;  // K elements of x held in LDS at a time
@@ -521,8 +523,12 @@ int launch_short(const GemvParams& p, hipStream_t st) {
   const bool glu = p.epi == EPI_SWIGLU;
   const int lg = p.K <= 64 ? 8 : p.K <= 128 ? 16 : 64;
   const int items = glu ? p.pair_offset : p.N;
-  // (2048 workgroups: eight per CU, what 64-register waves allow; more rows than that are looped over)
-  const int nwg = std::min(2048, (items + 4 * (64 / lg) - 1) / (4 * (64 / lg)));
+  // More rows than the grid holds are looped over.  Four workgroups per CU: that many of the largest instantiation (MT = 8: 105 to 125
+  // registers) run at once, and each further one loads and norms x again.  1024 against 2048 workgroups, us: int4, 64 inputs, 151936 outputs,
+  // float32 rows 8.8 / 10.2 (1 row), 11.2 / 14.8 (3), 17.8 / 25.3 (8); float32 weights, 512 inputs, 16384 outputs 10.2 / 14.9, 12.2 / 15.7, 18.3 /
+  // 27.0.  Eight where the small instantiation has four rounds of loads for all of them: int4, 256 inputs, 151936 outputs 30.8 / 27.2 (1 row).
+  const int per_wg = 4 * (64 / lg), per_cu = MT == 2 && items >= 4 * (8 * gemv_cu_count()) * per_wg * (glu ? 2 : 4) ? 8 : 4;
+  const int nwg = std::min(per_cu * gemv_cu_count(), (items + per_wg - 1) / per_wg);
   auto go = [&](auto kern) -> int {
     hipLaunchKernelGGL(kern, dim3(nwg), dim3(NTHR), 0, st, p);
     MI_HIP(hipGetLastError());
