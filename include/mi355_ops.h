@@ -129,6 +129,9 @@ int mi_op_attention_decode(const mi_op_attn_shape* s, const void* qkv, void* kca
 /* splits that a decode step's attention is launched with: `groups` (rows x kv heads) whose rows have `keys` cached keys of kv_dtype, on
  * ncu compute units (no device needed) */
 int mi_op_attention_decode_splits(int ncu, int groups, int keys, int kv_dtype);
+/* 1: logits (rounded = 0) or layer 0's rounded q|k|v (1) of `rows` rows of float32 activations go to the tile GEMM, 0: 32 rows at a time to the
+ * streaming kernel.  codes: int4 weights, hilo: an f16 matrix through its [hi | lo] copy (no device needed) */
+int mi_op_gemm_prefill_pays(int codes, int hilo, int rounded, int rows);
 int mi_op_sample(float* logits, int B, int V, float temperature, float top_p, const float* uniforms,
                  int top_logprobs, int32_t* tokens_out, float* logprob_out, float* prob_row0_out,
                  int32_t* topk_ids, float* topk_logprobs, float* row_stats);

@@ -371,7 +371,10 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
     if (produce) { e->sq_valid = true; e->sq_src = c.resid; e->sq_parts = tgroups; e->sq_K = f.W.N; e->sq_ld = leave_ld; }
     return MI_OK;
   }
-  if (e->opt_prefill_gemm && gemm_prefill_supported(f.W, c, rows)) {
+  // logits and the rounded call of layer 0 in the float32-cache mode: only the rows for which the tile GEMM is ahead leave the streaming kernel
+  const bool stream32 = e->opt_skinny_gemm && c.act == MI_F32 && rows > 32 && gemm_skinny_supported(f.W, c, 32) &&
+                        (c.rnd != RND_NONE || c.epi == EPI_STORE_F32) && !gemm_prefill_pays(quant, c.kx > 0, c.rnd != RND_NONE, rows);
+  if (e->opt_prefill_gemm && !stream32 && gemm_prefill_supported(f.W, c, rows)) {
     // prefill: one MFMA tile GEMM over all rows (the RMSNorm runs as its own row-wise kernel)
     Prof pr(e, prof);
     const GemvCall c_in = c;                 // (the LoRA down-projection reads the caller's x and normalises on its own)
@@ -388,6 +391,9 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
       // The rounded call of layer 0: its input is a bf16 value, i.e. one term (8 x 1024 rows of Mistral-7B: 256 launches of the
       // streaming kernel at 32 rows each, 4.6 ms, against 0.9 ms here).
       // (Logits keep the three terms that they had on the streaming kernel.)
+      // Quantised matrices, both calls: the codes are met as [hi | lo] pairs as in every other linear of a prefill.  A pair of bf16 is
+      // w = s q + b exactly while |w| <= 2^16 ulp(s), i.e. |b| up to some 2^9 scales -- int4 groups whose mean is up to 30 of their own standard
+      // deviations, int8 groups up to 3 (quantised on the CPU and compared) -- and w to 2^-17 beyond; of f16, int4 groups to 1000.
       const int terms = c.rnd == RND_BF16 ? 1 : (e->opt_prefill_x_terms == 2 && f.W.wk == WK_BF16 && c.kx == 0 && c.rnd == RND_NONE && c.epi != EPI_STORE_F32) ? 2 : 3;
       MI_TRY(launch_split3_rows(c.x, c.ldx, c.pro == PRO_NORM ? c.norm_w : nullptr, c.eps, e->xs, (int)rows, KT, e->stream, terms, c.rnd));
       c.x = e->xs; c.ldx = terms * KT; c.pro = PRO_NONE;

@@ -1205,6 +1205,20 @@ bool gemm_prefill_supported(const LinearW& W, const GemvCall& c, size_t rows) {
   return n % 16 == 0 && (c.epi != EPI_SWIGLU || c.pair_offset % 16 == 0);
 }
 
+// Measured as whole calls of one layer and the logits of every position, float32 caches (tile GEMM minus streaming kernel, us; Mistral-7B /
+// Qwen3-14B shapes):
+//   rounded q|k|v, dense  33 rows -10 / -7, 128 -37 / -27, 1024 -421 / -656 (one term, one walk of W)
+//                  int4   96 rows +19 / +23, 128 -7 / -13, 192 -30 / -64 (the copy of W first)
+//                  f16    96 rows +28 / +25, 192 -11 / +87, 768 +127 / +328, 1024 +27 / -81, 1536 -110, 2048 -555 (three terms against two)
+//   logits, dense and f16 64 rows +40 / +351, 128 -26 / -112, 192 -6 / -163, 256 -214 / -1257; f16 +111 / +796, -40 / -231, +35 / +59, -367 / -2179:
+//                         a row of 128-row tiles costs three to four launches of 32 rows; from 256 rows the 256 x 256 tile runs
+//           int4          64 rows +323 / +2144, 512 -103 / +88, 768 +42 / -412, 1024 -341 / -760 (the copy: 4 bytes per weight; six walks)
+bool gemm_prefill_pays(bool codes, bool hilo, bool rounded, size_t rows) {
+  if (rounded) return rows > (hilo ? 1535 : codes ? 96 : 31);
+  if (codes) return rows >= 1024;
+  return rows >= 256 || (rows + 31) / 32 > 3 * ((rows + 127) / 128);
+}
+
 int launch_rmsnorm_rows(const void* x, int ldx, const void* w, void* out, int ldo, int rows, int H, float eps, int act,
                         hipStream_t st, bool block_per_row, int rnd) {
   if (H % 8 != 0) return fail(MI_ERR_UNSUPPORTED, "rmsnorm_rows: hidden size must be a multiple of 8");

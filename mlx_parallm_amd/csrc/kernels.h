@@ -83,6 +83,9 @@ int gemv_pair_grid();
 
 // prefill (many rows): MFMA tile GEMM + row-wise RMSNorm (gemm_prefill.hip)
 bool gemm_prefill_supported(const LinearW& W, const GemvCall& c, size_t rows);
+// does the tile GEMM beat 32 rows per launch of the streaming kernel?  Logits and layer 0's rounded call on float32 activations only:
+// codes = int4 weights, hilo = the [hi | lo] copy of an f16 matrix
+bool gemm_prefill_pays(bool codes, bool hilo, bool rounded, size_t rows);
 // splitk_ws / splitk_cap: float32 workspace for the K-split form of the 128 x 128 tile (few hundred rows against a narrow
 // matrix); null = never split
 int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st, void* scratch = nullptr,

@@ -252,6 +252,10 @@ int mi_op_attention_decode_splits(int ncu, int groups, int keys, int kv_dtype) {
   return attention_decode_splits(ncu, groups, keys, kv_dtype == MI_F32);
 }
 
+int mi_op_gemm_prefill_pays(int codes, int hilo, int rounded, int rows) {
+  return rows > 0 && gemm_prefill_pays(codes != 0, hilo != 0, rounded != 0, (size_t)rows) ? 1 : 0;
+}
+
 int mi_op_sample(float* logits, int B, int V, float temperature, float top_p, const float* uniforms,
                  int top_logprobs, int32_t* tokens_out, float* logprob_out, float* prob_row0_out,
                  int32_t* topk_ids, float* topk_logprobs, float* row_stats) {

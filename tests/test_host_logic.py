@@ -371,3 +371,19 @@ def test_decode_attention_splits(f32):
     for b in range(1, 129):
         for keys in (0, 1, 95, 700, 5000, 32000):
             assert 1 <= splits(b, keys) <= 16
+
+
+def test_float32_rows_leave_the_streaming_kernel_where_the_tile_pays():
+    """Logits and layer 0's rounded call on float32 activations: at decode batches and short prompts the streaming kernel is ahead (int4 logits of
+    64 rows: 2.2 ms against 4.4 on a copy of the matrix), at long ones the tile GEMM."""
+    from mlx_parallm_amd import _lib as L
+
+    def pays(rows, codes=0, hilo=0, rounded=0):
+        return bool(L.lib().mi_op_gemm_prefill_pays(codes, hilo, rounded, rows))
+
+    assert not any(pays(n, codes=1) for n in (33, 64, 130, 300, 700)) and all(pays(n, codes=1) for n in (1024, 2048, 8192))
+    for hilo in (0, 1):
+        assert [pays(n, hilo=hilo) for n in (33, 64, 96, 97, 128, 129, 192, 193, 256, 257, 300, 8192)] == [False] * 3 + [True] * 2 + [False] * 2 + [True] * 5
+    assert all(pays(n, rounded=1) for n in (32, 33, 64, 8192))
+    assert not any(pays(n, codes=1, rounded=1) for n in (33, 64, 96)) and all(pays(n, codes=1, rounded=1) for n in (128, 700))
+    assert not any(pays(n, hilo=1, rounded=1) for n in (33, 768, 1024)) and pays(2048, hilo=1, rounded=1)
