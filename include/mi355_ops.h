@@ -118,6 +118,9 @@ int mi_op_attention(const mi_op_attn_shape* s, const void* q, const void* kcache
 int mi_op_attention_prefill(const mi_op_attn_shape* s, const int32_t* btab, int bt_stride, int bs_shift, const void* q,
                             const void* kcache, const void* vcache, const int32_t* offsets, void* out, float scale,
                             int nsplit, float* partial, int32_t* counters);
+/* slices over which the engine splits the keys of a prefill call whose longest row reaches max_keys keys, on ncu compute units (no device
+ * needed) */
+int mi_op_attention_prefill_slices(const mi_op_attn_shape* s, int max_keys, int ncu);
 /* fused decode attention (L == 1): q/k norm + RoPE + append + split-KV attention + combine.
  * counters: [B*Hkv] zero-initialised ints.  variant 0: MFMA kernel where it applies (16-bit caches,
  * head_dim % 32 == 0; float32 caches, head_dim 64 / 128), 1: VALU kernel (2: the MFMA kernel in its twelve-wave form,

@@ -154,6 +154,7 @@ SIGNATURES = {
     "mi_op_rope_append": (C.c_int, [C.POINTER(OpAttnShape), _P, _P, _P, _P, _P, _P, _P, C.c_float, _P, _P, C.c_int]),
     "mi_op_attention": (C.c_int, [C.POINTER(OpAttnShape), _P, _P, _P, _P, _P, C.c_float, C.c_int, _P]),
     "mi_op_attention_prefill": (C.c_int, [C.POINTER(OpAttnShape), _P, C.c_int, C.c_int, _P, _P, _P, _P, _P, C.c_float, C.c_int, _P, _P]),
+    "mi_op_attention_prefill_slices": (C.c_int, [C.POINTER(OpAttnShape), C.c_int, C.c_int]),
     "mi_op_attention_decode": (C.c_int, [C.POINTER(OpAttnShape), _P, _P, _P, _P, _P, _P, C.c_float, _P, _P, _P, C.c_float,
                                          C.c_int, C.c_int, _P, _P, C.c_int, C.c_int, C.POINTER(C.c_float)]),
     "mi_op_attention_decode_splits": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int]),

@@ -22,8 +22,6 @@
 
 namespace mi {
 
-int gemv_cu_count();      // gemv_mfma.hip
-
 namespace {
 
 constexpr int PREFILL_MAX_SLICES = 16;
@@ -337,7 +335,8 @@ __device__ __forceinline__ void dma_kib(const void* gsrc, unsigned lds_dst) {
 
 // (launch bounds: two waves per SIMD, i.e. up to 256 registers.  Left to itself hipcc aims at three, keeps the output
 // accumulators in AGPRs and moves them to VGPRs and back around every rescale: 88 v_accvgpr moves per block of 16 MFMAs.)
-template <typename T, int D, int G, bool PAGED, int QG>
+// SPLIT: keys over gridDim.z workgroups.  A kernel of its own: with the join in it an unsplit call took 0.4 to 0.9 us more (5 to 8).
+template <typename T, int D, int G, bool PAGED, int QG, bool SPLIT>
 __global__ __launch_bounds__(G * 64, G >= 2 ? 2 : 1) void attn_prefill_dma_kernel(AttnCall c) {
   static_assert(sizeof(T) == 2 && D % 32 == 0 && D <= 128, "16-bit activations / caches, head_dim 32..128");
   constexpr int KK = D / 32, DT = D / 16, NT = G * 64;
@@ -358,8 +357,8 @@ __global__ __launch_bounds__(G * 64, G >= 2 ? 2 : 1) void attn_prefill_dma_kerne
   const int nb = (nk + KB - 1) / KB;
   // this slice's blocks.  A workgroup beyond its row's slices has none and leaves at the end (a return here instead: 22.6 us against 22.2 at a chunk
   // of 32 tokens behind 700 keys, Qwen3-14B heads)
-  const int nz = prefill_row_slices(gridDim.z, off + s.L), z = min((int)blockIdx.z, nz);
-  const int j0 = z * nb / nz, j1 = min(z + 1, nz) * nb / nz;
+  const int nz = SPLIT ? prefill_row_slices(gridDim.z, off + s.L, c.join_cost, c.slice_cost) : 1, z = SPLIT ? min((int)blockIdx.z, nz) : 0;
+  const int j0 = SPLIT ? z * nb / nz : 0, j1 = SPLIT ? min(z + 1, nz) * nb / nz : nb;
   const int h = kh * G + wave;
 
   // K / V blocks go global -> LDS by LDS-DMA into a ring of THREE buffers: block j + 2 is issued at the head of
@@ -518,15 +517,15 @@ __global__ __launch_bounds__(G * 64, G >= 2 ? 2 : 1) void attn_prefill_dma_kerne
     buf = buf == 2 ? 0 : buf + 1;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // no DMA of this workgroup may land after it has left the CU
-  if (z == nz) return;
+  if (SPLIT && z == nz) return;
 
 #pragma unroll
   for (int u = 0; u < QG; ++u) {
     float l = l_run[u];
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
-    if (nz > 1) {                                     // (launched with one query group only)
-      if (!join_slices<DT>(c, bh * gridDim.x + qt, nz, G, wave, lane, accO[u], m_run[u], l)) return;
+    if constexpr (SPLIT) {                            // (launched with one query group only)
+      if (nz > 1 && !join_slices<DT>(c, bh * gridDim.x + qt, nz, G, wave, lane, accO[u], m_run[u], l)) return;
     }
     if (t0 + QT * u + c16 < s.L) {
       const float inv = 1.0f / l;
@@ -550,8 +549,11 @@ int launch_pg(const AttnCall& c, hipStream_t st) {
   const char* env = getenv("MI_ATTN_PREFILL_DMA");     // A/B and the bit-equality test: 0 = the register-staged kernel (read per call)
   if (env == nullptr || atoi(env) != 0) {
     grid.z = c.nsplit;
-    if (s.btab) hipLaunchKernelGGL((attn_prefill_dma_kernel<T, D, G, true, 1>), grid, block, 0, st, c);
-    else hipLaunchKernelGGL((attn_prefill_dma_kernel<T, D, G, false, 1>), grid, block, 0, st, c);
+    if (c.nsplit > 1) {
+      if (s.btab) hipLaunchKernelGGL((attn_prefill_dma_kernel<T, D, G, true, 1, true>), grid, block, 0, st, c);
+      else hipLaunchKernelGGL((attn_prefill_dma_kernel<T, D, G, false, 1, true>), grid, block, 0, st, c);
+    } else if (s.btab) hipLaunchKernelGGL((attn_prefill_dma_kernel<T, D, G, true, 1, false>), grid, block, 0, st, c);
+    else hipLaunchKernelGGL((attn_prefill_dma_kernel<T, D, G, false, 1, false>), grid, block, 0, st, c);
   } else {
     if (s.btab) hipLaunchKernelGGL((attn_prefill_kernel<T, D, G, true, 1>), grid, block, 0, st, c);
     else hipLaunchKernelGGL((attn_prefill_kernel<T, D, G, false, 1>), grid, block, 0, st, c);
@@ -729,7 +731,7 @@ __global__ __launch_bounds__(G * 64, 2) void attn_prefill_f32_kernel(AttnCall c)
 // from the float32 caches and split while they are written to LDS (each element once per workgroup, not once per wave).
 // What the 16+ bits cost was looked at on the CPU first (oracle/numerics.py SDPA_SPLIT2: the float32-accumulating
 // variants do not move).  MI_ATTN_PREFILL_F32_EXACT=1 (read per call) runs attn_prefill_f32_kernel instead.
-template <int D, int G, bool PAGED>
+template <int D, int G, bool PAGED, bool SPLIT>       // (SPLIT: as attn_prefill_dma_kernel)
 __global__ __launch_bounds__(G * 64, 2) void attn_prefill_f32s_kernel(AttnCall c) {
   static_assert(D % 32 == 0 && D <= 128, "head_dim 32..128");
   using T = bf16;
@@ -750,8 +752,8 @@ __global__ __launch_bounds__(G * 64, 2) void attn_prefill_f32s_kernel(AttnCall c
   const int nb = (nk + KB - 1) / KB;
   // this slice's blocks.  A workgroup beyond its row's slices has none and leaves at the end (a return here instead: 22.6 us against 22.2 at a chunk
   // of 32 tokens behind 700 keys, Qwen3-14B heads)
-  const int nz = prefill_row_slices(gridDim.z, off + s.L), z = min((int)blockIdx.z, nz);
-  const int j0 = z * nb / nz, j1 = min(z + 1, nz) * nb / nz;
+  const int nz = SPLIT ? prefill_row_slices(gridDim.z, off + s.L, c.join_cost, c.slice_cost) : 1, z = SPLIT ? min((int)blockIdx.z, nz) : 0;
+  const int j0 = SPLIT ? z * nb / nz : 0, j1 = SPLIT ? min(z + 1, nz) * nb / nz : nb;
   const int h = kh * G + wave;
 
   __shared__ __attribute__((aligned(16))) unsigned char khi[2][IMG];
@@ -900,11 +902,11 @@ __global__ __launch_bounds__(G * 64, 2) void attn_prefill_f32s_kernel(AttnCall c
     __syncthreads();
   }
 
-  if (z == nz) return;
+  if (SPLIT && z == nz) return;
   l_run += __shfl_xor(l_run, 16, 64);
   l_run += __shfl_xor(l_run, 32, 64);
-  if (nz > 1) {
-    if (!join_slices<DT>(c, bh * gridDim.x + qt, nz, G, wave, lane, accO, m_run, l_run)) return;
+  if constexpr (SPLIT) {
+    if (nz > 1 && !join_slices<DT>(c, bh * gridDim.x + qt, nz, G, wave, lane, accO, m_run, l_run)) return;
   }
   if (t0 + c16 < s.L) {
     const float inv = 1.0f / l_run;
@@ -925,8 +927,11 @@ int launch_pg32(const AttnCall& c, hipStream_t st) {
   const char* env = getenv("MI_ATTN_PREFILL_F32_EXACT");   // A/B and the comparison test (read per call): 1 = exact float32 products
   if (env == nullptr || atoi(env) == 0) {
     grid.z = c.nsplit;
-    if (s.btab) hipLaunchKernelGGL((attn_prefill_f32s_kernel<D, G, true>), grid, block, 0, st, c);
-    else hipLaunchKernelGGL((attn_prefill_f32s_kernel<D, G, false>), grid, block, 0, st, c);
+    if (c.nsplit > 1) {
+      if (s.btab) hipLaunchKernelGGL((attn_prefill_f32s_kernel<D, G, true, true>), grid, block, 0, st, c);
+      else hipLaunchKernelGGL((attn_prefill_f32s_kernel<D, G, false, true>), grid, block, 0, st, c);
+    } else if (s.btab) hipLaunchKernelGGL((attn_prefill_f32s_kernel<D, G, true, false>), grid, block, 0, st, c);
+    else hipLaunchKernelGGL((attn_prefill_f32s_kernel<D, G, false, false>), grid, block, 0, st, c);
   } else if (s.btab) hipLaunchKernelGGL((attn_prefill_f32_kernel<D, G, true>), grid, block, 0, st, c);
   else hipLaunchKernelGGL((attn_prefill_f32_kernel<D, G, false>), grid, block, 0, st, c);
   MI_HIP(hipGetLastError());
@@ -957,12 +962,21 @@ bool attention_prefill_supported(const AttnShape& s) {
   return s.D == 32 || s.D == 64 || s.D == 128;
 }
 
-// Slices of the keys: as many as fill the chip (one workgroup per CU), each with at least two blocks of the row's keys; a call that has
-// a workgroup for most CUs by itself is not cut (its slices would only queue behind each other and pay the join).
-int attention_prefill_slices(const AttnShape& s, int max_keys) {
+// Slices of the keys: at most as many as fill the chip (one workgroup per CU).  The costs, fitted to launches of 1 to 16 slices at 48 shapes (rocprof;
+// head groups of 1 to 8, head_dim 32 to 128, 8 to 132 key blocks; keys cold, the chunk's own warm): a key block takes 0.85 us, on float32
+// caches 1.3 + 2 / G; the join 2 + 0.47 G us, and a slice more per slice the more tiles publish theirs at once.  The rule's pick is within 2 % of
+// the fastest on average and at no shape slower than one workgroup.  us in 1 / 2 / 4 / 8 / 16 slices, G = 4, D = 128, bf16: 16 tiles, 23 blocks 22.8 /
+// 18.8 / 16.1 / 17.8 / 24.7, 126 blocks 100 / 58 / 36 / 28 / 31, 9 blocks 12.1 / 13.5 / 13.4 / 16.1; 128 tiles, 4 blocks 8.1 / 15.5 (when two blocks were
+// enough for a slice, a prompt of 128 tokens lost 4 us a layer, two of them 7).
+int attention_prefill_slices(AttnCall& c, int max_keys, int ncu) {
+  const AttnShape& s = c.s;
   if (!attention_prefill_supported(s)) return 1;
   static_assert(KB == PREFILL_KEY_BLOCK, "");
-  return prefill_row_slices(std::min(gemv_cu_count() / attention_prefill_tiles(s), PREFILL_MAX_SLICES), max_keys);
+  const int tiles = attention_prefill_tiles(s), G = s.Hq / s.Hkv;
+  const double block = s.act == MI_F32 ? 1.3 + 2.0 / G : 0.85;
+  c.join_cost = (int)(128 * (2.0 + 0.47 * G) / block + 0.5);
+  c.slice_cost = (int)(128 * (0.1 + 0.1 * G + 0.0058 * G * tiles) / block + 0.5);
+  return prefill_row_slices(std::min(ncu / tiles, PREFILL_MAX_SLICES), max_keys, c.join_cost, c.slice_cost);
 }
 size_t attention_prefill_part_floats(const AttnShape& s, int slices) {
   return (size_t)((s.L + QT - 1) / QT) * s.B * s.Hkv * slices * (s.Hq / s.Hkv) * 64 * (s.D / 16 + 1) * 4;

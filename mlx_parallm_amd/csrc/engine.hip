@@ -701,7 +701,7 @@ int choose_nsplit(const mi_kv* kv, int B, int Hkv, int L, const int32_t* rows = 
 int split_prefill(mi_engine* e, AttnCall& ac, int max_keys) {
   ac.nsplit = 1; ac.partial = nullptr;
   if (ac.variant == 1) return MI_OK;
-  const int n = attention_prefill_slices(ac.s, max_keys);
+  const int n = attention_prefill_slices(ac, max_keys, gemv_cu_count());
   if (n <= 1) return MI_OK;
   const size_t need = attention_prefill_part_floats(ac.s, n), ctr = attention_prefill_tiles(ac.s);
   if (need > e->ap_part_cap) {

@@ -251,22 +251,27 @@ struct AttnCall {
   float* partial;        // nsplit > 1: [B*L*Hq][nsplit][D+2], or attention_prefill_part_floats()
   int variant;           // 0: L > 1 goes to the MFMA prefill kernel where it applies; 1: always the VALU kernel
   int* counters = nullptr;   // nsplit > 1, L > 1: attention_prefill_tiles() arrival tickets, zero between launches
+  int join_cost = 0, slice_cost = 0;   // nsplit > 1, L > 1: prefill_row_slices() (0: every row takes as many slices as it can)
 };
 int launch_attention(const AttnCall& c, hipStream_t st);
 // causal prefill attention on the matrix cores (attn_prefill.hip); launch_attention dispatches to it
 bool attention_prefill_supported(const AttnShape& s);
-// over how many workgroups the keys of a call that reaches at most max_keys keys are split, and what that needs
-int attention_prefill_slices(const AttnShape& s, int max_keys);
+// over how many workgroups the keys of a call that reaches at most max_keys keys are split on ncu compute units (sets c's costs), and what
+// that needs
+int attention_prefill_slices(AttnCall& c, int max_keys, int ncu);
 size_t attention_prefill_part_floats(const AttnShape& s, int slices);
 int attention_prefill_tiles(const AttnShape& s);
 int launch_attention_prefill(const AttnCall& c, hipStream_t st);
 
 // Prefill attention: over how many of at most `most` workgroups the keys of a row that reaches `keys` of them are split (device: per row;
-// host: the longest row's): two blocks each at least.
+// host: the longest row's): two blocks each at least.  n slices cost blocks / n + join + n slice, in blocks (the costs come in 128ths): the
+// n that is cheapest by that, unless one workgroup is.  Never fewer slices for more keys.
 constexpr int PREFILL_KEY_BLOCK = 32;
-__host__ __device__ inline int prefill_row_slices(int most, int keys) {
-  const int pairs = (keys + PREFILL_KEY_BLOCK - 1) / PREFILL_KEY_BLOCK / 2, n = pairs < most ? pairs : most;
-  return n < 1 ? 1 : n;
+__host__ __device__ inline int prefill_row_slices(int most, int keys, int join, int slice) {
+  const int blocks = (keys + PREFILL_KEY_BLOCK - 1) / PREFILL_KEY_BLOCK;
+  int n = 1;
+  while (n < most && 2 * (n + 1) <= blocks && (n + 1) * (n + 1) * slice <= 128 * blocks) ++n;
+  return n > 1 && 128 * blocks / n + join + n * slice < 128 * blocks ? n : 1;
 }
 
 // Decode attention: over how many of at most `most` workgroups a row's `keys` cached keys are split (device: per row; host: the longest

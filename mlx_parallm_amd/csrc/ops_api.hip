@@ -221,6 +221,13 @@ int mi_op_attention_prefill(const mi_op_attn_shape* s, const int32_t* btab, int 
   return finish();
 }
 
+int mi_op_attention_prefill_slices(const mi_op_attn_shape* s, int max_keys, int ncu) {
+  if (!s || s->Hkv < 1 || s->B < 1 || s->L < 1 || ncu < 1 || max_keys < 0) return fail(MI_ERR_INVALID, "mi_op_attention_prefill_slices: counts");
+  AttnCall c{};
+  c.s = to_shape(s);
+  return attention_prefill_slices(c, max_keys, ncu);
+}
+
 int mi_op_attention_decode(const mi_op_attn_shape* s, const void* qkv, void* kcache, void* vcache,
                            const int32_t* offsets, const void* q_norm_w, const void* k_norm_w, float eps,
                            const float* cos_tab, const float* sin_tab, void* out, float scale, int rnd_out,

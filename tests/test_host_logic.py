@@ -387,3 +387,26 @@ def test_float32_rows_leave_the_streaming_kernel_where_the_tile_pays():
     assert all(pays(n, rounded=1) for n in (32, 33, 64, 8192))
     assert not any(pays(n, codes=1, rounded=1) for n in (33, 64, 96)) and all(pays(n, codes=1, rounded=1) for n in (128, 700))
     assert not any(pays(n, hilo=1, rounded=1) for n in (33, 768, 1024)) and pays(2048, hilo=1, rounded=1)
+
+
+@pytest.mark.parametrize("f32", [False, True])
+def test_prefill_attention_slices(f32):
+    """Over how many workgroups a prefill call's keys are split: not where the join costs more than it saves (a prompt from its start), several for
+    a chunk behind a long cache, never fewer for more keys -- a row's own number may not depend on a longer neighbour's."""
+    import ctypes as C
+
+    from mlx_parallm_amd import _lib as L
+
+    def slices(B, L_, keys, Hq=32, Hkv=8, D=128):
+        s = L.OpAttnShape()
+        s.B, s.L, s.Hq, s.Hkv, s.D, s.rnd, s.cap = B, L_, Hq, Hkv, D, 0, 8192
+        s.act = s.kv = L.MI_F32 if f32 else L.MI_BF16
+        return L.lib().mi_op_attention_prefill_slices(C.byref(s), keys, 256)
+
+    assert all(slices(B, L_, L_) == 1 for B, L_ in ((1, 16), (1, 64), (1, 128), (1, 200), (1, 256), (2, 64), (2, 128), (4, 64), (8, 1024)))
+    assert [slices(1, 32, k) > 1 for k in (64, 160, 732, 4032)] == [False, False, True, True]
+    assert slices(1, 16, 4016) >= 8 and 3 <= slices(1, 128, 4128) <= 4 and slices(2, 128, 4128) == 2 and slices(4, 256, 4000) == 1
+    for B, L_, Hq, Hkv in ((1, 16, 8, 8), (1, 40, 40, 8), (3, 17, 16, 2), (2, 200, 10, 2), (16, 32, 5, 1)):
+        got = [slices(B, L_, k, Hq, Hkv) for k in range(L_, 8192, 7)]
+        assert got == sorted(got) and 1 <= got[0] and got[-1] <= 16
+        assert all(n == 1 or 2 * n <= (k + 31) // 32 for n, k in zip(got, range(L_, 8192, 7)))
