@@ -186,9 +186,10 @@ def test_gemv_short_rows(act, kind, K, M):
 @pytest.mark.parametrize("act,kind,K", [("float32", "f32", 8), ("bfloat16", "bf16", 72), ("float16", "f16", 264)])      # 7 of 8, 7 of 16, 31 of 64 lanes past K
 def test_gemv_short_rows_keep_an_infinite_weight(act, kind, K):
     """Lanes past the row's end repeat its first weights: an infinite one must not meet their zeros."""
-    w = np.abs(RNG.standard_normal((80, K)).astype(np.float32)) + 0.5
+    rng = np.random.default_rng(K)                      # (its own: the file's generator feeds the tests behind this one)
+    w = np.abs(rng.standard_normal((80, K)).astype(np.float32)) + 0.5
     w[5, 3], w[46, 0] = np.inf, -np.inf
-    x = np.abs(RNG.standard_normal((3, K)).astype(np.float32)) + 0.5
+    x = np.abs(rng.standard_normal((3, K)).astype(np.float32)) + 0.5
     x[1] *= -1.0
     wd = dev(w, act)
     out = torch.zeros((3, 80), dtype=torch.float32, device="cuda")
