@@ -20,7 +20,8 @@
 // gate|up 21.3 -> 17.7, down 15.0 -> 14.8; int8 (3 rows) o 11.6 -> 7.4.  The stream itself is 9 to 66 MB = 1.6 to 11.2 us (int4); what is
 // left is the norm in front (2.5 us) and, in down, ~75 vector instructions per block.  The error against 64 bits is no larger than
 // gemm_skinny.hip's: bf16 results that round to another value than the exact one 3.4e-4 / 3.4e-4 (int4, K 4096 / 14336; 3.4e-4 /
-// 4.3e-4 there), int8 3e-5 (6e-5).
+// 4.3e-4 there), int8 3e-5 (6e-5); dense 16-bit rows (K 1024 to 5120, with and without the norm; gemv_mfma.hip there) bf16 1.1e-4 (1.3e-4), f16
+// 1.8e-3 (2.4e-3).
 #include <algorithm>
 
 #include "gemv_phase.h"
@@ -467,7 +468,9 @@ int quant_bits(const LinearW& W, int act) {           // 4 / 8: codes with scale
   if (((W.wk == WK_Q8_BF16 && act == MI_BF16) || (W.wk == WK_Q8_F16 && act == MI_F16)) && W.group == 64) return 8;
   return 0;
 }
-constexpr int REG_K = 8 * 640, LONG_K = 8 * 17 * 128;  // longest K whose activations stay in registers; longest K at all
+// Longest K whose activations stay in registers; longest K at all.  The second is no limit of the kernel (its registers do not grow past 12
+// blocks a wave): it is the longest that was measured, and what is longer stays on gemm_skinny.hip.
+constexpr int REG_K = 8 * 640, LONG_K = 8 * 17 * 128;
 
 }  // namespace
 
