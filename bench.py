@@ -887,9 +887,9 @@ def main():
         both reported in KiB.  null for any other workload / kernel / batch than the one that was profiled."""
         if args.workload != "mistral-7b-bf16" or kern != "gemv_gate_up" or B != 8 or args.lora:
             return None, None
-        # model-dtype KV: the M <= 8 kernel with the fused RMSNorm; float32 KV: the split-K kernel on float32 activations
-        want = "gemv_mfma_gu8_kernel<bf16,MB=8>" if kv_dtype == "model" else "skinny_kernel<bf16,0,1,true,true>"
-        for tag in (("round4_bf16kv", "round3_bf16kv", "round2", "round1") if kv_dtype == "model" else ("round4_f32kv", "round3_f32kv")):
+        # model-dtype KV: the M <= 8 kernel with the fused RMSNorm; float32 KV: the register kernel on float32 activations
+        want = "gemv_mfma_gu8_kernel<bf16,MB=8>" if kv_dtype == "model" else "gemv_dense_kernel<bf16,x32,gate|up,norm,512>"
+        for tag in (("round4_bf16kv", "round3_bf16kv", "round2", "round1") if kv_dtype == "model" else ("f32kv_gemv_dense",)):
             vals = {}
             for ctr in ("FETCH_SIZE", "WRITE_SIZE"):
                 f = ROOT / "profiles" / f"{tag}_pmc_{ctr}.csv"

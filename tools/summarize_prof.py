@@ -50,6 +50,9 @@ def pretty(name: str) -> str:
     own = _demangle_own(name)
     if own:
         name = own.replace("bf16", "__bf16")
+    m = re.search(r"gemv_dense_kernel<bool _Accum, bool, E, (true|false), (true|false), (\d+)", name)      # <__bf16, true (float32 x), ..>, as below
+    if m:
+        return "gemv_dense_kernel<bf16,x32,%s,%s,%s>" % ("gate|up" if m.group(1) == "true" else "plain", "norm" if m.group(2) == "true" else "-", m.group(3))
     if "_Accum" in name:   # rocprofv3's failed demangle of a <__bf16, true, ...> instantiation
         base = name.split("<")[0].replace("void ", "").replace("mi::(anonymous namespace)::", "").replace("mi::", "")
         return {"gemm_tile_kernel": "gemm_tile_kernel<bf16,swiglu>"}.get(base, base + "<bf16,...>")
