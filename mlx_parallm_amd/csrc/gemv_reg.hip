@@ -491,10 +491,15 @@ bool gemv_reg_supported(const LinearW& W, const GemvCall& c, size_t rows) {
   return c.ldx % 8 == 0 && (uintptr_t)c.x % 16 == 0 && (c.pro != PRO_NORM || (uintptr_t)c.norm_w % 16 == 0);
 }
 
-// f(k per wave of the instantiation, every wave has that): the smallest registers that hold a wave's blocks of bk
-template <class F>
+// f(k per wave of the instantiation, every wave has that): the smallest registers that hold a wave's blocks of bk.
+// FULL640 = false: the largest never takes the branchless form (with three terms of x and the norm that one spills three registers)
+template <bool FULL640 = true, class F>
 static int by_share(int nblk, int bk, F f) {
-  auto at = [&](auto kw) { return nblk * bk == 8 * kw ? f(kw, std::true_type{}) : f(kw, std::false_type{}); };
+  auto at = [&](auto kw) {
+    if constexpr (FULL640 || kw.value < 640)
+      if (nblk * bk == 8 * kw) return f(kw, std::true_type{});
+    return f(kw, std::false_type{});
+  };
   const int kw = (nblk + 7) / 8 * bk;
   return kw <= 256 ? at(std::integral_constant<int, 256>{}) : kw <= 512 ? at(std::integral_constant<int, 512>{}) : at(std::integral_constant<int, 640>{});
 }
@@ -559,7 +564,7 @@ static int launch_dense(const RegParams& p, bool gu, hipStream_t st) {
   };
   if constexpr (X32)
     if (gu) return by_share(p.nblk, 64, [&](auto kw, auto full) { return go(gemv_dense_kernel<AT, X32, true, true, kw.value, full.value>); });
-  if (p.norm) return by_share(p.nblk, 64, [&](auto kw, auto full) { return go(gemv_dense_kernel<AT, X32, false, true, kw.value, full.value>); });
+  if (p.norm) return by_share<!X32>(p.nblk, 64, [&](auto kw, auto full) { return go(gemv_dense_kernel<AT, X32, false, true, kw.value, full.value>); });
   return by_share(p.nblk, 64, [&](auto kw, auto full) { return go(gemv_dense_kernel<AT, X32, false, false, kw.value, full.value>); });
 }
 
