@@ -75,7 +75,7 @@ __device__ __forceinline__ void epi32_swiglu(const GemmParams& p, int m, int n, 
   ((float*)p.out)[(size_t)m * p.ldo + n] = sl * up;
 }
 __device__ __forceinline__ void epi32_plain(const GemmParams& p, int m, int n, float y) {
-  if (p.epi == EPI_STORE) ((float*)p.out)[(size_t)m * p.ldo + n] = round_rt(y, p.rnd);
+  if (p.epi == EPI_STORE) ((float*)p.out)[(size_t)m * p.ldo + n] = y;
   else { float* h = (float*)p.resid; h[(size_t)m * p.ldo + n] = h[(size_t)m * p.ldo + n] + y; }
 }
 
@@ -101,7 +101,9 @@ __device__ __forceinline__ bool group_of_tile(GemmParams& p, int bm, int n0, int
 // longer the chain, the more values round the other way (mean |logprob - exact| of three recorded float32-cache cases: streaming
 // kernel 1.64 / 1.27 / 2.08e-4, the 256 x 256 tile's one chain over K 2.02 / 1.74 / 2.53e-4, here 1.52 / 1.04 / 1.98e-4).  8 x 1024 rows
 // of Mistral-7B's q|k|v: 0.9 ms against 0.4 on the 256 x 256 tile and 4.6 streaming.
-template <typename AT, bool SWIGLU, bool GROUPED = false, bool FOLD = false>
+// LOGITS (here and in the 256 x 256 kernels): plain float32 stores of values rounded to AT.  A form of its own: p.rnd asked per element cost every
+// call of the kernels (one round of 256 workgroups, 8192 x 2048 outputs, 67.7 -> 76.0 us).
+template <typename AT, bool SWIGLU, bool GROUPED = false, bool FOLD = false, bool LOGITS = false>
 __global__ __launch_bounds__(256) void gemm_tile_kernel(GemmParams p) {
   __shared__ __attribute__((aligned(16))) AT As[2][BM][LDA];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -270,6 +272,7 @@ __global__ __launch_bounds__(256) void gemm_tile_kernel(GemmParams p) {
         for (int nt = 0; nt < 4; ++nt) {
           const int n = bn * BN + wn * 64 + nt * 16 + c16;
           if (n >= p.N) continue;
+          if constexpr (FOLD || LOGITS) { ((float*)p.out)[(size_t)m * p.ldo + n] = LOGITS ? (float)(AT)acc[mt][nt][r] : round_rt(acc[mt][nt][r], p.rnd); continue; }
           if (p.out32) { epi32_plain(p, m, n, acc[mt][nt][r]); continue; }
           const float y = (float)(AT)(VAR ? silu_col(p.silu_cols, n, acc[mt][nt][r]) : acc[mt][nt][r]);
           if (p.epi == EPI_STORE) out[(size_t)m * p.ldo + n] = (AT)y;
@@ -298,7 +301,7 @@ __global__ __launch_bounds__(256) void splitk_epilogue_kernel(GemmParams p) {
   for (int z = 0; z < p.ksplit; ++z) a += *(const f32x4*)(p.ws + (size_t)z * p.M * p.N + e0);
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    if (p.out32) { epi32_plain(p, m, n + j, a[j]); continue; }
+    if (p.out32) { epi32_plain(p, m, n + j, round_rt(a[j], p.rnd)); continue; }      // (p.rnd: plain stores only)
     const float y = (float)(AT)silu_col(p.silu_cols, n + j, a[j]);
     if (p.epi == EPI_STORE) ((AT*)p.out)[(size_t)m * p.ldo + n + j] = (AT)y;
     else { AT* h = (AT*)p.resid; h[(size_t)m * p.ldo + n + j] = (AT)((float)h[(size_t)m * p.ldo + n + j] + y); }
@@ -312,7 +315,7 @@ __device__ __forceinline__ bool epilogue_varies(const GemmParams& p, int bn) { r
 // the epilogue of the 256 x 256 tiles (2 x 4 waves, 128 x 64 per wave): lane (c16, g) holds C[m = 4g + r][n = c16] of
 // every 16 x 16 tile
 // VAR: another unit than silu, or a plain store with silu columns (common.h)
-template <typename AT, bool SWIGLU, bool VAR>
+template <typename AT, bool SWIGLU, bool VAR, bool LOGITS = false>
 __device__ __forceinline__ void tile256_epilogue(const GemmParams& p, f32x4 (&acc)[8][4], int m0, int bn, int wm, int wn, int c16, int g) {
   AT* out = (AT*)p.out;
 #pragma unroll
@@ -334,6 +337,7 @@ __device__ __forceinline__ void tile256_epilogue(const GemmParams& p, f32x4 (&ac
         for (int nt = 0; nt < 4; ++nt) {
           const int n = bn * BN2 + wn * 64 + nt * 16 + c16;
           if (n >= p.N) continue;
+          if constexpr (LOGITS) { ((float*)p.out)[(size_t)m * p.ldo + n] = (float)(AT)acc[mt][nt][r]; continue; }
           if (p.out32) { epi32_plain(p, m, n, acc[mt][nt][r]); continue; }
           const float y = (float)(AT)(VAR ? silu_col(p.silu_cols, n, acc[mt][nt][r]) : acc[mt][nt][r]);
           if (p.epi == EPI_STORE) out[(size_t)m * p.ldo + n] = (AT)y;
@@ -436,7 +440,7 @@ constexpr int STORE_AT = 11;                            // the item (of 16 per K
 // straight into a second register set (two sets in turn, the K loop is unrolled by two); LDS then carries only the X
 // tile (16 instead of 24 fragment reads per wave and step, half the stores).  Measured 2 % SLOWER than both operands
 // in LDS (68.5 k vs 69.9 k prefill tok/s): the LDS pipe was not the limit, the instruction order was (below).
-template <typename AT, bool SWIGLU, bool BD>
+template <typename AT, bool SWIGLU, bool BD, bool LOGITS = false>
 __global__ __launch_bounds__(512) void gemm_tile256_kernel(GemmParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem2[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -591,14 +595,15 @@ __global__ __launch_bounds__(512) void gemm_tile256_kernel(GemmParams p) {
     if (ks + 1 < nk) step(ks + 1, bset1, bset0);
   }
 
-  if constexpr (!SWIGLU) {
+  if constexpr (!SWIGLU && !LOGITS) {
     if (p.epi == EPI_RESID) {
       if (p.out32) tile256_epilogue_resid<AT, float>(p, acc, m0, bn, wm, wn, c16, g);
       else tile256_epilogue_resid<AT, AT>(p, acc, m0, bn, wm, wn, c16, g);
       return;
     }
   }
-  if (epilogue_varies<SWIGLU>(p, bn)) tile256_epilogue<AT, SWIGLU, true>(p, acc, m0, bn, wm, wn, c16, g);
+  if constexpr (LOGITS) tile256_epilogue<AT, SWIGLU, false, true>(p, acc, m0, bn, wm, wn, c16, g);
+  else if (epilogue_varies<SWIGLU>(p, bn)) tile256_epilogue<AT, SWIGLU, true>(p, acc, m0, bn, wm, wn, c16, g);
   else tile256_epilogue<AT, SWIGLU, false>(p, acc, m0, bn, wm, wn, c16, g);
 }
 
@@ -658,7 +663,7 @@ __device__ __forceinline__ void dma_kib(const void* gsrc, unsigned lds_dst) {
 typedef __attribute__((address_space(3))) u32x4 lds_u32x4_t;
 
 // GROUPED: as in gemm_tile_kernel
-template <typename AT, bool SWIGLU, bool GROUPED = false>
+template <typename AT, bool SWIGLU, bool GROUPED = false, bool LOGITS = false>
 __global__ __launch_bounds__(512) void gemm_dma256_kernel(GemmParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem2[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -808,7 +813,7 @@ __global__ __launch_bounds__(512) void gemm_dma256_kernel(GemmParams p) {
       return;
     }
   }
-  if constexpr (!SWIGLU) {
+  if constexpr (!SWIGLU && !LOGITS) {
     if (p.epi == EPI_RESID) {
       if (p.out32) tile256_epilogue_resid<AT, float>(p, acc, m0, bn, wm, wn, c16, g);
       else tile256_epilogue_resid<AT, AT>(p, acc, m0, bn, wm, wn, c16, g);
@@ -819,7 +824,8 @@ __global__ __launch_bounds__(512) void gemm_dma256_kernel(GemmParams p) {
     __syncthreads();
     if (SWIGLU && p.glu.kind != GLU_SILU) tile256_epilogue_rows<AT, SWIGLU, SWIGLU>(p, acc, smem2, bn, wave, lane, place0);
     else tile256_epilogue_rows<AT, SWIGLU, false>(p, acc, smem2, bn, wave, lane, place0);
-  } else if (epilogue_varies<SWIGLU>(p, bn)) tile256_epilogue<AT, SWIGLU, true>(p, acc, m0, bn, wm, wn, c16, g);
+  } else if constexpr (LOGITS) tile256_epilogue<AT, SWIGLU, false, true>(p, acc, m0, bn, wm, wn, c16, g);
+  else if (epilogue_varies<SWIGLU>(p, bn)) tile256_epilogue<AT, SWIGLU, true>(p, acc, m0, bn, wm, wn, c16, g);
   else tile256_epilogue<AT, SWIGLU, false>(p, acc, m0, bn, wm, wn, c16, g);
 }
 
@@ -1306,6 +1312,7 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
   const char* sk_env = getenv("MI_GEMM_DMA_SPLITK");     // (read per call: the tests switch it)
   const bool splitk256 = sk_env == nullptr || atoi(sk_env) != 0;
   const bool fold = x32 && c.rnd != RND_NONE;           // (plain stores: gemm_prefill_supported)
+  const bool logits = !x32 && p.rnd != RND_NONE;
   if (rows >= 256 && !small_only && !fold && dma && splitk256 && !sw && splitk_ws != nullptr && W.N % 4 == 0) {
     // one 128-KiB workgroup per CU: the launch runs in rounds of n_cu workgroups.  Pick the split whose last round is
     // fullest, charging 2 % per extra slice for its partial tile and its share of the reduce (q|k|v at 1024 rows: 96
@@ -1334,19 +1341,19 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
 #else
 #define GO256_M32(T, S)
 #endif
-#define GO256(T, S) do { \
-      if (use_dma) { auto k = gemm_dma256_kernel<T, S>; \
+#define GO256(T, S, LG) do { \
+      if (use_dma) { auto k = gemm_dma256_kernel<T, S, false, LG>; \
         MI_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * DMA_BUF)); \
         hipLaunchKernelGGL(k, grid2, block2, 2 * DMA_BUF, st, p); } \
       GO256_M32(T, S) \
-      else if (b_in_lds) { auto k = gemm_tile256_kernel<T, S, false>; \
+      else if (b_in_lds) { auto k = gemm_tile256_kernel<T, S, false, LG>; \
         MI_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, LDS2_BYTES)); \
         hipLaunchKernelGGL(k, grid2, block2, LDS2_BYTES, st, p); } \
-      else { auto k = gemm_tile256_kernel<T, S, true>; \
+      else { auto k = gemm_tile256_kernel<T, S, true, LG>; \
         MI_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * A2_BYTES)); \
         hipLaunchKernelGGL(k, grid2, block2, 2 * A2_BYTES, st, p); } } while (0)
-    if (c.act == MI_BF16 || x32) { if (sw) GO256(bf16, true); else GO256(bf16, false); }
-    else { if (sw) GO256(f16, true); else GO256(f16, false); }
+    if (c.act == MI_BF16 || x32) { if (sw) GO256(bf16, true, false); else if (logits) GO256(bf16, false, true); else GO256(bf16, false, false); }
+    else { if (sw) GO256(f16, true, false); else if (logits) GO256(f16, false, true); else GO256(f16, false, false); }
 #undef GO256
     MI_HIP(hipGetLastError());
     if (p.ksplit > 1) {
@@ -1374,9 +1381,11 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
   if (fold) hipLaunchKernelGGL((gemm_tile_kernel<bf16, false, false, true>), grid, block, 0, st, p);
   else if (c.act == MI_BF16 || x32) {
     if (sw) hipLaunchKernelGGL((gemm_tile_kernel<bf16, true>), grid, block, 0, st, p);
+    else if (logits) hipLaunchKernelGGL((gemm_tile_kernel<bf16, false, false, false, true>), grid, block, 0, st, p);
     else hipLaunchKernelGGL((gemm_tile_kernel<bf16, false>), grid, block, 0, st, p);
   } else {
     if (sw) hipLaunchKernelGGL((gemm_tile_kernel<f16, true>), grid, block, 0, st, p);
+    else if (logits) hipLaunchKernelGGL((gemm_tile_kernel<f16, false, false, false, true>), grid, block, 0, st, p);
     else hipLaunchKernelGGL((gemm_tile_kernel<f16, false>), grid, block, 0, st, p);
   }
   MI_HIP(hipGetLastError());
