@@ -95,6 +95,9 @@ int mi_op_gemm_skinny(const mi_op_linear* w, const mi_op_gemv_args* a, int kspli
  * nn.Linear over B x L rows at once).  a->M rows of 16-bit activations, tile-major dense 16-bit weights, a->pro =
  * MI_PRO_NONE; plain / residual / SwiGLU epilogues.  iters >= 1 also times that many back-to-back launches into *avg_ms. */
 int mi_op_gemm_prefill(const mi_op_linear* w, const mi_op_gemv_args* a, int iters, float* avg_ms);
+/* the same for tile-major int4 / int8 weights (group 64): the tile GEMM on their codes where it takes the call, else on their [hi | lo] copy.
+ * a->act: 16-bit, or float32 on a bf16 model (split into three terms here; a->rnd = MI_RND_BF16, plain stores only: one). */
+int mi_op_gemm_codes(const mi_op_linear* w, const mi_op_gemv_args* a, int iters, float* avg_ms);
 /* gemv_reg.hip on its own: the decode linears of at most 8 rows on tile-major weights -- int4 / int8 (group 64) with scales of the
  * activations' type (plain / float32 / residual / SwiGLU epilogues, the last with the norm), dense 16-bit ones with activations of
  * their type or float32 on bf16 (plain / float32 / residual; float32 also MI_EPI 4, SwiGLU on a row-interleaved gate|up matrix:

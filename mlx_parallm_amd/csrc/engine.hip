@@ -371,9 +371,15 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
     if (produce) { e->sq_valid = true; e->sq_src = c.resid; e->sq_parts = tgroups; e->sq_K = f.W.N; e->sq_ld = leave_ld; }
     return MI_OK;
   }
-  // logits and the rounded call of layer 0 in the float32-cache mode: only the rows for which the tile GEMM is ahead leave the streaming kernel
-  const bool stream32 = e->opt_skinny_gemm && c.act == MI_F32 && rows > 32 && gemm_skinny_supported(f.W, c, 32) &&
-                        (c.rnd != RND_NONE || c.epi == EPI_STORE_F32) && !gemm_prefill_pays(quant, c.kx > 0, c.rnd != RND_NONE, rows);
+  // float32-cache mode: only the rows for which the tile GEMM is ahead leave the streaming kernel.  Quantised matrices: by both sides' times; dense
+  // ones: logits, the rounded call of layer 0, and gate|up up to 64 rows (28672 x 4096, 64 rows: 103 us against 116; 34816 x 5120 162 / 230; 96 rows
+  // 154 / 117 and 243 / 244; the plain linears are ahead on the tile GEMM from 33 rows: 6144 x 4096 64 rows 38 / 31)
+  auto tile_pays = [&]() {
+    if (quant) return gemm_prefill_pays_codes(f.W, c, rows, c.rnd == RND_BF16 ? 1 : 3, rows < 4096 ? (size_t)128 << 20 : 0);
+    if (c.rnd != RND_NONE || c.epi == EPI_STORE_F32) return gemm_prefill_pays(false, c.kx > 0, c.rnd != RND_NONE, rows);
+    return c.epi != EPI_SWIGLU || rows > 64;
+  };
+  const bool stream32 = e->opt_skinny_gemm && c.act == MI_F32 && rows > 32 && gemm_skinny_supported(f.W, c, 32) && !tile_pays();
   if (e->opt_prefill_gemm && !stream32 && gemm_prefill_supported(f.W, c, rows)) {
     // prefill: one MFMA tile GEMM over all rows (the RMSNorm runs as its own row-wise kernel)
     Prof pr(e, prof);
@@ -391,7 +397,7 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
       // The rounded call of layer 0: its input is a bf16 value, i.e. one term (8 x 1024 rows of Mistral-7B: 256 launches of the
       // streaming kernel at 32 rows each, 4.6 ms, against 0.9 ms here).
       // (Logits keep the three terms that they had on the streaming kernel.)
-      // Quantised matrices, both calls: the codes are met as [hi | lo] pairs as in every other linear of a prefill.  A pair of bf16 is
+      // Quantised matrices: the exact three against their codes, or against [hi | lo] pairs (gemm_prefill.hip: codes_plan).  A pair of bf16 is
       // w = s q + b exactly while |w| <= 2^16 ulp(s), i.e. |b| up to some 2^9 scales -- int4 groups whose mean is up to 30 of their own standard
       // deviations, int8 groups up to 3 (quantised on the CPU and compared) -- and w to 2^-17 beyond; of f16, int4 groups to 1000.
       const int terms = c.rnd == RND_BF16 ? 1 : (e->opt_prefill_x_terms == 2 && f.W.wk == WK_BF16 && c.kx == 0 && c.rnd == RND_NONE && c.epi != EPI_STORE_F32) ? 2 : 3;
@@ -404,8 +410,10 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
     // logits of many positions against a quantised matrix: 32768 outputs at a time, so that the copy below stays within 4 x 32768 x K bytes
     const int ncol = (wk_is_quant(f.W.wk) && c.epi == EPI_STORE_F32) ? std::min(f.W.N, 32768) : f.W.N;
     void* scratch = nullptr;
-    if (wk_is_quant(f.W.wk)) {               // int4: the GEMM multiplies by a [hi | lo] 16-bit copy made on the fly
-      const size_t need = dequant_hilo_bytes(ncol, KT);
+    if (wk_is_quant(f.W.wk)) {               // the GEMM multiplies by 16-bit codes, or a [hi | lo] 16-bit copy, made on the fly
+      LinearW part = f.W;
+      part.N = ncol;
+      const size_t need = gemm_prefill_scratch_bytes(part, rows);
       if (need > e->deq_cap) {
         MI_HIP(hipStreamSynchronize(e->stream));
         hipFree(e->deq_scratch);
@@ -438,9 +446,8 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
     return MI_OK;
   }
   if (e->opt_skinny_gemm && c.act == MI_F32 && rows > 32 && gemm_skinny_supported(f.W, c, 32)) {
-    // PagedKVCache mode, more than 32 rows (its prefill): 32 rows per launch of the float32-activation streaming kernel
-    // (each row's arithmetic is that of a decode step, whatever the batch); the generic kernel took 8 rows per pass
-    // over W.  A tile GEMM with the three-way split of x is the next step for this mode.
+    // PagedKVCache mode, more than 32 rows: 32 rows per launch of the float32-activation streaming kernel (each row's arithmetic is
+    // that of a decode step, whatever the batch), where that is ahead of the tile GEMM; the generic kernel took 8 rows per pass over W.
     Prof pr(e, prof);
     const bool lora32 = f.W.lora_b[0] != nullptr || f.W.lora_b[1] != nullptr;
     if (lora32) { GemvCall cl = c; cl.M = (int)rows; MI_TRY(launch_lora_down(f0.W, cl, e->lora_t, 128, e->stream)); }

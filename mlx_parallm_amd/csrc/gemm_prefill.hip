@@ -65,6 +65,9 @@ struct GemmParams {
   // grouped form (GroupedGemm, kernels.h)
   const int32_t* tiles; const int32_t* x_rows; const int32_t* out_rows; int groups;
   const void* w_last; int N_last, K_last;
+  // codes form (gemm_codes256_kernel): w = the codes as 16-bit integers; scales [N/16][G][16], G = kw / 64; the group sums of x
+  // [M][kb] and the biases (tile-major, kb columns), whose product follows the K steps
+  const float* sc; const void* xs; const void* wb; int G, kb;
 };
 
 // the epilogues in float32 storage (PagedKVCache mode after layer 0: every op produces a float32 array)
@@ -831,6 +834,290 @@ __global__ __launch_bounds__(512) void gemm_dma256_kernel(GemmParams p) {
 
 
 // ---------------------------------------------------------------------------------------------------------------
+// Quantised weights (w = s q + b per group of 64 k): the 256 x 256 x 64 tile on the CODES.  A K tile is one group, so
+//     y[m][n] = sum_g s[n][g] (sum_k (q - c) x) + sum_g (b + c s)[n][g] (sum_k x),     c = 8 or 128, the middle of the codes,
+// the inner sums as MFMAs on q - c as 16-bit integers (exact: 4 or 8 bits in the 8 of bf16), one FMA per accumulator and group, and the
+// second term as a matrix product of its own: the group sums of x and b + c s in bf16 terms (hi + mid + lo = the float32 value), the six
+// products of the terms above 2^-24 of the whole, 6 K / 64 columns.
+// Why: the [hi | lo] copy that the dense tile takes doubles the products and the bytes of the copy.  The codes carry no rounding at all;
+// [hi | lo] drops what lies below 2^-17 of a weight.  Around their middle: codes of 0..15 (255) make sums of twice the size and more that
+// the biases take back; the float32 result is then 4.5e-7 from the 64-bit one (6144 x 4096, 1024 rows, 2-norm), here 1.5e-7, [hi | lo] 4.1e-7.
+// Registers: 128 accumulators + the group's sums.  A phase is two row tiles x both k blocks, so those are 32 (a quarter tile) and not
+// 64; the FMAs of the first row tile sit in the shadow of the second's MFMAs, those of the second in the next phase's read section.
+// Tile, LDS images, wave grid, ping-pong and epilogues: gemm_dma256_kernel.  What differs in the schedule: A-h0 is read in phases 0 and
+// 1, A-h1 in 2 and 3, B-k0 in the read section of phase 0, B-k1 in its MFMA section (so it is restaged in phase 2 at the earliest),
+// the scales (256 B of a wave's own, one dword per lane and tile) in phase 0.
+//   stage:  j=0: A-h1(t+1)   j=1: B-k0(t+2)   j=2: B-k1(t+2)   j=3: scales(t+2), A-h0(t+2)
+//     unit                           staged in     waited for in   first read in   DMAs issued since
+//     A-h1(t+1)                      (t, j=0)      (t+1, j=1)      (t+1, j=2)      2 + 2 + 3 + 2 + 2 -> vmcnt(11)
+//     B-k0, B-k1, scales, A-h0(t+2)  (t, j=1..3)   (t+1, j=3)      (t+2, j=0)      2 + 2 + 2 + 3     -> vmcnt(9)
+constexpr int CODES_LDS = 2 * DMA_BUF + 8 * 2 * 256;
+
+__device__ __forceinline__ void dma_kib_off(const void* base, uint32_t off, unsigned lds_dst) {
+  unsigned keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_dst) : "memory");
+}
+__device__ __forceinline__ void dma_dword_off(const void* base, uint32_t off, unsigned lds_dst) {
+  unsigned keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "v"(off), "s"(base), "s"(lds_dst) : "memory");
+}
+typedef __attribute__((address_space(3))) f32x4 lds_f32x4_t;
+
+template <typename AT, bool SWIGLU, bool LOGITS = false>
+__global__ __launch_bounds__(512) void gemm_codes256_kernel(GemmParams p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem2[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 2, wn = wave & 3;
+  const int c16 = lane & 15, g = lane >> 4;
+  const int bm = blockIdx.x, bn = blockIdx.y, m0 = bm * BM2;
+  // K tiles: [0, nkm) = the groups of x's terms in turn (W is walked once per term), [nkm, nk_all) = the bias columns
+  const int nkm = p.ka / BK, nk_all = nkm + p.kb / BK;
+  // this workgroup's: [tb, te) (divisions run on vector registers: back to scalar ones, the DMA bases are built of them)
+  const int tb = __builtin_amdgcn_readfirstlane((int)((blockIdx.z * (unsigned)nk_all) / gridDim.z));
+  const int te = __builtin_amdgcn_readfirstlane((int)(((blockIdx.z + 1) * (unsigned)nk_all) / gridDim.z));
+  const int ntiles_w = p.N / 16;
+  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem2;
+
+  auto w_tile_of = [&](int s) -> int {
+    int t;
+    if constexpr (!SWIGLU) t = (bn * BN2) / 16 + s;
+    else t = (bn * 128 + (s >> 2) * 32 + (s & 1) * 16 + ((s >> 1) & 1) * p.pair_offset) / 16;
+    return min(t, ntiles_w - 1);
+  };
+
+  // ---- DMA sources: a base in scalar registers + 32-bit offsets of the lanes (the host checks the sizes).  A unit h, instruction i of this wave
+  // = image rows (2 wave + i) * 8 + [0, 8)
+  uint32_t aoff[2][2];
+  const char *ga, *gb[2], *gs;                                   // of the run's first K tile: x (or the group sums), this wave's two W tiles, the scales
+  int last;                                                      // the run's last K tile
+  auto sources = [&](const void* x, uint32_t row_bytes, const void* w, size_t tile_bytes) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int rl = lane >> 4, col = lane & 15, ir = (2 * wave + i) * 8 + 2 * rl + (col >> 3);
+        aoff[h][i] = (uint32_t)min(m0 + (ir >> 6) * 128 + h * 64 + (ir & 63), p.M - 1) * row_bytes + (uint32_t)(((col & 7) ^ (4 * i + rl)) * 16);
+      }
+    ga = (const char*)x;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) gb[i] = (const char*)w + w_tile_of(2 * wave + i) * tile_bytes;
+    // (in scalar registers before the loop: a pending load of a kernel argument makes the compiler wait for every LDS read with it)
+    asm volatile("" : "+s"(ga), "+s"(gb[0]), "+s"(gb[1]), "+s"(gs));
+  };
+  const uint32_t lane16 = (uint32_t)lane * 16;
+  const uint32_t soff = (uint32_t)(w_tile_of(wn * 4 + (lane & 3)) * p.G * 64 + (lane >> 2) * 4);
+  const unsigned sc_lds = lds0 + 2 * DMA_BUF + wave * 512;
+  auto stage_a = [&](int t, int h) {
+    const char* base = ga + (size_t)((uint32_t)min(t, last) * (BK * 2));
+    const unsigned dst = lds0 + (t & 1) * DMA_BUF + h * DMA_UNIT + wave * 2048;
+    dma_kib_off(base, aoff[h][0], dst);
+    dma_kib_off(base, aoff[h][1], dst + 1024);
+  };
+  auto stage_b = [&](int t, int kb) {
+    const size_t koff = (uint32_t)min(t, last) * 2048 + kb * 1024;
+    const unsigned dst = lds0 + (t & 1) * DMA_BUF + (2 + kb) * DMA_UNIT + wave * 2048;
+    dma_kib_off(gb[0] + koff, lane16, dst);
+    dma_kib_off(gb[1] + koff, lane16, dst + 1024);
+  };
+  auto stage_s = [&](int t) { dma_dword_off(gs + (size_t)((uint32_t)min(t, last) * 64), soff, sc_lds + (t & 1) * 256); };
+  const unsigned a_lane = lds0 + (unsigned)((wm * 32 + (c16 >> 1)) * 256 + (((((c16 & 1) << 3) | g) ^ (c16 >> 1)) * 16));
+  const unsigned b_lane = lds0 + (unsigned)(wn * 4 * 1024 + lane * 16);
+  u32x4 af[2][2], b0[2][4], b1[4];                               // [row tile of the phase][k block]; [K tile & 1][column tile]; [column tile]
+  auto a_frags = [&](int t, int j) {
+    const unsigned off = (t & 1) * DMA_BUF + (j >> 1) * DMA_UNIT + (j & 1) * 2 * 8 * 256;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) af[i][kb] = *(const lds_u32x4_t*)(size_t)((a_lane ^ (unsigned)(kb << 6)) + off + i * 8 * 256);
+  };
+  auto b_frag = [&](int t, int kb, int nt) { return *(const lds_u32x4_t*)(size_t)(b_lane + (t & 1) * DMA_BUF + (2 + kb) * DMA_UNIT + nt * 1024); };
+
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 acc[8][4], tmp[2][4], sc = zero;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = zero;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) tmp[i][j] = zero;
+  auto fold2 = [&](int mt, int nt, int half) {
+#pragma unroll
+    for (int r = 2 * half; r < 2 * half + 2; ++r) acc[mt][nt][r] = fmaf(sc[nt], tmp[mt & 1][nt][r], acc[mt][nt][r]);
+    asm volatile("" : "+v"(acc[mt][nt]));                        // (here: hipcc sinks the FMAs behind the barriers and holds the sums of several phases)
+  };
+  auto fold = [&](int mt) {
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) { fold2(mt, nt, 0); fold2(mt, nt, 1); }
+  };
+
+  // (lgkmcnt(0) as the builtin: the compiler's own count then knows that the fragments are here, and waits for B-k1 alone)
+#define PP_READS_DONE(VM) do { __builtin_amdgcn_sched_barrier(0); __builtin_amdgcn_s_waitcnt(0xC07F); \
+      if (VM >= 0) asm volatile("s_waitcnt vmcnt(%0)" :: "i"(VM < 0 ? 0 : VM) : "memory"); \
+      asm volatile("s_barrier" ::: "memory"); __builtin_amdgcn_sched_barrier(0); __builtin_amdgcn_s_setprio(1); } while (0)
+#define PP_MMA_DONE() do { __builtin_amdgcn_sched_barrier(0); __builtin_amdgcn_s_setprio(0); asm volatile("s_barrier" ::: "memory"); \
+      __builtin_amdgcn_sched_barrier(0); } while (0)
+#define PP_ORDER() __builtin_amdgcn_sched_barrier(0)
+  auto phase = [&](int t, auto jt, auto pt, auto tail) __attribute__((always_inline)) {
+    constexpr int J = decltype(jt)::value, P = decltype(pt)::value;
+    constexpr bool TAIL = decltype(tail)::value;
+    f32x4 sn;
+    if constexpr (J == 0) {
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt) b1[nt] = b_frag(t, 1, nt);
+      if constexpr (!TAIL) sn = *(const lds_f32x4_t*)(size_t)(sc_lds + (t & 1) * 256 + c16 * 16);
+    }
+    a_frags(t, J);
+    if constexpr (J >= 2) {
+#pragma unroll
+      for (int nt = 2 * J - 4; nt < 2 * J - 2; ++nt) b0[P ^ 1][nt] = b_frag(t + 1, 0, nt);
+    }
+    PP_ORDER();
+    if constexpr (J == 0) stage_a(t + 1, 1);
+    if constexpr (J == 1) stage_b(t + 2, 0);
+    if constexpr (J == 2) stage_b(t + 2, 1);
+    if constexpr (J == 3) { if constexpr (!TAIL) stage_s(t + 2); stage_a(t + 2, 0); }
+    PP_READS_DONE((J & 1 ? (TAIL ? 8 : 9) : -1));
+    if constexpr (TAIL) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int nt = 0; nt < 4; ++nt) acc[2 * J + i][nt] = mfma16<bf16>(af[i][kb], kb ? b1[nt] : b0[P][nt], acc[2 * J + i][nt]);
+    } else {
+      // two FMAs behind every MFMA (16 cycles = four issues): first the last phase's second row tile (phase 0: the last K tile's), then
+      // this phase's first
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        tmp[0][i & 3] = i < 4 ? mfma16<AT>(af[0][0], b0[P][i], zero) : mfma16<AT>(af[0][1], b1[i & 3], tmp[0][i & 3]);
+        fold2((2 * J + 7) & 7, i >> 1, i & 1);
+        PP_ORDER();
+      }
+      if constexpr (J == 0) sc = sn;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        tmp[1][i & 3] = i < 4 ? mfma16<AT>(af[1][0], b0[P][i], zero) : mfma16<AT>(af[1][1], b1[i & 3], tmp[1][i & 3]);
+        fold2(2 * J, i >> 1, i & 1);
+        PP_ORDER();
+      }
+    }
+    PP_MMA_DONE();
+  };
+  auto ktile = [&](int t, auto pt, auto tail) __attribute__((always_inline)) {
+    phase(t, std::integral_constant<int, 0>{}, pt, tail);
+    phase(t, std::integral_constant<int, 1>{}, pt, tail);
+    phase(t, std::integral_constant<int, 2>{}, pt, tail);
+    phase(t, std::integral_constant<int, 3>{}, pt, tail);
+  };
+  // one run over n K tiles of the present sources, from an empty pipeline to an empty one
+  auto run = [&](int n, auto tail) __attribute__((always_inline)) {
+    constexpr bool TAIL = decltype(tail)::value;
+    const std::integral_constant<int, 0> even{};
+    const std::integral_constant<int, 1> odd{};
+    last = n - 1;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      stage_b(t, 0); stage_b(t, 1);
+      if constexpr (!TAIL) stage_s(t);
+      stage_a(t, 0);
+      if (t == 0) stage_a(0, 1);
+    }
+    asm volatile("s_waitcnt vmcnt(%0)" :: "i"(TAIL ? 8 : 9) : "memory");
+    asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) b0[0][nt] = b_frag(0, 0, nt);
+    if (wave >= 4) asm volatile("s_barrier" ::: "memory");
+    int t = 0;
+    for (; t + 1 < n; t += 2) {
+      ktile(t, even, tail);
+      ktile(t + 1, odd, tail);
+    }
+    if (t < n) ktile(t, even, tail);
+    if (wave < 4) asm volatile("s_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no DMA of this workgroup may land in the next run's units, or after it has left the CU
+    asm volatile("s_barrier" ::: "memory");
+  };
+  const uint32_t xrow = (uint32_t)(p.ldx * 2);
+  if (te > nkm) {                                                  // the bias columns, before the groups
+    const int lo = max(tb, nkm) - nkm;
+    gs = nullptr;
+    sources((const char*)p.xs + (size_t)lo * (BK * 2), (uint32_t)(p.kb * 2), (const char*)p.wb + (size_t)lo * 2048, (size_t)p.kb * 32);
+    run(te - nkm - lo, std::true_type{});
+  }
+  for (int t0 = 0; t0 < nkm; t0 += p.G) {                          // a run per term of x
+    const int lo = max(tb, t0), hi = min(te, t0 + p.G);
+    if (lo >= hi) continue;
+    gs = (const char*)p.sc + (size_t)(lo - t0) * 64;
+    sources((const char*)p.x + (size_t)lo * (BK * 2), xrow, (const char*)p.w + (size_t)(lo - t0) * 2048, (size_t)p.kw * 32);
+    run(hi - lo, std::false_type{});
+  }
+  fold(7);
+#undef PP_ORDER
+#undef PP_READS_DONE
+#undef PP_MMA_DONE
+
+  if constexpr (!SWIGLU) {
+    if (gridDim.z > 1) {                                   // this slice's partial tile, float32
+      float* wz = p.ws + (size_t)blockIdx.z * p.M * p.N;
+#pragma unroll
+      for (int mt = 0; mt < 8; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int m = m0 + wm * 128 + mt * 16 + 4 * g + r;
+          if (m >= p.M) continue;
+#pragma unroll
+          for (int nt = 0; nt < 4; ++nt) {
+            const int n = bn * BN2 + wn * 64 + nt * 16 + c16;
+            if (n < p.N) wz[(size_t)m * p.N + n] = acc[mt][nt][r];
+          }
+        }
+      return;
+    }
+  }
+  if constexpr (!SWIGLU && !LOGITS) {
+    if (p.epi == EPI_RESID) {
+      if (p.out32) tile256_epilogue_resid<AT, float>(p, acc, m0, bn, wm, wn, c16, g);
+      else tile256_epilogue_resid<AT, AT>(p, acc, m0, bn, wm, wn, c16, g);
+      return;
+    }
+  }
+  if constexpr (LOGITS) tile256_epilogue<AT, SWIGLU, false, true>(p, acc, m0, bn, wm, wn, c16, g);
+  else if (epilogue_varies<SWIGLU>(p, bn)) tile256_epilogue<AT, SWIGLU, true>(p, acc, m0, bn, wm, wn, c16, g);
+  else tile256_epilogue<AT, SWIGLU, false>(p, acc, m0, bn, wm, wn, c16, g);
+}
+
+// The group sums of x for the kernel above: row m -> `parts` terms of G columns each (kernels.h: codes16_sum_part; hi + mid + lo = the float32 sum
+// of the group's 64 values over x's `terms` of K columns), zeros up to kb.  One workgroup per row.
+template <typename AT>
+__global__ __launch_bounds__(256) void group_sums_kernel(const AT* x, int ldx, int terms, int K, uint16_t* xs, int kb) {
+  extern __shared__ float gsum[];
+  const int row = blockIdx.x, tid = threadIdx.x, G = K / 64;
+  const AT* xr = x + (size_t)row * ldx;
+  for (int k = tid * 8; k < K; k += 2048) {
+    float s = 0.f;
+    for (int t = terms - 1; t >= 0; --t) {                       // (the smallest terms first)
+      const u32x4 v = *(const u32x4*)(xr + (size_t)t * K + k);
+      const AT* e = (const AT*)&v;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s += (float)e[j];
+    }
+    s = lane8_sum(s);
+    if ((tid & 7) == 0) gsum[k >> 6] = s;
+  }
+  __syncthreads();
+  for (int c = tid; c < kb; c += 256) {
+    const int term = c / G, grp = c - term * G;
+    const float v = term < CODES16_TERMS ? bf16_part(gsum[grp], codes16_sum_part(term)) : 0.f;
+    xs[(size_t)row * kb + c] = __builtin_bit_cast(uint16_t, (bf16)v);
+  }
+}
+
+
+// ---------------------------------------------------------------------------------------------------------------
 // The same 256 x 256 x 64 tile on v_mfma_f32_32x32x16: per wave and K step 32 MFMAs of 32 cycles instead of 64 of 16.
 // Why: a 16x16x32 MFMA leaves 8 of its 16 cycles for other instructions to issue, the loop has ~135 of them per 64 MFMAs
 // (24 LDS reads, 8 + 8 staging loads / stores, ~45 address VALU, the waits) -- more than one wave's MFMA shadow holds;
@@ -1200,7 +1487,8 @@ bool gemm_prefill_supported(const LinearW& W, const GemvCall& c, size_t rows) {
   const bool q8 = ((W.wk == WK_Q8_BF16 && c.act == MI_BF16) || (W.wk == WK_Q8_F16 && c.act == MI_F16)) && W.group == 64;
   // float32 activations on a bf16 model (PagedKVCache mode): x goes through launch_split3_rows first
   static const bool f32_ok = getenv("MI_GEMM_NO_F32") == nullptr;
-  const bool x32 = f32_ok && c.act == MI_F32 && (W.wk == WK_BF16 || (W.wk == WK_Q4_BF16 && W.group == 64 && W.K % 128 == 0)) &&
+  const bool x32 = f32_ok && c.act == MI_F32 && (W.wk == WK_BF16 || (W.wk == WK_Q4_BF16 && W.group == 64 && W.K % 128 == 0) ||
+                                                 (W.wk == WK_Q8_BF16 && W.group == 64 && rows > 128)) &&
                    c.ldx % 4 == 0 && W.K % 4 == 0;
   if (!dense && !q4 && !q8 && !x32) return false;
   if (W.K % BK != 0 || (!x32 && c.ldx % 8 != 0)) return false;
@@ -1262,6 +1550,110 @@ int launch_split3_rows(const void* x, int ldx, const void* norm_w, float eps, vo
   return MI_OK;
 }
 
+// K slices of a 256 x 256 tile launch over `blocks` tiles: one 128-KiB workgroup per CU, so the launch runs in rounds of n_cu workgroups.  The
+// split whose last round is fullest, charging 2 % per extra slice for its partial tile and its share of the reduce (q|k|v at 1024 rows: 96
+// tiles -> 5 slices = 480 workgroups, 1.9 rounds; o_proj: 64 tiles -> 4 slices = one full round); at least 8 K tiles per slice.
+static int split256(long blocks, int ktiles, size_t slice_bytes, size_t cap) {
+  const int ncu = gemv_cu_count();
+  double best = 0.0;
+  int ks256 = 1;
+  for (int ks = 1; ks <= 8; ++ks) {
+    if (ks > 1 && (ktiles / ks < 8 || (size_t)ks * slice_bytes > cap)) break;
+    const long wgs = blocks * ks, rounds = (wgs + ncu - 1) / ncu;
+    const double score = (double)wgs / (double)(rounds * ncu) * (1.0 - 0.02 * (ks - 1));
+    if (score > best + 1e-9) { best = score; ks256 = ks; }
+  }
+  return ks256;
+}
+
+static int reduce_slices(const GemmParams& p, int act, hipStream_t st) {
+  const size_t total4 = (size_t)p.M * p.N / 4;
+  const dim3 rg((unsigned)((total4 + 255) / 256));
+  if (act == MI_F16) hipLaunchKernelGGL(splitk_epilogue_kernel<f16>, rg, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL(splitk_epilogue_kernel<bf16>, rg, dim3(256), 0, st, p);
+  MI_HIP(hipGetLastError());
+  return MI_OK;
+}
+
+size_t gemm_prefill_scratch_bytes(const LinearW& W, size_t rows) {
+  return std::max(dequant_hilo_bytes(W.N, W.K), codes16_bytes(W.N, W.K) + rows * codes16_bias_cols(W.K) * 2);
+}
+
+// Does gemm_codes256_kernel take this call of a quantised matrix?  It halves the products and the copy of the [hi | lo] form and costs a launch (the
+// group sums), the bias columns and a 256-row tile where the other has 128.  Whole calls, us, codes and [hi | lo], bf16 rows: 4096 x 4096 x
+// 129 rows 43 / 50, 28672 x 4096 SwiGLU 129 rows 196 / 317 and 700 rows 348 / 494, 4096 x 14336 x 700 144 / 221; 2048 x 5632 x 192 44 / 41, 256 44 / 50;
+// 4096 x 2048 x 768 47 / 53, 1536 59 / 101; 2048 x 1024 x 2048 43 / 43, 4096 57 / 55; 6144 x 1024 SwiGLU 768 57 / 54, 1536 60 / 82.  Float32 rows
+// (three walks against six): 2048 x 1024 x 768 42 / 42, 1536 55 / 62; 3072 x 1024 x 768 49 / 58.
+static bool codes_plan(const LinearW& W, const GemvCall& c, size_t rows, int ldx, int terms, bool split_ok, size_t cap, GemmParams& p, long& blocks) {
+  static const bool off = getenv("MI_GEMM_CODES") != nullptr && atoi(getenv("MI_GEMM_CODES")) == 0;       // A/B
+  const bool sw = c.epi == EPI_SWIGLU;
+  const int ncols = sw ? c.pair_offset : W.N;
+  if (off || !wk_is_quant(W.wk) || W.layout != 1 || W.group != 64 || W.K % BK != 0) return false;
+  if ((double)rows * W.N * W.K * terms < (W.K >= 4096 ? 2.1e9 : 4.3e9)) return false;
+  p.M = (int)rows; p.N = W.N; p.kw = W.K; p.ka = p.K = terms * W.K; p.ldx = ldx; p.G = W.K / 64;
+  p.kb = codes16_bias_cols(W.K);
+  // (32-bit offsets of the LDS-DMA sources)
+  const size_t lim = (size_t)1 << 32;
+  if (rows * (size_t)ldx * 2 >= lim || rows * (size_t)p.kb * 2 >= lim || (size_t)W.N * p.G * 4 >= lim) return false;
+  blocks = (long)((rows + BM2 - 1) / BM2) * ((ncols + (sw ? 128 : BN2) - 1) / (sw ? 128 : BN2));
+  p.ksplit = !sw && split_ok && W.N % 4 == 0 ? split256(blocks, (p.ka + p.kb) / BK, rows * W.N * sizeof(float), cap) : 1;
+  return true;
+}
+
+// Float32 rows against a quantised matrix: the tile GEMM, or 32 rows per launch of the streaming kernel?  us of both, fitted to 10 shapes of int4 and int8
+// within 20 %: a launch of the streaming kernel 10 + 0.36 per 2^20 weights (6144 x 4096 19.6, 28672 x 4096 40.6, 32000 x 4096 50); the codes' copy 0.65, a round
+// of workgroups 1.35 per K tile, the slices' reduce.  28672 x 4096 SwiGLU: 256 rows 363 against 325 streaming, 320 rows 405 / 406, 512 rows 425 / 650;
+// 6144 x 4096 96 rows 71 / 59, 160 rows 75 / 98.
+bool gemm_prefill_pays_codes(const LinearW& W, const GemvCall& c, size_t rows, int terms, size_t splitk_cap) {
+  GemmParams p{};
+  long blocks = 0;
+  if (!codes_plan(W, c, rows, terms * W.K, terms, splitk_cap > 0, splitk_cap, p, blocks))
+    return (c.rnd == RND_NONE && c.epi != EPI_STORE_F32) || gemm_prefill_pays(true, false, c.rnd != RND_NONE, rows);
+  const int ncu = gemv_cu_count(), tiles = ((p.ka + p.kb) / BK + p.ksplit - 1) / p.ksplit;
+  const double mw = (double)W.N * W.K / (1 << 20), rounds = (double)((blocks * p.ksplit + ncu - 1) / ncu);
+  const double reduce = p.ksplit > 1 ? 2e-6 * p.ksplit * rows * W.N : 0.0;
+  return 12.0 + 0.65 * mw + 1.35 * rounds * tiles + reduce < (double)((rows + 31) / 32) * (10.0 + 0.36 * mw);
+}
+
+// quantised matrices on gemm_codes256_kernel; *done = false: the [hi | lo] copy and the dense tiles take the call
+static int launch_gemm_codes(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st, void* scratch, void* splitk_ws, size_t splitk_cap, bool* done) {
+  *done = false;
+  const bool sw = c.epi == EPI_SWIGLU, x32 = c.act == MI_F32;
+  const int terms = x32 ? c.ldx / W.K : 1, ncols = sw ? c.pair_offset : W.N;
+  GemmParams p{};
+  long blocks = 0;
+  if (!codes_plan(W, c, rows, c.ldx, terms, splitk_ws != nullptr, splitk_cap, p, blocks)) return MI_OK;
+  p.x = c.x;
+  p.ws = (float*)splitk_ws;
+  MI_TRY(launch_codes16(W, scratch, st));
+  char* d = (char*)scratch;
+  p.w = d; p.wb = d + (size_t)W.N * W.K * 2; p.sc = (const float*)(d + (size_t)W.N * (W.K + p.kb) * 2);
+  uint16_t* xs = (uint16_t*)(d + codes16_bytes(W.N, W.K));
+  p.xs = xs;
+  if (c.act == MI_F16) hipLaunchKernelGGL(group_sums_kernel<f16>, dim3((unsigned)rows), dim3(256), p.G * sizeof(float), st, (const f16*)c.x, c.ldx, terms, W.K, xs, p.kb);
+  else hipLaunchKernelGGL(group_sums_kernel<bf16>, dim3((unsigned)rows), dim3(256), p.G * sizeof(float), st, (const bf16*)c.x, c.ldx, terms, W.K, xs, p.kb);
+  MI_HIP(hipGetLastError());
+  p.out32 = x32 || c.out32; p.rnd = x32 ? c.rnd : RND_NONE;
+  p.epi = c.epi; p.out = c.out; p.ldo = c.ldo; p.resid = c.resid; p.pair_offset = c.pair_offset; p.glu = c.glu; p.silu_cols = c.silu_cols;
+  if (c.epi == EPI_STORE_F32) {
+    p.epi = EPI_STORE;
+    if (!x32) { p.out32 = 1; p.rnd = c.act == MI_BF16 ? RND_BF16 : RND_F16; }
+  }
+  const dim3 grid((unsigned)((rows + BM2 - 1) / BM2), (ncols + (sw ? 128 : BN2) - 1) / (sw ? 128 : BN2), p.ksplit), block(512);
+  auto go = [&](auto k) -> int {
+    MI_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, CODES_LDS));
+    hipLaunchKernelGGL(k, grid, block, CODES_LDS, st, p);
+    MI_HIP(hipGetLastError());
+    return MI_OK;
+  };
+  const bool rounded = p.rnd != RND_NONE;               // (float32 stores of values rounded to 16 bits: logits, and layer 0 of the float32-cache mode)
+  if (c.act == MI_F16) MI_TRY(sw ? go(gemm_codes256_kernel<f16, true>) : rounded ? go(gemm_codes256_kernel<f16, false, true>) : go(gemm_codes256_kernel<f16, false>));
+  else MI_TRY(sw ? go(gemm_codes256_kernel<bf16, true>) : rounded ? go(gemm_codes256_kernel<bf16, false, true>) : go(gemm_codes256_kernel<bf16, false>));
+  if (p.ksplit > 1) MI_TRY(reduce_slices(p, c.act, st));
+  *done = true;
+  return MI_OK;
+}
+
 int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st, void* scratch, void* splitk_ws,
                         size_t splitk_cap) {
   if (c.pro != PRO_NONE) return fail(MI_ERR_INVALID, "gemm_prefill: normalise the rows first");
@@ -1270,6 +1662,10 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
   p.x = c.x; p.ldx = c.ldx; p.M = (int)rows; p.w = W.w; p.N = W.N; p.K = W.K; p.ka = W.K; p.kw = W.K;
   if (wk_is_quant(W.wk)) {
     if (scratch == nullptr) return fail(MI_ERR_INVALID, "gemm_prefill: int4 weights need a dequantisation scratch buffer");
+    const bool split_ok = c.act != MI_F32 || (c.ldx % W.K == 0 && (c.ldx == 3 * W.K || (c.ldx == W.K && c.rnd == RND_BF16)));
+    bool done = false;
+    if (split_ok) MI_TRY(launch_gemm_codes(W, c, rows, st, scratch, splitk_ws, splitk_cap, &done));
+    if (done) return MI_OK;
     MI_TRY(launch_dequant_q4_hilo(W, scratch, st));
     p.w = scratch; p.K = 2 * W.K; p.kw = 2 * W.K;
   }
@@ -1314,17 +1710,7 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
   const bool fold = x32 && c.rnd != RND_NONE;           // (plain stores: gemm_prefill_supported)
   const bool logits = !x32 && p.rnd != RND_NONE;
   if (rows >= 256 && !small_only && !fold && dma && splitk256 && !sw && splitk_ws != nullptr && W.N % 4 == 0) {
-    // one 128-KiB workgroup per CU: the launch runs in rounds of n_cu workgroups.  Pick the split whose last round is
-    // fullest, charging 2 % per extra slice for its partial tile and its share of the reduce (q|k|v at 1024 rows: 96
-    // tiles -> 5 slices = 480 workgroups, 1.9 rounds; o_proj: 64 tiles -> 4 slices = one full round)
-    const int ncu = gemv_cu_count();
-    double best = 0.0;
-    for (int ks = 1; ks <= 8; ++ks) {
-      if (ks > 1 && ((p.K / BK) / ks < 8 || (size_t)ks * rows * W.N * sizeof(float) > splitk_cap)) break;
-      const long wgs = blocks256 * ks, rounds = (wgs + ncu - 1) / ncu;
-      const double score = (double)wgs / (double)(rounds * ncu) * (1.0 - 0.02 * (ks - 1));
-      if (score > best + 1e-9) { best = score; ks256 = ks; }
-    }
+    ks256 = split256(blocks256, p.K / BK, rows * W.N * sizeof(float), splitk_cap);
   }
   if (rows >= 256 && !small_only && !fold && (blocks256 >= 192 || ks256 > 1)) {  // both operands through LDS (256 x 256 tile)
     const int bn = sw ? 128 : BN2;
@@ -1356,13 +1742,7 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
     else { if (sw) GO256(f16, true, false); else if (logits) GO256(f16, false, true); else GO256(f16, false, false); }
 #undef GO256
     MI_HIP(hipGetLastError());
-    if (p.ksplit > 1) {
-      const size_t total4 = rows * (size_t)W.N / 4;
-      const dim3 rg((unsigned)((total4 + 255) / 256));
-      if (c.act == MI_F16) hipLaunchKernelGGL(splitk_epilogue_kernel<f16>, rg, dim3(256), 0, st, p);
-      else hipLaunchKernelGGL(splitk_epilogue_kernel<bf16>, rg, dim3(256), 0, st, p);
-      MI_HIP(hipGetLastError());
-    }
+    if (p.ksplit > 1) MI_TRY(reduce_slices(p, c.act, st));
     return MI_OK;
   }
   dim3 grid(((int)rows + BM - 1) / BM, (ncols + (sw ? 64 : BN) - 1) / (sw ? 64 : BN)), block(256);
@@ -1389,13 +1769,7 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
     else hipLaunchKernelGGL((gemm_tile_kernel<f16, false>), grid, block, 0, st, p);
   }
   MI_HIP(hipGetLastError());
-  if (p.ksplit > 1) {
-    const size_t total4 = rows * (size_t)W.N / 4;
-    const dim3 rg((unsigned)((total4 + 255) / 256));
-    if (c.act == MI_F16) hipLaunchKernelGGL(splitk_epilogue_kernel<f16>, rg, dim3(256), 0, st, p);
-    else hipLaunchKernelGGL(splitk_epilogue_kernel<bf16>, rg, dim3(256), 0, st, p);
-    MI_HIP(hipGetLastError());
-  }
+  if (p.ksplit > 1) MI_TRY(reduce_slices(p, c.act, st));
   return MI_OK;
 }
 

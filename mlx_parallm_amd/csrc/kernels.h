@@ -86,6 +86,8 @@ bool gemm_prefill_supported(const LinearW& W, const GemvCall& c, size_t rows);
 // does the tile GEMM beat 32 rows per launch of the streaming kernel?  Logits and layer 0's rounded call on float32 activations only:
 // codes = int4 weights, hilo = the [hi | lo] copy of an f16 matrix
 bool gemm_prefill_pays(bool codes, bool hilo, bool rounded, size_t rows);
+// the same question for any call on a quantised matrix; terms: of x (launch_split3_rows)
+bool gemm_prefill_pays_codes(const LinearW& W, const GemvCall& c, size_t rows, int terms, size_t splitk_cap);
 // splitk_ws / splitk_cap: float32 workspace for the K-split form of the 128 x 128 tile (few hundred rows against a narrow
 // matrix); null = never split
 int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st, void* scratch = nullptr,
@@ -116,6 +118,21 @@ int launch_split3_rows(const void* x, int ldx, const void* norm_w, float eps, vo
 // int4 (tile-major) -> 16-bit tile-major [hi | lo], K' = 2K: the operand of the prefill GEMM for quantised weights
 size_t dequant_hilo_bytes(int N, int K);
 int launch_dequant_q4_hilo(const LinearW& src, void* dst, hipStream_t st);
+// the same matrices as 16-bit codes + biases + scales: the operands of the prefill GEMM on codes; codes16_bias_cols: its columns of group sums
+int codes16_bias_cols(int K);
+size_t codes16_bytes(int N, int K);
+int launch_codes16(const LinearW& src, void* dst, hipStream_t st);
+// term t of that product: part of x's group sum (0 = hi, 1 = mid, 2 = lo) and of the bias; products below 2^-24 of the whole are left out
+constexpr int CODES16_TERMS = 6;
+__host__ __device__ constexpr int codes16_sum_part(int t) { return t < 3 ? t : t == 5 ? 0 : t - 3; }
+__host__ __device__ constexpr int codes16_bias_part(int t) { return t < 3 ? 0 : t < 5 ? 1 : 2; }
+// v = hi + mid + lo in bf16 (an infinity is its own first part)
+__device__ __forceinline__ float bf16_part(float v, int part) {
+  const float hi = (float)(bf16)v, r = isinf(v) ? 0.f : v - hi, mid = (float)(bf16)r;
+  return part == 0 ? hi : part == 1 ? mid : r - mid;
+}
+// `scratch` bytes of launch_gemm_prefill for a quantised matrix
+size_t gemm_prefill_scratch_bytes(const LinearW& W, size_t rows);
 // block_per_row: one workgroup per row, row in registers -- for the few rows of a decode step (default: one wave
 // per row, the prefill's kernel; the two add the squares in different orders)
 // act = MI_F32: float32 rows and weights with the run-time logical rounding `rnd` (PagedKVCache mode)

@@ -149,6 +149,42 @@ int mi_op_gemm_prefill(const mi_op_linear* w, const mi_op_gemv_args* a, int iter
   return rc != MI_OK ? rc : rc2;
 }
 
+int mi_op_gemm_codes(const mi_op_linear* w, const mi_op_gemv_args* a, int iters, float* avg_ms) {
+  if (!w || !a) return fail(MI_ERR_INVALID, "null argument");
+  MI_TRY(ready());
+  const LinearW W = to_linear(w);
+  GemvCall c = to_call(a);
+  if (c.M < 1 || c.pro != PRO_NONE || !wk_is_quant(W.wk) || !gemm_prefill_supported(W, c, (size_t)c.M))
+    return fail(MI_ERR_UNSUPPORTED, "mi_op_gemm_codes: tile-major int4 / int8 weights (group 64), at least 32 rows, no prologue");
+  void *ws = nullptr, *scratch = nullptr, *xs = nullptr;
+  size_t cap = 0;
+  auto done = [&](int rc) { hipFree(ws); hipFree(scratch); hipFree(xs); return rc; };
+  if (c.M < 4096) { cap = (size_t)128 << 20; if (hipMalloc(&ws, cap) != hipSuccess) return done(fail(MI_ERR_RUNTIME, "mi_op_gemm_codes: workspace")); }
+  if (hipMalloc(&scratch, gemm_prefill_scratch_bytes(W, (size_t)c.M)) != hipSuccess) return done(fail(MI_ERR_RUNTIME, "mi_op_gemm_codes: scratch"));
+  int rc = MI_OK;
+  if (c.act == MI_F32) {                               // float32 activations: three bf16 terms (layer 0's rounded call: one)
+    const int terms = c.rnd == RND_BF16 ? 1 : 3;
+    if (hipMalloc(&xs, split3_bytes((size_t)c.M, W.K)) != hipSuccess) return done(fail(MI_ERR_RUNTIME, "mi_op_gemm_codes: split rows"));
+    rc = launch_split3_rows(c.x, c.ldx, nullptr, 0.f, xs, c.M, W.K, nullptr, terms, c.rnd);
+    c.x = xs; c.ldx = terms * W.K;
+  }
+  if (rc == MI_OK) rc = launch_gemm_prefill(W, c, (size_t)c.M, nullptr, scratch, ws, cap);
+  if (rc == MI_OK && iters >= 1 && avg_ms) {
+    hipEvent_t e0, e1;
+    hipEventCreate(&e0); hipEventCreate(&e1);
+    hipEventRecord(e0, nullptr);
+    for (int i = 0; i < iters && rc == MI_OK; ++i) rc = launch_gemm_prefill(W, c, (size_t)c.M, nullptr, scratch, ws, cap);
+    hipEventRecord(e1, nullptr);
+    hipEventSynchronize(e1);
+    float ms = 0.f;
+    hipEventElapsedTime(&ms, e0, e1);
+    *avg_ms = ms / iters;
+    hipEventDestroy(e0); hipEventDestroy(e1);
+  }
+  const int rc2 = finish();
+  return done(rc != MI_OK ? rc : rc2);
+}
+
 int mi_op_gemv_reg(const mi_op_linear* w, const mi_op_gemv_args* a) {
   if (!w || !a) return fail(MI_ERR_INVALID, "null argument");
   MI_TRY(ready());

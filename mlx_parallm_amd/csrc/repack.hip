@@ -134,7 +134,81 @@ __global__ void dequant_q8_hilo_kernel(const uint8_t* src, T* dst, int N, int K)
   }
 }
 
+// tile-major int4 / int8 -> the operands of the tile GEMM on codes (gemm_prefill.hip: gemm_codes256_kernel):
+//   codes  [N/16][K/32] KiB blocks of 16-bit integers (of T: -128..127 are exact in bf16 and f16), code - 8 (int4) or - 128 (int8), dense layout
+//   wb     [N/16][kb/32] KiB blocks of bf16: what meets the group sums of x, column c = term * K/64 + group: a part (codes16_bias_part) of
+//          bias + 8 s (128 s); zeros up to kb
+//   sc     [N/16][K/64][16] float32: the scales
+// Bound by its writes (2 bytes a code, half of the [hi | lo] copy's).
+template <typename T, int BITS>
+__global__ __launch_bounds__(256) void codes16_kernel(const uint8_t* src, T* codes, uint16_t* wb, float* sc, int N, int K, int kb) {
+  constexpr int MID = BITS == 4 ? 8 : 128;
+  const int G = K / 64;
+  const size_t pc = (size_t)N * (K / 8), pb = (size_t)N * (kb / 8), ps = (size_t)N * G;
+  auto at = [&](size_t row, int k) { return src + (BITS == 4 ? tiled_block_q4(row, k, K) : tiled_block_q8(row, k, K)); };
+  auto scale = [&](size_t row, int k) { return (const T*)(at(row, k) + (BITS == 4 ? tiled_q4_scale_off(row, k) : tiled_q8_scale_off(row))); };
+  for (size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x; idx < pc + pb + ps; idx += (size_t)gridDim.x * 256) {
+    if (idx < pc) {
+      const size_t blk = idx >> 6;
+      const int lane = (int)(idx & 63), r = lane & 15, g = lane >> 4;
+      const size_t i = blk / (K / 32), row = i * 16 + r;
+      const int k = (int)(blk % (K / 32)) * 32 + g * 8;
+      T v[8];
+      if constexpr (BITS == 4) {
+        const uint32_t q = *(const uint32_t*)(at(row, k) + tiled_q4_code_off(row, k));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = (T)(float)((int)((q >> (4 * e)) & 15u) - MID);
+      } else {
+        const uint2 q = *(const uint2*)(at(row, k) + tiled_q8_code_off(row, k));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = (T)(float)((int)(((e < 4 ? q.x : q.y) >> (8 * (e & 3))) & 255u) - MID);
+      }
+      *(u32x4*)(codes + idx * 8) = *(const u32x4*)v;
+    } else if (idx < pc + pb) {
+      const size_t o = idx - pc, blk = o >> 6;
+      const int lane = (int)(o & 63), r = lane & 15, g = lane >> 4;
+      const size_t i = blk / (kb / 32), row = i * 16 + r;
+      const int c0 = (int)(blk % (kb / 32)) * 32 + g * 8;
+      __bf16 v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int term = (c0 + e) / G, grp = (c0 + e) - term * G;
+        float b = 0.f;
+        if (term < CODES16_TERMS) {
+          const T* sb = scale(row, grp * 64);
+          b = bf16_part(fmaf((float)MID, (float)sb[0], (float)sb[BITS == 4 ? 32 : 16]), codes16_bias_part(term));
+        }
+        v[e] = (__bf16)b;
+      }
+      *(u32x4*)(wb + o * 8) = *(const u32x4*)v;
+    } else {
+      const size_t o = idx - pc - pb, blk = o >> 4;                  // (tile, group), row in tile
+      sc[o] = (float)*scale((blk / G) * 16 + (o & 15), (int)(blk % G) * 64);
+    }
+  }
+}
+
 }  // namespace
+
+int codes16_bias_cols(int K) { return (CODES16_TERMS * (K / 64) + 63) / 64 * 64; }
+size_t codes16_bytes(int N, int K) { return (size_t)N * ((size_t)K * 2 + (size_t)codes16_bias_cols(K) * 2 + (size_t)(K / 64) * 4); }
+
+int launch_codes16(const LinearW& src, void* dst, hipStream_t st) {
+  const int bits = wk_bits(src.wk), sdt = wk_scale_dtype(src.wk);
+  if (src.layout != 1 || (bits != 4 && bits != 8) || sdt == WK_F32 || src.group != 64 || src.K % (bits == 4 ? 128 : 64) != 0 || src.N % 16 != 0)
+    return fail(MI_ERR_UNSUPPORTED, "codes16: tile-major int4 / int8 (group 64) matrices only");
+  const int kb = codes16_bias_cols(src.K);
+  char* d = (char*)dst;
+  void* codes = d;
+  uint16_t* wb = (uint16_t*)(d + (size_t)src.N * src.K * 2);
+  float* sc = (float*)(d + (size_t)src.N * (src.K + kb) * 2);
+#define GO(T, B) hipLaunchKernelGGL((codes16_kernel<T, B>), dim3(4096), dim3(256), 0, st, (const uint8_t*)src.w, (T*)codes, wb, sc, src.N, src.K, kb)
+  if (sdt == WK_BF16) { if (bits == 4) GO(bf16, 4); else GO(bf16, 8); }
+  else { if (bits == 4) GO(f16, 4); else GO(f16, 8); }
+#undef GO
+  MI_HIP(hipGetLastError());
+  return MI_OK;
+}
 
 size_t dequant_hilo_bytes(int N, int K) { return (size_t)N * K * 2 * 2; }
 

@@ -1,0 +1,103 @@
+"""Kernel-level parity (-m gpu) of the tile GEMM on int4 / int8 codes (gemm_prefill.hip: gemm_codes256_kernel, the nn.QuantizedLinear of
+the prefill call, utils.py:243-262,679-690) through mi_op_gemm_codes: against the oracle's matmul over the dequantised weights on
+sampled rows, for every epilogue, at the edges of tiles and runs."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import ref_quant
+from oracle.numerics import matmul_nt, round_to
+
+pytestmark = pytest.mark.gpu
+
+from mlx_parallm_amd import _lib as L  # noqa: E402
+from gpu_helpers import dev, dev_u32, gemv_args, host, op_linear, to_tiled  # noqa: E402
+from test_gpu_gemm_prefill import _rows  # noqa: E402
+from test_gpu_kernels import _assert_close  # noqa: E402
+
+
+def _weight(bits, sdt, N, K, rng):
+    """groups whose mean is up to four of their own deviations: the bias term is no small one"""
+    w = (rng.standard_normal((N, K // 64, 64)) + 4 * rng.standard_normal((N, K // 64, 1))).astype(np.float32) * 0.05
+    packed, s, b = ref_quant.quantize(round_to(w.reshape(N, K), sdt), 64, bits, sdt)
+    kind = f"q{bits}_" + {"bfloat16": "bf16", "float16": "f16"}[sdt]
+    keep = [dev_u32(packed), dev(s, sdt), dev(b, sdt)]
+    ol = op_linear(kind, N, K, *keep)
+    assert to_tiled(ol, keep)
+    return ol, ref_quant.dequantize(packed, s, b, 64, bits), keep
+
+
+def _run(ol, x, M, act, rnd=0, **kw):
+    a = gemv_args(x, M, act, **kw)
+    a.rnd = rnd
+    torch.cuda.synchronize()
+    L.check(L.lib().mi_op_gemm_codes(C.byref(ol), C.byref(a), 0, None))
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("act", ["bfloat16", "float16"])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M,N,K", [
+    (256, 2048, 1024),       # one row tile, K split: slices that end inside a run
+    (300, 2064, 1152),       # ragged rows, a column tile of 16, 18 groups (the bias columns end inside a K tile)
+    (2085, 6144, 128),       # two groups: a run that is all prologue, unsplit
+    (2304, 5632, 640),       # an even number of groups, unsplit
+])
+def test_store_logits_and_residual(act, bits, M, N, K):
+    rng = np.random.default_rng(1000 * bits + M)
+    ol, w, keep = _weight(bits, act, N, K, rng)
+    x = round_to(rng.standard_normal((M, K)).astype(np.float32), act)
+    h0 = round_to(rng.standard_normal((M, N)).astype(np.float32), act)
+    xd, rows = dev(x, act), _rows(M)
+    y = round_to(matmul_nt(x[rows], w), act)
+    out = torch.full((M + 3, N), 7.0, dtype=xd.dtype, device="cuda")
+    _run(ol, xd, M, act, epi=L.EPI_STORE, out=out, ldo=N)
+    o = host(out)
+    assert np.all(o[M:] == 7.0), "rows past M were written"
+    _assert_close(o[:M][rows], y, act)
+    lg = torch.full((M + 3, N), 7.0, dtype=torch.float32, device="cuda")          # logits: the same values as float32
+    _run(ol, xd, M, act, epi=L.EPI_STORE_F32, out=lg, ldo=N)
+    assert np.array_equal(host(lg)[:M], o[:M]) and np.all(host(lg)[M:] == 7.0)
+    h = dev(h0, act)
+    _run(ol, xd, M, act, epi=L.EPI_RESID, resid=h, out=h, ldo=N)
+    _assert_close(host(h)[rows], round_to(h0[rows] + y, act), act)
+
+
+@pytest.mark.parametrize("act,bits,M,I,K", [("bfloat16", 4, 2085, 3072, 512), ("bfloat16", 8, 517, 8208, 192), ("float16", 4, 2048, 3200, 256)])
+def test_swiglu(act, bits, M, I, K):
+    rng = np.random.default_rng(M)
+    ol, w, keep = _weight(bits, act, 2 * I, K, rng)
+    x = round_to(rng.standard_normal((M, K)).astype(np.float32) * 0.3, act)
+    xd, rows = dev(x, act), _rows(M)
+    y = round_to(matmul_nt(x[rows], w), act)
+    gt, up = y[:, :I].astype(np.float64), y[:, I:]
+    sig = round_to((1.0 / (1.0 + np.exp(-gt))).astype(np.float32), act)
+    want = round_to(round_to(gt.astype(np.float32) * sig, act) * up, act)
+    out = torch.full((M + 1, I), 7.0, dtype=xd.dtype, device="cuda")
+    _run(ol, xd, M, act, epi=L.EPI_SWIGLU, out=out, ldo=I, pair_offset=I)
+    o = host(out)
+    assert np.all(o[M:] == 7.0)
+    _assert_close(o[:M][rows], want, act, scale=float(np.abs(y).max()))
+
+
+@pytest.mark.parametrize("M,N,K,rnd", [(300, 2048, 1024, 0), (2085, 6144, 256, 0), (1024, 6144, 640, L.RND_BF16)])
+def test_float32_rows(M, N, K, rnd):
+    """three bf16 terms of x (a run over the codes per term); rnd: layer 0's rounded call, x is one term"""
+    rng = np.random.default_rng(K)
+    ol, w, keep = _weight(4, "bfloat16", N, K, rng)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    if rnd:
+        x = round_to(x, "bfloat16")
+    rows = _rows(M)
+    want = matmul_nt(x[rows], w)
+    out = torch.full((M + 1, N), 7.0, dtype=torch.float32, device="cuda")
+    _run(ol, dev(x), M, "float32", rnd=rnd, epi=L.EPI_STORE, out=out, ldo=N)
+    o = host(out)
+    assert np.all(o[M:] == 7.0)
+    if rnd:
+        _assert_close(o[:M][rows], round_to(want, "bfloat16"), "bfloat16")
+    else:
+        # exact products; K / 64 + 2 float32 additions of a group's sums and the biases', of up to 16 scales x |x| each
+        assert np.max(np.abs(o[:M][rows] - want)) <= 2.0 ** -24 * (K / 64 + 8) * 4 * np.abs(x[rows]).sum(1).max() * np.abs(w).max()
