@@ -1,0 +1,35 @@
+"""gemm_q4.hip (-m gpu) where its loops turn: more than 16 blocks of 128 k per K lane (the biases' products run twice), lanes with unequal numbers of
+blocks, three row tiles, slices of K, tiles that end inside a workgroup's ten.  Against the oracle's matmul over the dequantised weights."""
+import numpy as np
+import pytest
+import torch
+
+from oracle.numerics import matmul_nt, round_to
+
+pytestmark = pytest.mark.gpu
+
+from mlx_parallm_amd import _lib as L  # noqa: E402
+from gpu_helpers import dev, gemm_skinny, host, q4_force  # noqa: E402
+from test_gpu_gemm_codes import _weight  # noqa: E402
+from test_gpu_kernels import _assert_close  # noqa: E402
+
+
+@pytest.mark.parametrize("act", ["bfloat16", "float16"])
+@pytest.mark.parametrize("M,N,K,mt,ks", [
+    (33, 176, 128 * 67, 3, 1),       # 17, 17, 17 and 16 blocks a lane
+    (64, 160, 128 * 129, 4, 2),      # two slices of 64 and 65
+    (17, 336, 128 * 2, 2, 1),        # two of four lanes without a block
+    (128, 96, 128 * 5, 4, 3),        # two slabs, slices of one and two blocks
+])
+def test_block_counts_and_slices(act, M, N, K, mt, ks):
+    rng = np.random.default_rng(K + M)
+    ol, w, keep = _weight(4, act, N, K, rng)
+    x = round_to(rng.standard_normal((M, K)).astype(np.float32), act)
+    xd = dev(x, act)
+    outs = []
+    for _ in range(2):
+        out = torch.full((M + 2, N), 7.0, dtype=xd.dtype, device="cuda")
+        gemm_skinny(ol, xd, M, act, epi=L.EPI_STORE, out=out, ldo=N, ksplit=q4_force(mt=mt, ksplit=ks))
+        outs.append(host(out))
+    assert np.array_equal(outs[0], outs[1]) and np.all(outs[0][M:] == 7.0)
+    _assert_close(outs[0][:M], round_to(matmul_nt(x, w), act), act)

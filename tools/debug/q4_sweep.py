@@ -1,6 +1,5 @@
 #!/usr/bin/env python3
-"""Times gemm_q4.hip's plans on the linears of one decoder block (int4 g64, bf16 activations) next to the split-K kernel it
-replaces (gemm_skinny.hip with its cost model: run the same command with MI_Q4=0 for that column).
+"""Times gemm_q4.hip's plans on the linears of one decoder block (int4 g64, bf16 activations).
 
     python tools/debug/q4_sweep.py [--model qwen3-14b] [--rows 64] [--iters 30] [--plans auto|all]
 """
