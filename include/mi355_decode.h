@@ -360,6 +360,8 @@ int mi_profile_read(mi_engine* e, int64_t* n_launches, double* total_ms);
  *                             staging of the next (default 1)
  *   "defer_norm"              0: float32-activation (PagedKVCache mode) decode steps run the RMSNorm as its own launch
  *                             instead of applying its row scale in the epilogue of the linear behind it (default 1)
+ *   "prefill_split_act"       0: that prefill's gate|up stores its SwiGLU as float32 and the down projection splits it in a pass of its own
+ *                             (default 1: stored as the two terms; the same bits)
  *   "prefill_x_terms"         3: float32-activation (PagedKVCache mode) prefill multiplies an EXACT three-term 16-bit split of x
  *                             by dense bf16 weights (three walks of W); default 2: hi + lo, 16+ mantissa bits of x, two walks
  *                             (the CPU float32-accumulating variants do not move under it: DESIGN 8d); int4 always 3

@@ -217,6 +217,13 @@ bool ensure_gu8(mi_engine* e, FusedLinear& f, int pair_offset) {
   return true;
 }
 
+// Float32-cache mode, a prompt: does the down projection read its input as the two bf16 terms that gate|up can leave in its place?  (Dense bf16, no
+// adapter -- that reads the float32 row --, the tile GEMM with two terms of x)
+bool down_takes_split(const mi_engine* e, const FusedLinear& down, int act, size_t rows) {
+  return act == MI_F32 && rows >= 256 && e->opt_prefill_gemm && !e->opt_force_v1 && e->opt_prefill_x_terms == 2 && e->opt_prefill_split_act && down.W.wk == WK_BF16 &&
+         down.W.layout == 1 && down.W.K % 64 == 0 && down.W.lora_b[0] == nullptr && down.W.lora_b[1] == nullptr;
+}
+
 // y = W x for `rows` rows, split into launches of at most 16 (MFMA) / 8 (generic) rows
 int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, GemvCall c, size_t rows, size_t es_in, size_t es_out,
                  const char* prof, bool sq_was_valid);
@@ -226,6 +233,7 @@ int gemv_rows(mi_engine* e, const FusedLinear& f0, GemvCall c, size_t rows, size
   if (c.act == MI_F32) c.out32 = 0;           // (float32 storage already)
   const bool sq_was_valid = e->sq_valid;      // whatever runs now consumes or invalidates the hand-over
   e->sq_valid = false;
+  e->act_split = false;
   // An f16 model in the PagedKVCache mode (float32 activations): the matrix-core kernels of that mode multiply an exact
   // three-way bf16 split of x by bf16 weights, so an f16 matrix is used through its exact [hi | lo] bf16 copy (2 K
   // columns, x walked twice: GemvCall::kx) -- made by mi_engine_finalize (here only if the option was switched on later),
@@ -401,8 +409,15 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
       // w = s q + b exactly while |w| <= 2^16 ulp(s), i.e. |b| up to some 2^9 scales -- int4 groups whose mean is up to 30 of their own standard
       // deviations, int8 groups up to 3 (quantised on the CPU and compared) -- and w to 2^-17 beyond; of f16, int4 groups to 1000.
       const int terms = c.rnd == RND_BF16 ? 1 : (e->opt_prefill_x_terms == 2 && f.W.wk == WK_BF16 && c.kx == 0 && c.rnd == RND_NONE && c.epi != EPI_STORE_F32) ? 2 : 3;
-      MI_TRY(launch_split3_rows(c.x, c.ldx, c.pro == PRO_NORM ? c.norm_w : nullptr, c.eps, e->xs, (int)rows, KT, e->stream, terms, c.rnd));
-      c.x = e->xs; c.ldx = terms * KT; c.pro = PRO_NONE;
+      if (c.x_split) {
+        if (terms != 2 || c.pro != PRO_NONE) return fail(MI_ERR_INVALID, "split rows in front of a call that multiplies other terms");
+      } else {
+        MI_TRY(launch_split3_rows(c.x, c.ldx, c.pro == PRO_NORM ? c.norm_w : nullptr, c.eps, e->xs, (int)rows, KT, e->stream, terms, c.rnd));
+        c.x = e->xs;
+      }
+      c.ldx = terms * KT; c.pro = PRO_NONE;
+      c.split_out = c.split_out && gemm_prefill_split_out(f.W, c, rows);
+      e->act_split = c.split_out != 0;
     } else if (c.pro == PRO_NORM) {    // (one workgroup per row also here: one L2 round trip per row instead of a wave's 16)
       MI_TRY(launch_rmsnorm_rows(c.x, c.ldx, c.norm_w, e->xn, KT, (int)rows, KT, c.eps, c.act, e->stream, true));
       c.x = e->xn; c.ldx = KT; c.pro = PRO_NONE;
@@ -445,6 +460,7 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
     }
     return MI_OK;
   }
+  if (c.x_split) return fail(MI_ERR_INVALID, "split rows in front of a call that reads float32");
   if (e->opt_skinny_gemm && c.act == MI_F32 && rows > 32 && gemm_skinny_supported(f.W, c, 32)) {
     // PagedKVCache mode, more than 32 rows: 32 rows per launch of the float32-activation streaming kernel (each row's arithmetic is
     // that of a decode step, whatever the batch), where that is ahead of the tile GEMM; the generic kernel took 8 rows per pass over W.
@@ -843,6 +859,7 @@ int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool wan
       // post_attention_layernorm + gate|up + SwiGLU (llama.py:189,165)
       GemvCall cg; cg.x = e->h; cg.ldx = H; cg.act = act; cg.rnd = RND_NONE; cg.pro = PRO_NORM; cg.norm_w = post_norm;
       cg.eps = d.rms_norm_eps; cg.epi = EPI_SWIGLU; cg.out = e->act; cg.ldo = I; cg.pair_offset = I;
+      cg.split_out = down_takes_split(e, lw.down, act, R);
       if ((e->opt_fused_pairs & 1) && can_pair(e, lw.o, co, lw.gate_up, cg, R)) {
         MI_TRY(gemv_pair(e, lw.o, co, lw.gate_up, cg, R, "gemv_o_gate_up"));
       } else {
@@ -851,7 +868,7 @@ int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool wan
       }
     }
     {  // down_proj + residual (llama.py:165,190); with the next layer's q|k|v behind it in the same launch
-      GemvCall c; c.x = e->act; c.ldx = I; c.act = act; c.rnd = RND_NONE; c.epi = EPI_RESID; c.resid = e->h; c.ldo = H;
+      GemvCall c; c.x = e->act; c.ldx = I; c.act = act; c.rnd = RND_NONE; c.epi = EPI_RESID; c.resid = e->h; c.ldo = H; c.x_split = e->act_split;
       if ((e->opt_fused_pairs & 2) && li + 1 < d.num_layers &&
           can_pair(e, lw.down, c, e->layers[li + 1].qkv, qkv_call(li + 1), R)) {
         MI_TRY(gemv_pair(e, lw.down, c, e->layers[li + 1].qkv, qkv_call(li + 1), R, "gemv_down_qkv"));
@@ -977,8 +994,9 @@ int forward_mixed(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t* l
       MI_TRY(gemv_rows(e, lw.o, co, R, es, es, "gemv_o"));
       GemvCall cg; cg.x = e->h; cg.ldx = H; cg.act = act; cg.rnd = RND_NONE; cg.pro = PRO_NORM; cg.norm_w = post_norm;
       cg.eps = d.rms_norm_eps; cg.epi = EPI_SWIGLU; cg.out = e->act; cg.ldo = I; cg.pair_offset = I;
+      cg.split_out = down_takes_split(e, lw.down, act, R);
       MI_TRY(gemv_rows(e, lw.gate_up, cg, R, es, es, "gemv_gate_up"));
-      GemvCall c; c.x = e->act; c.ldx = I; c.act = act; c.rnd = RND_NONE; c.epi = EPI_RESID; c.resid = e->h; c.ldo = H;
+      GemvCall c; c.x = e->act; c.ldx = I; c.act = act; c.rnd = RND_NONE; c.epi = EPI_RESID; c.resid = e->h; c.ldo = H; c.x_split = e->act_split;
       MI_TRY(gemv_rows(e, lw.down, c, R, es, es, "gemv_down")); }
   }
   if (n_out > 0) {                               // hidden states of the wanted positions -> compact rows -> head
@@ -1767,6 +1785,7 @@ int mi_engine_set_option(mi_engine* e, const char* key, int64_t value) {
   if (k == "norm_handover") { e->opt_norm_handover = value != 0; return MI_OK; }
   if (k == "defer_norm") { e->opt_defer_norm = value != 0; return MI_OK; }
   if (k == "prefill_x_terms") { if (value != 2 && value != 3) return fail(MI_ERR_INVALID, "prefill_x_terms: 2 or 3"); e->opt_prefill_x_terms = (int)value; return MI_OK; }
+  if (k == "prefill_split_act") { e->opt_prefill_split_act = value != 0; return MI_OK; }
   if (k == "short_prefill_skinny") { e->opt_short_prefill_skinny = value != 0; return MI_OK; }
   if (k == "decode_attention_mfma") { e->opt_attn_mfma = value != 0; return MI_OK; }
   if (k == "fused_gemv_pairs") { e->opt_fused_pairs = (int)value; return MI_OK; }

@@ -56,6 +56,7 @@ struct GemmParams {
                                     // every (x part, W part) pair once.
   int out32;                        // outputs / residual stream are float32 (PagedKVCache mode), no 16-bit rounding
   int rnd;                          // .. but for a plain store with logical rounding (layer 0 of that mode: RND_*)
+  int split_out;                    // .. or a SwiGLU stored as two bf16 terms (256 x 256 LDS-DMA tile only)
   int epi; void* out; int ldo; void* resid; int pair_offset;
   Glu glu; int silu_cols;
   // 128 x 128 tile only: K split over gridDim.z workgroups when the (M, N) grid alone leaves most CUs idle (a prompt of a
@@ -71,11 +72,14 @@ struct GemmParams {
 };
 
 // the epilogues in float32 storage (PagedKVCache mode after layer 0: every op produces a float32 array)
-__device__ __forceinline__ void epi32_swiglu(const GemmParams& p, int m, int n, float gt, float up) {
-  if (p.glu.kind != GLU_SILU) { ((float*)p.out)[(size_t)m * p.ldo + n] = glu_f(p.glu, gt, up); return; }
+__device__ __forceinline__ float glu32(const Glu& c, float gt, float up) {
+  if (c.kind != GLU_SILU) return glu_f(c, gt, up);
   const float sig = 1.0f / (1.0f + expf(-gt));
   const float sl = gt * sig;
-  ((float*)p.out)[(size_t)m * p.ldo + n] = sl * up;
+  return sl * up;
+}
+__device__ __forceinline__ void epi32_swiglu(const GemmParams& p, int m, int n, float gt, float up) {
+  ((float*)p.out)[(size_t)m * p.ldo + n] = glu32(p.glu, gt, up);
 }
 __device__ __forceinline__ void epi32_plain(const GemmParams& p, int m, int n, float y) {
   if (p.epi == EPI_STORE) ((float*)p.out)[(size_t)m * p.ldo + n] = y;
@@ -349,6 +353,31 @@ __device__ __forceinline__ void tile256_epilogue(const GemmParams& p, f32x4 (&ac
             h[(size_t)m * p.ldo + n] = (AT)((float)h[(size_t)m * p.ldo + n] + y);
           }
         }
+      }
+    }
+}
+
+// SwiGLU in float32 as two bf16 terms, hi = bf16(y), lo = bf16(y - hi): what the down projection multiplies.  Stored here they are the bytes of the
+// float32 row; a pass that split it (8192 x 14336: 157 us) is saved.  Neighbouring lanes hold neighbouring columns: the even one takes both hi, the odd
+// one both lo, a store of 4 bytes each.
+__device__ __forceinline__ void tile256_epilogue_split(const GemmParams& p, f32x4 (&acc)[8][4], int m0, int bn, int wm, int wn, int c16, int g) {
+  uint16_t* out = (uint16_t*)p.out;
+  const bool odd = c16 & 1;
+#pragma unroll
+  for (int mt = 0; mt < 8; ++mt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int m = m0 + wm * 128 + mt * 16 + 4 * g + r;
+      if (m >= p.M) continue;                                    // (16 lanes of a row, and below of a tile, together)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int n = bn * 128 + wn * 32 + j * 16 + c16;
+        if (n >= p.pair_offset) continue;
+        const float y = glu32(p.glu, acc[mt][j][r], acc[mt][j + 2][r]);
+        const bf16 hi = (bf16)y, lo = (bf16)(y - (float)hi);
+        const uint32_t h = __builtin_bit_cast(uint16_t, hi), l = __builtin_bit_cast(uint16_t, lo);
+        const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(odd ? h : l), 0xB1, 0xf, 0xf, false);      // quad_perm:[1,0,3,2]
+        *(uint32_t*)(out + (size_t)m * (2 * p.ldo) + (odd ? p.ldo + n - 1 : n)) = odd ? got | (l << 16) : h | (got << 16);
       }
     }
 }
@@ -822,6 +851,9 @@ __global__ __launch_bounds__(512) void gemm_dma256_kernel(GemmParams p) {
       else tile256_epilogue_resid<AT, AT>(p, acc, m0, bn, wm, wn, c16, g);
       return;
     }
+  }
+  if constexpr (SWIGLU && !GROUPED && std::is_same<AT, bf16>::value) {
+    if (p.split_out) { tile256_epilogue_split(p, acc, m0, bn, wm, wn, c16, g); return; }
   }
   if constexpr (GROUPED) {
     __syncthreads();
@@ -1654,6 +1686,15 @@ static int launch_gemm_codes(const LinearW& W, const GemvCall& c, size_t rows, h
   return MI_OK;
 }
 
+static bool gemm_small_only() { static const bool v = getenv("MI_GEMM_TILE128") != nullptr; return v; }        // A/B: always the 128 x 128 kernel
+static bool gemm_dma_on() { const char* v = getenv("MI_GEMM_DMA"); return v == nullptr || atoi(v) != 0; }      // A/B and the bit-equality test: 0 = the register-staged tile (read per call)
+
+bool gemm_prefill_split_out(const LinearW& W, const GemvCall& c, size_t rows) {
+  if (c.act != MI_F32 || c.epi != EPI_SWIGLU || c.kx > 0 || W.wk != WK_BF16 || c.pair_offset % 2 != 0 || rows < BM2) return false;
+  const long blocks256 = (long)((rows + BM2 - 1) / BM2) * ((c.pair_offset + 127) / 128);
+  return !gemm_small_only() && gemm_dma_on() && blocks256 >= 192 && 2 * W.K >= 2 * BK;
+}
+
 int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st, void* scratch, void* splitk_ws,
                         size_t splitk_cap) {
   if (c.pro != PRO_NONE) return fail(MI_ERR_INVALID, "gemm_prefill: normalise the rows first");
@@ -1693,14 +1734,15 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
   p.glu = c.glu; p.silu_cols = c.silu_cols;
   const bool sw = c.epi == EPI_SWIGLU;
   const int ncols = sw ? c.pair_offset : W.N;
-  static const bool small_only = getenv("MI_GEMM_TILE128") != nullptr;        // A/B: always the 128 x 128 kernel
+  const bool small_only = gemm_small_only();
   static const bool b_in_lds = getenv("MI_GEMM_B_DIRECT") == nullptr;         // A/B: set = W fragments straight from global
   // The 256 x 256 tile only where its grid fills the chip: at 8 x 1024 rows every linear has >= 512 blocks, but one prompt
   // of 256..1024 tokens gives N/256 x (1..4) blocks -- 16..64 for N = 4096 -- and measured 25 / 25 / 30 ms for 256 / 512 /
   // 1024 tokens against 14 / 17 / 23 ms on the 128 x 128 tile (Mistral-7B bf16; tools/debug/prefill_sweep.py).
   const long blocks256 = (long)(((int)rows + BM2 - 1) / BM2) * ((ncols + (sw ? 128 : BN2) - 1) / (sw ? 128 : BN2));
-  const char* dma_env = getenv("MI_GEMM_DMA");         // A/B and the bit-equality test: 0 = the register-staged tile (read per call)
-  const bool dma = dma_env == nullptr || atoi(dma_env) != 0;
+  const bool dma = gemm_dma_on();
+  if (c.split_out && !gemm_prefill_split_out(W, c, rows)) return fail(MI_ERR_INVALID, "gemm_prefill: this call does not store split rows");
+  p.split_out = c.split_out;
   // too few 256 x 256 tiles for the chip (one prompt of 256..4095 rows against N = 4096 / 6144): the LDS-DMA tile with K
   // split over up to 8 workgroups, each >= 8 K tiles (plain / residual epilogues; SwiGLU launches have enough tiles or
   // stay on the 128 x 128 kernel).  MI_GEMM_DMA_SPLITK=0 switches it off (A/B).

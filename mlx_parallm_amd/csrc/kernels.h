@@ -53,6 +53,9 @@ struct GemvCall {
                                   // unrounded -- a residual stream kept in 32 bits, logits of the layer-list models
   Glu glu;                        // EPI_SWIGLU: the unit (common.h); everything but silu is one float32 expression, rounded once
   int silu_cols = 0;              // EPI_STORE in the activation dtype: columns [0, silu_cols) are stored as silu(acc), rounded once
+  int split_out = 0;              // EPI_SWIGLU on float32 activations: out holds rows of [hi | lo] bf16 (2 ldo columns), the form launch_split3_rows makes
+                                  // of two terms, where gemm_prefill_split_out says so
+  int x_split = 0;                // float32 activations: x holds such rows already
   int kx = 0;                     // > 0: W is a [hi | lo] matrix of 2 kx columns (an f16 model in the float32-activation mode): the
                                   // activations have kx columns and are walked twice (k mod kx); 0: W.K columns
   // RMSNorm hand-over between two launches of gemm_skinny.hip's 16-row instantiation: a residual epilogue leaves
@@ -86,6 +89,8 @@ bool gemm_prefill_supported(const LinearW& W, const GemvCall& c, size_t rows);
 // does the tile GEMM beat 32 rows per launch of the streaming kernel?  Logits and layer 0's rounded call on float32 activations only:
 // codes = int4 weights, hilo = the [hi | lo] copy of an f16 matrix
 bool gemm_prefill_pays(bool codes, bool hilo, bool rounded, size_t rows);
+// can this call of split rows leave its SwiGLU as [hi | lo] rows (GemvCall::split_out)?  The 256 x 256 LDS-DMA tile alone does
+bool gemm_prefill_split_out(const LinearW& W, const GemvCall& c, size_t rows);
 // the same question for any call on a quantised matrix; terms: of x (launch_split3_rows)
 bool gemm_prefill_pays_codes(const LinearW& W, const GemvCall& c, size_t rows, int terms, size_t splitk_cap);
 // splitk_ws / splitk_cap: float32 workspace for the K-split form of the 128 x 128 tile (few hundred rows against a narrow
