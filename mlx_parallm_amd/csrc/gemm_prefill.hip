@@ -56,6 +56,7 @@ struct GemmParams {
                                     // every (x part, W part) pair once.
   int out32;                        // outputs / residual stream are float32 (PagedKVCache mode), no 16-bit rounding
   int rnd;                          // .. but for a plain store with logical rounding (layer 0 of that mode: RND_*)
+  int strips;                       // rows of the outputs (and the residual) are whole, aligned 16-byte pieces
   int split_out;                    // .. or a SwiGLU stored as two bf16 terms (256 x 256 LDS-DMA tile only)
   int epi; void* out; int ldo; void* resid; int pair_offset;
   Glu glu; int silu_cols;
@@ -357,31 +358,6 @@ __device__ __forceinline__ void tile256_epilogue(const GemmParams& p, f32x4 (&ac
     }
 }
 
-// SwiGLU in float32 as two bf16 terms, hi = bf16(y), lo = bf16(y - hi): what the down projection multiplies.  Stored here they are the bytes of the
-// float32 row; a pass that split it (8192 x 14336: 157 us) is saved.  Neighbouring lanes hold neighbouring columns: the even one takes both hi, the odd
-// one both lo, a store of 4 bytes each.
-__device__ __forceinline__ void tile256_epilogue_split(const GemmParams& p, f32x4 (&acc)[8][4], int m0, int bn, int wm, int wn, int c16, int g) {
-  uint16_t* out = (uint16_t*)p.out;
-  const bool odd = c16 & 1;
-#pragma unroll
-  for (int mt = 0; mt < 8; ++mt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = m0 + wm * 128 + mt * 16 + 4 * g + r;
-      if (m >= p.M) continue;                                    // (16 lanes of a row, and below of a tile, together)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int n = bn * 128 + wn * 32 + j * 16 + c16;
-        if (n >= p.pair_offset) continue;
-        const float y = glu32(p.glu, acc[mt][j][r], acc[mt][j + 2][r]);
-        const bf16 hi = (bf16)y, lo = (bf16)(y - (float)hi);
-        const uint32_t h = __builtin_bit_cast(uint16_t, hi), l = __builtin_bit_cast(uint16_t, lo);
-        const uint32_t got = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(odd ? h : l), 0xB1, 0xf, 0xf, false);      // quad_perm:[1,0,3,2]
-        *(uint32_t*)(out + (size_t)m * (2 * p.ldo) + (odd ? p.ldo + n - 1 : n)) = odd ? got | (l << 16) : h | (got << 16);
-      }
-    }
-}
-
 // Grouped form: whole rows.  A wave's tile goes through its own strip of LDS, 64 rows at a time, and leaves it as 16-byte pieces of
 // rows (out_rows may scatter them): 16 stores per wave instead of 128.  The LDS must be free (every DMA landed, every read done).
 template <typename AT, bool SWIGLU, bool VAR>
@@ -448,6 +424,109 @@ __device__ __forceinline__ void tile256_epilogue_resid(const GemmParams& p, f32x
         if constexpr (std::is_same<HT, float>::value) h[(size_t)m * p.ldo + n] = hv[r][nt] + acc[mt][nt][r];
         else h[(size_t)m * p.ldo + n] = (AT)((float)hv[r][nt] + (float)(AT)acc[mt][nt][r]);
       }
+  }
+}
+
+// The same epilogues through LDS: a wave writes ROWS rows of its tile to a strip of its own and takes them out as 16-byte pieces of rows -- 64 to
+// 128 bytes of a row side by side where a register is one column of four rows: 2 or 4 bytes a lane, 64 to 256 stores (and loads of the residual) a
+// wave, each of which takes the CU's address unit 16 cycles.  Element stores -> strips, us: 8192 rows, 6144 x 4096 318 -> 297, 28672 x 4096 SwiGLU
+// 1583 -> 1542, 4096 x 14336 with the residual 705 -> 690, 2048 x 2048 64 -> 56; 4096 rows, 16384 x 2048 249 -> 213.
+// Where rows are whole 16-byte pieces (host: GemmParams::strips); the LDS must be free.
+template <typename ST, int WC, typename Value, typename Emit>
+__device__ __forceinline__ void tile256_strips(unsigned char* lds, int wave, int lane, Value value, Emit emit) {
+  constexpr int ROWS = WC * sizeof(ST) > 128 ? 32 : 64, PER = 16 / sizeof(ST), LDW = WC + PER, NP = WC / PER, MTP = ROWS / 16;
+  const int c16 = lane & 15, g = lane >> 4;
+  ST* strip = (ST*)lds + (size_t)wave * ROWS * LDW;
+#pragma unroll
+  for (int pass = 0; pass < 128 / ROWS; ++pass) {
+#pragma unroll
+    for (int mt = 0; mt < MTP; ++mt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int ct = 0; ct < WC / 16; ++ct) strip[(mt * 16 + 4 * g + r) * LDW + ct * 16 + c16] = value(pass * MTP + mt, r, ct);
+    asm volatile("" ::: "memory");                     // (a wave's LDS operations complete in order)
+    __builtin_amdgcn_wave_barrier();
+    u32x4 v[ROWS * NP / 64];
+#pragma unroll
+    for (int i = 0; i < ROWS * NP / 64; ++i) {
+      const int piece = i * 64 + lane;
+      v[i] = *(const u32x4*)(strip + (piece / NP) * LDW + (piece % NP) * PER);
+    }
+    emit(pass * ROWS, v, [&](int i) { return (i * 64 + lane) / NP; }, [&](int i) { return (i * 64 + lane) % NP * PER; });
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+template <typename AT, bool SWIGLU, bool VAR, bool LOGITS = false>
+__device__ __forceinline__ void tile256_epilogue_strips(const GemmParams& p, f32x4 (&acc)[8][4], unsigned char* lds, int m0, int bn, int wave, int lane) {
+  constexpr int WC = SWIGLU ? 32 : 64;
+  const int n0 = bn * 4 * WC + (wave & 3) * WC, cols = SWIGLU ? p.pair_offset : p.N, c16 = lane & 15;
+  const int mw = m0 + (wave >> 2) * 128;
+  // pieces of ST into rows of `dst`, stride ld; add: the residual
+  auto store = [&](auto* dst, size_t ld, int row0, auto& v, auto row, auto col) {
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(v) / 16); ++i) {
+      const int m = mw + row0 + row(i), n = n0 + col(i);
+      if (m < p.M && n < cols) *(u32x4*)(dst + (size_t)m * ld + n) = v[i];
+    }
+  };
+  auto fetch = [&](const auto* src, int row0, auto& h, auto row, auto col) {
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(h) / 16); ++i)
+      h[i] = *(const u32x4*)(src + (size_t)min(mw + row0 + row(i), p.M - 1) * p.ldo + min(n0 + col(i), cols - (int)(16 / sizeof(*src))));
+  };
+  if constexpr (SWIGLU) {
+    if (p.split_out) {                                 // two bf16 terms, hi = bf16(y), lo = bf16(y - hi): what the down projection multiplies
+      tile256_strips<uint32_t, WC>(lds, wave, lane, [&](int mt, int r, int ct) {
+        float y = glu32(p.glu, acc[mt][ct][r], acc[mt][ct + 2][r]);
+        asm("" : "+v"(y));                               // (the product is rounded before lo takes hi off it: no FMA over both)
+        const bf16 hi = (bf16)y, lo = (bf16)(y - (float)hi);
+        return (uint32_t)__builtin_bit_cast(uint16_t, hi) | (uint32_t)__builtin_bit_cast(uint16_t, lo) << 16;
+      }, [&](int row0, auto& v, auto row, auto col) {
+#pragma unroll
+        for (int i = 0; i < (int)(sizeof(v) / 16); ++i) {
+          const int m = mw + row0 + row(i), n = n0 + col(i);
+          if (m >= p.M || n >= cols) continue;
+          uint16_t* o = (uint16_t*)p.out + (size_t)m * (2 * p.ldo) + n;
+          *(uint2*)o = uint2{(v[i].x & 0xffffu) | (v[i].y << 16), (v[i].z & 0xffffu) | (v[i].w << 16)};
+          *(uint2*)(o + p.ldo) = uint2{(v[i].x >> 16) | (v[i].y & 0xffff0000u), (v[i].z >> 16) | (v[i].w & 0xffff0000u)};
+        }
+      });
+    } else if (p.out32) {
+      tile256_strips<float, WC>(lds, wave, lane, [&](int mt, int r, int ct) { return glu32(p.glu, acc[mt][ct][r], acc[mt][ct + 2][r]); },
+                                [&](int row0, auto& v, auto row, auto col) { store((float*)p.out, p.ldo, row0, v, row, col); });
+    } else {
+      tile256_strips<AT, WC>(lds, wave, lane, [&](int mt, int r, int ct) {
+        return VAR ? (AT)glu_f(p.glu, acc[mt][ct][r], acc[mt][ct + 2][r]) : silu16<AT>(acc[mt][ct][r], acc[mt][ct + 2][r]);
+      }, [&](int row0, auto& v, auto row, auto col) { store((AT*)p.out, p.ldo, row0, v, row, col); });
+    }
+  } else if (LOGITS || p.out32) {
+    tile256_strips<float, WC>(lds, wave, lane, [&](int mt, int r, int ct) { return LOGITS ? (float)(AT)acc[mt][ct][r] : acc[mt][ct][r]; },
+                              [&](int row0, auto& v, auto row, auto col) {
+      if (LOGITS || p.epi == EPI_STORE) { store((float*)p.out, p.ldo, row0, v, row, col); return; }
+      f32x4 h[sizeof(v) / 16];
+      fetch((const float*)p.resid, row0, (u32x4(&)[sizeof(v) / 16])h, row, col);
+#pragma unroll
+      for (int i = 0; i < (int)(sizeof(v) / 16); ++i) v[i] = __builtin_bit_cast(u32x4, h[i] + __builtin_bit_cast(f32x4, v[i]));
+      store((float*)p.resid, p.ldo, row0, v, row, col);
+    });
+  } else {
+    tile256_strips<AT, WC>(lds, wave, lane, [&](int mt, int r, int ct) { return (AT)(VAR ? silu_col(p.silu_cols, n0 + ct * 16 + c16, acc[mt][ct][r]) : acc[mt][ct][r]); },
+                           [&](int row0, auto& v, auto row, auto col) {
+      if (p.epi == EPI_STORE) { store((AT*)p.out, p.ldo, row0, v, row, col); return; }
+      u32x4 h[sizeof(v) / 16];
+      fetch((const AT*)p.resid, row0, h, row, col);
+#pragma unroll
+      for (int i = 0; i < (int)(sizeof(v) / 16); ++i) {
+        AT* y = (AT*)&v[i];
+        const AT* hv = (const AT*)&h[i];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) y[j] = (AT)((float)hv[j] + (float)y[j]);
+      }
+      store((AT*)p.resid, p.ldo, row0, v, row, col);
+    });
   }
 }
 
@@ -845,15 +924,20 @@ __global__ __launch_bounds__(512) void gemm_dma256_kernel(GemmParams p) {
       return;
     }
   }
+  if constexpr (!GROUPED) {
+    if (p.strips) {
+      __syncthreads();
+      if (!LOGITS && epilogue_varies<SWIGLU>(p, bn)) tile256_epilogue_strips<AT, SWIGLU, true, LOGITS>(p, acc, smem2, m0, bn, wave, lane);
+      else tile256_epilogue_strips<AT, SWIGLU, false, LOGITS>(p, acc, smem2, m0, bn, wave, lane);
+      return;
+    }
+  }
   if constexpr (!SWIGLU && !LOGITS) {
     if (p.epi == EPI_RESID) {
       if (p.out32) tile256_epilogue_resid<AT, float>(p, acc, m0, bn, wm, wn, c16, g);
       else tile256_epilogue_resid<AT, AT>(p, acc, m0, bn, wm, wn, c16, g);
       return;
     }
-  }
-  if constexpr (SWIGLU && !GROUPED && std::is_same<AT, bf16>::value) {
-    if (p.split_out) { tile256_epilogue_split(p, acc, m0, bn, wm, wn, c16, g); return; }
   }
   if constexpr (GROUPED) {
     __syncthreads();
@@ -1109,6 +1193,12 @@ __global__ __launch_bounds__(512) void gemm_codes256_kernel(GemmParams p) {
         }
       return;
     }
+  }
+  if (p.strips) {
+    __syncthreads();
+    if (!LOGITS && epilogue_varies<SWIGLU>(p, bn)) tile256_epilogue_strips<AT, SWIGLU, true, LOGITS>(p, acc, smem2, m0, bn, wave, lane);
+    else tile256_epilogue_strips<AT, SWIGLU, false, LOGITS>(p, acc, smem2, m0, bn, wave, lane);
+    return;
   }
   if constexpr (!SWIGLU && !LOGITS) {
     if (p.epi == EPI_RESID) {
@@ -1598,6 +1688,12 @@ static int split256(long blocks, int ktiles, size_t slice_bytes, size_t cap) {
   return ks256;
 }
 
+// 16-byte pieces of the output rows (and of the residual's): strides and bases of float or AT elements (split_out: 8 bytes of bf16)
+static int strips_ok(const GemmParams& p) {
+  const void* dst = p.epi == EPI_RESID ? p.resid : p.out;
+  return p.ldo % (p.out32 ? 4 : 8) == 0 && ((uintptr_t)dst & 15) == 0;
+}
+
 static int reduce_slices(const GemmParams& p, int act, hipStream_t st) {
   const size_t total4 = (size_t)p.M * p.N / 4;
   const dim3 rg((unsigned)((total4 + 255) / 256));
@@ -1617,10 +1713,9 @@ size_t gemm_prefill_scratch_bytes(const LinearW& W, size_t rows) {
 // 4096 x 2048 x 768 47 / 53, 1536 59 / 101; 2048 x 1024 x 2048 43 / 43, 4096 57 / 55; 6144 x 1024 SwiGLU 768 57 / 54, 1536 60 / 82.  Float32 rows
 // (three walks against six): 2048 x 1024 x 768 42 / 42, 1536 55 / 62; 3072 x 1024 x 768 49 / 58.
 static bool codes_plan(const LinearW& W, const GemvCall& c, size_t rows, int ldx, int terms, bool split_ok, size_t cap, GemmParams& p, long& blocks) {
-  static const bool off = getenv("MI_GEMM_CODES") != nullptr && atoi(getenv("MI_GEMM_CODES")) == 0;       // A/B
   const bool sw = c.epi == EPI_SWIGLU;
   const int ncols = sw ? c.pair_offset : W.N;
-  if (off || !wk_is_quant(W.wk) || W.layout != 1 || W.group != 64 || W.K % BK != 0) return false;
+  if (!wk_is_quant(W.wk) || W.layout != 1 || W.group != 64 || W.K % BK != 0) return false;
   if ((double)rows * W.N * W.K * terms < (W.K >= 4096 ? 2.1e9 : 4.3e9)) return false;
   p.M = (int)rows; p.N = W.N; p.kw = W.K; p.ka = p.K = terms * W.K; p.ldx = ldx; p.G = W.K / 64;
   p.kb = codes16_bias_cols(W.K);
@@ -1671,6 +1766,7 @@ static int launch_gemm_codes(const LinearW& W, const GemvCall& c, size_t rows, h
     p.epi = EPI_STORE;
     if (!x32) { p.out32 = 1; p.rnd = c.act == MI_BF16 ? RND_BF16 : RND_F16; }
   }
+  p.strips = strips_ok(p);
   const dim3 grid((unsigned)((rows + BM2 - 1) / BM2), (ncols + (sw ? 128 : BN2) - 1) / (sw ? 128 : BN2), p.ksplit), block(512);
   auto go = [&](auto k) -> int {
     MI_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, CODES_LDS));
@@ -1692,7 +1788,7 @@ static bool gemm_dma_on() { const char* v = getenv("MI_GEMM_DMA"); return v == n
 bool gemm_prefill_split_out(const LinearW& W, const GemvCall& c, size_t rows) {
   if (c.act != MI_F32 || c.epi != EPI_SWIGLU || c.kx > 0 || W.wk != WK_BF16 || c.pair_offset % 2 != 0 || rows < BM2) return false;
   const long blocks256 = (long)((rows + BM2 - 1) / BM2) * ((c.pair_offset + 127) / 128);
-  return !gemm_small_only() && gemm_dma_on() && blocks256 >= 192 && 2 * W.K >= 2 * BK;
+  return !gemm_small_only() && gemm_dma_on() && blocks256 >= 192 && 2 * W.K >= 2 * BK && c.ldo % 4 == 0 && ((uintptr_t)c.out & 15) == 0;
 }
 
 int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st, void* scratch, void* splitk_ws,
@@ -1743,6 +1839,7 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
   const bool dma = gemm_dma_on();
   if (c.split_out && !gemm_prefill_split_out(W, c, rows)) return fail(MI_ERR_INVALID, "gemm_prefill: this call does not store split rows");
   p.split_out = c.split_out;
+  p.strips = strips_ok(p);
   // too few 256 x 256 tiles for the chip (one prompt of 256..4095 rows against N = 4096 / 6144): the LDS-DMA tile with K
   // split over up to 8 workgroups, each >= 8 K tiles (plain / residual epilogues; SwiGLU launches have enough tiles or
   // stay on the 128 x 128 kernel).  MI_GEMM_DMA_SPLITK=0 switches it off (A/B).

@@ -42,3 +42,35 @@ def test_same_bits_as_the_separate_pass(B, lengths, ff):
     for a, b in zip(*got):
         assert np.all(np.isfinite(a)) and np.array_equal(a, b)
     eng.close()
+
+
+@pytest.mark.parametrize("epi", ["store", "resid", "swiglu", "logits"])
+@pytest.mark.parametrize("M,N", [(2085, 6160), (2304, 5632)])
+def test_rows_in_pieces_and_by_elements_store_the_same(epi, M, N):
+    """The 256 x 256 tile takes 16-byte pieces of rows where stride and base allow it, single elements elsewhere: the same bits, nothing beside them."""
+    from gpu_helpers import dev, gemm_prefill, host, op_linear, to_tiled
+    from mlx_parallm_amd import _lib as L
+
+    rng = np.random.default_rng(N)
+    K = 192
+    wd = dev(rng.standard_normal((N, K)).astype(np.float32) * 0.05, "bfloat16")
+    ol, keep = op_linear("bf16", N, K, wd), [wd]
+    assert to_tiled(ol, keep)
+    xd = dev(rng.standard_normal((M, K)).astype(np.float32), "bfloat16")
+    cols = N // 2 if epi == "swiglu" else N
+    h = rng.standard_normal((M, cols)).astype(np.float32)
+    dt = torch.float32 if epi == "logits" else torch.bfloat16
+    got = []
+    for pad, shift in ((8, 0), (2, 0), (8, 2)):                   # strides and bases of whole pieces; a stride that is none; a base that is none
+        buf = torch.full(((M + 1) * (cols + pad) + 8,), 7.0, dtype=dt, device="cuda")
+        out = buf[shift:shift + (M + 1) * (cols + pad)].view(M + 1, cols + pad)
+        if epi == "resid":
+            out[:M, :cols] = dev(h, "bfloat16")
+        kw = {"store": dict(epi=L.EPI_STORE), "resid": dict(epi=L.EPI_RESID, resid=out), "logits": dict(epi=L.EPI_STORE_F32),
+              "swiglu": dict(epi=L.EPI_SWIGLU, pair_offset=cols)}[epi]
+        gemm_prefill(ol, xd, M, "bfloat16", out=out, ldo=cols + pad, **kw)
+        torch.cuda.synchronize()
+        o = host(out)
+        assert np.all(o[M:] == 7.0) and np.all(o[:, cols:] == 7.0)
+        got.append(o[:M, :cols])
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
