@@ -1715,7 +1715,7 @@ size_t gemm_prefill_scratch_bytes(const LinearW& W, size_t rows) {
 static bool codes_plan(const LinearW& W, const GemvCall& c, size_t rows, int ldx, int terms, bool split_ok, size_t cap, GemmParams& p, long& blocks) {
   const bool sw = c.epi == EPI_SWIGLU;
   const int ncols = sw ? c.pair_offset : W.N;
-  if (!wk_is_quant(W.wk) || W.layout != 1 || W.group != 64 || W.K % BK != 0) return false;
+  if (!wk_is_quant(W.wk) || W.layout != 1 || W.group != 64 || W.K % BK != 0 || W.K > 65536) return false;      // (the biases of a row tile in 64 KiB of LDS)
   if ((double)rows * W.N * W.K * terms < (W.K >= 4096 ? 2.1e9 : 4.3e9)) return false;
   p.M = (int)rows; p.N = W.N; p.kw = W.K; p.ka = p.K = terms * W.K; p.ldx = ldx; p.G = W.K / 64;
   p.kb = codes16_bias_cols(W.K);
