@@ -44,6 +44,7 @@ def _run(ol, x, M, act, rnd=0, **kw):
     (300, 2064, 1152),       # ragged rows, a column tile of 16, 18 groups (the bias columns end inside a K tile)
     (2085, 6144, 128),       # two groups: a run that is all prologue, unsplit
     (2304, 5632, 640),       # an even number of groups, unsplit
+    (129, 4096, 4096),       # fewer rows than half a tile, eight slices
 ])
 def test_store_logits_and_residual(act, bits, M, N, K):
     rng = np.random.default_rng(1000 * bits + M)
@@ -82,7 +83,7 @@ def test_swiglu(act, bits, M, I, K):
     _assert_close(o[:M][rows], want, act, scale=float(np.abs(y).max()))
 
 
-@pytest.mark.parametrize("M,N,K,rnd", [(300, 2048, 1024, 0), (2085, 6144, 256, 0), (1024, 6144, 640, L.RND_BF16)])
+@pytest.mark.parametrize("M,N,K,rnd", [(300, 2048, 1024, 0), (2085, 6144, 256, 0), (64, 2768, 4096, 0), (1024, 6144, 640, L.RND_BF16)])
 def test_float32_rows(M, N, K, rnd):
     """three bf16 terms of x (a run over the codes per term); rnd: layer 0's rounded call, x is one term"""
     rng = np.random.default_rng(K)
