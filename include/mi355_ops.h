@@ -96,8 +96,12 @@ int mi_op_gemm_skinny(const mi_op_linear* w, const mi_op_gemv_args* a, int kspli
  * MI_PRO_NONE; plain / residual / SwiGLU epilogues.  iters >= 1 also times that many back-to-back launches into *avg_ms. */
 int mi_op_gemm_prefill(const mi_op_linear* w, const mi_op_gemv_args* a, int iters, float* avg_ms);
 /* the same for tile-major int4 / int8 weights (group 64): the tile GEMM on their codes where it takes the call, else on their [hi | lo] copy.
- * a->act: 16-bit, or float32 on a bf16 model (split into three terms here; a->rnd = MI_RND_BF16, plain stores only: one). */
+ * a->act: 16-bit, or float32 on a bf16 model (split into three terms here; a->rnd = MI_RND_BF16, plain stores only: one).
+ * iters < 0: on the codes whatever the size, or an error. */
 int mi_op_gemm_codes(const mi_op_linear* w, const mi_op_gemv_args* a, int iters, float* avg_ms);
+/* what a prefill call of a->M rows on tile-major int4 / int8 weights runs on: 2 the tile GEMM on their codes, 1 the tile GEMM on their [hi | lo] copy, 0
+ * another kernel (float32 activations: 32 rows per launch of the streaming one); a negative error code.  No device needed; no pointer is read. */
+int mi_op_gemm_quant_route(const mi_op_linear* w, const mi_op_gemv_args* a);
 /* gemv_reg.hip on its own: the decode linears of at most 8 rows on tile-major weights -- int4 / int8 (group 64) with scales of the
  * activations' type (plain / float32 / residual / SwiGLU epilogues, the last with the norm), dense 16-bit ones with activations of
  * their type or float32 on bf16 (plain / float32 / residual; float32 also MI_EPI 4, SwiGLU on a row-interleaved gate|up matrix:

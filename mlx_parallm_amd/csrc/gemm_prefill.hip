@@ -1583,6 +1583,13 @@ int launch_rmsnorm_block(const void* x, int ldx, const void* w, void* out, int l
 
 }  // namespace
 
+// What gemm_codes256_kernel can do at all, rows of stride ldx
+static bool codes_fits(const LinearW& W, const GemvCall& c, size_t rows, size_t ldx) {
+  if (!wk_is_quant(W.wk) || W.layout != 1 || W.group != 64 || W.K % BK != 0 || W.K > 65536) return false;      // (the biases of a row tile in 64 KiB of LDS)
+  const size_t lim = (size_t)1 << 32;                    // (32-bit offsets of the LDS-DMA sources)
+  return rows * ldx * 2 < lim && rows * codes16_bias_cols(W.K) * 2 < lim && (size_t)W.N * (W.K / 64) * 4 < lim;
+}
+
 bool gemm_prefill_supported(const LinearW& W, const GemvCall& c, size_t rows) {
   if (c.force_v1 || W.layout != 1) return false;
   // logical rounding (layer 0 of the PagedKVCache mode): plain stores of float32 activations
@@ -1592,10 +1599,12 @@ bool gemm_prefill_supported(const LinearW& W, const GemvCall& c, size_t rows) {
   const bool q4 = ((W.wk == WK_Q4_BF16 && c.act == MI_BF16) || (W.wk == WK_Q4_F16 && c.act == MI_F16)) && W.group == 64 &&
                   W.K % 128 == 0;                       // through a [hi | lo] 16-bit copy (launch_dequant_q4_hilo)
   const bool q8 = ((W.wk == WK_Q8_BF16 && c.act == MI_BF16) || (W.wk == WK_Q8_F16 && c.act == MI_F16)) && W.group == 64;
-  // float32 activations on a bf16 model (PagedKVCache mode): x goes through launch_split3_rows first
+  // float32 activations on a bf16 model (PagedKVCache mode): x goes through launch_split3_rows first.  int8: on the codes alone (codes_plan says
+  // why), and above 128 rows: up to there (a decode batch) the streaming kernel is ahead where the time is (us, streaming / codes: 64 rows
+  // 6144 x 4096 41 / 69, 4096 x 14336 68 / 178, 2048 x 2048 30 / 40; 96 rows 62 / 70, 102 / 179, 45 / 42; 1024 x 1024, 96 rows 36 / 29)
   static const bool f32_ok = getenv("MI_GEMM_NO_F32") == nullptr;
   const bool x32 = f32_ok && c.act == MI_F32 && (W.wk == WK_BF16 || (W.wk == WK_Q4_BF16 && W.group == 64 && W.K % 128 == 0) ||
-                                                 (W.wk == WK_Q8_BF16 && W.group == 64 && rows > 128)) &&
+                                                 (W.wk == WK_Q8_BF16 && rows > 128 && codes_fits(W, c, rows, 3 * (size_t)W.K))) &&
                    c.ldx % 4 == 0 && W.K % 4 == 0;
   if (!dense && !q4 && !q8 && !x32) return false;
   if (W.K % BK != 0 || (!x32 && c.ldx % 8 != 0)) return false;
@@ -1697,16 +1706,18 @@ size_t gemm_prefill_scratch_bytes(const LinearW& W, size_t rows) {
 // 129 rows 43 / 50, 28672 x 4096 SwiGLU 129 rows 196 / 317 and 700 rows 348 / 494, 4096 x 14336 x 700 144 / 221; 2048 x 5632 x 192 44 / 41, 256 44 / 50;
 // 4096 x 2048 x 768 47 / 53, 1536 59 / 101; 2048 x 1024 x 2048 43 / 43, 4096 57 / 55; 6144 x 1024 SwiGLU 768 57 / 54, 1536 60 / 82.  Float32 rows
 // (three walks against six): 2048 x 1024 x 768 42 / 42, 1536 55 / 62; 3072 x 1024 x 768 49 / 58.
+// Int8 on float32 rows at any size: the alternative there is the streaming kernel on exact codes, and a pair of bf16 is no match for it once a group's
+// mean exceeds 3 of its deviations.  2-norm from 64 bits, 1024 x 1024, 256 rows, means of 0 / 4 / 12 deviations: pair 1.8e-7 / 7.0e-7 / 1.9e-6,
+// streaming 3.3e-7 / 1.3e-7 / 1.0e-7, here 0.9e-7 / 1.1e-7 / 1.1e-7 (K = 8192, 64 rows: 5.3e-7 / 8.4e-7 / 1.9e-6, 3.4e-7 / 1.5e-7 / 1.3e-7, 1.7e-7 / 2.5e-7 / 2.3e-7);
+// us, streaming / here: 129 rows 59 / 29, 1365 rows 511 / 40.
 static bool codes_plan(const LinearW& W, const GemvCall& c, size_t rows, int ldx, int terms, bool split_ok, size_t cap, GemmParams& p, long& blocks) {
   const bool sw = c.epi == EPI_SWIGLU;
   const int ncols = sw ? c.pair_offset : W.N;
-  if (!wk_is_quant(W.wk) || W.layout != 1 || W.group != 64 || W.K % BK != 0 || W.K > 65536) return false;      // (the biases of a row tile in 64 KiB of LDS)
-  if ((double)rows * W.N * W.K * terms < (W.K >= 4096 ? 2.1e9 : 4.3e9)) return false;
+  if (!codes_fits(W, c, rows, ldx)) return false;
+  const bool any = c.codes || (c.act == MI_F32 && wk_bits(W.wk) == 8);
+  if (!any && (double)rows * W.N * W.K * terms < (W.K >= 4096 ? 2.1e9 : 4.3e9)) return false;
   p.M = (int)rows; p.N = W.N; p.kw = W.K; p.ka = p.K = terms * W.K; p.ldx = ldx; p.G = W.K / 64;
   p.kb = codes16_bias_cols(W.K);
-  // (32-bit offsets of the LDS-DMA sources)
-  const size_t lim = (size_t)1 << 32;
-  if (rows * (size_t)ldx * 2 >= lim || rows * (size_t)p.kb * 2 >= lim || (size_t)W.N * p.G * 4 >= lim) return false;
   blocks = (long)((rows + BM2 - 1) / BM2) * ((ncols + (sw ? 128 : BN2) - 1) / (sw ? 128 : BN2));
   p.ksplit = !sw && split_ok && W.N % 4 == 0 ? split256(blocks, (p.ka + p.kb) / BK, rows * W.N * sizeof(float), cap) : 1;
   return true;
@@ -1716,7 +1727,7 @@ static bool codes_plan(const LinearW& W, const GemvCall& c, size_t rows, int ldx
 // within 20 %: a launch of the streaming kernel 10 + 0.36 per 2^20 weights (6144 x 4096 19.6, 28672 x 4096 40.6, 32000 x 4096 50); the codes' copy 0.65, a round
 // of workgroups 1.35 per K tile, the slices' reduce.  28672 x 4096 SwiGLU: 256 rows 363 against 325 streaming, 320 rows 405 / 406, 512 rows 425 / 650;
 // 6144 x 4096 96 rows 71 / 59, 160 rows 75 / 98.
-bool gemm_prefill_pays_codes(const LinearW& W, const GemvCall& c, size_t rows, int terms, size_t splitk_cap) {
+static bool gemm_prefill_pays_codes(const LinearW& W, const GemvCall& c, size_t rows, int terms, size_t splitk_cap) {
   GemmParams p{};
   long blocks = 0;
   if (!codes_plan(W, c, rows, terms * W.K, terms, splitk_cap > 0, splitk_cap, p, blocks))
@@ -1725,6 +1736,17 @@ bool gemm_prefill_pays_codes(const LinearW& W, const GemvCall& c, size_t rows, i
   const double mw = (double)W.N * W.K / (1 << 20), rounds = (double)((blocks * p.ksplit + ncu - 1) / ncu);
   const double reduce = p.ksplit > 1 ? 2e-6 * p.ksplit * rows * W.N : 0.0;
   return 12.0 + 0.65 * mw + 1.35 * rounds * tiles + reduce < (double)((rows + 31) / 32) * (10.0 + 0.36 * mw);
+}
+
+int gemm_prefill_quant_route(const LinearW& W, const GemvCall& c, size_t rows) {
+  if (!gemm_prefill_supported(W, c, rows)) return 0;
+  const bool x32 = c.act == MI_F32;
+  const int terms = x32 && c.rnd != RND_BF16 ? 3 : 1;
+  const size_t cap = rows < 4096 ? (size_t)128 << 20 : 0;                       // (of the engine's workspace for slices)
+  if (x32 && rows > 32 && gemm_skinny_supported(W, c, 32) && !gemm_prefill_pays_codes(W, c, rows, terms, cap)) return 0;
+  GemmParams p{};
+  long blocks = 0;
+  return codes_plan(W, c, rows, x32 ? terms * W.K : c.ldx, terms, cap > 0, cap, p, blocks) ? 2 : 1;
 }
 
 // quantised matrices on gemm_codes256_kernel; *done = false: the [hi | lo] copy and the dense tiles take the call
@@ -1788,6 +1810,7 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
     bool done = false;
     if (split_ok) MI_TRY(launch_gemm_codes(W, c, rows, st, scratch, splitk_ws, splitk_cap, &done));
     if (done) return MI_OK;
+    if (c.codes || (c.act == MI_F32 && wk_bits(W.wk) == 8)) return fail(MI_ERR_UNSUPPORTED, "gemm_prefill: this call does not run on the codes");
     MI_TRY(launch_dequant_q4_hilo(W, scratch, st));
     p.w = scratch; p.K = 2 * W.K; p.kw = 2 * W.K;
   }

@@ -156,6 +156,7 @@ int mi_op_gemm_codes(const mi_op_linear* w, const mi_op_gemv_args* a, int iters,
   GemvCall c = to_call(a);
   if (c.M < 1 || c.pro != PRO_NONE || !wk_is_quant(W.wk) || !gemm_prefill_supported(W, c, (size_t)c.M))
     return fail(MI_ERR_UNSUPPORTED, "mi_op_gemm_codes: tile-major int4 / int8 weights (group 64), at least 32 rows, no prologue");
+  c.codes = iters < 0;
   void *ws = nullptr, *scratch = nullptr, *xs = nullptr;
   size_t cap = 0;
   auto done = [&](int rc) { hipFree(ws); hipFree(scratch); hipFree(xs); return rc; };
@@ -183,6 +184,14 @@ int mi_op_gemm_codes(const mi_op_linear* w, const mi_op_gemv_args* a, int iters,
   }
   const int rc2 = finish();
   return done(rc != MI_OK ? rc : rc2);
+}
+
+int mi_op_gemm_quant_route(const mi_op_linear* w, const mi_op_gemv_args* a) {
+  if (!w || !a || a->M < 1) return fail(MI_ERR_INVALID, "mi_op_gemm_quant_route: arguments");
+  const LinearW W = to_linear(w);
+  const GemvCall c = to_call(a);
+  if (!wk_is_quant(W.wk)) return fail(MI_ERR_INVALID, "mi_op_gemm_quant_route: int4 / int8 weights");
+  return gemm_prefill_quant_route(W, c, (size_t)c.M);
 }
 
 int mi_op_gemv_reg(const mi_op_linear* w, const mi_op_gemv_args* a) {

@@ -102,3 +102,34 @@ def test_float32_rows(M, N, K, rnd):
     else:
         # exact products; K / 64 + 2 float32 additions of a group's sums and the biases', of up to 16 scales x |x| each
         assert np.max(np.abs(o[:M][rows] - want)) <= 2.0 ** -24 * (K / 64 + 8) * 4 * np.abs(x[rows]).sum(1).max() * np.abs(w).max()
+
+
+@pytest.mark.parametrize("M,N,K,epi", [(129, 1024, 1024, "STORE"), (300, 208, 704, "STORE"), (1365, 1024, 1024, "RESID"), (200, 2048, 1024, "SWIGLU"), (160, 48, 64, "STORE"),
+                                       (256, 16, 1024, "STORE_F32")])
+def test_int8_on_float32_rows_is_as_close_as_float32_sums(M, N, K, epi):
+    """Small matrices, groups whose mean is twelve of their deviations: a [hi | lo] pair of the weight is 1.9e-6 off in 2-norm.  Here the products are exact,
+    and a result takes one rounding per group of 64 and one per 32 of the 6 K / 64 bias columns, each of at most half an ulp of the partial sum: in 2-norm
+    some 2^-24 sqrt(K / 64 + 6 K / 2048 + 2), the residual's and the unit's own roundings among the last two."""
+    rng = np.random.default_rng(M)
+    w = (rng.standard_normal((N, K // 64, 64)) + 12 * rng.standard_normal((N, K // 64, 1))).astype(np.float32) * 0.05
+    packed, s, b = ref_quant.quantize(w.reshape(N, K), 64, 8, "bfloat16")
+    keep = [dev_u32(packed), dev(s, "bfloat16"), dev(b, "bfloat16")]
+    ol = op_linear("q8_bf16", N, K, *keep)
+    assert to_tiled(ol, keep)
+    codes = packed.view(np.uint8).reshape(N, K).astype(np.float64)
+    w = codes * np.repeat(s, 64, 1).astype(np.float64) + np.repeat(b, 64, 1)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    want = x.astype(np.float64) @ w.T
+    cols = N
+    if epi == "SWIGLU":
+        cols = N // 2
+        gt, up = want[:, :cols], want[:, cols:]
+        want = gt / (1 + np.exp(-np.clip(gt, -700, None))) * up
+    h = rng.standard_normal((M, cols)).astype(np.float32) if epi == "RESID" else np.zeros((M, cols), np.float32)
+    out = dev(h)
+    _run(ol, dev(x), M, "float32", epi=getattr(L, "EPI_" + epi), out=out, ldo=cols, resid=out if epi == "RESID" else None, pair_offset=cols if epi == "SWIGLU" else 0)
+    got = host(out).astype(np.float64)
+    off = np.linalg.norm(got - (want + h)) / np.linalg.norm(want + h)
+    # (SwiGLU: two such factors, and the sigmoid's expf and quotient, 3 ulp)
+    n = K / 64 + 6 * K / 2048 + 2
+    assert off <= 2.0 ** -24 * np.sqrt(n if epi != "SWIGLU" else 2 * n + 12), off

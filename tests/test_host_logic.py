@@ -389,6 +389,32 @@ def test_float32_rows_leave_the_streaming_kernel_where_the_tile_pays():
     assert not any(pays(n, hilo=1, rounded=1) for n in (33, 768, 1024)) and pays(2048, hilo=1, rounded=1)
 
 
+def _quant_route(rows, N, K, kind="q8_bf16", act="float32", epi="STORE", rnd=0):
+    """2: the tile GEMM on the codes, 1: on their [hi | lo] copy, 0: another kernel (include/mi355_ops.h)"""
+    import ctypes as C
+
+    from mlx_parallm_amd import _lib as L
+
+    w, a = L.OpLinear(), L.OpGemvArgs()
+    w.wk, w.N, w.K, w.group, w.layout = L.WK[kind], N, K, 64, 1
+    a.M, a.ldx, a.act, a.rnd = rows, K, {"float32": L.MI_F32, "bfloat16": L.MI_BF16, "float16": L.MI_F16}[act], rnd
+    a.epi, a.ldo = getattr(L, "EPI_" + epi), N
+    a.pair_offset = N // 2 if epi == "SWIGLU" else 0
+    return L.lib().mi_op_gemm_quant_route(C.byref(w), C.byref(a))
+
+
+def test_int8_on_float32_rows_is_never_multiplied_as_a_pair():
+    """A pair of bf16 holds an int8 weight to 2^-17 only once its group's mean exceeds 3 deviations; the streaming kernel and the codes hold it."""
+    from mlx_parallm_amd import _lib as L
+
+    for rows in (33, 64, 128, 129, 150, 300, 700, 1024, 1365, 3000, 9000):
+        for N, K in ((64, 64), (256, 128), (1024, 1024), (1536, 1024), (1024, 3072), (4096, 2048), (28672, 4096), (32784, 512), (4096, 14336), (160, 65600)):
+            for epi, rnd in (("STORE", 0), ("STORE", L.RND_BF16), ("STORE_F32", 0), ("RESID", 0), ("SWIGLU", 0)):
+                got = _quant_route(rows, N, K, epi=epi, rnd=rnd)
+                assert got in (0, 2) and (got == 0 or 128 < rows), (rows, N, K, epi, rnd, got)
+    assert [_quant_route(n, 1024, 1024) for n in (64, 128, 129, 1365)] == [0, 0, 2, 2]
+
+
 @pytest.mark.parametrize("f32", [False, True])
 def test_prefill_attention_slices(f32):
     """Over how many workgroups a prefill call's keys are split: not where the join costs more than it saves (a prompt from its start), several for
