@@ -957,7 +957,10 @@ __global__ __launch_bounds__(512) void gemm_dma256_kernel(GemmParams p) {
 // products of the terms above 2^-24 of the whole, 6 K / 64 columns.
 // Why: the [hi | lo] copy that the dense tile takes doubles the products and the bytes of the copy.  The codes carry no rounding at all;
 // [hi | lo] drops what lies below 2^-17 of a weight.  Around their middle: codes of 0..15 (255) make sums of twice the size and more that
-// the biases take back; the float32 result is then 4.5e-7 from the 64-bit one (6144 x 4096, 1024 rows, 2-norm), here 1.5e-7, [hi | lo] 4.1e-7.
+// the biases take back; the float32 result is then 4.5e-7 from the 64-bit one (6144 x 4096, 1024 rows, 2-norm), here 1.4e-7, [hi | lo] 4.1e-7.
+// The largest last -- x's lo, mid and hi, then the bias columns, their smallest parts first --, so that few roundings are of the size of the result: 1024
+// x 8192, 64 float32 rows, groups of int4 whose means are 0 / 4 / 12 of their deviations, 1.6e-7 / 0.9e-7 / 0.8e-7; the biases and the hi parts in front 1.8e-7 /
+// 2.4e-7 / 2.3e-7; the streaming kernel 9.7e-7 / 2.7e-7 / 1.5e-7.
 // Registers: 128 accumulators + the group's sums.  A phase is two row tiles x both k blocks, so those are 32 (a quarter tile) and not
 // 64; the FMAs of the first row tile sit in the shadow of the second's MFMAs, those of the second in the next phase's read section.
 // Tile, LDS images, wave grid, ping-pong and epilogues: gemm_dma256_kernel.  What differs in the schedule: A-h0 is read in phases 0 and
@@ -988,7 +991,7 @@ __global__ __launch_bounds__(512) void gemm_codes256_kernel(GemmParams p) {
   const int wm = wave >> 2, wn = wave & 3;
   const int c16 = lane & 15, g = lane >> 4;
   const int bm = blockIdx.x, bn = blockIdx.y, m0 = bm * BM2;
-  // K tiles: [0, nkm) = the groups of x's terms in turn (W is walked once per term), [nkm, nk_all) = the bias columns
+  // K tiles: [0, nkm) = the groups of x's terms in turn, the last term first (W is walked once per term), [nkm, nk_all) = the bias columns
   const int nkm = p.ka / BK, nk_all = nkm + p.kb / BK;
   // this workgroup's: [tb, te) (divisions run on vector registers: back to scalar ones, the DMA bases are built of them)
   const int tb = __builtin_amdgcn_readfirstlane((int)((blockIdx.z * (unsigned)nk_all) / gridDim.z));
@@ -1158,20 +1161,20 @@ __global__ __launch_bounds__(512) void gemm_codes256_kernel(GemmParams p) {
     asm volatile("s_barrier" ::: "memory");
   };
   const uint32_t xrow = (uint32_t)(p.ldx * 2);
-  if (te > nkm) {                                                  // the bias columns, before the groups
+  for (int t0 = 0; t0 < nkm; t0 += p.G) {                          // a run per term of x, the last one (the smallest) first
+    const int lo = max(tb, t0), hi = min(te, t0 + p.G);
+    if (lo >= hi) continue;
+    gs = (const char*)p.sc + (size_t)(lo - t0) * 64;
+    sources((const char*)p.x + (size_t)(nkm - p.G - 2 * t0 + lo) * (BK * 2), xrow, (const char*)p.w + (size_t)(lo - t0) * 2048, (size_t)p.kw * 32);
+    run(hi - lo, std::false_type{});
+  }
+  fold(7);
+  if (te > nkm) {                                                  // the bias columns
     const int lo = max(tb, nkm) - nkm;
     gs = nullptr;
     sources((const char*)p.xs + (size_t)lo * (BK * 2), (uint32_t)(p.kb * 2), (const char*)p.wb + (size_t)lo * 2048, (size_t)p.kb * 32);
     run(te - nkm - lo, std::true_type{});
   }
-  for (int t0 = 0; t0 < nkm; t0 += p.G) {                          // a run per term of x
-    const int lo = max(tb, t0), hi = min(te, t0 + p.G);
-    if (lo >= hi) continue;
-    gs = (const char*)p.sc + (size_t)(lo - t0) * 64;
-    sources((const char*)p.x + (size_t)lo * (BK * 2), xrow, (const char*)p.w + (size_t)(lo - t0) * 2048, (size_t)p.kw * 32);
-    run(hi - lo, std::false_type{});
-  }
-  fold(7);
 #undef PP_ORDER
 #undef PP_READS_DONE
 #undef PP_MMA_DONE
@@ -1708,7 +1711,7 @@ size_t gemm_prefill_scratch_bytes(const LinearW& W, size_t rows) {
 // (three walks against six): 2048 x 1024 x 768 42 / 42, 1536 55 / 62; 3072 x 1024 x 768 49 / 58.
 // Int8 on float32 rows at any size: the alternative there is the streaming kernel on exact codes, and a pair of bf16 is no match for it once a group's
 // mean exceeds 3 of its deviations.  2-norm from 64 bits, 1024 x 1024, 256 rows, means of 0 / 4 / 12 deviations: pair 1.8e-7 / 7.0e-7 / 1.9e-6,
-// streaming 3.3e-7 / 1.3e-7 / 1.0e-7, here 0.9e-7 / 1.1e-7 / 1.1e-7 (K = 8192, 64 rows: 5.3e-7 / 8.4e-7 / 1.9e-6, 3.4e-7 / 1.5e-7 / 1.3e-7, 1.7e-7 / 2.5e-7 / 2.3e-7);
+// streaming 3.3e-7 / 1.3e-7 / 1.0e-7, here 0.8e-7 / 0.7e-7 / 0.7e-7 (2048 x 4096, 160 rows: 3.7e-7 / 7.7e-7 / 1.9e-6, 3.4e-7 / 1.4e-7 / 1.2e-7, 1.2e-7 / 0.8e-7 / 0.8e-7);
 // us, streaming / here: 129 rows 59 / 29, 1365 rows 511 / 40.
 static bool codes_plan(const LinearW& W, const GemvCall& c, size_t rows, int ldx, int terms, bool split_ok, size_t cap, GemmParams& p, long& blocks) {
   const bool sw = c.epi == EPI_SWIGLU;

@@ -128,10 +128,10 @@ int launch_dequant_q4_hilo(const LinearW& src, void* dst, hipStream_t st);
 int codes16_bias_cols(int K);
 size_t codes16_bytes(int N, int K);
 int launch_codes16(const LinearW& src, void* dst, hipStream_t st);
-// term t of that product: part of x's group sum (0 = hi, 1 = mid, 2 = lo) and of the bias; products below 2^-24 of the whole are left out
+// term t of that product, the smallest first: part of x's group sum (0 = hi, 1 = mid, 2 = lo) and of the bias; products below 2^-24 of the whole are left out
 constexpr int CODES16_TERMS = 6;
-__host__ __device__ constexpr int codes16_sum_part(int t) { return t < 3 ? t : t == 5 ? 0 : t - 3; }
-__host__ __device__ constexpr int codes16_bias_part(int t) { return t < 3 ? 0 : t < 5 ? 1 : 2; }
+__host__ __device__ constexpr int codes16_sum_part(int t) { return t < 3 ? t & 1 : 5 - t; }
+__host__ __device__ constexpr int codes16_bias_part(int t) { return t < 1 ? 2 : t < 3 ? 1 : 0; }
 // v = hi + mid + lo in bf16 (an infinity is its own first part)
 __device__ __forceinline__ float bf16_part(float v, int part) {
   const float hi = (float)(bf16)v, r = isinf(v) ? 0.f : v - hi, mid = (float)(bf16)r;

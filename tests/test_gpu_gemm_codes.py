@@ -13,7 +13,7 @@ from oracle.numerics import matmul_nt, round_to
 pytestmark = pytest.mark.gpu
 
 from mlx_parallm_amd import _lib as L  # noqa: E402
-from gpu_helpers import dev, dev_u32, gemv_args, host, op_linear, to_tiled  # noqa: E402
+from gpu_helpers import dev, dev_u32, gemm_skinny, gemv_args, host, op_linear, to_tiled  # noqa: E402
 from test_gpu_gemm_prefill import _rows  # noqa: E402
 from test_gpu_kernels import _assert_close  # noqa: E402
 
@@ -29,11 +29,12 @@ def _weight(bits, sdt, N, K, rng):
     return ol, ref_quant.dequantize(packed, s, b, 64, bits), keep
 
 
-def _run(ol, x, M, act, rnd=0, **kw):
+def _run(ol, x, M, act, rnd=0, force=False, **kw):
+    """force: the codes kernel at any size, or an error"""
     a = gemv_args(x, M, act, **kw)
     a.rnd = rnd
     torch.cuda.synchronize()
-    L.check(L.lib().mi_op_gemm_codes(C.byref(ol), C.byref(a), 0, None))
+    L.check(L.lib().mi_op_gemm_codes(C.byref(ol), C.byref(a), -1 if force else 0, None))
     torch.cuda.synchronize()
 
 
@@ -133,3 +134,26 @@ def test_int8_on_float32_rows_is_as_close_as_float32_sums(M, N, K, epi):
     # (SwiGLU: two such factors, and the sigmoid's expf and quotient, 3 ulp)
     n = K / 64 + 6 * K / 2048 + 2
     assert off <= 2.0 ** -24 * np.sqrt(n if epi != "SWIGLU" else 2 * n + 12), off
+
+
+@pytest.mark.parametrize("bits,M,N,K", [(4, 64, 256, 8192), (8, 160, 512, 8192), (8, 192, 256, 14336), (4, 96, 512, 2048)])
+@pytest.mark.parametrize("mean", [0, 4, 12])
+def test_float32_rows_are_no_further_off_than_the_streaming_kernel(bits, M, N, K, mean):
+    """The codes kernel takes float32 rows from the streaming kernel: its 2-norm from 64 bits is no larger, whatever the biases' share of the result."""
+    rng = np.random.default_rng(K + mean)
+    w = (rng.standard_normal((N, K // 64, 64)) + mean * rng.standard_normal((N, K // 64, 1))).astype(np.float32) * 0.05
+    packed, s, b = ref_quant.quantize(w.reshape(N, K), 64, bits, "bfloat16")
+    keep = [dev_u32(packed), dev(s, "bfloat16"), dev(b, "bfloat16")]
+    ol = op_linear(f"q{bits}_bf16", N, K, *keep)
+    assert to_tiled(ol, keep)
+    codes = np.stack([packed >> np.uint32(bits * i) & np.uint32((1 << bits) - 1) for i in range(32 // bits)], -1).reshape(N, K).astype(np.float64)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    want = x.astype(np.float64) @ (codes * np.repeat(s, 64, 1).astype(np.float64) + np.repeat(b, 64, 1)).T
+    xd, out = dev(x), torch.zeros((M, N), dtype=torch.float32, device="cuda")
+    _run(ol, xd, M, "float32", force=True, epi=L.EPI_STORE, out=out, ldo=N)
+    off = np.linalg.norm(host(out) - want)
+    out.zero_()
+    for r in range(0, M, 32):
+        gemm_skinny(ol, xd[r:r + 32], 32, "float32", epi=L.EPI_STORE, out=out[r:r + 32], ldo=N)
+    ref = np.linalg.norm(host(out) - want)
+    assert off <= ref, (off / np.linalg.norm(want), ref / np.linalg.norm(want))
