@@ -422,7 +422,9 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
       MI_TRY(launch_rmsnorm_rows(c.x, c.ldx, c.norm_w, e->xn, KT, (int)rows, KT, c.eps, c.act, e->stream, true));
       c.x = e->xn; c.ldx = KT; c.pro = PRO_NONE;
     }
-    // logits of many positions against a quantised matrix: 32768 outputs at a time, so that the copy below stays within 4 x 32768 x K bytes
+    // logits of many positions against a quantised matrix: 32768 outputs at a time, so that the copy below stays within 4 x 32768 x K bytes.  The
+    // kernel is chosen for all of them: a last piece of few columns is no reason for the [hi | lo] copy
+    c.codes = quant && gemm_prefill_on_codes(f.W, c, rows);
     const int ncol = (wk_is_quant(f.W.wk) && c.epi == EPI_STORE_F32) ? std::min(f.W.N, 32768) : f.W.N;
     void* scratch = nullptr;
     if (wk_is_quant(f.W.wk)) {               // the GEMM multiplies by 16-bit codes, or a [hi | lo] 16-bit copy, made on the fly

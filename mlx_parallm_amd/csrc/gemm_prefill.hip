@@ -1741,15 +1741,20 @@ static bool gemm_prefill_pays_codes(const LinearW& W, const GemvCall& c, size_t 
   return 12.0 + 0.65 * mw + 1.35 * rounds * tiles + reduce < (double)((rows + 31) / 32) * (10.0 + 0.36 * mw);
 }
 
+bool gemm_prefill_on_codes(const LinearW& W, const GemvCall& c, size_t rows) {
+  const int terms = c.act == MI_F32 && c.rnd != RND_BF16 ? 3 : 1;
+  GemmParams p{};
+  long blocks = 0;
+  return codes_plan(W, c, rows, c.act == MI_F32 ? terms * W.K : c.ldx, terms, false, 0, p, blocks);
+}
+
 int gemm_prefill_quant_route(const LinearW& W, const GemvCall& c, size_t rows) {
   if (!gemm_prefill_supported(W, c, rows)) return 0;
   const bool x32 = c.act == MI_F32;
   const int terms = x32 && c.rnd != RND_BF16 ? 3 : 1;
   const size_t cap = rows < 4096 ? (size_t)128 << 20 : 0;                       // (of the engine's workspace for slices)
   if (x32 && rows > 32 && gemm_skinny_supported(W, c, 32) && !gemm_prefill_pays_codes(W, c, rows, terms, cap)) return 0;
-  GemmParams p{};
-  long blocks = 0;
-  return codes_plan(W, c, rows, x32 ? terms * W.K : c.ldx, terms, cap > 0, cap, p, blocks) ? 2 : 1;
+  return gemm_prefill_on_codes(W, c, rows) ? 2 : 1;
 }
 
 // quantised matrices on gemm_codes256_kernel; *done = false: the [hi | lo] copy and the dense tiles take the call

@@ -56,7 +56,7 @@ struct GemvCall {
   int split_out = 0;              // EPI_SWIGLU on float32 activations: out holds rows of [hi | lo] bf16 (2 ldo columns), the form launch_split3_rows makes
                                   // of two terms, where gemm_prefill_split_out says so
   int x_split = 0;                // float32 activations: x holds such rows already
-  int codes = 0;                  // quantised matrices: the tile GEMM on their codes whatever the size, or an error
+  int codes = 0;                  // quantised matrices: the tile GEMM on their codes whatever the size, or an error (a piece of a larger matrix)
   int kx = 0;                     // > 0: W is a [hi | lo] matrix of 2 kx columns (an f16 model in the float32-activation mode): the
                                   // activations have kx columns and are walked twice (k mod kx); 0: W.K columns
   // RMSNorm hand-over between two launches of gemm_skinny.hip's 16-row instantiation: a residual epilogue leaves
@@ -94,6 +94,7 @@ bool gemm_prefill_pays(bool codes, bool hilo, bool rounded, size_t rows);
 bool gemm_prefill_split_out(const LinearW& W, const GemvCall& c, size_t rows);
 // any prefill call on a quantised matrix: 2 = the tile GEMM on its codes, 1 = on its [hi | lo] copy, 0 = not the tile GEMM
 int gemm_prefill_quant_route(const LinearW& W, const GemvCall& c, size_t rows);
+bool gemm_prefill_on_codes(const LinearW& W, const GemvCall& c, size_t rows);     // .. once it is the tile GEMM
 // splitk_ws / splitk_cap: float32 workspace for the K-split form of the 128 x 128 tile (few hundred rows against a narrow
 // matrix); null = never split
 int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st, void* scratch = nullptr,

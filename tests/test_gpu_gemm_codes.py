@@ -157,3 +157,41 @@ def test_float32_rows_are_no_further_off_than_the_streaming_kernel(bits, M, N, K
         gemm_skinny(ol, xd[r:r + 32], 32, "float32", epi=L.EPI_STORE, out=out[r:r + 32], ldo=N)
     ref = np.linalg.norm(host(out) - want)
     assert off <= ref, (off / np.linalg.norm(want), ref / np.linalg.norm(want))
+
+
+@pytest.mark.parametrize("kv", ["float32", "model"])
+def test_the_last_piece_of_wide_logits_is_no_other_kernel(kv):
+    """Logits of many positions are made 32768 columns at a time.  The last sixteen of these have the weights of the first sixteen: the same numbers, up to
+    the sums' roundings (two results, each as above) -- with a [hi | lo] copy for them it is 5.1e-7 (int4 groups, means of 100 of their deviations)."""
+    from mlx_parallm_amd.engine import Engine
+
+    H, V, K = 1024, 32784, 1024
+    cfg = dict(model_type="llama", hidden_size=H, num_hidden_layers=1, num_attention_heads=8, num_key_value_heads=8, head_dim=128, intermediate_size=1024,
+               vocab_size=V, rms_norm_eps=1e-5, rope_theta=10000.0, tie_word_embeddings=False, max_position_embeddings=1024, quantization={"bits": 4, "group_size": 64})
+    eng = Engine(cfg, device=0, max_positions=512, act_dtype="bfloat16")
+    rng = np.random.default_rng(7)
+
+    def put(name, n, mean=0.0, repeat=0):
+        w = ((rng.standard_normal((n, K // 64, 64)) + mean * rng.standard_normal((n, K // 64, 1))) * 0.03).astype(np.float32).reshape(n, K)
+        if repeat:
+            w[-repeat:] = w[:repeat]
+        packed, s, b = ref_quant.quantize(w, 64, 4, "bfloat16")
+        for part, t in ((".weight", dev_u32(packed)), (".scales", dev(s, "bfloat16")), (".biases", dev(b, "bfloat16"))):
+            eng.set_tensor(name + part, t)
+    put("model.embed_tokens", V)
+    p = "model.layers.0."
+    for n in ("self_attn.q_proj", "self_attn.k_proj", "self_attn.v_proj", "self_attn.o_proj", "mlp.gate_proj", "mlp.up_proj", "mlp.down_proj"):
+        put(p + n, H)
+    for n in (p + "input_layernorm", p + "post_attention_layernorm", "model.norm"):
+        eng.set_tensor(n + ".weight", torch.ones(H, dtype=torch.bfloat16, device="cuda"))
+    put("lm_head", V, mean=100.0, repeat=16)
+    eng.finalize()
+    got = np.array(eng.forward(rng.integers(0, V, (1, 256)).astype(np.int32), eng.new_kv(1, capacity=300, kv_dtype=kv), all_positions=True), dtype=np.float64)[0]
+    eng.close()
+    first, last = got[:, :16], got[:, -16:]
+    assert np.all(np.isfinite(got)) and np.linalg.norm(first) > 0
+    off = np.linalg.norm(first - last) / np.linalg.norm(first)
+    if kv == "model":                                            # (bfloat16 logits: at most some that fall to the other neighbour)
+        assert np.mean(first != last) <= 0.01 and off <= 2.0 ** -8
+    else:
+        assert off <= 2.0 ** -24 * np.sqrt(2 * (K / 64 + 6 * K / 2048 + 2)), off
