@@ -484,7 +484,8 @@ __global__ __launch_bounds__(512, 2) void q4_kernel(const Q4Params p) {
 
 struct Q4Plan { int mt, nslab, ksplit, ntu, ntiles, ngroups, nblk; size_t xq_bytes, sx_bytes, sxo_bytes, ws_bytes; };
 
-thread_local int q4_force_mt = 0, q4_force_ks = 0;               // test hook: row tiles per workgroup, K slices
+thread_local int q4_force_mt = 0, q4_force_ks = 0;               // test hook: row tiles per workgroup, K slices (0: the plan's own)
+thread_local bool q4_forced = false;                             // .. and whatever the width
 
 Q4Plan q4_plan(const LinearW& W, const GemvCall& c, size_t rows) {
   Q4Plan pl{};
@@ -541,21 +542,19 @@ int q4_launch_at(const Q4Params& p, int mt, bool sw, int grid, hipStream_t st) {
 }  // namespace
 
 // test hook: row tiles | .. << 3 | .. << 7 | K slices << 11 (the fields between are this kernel's fixed shape); 0 clears
-void gemm_q4_force(int code) { q4_force_mt = code & 7; q4_force_ks = (code >> 11) & 15; }
+void gemm_q4_force(int code) { q4_force_mt = code & 7; q4_force_ks = (code >> 11) & 15; q4_forced = code != 0; }
 
 // The wide matrices.  us, 64 rows (32 rows), against gemm_skinny.hip's K over workgroups; with the preparation pass, which replaces a norm launch of
 // 4.7 us in front of gate|up and the logits: 34816 x 5120 SwiGLU 42 (31) against 71 (40), 28672 x 4096 33 (25) against 40 (25), 151936 x 5120
 // 172 (131) against 272 (149), 20480 x 5120 37 (27) against 42 (26).  A workgroup's head and tail are some 10 us, slices of K another 8: 7168 x 5120
 // 30 (21) against 23 (16), 5120 x 17408 42 (31) against 37 (26); few rows on short K: 50304 x 2048 45 (34) against 40 (22).
-constexpr int Q4_MIN_TILES = 1024;
-
 bool gemm_q4_supported(const LinearW& W, const GemvCall& c, size_t rows) {
   if (c.force_v1 || W.layout != 1 || c.rnd != RND_NONE || c.out32) return false;
   const bool q4 = ((W.wk == WK_Q4_BF16 && c.act == MI_BF16) || (W.wk == WK_Q4_F16 && c.act == MI_F16)) && W.group == 64 && W.K % 128 == 0;
   if (!q4 || rows < 17 || rows > 128 || c.ldx % 8 != 0) return false;
   if (c.epi == EPI_SWIGLU_GU8 || c.glu.kind != GLU_SILU || c.silu_cols > 0) return false;
   if (W.N % 16 != 0 || (c.epi == EPI_SWIGLU && c.pair_offset % 16 != 0)) return false;
-  if (q4_force_mt == 0 && q4_force_ks == 0 && (W.N / 16 < Q4_MIN_TILES || (rows <= 32 && W.K < 3072))) return false;
+  if (!q4_forced && (W.N / 16 < GEMM_Q4_MIN_TILES || (rows <= 32 && W.K < 3072))) return false;
   return (size_t)(W.N / 16) * (W.K / 128) * 1152 < ((size_t)1 << 32);          // (32-bit offsets of the LDS-DMA sources)
 }
 

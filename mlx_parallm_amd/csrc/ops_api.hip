@@ -88,7 +88,10 @@ int mi_op_gemm_skinny(const mi_op_linear* w, const mi_op_gemv_args* a, int kspli
   MI_TRY(ready());
   const LinearW W = to_linear(w);
   const GemvCall c = to_call(a);
-  struct ForceGuard { bool on; ~ForceGuard() { if (on) gemm_q4_force(0); } } guard{ksplit < 0};
+  // a norm in front of a wide int4 matrix: gemm_q4.hip applies it, also at the few rows and short K where the engine runs the norm and gemm_skinny.hip
+  const bool wide_norm = ksplit == 0 && c.pro == PRO_NORM && c.act != MI_F32 && wk_bits(W.wk) == 4 && W.N / 16 >= GEMM_Q4_MIN_TILES;
+  struct ForceGuard { bool on; ~ForceGuard() { if (on) gemm_q4_force(0); } } guard{ksplit < 0 || wide_norm};
+  if (wide_norm) gemm_q4_force(1 << 3);
   if (ksplit < 0) {
     gemm_q4_force(-ksplit);
     if (!gemm_q4_supported(W, c, (size_t)c.M)) return fail(MI_ERR_UNSUPPORTED, "mi_op_gemm_skinny: ksplit < 0 forces gemm_q4, which does not take this call");

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 import torch
 
+from oracle import ref_model
 from oracle.numerics import matmul_nt, round_to
 
 pytestmark = pytest.mark.gpu
@@ -33,3 +34,24 @@ def test_block_counts_and_slices(act, M, N, K, mt, ks):
         outs.append(host(out))
     assert np.array_equal(outs[0], outs[1]) and np.all(outs[0][M:] == 7.0)
     _assert_close(outs[0][:M], round_to(matmul_nt(x, w), act), act)
+
+
+def test_every_forced_plan_and_every_norm_in_front_of_a_wide_matrix_is_taken():
+    """ksplit < 0 forces the kernel also where only fields are set that it ignores; a norm in front of >= 1024 column tiles is applied at any row count and K."""
+    act, M, N, K = "bfloat16", 20, 16384, 256
+    rng = np.random.default_rng(5)
+    ol, w, keep = _weight(4, act, N, K, rng)
+    x = round_to(rng.standard_normal((M, K)).astype(np.float32), act)
+    nw = round_to(1.0 + 0.1 * rng.standard_normal(K).astype(np.float32), act)
+    xd, nwd = dev(x, act), dev(nw, act)
+    out = torch.full((M + 2, N), 7.0, dtype=xd.dtype, device="cuda")
+    gemm_skinny(ol, xd, M, act, epi=L.EPI_STORE, out=out, ldo=N, norm_w=nwd, eps=1e-5)
+    assert np.all(host(out)[M:] == 7.0)
+    _assert_close(host(out)[:M], round_to(matmul_nt(ref_model.rms_norm(x, act, nw, act, 1e-5)[0], w), act), act)
+    ol.N = 208                                                   # (its first rows alone)
+    want = round_to(matmul_nt(x, w[:208]), act)
+    for code in (4 << 3, 2 << 7, 2 << 15):                       # tile units, K lanes, staging waves
+        out = torch.full((M + 2, 208), 7.0, dtype=xd.dtype, device="cuda")
+        gemm_skinny(ol, xd, M, act, epi=L.EPI_STORE, out=out, ldo=208, ksplit=-code)
+        assert np.all(host(out)[M:] == 7.0)
+        _assert_close(host(out)[:M], want, act)
