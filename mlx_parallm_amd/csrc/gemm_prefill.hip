@@ -1182,22 +1182,13 @@ __global__ __launch_bounds__(512) void gemm_codes256_kernel(GemmParams p) {
   if constexpr (!SWIGLU) {
     if (gridDim.z > 1) { tile256_partial(p, acc, smem2, m0, bn, wave, lane); return; }
   }
+  // (one gated unit, no silu columns: codes_fits; rows that are no whole pieces are none of the engine's)
   if (p.strips) {
     __syncthreads();
-    if (!LOGITS && epilogue_varies<SWIGLU>(p, bn)) tile256_epilogue_strips<AT, SWIGLU, true, LOGITS>(p, acc, smem2, m0, bn, wave, lane);
-    else tile256_epilogue_strips<AT, SWIGLU, false, LOGITS>(p, acc, smem2, m0, bn, wave, lane);
-    return;
+    tile256_epilogue_strips<AT, SWIGLU, false, LOGITS>(p, acc, smem2, m0, bn, wave, lane);
+  } else {
+    tile256_epilogue<AT, SWIGLU, false, LOGITS>(p, acc, m0, bn, wm, wn, c16, g);
   }
-  if constexpr (!SWIGLU && !LOGITS) {
-    if (p.epi == EPI_RESID) {
-      if (p.out32) tile256_epilogue_resid<AT, float>(p, acc, m0, bn, wm, wn, c16, g);
-      else tile256_epilogue_resid<AT, AT>(p, acc, m0, bn, wm, wn, c16, g);
-      return;
-    }
-  }
-  if constexpr (LOGITS) tile256_epilogue<AT, SWIGLU, false, true>(p, acc, m0, bn, wm, wn, c16, g);
-  else if (epilogue_varies<SWIGLU>(p, bn)) tile256_epilogue<AT, SWIGLU, true>(p, acc, m0, bn, wm, wn, c16, g);
-  else tile256_epilogue<AT, SWIGLU, false>(p, acc, m0, bn, wm, wn, c16, g);
 }
 
 // The group sums of x for the kernel above: row m -> `parts` terms of G columns each (kernels.h: codes16_sum_part; hi + mid + lo = the float32 sum
@@ -1589,6 +1580,7 @@ int launch_rmsnorm_block(const void* x, int ldx, const void* w, void* out, int l
 // What gemm_codes256_kernel can do at all, rows of stride ldx
 static bool codes_fits(const LinearW& W, const GemvCall& c, size_t rows, size_t ldx) {
   if (!wk_is_quant(W.wk) || W.layout != 1 || W.group != 64 || W.K % BK != 0 || W.K > 65536) return false;      // (the biases of a row tile in 64 KiB of LDS)
+  if (c.glu.kind != GLU_SILU || c.silu_cols > 0) return false;                 // (no quantised model has another unit)
   const size_t lim = (size_t)1 << 32;                    // (32-bit offsets of the LDS-DMA sources)
   return rows * ldx * 2 < lim && rows * codes16_bias_cols(W.K) * 2 < lim && (size_t)W.N * (W.K / 64) * 4 < lim;
 }
