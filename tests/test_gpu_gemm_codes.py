@@ -1,6 +1,7 @@
 """Kernel-level parity (-m gpu) of the tile GEMM on int4 / int8 codes (gemm_prefill.hip: gemm_codes256_kernel, the nn.QuantizedLinear of
 the prefill call, utils.py:243-262,679-690) through mi_op_gemm_codes: against the oracle's matmul over the dequantised weights on
-sampled rows, for every epilogue, at the edges of tiles and runs."""
+sampled rows, for every epilogue, at the edges of tiles and runs.  The codes kernel is forced: below some 4e9 products the call alone would run on the
+[hi | lo] copy."""
 import ctypes as C
 
 import numpy as np
@@ -41,7 +42,7 @@ def _run(ol, x, M, act, rnd=0, force=False, **kw):
 @pytest.mark.parametrize("act", ["bfloat16", "float16"])
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("M,N,K", [
-    (256, 2048, 1024),       # one row tile, K split: slices that end inside a run
+    (256, 2048, 1024),       # one row tile, K split: slices that end inside the groups
     (300, 2064, 1152),       # ragged rows, a column tile of 16, 18 groups (the bias columns end inside a K tile)
     (2085, 6144, 128),       # two groups: a run that is all prologue, unsplit
     (2304, 5632, 640),       # an even number of groups, unsplit
@@ -55,19 +56,26 @@ def test_store_logits_and_residual(act, bits, M, N, K):
     xd, rows = dev(x, act), _rows(M)
     y = round_to(matmul_nt(x[rows], w), act)
     out = torch.full((M + 3, N), 7.0, dtype=xd.dtype, device="cuda")
-    _run(ol, xd, M, act, epi=L.EPI_STORE, out=out, ldo=N)
+    _run(ol, xd, M, act, force=True, epi=L.EPI_STORE, out=out, ldo=N)
     o = host(out)
     assert np.all(o[M:] == 7.0), "rows past M were written"
     _assert_close(o[:M][rows], y, act)
     lg = torch.full((M + 3, N), 7.0, dtype=torch.float32, device="cuda")          # logits: the same values as float32
-    _run(ol, xd, M, act, epi=L.EPI_STORE_F32, out=lg, ldo=N)
+    _run(ol, xd, M, act, force=True, epi=L.EPI_STORE_F32, out=lg, ldo=N)
     assert np.array_equal(host(lg)[:M], o[:M]) and np.all(host(lg)[M:] == 7.0)
     h = dev(h0, act)
-    _run(ol, xd, M, act, epi=L.EPI_RESID, resid=h, out=h, ldo=N)
+    _run(ol, xd, M, act, force=True, epi=L.EPI_RESID, resid=h, out=h, ldo=N)
     _assert_close(host(h)[rows], round_to(h0[rows] + y, act), act)
+    odd = torch.full((M + 1, N + 2), 7.0, dtype=xd.dtype, device="cuda")          # rows that are no whole 16-byte pieces
+    _run(ol, xd, M, act, force=True, epi=L.EPI_STORE, out=odd, ldo=N + 2)
+    assert np.array_equal(host(odd)[:M, :N], o[:M]) and np.all(host(odd)[M:] == 7.0) and np.all(host(odd)[:, N:] == 7.0)
+    odd[:M, :N] = dev(h0, act)
+    _run(ol, xd, M, act, force=True, epi=L.EPI_RESID, resid=odd, out=odd, ldo=N + 2)
+    assert np.array_equal(host(odd)[:M, :N], host(h)) and np.all(host(odd)[M:] == 7.0) and np.all(host(odd)[:, N:] == 7.0)
 
 
-@pytest.mark.parametrize("act,bits,M,I,K", [("bfloat16", 4, 2085, 3072, 512), ("bfloat16", 8, 517, 8208, 192), ("float16", 4, 2048, 3200, 256)])
+@pytest.mark.parametrize("act", ["bfloat16", "float16"])
+@pytest.mark.parametrize("bits,M,I,K", [(4, 2085, 3072, 512), (8, 517, 8208, 192), (4, 2048, 3200, 256), (8, 130, 144, 64)])
 def test_swiglu(act, bits, M, I, K):
     rng = np.random.default_rng(M)
     ol, w, keep = _weight(bits, act, 2 * I, K, rng)
@@ -78,31 +86,55 @@ def test_swiglu(act, bits, M, I, K):
     sig = round_to((1.0 / (1.0 + np.exp(-gt))).astype(np.float32), act)
     want = round_to(round_to(gt.astype(np.float32) * sig, act) * up, act)
     out = torch.full((M + 1, I), 7.0, dtype=xd.dtype, device="cuda")
-    _run(ol, xd, M, act, epi=L.EPI_SWIGLU, out=out, ldo=I, pair_offset=I)
+    _run(ol, xd, M, act, force=True, epi=L.EPI_SWIGLU, out=out, ldo=I, pair_offset=I)
     o = host(out)
     assert np.all(o[M:] == 7.0)
     _assert_close(o[:M][rows], want, act, scale=float(np.abs(y).max()))
+    odd = torch.full((M + 1, I + 2), 7.0, dtype=xd.dtype, device="cuda")
+    _run(ol, xd, M, act, force=True, epi=L.EPI_SWIGLU, out=odd, ldo=I + 2, pair_offset=I)
+    assert np.array_equal(host(odd)[:M, :I], o[:M]) and np.all(host(odd)[M:] == 7.0) and np.all(host(odd)[:, I:] == 7.0)
 
 
-@pytest.mark.parametrize("M,N,K,rnd", [(300, 2048, 1024, 0), (2085, 6144, 256, 0), (64, 2768, 4096, 0), (1024, 6144, 640, L.RND_BF16)])
-def test_float32_rows(M, N, K, rnd):
-    """three bf16 terms of x (a run over the codes per term); rnd: layer 0's rounded call, x is one term"""
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M,N,K,rnd", [(300, 2048, 1024, 0), (2085, 6144, 256, 0), (64, 2768, 4096, 0), (131, 48, 4096, 0), (1024, 6144, 640, L.RND_BF16)])
+def test_float32_rows(bits, M, N, K, rnd):
+    """three bf16 terms of x (a run over the codes per term), every epilogue; rnd: layer 0's rounded call, x is one term"""
+    if bits == 8 and M <= 128:
+        M += 128                                                 # (up to there int8 keeps the streaming kernel)
     rng = np.random.default_rng(K)
-    ol, w, keep = _weight(4, "bfloat16", N, K, rng)
+    ol, w, keep = _weight(bits, "bfloat16", N, K, rng)
     x = rng.standard_normal((M, K)).astype(np.float32)
     if rnd:
         x = round_to(x, "bfloat16")
-    rows = _rows(M)
+    rows, xd = _rows(M), dev(x)
     want = matmul_nt(x[rows], w)
-    out = torch.full((M + 1, N), 7.0, dtype=torch.float32, device="cuda")
-    _run(ol, dev(x), M, "float32", rnd=rnd, epi=L.EPI_STORE, out=out, ldo=N)
-    o = host(out)
-    assert np.all(o[M:] == 7.0)
+    # exact products; K / 64 + 2 float32 additions of a group's sums and the biases', of up to 16 scales x |x| each
+    tol = 2.0 ** -24 * (K / 64 + 8) * 4 * np.abs(x[rows]).sum(1).max() * np.abs(w).max()
+
+    def call(epi, cols, fill=None, pad=0):
+        out = torch.full((M + 1, cols + pad), 7.0, dtype=torch.float32, device="cuda")
+        if fill is not None:
+            out[:M, :cols] = dev(fill)
+        _run(ol, xd, M, "float32", rnd=rnd, force=True, epi=epi, out=out, resid=out if epi == L.EPI_RESID else None, ldo=cols + pad, pair_offset=cols if epi == L.EPI_SWIGLU else 0)
+        o = host(out)
+        assert np.all(o[M:] == 7.0) and np.all(o[:, cols:] == 7.0)
+        return o[:M, :cols]
+    got = call(L.EPI_STORE, N)
+    assert np.array_equal(call(L.EPI_STORE, N, pad=2), got)      # (rows that are no whole 16-byte pieces)
     if rnd:
-        _assert_close(o[:M][rows], round_to(want, "bfloat16"), "bfloat16")
-    else:
-        # exact products; K / 64 + 2 float32 additions of a group's sums and the biases', of up to 16 scales x |x| each
-        assert np.max(np.abs(o[:M][rows] - want)) <= 2.0 ** -24 * (K / 64 + 8) * 4 * np.abs(x[rows]).sum(1).max() * np.abs(w).max()
+        _assert_close(got[rows], round_to(want, "bfloat16"), "bfloat16")
+        return
+    assert np.max(np.abs(got[rows] - want)) <= tol
+    assert np.array_equal(call(L.EPI_STORE_F32, N), got)
+    h = rng.standard_normal((M, N)).astype(np.float32)
+    for pad in (0, 2):
+        assert np.array_equal(call(L.EPI_RESID, N, fill=h, pad=pad), h + got)
+    I = N // 32 * 16
+    gt, up = want[:, :I].astype(np.float64), want[:, I:2 * I].astype(np.float64)
+    unit = gt / (1 + np.exp(-gt))
+    for pad in (0, 2):                                           # |silu'| <= 1.1; its expf, quotient and two products: 2^-21 of the result
+        y = call(L.EPI_SWIGLU, I, pad=pad)[rows]
+        assert np.all(np.abs(y - unit * up) <= tol * (1.1 * np.abs(up) + np.abs(unit) + tol) + 2.0 ** -21 * np.abs(unit * up))
 
 
 @pytest.mark.parametrize("M,N,K,epi", [(129, 1024, 1024, "STORE"), (300, 208, 704, "STORE"), (1365, 1024, 1024, "RESID"), (200, 2048, 1024, "SWIGLU"), (160, 48, 64, "STORE"),
