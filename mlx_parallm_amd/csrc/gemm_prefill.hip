@@ -16,6 +16,7 @@
 //   * SwiGLU: a wave's four N tiles are two gate tiles and the two matching up tiles, so
 //     silu(gate) * up happens in registers.
 #include <algorithm>
+#include <atomic>
 #include <cstdlib>
 #include <type_traits>
 
@@ -1749,6 +1750,21 @@ int gemm_prefill_quant_route(const LinearW& W, const GemvCall& c, size_t rows) {
   return gemm_prefill_on_codes(W, c, rows) ? 2 : 1;
 }
 
+template <typename AT, bool SWIGLU, bool LOGITS>
+static int codes_launch(const GemmParams& p, dim3 grid, hipStream_t st) {
+  auto k = gemm_codes256_kernel<AT, SWIGLU, LOGITS>;
+  static std::atomic<bool> opted_in[64];                // per device: several engines, and threads, may live in one process
+  int dev = 0;
+  MI_HIP(hipGetDevice(&dev));
+  if (dev < 0 || dev >= 64 || !opted_in[dev].load(std::memory_order_acquire)) {
+    MI_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, CODES_LDS));
+    if (dev >= 0 && dev < 64) opted_in[dev].store(true, std::memory_order_release);
+  }
+  hipLaunchKernelGGL(k, grid, dim3(512), CODES_LDS, st, p);
+  MI_HIP(hipGetLastError());
+  return MI_OK;
+}
+
 // quantised matrices on gemm_codes256_kernel; *done = false: the [hi | lo] copy and the dense tiles take the call
 static int launch_gemm_codes(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st, void* scratch, void* splitk_ws, size_t splitk_cap, bool* done) {
   *done = false;
@@ -1774,16 +1790,10 @@ static int launch_gemm_codes(const LinearW& W, const GemvCall& c, size_t rows, h
     if (!x32) { p.out32 = 1; p.rnd = c.act == MI_BF16 ? RND_BF16 : RND_F16; }
   }
   p.strips = strips_ok(p);
-  const dim3 grid((unsigned)((rows + BM2 - 1) / BM2), (ncols + (sw ? 128 : BN2) - 1) / (sw ? 128 : BN2), p.ksplit), block(512);
-  auto go = [&](auto k) -> int {
-    MI_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, CODES_LDS));
-    hipLaunchKernelGGL(k, grid, block, CODES_LDS, st, p);
-    MI_HIP(hipGetLastError());
-    return MI_OK;
-  };
+  const dim3 grid((unsigned)((rows + BM2 - 1) / BM2), (ncols + (sw ? 128 : BN2) - 1) / (sw ? 128 : BN2), p.ksplit);
   const bool rounded = p.rnd != RND_NONE;               // (float32 stores of values rounded to 16 bits: logits, and layer 0 of the float32-cache mode)
-  if (c.act == MI_F16) MI_TRY(sw ? go(gemm_codes256_kernel<f16, true>) : rounded ? go(gemm_codes256_kernel<f16, false, true>) : go(gemm_codes256_kernel<f16, false>));
-  else MI_TRY(sw ? go(gemm_codes256_kernel<bf16, true>) : rounded ? go(gemm_codes256_kernel<bf16, false, true>) : go(gemm_codes256_kernel<bf16, false>));
+  if (c.act == MI_F16) MI_TRY((sw ? codes_launch<f16, true, false> : rounded ? codes_launch<f16, false, true> : codes_launch<f16, false, false>)(p, grid, st));
+  else MI_TRY((sw ? codes_launch<bf16, true, false> : rounded ? codes_launch<bf16, false, true> : codes_launch<bf16, false, false>)(p, grid, st));
   if (p.ksplit > 1) MI_TRY(reduce_slices(p, c.act, st));
   *done = true;
   return MI_OK;
