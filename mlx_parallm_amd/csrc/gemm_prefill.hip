@@ -963,14 +963,19 @@ __global__ __launch_bounds__(512) void gemm_dma256_kernel(GemmParams p) {
 // x 8192, 64 float32 rows, groups of int4 whose means are 0 / 4 / 12 of their deviations, 1.6e-7 / 0.9e-7 / 0.8e-7; the biases and the hi parts in front 1.8e-7 /
 // 2.4e-7 / 2.3e-7; the streaming kernel 9.7e-7 / 2.7e-7 / 1.5e-7.
 // Registers: 128 accumulators + the group's sums.  A phase is two row tiles x both k blocks, so those are 32 (a quarter tile) and not
-// 64; the FMAs of the first row tile sit in the shadow of the second's MFMAs, those of the second in the next phase's read section.
-// Tile, LDS images, wave grid, ping-pong and epilogues: gemm_dma256_kernel.  What differs in the schedule: A-h0 is read in phases 0 and
-// 1, A-h1 in 2 and 3, B-k0 in the read section of phase 0, B-k1 in its MFMA section (so it is restaged in phase 2 at the earliest),
-// the scales (256 B of a wave's own, one dword per lane and tile) in phase 0.
-//   stage:  j=0: A-h1(t+1)   j=1: B-k0(t+2)   j=2: B-k1(t+2)   j=3: scales(t+2), A-h0(t+2)
-//     unit                           staged in     waited for in   first read in   DMAs issued since
-//     A-h1(t+1)                      (t, j=0)      (t+1, j=1)      (t+1, j=2)      2 + 2 + 3 + 2 + 2 -> vmcnt(11)
-//     B-k0, B-k1, scales, A-h0(t+2)  (t, j=1..3)   (t+1, j=3)      (t+2, j=0)      2 + 2 + 2 + 3     -> vmcnt(9)
+// 64.  All FMAs sit behind MFMAs, two each: those of a phase's first row tile behind the MFMAs of its second, those of its second behind the
+// first MFMAs of the next phase.
+// Tile, LDS images, wave grid, ping-pong and epilogues: gemm_dma256_kernel.  What differs in the schedule, all reads in read sections: phase 0 reads B-k1 and
+// the scales of its own K tile (256 B of a wave's own, one dword per lane and tile), phases 0 and 1 a half of A-h0 each, 2 and 3 of A-h1, and, for the NEXT K
+// tile, 2 and 3 a half of B-k0 each (into the other of two register sets).
+//   stage:  j=0: A-h1(t+1)   j=1: B-k0(t+2)   j=2: B-k1(t+2)   j=3: scales(t+2), A-h0(t+2)        2 + 2 + 2 + 3 DMAs of a wave (tail: no scales, 8)
+//     unit                        over a unit last read in   staged in     waited for in   first read in   DMAs issued behind it by then
+//     A-h1(t+1)                   (t-1, j=3)                 (t, j=0)      (t+1, j=1)      (t+1, j=2)      2 + 2 + 3 + 2 + 2 = 11
+//     B-k0(t+2)                   (t-1, j=3)                 (t, j=1)      (t+1, j=1)      (t+1, j=2)      2 + 3 + 2 + 2     = 9
+//     B-k1(t+2)                   (t, j=0)                   (t, j=2)      (t+1, j=3)      (t+2, j=0)      3 + 2 + 2 + 2 + 3 = 12
+//     scales(t+2), A-h0(t+2)      (t, j=0), (t, j=1)         (t, j=3)      (t+1, j=3)      (t+2, j=0)      2 + 2 + 2 + 3     = 9
+// Both waits are vmcnt(9) (tail: 8), behind the phase's own staging: at j=1 B-k0 sets the number (with A-h1's 11 it would be read before it has landed), at j=3
+// the scales and A-h0 do.  A unit's last readers have their data before the barrier that its next stager passes first.
 constexpr int CODES_LDS = 2 * DMA_BUF + 8 * 2 * 256;
 
 __device__ __forceinline__ void dma_kib_off(const void* base, uint32_t off, unsigned lds_dst) {
