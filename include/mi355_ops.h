@@ -140,7 +140,8 @@ int mi_op_attention_decode(const mi_op_attn_shape* s, const void* qkv, void* kca
  * ncu compute units (no device needed) */
 int mi_op_attention_decode_splits(int ncu, int groups, int keys, int kv_dtype);
 /* 1: logits (rounded = 0) or layer 0's rounded q|k|v (1) of `rows` rows of float32 activations go to the tile GEMM, 0: 32 rows at a time to the
- * streaming kernel.  codes: int4 weights, hilo: an f16 matrix through its [hi | lo] copy (no device needed) */
+ * streaming kernel.  codes: int4 weights too small for the tile GEMM on codes (the others: mi_op_gemm_quant_route), hilo: an
+ * f16 matrix through its [hi | lo] copy (no device needed) */
 int mi_op_gemm_prefill_pays(int codes, int hilo, int rounded, int rows);
 int mi_op_sample(float* logits, int B, int V, float temperature, float top_p, const float* uniforms,
                  int top_logprobs, int32_t* tokens_out, float* logprob_out, float* prob_row0_out,

@@ -1624,6 +1624,8 @@ bool gemm_prefill_supported(const LinearW& W, const GemvCall& c, size_t rows) {
 //   logits, dense and f16 64 rows +40 / +351, 128 -26 / -112, 192 -6 / -163, 256 -214 / -1257; f16 +111 / +796, -40 / -231, +35 / +59, -367 / -2179:
 //                         a row of 128-row tiles costs three to four launches of 32 rows; from 256 rows the 256 x 256 tile runs
 //           int4          64 rows +323 / +2144, 512 -103 / +88, 768 +42 / -412, 1024 -341 / -760 (the copy: 4 bytes per weight; six walks)
+// (int4: figures of the [hi | lo] copy.  These lines are left with the matrices that are too small for the codes at the call's rows; the others:
+// gemm_prefill_pays_codes)
 bool gemm_prefill_pays(bool codes, bool hilo, bool rounded, size_t rows) {
   if (rounded) return rows > (hilo ? 1535 : codes ? 96 : 31);
   if (codes) return rows >= 1024;
@@ -1724,10 +1726,11 @@ static bool codes_plan(const LinearW& W, const GemvCall& c, size_t rows, int ldx
   return true;
 }
 
-// Float32 rows against a quantised matrix: the tile GEMM, or 32 rows per launch of the streaming kernel?  us of both, fitted to 10 shapes of int4 and int8
-// within 20 %: a launch of the streaming kernel 10 + 0.36 per 2^20 weights (6144 x 4096 19.6, 28672 x 4096 40.6, 32000 x 4096 50); the codes' copy 0.65, a round
-// of workgroups 1.35 per K tile, the slices' reduce.  28672 x 4096 SwiGLU: 256 rows 363 against 325 streaming, 320 rows 405 / 406, 512 rows 425 / 650;
-// 6144 x 4096 96 rows 71 / 59, 160 rows 75 / 98.
+// Float32 rows against a quantised matrix: the tile GEMM, or 32 rows per launch of the streaming kernel?  us of both, fitted to 16 shapes of int4 and int8:
+// a launch of the streaming kernel 11 + 0.30 per 2^20 weights + 0.5 per 1024 columns (6144 x 4096 20, 28672 x 4096 42 int4 and 45 int8, 2048 x 6400 20, 5120 x
+// 17408 54 and 57); the codes' copy 0.65, a round of workgroups 1.35 per K tile, the slices' reduce.  At 40 to 1365 rows of these the choice costs 0.2 % on
+// average over the better side, 12 % at most (28672 x 4096 SwiGLU: codes / streaming 192 rows 352 / 272, 256 rows 357 / 363, 512 rows 414 / 725; 6144 x 4096 96
+// rows 70 / 62, 129 rows 71 / 103; all int8), and int8, which the streaming kernel had at every size, is nowhere slower than there.
 static bool gemm_prefill_pays_codes(const LinearW& W, const GemvCall& c, size_t rows, int terms, size_t splitk_cap) {
   GemmParams p{};
   long blocks = 0;
@@ -1736,7 +1739,7 @@ static bool gemm_prefill_pays_codes(const LinearW& W, const GemvCall& c, size_t 
   const int ncu = gemv_cu_count(), tiles = ((p.ka + p.kb) / BK + p.ksplit - 1) / p.ksplit;
   const double mw = (double)W.N * W.K / (1 << 20), rounds = (double)((blocks * p.ksplit + ncu - 1) / ncu);
   const double reduce = p.ksplit > 1 ? 2e-6 * p.ksplit * rows * W.N : 0.0;
-  return 12.0 + 0.65 * mw + 1.35 * rounds * tiles + reduce < (double)((rows + 31) / 32) * (10.0 + 0.36 * mw);
+  return 12.0 + 0.65 * mw + 1.35 * rounds * tiles + reduce < (double)((rows + 31) / 32) * (11.0 + 0.30 * mw + 0.5 * W.K / 1024);
 }
 
 bool gemm_prefill_on_codes(const LinearW& W, const GemvCall& c, size_t rows) {

@@ -88,7 +88,7 @@ int gemv_pair_grid();
 // prefill (many rows): MFMA tile GEMM + row-wise RMSNorm (gemm_prefill.hip)
 bool gemm_prefill_supported(const LinearW& W, const GemvCall& c, size_t rows);
 // does the tile GEMM beat 32 rows per launch of the streaming kernel?  Logits and layer 0's rounded call on float32 activations only:
-// codes = int4 weights, hilo = the [hi | lo] copy of an f16 matrix
+// codes = int4 weights that run on their [hi | lo] copy (too small for the codes), hilo = the [hi | lo] copy of an f16 matrix
 bool gemm_prefill_pays(bool codes, bool hilo, bool rounded, size_t rows);
 // can this call of split rows leave its SwiGLU as [hi | lo] rows (GemvCall::split_out)?  The 256 x 256 LDS-DMA tile alone does
 bool gemm_prefill_split_out(const LinearW& W, const GemvCall& c, size_t rows);

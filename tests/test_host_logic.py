@@ -375,7 +375,7 @@ def test_decode_attention_splits(f32):
 
 def test_float32_rows_leave_the_streaming_kernel_where_the_tile_pays():
     """Logits and layer 0's rounded call on float32 activations: at decode batches and short prompts the streaming kernel is ahead (int4 logits of
-    64 rows: 2.2 ms against 4.4 on a copy of the matrix), at long ones the tile GEMM."""
+    64 rows: 2.2 ms against 4.4 on a copy of the matrix), at long ones the tile GEMM.  (codes: int4 matrices too small for the codes kernel; the others below)"""
     from mlx_parallm_amd import _lib as L
 
     def pays(rows, codes=0, hilo=0, rounded=0):
@@ -413,6 +413,29 @@ def test_int8_on_float32_rows_is_never_multiplied_as_a_pair():
                 got = _quant_route(rows, N, K, epi=epi, rnd=rnd)
                 assert got in (0, 2) and (got == 0 or 128 < rows), (rows, N, K, epi, rnd, got)
     assert [_quant_route(n, 1024, 1024) for n in (64, 128, 129, 1365)] == [0, 0, 2, 2]
+
+
+def test_prefill_routes_of_quantised_matrices():
+    """Float32 rows leave the streaming kernel where the codes kernel is ahead by both sides' times; 16-bit rows, and float32 rows of int4, take the codes from
+    some 2e9 (K >= 4096) or 4e9 products on and the [hi | lo] copy below; what the kernels refuse stays refused."""
+    def first(rows, *a, **kw):
+        got = [_quant_route(n, *a, **kw) for n in rows]
+        assert got == sorted(got), got                            # (no way back with more rows)
+        return got.index(2)
+
+    rows = list(range(33, 700))
+    for kind in ("q4_bf16", "q8_bf16"):                           # int8: 224 rows 317 us on the streaming kernel, 352 on the codes; 256: 363, 357
+        assert 224 < rows[first(rows, 28672, 4096, kind, epi="SWIGLU")] <= 256
+    assert 96 < rows[first(rows, 6144, 4096, "q4_bf16")] <= 129   # 96 rows 59, 68; 129: 99, 69
+    assert rows[first(rows, 6144, 4096, "q8_bf16")] == 129        # (a decode batch stays on the streaming kernel)
+    assert 96 < rows[first(rows, 32000, 2048, "q4_bf16", epi="STORE_F32")] <= 192      # 129 rows 138, 133
+    for act, q in (("bfloat16", "q4_bf16"), ("float16", "q8_f16")):
+        assert [_quant_route(n, 4096, 4096, q, act) for n in (31, 32, 125, 126, 700)] == [0, 1, 1, 2, 2]
+        assert [_quant_route(n, 2048, 1024, q, act, epi="RESID") for n in (129, 2048, 2051)] == [1, 1, 2]
+    assert [_quant_route(n, 512, 512, "q4_bf16") for n in (64, 300)] == [1, 1]
+    assert _quant_route(8192, 4096, 65536 + 128, "q4_bf16", "bfloat16") == 1           # (more biases of a row tile than 64 KiB)
+    assert _quant_route(300, 4096, 192, "q4_bf16", "bfloat16") == 0 and _quant_route(300, 4096, 4096, "q4_f16", "float32") == 0
+    assert _quant_route(300, 4104, 4096, "q4_bf16", "bfloat16") == 0
 
 
 @pytest.mark.parametrize("f32", [False, True])
