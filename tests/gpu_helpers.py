@@ -100,10 +100,10 @@ def close_frac(got: np.ndarray, want: np.ndarray, dtype: str, atol: float = 0.0)
     return float(np.mean(np.abs(got - want) > tol))
 
 
-def q4_force(mt=0, tw=0, kw=0, ksplit=0, ns=0) -> int:
-    """`ksplit` argument of gemm_skinny() that forces gemm_q4.hip's plan (include/mi355_ops.h): row tiles per workgroup, tile
-    units x K lanes (= compute waves), K slices over workgroups, staging waves; 0 = the cost model's choice."""
-    return -(mt | tw << 3 | kw << 7 | ksplit << 11 | ns << 15)
+def q4_force(mt=0, ksplit=0) -> int:
+    """`ksplit` argument of gemm_skinny() that forces gemm_q4.hip and its plan (include/mi355_ops.h): row tiles per workgroup, K slices over
+    workgroups; 0 = the cost model's choice."""
+    return -(mt | ksplit << 11)
 
 
 def gemm_skinny(ol: L.OpLinear, x, M, act, *, epi=0, out=None, ldo=0, resid=None, pair_offset=0, ksplit=0, iters=0, ldx=None,
