@@ -35,6 +35,11 @@ namespace {
 
 using namespace gemv;
 
+// Five tiles: the most whose accumulators and biases fit 256 registers, and for wide matrices the fewest rounds of workgroups (34816 x 5120 SwiGLU 218
+// workgroups, four tiles 272: two rounds).  Where both fit one round, four are faster, 180 against 224 of 256 CUs at 28672 x 4096: us at 32 / 64 / 128 rows,
+// five and four tiles, 28672 x 4096 26.6 / 34.6 / 63.6 and 24.9 / 30.4 / 54.0, 34816 x 5120 32.5 / 40.6 / 74.2 and 50.1 / 63.2 / 92.9, 151936 x 5120 138 /
+// 174 / 308 and 138 / 183 / 340, 16384 x 4096 22.9 / 30.7 / 35.0 and 21.4 / 27.7 / 31.3, 19200 x 3072 21.2 / 28.5 / 30.4 and 19.9 / 25.5 / 45.7.  A choice
+// per call has not been built.
 constexpr int TN = 5, TW = 2, KW = 4, NW = TW * KW;
 constexpr int W_SLOT = TN * (1024 + 128);                       // codes of five tiles, then their scales | biases (64 + 64 bytes)
 constexpr int Q4_LDS = 160 * 1024;
