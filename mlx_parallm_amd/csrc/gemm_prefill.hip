@@ -959,7 +959,8 @@ __global__ __launch_bounds__(512) void gemm_dma256_kernel(GemmParams p) {
 // Why: the [hi | lo] copy that the dense tile takes doubles the products and the bytes of the copy.  The codes carry no rounding at all;
 // [hi | lo] drops what lies below 2^-17 of a weight.  Around their middle: codes of 0..15 (255) make sums of twice the size and more that
 // the biases take back; the float32 result is then 4.5e-7 from the 64-bit one (6144 x 4096, 1024 rows, 2-norm), here 1.4e-7, [hi | lo] 4.1e-7.
-// The largest last -- x's lo, mid and hi, then the bias columns, their smallest parts first --, so that few roundings are of the size of the result: 1024
+// Float32 rows: the largest last -- x's lo, mid and hi, then the bias columns, their smallest parts first --, so that few roundings are of the size of the
+// result (16-bit rows are rounded to 16 bits behind all of this, and take the biases, largest parts first, in front: recorded greedy sequences have ties there): 1024
 // x 8192, 64 float32 rows, groups of int4 whose means are 0 / 4 / 12 of their deviations, 1.6e-7 / 0.9e-7 / 0.8e-7; the biases and the hi parts in front 1.8e-7 /
 // 2.4e-7 / 2.3e-7; the streaming kernel 9.7e-7 / 2.7e-7 / 1.5e-7.
 // Registers: 128 accumulators + the group's sums.  A phase is two row tiles x both k blocks, so those are 32 (a quarter tile) and not
@@ -990,7 +991,7 @@ __device__ __forceinline__ void dma_dword_off(const void* base, uint32_t off, un
 }
 typedef __attribute__((address_space(3))) f32x4 lds_f32x4_t;
 
-template <typename AT, bool SWIGLU, bool LOGITS = false>
+template <typename AT, bool SWIGLU, bool LOGITS, bool X3>
 __global__ __launch_bounds__(512) void gemm_codes256_kernel(GemmParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem2[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1167,20 +1168,24 @@ __global__ __launch_bounds__(512) void gemm_codes256_kernel(GemmParams p) {
     asm volatile("s_barrier" ::: "memory");
   };
   const uint32_t xrow = (uint32_t)(p.ldx * 2);
-  for (int t0 = 0; t0 < nkm; t0 += p.G) {                          // a run per term of x, the last one (the smallest) first
-    const int lo = max(tb, t0), hi = min(te, t0 + p.G);
-    if (lo >= hi) continue;
-    gs = (const char*)p.sc + (size_t)(lo - t0) * 64;
-    sources((const char*)p.x + (size_t)(nkm - p.G - 2 * t0 + lo) * (BK * 2), xrow, (const char*)p.w + (size_t)(lo - t0) * 2048, (size_t)p.kw * 32);
-    run(hi - lo, std::false_type{});
-  }
-  fold(7);
+  auto groups = [&]() __attribute__((always_inline)) {                    // a run per term of x, the last one (the smallest) first
+    for (int t0 = 0; t0 < nkm; t0 += p.G) {
+      const int lo = max(tb, t0), hi = min(te, t0 + p.G);
+      if (lo >= hi) continue;
+      gs = (const char*)p.sc + (size_t)(lo - t0) * 64;
+      sources((const char*)p.x + (size_t)(nkm - p.G - 2 * t0 + lo) * (BK * 2), xrow, (const char*)p.w + (size_t)(lo - t0) * 2048, (size_t)p.kw * 32);
+      run(hi - lo, std::false_type{});
+    }
+    fold(7);
+  };
+  if constexpr (X3) groups();
   if (te > nkm) {                                                  // the bias columns
     const int lo = max(tb, nkm) - nkm;
     gs = nullptr;
     sources((const char*)p.xs + (size_t)lo * (BK * 2), (uint32_t)(p.kb * 2), (const char*)p.wb + (size_t)lo * 2048, (size_t)p.kb * 32);
     run(te - nkm - lo, std::true_type{});
   }
+  if constexpr (!X3) groups();
 #undef PP_ORDER
 #undef PP_READS_DONE
 #undef PP_MMA_DONE
@@ -1200,7 +1205,7 @@ __global__ __launch_bounds__(512) void gemm_codes256_kernel(GemmParams p) {
 // The group sums of x for the kernel above: row m -> `parts` terms of G columns each (kernels.h: codes16_sum_part; hi + mid + lo = the float32 sum
 // of the group's 64 values over x's `terms` of K columns), zeros up to kb.  One workgroup per row.
 template <typename AT>
-__global__ __launch_bounds__(256) void group_sums_kernel(const AT* x, int ldx, int terms, int K, uint16_t* xs, int kb) {
+__global__ __launch_bounds__(256) void group_sums_kernel(const AT* x, int ldx, int terms, int K, uint16_t* xs, int kb, int big_first) {
   extern __shared__ float gsum[];
   const int row = blockIdx.x, tid = threadIdx.x, G = K / 64;
   const AT* xr = x + (size_t)row * ldx;
@@ -1218,7 +1223,7 @@ __global__ __launch_bounds__(256) void group_sums_kernel(const AT* x, int ldx, i
   __syncthreads();
   for (int c = tid; c < kb; c += 256) {
     const int term = c / G, grp = c - term * G;
-    const float v = term < CODES16_TERMS ? bf16_part(gsum[grp], codes16_sum_part(term)) : 0.f;
+    const float v = term < CODES16_TERMS ? bf16_part(gsum[grp], codes16_sum_part(big_first ? CODES16_TERMS - 1 - term : term)) : 0.f;
     xs[(size_t)row * kb + c] = __builtin_bit_cast(uint16_t, (bf16)v);
   }
 }
@@ -1758,9 +1763,9 @@ int gemm_prefill_quant_route(const LinearW& W, const GemvCall& c, size_t rows) {
   return gemm_prefill_on_codes(W, c, rows) ? 2 : 1;
 }
 
-template <typename AT, bool SWIGLU, bool LOGITS>
+template <typename AT, bool SWIGLU, bool LOGITS, bool X3 = false>
 static int codes_launch(const GemmParams& p, dim3 grid, hipStream_t st) {
-  auto k = gemm_codes256_kernel<AT, SWIGLU, LOGITS>;
+  auto k = gemm_codes256_kernel<AT, SWIGLU, LOGITS, X3>;
   static std::atomic<bool> opted_in[64];                // per device: several engines, and threads, may live in one process
   int dev = 0;
   MI_HIP(hipGetDevice(&dev));
@@ -1783,13 +1788,13 @@ static int launch_gemm_codes(const LinearW& W, const GemvCall& c, size_t rows, h
   if (!codes_plan(W, c, rows, c.ldx, terms, splitk_ws != nullptr, splitk_cap, p, blocks)) return MI_OK;
   p.x = c.x;
   p.ws = (float*)splitk_ws;
-  MI_TRY(launch_codes16(W, scratch, st));
+  MI_TRY(launch_codes16(W, scratch, st, terms == 1));
   char* d = (char*)scratch;
   p.w = d; p.wb = d + (size_t)W.N * W.K * 2; p.sc = (const float*)(d + (size_t)W.N * (W.K + p.kb) * 2);
   uint16_t* xs = (uint16_t*)(d + codes16_bytes(W.N, W.K));
   p.xs = xs;
-  if (c.act == MI_F16) hipLaunchKernelGGL(group_sums_kernel<f16>, dim3((unsigned)rows), dim3(256), p.G * sizeof(float), st, (const f16*)c.x, c.ldx, terms, W.K, xs, p.kb);
-  else hipLaunchKernelGGL(group_sums_kernel<bf16>, dim3((unsigned)rows), dim3(256), p.G * sizeof(float), st, (const bf16*)c.x, c.ldx, terms, W.K, xs, p.kb);
+  if (c.act == MI_F16) hipLaunchKernelGGL(group_sums_kernel<f16>, dim3((unsigned)rows), dim3(256), p.G * sizeof(float), st, (const f16*)c.x, c.ldx, terms, W.K, xs, p.kb, terms == 1);
+  else hipLaunchKernelGGL(group_sums_kernel<bf16>, dim3((unsigned)rows), dim3(256), p.G * sizeof(float), st, (const bf16*)c.x, c.ldx, terms, W.K, xs, p.kb, terms == 1);
   MI_HIP(hipGetLastError());
   p.out32 = x32 || c.out32; p.rnd = x32 ? c.rnd : RND_NONE;
   p.epi = c.epi; p.out = c.out; p.ldo = c.ldo; p.resid = c.resid; p.pair_offset = c.pair_offset; p.glu = c.glu; p.silu_cols = c.silu_cols;
@@ -1800,7 +1805,8 @@ static int launch_gemm_codes(const LinearW& W, const GemvCall& c, size_t rows, h
   p.strips = strips_ok(p);
   const dim3 grid((unsigned)((rows + BM2 - 1) / BM2), (ncols + (sw ? 128 : BN2) - 1) / (sw ? 128 : BN2), p.ksplit);
   const bool rounded = p.rnd != RND_NONE;               // (float32 stores of values rounded to 16 bits: logits, and layer 0 of the float32-cache mode)
-  if (c.act == MI_F16) MI_TRY((sw ? codes_launch<f16, true, false> : rounded ? codes_launch<f16, false, true> : codes_launch<f16, false, false>)(p, grid, st));
+  if (terms > 1 && !rounded) MI_TRY((sw ? codes_launch<bf16, true, false, true> : codes_launch<bf16, false, false, true>)(p, grid, st));
+  else if (c.act == MI_F16) MI_TRY((sw ? codes_launch<f16, true, false> : rounded ? codes_launch<f16, false, true> : codes_launch<f16, false, false>)(p, grid, st));
   else MI_TRY((sw ? codes_launch<bf16, true, false> : rounded ? codes_launch<bf16, false, true> : codes_launch<bf16, false, false>)(p, grid, st));
   if (p.ksplit > 1) MI_TRY(reduce_slices(p, c.act, st));
   *done = true;

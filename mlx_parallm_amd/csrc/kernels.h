@@ -128,8 +128,9 @@ int launch_dequant_q4_hilo(const LinearW& src, void* dst, hipStream_t st);
 // the same matrices as 16-bit codes + biases + scales: the operands of the prefill GEMM on codes; codes16_bias_cols: its columns of group sums
 int codes16_bias_cols(int K);
 size_t codes16_bytes(int N, int K);
-int launch_codes16(const LinearW& src, void* dst, hipStream_t st);
-// term t of that product, the smallest first: part of x's group sum (0 = hi, 1 = mid, 2 = lo) and of the bias; products below 2^-24 of the whole are left out
+int launch_codes16(const LinearW& src, void* dst, hipStream_t st, bool big_first = false);
+// term t of that product, the smallest first: part of x's group sum (0 = hi, 1 = mid, 2 = lo) and of the bias; products below 2^-24 of the whole are left
+// out.  big_first: these terms in reverse
 constexpr int CODES16_TERMS = 6;
 __host__ __device__ constexpr int codes16_sum_part(int t) { return t < 3 ? t & 1 : 5 - t; }
 __host__ __device__ constexpr int codes16_bias_part(int t) { return t < 1 ? 2 : t < 3 ? 1 : 0; }

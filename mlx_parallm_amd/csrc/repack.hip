@@ -142,7 +142,7 @@ __global__ void dequant_q8_hilo_kernel(const uint8_t* src, T* dst, int N, int K)
 // Bound by its writes (2 bytes a code, half of the [hi | lo] copy's).  28672 x 4096: 52 us with the scales and biases, 6.2 TB/s
 // the scales and biases of a row tile; bias: [K/64][16] of LDS
 template <typename T, int BITS>
-__device__ __forceinline__ void codes16_side(const uint8_t* src, uint16_t* wb, float* sc, int K, int kb, size_t tile, float* bias) {
+__device__ __forceinline__ void codes16_side(const uint8_t* src, uint16_t* wb, float* sc, int K, int kb, int big_first, size_t tile, float* bias) {
   constexpr int MID = BITS == 4 ? 8 : 128;
   const int G = K / 64, tid = threadIdx.x;
   for (int o = tid; o < G * 16; o += 256) {
@@ -160,7 +160,7 @@ __device__ __forceinline__ void codes16_side(const uint8_t* src, uint16_t* wb, f
     __bf16 v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      v[e] = term < CODES16_TERMS ? (__bf16)bf16_part(bias[grp * 16 + r], codes16_bias_part(term)) : (__bf16)0.f;
+      v[e] = term < CODES16_TERMS ? (__bf16)bf16_part(bias[grp * 16 + r], codes16_bias_part(big_first ? CODES16_TERMS - 1 - term : term)) : (__bf16)0.f;
       if (++grp == G) { grp = 0; ++term; }
     }
     *(u32x4*)(wb + (tile * kb * 2 + o) * 8) = *(const u32x4*)v;
@@ -170,12 +170,12 @@ __device__ __forceinline__ void codes16_side(const uint8_t* src, uint16_t* wb, f
 // blockIdx.y = row tile; workgroup 0 of a tile its scales and biases, the others a block of 1024 bytes of codes a wave: 16 bytes a lane in, 32 (16) codes
 // out as pieces of 8 k.
 template <typename T, int BITS>
-__global__ __launch_bounds__(256) void codes16_kernel(const uint8_t* src, T* codes, uint16_t* wb, float* sc, int K, int kb) {
+__global__ __launch_bounds__(256) void codes16_kernel(const uint8_t* src, T* codes, uint16_t* wb, float* sc, int K, int kb, int big_first) {
   constexpr int KB = BITS == 4 ? 128 : 64, BYTES = BITS == 4 ? 1152 : 1088, MID = BITS == 4 ? 8 : 128;
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, nb = K / KB;
   const size_t tile = blockIdx.y;
   extern __shared__ float bias[];
-  if (blockIdx.x == 0) { codes16_side<T, BITS>(src, wb, sc, K, kb, tile, bias); return; }
+  if (blockIdx.x == 0) { codes16_side<T, BITS>(src, wb, sc, K, kb, big_first, tile, bias); return; }
   for (int j = (blockIdx.x - 1) * 4 + (threadIdx.x >> 6); j < nb; j += (gridDim.x - 1) * 4) {
     const u32x4 q = *(const u32x4*)(src + (tile * nb + j) * BYTES + lane * 16);
     T* out = codes + tile * 16 * (size_t)K;
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(256) void codes16_kernel(const uint8_t* src, T* cod
 int codes16_bias_cols(int K) { return (CODES16_TERMS * (K / 64) + 63) / 64 * 64; }
 size_t codes16_bytes(int N, int K) { return (size_t)N * ((size_t)K * 2 + (size_t)codes16_bias_cols(K) * 2 + (size_t)(K / 64) * 4); }
 
-int launch_codes16(const LinearW& src, void* dst, hipStream_t st) {
+int launch_codes16(const LinearW& src, void* dst, hipStream_t st, bool big_first) {
   const int bits = wk_bits(src.wk), sdt = wk_scale_dtype(src.wk);
   if (src.layout != 1 || (bits != 4 && bits != 8) || sdt == WK_F32 || src.group != 64 || src.K % (bits == 4 ? 128 : 64) != 0 || src.N % 16 != 0)
     return fail(MI_ERR_UNSUPPORTED, "codes16: tile-major int4 / int8 (group 64) matrices only");
@@ -214,7 +214,7 @@ int launch_codes16(const LinearW& src, void* dst, hipStream_t st) {
   float* sc = (float*)(d + (size_t)src.N * (src.K + kb) * 2);
   const int nb = src.K / (bits == 4 ? 128 : 64), tiles = src.N / 16;
   const dim3 grid(1 + (nb + 7) / 8, tiles);                          // (two blocks a wave)
-#define GO(T, B) hipLaunchKernelGGL((codes16_kernel<T, B>), grid, dim3(256), (size_t)(src.K / 64) * 64, st, (const uint8_t*)src.w, (T*)codes, wb, sc, src.K, kb)
+#define GO(T, B) hipLaunchKernelGGL((codes16_kernel<T, B>), grid, dim3(256), (size_t)(src.K / 64) * 64, st, (const uint8_t*)src.w, (T*)codes, wb, sc, src.K, kb, (int)big_first)
   if (sdt == WK_BF16) { if (bits == 4) GO(bf16, 4); else GO(bf16, 8); }
   else { if (bits == 4) GO(f16, 4); else GO(f16, 8); }
 #undef GO
