@@ -40,7 +40,7 @@ using namespace gemv;
 // five and four tiles, 28672 x 4096 26.6 / 34.6 / 63.6 and 24.9 / 30.4 / 54.0, 34816 x 5120 32.5 / 40.6 / 74.2 and 50.1 / 63.2 / 92.9, 151936 x 5120 138 /
 // 174 / 308 and 138 / 183 / 340, 16384 x 4096 22.9 / 30.7 / 35.0 and 21.4 / 27.7 / 31.3, 19200 x 3072 21.2 / 28.5 / 30.4 and 19.9 / 25.5 / 45.7.  A choice
 // per call has not been built.
-constexpr int TN = 5, TW = 2, KW = 4, NW = TW * KW;
+constexpr int TN = 5, TW = 2, KW = 4, NW = TW * KW, RT = 2;       // (RT: column tiles of a workgroup of q4_rows_kernel)
 constexpr int W_SLOT = TN * (1024 + 128);                       // codes of five tiles, then their scales | biases (64 + 64 bytes)
 constexpr int Q4_LDS = 160 * 1024;
 
@@ -50,6 +50,7 @@ struct Q4Params {
   const void* w;
   int epi; void* out; int ldo; void* resid; int pair_tiles;
   int ntu, ntiles;                                              // column tiles of a half of the matrix (SwiGLU: gate tiles), of all of it
+  int wgs;                                                      // (q4_rows_kernel: without those that only load)
   int nblk, ksplit, nslab, ngroups, nunits;                              // K / 128; units = tile groups x ksplit
   float* ws; unsigned* ctr;
   const float* lora_t; int lora_t_ld;
@@ -487,10 +488,215 @@ __global__ __launch_bounds__(512, 2) void q4_kernel(const Q4Params p) {
   }
 }
 
-struct Q4Plan { int mt, nslab, ksplit, ntu, ntiles, ngroups, nblk; size_t xq_bytes, sx_bytes, sxo_bytes, ws_bytes; };
+// Narrow matrices (q|k|v, o, down: 17..128 rows).  The kernel above cuts their K over workgroups, and the partial tiles' way through memory costs more than
+// the products (7168 x 5120, 64 rows: 9 us behind a loop of 11).  Here a workgroup owns two column tiles (SwiGLU: a gate tile and its up tile) and all of K:
+// wave w takes the blocks of 128 k w, w + 8, ..  Every fragment of x goes to one wave of the workgroup, so it comes from L2 straight into registers (whole KiB
+// of prepared fragments: 70 bytes a clock and CU; the 16 rows of a fragment read from x itself: 17), and the loop has neither LDS nor barriers.  A block's
+// loads go out as the last one's registers come free.  Results return in order, so x brings the codes asked for before it with it: a workgroup keeps no more
+// than a block a wave in flight, and CUs without a unit read the codes ahead into the XCD's L2 (5120 x 5120 in a cold pass 16.5 us without, 14.2).
+// sum x comes from the matrix core (a fragment of -16, or of ones where codes have no offset): it is the C operand of the codes' product and the biases' factor.
+template <typename AT, int MT, bool SWIGLU>
+__global__ __launch_bounds__(512, 2) void q4_rows_kernel(const Q4Params p) {
+  constexpr int T = RT, X_HALF = MT * 1024;
+  constexpr bool OFFS = std::is_same<AT, bf16>::value;          // (f16: the codes are unpacked without an offset)
+  __shared__ f32x4 red[NW * T * MT * 64];
+  const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int bid = blockIdx.x, slab = 0;
+  if (bid >= p.wgs) {                                            // CUs that the units leave idle bring the codes into their XCD's L2, in the order of their use
+    const int xcd = bid & 7, first = p.wgs + ((xcd - p.wgs) & 7), helpers = ((int)gridDim.x - first + 7) >> 3, units = (p.nunits - xcd + 7) >> 3;
+    const int rounds = (p.nblk + NW - 1) / NW, end = p.nblk * 1152;
+    u32x4 any = {0u, 0u, 0u, 0u};
+    for (int i = (bid - first) >> 3; i < rounds * units; i += helpers) {
+      const int rd = i / units, u = (i - rd * units) * 8 + xcd;
+#pragma unroll
+      for (int a = 0; a < T; ++a) {
+        const char* w = (const char*)p.w + (size_t)(SWIGLU ? u + a * p.pair_tiles : min(u * T + a, p.ntiles - 1)) * end;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) any |= *(const u32x4*)(w + min(rd * NW * 1152 + min(j * 8192 + tid * 16, NW * 1152 - 16), end - 16));
+      }
+    }
+    asm volatile("" :: "v"(any));
+    return;
+  }
+  if (p.nslab > 1) {                                            // (slabs of a unit 8 block ids apart, as above)
+    const int per = 8 * p.nslab, blk = bid / per, rem = bid - blk * per;
+    slab = rem >> 3;
+    bid = blk * 8 + (rem & 7);
+  }
+  if (bid >= p.nunits) return;
+  const int unit = __builtin_amdgcn_readfirstlane(bid), row0 = __builtin_amdgcn_readfirstlane(slab) * 16 * MT;
+  const int mine = (p.nblk - wave + NW - 1) / NW;               // (nblk < 8: a wave may have none)
+  auto tile_of = [&](int a) { return SWIGLU ? unit + a * p.pair_tiles : min(unit * T + a, p.ntiles - 1); };
+  const char* gx = (const char*)p.xq + (size_t)__builtin_amdgcn_readfirstlane(slab) * p.G * 2 * X_HALF;
+  const char* gw[T];
+#pragma unroll
+  for (int a = 0; a < T; ++a) gw[a] = (const char*)p.w + (size_t)tile_of(a) * p.nblk * 1152;
+  const uint32_t lane16 = lane * 16, code_off = ((g >> 1) * 16 + c16) * 16 + (g & 1) * 8, sb_off = 1024 + c16 * 4;
+
+  u32x4 x[2][2][MT];                                            // [group][k block][row tile]
+  u32x2 cd[T][2];
+  uint32_t sd[T], bd[T];
+  f32x4 acc[T][MT];
+#pragma unroll
+  for (int a = 0; a < T; ++a)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[a][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  constexpr int LOADS = 4 * T + 4 * MT;                          // of a block: codes, scales, biases, x in the order of its use
+  auto load = [&](int i, int l0, int l1) __attribute__((always_inline)) {
+    const size_t blk = (size_t)(wave + NW * min(i, mine - 1));
+    const char* xb = gx + blk * (4 * X_HALF);
+#pragma unroll
+    for (int l = l0; l < l1; ++l) {
+      const char* w = gw[l % T] + blk * 1152;
+      if (l < 2 * T) cd[l % T][l / T] = *(const u32x2*)(w + l / T * 512 + code_off);
+      else if (l < 3 * T) sd[l % T] = *(const uint32_t*)(w + sb_off);
+      else if (l < 4 * T) bd[l % T] = *(const uint32_t*)(w + sb_off + 64);
+      else {
+        const int j = l - 4 * T, sg = j / (2 * MT), m = j / 2 % MT, t = j & 1;
+        x[sg][t][m] = *(const u32x4*)(xb + (sg * 2 + t) * X_HALF + m * 1024 + lane16);
+      }
+    }
+  };
+  uint32_t mask = 0x00780078u, magic = 0x41804180u;
+  asm("" : "+v"(mask), "+v"(magic));
+  auto unpack = [&](uint32_t q, int c) -> uint32_t {             // unpack_q4, a register at a time
+    if constexpr (OFFS) return (c == 0 ? q << 3 : c == 1 ? q >> 1 : c == 2 ? q >> 5 : q >> 9) & mask | magic;
+    else return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, ((q >> (4 * c)) & 0x000F000Fu) | 0x64006400u) - f16x2{(_Float16)1024.f, (_Float16)1024.f});
+  };
+  const uint32_t one = OFFS ? 0xC180C180u : 0x3C003C00u;         // -16 (bf16), 1 (f16)
+  const u32x4 ones = {one, one, one, one};
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  // block i; the next one's loads go out between its products, a few at a time: in one piece they hold the wave up for what the CU's path takes of all
+  f32x4 d[2][T], sx[2];
+  float sc[2][T], bi[2][T];
+#pragma unroll
+  for (int v = 0; v < 2; ++v) {
+    sx[v] = zero;
+#pragma unroll
+    for (int a = 0; a < T; ++a) { d[v][a] = zero; sc[v][a] = bi[v][a] = 0.f; }
+  }
+  auto fold = [&](int v, int m, int sv) {
+#pragma unroll
+    for (int a = 0; a < T; ++a)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[a][m][r] = fmaf(bi[sv][a], sx[v][r], fmaf(sc[sv][a], d[v][a][r], acc[a][m][r]));
+  };
+  auto mult = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+    for (int sg = 0; sg < 2; ++sg) {
+      u32x4 w[T][2];
+#pragma unroll
+      for (int a = 0; a < T; ++a) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) { w[a][0][c] = unpack(cd[a][sg].x, c); w[a][1][c] = unpack(cd[a][sg].y, c); }
+      }
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const int j = sg * MT + m, v = j & 1;
+        __builtin_amdgcn_sched_barrier(0);
+        sx[v] = mfma16<AT>(x[sg][0][m], ones, zero);
+        sx[v] = mfma16<AT>(x[sg][1][m], ones, sx[v]);
+#pragma unroll
+        for (int a = 0; a < T; ++a) d[v][a] = mfma16<AT>(x[sg][0][m], w[a][0], OFFS ? sx[v] : zero);
+#pragma unroll
+        for (int a = 0; a < T; ++a) d[v][a] = mfma16<AT>(x[sg][1][m], w[a][1], d[v][a]);
+        fold(v ^ 1, (m + MT - 1) % MT, j == 0 ? 1 : m == 0 ? 0 : sg);
+        if (j == 0) {
+#pragma unroll
+          for (int a = 0; a < T; ++a)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              if constexpr (OFFS) {
+                sc[u][a] = __uint_as_float(u ? sd[a] & 0xffff0000u : sd[a] << 16);
+                bi[u][a] = __uint_as_float(u ? bd[a] & 0xffff0000u : bd[a] << 16) * -0.0625f;
+              } else {
+                sc[u][a] = (float)__builtin_bit_cast(f16, (unsigned short)(sd[a] >> (16 * u)));
+                bi[u][a] = (float)__builtin_bit_cast(f16, (unsigned short)(bd[a] >> (16 * u)));
+              }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // what this row tile leaves free takes the next block's
+        if (m == 0) load(i + 1, T * sg, T * sg + T);
+        if (j == 0) load(i + 1, 2 * T, 4 * T);
+        load(i + 1, 4 * T + 2 * j, 4 * T + 2 * j + 2);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (mine > 0) {
+    load(0, 0, LOADS);
+    for (int i = 0; i < mine; ++i) mult(i);
+    fold((2 * MT - 1) & 1, MT - 1, 1);
+  }
+
+#pragma unroll
+  for (int a = 0; a < T; ++a)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) red[((wave * T + a) * MT + m) * 64 + lane] = acc[a][m];
+  // a wave's output tile (SwiGLU: pair): lane (c16, g) finishes rows 4 g .. 4 g + 3, column c16
+  const int a_out = SWIGLU ? 0 : wave / MT, m_out = SWIGLU ? wave : wave % MT;
+  const bool live = (SWIGLU ? wave < MT : wave < T * MT && unit * T + a_out < p.ntiles);
+  const int n = tile_of(a_out) * 16 + c16, r0 = row0 + m_out * 16 + g * 4;
+  float hres[4] = {0.f, 0.f, 0.f, 0.f};
+  if (!SWIGLU && live && p.epi == EPI_RESID) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) hres[r] = (float)((const AT*)p.resid)[(size_t)min(r0 + r, p.M - 1) * p.ldo + n];
+  }
+  __syncthreads();
+  if (!live) return;
+  f32x4 y[SWIGLU ? 2 : 1];
+#pragma unroll
+  for (int v = 0; v < (SWIGLU ? 2 : 1); ++v) {
+    const f32x4* src = red + ((a_out + v) * MT + m_out) * 64 + lane;
+    y[v] = src[0];
+#pragma unroll
+    for (int k = 1; k < NW; ++k) y[v] += src[k * T * MT * 64];
+  }
+  AT* out = (AT*)p.out;
+#pragma unroll 1
+  for (int r = 0; r < 4; ++r) {                                  // (rolled: its branches stand once)
+    const int row = r0 + r;
+    if (row >= p.M) break;
+    const float v = r == 0 ? y[0].x : r == 1 ? y[0].y : r == 2 ? y[0].z : y[0].w;
+    if constexpr (SWIGLU) {
+      const float up = r == 0 ? y[1].x : r == 1 ? y[1].y : r == 2 ? y[1].z : y[1].w;
+      out[(size_t)row * p.ldo + n] = silu16<AT>(v, up);
+    } else {
+      float z = (float)(AT)v;
+      if (p.lora_t != nullptr) {
+        for (int sl = 0; sl < 2; ++sl) {
+          const int l0 = sl ? p.lora_row0_1 : p.lora_row0_0, ln = sl ? p.lora_n_1 : p.lora_n_0, rk = sl ? p.lora_rank_1 : p.lora_rank_0;
+          const float* lb = sl ? p.lora_b1 : p.lora_b0;
+          if (lb != nullptr && n >= l0 && n < l0 + ln) {
+            const float t = (sl ? p.lora_scale_1 : p.lora_scale_0) * lora_dot(p.lora_t + (size_t)row * p.lora_t_ld + sl * (p.lora_t_ld / 2), lb + (n - l0), ln, rk);
+            z = (float)(AT)(z + (float)(AT)t);
+          }
+        }
+      }
+      if (p.epi == EPI_STORE) out[(size_t)row * p.ldo + n] = (AT)z;
+      else if (p.epi == EPI_STORE_F32) ((float*)p.out)[(size_t)row * p.ldo + n] = z;
+      else ((AT*)p.resid)[(size_t)row * p.ldo + n] = (AT)((r == 0 ? hres[0] : r == 1 ? hres[1] : r == 2 ? hres[2] : hres[3]) + z);
+    }
+  }
+}
+
+struct Q4Plan { bool rows; int mt, nslab, ksplit, ntu, ntiles, ngroups, nblk; size_t xq_bytes, sx_bytes, sxo_bytes, ws_bytes; };
 
 thread_local int q4_force_mt = 0, q4_force_ks = 0;               // test hook: row tiles per workgroup, K slices (0: the plan's own)
+thread_local int q4_force_rows = 0;
 thread_local bool q4_forced = false;                             // .. and whatever the width
+
+// Narrow matrices: q4_rows_kernel or gemm_skinny.hip?  us, both with their preparation but without the norm launch of 4.7 that q4_prep_kernel saves, warm weights,
+// here / there at 32, 64 and 128 rows: 7168 x 5120 14 / 16, 17 / 23, 31 / 30; 5120 x 5120 15 / 17, 17 / 22, 31 / 28; 4096 x 4096 13 / 15, 15 / 21, 16 / 23; 2048 x 6400 16 / 17,
+// 19 / 23, 20 / 24; 3072 x 1024 8 / 9, 9 / 10, 9 / 13; SwiGLU 6400 x 2048 10 / 16, 11 / 25, 17 / 23.  A longer K: 4096 x 14336 26 / 23, 41 / 33, 43 / 45; 5120 x 17408 32 / 28, 50 / 40, 87 /
+// 62.  So: K up to 8192, and one round of workgroups, or two where a norm launch goes with the other kernel.
+bool q4_rows_ahead(const LinearW& W, const GemvCall& c, size_t rows) {
+  const long units = c.epi == EPI_SWIGLU ? c.pair_offset / 16 : (W.N / 16 + RT - 1) / RT, slabs = (long)((rows + 63) / 64);
+  return W.K <= 8192 && (c.pro == PRO_NORM || c.epi == EPI_SWIGLU || units * slabs <= gemv_cu_count());
+}
+bool q4_rows(const LinearW& W, const GemvCall& c) { return q4_force_rows > 0 || (!q4_forced && W.N / 16 < GEMM_Q4_MIN_TILES); }
 
 Q4Plan q4_plan(const LinearW& W, const GemvCall& c, size_t rows) {
   Q4Plan pl{};
@@ -503,9 +709,11 @@ Q4Plan q4_plan(const LinearW& W, const GemvCall& c, size_t rows) {
   pl.nslab = (tiles + 3) / 4;
   pl.mt = std::max(2, (tiles + pl.nslab - 1) / pl.nslab);
   if (q4_force_mt > 0) { pl.mt = std::min(4, std::max(2, q4_force_mt)); pl.nslab = (tiles + pl.mt - 1) / pl.mt; }
+  pl.rows = q4_rows(W, c);
   const double cus = gemv_cu_count(), step = 0.35 + 0.2 * pl.mt;
   double best = 1e30;
-  for (int ks = 1; ks <= 8 && ks <= pl.nblk; ++ks) {
+  if (pl.rows) { pl.ksplit = 1; pl.ngroups = sw ? pl.ntu : (pl.ntiles + RT - 1) / RT; }
+  else for (int ks = 1; ks <= 8 && ks <= pl.nblk; ++ks) {
     const double rounds = std::ceil(pl.ngroups * pl.nslab * ks / cus), iters = ((pl.nblk + ks - 1) / ks + KW - 1) / KW;
     double t = rounds * (2.0 * iters * step + 5.0);
     if (ks > 1) t += 2.0 + 2.0 * ks * (double)pl.ngroups * TW * TN * pl.nslab * pl.mt * 1024 / 4.0e6;
@@ -544,22 +752,35 @@ int q4_launch_at(const Q4Params& p, int mt, bool sw, int grid, hipStream_t st) {
   return fail(MI_ERR_INVALID, "gemm_q4: 2..4 row tiles per workgroup");
 }
 
+template <typename AT>
+int q4_rows_launch(const Q4Params& p, int mt, bool sw, int grid, hipStream_t st) {
+  switch (mt) {
+#define RK(MT) case MT: if (sw) hipLaunchKernelGGL((q4_rows_kernel<AT, MT, true>), dim3(grid), dim3(NW * 64), 0, st, p); \
+                        else hipLaunchKernelGGL((q4_rows_kernel<AT, MT, false>), dim3(grid), dim3(NW * 64), 0, st, p); break;
+    RK(2) RK(3) RK(4)
+#undef RK
+    default: return fail(MI_ERR_INVALID, "gemm_q4: 2..4 row tiles per workgroup");
+  }
+  MI_HIP(hipGetLastError());
+  return MI_OK;
+}
+
 }  // namespace
 
-// test hook: row tiles | .. << 3 | .. << 7 | K slices << 11 (the fields between are this kernel's fixed shape); 0 clears
-void gemm_q4_force(int code) { q4_force_mt = code & 7; q4_force_ks = (code >> 11) & 15; q4_forced = code != 0; }
+// test hook: row tiles | .. << 3 | .. << 7 | K slices << 11 (the fields between are q4_kernel's fixed shape) | q4_rows_kernel << 15; 0 clears
+void gemm_q4_force(int code) { q4_force_mt = code & 7; q4_force_ks = (code >> 11) & 15; q4_force_rows = (code >> 15) & 1; q4_forced = code != 0; }
 
-// The wide matrices.  us, 64 rows (32 rows), against gemm_skinny.hip's K over workgroups; with the preparation pass, which replaces a norm launch of
+// The wide matrices, and the narrow ones of q4_rows_ahead.  Wide: us, 64 rows (32 rows), against gemm_skinny.hip's K over workgroups; with the preparation pass, which replaces a norm launch of
 // 4.7 us in front of gate|up and the logits: 34816 x 5120 SwiGLU 42 (31) against 71 (40), 28672 x 4096 33 (25) against 40 (25), 151936 x 5120
-// 172 (131) against 272 (149), 20480 x 5120 37 (27) against 42 (26).  A workgroup's head and tail are some 10 us, slices of K another 8: 7168 x 5120
-// 30 (21) against 23 (16), 5120 x 17408 42 (31) against 37 (26); few rows on short K: 50304 x 2048 45 (34) against 40 (22).
+// 172 (131) against 272 (149), 20480 x 5120 37 (27) against 42 (26).  A workgroup's head and tail are some 10 us, slices of K another 8: 5120 x 17408
+// 42 (31) against 37 (26); few rows on short K: 50304 x 2048 45 (34) against 40 (22).
 bool gemm_q4_supported(const LinearW& W, const GemvCall& c, size_t rows) {
   if (c.force_v1 || W.layout != 1 || c.rnd != RND_NONE || c.out32) return false;
   const bool q4 = ((W.wk == WK_Q4_BF16 && c.act == MI_BF16) || (W.wk == WK_Q4_F16 && c.act == MI_F16)) && W.group == 64 && W.K % 128 == 0;
   if (!q4 || rows < 17 || rows > 128 || c.ldx % 8 != 0) return false;
   if (c.epi == EPI_SWIGLU_GU8 || c.glu.kind != GLU_SILU || c.silu_cols > 0) return false;
   if (W.N % 16 != 0 || (c.epi == EPI_SWIGLU && c.pair_offset % 16 != 0)) return false;
-  if (!q4_forced && (W.N / 16 < GEMM_Q4_MIN_TILES || (rows <= 32 && W.K < 3072))) return false;
+  if (!q4_forced && (W.N / 16 < GEMM_Q4_MIN_TILES ? !q4_rows_ahead(W, c, rows) : (rows <= 32 && W.K < 3072))) return false;
   return (size_t)(W.N / 16) * (W.K / 128) * 1152 < ((size_t)1 << 32);          // (32-bit offsets of the LDS-DMA sources)
 }
 
@@ -593,6 +814,11 @@ int launch_gemm_q4(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t
   p.lora_b0 = W.lora_b[0]; p.lora_b1 = W.lora_b[1];
   p.lora_row0_0 = W.lora_row0[0]; p.lora_n_0 = W.lora_n[0]; p.lora_rank_0 = W.lora_rank[0]; p.lora_scale_0 = W.lora_scale[0];
   p.lora_row0_1 = W.lora_row0[1]; p.lora_n_1 = W.lora_n[1]; p.lora_rank_1 = W.lora_rank[1]; p.lora_scale_1 = W.lora_scale[1];
+  if (pl.rows) {
+    p.wgs = pl.nslab > 1 ? (p.nunits + 7) / 8 * 8 * pl.nslab : p.nunits;
+    const int grid = std::max(p.wgs, gemv_cu_count());
+    return c.act == MI_BF16 ? q4_rows_launch<bf16>(p, pl.mt, c.epi == EPI_SWIGLU, grid, st) : q4_rows_launch<f16>(p, pl.mt, c.epi == EPI_SWIGLU, grid, st);
+  }
   const int blocks = pl.nslab > 1 ? (p.nunits + 7) / 8 * 8 * pl.nslab : p.nunits;
   return c.act == MI_BF16 ? q4_launch_at<bf16>(p, pl.mt, c.epi == EPI_SWIGLU, blocks, st) : q4_launch_at<f16>(p, pl.mt, c.epi == EPI_SWIGLU, blocks, st);
 }

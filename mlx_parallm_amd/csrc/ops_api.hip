@@ -98,6 +98,9 @@ int mi_op_gemm_skinny(const mi_op_linear* w, const mi_op_gemv_args* a, int kspli
   }
   if (!gemm_skinny_supported(W, c, (size_t)c.M) && !gemm_q4_supported(W, c, (size_t)c.M))
     return fail(MI_ERR_UNSUPPORTED, "mi_op_gemm_skinny: call not supported by this kernel");
+  // (a norm in front of a narrow int4 matrix: the engine's calls alone)
+  if (c.pro == PRO_NORM && c.act != MI_F32 && wk_is_quant(W.wk) && ksplit == 0 && !wide_norm)
+    return fail(MI_ERR_INVALID, "mi_op_gemm_skinny: normalise the activations first");
   const int groups = std::max(1, gemm_skinny_groups(W, c, (size_t)c.M));
   void* ws = nullptr; unsigned* ctr = nullptr;
   // 16 slices x N x 128 rows x 4 B: any ksplit of gemm_skinny; gemm_q4: its preparation buffers + partial tiles

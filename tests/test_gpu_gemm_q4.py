@@ -55,3 +55,42 @@ def test_every_forced_plan_and_every_norm_in_front_of_a_wide_matrix_is_taken():
         gemm_skinny(ol, xd, M, act, epi=L.EPI_STORE, out=out, ldo=208, ksplit=-code)
         assert np.all(host(out)[M:] == 7.0)
         _assert_close(host(out)[:M], want, act)
+
+
+@pytest.mark.parametrize("act", ["bfloat16", "float16"])
+@pytest.mark.parametrize("M,N,K,epi", [
+    (17, 48, 128, "store"),          # one block of K: seven waves without one; an odd number of column tiles
+    (33, 176, 128 * 9, "resid"),     # three row tiles; one wave with two blocks
+    (64, 4112, 128 * 17, "f32"),     # 129 units (the other CUs read ahead), blocks that differ by wave
+    (100, 96, 128 * 5, "norm"),      # two slabs
+    (128, 8224, 128 * 2, "store"),   # two slabs, more workgroups than CUs
+    (40, 2 * 80, 128 * 8, "swiglu"),
+    (97, 2 * 48, 128 * 7, "swiglu"),
+])
+def test_narrow_matrices(act, M, N, K, epi):
+    """q4_rows_kernel: partial waves, units, slabs and row tiles, every epilogue and the norm in front."""
+    rng = np.random.default_rng(K + M)
+    ol, w, keep = _weight(4, act, N, K, rng)
+    x = round_to(rng.standard_normal((M, K)).astype(np.float32), act)
+    h = round_to(rng.standard_normal((M, N)).astype(np.float32), act)
+    nw = round_to(1.0 + 0.1 * rng.standard_normal(K).astype(np.float32), act)
+    xd, nwd = dev(x, act), dev(nw, act)
+    y = matmul_nt(ref_model.rms_norm(x, act, nw, act, 1e-5)[0] if epi == "norm" else x, w)
+    cols = N // 2 if epi == "swiglu" else N
+    outs = []
+    for _ in range(2):
+        out = torch.full((M + 2, cols), 7.0, dtype=torch.float32 if epi == "f32" else xd.dtype, device="cuda")
+        if epi == "resid":
+            out[:M] = dev(h, act)
+        kw = {"store": {}, "resid": dict(resid=out), "f32": {}, "norm": dict(norm_w=nwd, eps=1e-5), "swiglu": dict(pair_offset=N // 2)}[epi]
+        code = {"resid": L.EPI_RESID, "f32": L.EPI_STORE_F32, "swiglu": L.EPI_SWIGLU}.get(epi, L.EPI_STORE)
+        gemm_skinny(ol, xd, M, act, epi=code, out=out, ldo=cols, ksplit=q4_force(rows=1), **kw)
+        outs.append(host(out))
+    assert np.array_equal(outs[0], outs[1]) and np.all(outs[0][M:] == 7.0)
+    want = round_to(y, act)
+    if epi == "resid":
+        want = round_to(h + want, act)
+    if epi == "swiglu":
+        g, u = want[:, :cols], want[:, cols:]
+        want = round_to(round_to(g * round_to(1.0 / (1.0 + np.exp(-g.astype(np.float64))), act), act) * u, act)
+    _assert_close(outs[0][:M], want, act)
