@@ -408,89 +408,98 @@ __global__ __launch_bounds__(NTHR) void gemv_short_kernel(GemvParams p) {
 }
 
 // t[m][slot][j] = round(sum_k xin[m][k] * A[k][j]); xin = (normed) x, same prologue as above.
-template <typename AT>
-__global__ __launch_bounds__(NTHR) void lora_down_kernel(GemvParams p, const float* a0, const float* a1,
-                                                          float* t, int t_ld) {
-  __shared__ float rs_sh;
-  __shared__ float red[4];
+// What bounds it is round trips to L2, so a workgroup is 8 waves and takes 2048 k at a time with all loads in flight; four lanes read a row of A (16 ranks), a
+// wave one KiB -- a lane that reads whole rows, 64 bytes apart, costs the CU's path four times the cycles.  x goes through LDS, normalised once.
+// 64 rows x 5120 at rank 16, both slots: 23.5 us (four waves, a row of A per lane) -> 11.8.
+constexpr int LD_NTHR = 512, LD_KC = 2048;
+// VEC: ranks in fours.  (NORM and VEC are forms: asked inside, they make a branch of every load)
+template <typename AT, bool NORM, bool VEC>
+__global__ __launch_bounds__(LD_NTHR) void lora_down_kernel(GemvParams p, const float* a0, const float* a1,
+                                                            float* t, int t_ld) {
+  constexpr int NW = LD_NTHR / 64, ROWS = LD_NTHR / 4, U = LD_KC / ROWS, XU = LD_KC / LD_NTHR;
+  __shared__ float red[NW], red16[NW][16], xs[LD_KC];
   const int m = blockIdx.x, slot = blockIdx.y;
   const float* A = slot ? a1 : a0;
   const int rk = slot ? p.lora_rank_1 : p.lora_rank_0;
   if (A == nullptr) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = tid & 3;
   const AT* x = (const AT*)p.x + (size_t)m * p.ldx;
-  if (p.pro == PRO_NORM) {
+  float rs = 1.0f;
+  if constexpr (NORM) {
     float ss = 0.f;
-    for (int k = tid; k < p.K; k += NTHR) { float v = to_f32(x[k]); ss += v * v; }
+    for (int k0 = tid; k0 < p.K; k0 += 8 * LD_NTHR) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = to_f32(x[min(k0 + u * LD_NTHR, p.K - 1)]);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) ss = k0 + u * LD_NTHR < p.K ? fmaf(v[u], v[u], ss) : ss;
+    }
     ss = wave_sum(ss);
     if (lane == 0) red[wave] = ss;
     __syncthreads();
-    if (tid == 0) rs_sh = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)p.K + p.eps);
-    __syncthreads();
+    ss = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) ss += red[w];
+    rs = 1.0f / sqrtf(ss / (float)p.K + p.eps);
   }
-  // 16 columns of A at a time: one pass over x per 16 ranks instead of one per rank (the per-thread order of the
-  // k sum, the wave reduction and the order of the four wave partials are those of a single-column pass, so t is
-  // unchanged bit for bit)
-  __shared__ float red16[4][16];
   for (int j0 = 0; j0 < rk; j0 += 16) {
-    float s[16];
+    const int jq = j0 + 4 * q;
+    float s[4][4];                                               // four chains per column
 #pragma unroll
-    for (int j = 0; j < 16; ++j) s[j] = 0.f;
-    // four k per trip with all their loads issued before the first fma (a thread's 20 k at K = 5120 were 20
-    // dependent L2 round trips: 37 us per launch); the fma order per column is still k ascending
-    const bool vec = (rk % 4 == 0) && (j0 + 16 <= rk);
-    for (int k0 = tid; k0 < p.K; k0 += 4 * NTHR) {
-      float v[4], nw[4];
-      float4 a4[4][4];
-      float a1[4][16];
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int k = k0 + u * NTHR, kc = k < p.K ? k : tid;
-        v[u] = to_f32(x[kc]);
-        nw[u] = p.pro == PRO_NORM ? to_f32(((const AT*)p.norm_w)[kc]) : 1.0f;
-        const float* ar = A + (size_t)kc * rk + j0;
-        if (vec) {
+      for (int j = 0; j < 4; ++j) s[u][j] = 0.f;
+    for (int c0 = 0; c0 < p.K; c0 += LD_KC) {
+      const int n = min(LD_KC, p.K - c0);
+      float4 a4[U];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) a4[u][q] = ((const float4*)ar)[q];
-        } else {
-#pragma unroll
-          for (int j = 0; j < 16; ++j) a1[u][j] = ar[j0 + j < rk ? j : 0];
-        }
+      for (int u = 0; u < U; ++u) {
+        const float* ar = A + (size_t)(c0 + min((tid >> 2) + u * ROWS, n - 1)) * rk;
+        if constexpr (VEC) a4[u] = *(const float4*)(ar + (jq < rk ? jq : 0));
+        else a4[u] = {ar[min(jq, rk - 1)], ar[min(jq + 1, rk - 1)], ar[min(jq + 2, rk - 1)], ar[min(jq + 3, rk - 1)]};
       }
+      float v[XU], nw[XU];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int k = k0 + u * NTHR;
-        if (k >= p.K) break;
-        float vv = v[u];
-        if (p.pro == PRO_NORM) {
-          AT xn = store_act<AT>(vv * rs_sh, p.rnd);
-          vv = to_f32(store_act<AT>(to_f32(xn) * nw[u], p.rnd));
+      for (int u = 0; u < XU; ++u) {
+        const int k = c0 + min(tid + u * LD_NTHR, n - 1);
+        v[u] = to_f32(x[k]);
+        nw[u] = NORM ? to_f32(((const AT*)p.norm_w)[k]) : 1.0f;
+      }
+      __syncthreads();                                           // (the last chunk has been read)
+#pragma unroll
+      for (int u = 0; u < XU; ++u) {
+        if constexpr (NORM) {
+          const AT xn = store_act<AT>(v[u] * rs, p.rnd);
+          v[u] = to_f32(store_act<AT>(to_f32(xn) * nw[u], p.rnd));
         }
-        if (vec) {
+        xs[tid + u * LD_NTHR] = tid + u * LD_NTHR < n ? v[u] : 0.f;
+      }
+      __syncthreads();
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            s[4 * q + 0] = fmaf(vv, a4[u][q].x, s[4 * q + 0]);
-            s[4 * q + 1] = fmaf(vv, a4[u][q].y, s[4 * q + 1]);
-            s[4 * q + 2] = fmaf(vv, a4[u][q].z, s[4 * q + 2]);
-            s[4 * q + 3] = fmaf(vv, a4[u][q].w, s[4 * q + 3]);
-          }
-        } else {
-#pragma unroll
-          for (int j = 0; j < 16; ++j)
-            if (j0 + j < rk) s[j] = fmaf(vv, a1[u][j], s[j]);
-        }
+      for (int u = 0; u < U; ++u) {
+        const int i = (tid >> 2) + u * ROWS;
+        const bool on = i < n;                                   // (xs is zero there, but A may be infinite)
+        const float xv = xs[i];
+        s[u & 3][0] = fmaf(xv, on ? a4[u].x : 0.f, s[u & 3][0]);
+        s[u & 3][1] = fmaf(xv, on ? a4[u].y : 0.f, s[u & 3][1]);
+        s[u & 3][2] = fmaf(xv, on ? a4[u].z : 0.f, s[u & 3][2]);
+        s[u & 3][3] = fmaf(xv, on ? a4[u].w : 0.f, s[u & 3][3]);
       }
     }
-    __syncthreads();
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const float w = wave_sum(s[j]);
-      if (lane == 0) red16[wave][j] = w;
+    for (int j = 0; j < 4; ++j) {                                // (columns past the rank: of others, never stored)
+      float w = (s[0][j] + s[1][j]) + (s[2][j] + s[3][j]);
+#pragma unroll
+      for (int o = 4; o < 64; o <<= 1) w += __shfl_xor(w, o, 64);
+      if (lane < 4) red16[wave][4 * q + j] = w;
     }
     __syncthreads();
-    if (tid < 16 && j0 + tid < rk)
-      t[(size_t)m * t_ld + slot * (t_ld / 2) + j0 + tid] =
-          round_rt(red16[0][tid] + red16[1][tid] + red16[2][tid] + red16[3][tid], p.lora_rnd);
+    if (tid < 16 && j0 + tid < rk) {
+      float w = 0.f;
+#pragma unroll
+      for (int i = 0; i < NW; ++i) w += red16[i][tid];
+      t[(size_t)m * t_ld + slot * (t_ld / 2) + j0 + tid] = round_rt(w, p.lora_rnd);
+    }
   }
 }
 
@@ -615,13 +624,22 @@ int launch_gemv_v1(const LinearW& W, const GemvCall& c, hipStream_t st) {
   return fail(MI_ERR_INVALID, "gemv: bad activation dtype");
 }
 
+template <typename AT>
+static void lora_down_at(const GemvParams& p, const LinearW& W, float* t, int t_ld, hipStream_t st) {
+  const dim3 grid(p.M, 2), block(LD_NTHR);
+  const bool vec = (W.lora_rank[0] | W.lora_rank[1]) % 4 == 0;
+#define LD_GO(N, V) hipLaunchKernelGGL((lora_down_kernel<AT, N, V>), grid, block, 0, st, p, W.lora_a[0], W.lora_a[1], t, t_ld)
+  if (p.pro == PRO_NORM) { if (vec) LD_GO(true, true); else LD_GO(true, false); }
+  else { if (vec) LD_GO(false, true); else LD_GO(false, false); }
+#undef LD_GO
+}
+
 int launch_lora_down(const LinearW& W, const GemvCall& c, float* t, int t_ld, hipStream_t st) {
-  GemvParams p = make_params(W, c);
-  dim3 grid(c.M, 2);
+  const GemvParams p = make_params(W, c);
   switch (c.act) {
-    case MI_F32: hipLaunchKernelGGL(lora_down_kernel<float>, grid, dim3(NTHR), 0, st, p, W.lora_a[0], W.lora_a[1], t, t_ld); break;
-    case MI_BF16: hipLaunchKernelGGL(lora_down_kernel<bf16>, grid, dim3(NTHR), 0, st, p, W.lora_a[0], W.lora_a[1], t, t_ld); break;
-    case MI_F16: hipLaunchKernelGGL(lora_down_kernel<f16>, grid, dim3(NTHR), 0, st, p, W.lora_a[0], W.lora_a[1], t, t_ld); break;
+    case MI_F32: lora_down_at<float>(p, W, t, t_ld, st); break;
+    case MI_BF16: lora_down_at<bf16>(p, W, t, t_ld, st); break;
+    case MI_F16: lora_down_at<f16>(p, W, t, t_ld, st); break;
     default: return fail(MI_ERR_INVALID, "lora_down: bad activation dtype");
   }
   MI_HIP(hipGetLastError());

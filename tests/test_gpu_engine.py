@@ -725,6 +725,46 @@ def test_a_chunk_s_bits_do_not_depend_on_its_neighbours_caches(tiny_dirs, kvd):
     eng.close()
 
 
+@pytest.mark.parametrize("hidden,rank", [(256, 3), (256, 18), (256, 64), (2304, 16)])       # rows of A that are no fours; several 16-rank passes; a second chunk of K
+def test_lora_ranks_and_widths(hidden, rank):
+    """lora_down_kernel against the same engine with the adapter merged (in float64) into the layer's values."""
+    import torch
+
+    from mlx_parallm_amd.engine import Engine
+
+    heads, hd, V, ff, L_ = hidden // 64, 64, 256, 256, 1
+    cfg = dict(model_type="llama", hidden_size=hidden, num_hidden_layers=L_, num_attention_heads=heads, num_key_value_heads=heads, head_dim=hd, intermediate_size=ff,
+               vocab_size=V, rms_norm_eps=1e-5, rope_theta=10000.0, tie_word_embeddings=False, max_position_embeddings=64)
+    rng = np.random.default_rng(hidden + rank)
+    w = lambda *s: torch.from_numpy((rng.standard_normal(s) / np.sqrt(s[-1])).astype(np.float32)).cuda()
+    t = {"model.embed_tokens.weight": w(V, hidden) * hidden ** 0.5, "lm_head.weight": w(V, hidden), "model.norm.weight": torch.ones(hidden).cuda()}
+    p = "model.layers.0."
+    for n, s in (("self_attn.q_proj", (hidden, hidden)), ("self_attn.k_proj", (hidden, hidden)), ("self_attn.v_proj", (hidden, hidden)), ("self_attn.o_proj", (hidden, hidden)),
+                 ("mlp.gate_proj", (ff, hidden)), ("mlp.up_proj", (ff, hidden)), ("mlp.down_proj", (hidden, ff))):
+        t[p + n + ".weight"] = w(*s)
+    t[p + "input_layernorm.weight"] = t[p + "post_attention_layernorm.weight"] = torch.ones(hidden).cuda()
+    a = torch.from_numpy((rng.uniform(-1, 1, (hidden, rank)) / np.sqrt(hidden)).astype(np.float32)).cuda()
+    b = torch.from_numpy(rng.standard_normal((rank, hidden)).astype(np.float32)).cuda()
+    toks = rng.integers(0, V, (3, 4)).astype(np.int32)
+
+    def logits(tensors, adapter):
+        e = Engine(cfg, device=0, max_positions=64, act_dtype="float32")
+        for n, x in tensors.items():
+            e.set_tensor(n, x)
+        e.finalize()
+        if adapter:
+            e.set_lora(0, "self_attn.v_proj", a, b, 2.0)
+        out = e.forward(toks, e.new_kv(3, capacity=8, kv_dtype="float32"))
+        e.close()
+        return out
+    merged = dict(t)
+    merged[p + "self_attn.v_proj.weight"] = (t[p + "self_attn.v_proj.weight"].double() + 2.0 * (a.double() @ b.double()).T).float()
+    got, want, plain = logits(t, True), logits(merged, False), logits(t, False)
+    assert np.abs(want - plain).max() > 0.1
+    # float32 throughout: the merged matrix is rounded once (2^-24 of its elements), the sums have at most K = 2304 terms
+    assert np.abs(got - want).max() <= 2304 ** 0.5 * 2.0 ** -24 * 8 * np.abs(want).max(), np.abs(got - want).max()
+
+
 def test_converted_checkpoint_and_lora_hot_swap(tiny_dirs, tmp_path):
     """a directory written by convert(quantize=True) loads and matches the oracle on the same
     files; weight_updater swaps adapters on the live engine (adapters.safetensors + config, then adapter.npz)."""
