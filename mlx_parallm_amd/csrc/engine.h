@@ -27,6 +27,7 @@ struct FusedLinear {
   // copy is marked unavailable and the linear keeps its plain path -- ensure_hilo / ensure_gu8)
   void* w_hilo = nullptr;        // f16 dense weights in the float32-activation (PagedKVCache) mode: [hi | lo] bf16 copy
   void* w_gu8 = nullptr;         // dense 16-bit gate|up: row-interleaved copy for the decode GEMV (EPI_SWIGLU_GU8)
+  void* w_codes = nullptr;       // quantised weights: 16-bit codes for the prefill GEMM (W.codes)
   bool hilo_failed = false, gu8_failed = false;
   float* lora_a[2] = {nullptr, nullptr};
   float* lora_b[2] = {nullptr, nullptr};
@@ -164,6 +165,7 @@ struct mi_engine {
   int opt_attn_mfma = 1;                 // decode attention on the matrix cores where the shape allows
   int opt_tile_weights = 1;
   int opt_prefill_gemm = 1;
+  int opt_codes_copy = 1;       // prefills of quantised models multiply the copies of the codes that mi_engine_finalize made (0: a copy per call)
   int opt_skinny_gemm = 1;      // decode steps of 9..128 rows (int4 / int8: 1..128): the split-K weight-streaming GEMM (gemm_skinny.hip; int4 / int8 up to 8 rows: gemv_reg.hip)
   int cur_L = 0;                // tokens per sequence of the forward pass being enqueued
   // RMSNorm hand-over between gemm_skinny launches (GemvCall::sq_out / sq_in): the residual linear in front of a norm

@@ -126,7 +126,7 @@ int make_f32_copy(mi_engine* e, const void* src, int n, void** dst) {
 }
 
 void free_linear(FusedLinear& f) {
-  hipFree(f.w); hipFree(f.scales); hipFree(f.biases); hipFree(f.w_hilo); hipFree(f.w_gu8);
+  hipFree(f.w); hipFree(f.scales); hipFree(f.biases); hipFree(f.w_hilo); hipFree(f.w_gu8); hipFree(f.w_codes);
   for (int i = 0; i < 2; ++i) { hipFree(f.lora_a[i]); hipFree(f.lora_b[i]); }
 }
 
@@ -201,6 +201,21 @@ bool ensure_hilo(mi_engine* e, FusedLinear& f) {
   if (launch_f16_to_hilo(f.W, p, e->stream) != MI_OK) { hipFree(p); f.hilo_failed = true; return false; }
   f.w_hilo = p;
   return true;
+}
+// Codes of quantised weights as the prefill GEMM multiplies them: made once, a prompt no longer writes and reads 2 bytes per weight in front of every product
+// (28672 x 4096 int4: 51 us of 314 at 700 rows).  2.2 bytes per weight, while half of the device's memory stays free.
+void make_codes_copy(mi_engine* e, FusedLinear& f) {
+  if (!wk_is_quant(f.W.wk) || f.W.layout != 1 || f.W.group != 64 || f.W.K > 65536 || wk_scale_dtype(f.W.wk) == WK_F32 || f.w_codes != nullptr || e->opt_force_v1) return;
+  size_t avail = 0, total = 0;
+  const size_t need = codes16_kept_bytes(f.W.N, f.W.K);
+  if (hipMemGetInfo(&avail, &total) != hipSuccess) { (void)hipGetLastError(); return; }
+  if (avail < need + total / 2) return;
+  void* p = nullptr;
+  if (hipMalloc(&p, need) != hipSuccess) { (void)hipGetLastError(); return; }
+  Codes16 c;
+  if (launch_codes16_kept(f.W, p, e->stream, c) != MI_OK) { hipFree(p); return; }
+  f.w_codes = p;
+  f.W.codes = c;
 }
 bool gu8_wanted(const mi_engine* e, const FusedLinear& f, int pair_offset) {
   const bool has_lora = f.W.lora_b[0] != nullptr || f.W.lora_b[1] != nullptr;
@@ -448,6 +463,7 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
     for (int n0 = 0; n0 < f.W.N; n0 += ncol) {
       LinearW part = f.W;
       GemvCall cp = c;
+      part.codes = e->opt_codes_copy ? codes16_rows(f.W.codes, n0, f.W.K) : Codes16{};
       if (ncol < f.W.N) {
         part.N = std::min(ncol, f.W.N - n0);
         part.w = (const char*)f.W.w + (wk_bits(f.W.wk) == 4 ? tiled_block_q4(n0, 0, f.W.K) : tiled_block_q8(n0, 0, f.W.K));
@@ -1269,11 +1285,13 @@ int mi_engine_finalize(mi_engine* e) {
     MI_TRY(make_f32_copy(e, l.k_norm, d.head_dim, &l.k_norm32));
     // persistent second copies, while mem_get_info still tells a scheduler the truth about what is left for its KV arena
     (void)ensure_gu8(e, l.gate_up, d.intermediate_size);
+    make_codes_copy(e, l.qkv); make_codes_copy(e, l.o); make_codes_copy(e, l.gate_up); make_codes_copy(e, l.down);
     if (d.act_dtype == MI_F16) { (void)ensure_hilo(e, l.qkv); (void)ensure_hilo(e, l.o); (void)ensure_hilo(e, l.gate_up); (void)ensure_hilo(e, l.down); }
   }
   MI_TRY(finalize_linear(e, e->embed, H, "model.embed_tokens"));
   if (!d.tie_word_embeddings) MI_TRY(finalize_linear(e, e->lm_head, H, "lm_head"));
   if (d.act_dtype == MI_F16) (void)ensure_hilo(e, d.tie_word_embeddings ? e->embed : e->lm_head);
+  make_codes_copy(e, d.tie_word_embeddings ? e->embed : e->lm_head);
   if (!e->final_norm) return fail(MI_ERR_NOTFOUND, "model.norm.weight not set");
   MI_TRY(make_f32_copy(e, e->final_norm, H, &e->final_norm32));
   const size_t n = (size_t)d.max_positions * (d.head_dim / 2);
@@ -1793,6 +1811,7 @@ int mi_engine_set_option(mi_engine* e, const char* key, int64_t value) {
   if (k == "decode_attention_mfma") { e->opt_attn_mfma = value != 0; return MI_OK; }
   if (k == "fused_gemv_pairs") { e->opt_fused_pairs = (int)value; return MI_OK; }
   if (k == "f16_hilo") { e->opt_f16_hilo = value != 0; return MI_OK; }
+  if (k == "prefill_codes_copy") { e->opt_codes_copy = value != 0; return MI_OK; }
   if (k == "gate_up_interleave") { e->opt_gu8 = value != 0; return MI_OK; }
   if (k == "seam_spin_limit") {
     if (value < 0 || value > (int64_t)0x7fffffff) return fail(MI_ERR_INVALID, "seam_spin_limit out of range");

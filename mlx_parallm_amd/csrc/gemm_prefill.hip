@@ -1733,7 +1733,7 @@ static bool codes_plan(const LinearW& W, const GemvCall& c, size_t rows, int ldx
 
 // Float32 rows against a quantised matrix: the tile GEMM, or 32 rows per launch of the streaming kernel?  us of both, fitted to 16 shapes of int4 and int8:
 // a launch of the streaming kernel 11 + 0.30 per 2^20 weights + 0.5 per 1024 columns (6144 x 4096 20, 28672 x 4096 42 int4 and 45 int8, 2048 x 6400 20, 5120 x
-// 17408 54 and 57); the codes' copy 0.65, a round of workgroups 1.35 per K tile, the slices' reduce.  At 40 to 1365 rows of these the choice costs 0.2 % on
+// 17408 54 and 57); the codes' copy 0.65 (none where one is kept), a round of workgroups 1.35 per K tile, the slices' reduce.  At 40 to 1365 rows of these the choice costs 0.2 % on
 // average over the better side, 12 % at most (28672 x 4096 SwiGLU: codes / streaming 192 rows 352 / 272, 256 rows 357 / 363, 512 rows 414 / 725; 6144 x 4096 96
 // rows 70 / 62, 129 rows 71 / 103; all int8), and int8, which the streaming kernel had at every size, is nowhere slower than there.
 static bool gemm_prefill_pays_codes(const LinearW& W, const GemvCall& c, size_t rows, int terms, size_t splitk_cap) {
@@ -1744,7 +1744,7 @@ static bool gemm_prefill_pays_codes(const LinearW& W, const GemvCall& c, size_t 
   const int ncu = gemv_cu_count(), tiles = ((p.ka + p.kb) / BK + p.ksplit - 1) / p.ksplit;
   const double mw = (double)W.N * W.K / (1 << 20), rounds = (double)((blocks * p.ksplit + ncu - 1) / ncu);
   const double reduce = p.ksplit > 1 ? 2e-6 * p.ksplit * rows * W.N : 0.0;
-  return 12.0 + 0.65 * mw + 1.35 * rounds * tiles + reduce < (double)((rows + 31) / 32) * (11.0 + 0.30 * mw + 0.5 * W.K / 1024);
+  return 12.0 + (W.codes.codes != nullptr ? 0.0 : 0.65 * mw) + 1.35 * rounds * tiles + reduce < (double)((rows + 31) / 32) * (11.0 + 0.30 * mw + 0.5 * W.K / 1024);
 }
 
 bool gemm_prefill_on_codes(const LinearW& W, const GemvCall& c, size_t rows) {
@@ -1788,9 +1788,13 @@ static int launch_gemm_codes(const LinearW& W, const GemvCall& c, size_t rows, h
   if (!codes_plan(W, c, rows, c.ldx, terms, splitk_ws != nullptr, splitk_cap, p, blocks)) return MI_OK;
   p.x = c.x;
   p.ws = (float*)splitk_ws;
-  MI_TRY(launch_codes16(W, scratch, st, terms == 1));
   char* d = (char*)scratch;
-  p.w = d; p.wb = d + (size_t)W.N * W.K * 2; p.sc = (const float*)(d + (size_t)W.N * (W.K + p.kb) * 2);
+  if (W.codes.codes != nullptr) {                        // (a copy that was made when the weights were loaded)
+    p.w = W.codes.codes; p.wb = W.codes.bias[terms != 1]; p.sc = W.codes.scales;
+  } else {
+    MI_TRY(launch_codes16(W, scratch, st, terms == 1));
+    p.w = d; p.wb = d + (size_t)W.N * W.K * 2; p.sc = (const float*)(d + (size_t)W.N * (W.K + p.kb) * 2);
+  }
   uint16_t* xs = (uint16_t*)(d + codes16_bytes(W.N, W.K));
   p.xs = xs;
   if (c.act == MI_F16) hipLaunchKernelGGL(group_sums_kernel<f16>, dim3((unsigned)rows), dim3(256), p.G * sizeof(float), st, (const f16*)c.x, c.ldx, terms, W.K, xs, p.kb, terms == 1);

@@ -5,6 +5,13 @@
 namespace mi {
 
 // One (possibly fused) weight matrix W[N][K] as the kernels see it.
+// The operands of the prefill GEMM on codes (repack.hip): the codes as 16-bit integers, the biases (of 16-bit rows: the largest parts first, of float32 rows: last), the scales
+struct Codes16 {
+  const void* codes = nullptr;
+  const void* bias[2] = {nullptr, nullptr};      // [float32 rows]
+  const float* scales = nullptr;
+};
+
 struct LinearW {
   int wk = WK_F32;             // weight kind (common.h)
   const void* w = nullptr;     // dense [N][K] or MLX-packed [N][K*bits/32] uint32
@@ -19,6 +26,7 @@ struct LinearW {
   const float* lora_b[2] = {nullptr, nullptr};
   int lora_row0[2] = {0, 0}, lora_n[2] = {0, 0}, lora_rank[2] = {0, 0};
   float lora_scale[2] = {0.f, 0.f};
+  Codes16 codes;               // quantised matrices: a copy of the codes that the prefill GEMM multiplies, if one is kept
 };
 
 enum : int { PRO_NONE = 0, PRO_NORM = 1 };
@@ -129,6 +137,10 @@ int launch_dequant_q4_hilo(const LinearW& src, void* dst, hipStream_t st);
 int codes16_bias_cols(int K);
 size_t codes16_bytes(int N, int K);
 int launch_codes16(const LinearW& src, void* dst, hipStream_t st, bool big_first = false);
+// .. kept for good: both orders of the biases
+size_t codes16_kept_bytes(int N, int K);
+int launch_codes16_kept(const LinearW& src, void* dst, hipStream_t st, Codes16& out);
+Codes16 codes16_rows(const Codes16& c, int n0, int K);       // of the outputs from n0 (a multiple of 16) on
 // term t of that product, the smallest first: part of x's group sum (0 = hi, 1 = mid, 2 = lo) and of the bias; products below 2^-24 of the whole are left
 // out.  big_first: these terms in reverse
 constexpr int CODES16_TERMS = 6;

@@ -203,23 +203,45 @@ __global__ __launch_bounds__(256) void codes16_kernel(const uint8_t* src, T* cod
 int codes16_bias_cols(int K) { return (CODES16_TERMS * (K / 64) + 63) / 64 * 64; }
 size_t codes16_bytes(int N, int K) { return (size_t)N * ((size_t)K * 2 + (size_t)codes16_bias_cols(K) * 2 + (size_t)(K / 64) * 4); }
 
-int launch_codes16(const LinearW& src, void* dst, hipStream_t st, bool big_first) {
+size_t codes16_kept_bytes(int N, int K) { return codes16_bytes(N, K) + (size_t)N * codes16_bias_cols(K) * 2; }
+
+// side_only: biases and scales without the codes
+static int codes16_into(const LinearW& src, void* codes, uint16_t* wb, float* sc, hipStream_t st, bool big_first, bool side_only) {
   const int bits = wk_bits(src.wk), sdt = wk_scale_dtype(src.wk);
   if (src.layout != 1 || (bits != 4 && bits != 8) || sdt == WK_F32 || src.group != 64 || src.K % (bits == 4 ? 128 : 64) != 0 || src.N % 16 != 0)
     return fail(MI_ERR_UNSUPPORTED, "codes16: tile-major int4 / int8 (group 64) matrices only");
   const int kb = codes16_bias_cols(src.K);
-  char* d = (char*)dst;
-  void* codes = d;
-  uint16_t* wb = (uint16_t*)(d + (size_t)src.N * src.K * 2);
-  float* sc = (float*)(d + (size_t)src.N * (src.K + kb) * 2);
   const int nb = src.K / (bits == 4 ? 128 : 64), tiles = src.N / 16;
-  const dim3 grid(1 + (nb + 7) / 8, tiles);                          // (two blocks a wave)
+  const dim3 grid(side_only ? 1 : 1 + (nb + 7) / 8, tiles);          // (two blocks a wave)
 #define GO(T, B) hipLaunchKernelGGL((codes16_kernel<T, B>), grid, dim3(256), (size_t)(src.K / 64) * 64, st, (const uint8_t*)src.w, (T*)codes, wb, sc, src.K, kb, (int)big_first)
   if (sdt == WK_BF16) { if (bits == 4) GO(bf16, 4); else GO(bf16, 8); }
   else { if (bits == 4) GO(f16, 4); else GO(f16, 8); }
 #undef GO
   MI_HIP(hipGetLastError());
   return MI_OK;
+}
+
+int launch_codes16(const LinearW& src, void* dst, hipStream_t st, bool big_first) {
+  char* d = (char*)dst;
+  return codes16_into(src, d, (uint16_t*)(d + (size_t)src.N * src.K * 2), (float*)(d + (size_t)src.N * (src.K + codes16_bias_cols(src.K)) * 2), st, big_first, false);
+}
+
+int launch_codes16_kept(const LinearW& src, void* dst, hipStream_t st, Codes16& out) {
+  char* d = (char*)dst;
+  uint16_t* wb[2] = {(uint16_t*)(d + (size_t)src.N * src.K * 2), (uint16_t*)(d + codes16_bytes(src.N, src.K))};
+  float* sc = (float*)(d + (size_t)src.N * (src.K + codes16_bias_cols(src.K)) * 2);
+  for (int f32 = 0; f32 < 2; ++f32) MI_TRY(codes16_into(src, d, wb[f32], sc, st, f32 == 0, f32 == 1));
+  out.codes = d; out.bias[0] = wb[0]; out.bias[1] = wb[1]; out.scales = sc;
+  return MI_OK;
+}
+
+Codes16 codes16_rows(const Codes16& c, int n0, int K) {
+  Codes16 r = c;
+  if (c.codes == nullptr) return r;
+  r.codes = (const char*)c.codes + (size_t)n0 * K * 2;
+  for (int f32 = 0; f32 < 2; ++f32) r.bias[f32] = (const char*)c.bias[f32] + (size_t)n0 * codes16_bias_cols(K) * 2;
+  r.scales = c.scales + (size_t)n0 * (K / 64);
+  return r;
 }
 
 size_t dequant_hilo_bytes(int N, int K) { return (size_t)N * K * 2 * 2; }

@@ -227,3 +227,50 @@ def test_the_last_piece_of_wide_logits_is_no_other_kernel(kv):
         assert np.mean(first != last) <= 0.01 and off <= 2.0 ** -8
     else:
         assert off <= 2.0 ** -24 * np.sqrt(2 * (K / 64 + 6 * K / 2048 + 2)), off
+
+
+@pytest.mark.parametrize("act", ["bfloat16", "float16"])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("kv_dtype", ["model", "float32"])
+def test_kept_codes_and_codes_per_call_give_the_same_bits(bits, act, kv_dtype):
+    """The copy that an engine makes of its quantised weights and the one made in front of a product hold the same: prompts' logits, and the logits of every position
+    in pieces of 32768 columns, with and without it (float32 caches: the other order of the biases)."""
+    from mlx_parallm_amd.engine import Engine, SampleArgs
+
+    H, F, V = 1024, 2816, 33024
+    cfg = dict(model_type="llama", hidden_size=H, num_hidden_layers=2, num_attention_heads=8, num_key_value_heads=8, head_dim=128, intermediate_size=F, vocab_size=V,
+               rms_norm_eps=1e-5, rope_theta=10000.0, tie_word_embeddings=False, max_position_embeddings=1024, quantization={"bits": bits, "group_size": 64})
+    dt = getattr(torch, act)
+    g = torch.Generator(device="cuda").manual_seed(bits)
+
+    def put(e, name, n, k):
+        e.set_tensor(name + ".weight", torch.randint(-2 ** 31, 2 ** 31 - 1, (n, k * bits // 32), generator=g, device="cuda", dtype=torch.int32))
+        scale = 2.0 / (2 ** bits - 1) / k ** 0.5
+        e.set_tensor(name + ".scales", (scale * (1.0 + torch.rand((n, k // 64), generator=g, device="cuda"))).to(dt))
+        e.set_tensor(name + ".biases", (-1.5 / k ** 0.5 * (1.0 + 0.3 * torch.randn((n, k // 64), generator=g, device="cuda"))).to(dt))
+    e = Engine(cfg, device=0, max_positions=1024, act_dtype=act)
+    put(e, "model.embed_tokens", V, H)
+    put(e, "lm_head", V, H)
+    for i in range(2):
+        p = f"model.layers.{i}."
+        for n, rows, cols in (("self_attn.q_proj", H, H), ("self_attn.k_proj", H, H), ("self_attn.v_proj", H, H), ("self_attn.o_proj", H, H), ("mlp.gate_proj", F, H),
+                              ("mlp.up_proj", F, H), ("mlp.down_proj", H, F)):
+            put(e, p + n, rows, cols)
+        for n in ("input_layernorm", "post_attention_layernorm"):
+            e.set_tensor(p + n + ".weight", torch.ones(H, device="cuda", dtype=dt))
+    e.set_tensor("model.norm.weight", torch.ones(H, device="cuda", dtype=dt))
+    e.finalize()
+    toks = np.random.default_rng(3).integers(0, V, (2, 450)).astype(np.int32)
+    kv = e.new_kv(2, capacity=512, kv_dtype=kv_dtype)
+    out = []
+    for kept in (1, 0):
+        e.set_option("prefill_codes_copy", kept)
+        kv.reset()
+        logits = np.asarray(e.forward(toks, kv)).copy()
+        kv.reset()
+        r = e.score_tokens(kv, toks, toks, SampleArgs(top_logprobs=3))
+        out.append((logits, np.asarray(r["logprobs"]).copy(), np.asarray(r["top_logprobs"]).copy()))
+    e.close()
+    assert np.all(np.isfinite(out[0][0]))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
