@@ -65,6 +65,9 @@ struct GemmParams {
   // few hundred tokens against N = 4096: 32 x 2..8 blocks); slice z leaves its float32 partial tile in ws[z][M][N] and
   // splitk_epilogue_kernel adds the slices in order and applies the epilogue
   int ksplit; float* ws;
+  // codes form, K slices of the last tiles alone: `mb` row blocks (0: the plain grid); the tiles from `tail` on (row blocks fastest) are ksplit workgroups
+  // each, which leave their accumulators in ws[tile][slice] for tail_reduce_kernel
+  int mb, tail;
   // grouped form (GroupedGemm, kernels.h)
   const int32_t* tiles; const int32_t* x_rows; const int32_t* out_rows; int groups;
   const void* w_last; int N_last, K_last;
@@ -324,31 +327,30 @@ __device__ __forceinline__ bool epilogue_varies(const GemmParams& p, int bn) { r
 // the epilogue of the 256 x 256 tiles (2 x 4 waves, 128 x 64 per wave): lane (c16, g) holds C[m = 4g + r][n = c16] of
 // every 16 x 16 tile
 // VAR: another unit than silu, or a plain store with silu columns (common.h)
+// (rows m4 .. m4 + 3 of the wave's 64 columns)
 template <typename AT, bool SWIGLU, bool VAR, bool LOGITS = false>
-__device__ __forceinline__ void tile256_epilogue(const GemmParams& p, f32x4 (&acc)[8][4], int m0, int bn, int wm, int wn, int c16, int g) {
+__device__ __forceinline__ void tile256_epilogue_row(const GemmParams& p, const f32x4 (&acc)[4], int m4, int bn, int wn, int c16) {
   AT* out = (AT*)p.out;
 #pragma unroll
-  for (int mt = 0; mt < 8; ++mt)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = m0 + wm * 128 + mt * 16 + 4 * g + r;
+  for (int r = 0; r < 4; ++r) {
+      const int m = m4 + r;
       if (m >= p.M) continue;
       if constexpr (SWIGLU) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           const int n = bn * 128 + wn * 32 + j * 16 + c16;
           if (n >= p.pair_offset) continue;
-          if (p.out32) { epi32_swiglu(p, m, n, acc[mt][j][r], acc[mt][j + 2][r]); continue; }
-          out[(size_t)m * p.ldo + n] = VAR ? (AT)glu_f(p.glu, acc[mt][j][r], acc[mt][j + 2][r]) : silu16<AT>(acc[mt][j][r], acc[mt][j + 2][r]);
+          if (p.out32) { epi32_swiglu(p, m, n, acc[j][r], acc[j + 2][r]); continue; }
+          out[(size_t)m * p.ldo + n] = VAR ? (AT)glu_f(p.glu, acc[j][r], acc[j + 2][r]) : silu16<AT>(acc[j][r], acc[j + 2][r]);
         }
       } else {
 #pragma unroll
         for (int nt = 0; nt < 4; ++nt) {
           const int n = bn * BN2 + wn * 64 + nt * 16 + c16;
           if (n >= p.N) continue;
-          if constexpr (LOGITS) { ((float*)p.out)[(size_t)m * p.ldo + n] = (float)(AT)acc[mt][nt][r]; continue; }
-          if (p.out32) { epi32_plain(p, m, n, acc[mt][nt][r]); continue; }
-          const float y = (float)(AT)(VAR ? silu_col(p.silu_cols, n, acc[mt][nt][r]) : acc[mt][nt][r]);
+          if constexpr (LOGITS) { ((float*)p.out)[(size_t)m * p.ldo + n] = (float)(AT)acc[nt][r]; continue; }
+          if (p.out32) { epi32_plain(p, m, n, acc[nt][r]); continue; }
+          const float y = (float)(AT)(VAR ? silu_col(p.silu_cols, n, acc[nt][r]) : acc[nt][r]);
           if (p.epi == EPI_STORE) out[(size_t)m * p.ldo + n] = (AT)y;
           else {
             AT* h = (AT*)p.resid;
@@ -357,6 +359,12 @@ __device__ __forceinline__ void tile256_epilogue(const GemmParams& p, f32x4 (&ac
         }
       }
     }
+}
+
+template <typename AT, bool SWIGLU, bool VAR, bool LOGITS = false>
+__device__ __forceinline__ void tile256_epilogue(const GemmParams& p, f32x4 (&acc)[8][4], int m0, int bn, int wm, int wn, int c16, int g) {
+#pragma unroll
+  for (int mt = 0; mt < 8; ++mt) tile256_epilogue_row<AT, SWIGLU, VAR, LOGITS>(p, acc[mt], m0 + wm * 128 + mt * 16 + 4 * g, bn, wn, c16);
 }
 
 // Grouped form: whole rows.  A wave's tile goes through its own strip of LDS, 64 rows at a time, and leaves it as 16-byte pieces of
@@ -997,12 +1005,19 @@ __global__ __launch_bounds__(512) void gemm_codes256_kernel(GemmParams p) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 2, wn = wave & 3;
   const int c16 = lane & 15, g = lane >> 4;
-  const int bm = blockIdx.x, bn = blockIdx.y, m0 = bm * BM2;
+  int bm = blockIdx.x, bn = blockIdx.y, z = 0, nz = 1;
+  if (p.mb > 0) {                                               // (uniform) K slices of the last tiles alone
+    int tile = blockIdx.x;
+    if (tile >= p.tail) { const int u = tile - p.tail; nz = p.ksplit; tile = p.tail + u / nz; z = u - u / nz * nz; }
+    bn = tile / p.mb; bm = tile - bn * p.mb;
+    bm = __builtin_amdgcn_readfirstlane(bm); bn = __builtin_amdgcn_readfirstlane(bn); z = __builtin_amdgcn_readfirstlane(z); nz = __builtin_amdgcn_readfirstlane(nz);
+  }
+  const int m0 = bm * BM2;
   // K tiles: [0, nkm) = the groups of x's terms in turn, the last term first (W is walked once per term), [nkm, nk_all) = the bias columns
   const int nkm = p.ka / BK, nk_all = nkm + p.kb / BK;
   // this workgroup's: [tb, te) (divisions run on vector registers: back to scalar ones, the DMA bases are built of them)
-  const int tb = __builtin_amdgcn_readfirstlane((int)((blockIdx.z * (unsigned)nk_all) / gridDim.z));
-  const int te = __builtin_amdgcn_readfirstlane((int)(((blockIdx.z + 1) * (unsigned)nk_all) / gridDim.z));
+  const int tb = __builtin_amdgcn_readfirstlane((int)((z * (unsigned)nk_all) / nz));
+  const int te = __builtin_amdgcn_readfirstlane((int)(((z + 1) * (unsigned)nk_all) / nz));
   const int ntiles_w = p.N / 16;
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem2;
 
@@ -1190,8 +1205,11 @@ __global__ __launch_bounds__(512) void gemm_codes256_kernel(GemmParams p) {
 #undef PP_READS_DONE
 #undef PP_MMA_DONE
 
-  if constexpr (!SWIGLU) {
-    if (gridDim.z > 1) { tile256_partial(p, acc, smem2, m0, bn, wave, lane); return; }
+  if (nz > 1) {                                                  // (whole KiB, in the registers' order)
+    f32x4* dst = (f32x4*)p.ws + (((size_t)(bn * p.mb + bm - p.tail) * nz + z) * 8 + wave) * (32 * 64) + lane;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) dst[i * 64] = acc[i >> 2][i & 3];
+    return;
   }
   // (one gated unit, no silu columns: codes_fits; rows that are no whole pieces are none of the engine's)
   if (p.strips) {
@@ -1200,6 +1218,23 @@ __global__ __launch_bounds__(512) void gemm_codes256_kernel(GemmParams p) {
   } else {
     tile256_epilogue<AT, SWIGLU, false, LOGITS>(p, acc, m0, bn, wm, wn, c16, g);
   }
+}
+
+// The K slices of the kernel above, added in order, and its epilogues: a workgroup per tile and row tile of its waves
+template <typename AT, bool SWIGLU, bool LOGITS>
+__global__ __launch_bounds__(512) void tail_reduce_kernel(GemmParams p) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, tile = blockIdx.x, mt = blockIdx.y;
+  const int bn = (p.tail + tile) / p.mb, bm = (p.tail + tile) % p.mb, m4 = bm * BM2 + (wave >> 2) * 128 + mt * 16 + 4 * (lane >> 4);
+  if (bm * BM2 + (wave >> 2) * 128 + mt * 16 >= p.M) return;
+  const f32x4* src = (const f32x4*)p.ws + ((size_t)tile * p.ksplit * 8 + wave) * (32 * 64) + mt * 4 * 64 + lane;
+  f32x4 a[4];
+#pragma unroll
+  for (int nt = 0; nt < 4; ++nt) a[nt] = src[nt * 64];
+#pragma unroll 2
+  for (int z = 1; z < p.ksplit; ++z)
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) a[nt] += src[(size_t)z * (8 * 32 * 64) + nt * 64];
+  tile256_epilogue_row<AT, SWIGLU, false, LOGITS>(p, a, m4, bn, wave & 3, lane & 15);
 }
 
 // The group sums of x for the kernel above: row m -> `parts` terms of G columns each (kernels.h: codes16_sum_part; hi + mid + lo = the float32 sum
@@ -1718,6 +1753,31 @@ size_t gemm_prefill_scratch_bytes(const LinearW& W, size_t rows) {
 // mean exceeds 3 of its deviations.  2-norm from 64 bits, 1024 x 1024, 256 rows, means of 0 / 4 / 12 deviations: pair 1.8e-7 / 7.0e-7 / 1.9e-6,
 // streaming 3.3e-7 / 1.3e-7 / 1.0e-7, here 0.8e-7 / 0.7e-7 / 0.7e-7 (2048 x 4096, 160 rows: 3.7e-7 / 7.7e-7 / 1.9e-6, 3.4e-7 / 1.4e-7 / 1.2e-7, 1.2e-7 / 0.8e-7 / 0.8e-7);
 // us, streaming / here: 129 rows 59 / 29, 1365 rows 511 / 40.
+// us of a launch over `blocks` tiles of `nk` K tiles in rounds of one workgroup per CU, those from `tail` on as `ks` slices: a round 10 + 2 per K tile, what joins the slices
+// 3 + their 256 KiB each at 4.9 TB/s (fitted: 6144 x 4096, 700 rows, 7 slices 66 + 23, 4096 x 14336 with 5 94 + 15, 28672 x 4096 SwiGLU, unsplit, 277)
+static double tail_us(long blocks, long tail, int nk, int ks, int ncu) {
+  const auto rounds = [&](long n) { return (double)((n + ncu - 1) / ncu); };
+  const double full = rounds(tail) * (10.0 + 2.0 * nk);
+  if (tail == blocks) return full;
+  const long t = blocks - tail;
+  return full + rounds(t * ks) * (10.0 + 2.0 * ((nk + ks - 1) / ks)) + 3.0 + t * ks * 0.262144 / 4.9;
+}
+
+// K slices for the tiles of a last, partly filled round (all of them where there is only that round): the cheapest by the line above, at least 8 K tiles a slice.  Whole
+// columns of tiles: all rows of a call have one order of sums.  700 rows, us: 28672 x 4096 SwiGLU (336 tiles, the last 81 in three) 277 -> 200 + 16, 6144 x 4096 (72 tiles: three slices
+// for seven) 89 -> 54 + 13, 32000 x 4096 logits 284 -> 235 + 18.
+static void tail_plan(long mb, long blocks, int nk, size_t cap, GemmParams& p) {
+  const int ncu = gemv_cu_count();
+  double best = tail_us(blocks, blocks, nk, 1, ncu) - 5.0;       // (what the line is sure of)
+  for (const long tail : {blocks / ncu * ncu / mb * mb, 0L}) {
+    for (int ks = 2; ks <= 8 && nk / ks >= 8 && (size_t)(blocks - tail) * ks * (BM2 * BN2 * 4) <= cap; ++ks) {
+      if (tail == blocks) break;
+      const double t = tail_us(blocks, tail, nk, ks, ncu);
+      if (t < best) { best = t; p.mb = (int)mb; p.tail = (int)tail; p.ksplit = ks; }
+    }
+  }
+}
+
 static bool codes_plan(const LinearW& W, const GemvCall& c, size_t rows, int ldx, int terms, bool split_ok, size_t cap, GemmParams& p, long& blocks) {
   const bool sw = c.epi == EPI_SWIGLU;
   const int ncols = sw ? c.pair_offset : W.N;
@@ -1727,7 +1787,8 @@ static bool codes_plan(const LinearW& W, const GemvCall& c, size_t rows, int ldx
   p.M = (int)rows; p.N = W.N; p.kw = W.K; p.ka = p.K = terms * W.K; p.ldx = ldx; p.G = W.K / 64;
   p.kb = codes16_bias_cols(W.K);
   blocks = (long)((rows + BM2 - 1) / BM2) * ((ncols + (sw ? 128 : BN2) - 1) / (sw ? 128 : BN2));
-  p.ksplit = !sw && split_ok && W.N % 4 == 0 ? split256(blocks, (p.ka + p.kb) / BK, rows * W.N * sizeof(float), cap) : 1;
+  p.ksplit = 1;
+  if (split_ok) tail_plan((long)((rows + BM2 - 1) / BM2), blocks, (p.ka + p.kb) / BK, cap, p);
   return true;
 }
 
@@ -1741,10 +1802,8 @@ static bool gemm_prefill_pays_codes(const LinearW& W, const GemvCall& c, size_t 
   long blocks = 0;
   if (!codes_plan(W, c, rows, terms * W.K, terms, splitk_cap > 0, splitk_cap, p, blocks))
     return (c.rnd == RND_NONE && c.epi != EPI_STORE_F32) || gemm_prefill_pays(true, false, c.rnd != RND_NONE, rows);
-  const int ncu = gemv_cu_count(), tiles = ((p.ka + p.kb) / BK + p.ksplit - 1) / p.ksplit;
-  const double mw = (double)W.N * W.K / (1 << 20), rounds = (double)((blocks * p.ksplit + ncu - 1) / ncu);
-  const double reduce = p.ksplit > 1 ? 2e-6 * p.ksplit * rows * W.N : 0.0;
-  return 12.0 + (W.codes.codes != nullptr ? 0.0 : 0.65 * mw) + 1.35 * rounds * tiles + reduce < (double)((rows + 31) / 32) * (11.0 + 0.30 * mw + 0.5 * W.K / 1024);
+  const double mw = (double)W.N * W.K / (1 << 20), gemm = tail_us(blocks, p.mb > 0 ? p.tail : blocks, (p.ka + p.kb) / BK, p.ksplit, gemv_cu_count());
+  return 5.0 + (W.codes.codes != nullptr ? 0.0 : 0.65 * mw) + gemm < (double)((rows + 31) / 32) * (11.0 + 0.30 * mw + 0.5 * W.K / 1024);
 }
 
 bool gemm_prefill_on_codes(const LinearW& W, const GemvCall& c, size_t rows) {
@@ -1807,12 +1866,20 @@ static int launch_gemm_codes(const LinearW& W, const GemvCall& c, size_t rows, h
     if (!x32) { p.out32 = 1; p.rnd = c.act == MI_BF16 ? RND_BF16 : RND_F16; }
   }
   p.strips = strips_ok(p);
-  const dim3 grid((unsigned)((rows + BM2 - 1) / BM2), (ncols + (sw ? 128 : BN2) - 1) / (sw ? 128 : BN2), p.ksplit);
+  const dim3 grid = p.mb > 0 ? dim3((unsigned)(p.tail + (blocks - p.tail) * p.ksplit)) : dim3((unsigned)((rows + BM2 - 1) / BM2), (ncols + (sw ? 128 : BN2) - 1) / (sw ? 128 : BN2));
   const bool rounded = p.rnd != RND_NONE;               // (float32 stores of values rounded to 16 bits: logits, and layer 0 of the float32-cache mode)
   if (terms > 1 && !rounded) MI_TRY((sw ? codes_launch<bf16, true, false, true> : codes_launch<bf16, false, false, true>)(p, grid, st));
   else if (c.act == MI_F16) MI_TRY((sw ? codes_launch<f16, true, false> : rounded ? codes_launch<f16, false, true> : codes_launch<f16, false, false>)(p, grid, st));
   else MI_TRY((sw ? codes_launch<bf16, true, false> : rounded ? codes_launch<bf16, false, true> : codes_launch<bf16, false, false>)(p, grid, st));
-  if (p.ksplit > 1) MI_TRY(reduce_slices(p, c.act, st));
+  if (p.ksplit > 1) {
+    const dim3 rg((unsigned)(blocks - p.tail), 8), rb(512);
+#define TAIL_GO(T) do { if (sw) hipLaunchKernelGGL((tail_reduce_kernel<T, true, false>), rg, rb, 0, st, p); \
+      else if (rounded) hipLaunchKernelGGL((tail_reduce_kernel<T, false, true>), rg, rb, 0, st, p); \
+      else hipLaunchKernelGGL((tail_reduce_kernel<T, false, false>), rg, rb, 0, st, p); } while (0)
+    if (c.act == MI_F16) TAIL_GO(f16); else TAIL_GO(bf16);
+#undef TAIL_GO
+    MI_HIP(hipGetLastError());
+  }
   *done = true;
   return MI_OK;
 }

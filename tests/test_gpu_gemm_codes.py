@@ -274,3 +274,35 @@ def test_kept_codes_and_codes_per_call_give_the_same_bits(bits, act, kv_dtype):
     assert np.all(np.isfinite(out[0][0]))
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("act", ["bfloat16", "float16"])
+@pytest.mark.parametrize("bits,M,N,K,epi", [
+    (4, 700, 2 * 11520, 1024, "swiglu"),     # 270 tiles: one round, and 15 in K slices
+    (8, 300, 2 * 1040, 1088, "swiglu"),      # fewer tiles than CUs, the last ones ragged: all in slices
+    (4, 700, 24016, 1024, "f32"),            # 282 tiles; the last column of tiles holds 208 columns
+    (8, 601, 22032, 1024, "resid"),
+])
+def test_tiles_of_a_last_round_in_slices(act, bits, M, N, K, epi):
+    """Against the oracle; every row of a call has one order of sums, whatever its place: a row's copy at the end gives the same bits."""
+    rng = np.random.default_rng(M + N)
+    ol, w, keep = _weight(bits, act, N, K, rng)
+    x = round_to(rng.standard_normal((M, K)).astype(np.float32) * 0.3, act)
+    h0 = round_to(rng.standard_normal((M, N)).astype(np.float32), act)
+    x[M - 1], h0[M - 1] = x[5], h0[5]
+    xd, rows = dev(x, act), _rows(M)
+    y = want = round_to(matmul_nt(x[rows], w), act)
+    cols, kw, code = N, {}, L.EPI_STORE_F32
+    if epi == "swiglu":
+        cols, code = N // 2, L.EPI_SWIGLU
+        kw = dict(pair_offset=cols)
+        sig = round_to((1.0 / (1.0 + np.exp(-y[:, :cols].astype(np.float64)))).astype(np.float32), act)
+        want = round_to(round_to(y[:, :cols] * sig, act) * y[:, cols:], act)
+    out = torch.full((M + 1, cols), 7.0, dtype=torch.float32 if epi == "f32" else xd.dtype, device="cuda")
+    if epi == "resid":
+        out[:M] = dev(h0, act)
+        code, kw, want = L.EPI_RESID, dict(resid=out), round_to(h0[rows] + y, act)
+    _run(ol, xd, M, act, force=True, epi=code, out=out, ldo=cols, **kw)
+    o = host(out)
+    assert np.all(o[M:] == 7.0) and np.array_equal(o[M - 1], o[5])
+    _assert_close(o[:M][rows], want, act, scale=float(np.abs(y).max()))
