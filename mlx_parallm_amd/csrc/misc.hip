@@ -113,30 +113,40 @@ int launch_embed_wk(const LinearW& W, const EmbedCall& c, hipStream_t st) {
 // result does not depend on the order in which threads add.
 constexpr int ST = 1024;
 
-// f(value, index) over one row of logits.  A pass is latency-bound if every thread walks it one dependent 4-byte load
-// at a time (measured: ~9 us per pass over 32000 logits); 16-byte loads, two in flight per thread.  (Four in flight:
-// measured in round 4, no change -- 55.7 us per top-p draw at V = 32000 either way.  What bounds the histogram passes is
-// the same-address serialisation of their LDS atomics: a row's logits share a handful of exponents.)
+// A thread's elements of one row of logits, up to eight at a time: f(values, indices, how many).  A pass is latency-bound if every thread walks it one
+// dependent 4-byte load at a time (measured: ~9 us per pass over 32000 logits); 16-byte loads, two in flight per thread (four in flight: no change;
+// what bounds the histogram passes is the LDS atomics).
+__device__ __forceinline__ bool row_vec(const float* lg, int V) { return (V & 3) == 0 && (((uintptr_t)lg) & 15) == 0; }
 template <class F>
-__device__ __forceinline__ void for_row(const float* lg, int V, F f) {
-  if ((V & 3) == 0 && (((uintptr_t)lg) & 15) == 0) {
+__device__ __forceinline__ void for_row8(const float* lg, int V, F f) {
+  if (row_vec(lg, V)) {
     const float4* p4 = (const float4*)lg;
     const int n4 = V >> 2;
     int i = threadIdx.x;
     for (; i + ST < n4; i += 2 * ST) {
       const float4 a = p4[i], b = p4[i + ST];
       const int j = 4 * i, k = 4 * (i + ST);
-      f(a.x, j); f(a.y, j + 1); f(a.z, j + 2); f(a.w, j + 3);
-      f(b.x, k); f(b.y, k + 1); f(b.z, k + 2); f(b.w, k + 3);
+      const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      const int at[8] = {j, j + 1, j + 2, j + 3, k, k + 1, k + 2, k + 3};
+      f(v, at, std::integral_constant<int, 8>{});
     }
     if (i < n4) {
       const float4 a = p4[i];
       const int j = 4 * i;
-      f(a.x, j); f(a.y, j + 1); f(a.z, j + 2); f(a.w, j + 3);
+      const float v[4] = {a.x, a.y, a.z, a.w};
+      const int at[4] = {j, j + 1, j + 2, j + 3};
+      f(v, at, std::integral_constant<int, 4>{});
     }
   } else {
-    for (int i = threadIdx.x; i < V; i += ST) f(lg[i], i);
+    for (int i = threadIdx.x; i < V; i += ST) { const float v[1] = {lg[i]}; const int at[1] = {i}; f(v, at, std::integral_constant<int, 1>{}); }
   }
+}
+template <class F>
+__device__ __forceinline__ void for_row(const float* lg, int V, F f) {
+  for_row8(lg, V, [&](const float* v, const int* at, auto n) {
+#pragma unroll
+    for (int j = 0; j < decltype(n)::value; ++j) f(v[j], at[j]);
+  });
 }
 
 __device__ __forceinline__ uint32_t order_key(float f) {  // larger float -> larger key
@@ -422,14 +432,23 @@ __global__ __launch_bounds__(ST) void sample_kernel(SampleCall c) {
     }
     __syncthreads();
   }
-  // ---- max / argmax, log-sum-exp
-  ArgMax a{-INFINITY, 0x7fffffff};
-  for_row(lg, V, [&](float l, int i) { a = am_better(a, ArgMax{l, i}); });
-  a = block_argmax(a, sh_am);
+  // ---- max / argmax, log-sum-exp: one walk, a thread's sum relative to its own maximum so far
+  ArgMax mine{-INFINITY, 0x7fffffff};
+  float part = 0.f;
+  const auto take = [&](const float* l, const int* idx, auto nt) {
+    constexpr int N = decltype(nt)::value;
+    const float was = mine.v;
+#pragma unroll
+    for (int j = 0; j < N; ++j) mine = am_better(mine, ArgMax{l[j], idx[j]});
+    if (mine.v > was) part *= __expf(was - mine.v);
+    const float ref = mine.v == -INFINITY ? 0.f : mine.v;
+#pragma unroll
+    for (int j = 0; j < N; ++j) part += __expf(l[j] - ref);
+  };
+  for_row8(lg, V, take);
+  ArgMax a = block_argmax(mine, sh_am);
   const float mx = a.v;
-  float se = 0.f;
-  for_row(lg, V, [&](float l, int) { se += __expf(l - mx); });
-  se = block_sum(se, sh_f);
+  const float se = block_sum(mine.v == -INFINITY ? part : part * __expf(mine.v - mx), sh_f);
   const float lse = mx + __logf(se);
   if (threadIdx.x == 0 && c.row_stats) { c.row_stats[2 * b] = mx; c.row_stats[2 * b + 1] = lse; }
 
@@ -490,21 +509,28 @@ __global__ __launch_bounds__(ST) void sample_kernel(SampleCall c) {
     c.tokens_out[b] = token;
     if (c.logprob_out) c.logprob_out[b] = (c.forced && forced < 0) ? 0.f : (lg[token] - mx) * lp_scale - lp_lse;
   }
-  // ---- top-k logprobs: k rounds of arg-max with exclusion of already emitted ids
-  if (c.top_logprobs > 0) {
-    float prev_v = INFINITY; int prev_i = -1;
-    for (int r = 0; r < c.top_logprobs; ++r) {
-      ArgMax t{-INFINITY, 0x7fffffff};
-      for_row(lg, V, [&](float v, int i) {
-        if (v < prev_v || (v == prev_v && i > prev_i)) t = am_better(t, ArgMax{v, i});
-      });
-      t = block_argmax(t, sh_am);
-      if (threadIdx.x == 0) {
-        c.topk_ids[(size_t)b * c.top_logprobs + r] = t.i < V ? t.i : 0;
-        c.topk_logprobs[(size_t)b * c.top_logprobs + r] = (t.v - mx) * lp_scale - lp_lse;
-      }
-      prev_v = t.v; prev_i = t.i;
+  // ---- top-k logprobs: k rounds of arg-max over the threads' best remaining elements; the winner's wave looks for its next one
+  const bool vec = row_vec(lg, V);
+  for (int r = 0; r < c.top_logprobs; ++r) {
+    const ArgMax t = block_argmax(mine, sh_am);
+    if (threadIdx.x == 0) {
+      c.topk_ids[(size_t)b * c.top_logprobs + r] = t.i < V ? t.i : 0;
+      c.topk_logprobs[(size_t)b * c.top_logprobs + r] = (t.v - mx) * lp_scale - lp_lse;
     }
+    if (t.i >= V || r + 1 == c.top_logprobs) continue;            // (uniform)
+    const int owner = (vec ? t.i >> 2 : t.i) % ST;
+    if ((int)threadIdx.x >> 6 != owner >> 6) continue;
+    ArgMax best{-INFINITY, 0x7fffffff};
+    const auto next = [&](float v, int i) { if (v < t.v || (v == t.v && i > t.i)) best = am_better(best, ArgMax{v, i}); };
+    for (int i = owner + (threadIdx.x & 63) * ST; i < (vec ? V >> 2 : V); i += 64 * ST) {
+      if (vec) {
+        const float4 q = ((const float4*)lg)[i];
+        next(q.x, 4 * i); next(q.y, 4 * i + 1); next(q.z, 4 * i + 2); next(q.w, 4 * i + 3);
+      } else next(lg[i], i);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) best = am_better(best, ArgMax{__shfl_xor(best.v, o, 64), __shfl_xor(best.i, o, 64)});
+    if ((int)threadIdx.x == owner) mine = best;
   }
 }
 

@@ -569,6 +569,25 @@ def test_sampler_greedy_logprobs_topk(V):
         assert np.allclose(kl[b], lsm[b, order], atol=1e-4)
 
 
+@pytest.mark.parametrize("V", [61, 1001, 4096, 5000, 32768 + 8])
+def test_sampler_top_logprobs_of_one_thread(V):
+    """The k best where one thread of the workgroup holds many of them (ids 4096 apart, and a run of four), where they tie (lowest id first), where a row
+    is mostly -inf; rows of whole 16-byte pieces and of others."""
+    lg = RNG.standard_normal((4, V)).astype(np.float32)
+    lg[0, np.arange(0, V, 4096)] = 9.0 + np.arange(len(np.arange(0, V, 4096)))
+    lg[0, :4] += 20.0
+    lg[1] = round_to(lg[1], "bfloat16")
+    lg[1, ::7] = 5.0
+    lg[2, 3:] = -np.inf
+    k = 20
+    toks, _lp, _p0, ki, kl = _run_sampler(lg, 0.0, 1.0, np.zeros(4), k=k)
+    lse = np.log(np.sum(np.exp(lg.astype(np.float64) - lg.max(1, keepdims=True)), 1)) + lg.max(1)
+    for b in range(4):
+        order = np.lexsort((np.arange(V), -lg[b]))[:k]
+        assert toks[b] == order[0] and np.array_equal(ki[b], order), (b, ki[b], order)
+        assert np.allclose(kl[b], lg[b, order] - lse[b], atol=1e-4)
+
+
 def _oracle_candidates(lg_row, temp, top_p):
     """The oracle's candidate list in draw order (descending probability, ties by ascending id) with float64 masses."""
     if top_p < 1.0:
