@@ -745,15 +745,17 @@ __global__ __launch_bounds__(512) void gemm_tile256_kernel(GemmParams p) {
 
 // ---------------------------------------------------------------------------------------------------------------
 // 256 x 256 x 64 tile, both operands staged by LDS-DMA (global_load_lds_dwordx4): no staging registers, no ds_write, the
-// copies of a K tile stay in flight across barriers for three to four phases, and the two waves of a SIMD take the matrix
+// copies of a K tile stay in flight across barriers for two to four phases, and the two waves of a SIMD take the matrix
 // core in turn.  Same wave grid and accumulator layout as gemm_tile256_kernel (2 x 4 waves, 128 x 64 per wave,
 // acc[8][4]), same MFMA chain per accumulator (so the same float32 sums, bit for bit), same epilogue.
 // Mistral-7B linears over 8 x 1024 rows, random bf16 operands, interleaved rounds in one process (tools/debug/
 // gemm_prefill_ab.py): 1.15 / 1.03 / 1.15 / 1.14 PFLOP/s (q|k|v, o, gate|up, down) on the register-staged tile,
-// 1.38 / 1.17 / 1.35 / 1.38 here.
+// 1.38 / 1.17 / 1.35 / 1.38 here with phases of 16 MFMAs; the float32-cache prompt's products (two terms of x) 617 / 2790 us
+// (q|k|v, gate|up) so, 613 / 2757 with the 32 of now.  What bounds it is power: the matrix core is busy three cycles of four at 1.6 to 1.75 GHz
+// (s_memtime against the wall clock in the loop; the same clock counts 2.2 in a light kernel).
 //
-// LDS: two K-tile buffers of 64 KiB, each four UNITS of 16 KiB -- a unit is what all 8 waves stage together in one
-// phase (two 1-KiB DMA instructions per wave):
+// LDS, all 160 KiB: three buffers of 32 KiB for A, two for B; each is two UNITS of 16 KiB -- a unit is what all 8 waves stage together
+// (two 1-KiB DMA instructions per wave):
 //     A-h0 / A-h1   rows {wm * 128 + h * 64 + [0, 64)} of the X tile (128 rows x 128 B), image row ir = wm * 64 + r
 //     B-k0 / B-k1   the 16 W row tiles of k block kb: 16 fragments of 1 KiB in tile-major order (a fragment read is one
 //                   contiguous KiB: conflict-free as it lies)
@@ -763,32 +765,30 @@ __global__ __launch_bounds__(512) void gemm_tile256_kernel(GemmParams p) {
 // -- every lane group of a ds_read_b128 fragment read ({0-3, 12-15, 20-27}, ... : 16 rows x one or two q) hits 16
 // different 16-byte columns (checked exhaustively), and the 8 lanes that fill a row fetch its whole 128-byte line.
 //
-// Schedule (ping-pong).  A K tile is four phases of 16 MFMAs per wave: (k block, row half) = (0,0) (0,1) (1,0) (1,1).  A
-// phase is  [reads of ITS fragments, stage one unit, s_waitcnt lgkmcnt(0), s_waitcnt vmcnt(N)] s_barrier [16 MFMAs] s_barrier;
+// Schedule (ping-pong).  A K tile is two phases of 32 MFMAs per wave, one per k block.  A phase is
+//     [reads of ITS fragments, stage two units, s_waitcnt lgkmcnt(0), s_waitcnt vmcnt(8)] s_barrier [32 MFMAs] s_barrier;
 // waves 4..7 -- the second wave of every SIMD -- enter through one extra barrier (and waves 0..3 leave through one), so
 // every s_barrier pairs the end of one group's read section with the end of the other's MFMA section: while one wave of a
 // SIMD reads and issues its DMA, the other has the matrix core.  Reads come BEFORE the DMA issue: an LDS-DMA instruction
 // holds the wave's issue for 60..180 cycles (the CU's one address unit serves four waves at once), the fragments arrive
 // meanwhile.
-//   stage:  j=0: A-h1(t+1)   j=1: B-k0(t+2)   j=2: B-k1(t+1)   j=3: A-h0(t+2)
+//   stage:  j=0: A-h0(t+2), B-k1(t+1)     j=1: A-h1(t+2), B-k0(t+2)
 // Write-after-read: the reads a group issues in phase Q have completed at that group's next barrier (lgkmcnt(0)), both
 // groups' two barriers after phase Q began; a unit last read in phase Q is restaged in phase Q + 1 at the earliest
-// (A-h0: read (t,0) (t,2) -> (t,3); A-h1: (t,1) (t,3) -> (t+1,0); B-k0: (t,0) -> (t,1); B-k1: (t,2) -> (t+1,2)).
+// (A(t-1), whose buffer A(t+2) takes: (t-1, 1) -> (t, 0); B-k1(t-1): (t-1, 1) -> (t, 0); B-k0(t): (t, 0) -> (t, 1)).
 // Read-after-write: a wave's DMA has landed when its counted vmcnt wait says so, everybody's when both groups have passed
 // the barrier behind that wait -- waited for in the read section of phase W, first read in phase W + 1:
 //     unit          staged in     waited for in   first read in   DMAs issued since (may stay in flight)
-//     A-h1(t+1)     (t, j=0)      (t+1, j=0)      (t+1, j=1)      4 units -> vmcnt(8)
-//     B-k1(t+1)     (t, j=2)      (t+1, j=1)      (t+1, j=2)      3 units -> vmcnt(6)
-//     B-k0(t+2)     (t, j=1)      (t+1, j=3)      (t+2, j=0)      (in order: landed before A-h0(t+2))
-//     A-h0(t+2)     (t, j=3)      (t+1, j=3)      (t+2, j=0)      4 units -> vmcnt(8)
+//     A-h0(t+2)     (t, j=0)      (t+1, j=1)      (t+2, j=0)      (in order: landed before A-h1(t+2))
+//     B-k1(t+1)     (t, j=0)      (t+1, j=0)      (t+1, j=1)      4 units -> vmcnt(8)
+//     A-h1(t+2), B-k0(t+2)  (t, j=1)  (t+1, j=1)  (t+2, j=0)      4 units -> vmcnt(8)
 // (vmcnt counts in order, and these DMAs are the loop's only vector-memory instructions.)  Past the last tile the stages
 // repeat the last tile's sources -- straight-line, the counts stay what the table says -- into units nobody reads again.
-// Measured and dropped (same tool, same box; the numbers are q|k|v / down): lockstep phases with the next phase's
+// Measured and dropped with phases of 16 MFMAs (q|k|v / down): lockstep phases with the next phase's
 // fragments read one phase ahead and ONE barrier per phase 1.26 / 1.25 PFLOP/s; this ping-pong with the DMA issued in
-// front of the reads 1.29 / 1.30; the DMA issued at the head of the MFMA section 1.25 / 1.24; the units going round
-// rings of five slots (all 160 KiB, every unit staged a tile earlier: five to seven phases in flight) 1.26 / 1.27 -- the
-// copies' latency is covered with two buffers, what counts is the length of the read section; no s_setprio: the same.
+// front of the reads 1.29 / 1.30; the DMA issued at the head of the MFMA section 1.25 / 1.24; no s_setprio: the same.
 constexpr int DMA_BUF = 65536, DMA_UNIT = 16384;
+constexpr int DMA256_B = 6 * DMA_UNIT, DMA256_LDS = 10 * DMA_UNIT;
 
 __device__ __forceinline__ void dma_kib(const void* gsrc, unsigned lds_dst) {
   unsigned keep;
@@ -873,18 +873,16 @@ __global__ __launch_bounds__(512) void gemm_dma256_kernel(GemmParams p) {
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) dst[nt] = *(const lds_u32x4_t*)(size_t)(b_lane + off + nt * 1024);
   };
-  // tile t in buffer t & 1 = [A-h0][A-h1][B-k0][B-k1]
-  auto stage_a = [&](int t, int h) { stage_a_at(t, h, (t & 1) * DMA_BUF + h * DMA_UNIT); };
-  auto stage_b = [&](int t, int kb) { stage_b_at(t, kb, (t & 1) * DMA_BUF + (2 + kb) * DMA_UNIT); };
-  auto a_frags = [&](int t, int kb, int h, u32x4 (&dst)[4]) { a_frags_at((t & 1) * DMA_BUF + h * DMA_UNIT, kb, dst); };
-  auto b_frags = [&](int t, int kb, u32x4 (&dst)[4]) { b_frags_at((t & 1) * DMA_BUF + (2 + kb) * DMA_UNIT, dst); };
+  // A of tile t in buffer t mod 3 = [A-h0][A-h1], B behind them in buffer t & 1 = [B-k0][B-k1]
+  auto stage_b = [&](int t, int kb) { stage_b_at(t, kb, DMA256_B + (t & 1) * (2 * DMA_UNIT) + kb * DMA_UNIT); };
+  auto b_frags = [&](int t, int kb, u32x4 (&dst)[4]) { b_frags_at(DMA256_B + (t & 1) * (2 * DMA_UNIT) + kb * DMA_UNIT, dst); };
 
   f32x4 acc[8][4];
 #pragma unroll
   for (int i = 0; i < 8; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  u32x4 af[1][4], bf[2][4];
+  u32x4 af[2][4], bf[4];
 
   auto mma = [&](int h, const u32x4 (&a)[4], const u32x4 (&b)[4]) {
 #pragma unroll
@@ -894,8 +892,9 @@ __global__ __launch_bounds__(512) void gemm_dma256_kernel(GemmParams p) {
   };
 
   {
-    // prologue: tile 0 whole and what the phases of tiles -2 / -1 would have staged, in their order
-    stage_b(0, 0); stage_a(0, 0); stage_a(0, 1); stage_b(1, 0); stage_b(0, 1); stage_a(1, 0);
+    // prologue: tile 0 and what the phases of tiles -2 / -1 would have staged, in their order
+    stage_a_at(0, 0, 0); stage_a_at(0, 1, DMA_UNIT); stage_b(0, 0);
+    stage_a_at(1, 0, 2 * DMA_UNIT); stage_b(0, 1); stage_a_at(1, 1, 3 * DMA_UNIT); stage_b(1, 0);
     asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
     asm volatile("s_barrier" ::: "memory");
     if (wave >= 4) asm volatile("s_barrier" ::: "memory");
@@ -905,23 +904,20 @@ __global__ __launch_bounds__(512) void gemm_dma256_kernel(GemmParams p) {
 #define PP_MMA_DONE() do { __builtin_amdgcn_sched_barrier(0); __builtin_amdgcn_s_setprio(0); asm volatile("s_barrier" ::: "memory"); \
       __builtin_amdgcn_sched_barrier(0); } while (0)
 #define PP_ORDER() __builtin_amdgcn_sched_barrier(0)
+    unsigned ra = 0, sa = 4 * DMA_UNIT;                            // A of tile t, of tile t + 2
     for (int t = 0; t < nk; ++t) {
-      b_frags(t, 0, bf[0]); a_frags(t, 0, 0, af[0]); PP_ORDER(); stage_a(t + 1, 1);
+      b_frags(t, 0, bf); a_frags_at(ra, 0, af[0]); a_frags_at(ra + DMA_UNIT, 0, af[1]); PP_ORDER();
+      stage_a_at(t + 2, 0, sa); stage_b(t + 1, 1);
       PP_READS_DONE(8);
-      mma(0, af[0], bf[0]);
+      mma(0, af[0], bf); mma(1, af[1], bf);
       PP_MMA_DONE();
-      a_frags(t, 0, 1, af[0]); PP_ORDER(); stage_b(t + 2, 0);
-      PP_READS_DONE(6);
-      mma(1, af[0], bf[0]);
-      PP_MMA_DONE();
-      b_frags(t, 1, bf[1]); a_frags(t, 1, 0, af[0]); PP_ORDER(); stage_b(t + 1, 1);
-      PP_READS_DONE(-1);
-      mma(0, af[0], bf[1]);
-      PP_MMA_DONE();
-      a_frags(t, 1, 1, af[0]); PP_ORDER(); stage_a(t + 2, 0);
+      b_frags(t, 1, bf); a_frags_at(ra, 1, af[0]); a_frags_at(ra + DMA_UNIT, 1, af[1]); PP_ORDER();
+      stage_a_at(t + 2, 1, sa + DMA_UNIT); stage_b(t + 2, 0);
       PP_READS_DONE(8);
-      mma(1, af[0], bf[1]);
+      mma(0, af[0], bf); mma(1, af[1], bf);
       PP_MMA_DONE();
+      ra = ra == 4 * DMA_UNIT ? 0 : ra + 2 * DMA_UNIT;
+      sa = sa == 4 * DMA_UNIT ? 0 : sa + 2 * DMA_UNIT;
     }
 #undef PP_ORDER
 #undef PP_READS_DONE
@@ -1971,8 +1967,8 @@ int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStr
 #endif
 #define GO256(T, S, LG) do { \
       if (use_dma) { auto k = gemm_dma256_kernel<T, S, false, LG>; \
-        MI_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * DMA_BUF)); \
-        hipLaunchKernelGGL(k, grid2, block2, 2 * DMA_BUF, st, p); } \
+        MI_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, DMA256_LDS)); \
+        hipLaunchKernelGGL(k, grid2, block2, DMA256_LDS, st, p); } \
       GO256_M32(T, S) \
       else if (b_in_lds) { auto k = gemm_tile256_kernel<T, S, false, LG>; \
         MI_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, LDS2_BYTES)); \
@@ -2032,8 +2028,8 @@ int launch_gemm_grouped(const GroupedGemm& g, hipStream_t st) {
     if (g.W.K < 2 * BK || (last && g.last.K < 2 * BK)) return fail(MI_ERR_UNSUPPORTED, "gemm_grouped: the 256 x 256 tile needs two K tiles");
     const dim3 grid(g.max_tiles, (cols + (g.swiglu ? 128 : BN2) - 1) / (g.swiglu ? 128 : BN2)), block(512);
     auto go = [&](auto k) -> int {
-      MI_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * DMA_BUF));
-      hipLaunchKernelGGL(k, grid, block, 2 * DMA_BUF, st, p);
+      MI_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, DMA256_LDS));
+      hipLaunchKernelGGL(k, grid, block, DMA256_LDS, st, p);
       MI_HIP(hipGetLastError());
       return MI_OK;
     };
