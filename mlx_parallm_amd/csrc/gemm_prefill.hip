@@ -1798,8 +1798,12 @@ static bool gemm_prefill_pays_codes(const LinearW& W, const GemvCall& c, size_t 
   long blocks = 0;
   if (!codes_plan(W, c, rows, terms * W.K, terms, splitk_cap > 0, splitk_cap, p, blocks))
     return (c.rnd == RND_NONE && c.epi != EPI_STORE_F32) || gemm_prefill_pays(true, false, c.rnd != RND_NONE, rows);
-  const double mw = (double)W.N * W.K / (1 << 20), gemm = tail_us(blocks, p.mb > 0 ? p.tail : blocks, (p.ka + p.kb) / BK, p.ksplit, gemv_cu_count());
-  return 5.0 + (W.codes.codes != nullptr ? 0.0 : 0.65 * mw) + gemm < (double)((rows + 31) / 32) * (11.0 + 0.30 * mw + 0.5 * W.K / 1024);
+  // (the slices as they were when this was fitted; those of a last round alone, tail_plan, are no slower)
+  const int ks = c.epi != EPI_SWIGLU && splitk_cap > 0 && W.N % 4 == 0 ? split256(blocks, (p.ka + p.kb) / BK, rows * W.N * sizeof(float), splitk_cap) : 1;
+  const int ncu = gemv_cu_count(), tiles = ((p.ka + p.kb) / BK + ks - 1) / ks;
+  const double mw = (double)W.N * W.K / (1 << 20), rounds = (double)((blocks * ks + ncu - 1) / ncu);
+  const double reduce = ks > 1 ? 2e-6 * ks * rows * W.N : 0.0;
+  return 12.0 + (W.codes.codes != nullptr ? 0.0 : 0.65 * mw) + 1.35 * rounds * tiles + reduce < (double)((rows + 31) / 32) * (11.0 + 0.30 * mw + 0.5 * W.K / 1024);
 }
 
 bool gemm_prefill_on_codes(const LinearW& W, const GemvCall& c, size_t rows) {
