@@ -408,6 +408,7 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
     // prefill: one MFMA tile GEMM over all rows (the RMSNorm runs as its own row-wise kernel)
     Prof pr(e, prof);
     const GemvCall c_in = c;                 // (the LoRA down-projection reads the caller's x and normalises on its own)
+    bool norm_sums = false;                  // multiplied as codes: the norm is launched with the sums of its groups (rmsnorm_row_block_kernel)
     if (c.act == MI_F32) {      // PagedKVCache mode: (norm +) exact three-way split of x, then the same tile GEMM over 3 K
       const size_t need = split3_bytes(rows, KT);
       if (need > e->xs_cap) {
@@ -435,12 +436,18 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
       c.split_out = c.split_out && gemm_prefill_split_out(f.W, c, rows);
       e->act_split = c.split_out != 0;
     } else if (c.pro == PRO_NORM) {    // (one workgroup per row also here: one L2 round trip per row instead of a wave's 16)
-      MI_TRY(launch_rmsnorm_rows(c.x, c.ldx, c.norm_w, e->xn, KT, (int)rows, KT, c.eps, c.act, e->stream, true));
-      c.x = e->xn; c.ldx = KT; c.pro = PRO_NONE;
+      GemvCall cn = c;
+      cn.x = e->xn; cn.ldx = KT; cn.pro = PRO_NONE;
+      norm_sums = quant && KT <= 8192 && gemm_prefill_on_codes(f.W, cn, rows);
+      if (norm_sums) c.norm_out = e->xn;
+      else {
+        MI_TRY(launch_rmsnorm_rows(c.x, c.ldx, c.norm_w, e->xn, KT, (int)rows, KT, c.eps, c.act, e->stream, true));
+        c = cn;
+      }
     }
     // logits of many positions against a quantised matrix: 32768 outputs at a time, so that the copy below stays within 4 x 32768 x K bytes.  The
     // kernel is chosen for all of them: a last piece of few columns is no reason for the [hi | lo] copy
-    c.codes = quant && gemm_prefill_on_codes(f.W, c, rows);
+    c.codes = norm_sums || (quant && gemm_prefill_on_codes(f.W, c, rows));
     const int ncol = (wk_is_quant(f.W.wk) && c.epi == EPI_STORE_F32) ? std::min(f.W.N, 32768) : f.W.N;
     void* scratch = nullptr;
     if (wk_is_quant(f.W.wk)) {               // the GEMM multiplies by 16-bit codes, or a [hi | lo] 16-bit copy, made on the fly
@@ -471,6 +478,7 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
       }
       MI_TRY(launch_gemm_prefill(part, cp, rows, e->stream, scratch, rows < 4096 ? e->gk_ws : nullptr, e->gk_cap));
     }
+    if (norm_sums) { c.x = e->xn; c.ldx = KT; c.pro = PRO_NONE; }
     if (f.W.lora_b[0] != nullptr || f.W.lora_b[1] != nullptr) {   // y = T(y + T(scale (x A) B)) on the adapted columns
       GemvCall cl = c.act == MI_F32 ? c_in : c;
       cl.M = (int)rows;

@@ -1234,7 +1234,16 @@ __global__ __launch_bounds__(512) void tail_reduce_kernel(GemmParams p) {
 }
 
 // The group sums of x for the kernel above: row m -> `parts` terms of G columns each (kernels.h: codes16_sum_part; hi + mid + lo = the float32 sum
-// of the group's 64 values over x's `terms` of K columns), zeros up to kb.  One workgroup per row.
+// of the group's 64 values over x's `terms` of K columns), zeros up to kb.  One workgroup per row.  (A norm in front makes them on its way:
+// rmsnorm_row_block_kernel.)
+__device__ __forceinline__ void store_group_sums(const float* gsum, int G, uint16_t* xs_row, int kb, int big_first) {
+  for (int c = threadIdx.x; c < kb; c += 256) {
+    const int term = c / G, grp = c - term * G;
+    const float v = term < CODES16_TERMS ? bf16_part(gsum[grp], codes16_sum_part(big_first ? CODES16_TERMS - 1 - term : term)) : 0.f;
+    xs_row[c] = __builtin_bit_cast(uint16_t, (bf16)v);
+  }
+}
+
 template <typename AT>
 __global__ __launch_bounds__(256) void group_sums_kernel(const AT* x, int ldx, int terms, int K, uint16_t* xs, int kb, int big_first) {
   extern __shared__ float gsum[];
@@ -1252,11 +1261,7 @@ __global__ __launch_bounds__(256) void group_sums_kernel(const AT* x, int ldx, i
     if ((tid & 7) == 0) gsum[k >> 6] = s;
   }
   __syncthreads();
-  for (int c = tid; c < kb; c += 256) {
-    const int term = c / G, grp = c - term * G;
-    const float v = term < CODES16_TERMS ? bf16_part(gsum[grp], codes16_sum_part(big_first ? CODES16_TERMS - 1 - term : term)) : 0.f;
-    xs[(size_t)row * kb + c] = __builtin_bit_cast(uint16_t, (bf16)v);
-  }
+  store_group_sums(gsum, G, xs + (size_t)row * kb, kb, big_first);
 }
 
 
@@ -1455,9 +1460,12 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const AT* x, int ldx,
 // The same operator with one 256-thread workgroup per row and the row held in registers (NP 16-byte pieces per
 // thread): for the few rows of a decode step (gemm_skinny.hip), where one wave per row means a handful of
 // workgroups walking their rows in dependent L2 round trips (9 us at 32 x 4096; this one: one round trip).
-template <typename AT, int NP>
+// SUMS: in front of a matrix that is multiplied as codes, with what group_sums_kernel would read back for (its additions, the same bits;
+// 700 x 4096: 5.5 us and 5.9 as two launches, 5.9 as one).
+template <typename AT, int NP, bool SUMS>
 __global__ __launch_bounds__(256) void rmsnorm_row_block_kernel(const AT* x, int ldx, const AT* w, AT* out, int ldo, int H,
-                                                                float eps) {
+                                                                float eps, uint16_t* xs, int kb) {
+  __shared__ float gsum[SUMS ? NP * 32 : 1];
   __shared__ float part[4];
   const int row = blockIdx.x, tid = threadIdx.x;
   const AT* xr = x + (size_t)row * ldx;
@@ -1494,7 +1502,18 @@ __global__ __launch_bounds__(256) void rmsnorm_row_block_kernel(const AT* x, int
         e[j] = (AT)((float)xn * (float)we[j]);
       }
       *(u32x4*)(out + (size_t)row * ldo + k) = v[i];
+      if constexpr (SUMS) {                                      // (H is a multiple of 64: a group's eight lanes are all here)
+        float s = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s += (float)e[j];
+        s = lane8_sum(s);
+        if ((tid & 7) == 0) gsum[k >> 6] = s;
+      }
     }
+  }
+  if constexpr (SUMS) {
+    __syncthreads();
+    store_group_sums(gsum, H / 64, xs + (size_t)row * kb, kb, 1);
   }
 }
 
@@ -1601,10 +1620,11 @@ __global__ __launch_bounds__(256) void split3_rows_kernel(const float* x, int ld
 }
 
 template <typename AT>
-int launch_rmsnorm_block(const void* x, int ldx, const void* w, void* out, int ldo, int rows, int H, float eps, hipStream_t st) {
+int launch_rmsnorm_block(const void* x, int ldx, const void* w, void* out, int ldo, int rows, int H, float eps, hipStream_t st, uint16_t* xs = nullptr, int kb = 0) {
   const int np = (H / 8 + 255) / 256;
   const dim3 grid(rows), block(256);
-#define GO(NP) hipLaunchKernelGGL((rmsnorm_row_block_kernel<AT, NP>), grid, block, 0, st, (const AT*)x, ldx, (const AT*)w, (AT*)out, ldo, H, eps)
+#define GO(NP) do { if (xs != nullptr) hipLaunchKernelGGL((rmsnorm_row_block_kernel<AT, NP, true>), grid, block, 0, st, (const AT*)x, ldx, (const AT*)w, (AT*)out, ldo, H, eps, xs, kb); \
+    else hipLaunchKernelGGL((rmsnorm_row_block_kernel<AT, NP, false>), grid, block, 0, st, (const AT*)x, ldx, (const AT*)w, (AT*)out, ldo, H, eps, xs, kb); } while (0)
   switch (np) {
     case 1: GO(1); break;
     case 2: GO(2); break;
@@ -1844,7 +1864,7 @@ static int launch_gemm_codes(const LinearW& W, const GemvCall& c, size_t rows, h
   const int terms = x32 ? c.ldx / W.K : 1, ncols = sw ? c.pair_offset : W.N;
   GemmParams p{};
   long blocks = 0;
-  if (!codes_plan(W, c, rows, c.ldx, terms, splitk_ws != nullptr, splitk_cap, p, blocks)) return MI_OK;
+  if (!codes_plan(W, c, rows, c.pro == PRO_NORM ? W.K : c.ldx, terms, splitk_ws != nullptr, splitk_cap, p, blocks)) return MI_OK;
   p.x = c.x;
   p.ws = (float*)splitk_ws;
   char* d = (char*)scratch;
@@ -1856,7 +1876,10 @@ static int launch_gemm_codes(const LinearW& W, const GemvCall& c, size_t rows, h
   }
   uint16_t* xs = (uint16_t*)(d + codes16_bytes(W.N, W.K));
   p.xs = xs;
-  if (c.act == MI_F16) hipLaunchKernelGGL(group_sums_kernel<f16>, dim3((unsigned)rows), dim3(256), p.G * sizeof(float), st, (const f16*)c.x, c.ldx, terms, W.K, xs, p.kb, terms == 1);
+  if (c.pro == PRO_NORM) {
+    MI_TRY((c.act == MI_F16 ? launch_rmsnorm_block<f16> : launch_rmsnorm_block<bf16>)(c.x, c.ldx, c.norm_w, c.norm_out, W.K, (int)rows, W.K, c.eps, st, xs, p.kb));
+    p.x = c.norm_out; p.ldx = W.K;
+  } else if (c.act == MI_F16) hipLaunchKernelGGL(group_sums_kernel<f16>, dim3((unsigned)rows), dim3(256), p.G * sizeof(float), st, (const f16*)c.x, c.ldx, terms, W.K, xs, p.kb, terms == 1);
   else hipLaunchKernelGGL(group_sums_kernel<bf16>, dim3((unsigned)rows), dim3(256), p.G * sizeof(float), st, (const bf16*)c.x, c.ldx, terms, W.K, xs, p.kb, terms == 1);
   MI_HIP(hipGetLastError());
   p.out32 = x32 || c.out32; p.rnd = x32 ? c.rnd : RND_NONE;
@@ -1895,7 +1918,7 @@ bool gemm_prefill_split_out(const LinearW& W, const GemvCall& c, size_t rows) {
 
 int launch_gemm_prefill(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st, void* scratch, void* splitk_ws,
                         size_t splitk_cap) {
-  if (c.pro != PRO_NONE) return fail(MI_ERR_INVALID, "gemm_prefill: normalise the rows first");
+  if (c.pro != PRO_NONE && !(c.norm_out != nullptr && c.codes && c.act != MI_F32 && W.K <= 8192)) return fail(MI_ERR_INVALID, "gemm_prefill: normalise the rows first");
   GemmParams p{};
   p.ksplit = 1;
   p.x = c.x; p.ldx = c.ldx; p.M = (int)rows; p.w = W.w; p.N = W.N; p.K = W.K; p.ka = W.K; p.kw = W.K;

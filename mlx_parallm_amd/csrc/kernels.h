@@ -49,6 +49,7 @@ struct GemvCall {
   int pro = PRO_NONE;
   const void* norm_w = nullptr;  // [K] RMSNorm weight (PRO_NORM)
   float eps = 0.f;
+  void* norm_out = nullptr; // [M][K], PRO_NORM in front of gemm_prefill.hip's codes: the normalised rows, left by the launch that adds up their groups
   int epi = EPI_STORE;
   void* out = nullptr;
   int ldo = 0;

@@ -306,3 +306,45 @@ def test_tiles_of_a_last_round_in_slices(act, bits, M, N, K, epi):
     o = host(out)
     assert np.all(o[M:] == 7.0) and np.array_equal(o[M - 1], o[5])
     _assert_close(o[:M][rows], want, act, scale=float(np.abs(y).max()))
+
+
+@pytest.mark.parametrize("bits,act,H,V", [(4, "bfloat16", 384, 36864), (8, "float16", 2112, 6656), (4, "float16", 4224, 1680), (8, "bfloat16", 8192, 832), (4, "bfloat16", 8320, 832)])
+def test_norm_and_group_sums_in_one_launch(bits, act, H, V):
+    """The norm in front of a product on codes leaves the sums of its groups (one to four pieces of a row a thread, the last ones partly filled; above 8192 columns a launch
+    of its own; logits in two pieces of columns).  Layers that add nothing, so the logits of every position are W_hat . norm(embedding): two roundings to 16 bits (the
+    logits' and the embedding's own) of 2^-9 (2^-12) in root mean square at most; a sum that went astray is off by the groups' means, four deviations."""
+    from mlx_parallm_amd.engine import Engine
+
+    cfg = dict(model_type="llama", hidden_size=H, num_hidden_layers=1, num_attention_heads=2, num_key_value_heads=2, head_dim=64, intermediate_size=128, vocab_size=V,
+               rms_norm_eps=1e-5, rope_theta=10000.0, tie_word_embeddings=False, max_position_embeddings=512, quantization={"bits": bits, "group_size": 64})
+    e = Engine(cfg, device=0, max_positions=512, act_dtype=act)
+    rng = np.random.default_rng(H)
+
+    def put(name, n, k, zero=False):
+        w = (rng.standard_normal((n, k // 64, 64)) + 4 * rng.standard_normal((n, k // 64, 1))).astype(np.float32).reshape(n, k) * 0.05
+        packed, s, b = ref_quant.quantize(round_to(w, act), 64, bits, act)
+        if zero:
+            s, b = np.zeros_like(s), np.zeros_like(b)
+        for part, t in ((".weight", dev_u32(packed)), (".scales", dev(s, act)), (".biases", dev(b, act))):
+            e.set_tensor(name + part, t)
+        return ref_quant.dequantize(packed, s, b, 64, bits)
+    emb = put("model.embed_tokens", V, H)
+    head = put("lm_head", V, H)
+    p = "model.layers.0."
+    for n, rows, cols in (("self_attn.q_proj", 128, H), ("self_attn.k_proj", 128, H), ("self_attn.v_proj", 128, H), ("mlp.gate_proj", 128, H), ("mlp.up_proj", 128, H)):
+        put(p + n, rows, cols)
+    put(p + "self_attn.o_proj", H, 128, zero=True)
+    put(p + "mlp.down_proj", H, 128, zero=True)
+    nw = round_to(1.0 + 0.2 * rng.standard_normal(H).astype(np.float32), act)
+    for n in (p + "input_layernorm", p + "post_attention_layernorm", "model.norm"):
+        e.set_tensor(n + ".weight", dev(nw, act))
+    e.finalize()
+    toks = rng.integers(0, V, (1, 320)).astype(np.int32)
+    got = np.array(e.forward(toks, e.new_kv(1, capacity=384), all_positions=True), dtype=np.float64)[0]
+    e.close()
+    x = np.asarray(round_to(emb[toks[0]], act), dtype=np.float64)
+    xn = round_to((x / np.sqrt((x * x).mean(-1, keepdims=True) + 1e-5)).astype(np.float32), act)
+    xn = round_to(np.asarray(xn, dtype=np.float32) * np.asarray(nw, dtype=np.float32), act)
+    want = (torch.from_numpy(np.asarray(xn, dtype=np.float64)) @ torch.from_numpy(np.asarray(head, dtype=np.float64)).T).numpy()
+    off = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert off <= 2.0 * 2.0 ** (-9 if act == "bfloat16" else -12), off
