@@ -86,9 +86,9 @@ int mi_op_gemv_bench(const mi_op_linear* w, const mi_op_gemv_args* a, int iters,
 /* the split-K weight-streaming GEMM the engine uses for decode steps of 9..128 rows (int4 / int8 weights: 1..128), on its own:
  * a->M in that range, a->pro = MI_PRO_NONE, tile-major 16-bit, int4 or int8 (group 64) weights.  ksplit 0 = the library's
  * cost model (returned in *ksplit_used); iters >= 1 also times that many back-to-back launches into *avg_ms.
- * wide int4 matrices above 16 rows with ksplit <= 0 run gemm_q4.hip (x prepared once per launch, K split over the waves of a workgroup;
- * a->pro may then be MI_PRO_NORM); ksplit < 0 forces it, and its plan, for tests and A/B runs: -(row_tiles | ksplit << 11), 0 = the cost model's
- * choice; what the fields between carried (tile units, K lanes, staging waves) is fixed by the kernel and is ignored. */
+ * wide int4 matrices above 16 rows, and narrow ones where its rule says so, with ksplit <= 0 run gemm_q4.hip (x prepared once per launch, K split over the
+ * waves of a workgroup; in front of a wide matrix a->pro may then be MI_PRO_NORM); ksplit < 0 forces it, and its plan, for tests and A/B runs:
+ * -(row_tiles | ksplit << 11 | 1 << 15 for the narrow matrices' kernel), 0 = the cost model's choice; what the fields between carried (tile units, K lanes, staging waves) is fixed by the kernel and is ignored. */
 int mi_op_gemm_skinny(const mi_op_linear* w, const mi_op_gemv_args* a, int ksplit, int* ksplit_used, int iters,
                       float* avg_ms);
 /* gemm_prefill.hip on its own: the tile GEMM of the prefill call (generate_step's first model call, utils.py:243-262: every
