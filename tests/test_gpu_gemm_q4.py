@@ -94,3 +94,18 @@ def test_narrow_matrices(act, M, N, K, epi):
         g, u = want[:, :cols], want[:, cols:]
         want = round_to(round_to(g * round_to(1.0 / (1.0 + np.exp(-g.astype(np.float64))), act), act) * u, act)
     _assert_close(outs[0][:M], want, act)
+
+
+@pytest.mark.parametrize("act", ["bfloat16", "float16"])
+@pytest.mark.parametrize("M,K", [(17, 128), (128, 2048), (33, 2176), (64, 4224), (48, 8192), (20, 8320)])
+def test_norm_in_front_by_pieces_of_the_row(act, M, K):
+    """The preparation with a norm: one to four pieces of a row a thread, the last ones partly filled, and the loop above 8192 columns."""
+    rng = np.random.default_rng(K)
+    ol, w, keep = _weight(4, act, 48, K, rng)
+    x = round_to(rng.standard_normal((M, K)).astype(np.float32), act)
+    nw = round_to(1.0 + 0.1 * rng.standard_normal(K).astype(np.float32), act)
+    xd, nwd = dev(x, act), dev(nw, act)
+    out = torch.full((M + 2, 48), 7.0, dtype=xd.dtype, device="cuda")
+    gemm_skinny(ol, xd, M, act, epi=L.EPI_STORE, out=out, ldo=48, norm_w=nwd, eps=1e-5, ksplit=q4_force(rows=1))
+    assert np.all(host(out)[M:] == 7.0)
+    _assert_close(host(out)[:M], round_to(matmul_nt(ref_model.rms_norm(x, act, nw, act, 1e-5)[0], w), act), act)
