@@ -1001,9 +1001,10 @@ __global__ __launch_bounds__(512) void gemm_codes256_kernel(GemmParams p) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 2, wn = wave & 3;
   const int c16 = lane & 15, g = lane >> 4;
-  int bm = blockIdx.x, bn = blockIdx.y, z = 0, nz = 1;
+  int bm = blockIdx.x, bn = blockIdx.y, z = blockIdx.z, nz = gridDim.z;
   if (p.mb > 0) {                                               // (uniform) K slices of the last tiles alone
     int tile = blockIdx.x;
+    z = 0; nz = 1;
     if (tile >= p.tail) { const int u = tile - p.tail; nz = p.ksplit; tile = p.tail + u / nz; z = u - u / nz * nz; }
     bn = tile / p.mb; bm = tile - bn * p.mb;
     bm = __builtin_amdgcn_readfirstlane(bm); bn = __builtin_amdgcn_readfirstlane(bn); z = __builtin_amdgcn_readfirstlane(z); nz = __builtin_amdgcn_readfirstlane(nz);
@@ -1201,6 +1202,9 @@ __global__ __launch_bounds__(512) void gemm_codes256_kernel(GemmParams p) {
 #undef PP_READS_DONE
 #undef PP_MMA_DONE
 
+  if constexpr (!SWIGLU) {
+    if (gridDim.z > 1) { tile256_partial(p, acc, smem2, m0, bn, wave, lane); return; }
+  }
   if (nz > 1) {                                                  // (whole KiB, in the registers' order)
     f32x4* dst = (f32x4*)p.ws + (((size_t)(bn * p.mb + bm - p.tail) * nz + z) * 8 + wave) * (32 * 64) + lane;
 #pragma unroll
@@ -1760,6 +1764,36 @@ size_t gemm_prefill_scratch_bytes(const LinearW& W, size_t rows) {
   return std::max(dequant_hilo_bytes(W.N, W.K), codes16_bytes(W.N, W.K) + rows * codes16_bias_cols(W.K) * 2);
 }
 
+// us of a launch over `blocks` tiles of `nk` K tiles in rounds of one workgroup per CU, those from `tail` on as `ks` slices: a round 10 + 2 per K tile (float32 rows, whose three walks
+// find W and x in the caches: 1.35), what joins the slices 3 + their 256 KiB each at 4.9 TB/s (fitted: 6144 x 4096, 700 rows, 7 slices 66 + 23, 4096 x 14336 with 5 94 + 15,
+// 28672 x 4096 SwiGLU, unsplit, 277)
+static double tail_us(long blocks, long tail, int nk, int ks, double tile_us, int ncu) {
+  const auto rounds = [&](long n) { return (double)((n + ncu - 1) / ncu); };
+  const double full = rounds(tail) * (10.0 + tile_us * nk);
+  if (tail == blocks) return full;
+  const long t = blocks - tail;
+  return full + rounds(t * ks) * (10.0 + tile_us * ((nk + ks - 1) / ks)) + 3.0 + t * ks * 0.262144 / 4.9;
+}
+
+// K slices for the tiles of a last, partly filled round (all of them where there is only that round) of a call that split256 leaves whole: the cheapest by the line above, at least
+// 8 K tiles a slice.  Whole columns of tiles: all rows of a call have one order of sums.  700 rows, us: 28672 x 4096 SwiGLU (336 tiles, the last 81 in three) 277 -> 200 + 16.
+// Calls that split256 splits keep its slices.  Fewer of them, or of the last tiles alone, are faster (6144 x 4096, 700 rows: three for seven 54 + 13 us against 66 + 23), but an output's
+// chain of additions is as long as its slice: float32 rows 1.8e-7 from 64 bits in 2-norm for 1.2e-7, and of 16-bit results 14 % more rounded the other way.
+// Float32 rows take three slices or more: with two, x's largest term, which is walked last, stays one chain and the join is a rounding more (2-norm from 64 bits against the unsplit call,
+// 28672 x 4096, 64 rows 1.008, 12800 x 2048, 300 rows 1.02, 6144 x 1024, 1024 rows 1.03; three to eight slices 0.78 to 1.00 over 4 shapes and 7 row counts).
+static void tail_plan(long mb, long blocks, int nk, bool x3, size_t cap, GemmParams& p) {
+  const int ncu = gemv_cu_count();
+  const double tile_us = x3 ? 1.35 : 2.0;
+  double best = tail_us(blocks, blocks, nk, 1, tile_us, ncu) - (x3 ? 10.0 : 5.0);       // (what the line is sure of)
+  for (const long tail : {blocks / ncu * ncu / mb * mb, 0L}) {
+    for (int ks = x3 ? 3 : 2; ks <= 8 && nk / ks >= 8 && (size_t)(blocks - tail) * ks * (BM2 * BN2 * 4) <= cap; ++ks) {
+      if (tail == blocks) break;
+      const double t = tail_us(blocks, tail, nk, ks, tile_us, ncu);
+      if (t < best) { best = t; p.mb = (int)mb; p.tail = (int)tail; p.ksplit = ks; }
+    }
+  }
+}
+
 // Does gemm_codes256_kernel take this call of a quantised matrix?  It halves the products and the copy of the [hi | lo] form and costs a launch (the
 // group sums), the bias columns and a 256-row tile where the other has 128.  Whole calls, us, codes and [hi | lo], bf16 rows: 4096 x 4096 x
 // 129 rows 43 / 50, 28672 x 4096 SwiGLU 129 rows 196 / 317 and 700 rows 348 / 494, 4096 x 14336 x 700 144 / 221; 2048 x 5632 x 192 44 / 41, 256 44 / 50;
@@ -1769,31 +1803,6 @@ size_t gemm_prefill_scratch_bytes(const LinearW& W, size_t rows) {
 // mean exceeds 3 of its deviations.  2-norm from 64 bits, 1024 x 1024, 256 rows, means of 0 / 4 / 12 deviations: pair 1.8e-7 / 7.0e-7 / 1.9e-6,
 // streaming 3.3e-7 / 1.3e-7 / 1.0e-7, here 0.8e-7 / 0.7e-7 / 0.7e-7 (2048 x 4096, 160 rows: 3.7e-7 / 7.7e-7 / 1.9e-6, 3.4e-7 / 1.4e-7 / 1.2e-7, 1.2e-7 / 0.8e-7 / 0.8e-7);
 // us, streaming / here: 129 rows 59 / 29, 1365 rows 511 / 40.
-// us of a launch over `blocks` tiles of `nk` K tiles in rounds of one workgroup per CU, those from `tail` on as `ks` slices: a round 10 + 2 per K tile, what joins the slices
-// 3 + their 256 KiB each at 4.9 TB/s (fitted: 6144 x 4096, 700 rows, 7 slices 66 + 23, 4096 x 14336 with 5 94 + 15, 28672 x 4096 SwiGLU, unsplit, 277)
-static double tail_us(long blocks, long tail, int nk, int ks, int ncu) {
-  const auto rounds = [&](long n) { return (double)((n + ncu - 1) / ncu); };
-  const double full = rounds(tail) * (10.0 + 2.0 * nk);
-  if (tail == blocks) return full;
-  const long t = blocks - tail;
-  return full + rounds(t * ks) * (10.0 + 2.0 * ((nk + ks - 1) / ks)) + 3.0 + t * ks * 0.262144 / 4.9;
-}
-
-// K slices for the tiles of a last, partly filled round (all of them where there is only that round): the cheapest by the line above, at least 8 K tiles a slice.  Whole
-// columns of tiles: all rows of a call have one order of sums.  700 rows, us: 28672 x 4096 SwiGLU (336 tiles, the last 81 in three) 277 -> 200 + 16, 6144 x 4096 (72 tiles: three slices
-// for seven) 89 -> 54 + 13, 32000 x 4096 logits 284 -> 235 + 18.
-static void tail_plan(long mb, long blocks, int nk, size_t cap, GemmParams& p) {
-  const int ncu = gemv_cu_count();
-  double best = tail_us(blocks, blocks, nk, 1, ncu) - 5.0;       // (what the line is sure of)
-  for (const long tail : {blocks / ncu * ncu / mb * mb, 0L}) {
-    for (int ks = 2; ks <= 8 && nk / ks >= 8 && (size_t)(blocks - tail) * ks * (BM2 * BN2 * 4) <= cap; ++ks) {
-      if (tail == blocks) break;
-      const double t = tail_us(blocks, tail, nk, ks, ncu);
-      if (t < best) { best = t; p.mb = (int)mb; p.tail = (int)tail; p.ksplit = ks; }
-    }
-  }
-}
-
 static bool codes_plan(const LinearW& W, const GemvCall& c, size_t rows, int ldx, int terms, bool split_ok, size_t cap, GemmParams& p, long& blocks) {
   const bool sw = c.epi == EPI_SWIGLU;
   const int ncols = sw ? c.pair_offset : W.N;
@@ -1803,8 +1812,8 @@ static bool codes_plan(const LinearW& W, const GemvCall& c, size_t rows, int ldx
   p.M = (int)rows; p.N = W.N; p.kw = W.K; p.ka = p.K = terms * W.K; p.ldx = ldx; p.G = W.K / 64;
   p.kb = codes16_bias_cols(W.K);
   blocks = (long)((rows + BM2 - 1) / BM2) * ((ncols + (sw ? 128 : BN2) - 1) / (sw ? 128 : BN2));
-  p.ksplit = 1;
-  if (split_ok) tail_plan((long)((rows + BM2 - 1) / BM2), blocks, (p.ka + p.kb) / BK, cap, p);
+  p.ksplit = !sw && split_ok && W.N % 4 == 0 ? split256(blocks, (p.ka + p.kb) / BK, rows * W.N * sizeof(float), cap) : 1;
+  if (split_ok && p.ksplit == 1) tail_plan((long)((rows + BM2 - 1) / BM2), blocks, (p.ka + p.kb) / BK, terms > 1, cap, p);
   return true;
 }
 
@@ -1889,12 +1898,13 @@ static int launch_gemm_codes(const LinearW& W, const GemvCall& c, size_t rows, h
     if (!x32) { p.out32 = 1; p.rnd = c.act == MI_BF16 ? RND_BF16 : RND_F16; }
   }
   p.strips = strips_ok(p);
-  const dim3 grid = p.mb > 0 ? dim3((unsigned)(p.tail + (blocks - p.tail) * p.ksplit)) : dim3((unsigned)((rows + BM2 - 1) / BM2), (ncols + (sw ? 128 : BN2) - 1) / (sw ? 128 : BN2));
+  const dim3 grid = p.mb > 0 ? dim3((unsigned)(p.tail + (blocks - p.tail) * p.ksplit)) : dim3((unsigned)((rows + BM2 - 1) / BM2), (ncols + (sw ? 128 : BN2) - 1) / (sw ? 128 : BN2), p.ksplit);
   const bool rounded = p.rnd != RND_NONE;               // (float32 stores of values rounded to 16 bits: logits, and layer 0 of the float32-cache mode)
   if (terms > 1 && !rounded) MI_TRY((sw ? codes_launch<bf16, true, false, true> : codes_launch<bf16, false, false, true>)(p, grid, st));
   else if (c.act == MI_F16) MI_TRY((sw ? codes_launch<f16, true, false> : rounded ? codes_launch<f16, false, true> : codes_launch<f16, false, false>)(p, grid, st));
   else MI_TRY((sw ? codes_launch<bf16, true, false> : rounded ? codes_launch<bf16, false, true> : codes_launch<bf16, false, false>)(p, grid, st));
-  if (p.ksplit > 1) {
+  if (p.mb == 0 && p.ksplit > 1) MI_TRY(reduce_slices(p, c.act, st));
+  if (p.mb > 0) {
     const dim3 rg((unsigned)(blocks - p.tail), 8), rb(512);
 #define TAIL_GO(T) do { if (sw) hipLaunchKernelGGL((tail_reduce_kernel<T, true, false>), rg, rb, 0, st, p); \
       else if (rounded) hipLaunchKernelGGL((tail_reduce_kernel<T, false, true>), rg, rb, 0, st, p); \

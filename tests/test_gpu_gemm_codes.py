@@ -282,6 +282,7 @@ def test_kept_codes_and_codes_per_call_give_the_same_bits(bits, act, kv_dtype):
     (8, 300, 2 * 1040, 1088, "swiglu"),      # fewer tiles than CUs, the last ones ragged: all in slices
     (4, 700, 24016, 1024, "f32"),            # 282 tiles; the last column of tiles holds 208 columns
     (8, 601, 22032, 1024, "resid"),
+    (8, 800, 22032, 1024, "resid"),          # whole slices do not fit the workspace: 92 of 348 tiles in slices
 ])
 def test_tiles_of_a_last_round_in_slices(act, bits, M, N, K, epi):
     """Against the oracle; every row of a call has one order of sums, whatever its place: a row's copy at the end gives the same bits."""
@@ -306,6 +307,31 @@ def test_tiles_of_a_last_round_in_slices(act, bits, M, N, K, epi):
     o = host(out)
     assert np.all(o[M:] == 7.0) and np.array_equal(o[M - 1], o[5])
     _assert_close(o[:M][rows], want, act, scale=float(np.abs(y).max()))
+
+
+@pytest.mark.parametrize("M,N,K,swiglu,most", [
+    (700, 6144, 4096, False, 1.4e-7),         # 72 tiles: seven slices of K 1.22e-7, three 1.80e-7
+    (300, 2 * 6400, 2048, True, 1.85e-7),     # 100 tiles: five slices 1.62e-7, two 2.10e-7, none 2.07e-7
+])
+def test_float32_rows_stay_as_close_to_64_bits(M, N, K, swiglu, most):
+    """How K is split decides how far float32 rows are from 64 bits: 2-norms as measured for the slices named, the bound between them."""
+    rng = np.random.default_rng(0)
+    w = rng.standard_normal((N, K)).astype(np.float32) * 0.05
+    lo, hi = w.reshape(N, K // 64, 64).min(-1), w.reshape(N, K // 64, 64).max(-1)
+    s, b = round_to((hi - lo) / 15, "bfloat16"), round_to(lo, "bfloat16")
+    q = np.clip(np.rint((w.reshape(N, K // 64, 64) - b[..., None]) / s[..., None]), 0, 15).astype(np.uint32)
+    packed = np.bitwise_or.reduce(q.reshape(N, K // 8, 8) << (np.arange(8, dtype=np.uint32) * 4), axis=-1).astype(np.uint32)
+    keep = [dev_u32(packed), dev(s, "bfloat16"), dev(b, "bfloat16")]
+    ol = op_linear("q4_bf16", N, K, *keep)
+    assert to_tiled(ol, keep)
+    x, rows = rng.standard_normal((M, K)).astype(np.float32), _rows(M)
+    y = x[rows].astype(np.float64) @ (q * s[..., None].astype(np.float64) + b[..., None]).reshape(N, K).T
+    cols = N // 2 if swiglu else N
+    want = y[:, :cols] / (1.0 + np.exp(-y[:, :cols])) * y[:, cols:] if swiglu else y
+    out = torch.zeros((M, cols), dtype=torch.float32, device="cuda")
+    _run(ol, dev(x), M, "float32", force=True, epi=L.EPI_SWIGLU if swiglu else L.EPI_STORE, out=out, ldo=cols, pair_offset=cols if swiglu else 0)
+    off = np.linalg.norm(host(out)[rows].astype(np.float64) - want) / np.linalg.norm(want)
+    assert off <= most, off
 
 
 @pytest.mark.parametrize("bits,act,H,V", [(4, "bfloat16", 384, 36864), (8, "float16", 2112, 6656), (4, "float16", 4224, 1680), (8, "bfloat16", 8192, 832), (4, "bfloat16", 8320, 832)])
