@@ -857,7 +857,10 @@ int launch_gemm_q4(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t
   p.lora_row0_1 = W.lora_row0[1]; p.lora_n_1 = W.lora_n[1]; p.lora_rank_1 = W.lora_rank[1]; p.lora_scale_1 = W.lora_scale[1];
   if (pl.rows) {
     p.wgs = pl.nslab > 1 ? (p.nunits + 7) / 8 * 8 * pl.nslab : p.nunits;
-    const int grid = std::max(p.wgs, gemv_cu_count());
+    // Read ahead only where a spare CU has at most four units to read for: what one asks for takes 0.4 us, a unit's round of blocks some 2.  Beyond, the launch waits for it: cold
+    // matrices, 32 / 64 rows, us with and without, 160 units of 5120 x 5120 11.1 / 13.9 and 12.2 / 17.0, 192 of 6144 x 8192 16.2 / 21.2 and 16.6 / 23.7, 200 of 6400 x 5120
+    // 12.3 / 16.1 and 12.4 / 17.4, 224 of 7168 x 5120 12.3 / 16.5 and 12.2 / 17.0, 240 of 7680 x 5120 20.8 / 23.0 and 12.4 / 17.2, 252 of 8064 x 5120 41 / 46 and 12.4 / 17.1.
+    const int spare = gemv_cu_count() - p.wgs, grid = p.wgs + (spare * 4 >= p.nunits ? spare : 0);
     return c.act == MI_BF16 ? q4_rows_launch<bf16>(p, pl.mt, c.epi == EPI_SWIGLU, grid, st) : q4_rows_launch<f16>(p, pl.mt, c.epi == EPI_SWIGLU, grid, st);
   }
   const int blocks = pl.nslab > 1 ? (p.nunits + 7) / 8 * 8 * pl.nslab : p.nunits;

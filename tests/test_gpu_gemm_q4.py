@@ -10,7 +10,7 @@ from oracle.numerics import matmul_nt, round_to
 pytestmark = pytest.mark.gpu
 
 from mlx_parallm_amd import _lib as L  # noqa: E402
-from gpu_helpers import dev, gemm_skinny, host, q4_force  # noqa: E402
+from gpu_helpers import dev, gemm_skinny, host, op_linear, q4_force, to_tiled  # noqa: E402
 from test_gpu_gemm_codes import _weight  # noqa: E402
 from test_gpu_kernels import _assert_close  # noqa: E402
 
@@ -64,6 +64,7 @@ def test_every_forced_plan_and_every_norm_in_front_of_a_wide_matrix_is_taken():
     (64, 4112, 128 * 17, "f32"),     # 129 units (the other CUs read ahead), blocks that differ by wave
     (100, 96, 128 * 5, "norm"),      # two slabs
     (128, 8224, 128 * 2, "store"),   # two slabs, more workgroups than CUs
+    (33, 7376, 128 * 3, "store"),    # 231 units: too few other CUs to read ahead
     (40, 2 * 80, 128 * 8, "swiglu"),
     (97, 2 * 48, 128 * 7, "swiglu"),
 ])
@@ -94,6 +95,19 @@ def test_narrow_matrices(act, M, N, K, epi):
         g, u = want[:, :cols], want[:, cols:]
         want = round_to(round_to(g * round_to(1.0 / (1.0 + np.exp(-g.astype(np.float64))), act), act) * u, act)
     _assert_close(outs[0][:M], want, act)
+
+
+def test_a_few_spare_cus_do_not_hold_the_launch_up():
+    """252 and 256 units of two column tiles: nearly the same work, so nearly the same time (15 us each; 98 and 15 where four CUs read ahead for 252 units)."""
+    M, K, us = 32, 8192, []
+    x = torch.randn((M, K), device="cuda").to(torch.bfloat16)
+    for N in (8064, 8192):
+        keep = [torch.randint(-2 ** 31, 2 ** 31 - 1, (N, K // 8), device="cuda", dtype=torch.int32)] + [torch.full((N, K // 64), 0.01, device="cuda", dtype=torch.bfloat16)] * 2
+        ol = op_linear("q4_bf16", N, K, *keep)
+        assert to_tiled(ol, keep)
+        out = torch.zeros((M, N), dtype=torch.bfloat16, device="cuda")
+        us.append(min(gemm_skinny(ol, x, M, "bfloat16", epi=L.EPI_STORE, out=out, ldo=N, ksplit=q4_force(rows=1), iters=20)[1] * 1e3 for _ in range(4)))
+    assert us[0] <= 2.0 * us[1], us
 
 
 @pytest.mark.parametrize("act", ["bfloat16", "float16"])
