@@ -94,16 +94,17 @@ __global__ __launch_bounds__(256) void q4_prep_kernel(const AT* x, int ldx, int 
   };
   const auto put = [&](int k, u32x4 v) {
     const AT* e = (const AT*)&v;
-    float sum = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) sum += (float)e[j];
-    sum = lane8_sum(sum);
     AT t2[8];
 #pragma unroll
     for (int q = 0; q < 4; ++q) { t2[2 * q] = e[q]; t2[2 * q + 1] = e[q + 4]; }
     const int grp = k >> 6, d = (k >> 3) & 7;
     const size_t frag = (((size_t)slab * G + grp) * 2 + (d & 1)) * MT + (r >> 4);
     *(u32x4*)((char*)xq + (frag * 64 + (d >> 1) * 16 + (r & 15)) * 16) = *(const u32x4*)t2;
+    if (sx == nullptr) return;                                   // (uniform: q4_rows_kernel makes its own sums)
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sum += (float)e[j];
+    sum = lane8_sum(sum);
     if ((tid & 7) == 0) {
       sx[((size_t)slab * G + grp) * MB + r] = sum;
       sxo[((size_t)slab * G + grp) * 64 + r] = -Magic<AT>::offs * sum;
@@ -765,8 +766,8 @@ Q4Plan q4_plan(const LinearW& W, const GemvCall& c, size_t rows) {
   }
   const size_t G = W.K / 64;
   pl.xq_bytes = (size_t)pl.nslab * G * 2 * pl.mt * 1024;
-  pl.sx_bytes = (pl.nslab * G * 16 * pl.mt * sizeof(float) + 255) & ~(size_t)255;
-  pl.sxo_bytes = pl.nslab * G * 256;
+  pl.sx_bytes = pl.rows ? 0 : (pl.nslab * G * 16 * pl.mt * sizeof(float) + 255) & ~(size_t)255;
+  pl.sxo_bytes = pl.rows ? 0 : pl.nslab * G * 256;
   pl.ws_bytes = pl.xq_bytes + pl.sx_bytes + pl.sxo_bytes + (pl.ksplit > 1 ? (size_t)pl.nslab * pl.ksplit * pl.ngroups * TW * TN * pl.mt * 1024 : 0);
   return pl;
 }
@@ -844,7 +845,7 @@ int launch_gemm_q4(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t
   float* sxo = (float*)((char*)sx + pl.sx_bytes);
   const void* nw = c.pro == PRO_NORM ? c.norm_w : nullptr;
   const dim3 grid(pl.nslab * pl.mt * 16, nw != nullptr ? 1 : (W.K + 2047) / 2048);
-  (c.act == MI_BF16 ? q4_prep_launch<bf16> : q4_prep_launch<f16>)(c, grid, (int)rows, pl.mt, W.K, nw, xq, sx, sxo, st);
+  (c.act == MI_BF16 ? q4_prep_launch<bf16> : q4_prep_launch<f16>)(c, grid, (int)rows, pl.mt, W.K, nw, xq, pl.rows ? nullptr : sx, sxo, st);
   MI_HIP(hipGetLastError());
   Q4Params p{};
   p.xq = xq; p.sx = sx; p.sxo = sxo; p.M = (int)rows; p.G = W.K / 64; p.w = W.w;
