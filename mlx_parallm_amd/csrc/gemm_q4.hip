@@ -734,9 +734,12 @@ thread_local int q4_force_rows = 0;
 thread_local bool q4_forced = false;                             // .. and whatever the width
 
 // Narrow matrices: q4_rows_kernel or gemm_skinny.hip?  us, both with their preparation but without the norm launch of 4.7 that q4_prep_kernel saves, warm weights,
-// here / there at 32, 64 and 128 rows: 7168 x 5120 14 / 16, 17 / 23, 31 / 30; 5120 x 5120 15 / 17, 17 / 22, 31 / 28; 4096 x 4096 13 / 15, 15 / 21, 16 / 23; 2048 x 6400 16 / 17,
-// 19 / 23, 20 / 24; 3072 x 1024 8 / 9, 9 / 10, 9 / 13; SwiGLU 6400 x 2048 10 / 16, 11 / 25, 17 / 23.  A longer K: 4096 x 14336 26 / 23, 41 / 33, 43 / 45; 5120 x 17408 32 / 28, 50 / 40, 87 /
-// 62.  So: K up to 8192, and one round of workgroups, or two where a norm launch goes with the other kernel.
+// here / there at 32, 64 and 128 rows: 7168 x 5120 11 / 15, 14 / 22, 26 / 30; 5120 x 5120 11 / 17, 15 / 22, 26 / 27; 4096 x 4096 10 / 15, 13 / 21, 15 / 23; 4096 x 6400 12 / 17,
+// 16 / 24, 19 / 29; 8192 x 8192 15 / 22, 21 / 30, 38 / 45; 4096 x 10240 15 / 19, 22 / 29, 26 / 35; 4096 x 12288 17 / 22, 25 / 29, 29 / 38.  More than one round of workgroups: 5120 x 10240
+// at 65 rows 36 / 33, 128 43 / 41; with a norm (to be added to the other side) or a SwiGLU 10240 x 5120 16 / 17, 25 / 25, 36 / 45; 10240 x 8192 22 / 22, 35 / 34, 51 / 59; 16128 x 8192
+// 23 / 27, 36 / 44, 68 / 72; 16128 x 4096 15 / 18, 23 / 28, 41 / 38 (four rounds: behind by less than the norm); SwiGLU 14336 x 4096 15 / 19, 22 / 30, 39 / 41, 16128 x 8192 23 / 28, 36 / 43, 67 / 68.
+// A longer K: 4096 x 14336 26 / 23, 41 / 33, 43 / 45; 5120 x 17408 32 / 28, 50 / 40, 87 / 62.  So: K up to 8192 (to 12288 it would still be the faster one), and one round of workgroups,
+// or any number where a norm launch goes with the other kernel.
 bool q4_rows_ahead(const LinearW& W, const GemvCall& c, size_t rows) {
   const long units = c.epi == EPI_SWIGLU ? c.pair_offset / 16 : (W.N / 16 + RT - 1) / RT, slabs = (long)((rows + 63) / 64);
   return W.K <= 8192 && (c.pro == PRO_NORM || c.epi == EPI_SWIGLU || units * slabs <= gemv_cu_count());
