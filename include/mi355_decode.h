@@ -365,8 +365,11 @@ int mi_profile_read(mi_engine* e, int64_t* n_launches, double* total_ms);
  *   "prefill_x_terms"         3: float32-activation (PagedKVCache mode) prefill multiplies an EXACT three-term 16-bit split of x
  *                             by dense bf16 weights (three walks of W); default 2: hi + lo, 16+ mantissa bits of x, two walks
  *                             (the CPU float32-accumulating variants do not move under it: DESIGN 8d); int4 always 3
- *   "prefill_codes_copy"      0: prefills of int4 / int8 models copy the 16-bit codes in front of every product instead of multiplying the
- *                             copies that mi_engine_finalize made while half of the device's memory stayed free (default 1; the same bits)
+ *   "prefill_codes_copy"      0: prefills of int4 / int8 models copy the 16-bit codes in front of every product instead of multiplying copies
+ *                             that mi_engine_finalize makes (default 1; the same bits).  The copies take 2.3 bytes per weight (float16: 2.2), of as many
+ *                             matrices as an eighth of the memory that the weights leave free holds; they go where memory for a cache or a
+ *                             workspace runs out.  0 before mi_engine_finalize: none are made (a program that only decodes); later: they are
+ *                             given back, and 1 makes them again
  *   "short_prefill_skinny"    0: prefill calls of <= 128 rows in all through the tile GEMM like longer ones (default 1: the
  *                             weight-streaming split-K kernel of the decode steps, ~2x faster at that size)
  *   "tile_weights"            0: keep weights row-major (before mi_engine_finalize only; default 1)
@@ -377,6 +380,8 @@ int mi_profile_read(mi_engine* e, int64_t* n_launches, double* total_ms);
  * MI_ATTN_PREFILL_F32_EXACT (1: float32-KV prefill attention with exact float32 products instead of two-term bf16 operands;
  * read per call). */
 int mi_engine_set_option(mi_engine* e, const char* key, int64_t value);
+/* Device memory that the copies of "prefill_codes_copy" take now. */
+uint64_t mi_engine_codes_bytes(mi_engine* e);
 /* Blocks until the engine's stream is idle. */
 int mi_engine_sync(mi_engine* e);
 

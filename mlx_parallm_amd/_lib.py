@@ -132,6 +132,7 @@ SIGNATURES = {
     "mi_profile_select": (C.c_int, [_P, C.c_char_p]),
     "mi_profile_read": (C.c_int, [_P, C.POINTER(C.c_int64), C.POINTER(C.c_double)]),
     "mi_engine_set_option": (C.c_int, [_P, C.c_char_p, C.c_int64]),
+    "mi_engine_codes_bytes": (C.c_uint64, [_P]),
     "mi_engine_sync": (C.c_int, [_P]),
     "mi_host_alloc": (C.c_int, [C.c_uint64, C.POINTER(_P)]),
     "mi_engine_host_alloc": (C.c_int, [_P, C.c_uint64, C.POINTER(_P)]),

@@ -130,6 +130,29 @@ void free_linear(FusedLinear& f) {
   for (int i = 0; i < 2; ++i) { hipFree(f.lora_a[i]); hipFree(f.lora_b[i]); }
 }
 
+// Copies of the codes (make_codes_copies below): the linears that can have one, in the order in which they get it
+template <typename F>
+void each_codes_linear(mi_engine* e, F f) {
+  for (LayerW& l : e->layers) { f(l.qkv); f(l.o); f(l.gate_up); f(l.down); }
+  f(e->d.tie_word_embeddings ? e->embed : e->lm_head);
+}
+bool drop_codes_copies(mi_engine* e) {                            // -> whether there were any
+  size_t had = 0;
+  each_codes_linear(e, [&](FusedLinear& f) { had += f.w_codes != nullptr; });
+  if (had == 0) return false;
+  (void)hipStreamSynchronize(e->stream);
+  each_codes_linear(e, [](FusedLinear& f) { hipFree(f.w_codes); f.w_codes = nullptr; f.W.codes = Codes16{}; });
+  return true;
+}
+// Memory that a caller asked for comes before the copies: where there is not enough, they go.  (A failure leaves no error behind for the next launch to report)
+template <typename T>
+hipError_t dev_malloc(mi_engine* e, T** p, size_t bytes) {
+  hipError_t rc = hipMalloc(p, bytes);
+  if (rc != hipSuccess && ((void)hipGetLastError(), drop_codes_copies(e))) rc = hipMalloc(p, bytes);
+  if (rc != hipSuccess) { (void)hipGetLastError(); *p = nullptr; }
+  return rc;
+}
+
 int ensure_workspace(mi_engine* e, size_t rows, size_t logit_rows, int B) {
   const mi_model_desc& d = e->d;
   if (e->layered) MI_TRY(layers_ensure_workspace(e, rows));
@@ -138,20 +161,20 @@ int ensure_workspace(mi_engine* e, size_t rows, size_t logit_rows, int B) {
     hipFree(e->h); hipFree(e->qkv); hipFree(e->q); hipFree(e->attn); hipFree(e->act); hipFree(e->lora_t);
     const size_t es = 4;  // sized for float32 activations (the widest mode)
     const size_t nqkv = (size_t)(d.num_heads + 2 * d.num_kv_heads) * d.head_dim;
-    MI_HIP(hipMalloc(&e->h, rows * d.hidden_size * es));
-    MI_HIP(hipMalloc(&e->qkv, rows * nqkv * es));
-    MI_HIP(hipMalloc(&e->q, rows * (size_t)d.num_heads * d.head_dim * es));
-    MI_HIP(hipMalloc(&e->attn, rows * (size_t)d.num_heads * d.head_dim * es));
-    MI_HIP(hipMalloc(&e->act, rows * (size_t)d.intermediate_size * es));
-    MI_HIP(hipMalloc(&e->lora_t, rows * 2 * 64 * sizeof(float)));
+    MI_HIP(dev_malloc(e, &e->h, rows * d.hidden_size * es));
+    MI_HIP(dev_malloc(e, &e->qkv, rows * nqkv * es));
+    MI_HIP(dev_malloc(e, &e->q, rows * (size_t)d.num_heads * d.head_dim * es));
+    MI_HIP(dev_malloc(e, &e->attn, rows * (size_t)d.num_heads * d.head_dim * es));
+    MI_HIP(dev_malloc(e, &e->act, rows * (size_t)d.intermediate_size * es));
+    MI_HIP(dev_malloc(e, &e->lora_t, rows * 2 * 64 * sizeof(float)));
     hipFree(e->xn);
-    MI_HIP(hipMalloc(&e->xn, rows * (size_t)d.hidden_size * es));
+    MI_HIP(dev_malloc(e, &e->xn, rows * (size_t)d.hidden_size * es));
     e->ws_rows = rows;
   }
   if (logit_rows > e->ws_logit_rows) {
     MI_HIP(hipStreamSynchronize(e->stream));
     hipFree(e->logits);
-    MI_HIP(hipMalloc(&e->logits, logit_rows * (size_t)d.vocab_size * sizeof(float)));
+    MI_HIP(dev_malloc(e, &e->logits, logit_rows * (size_t)d.vocab_size * sizeof(float)));
     e->ws_logit_rows = logit_rows;
   }
   if (rows > e->d_tokens_cap) {
@@ -203,19 +226,25 @@ bool ensure_hilo(mi_engine* e, FusedLinear& f) {
   return true;
 }
 // Codes of quantised weights as the prefill GEMM multiplies them: made once, a prompt no longer writes and reads 2 bytes per weight in front of every product
-// (28672 x 4096 int4: 51 us of 314 at 700 rows).  2.2 bytes per weight, while half of the device's memory stays free.
-void make_codes_copy(mi_engine* e, FusedLinear& f) {
-  if (!wk_is_quant(f.W.wk) || f.W.layout != 1 || f.W.group != 64 || f.W.K > 65536 || wk_scale_dtype(f.W.wk) == WK_F32 || f.w_codes != nullptr || e->opt_force_v1) return;
+// (28672 x 4096 int4: 51 us of 314 at 700 rows).  2.3 bytes per weight (2.2 in float16), for as many matrices as an eighth of the memory that the weights leave free holds: a
+// scheduler's arena, 80 % of what is free without them, and the workspaces fit beside them; a caller that asks for more gets it (dev_malloc).
+void make_codes_copies(mi_engine* e) {
+  if (!e->opt_codes_copy || e->opt_force_v1 || e->layered) return;
   size_t avail = 0, total = 0;
-  const size_t need = codes16_kept_bytes(f.W.N, f.W.K);
   if (hipMemGetInfo(&avail, &total) != hipSuccess) { (void)hipGetLastError(); return; }
-  if (avail < need + total / 2) return;
-  void* p = nullptr;
-  if (hipMalloc(&p, need) != hipSuccess) { (void)hipGetLastError(); return; }
-  Codes16 c;
-  if (launch_codes16_kept(f.W, p, e->stream, c) != MI_OK) { hipFree(p); return; }
-  f.w_codes = p;
-  f.W.codes = c;
+  size_t left = avail / 8;
+  each_codes_linear(e, [&](FusedLinear& f) {
+    if (!wk_is_quant(f.W.wk) || f.W.layout != 1 || f.W.group != 64 || f.W.K > 65536 || wk_scale_dtype(f.W.wk) == WK_F32 || f.w_codes != nullptr) return;
+    const size_t need = codes16_kept_bytes(f.W);
+    if (need > left) return;
+    void* p = nullptr;
+    if (hipMalloc(&p, need) != hipSuccess) { (void)hipGetLastError(); left = 0; return; }
+    Codes16 c;
+    if (launch_codes16_kept(f.W, p, e->stream, c) != MI_OK) { hipFree(p); return; }
+    f.w_codes = p;
+    f.W.codes = c;
+    left -= need;
+  });
 }
 bool gu8_wanted(const mi_engine* e, const FusedLinear& f, int pair_offset) {
   const bool has_lora = f.W.lora_b[0] != nullptr || f.W.lora_b[1] != nullptr;
@@ -301,7 +330,7 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
           MI_HIP(hipStreamSynchronize(e->stream));
           if (need > e->sk_ws_cap) {
             hipFree(e->sk_ws); e->sk_ws = nullptr; e->sk_ws_cap = 0;
-            MI_HIP(hipMalloc(&e->sk_ws, need));
+            MI_HIP(dev_malloc(e, &e->sk_ws, need));
             e->sk_ws_cap = need;
           }
           if (groups > e->sk_ctr_cap) {
@@ -380,7 +409,7 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
       MI_HIP(hipStreamSynchronize(e->stream));
       if (need > e->sk_ws_cap) {
         hipFree(e->sk_ws); e->sk_ws = nullptr; e->sk_ws_cap = 0;
-        MI_HIP(hipMalloc(&e->sk_ws, need));
+        MI_HIP(dev_malloc(e, &e->sk_ws, need));
         e->sk_ws_cap = need;
       }
       if (groups > e->sk_ctr_cap) {
@@ -414,7 +443,7 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
       if (need > e->xs_cap) {
         MI_HIP(hipStreamSynchronize(e->stream));
         hipFree(e->xs); e->xs = nullptr; e->xs_cap = 0;
-        MI_HIP(hipMalloc(&e->xs, need));
+        MI_HIP(dev_malloc(e, &e->xs, need));
         e->xs_cap = need;
       }
       // dense bf16 weights: two terms (16+ mantissa bits of x, two walks of W; option "prefill_x_terms"); int4 / [hi | lo]
@@ -451,26 +480,27 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
     const int ncol = (wk_is_quant(f.W.wk) && c.epi == EPI_STORE_F32) ? std::min(f.W.N, 32768) : f.W.N;
     void* scratch = nullptr;
     if (wk_is_quant(f.W.wk)) {               // the GEMM multiplies by 16-bit codes, or a [hi | lo] 16-bit copy, made on the fly
-      LinearW part = f.W;
-      part.N = ncol;
-      const size_t need = gemm_prefill_scratch_bytes(part, rows);
-      if (need > e->deq_cap) {
+      for (;;) {
+        LinearW part = f.W;
+        part.N = ncol;
+        const size_t need = gemm_prefill_scratch_bytes(part, c, rows);
+        if (need <= e->deq_cap) break;
         MI_HIP(hipStreamSynchronize(e->stream));
         hipFree(e->deq_scratch);
         e->deq_scratch = nullptr; e->deq_cap = 0;
-        MI_HIP(hipMalloc(&e->deq_scratch, need));
+        MI_HIP(dev_malloc(e, &e->deq_scratch, need));             // (where the kept codes went for it, the scratch takes them: once more)
         e->deq_cap = need;
       }
       scratch = e->deq_scratch;
     }
     if (rows < 4096 && e->gk_ws == nullptr) {     // K-split partial tiles of the tile GEMMs (one prompt of a few hundred to a few thousand rows)
       e->gk_cap = (size_t)128 << 20;
-      if (hipMalloc(&e->gk_ws, e->gk_cap) != hipSuccess) { e->gk_ws = nullptr; e->gk_cap = 0; }
+      if (dev_malloc(e, &e->gk_ws, e->gk_cap) != hipSuccess) e->gk_cap = 0;
     }
     for (int n0 = 0; n0 < f.W.N; n0 += ncol) {
       LinearW part = f.W;
       GemvCall cp = c;
-      part.codes = e->opt_codes_copy ? codes16_rows(f.W.codes, n0, f.W.K) : Codes16{};
+      part.codes = codes16_rows(f.W.codes, n0, f.W.K);
       if (ncol < f.W.N) {
         part.N = std::min(ncol, f.W.N - n0);
         part.w = (const char*)f.W.w + (wk_bits(f.W.wk) == 4 ? tiled_block_q4(n0, 0, f.W.K) : tiled_block_q8(n0, 0, f.W.K));
@@ -513,7 +543,7 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
       MI_HIP(hipStreamSynchronize(e->stream));
       if (need > e->sk_ws_cap) {
         hipFree(e->sk_ws); e->sk_ws = nullptr; e->sk_ws_cap = 0;
-        MI_HIP(hipMalloc(&e->sk_ws, need));
+        MI_HIP(dev_malloc(e, &e->sk_ws, need));
         e->sk_ws_cap = need;
       }
       if (groups > e->sk_ctr_cap) {
@@ -1293,19 +1323,18 @@ int mi_engine_finalize(mi_engine* e) {
     MI_TRY(make_f32_copy(e, l.k_norm, d.head_dim, &l.k_norm32));
     // persistent second copies, while mem_get_info still tells a scheduler the truth about what is left for its KV arena
     (void)ensure_gu8(e, l.gate_up, d.intermediate_size);
-    make_codes_copy(e, l.qkv); make_codes_copy(e, l.o); make_codes_copy(e, l.gate_up); make_codes_copy(e, l.down);
     if (d.act_dtype == MI_F16) { (void)ensure_hilo(e, l.qkv); (void)ensure_hilo(e, l.o); (void)ensure_hilo(e, l.gate_up); (void)ensure_hilo(e, l.down); }
   }
   MI_TRY(finalize_linear(e, e->embed, H, "model.embed_tokens"));
   if (!d.tie_word_embeddings) MI_TRY(finalize_linear(e, e->lm_head, H, "lm_head"));
   if (d.act_dtype == MI_F16) (void)ensure_hilo(e, d.tie_word_embeddings ? e->embed : e->lm_head);
-  make_codes_copy(e, d.tie_word_embeddings ? e->embed : e->lm_head);
   if (!e->final_norm) return fail(MI_ERR_NOTFOUND, "model.norm.weight not set");
   MI_TRY(make_f32_copy(e, e->final_norm, H, &e->final_norm32));
   const size_t n = (size_t)d.max_positions * (d.head_dim / 2);
   MI_HIP(hipMalloc(&e->cos_tab, n * sizeof(float)));
   MI_HIP(hipMalloc(&e->sin_tab, n * sizeof(float)));
   MI_TRY(launch_rope_tables(e->cos_tab, e->sin_tab, d.max_positions, d.head_dim, d.rope_theta, d.rope_scale, e->stream));
+  make_codes_copies(e);
   MI_HIP(hipStreamSynchronize(e->stream));
   e->finalized = true;
   return MI_OK;
@@ -1326,10 +1355,10 @@ int mi_kv_create(mi_engine* e, int batch, int capacity_tokens, int kv_dtype, mi_
   if (e->layered) layers_kv_plan(e, kv);
   const size_t bytes = e->layered ? kv->list_bytes : (size_t)e->d.num_layers * batch * e->d.num_kv_heads * capacity_tokens * e->d.head_dim * dtype_size(kv->dtype);
   const size_t nctr = e->layered ? 1 : (size_t)batch * e->d.num_kv_heads;
-  if (hipMalloc(&kv->k, bytes) != hipSuccess || (!e->layered && hipMalloc(&kv->v, bytes) != hipSuccess) ||
-      (e->layered && hipMalloc(&kv->state, kv->state_bytes) != hipSuccess) ||
-      hipMalloc(&kv->d_off, batch * sizeof(int32_t)) != hipSuccess ||
-      hipMalloc(&kv->counters, nctr * sizeof(int)) != hipSuccess) {
+  if (dev_malloc(e, &kv->k, bytes) != hipSuccess || (!e->layered && dev_malloc(e, &kv->v, bytes) != hipSuccess) ||
+      (e->layered && dev_malloc(e, &kv->state, kv->state_bytes) != hipSuccess) ||
+      dev_malloc(e, &kv->d_off, batch * sizeof(int32_t)) != hipSuccess ||
+      dev_malloc(e, &kv->counters, nctr * sizeof(int)) != hipSuccess) {
     hipFree(kv->k); hipFree(kv->v); hipFree(kv->state); hipFree(kv->d_off); hipFree(kv->counters); delete kv;
     return fail(MI_ERR_RUNTIME, "out of device memory allocating the KV cache");
   }
@@ -1365,10 +1394,10 @@ int mi_kv_create_paged(mi_engine* e, int slots, int block_tokens, int n_blocks, 
   const size_t bytes = e->layered ? kv->list_bytes : (size_t)e->d.num_layers * n_blocks * e->d.num_kv_heads * block_tokens * e->d.head_dim * dtype_size(kv->dtype);
   const size_t nctr = e->layered ? 1 : (size_t)slots * e->d.num_kv_heads;
   const size_t ntab = (size_t)slots * kv->bt_stride;
-  if (hipMalloc(&kv->k, bytes) != hipSuccess || (!e->layered && hipMalloc(&kv->v, bytes) != hipSuccess) ||
-      (e->layered && hipMalloc(&kv->state, kv->state_bytes) != hipSuccess) ||
-      hipMalloc(&kv->d_off, slots * sizeof(int32_t)) != hipSuccess || hipMalloc(&kv->counters, nctr * sizeof(int)) != hipSuccess ||
-      hipMalloc(&kv->d_btab, ntab * sizeof(int32_t)) != hipSuccess) {
+  if (dev_malloc(e, &kv->k, bytes) != hipSuccess || (!e->layered && dev_malloc(e, &kv->v, bytes) != hipSuccess) ||
+      (e->layered && dev_malloc(e, &kv->state, kv->state_bytes) != hipSuccess) ||
+      dev_malloc(e, &kv->d_off, slots * sizeof(int32_t)) != hipSuccess || dev_malloc(e, &kv->counters, nctr * sizeof(int)) != hipSuccess ||
+      dev_malloc(e, &kv->d_btab, ntab * sizeof(int32_t)) != hipSuccess) {
     hipFree(kv->k); hipFree(kv->v); hipFree(kv->state); hipFree(kv->d_off); hipFree(kv->counters); hipFree(kv->d_btab); delete kv;
     return fail(MI_ERR_RUNTIME, "out of device memory allocating the paged KV arena");
   }
@@ -1520,7 +1549,7 @@ int mi_kv_reserve(mi_kv* kv, int capacity_tokens) {
     kv->cap = capacity_tokens;
     layers_kv_plan(e, kv);
     void* nk = nullptr;
-    if (hipMalloc(&nk, kv->list_bytes) != hipSuccess) {
+    if (dev_malloc(e, &nk, kv->list_bytes) != hipSuccess) {
       kv->cap = old_cap; layers_kv_plan(e, kv);
       return fail(MI_ERR_RUNTIME, "out of device memory growing the KV cache");
     }
@@ -1538,7 +1567,7 @@ int mi_kv_reserve(mi_kv* kv, int capacity_tokens) {
   const size_t slabs = (size_t)e->d.num_layers * kv->B * e->d.num_kv_heads;
   const size_t old_pitch = (size_t)kv->cap * e->d.head_dim * es, new_pitch = (size_t)capacity_tokens * e->d.head_dim * es;
   void* nk = nullptr; void* nv = nullptr;
-  if (hipMalloc(&nk, slabs * new_pitch) != hipSuccess || hipMalloc(&nv, slabs * new_pitch) != hipSuccess) {
+  if (dev_malloc(e, &nk, slabs * new_pitch) != hipSuccess || dev_malloc(e, &nv, slabs * new_pitch) != hipSuccess) {
     hipFree(nk); hipFree(nv);
     return fail(MI_ERR_RUNTIME, "out of device memory growing the KV cache");
   }
@@ -1819,7 +1848,13 @@ int mi_engine_set_option(mi_engine* e, const char* key, int64_t value) {
   if (k == "decode_attention_mfma") { e->opt_attn_mfma = value != 0; return MI_OK; }
   if (k == "fused_gemv_pairs") { e->opt_fused_pairs = (int)value; return MI_OK; }
   if (k == "f16_hilo") { e->opt_f16_hilo = value != 0; return MI_OK; }
-  if (k == "prefill_codes_copy") { e->opt_codes_copy = value != 0; return MI_OK; }
+  if (k == "prefill_codes_copy") {
+    e->opt_codes_copy = value != 0;
+    MI_HIP(hipSetDevice(e->device));
+    if (!e->opt_codes_copy) (void)drop_codes_copies(e);
+    else if (e->finalized) { make_codes_copies(e); MI_HIP(hipStreamSynchronize(e->stream)); }
+    return MI_OK;
+  }
   if (k == "gate_up_interleave") { e->opt_gu8 = value != 0; return MI_OK; }
   if (k == "seam_spin_limit") {
     if (value < 0 || value > (int64_t)0x7fffffff) return fail(MI_ERR_INVALID, "seam_spin_limit out of range");
@@ -1830,6 +1865,12 @@ int mi_engine_set_option(mi_engine* e, const char* key, int64_t value) {
     e->opt_tile_weights = value != 0; return MI_OK;
   }
   return fail(MI_ERR_NOTFOUND, "unknown option: " + k);
+}
+
+uint64_t mi_engine_codes_bytes(mi_engine* e) {
+  uint64_t n = 0;
+  if (e) each_codes_linear(e, [&](FusedLinear& f) { n += f.w_codes != nullptr ? codes16_kept_bytes(f.W) : 0; });
+  return n;
 }
 
 int mi_host_alloc(uint64_t bytes, void** out) {

@@ -1760,8 +1760,10 @@ static int reduce_slices(const GemmParams& p, int act, hipStream_t st) {
   return MI_OK;
 }
 
-size_t gemm_prefill_scratch_bytes(const LinearW& W, size_t rows) {
-  return std::max(dequant_hilo_bytes(W.N, W.K), codes16_bytes(W.N, W.K) + rows * codes16_bias_cols(W.K) * 2);
+size_t gemm_prefill_scratch_bytes(const LinearW& W, const GemvCall& c, size_t rows) {
+  const size_t sums = rows * codes16_bias_cols(W.K) * 2;
+  if (c.codes && W.codes.codes != nullptr) return sums;          // (the copy is kept)
+  return std::max(dequant_hilo_bytes(W.N, W.K), codes16_bytes(W.N, W.K) + sums);
 }
 
 // us of a launch over `blocks` tiles of `nk` K tiles in rounds of one workgroup per CU, those from `tail` on as `ks` slices: a round 10 + 2 per K tile (float32 rows, whose three walks
@@ -1877,13 +1879,14 @@ static int launch_gemm_codes(const LinearW& W, const GemvCall& c, size_t rows, h
   p.x = c.x;
   p.ws = (float*)splitk_ws;
   char* d = (char*)scratch;
-  if (W.codes.codes != nullptr) {                        // (a copy that was made when the weights were loaded)
+  if (c.codes && W.codes.codes != nullptr) {             // (a copy that was made when the weights were loaded; gemm_prefill_scratch_bytes asks the same)
     p.w = W.codes.codes; p.wb = W.codes.bias[terms != 1]; p.sc = W.codes.scales;
   } else {
     MI_TRY(launch_codes16(W, scratch, st, terms == 1));
     p.w = d; p.wb = d + (size_t)W.N * W.K * 2; p.sc = (const float*)(d + (size_t)W.N * (W.K + p.kb) * 2);
+    d += codes16_bytes(W.N, W.K);
   }
-  uint16_t* xs = (uint16_t*)(d + codes16_bytes(W.N, W.K));
+  uint16_t* xs = (uint16_t*)d;
   p.xs = xs;
   if (c.pro == PRO_NORM) {
     MI_TRY((c.act == MI_F16 ? launch_rmsnorm_block<f16> : launch_rmsnorm_block<bf16>)(c.x, c.ldx, c.norm_w, c.norm_out, W.K, (int)rows, W.K, c.eps, st, xs, p.kb));

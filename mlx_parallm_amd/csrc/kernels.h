@@ -4,7 +4,6 @@
 
 namespace mi {
 
-// One (possibly fused) weight matrix W[N][K] as the kernels see it.
 // The operands of the prefill GEMM on codes (repack.hip): the codes as 16-bit integers, the biases (of 16-bit rows: the largest parts first, of float32 rows: last), the scales
 struct Codes16 {
   const void* codes = nullptr;
@@ -12,6 +11,7 @@ struct Codes16 {
   const float* scales = nullptr;
 };
 
+// One (possibly fused) weight matrix W[N][K] as the kernels see it.
 struct LinearW {
   int wk = WK_F32;             // weight kind (common.h)
   const void* w = nullptr;     // dense [N][K] or MLX-packed [N][K*bits/32] uint32
@@ -138,8 +138,8 @@ int launch_dequant_q4_hilo(const LinearW& src, void* dst, hipStream_t st);
 int codes16_bias_cols(int K);
 size_t codes16_bytes(int N, int K);
 int launch_codes16(const LinearW& src, void* dst, hipStream_t st, bool big_first = false);
-// .. kept for good: both orders of the biases
-size_t codes16_kept_bytes(int N, int K);
+// .. kept for good: of a bf16 model both orders of the biases
+size_t codes16_kept_bytes(const LinearW& W);
 int launch_codes16_kept(const LinearW& src, void* dst, hipStream_t st, Codes16& out);
 Codes16 codes16_rows(const Codes16& c, int n0, int K);       // of the outputs from n0 (a multiple of 16) on
 // term t of that product, the smallest first: part of x's group sum (0 = hi, 1 = mid, 2 = lo) and of the bias; products below 2^-24 of the whole are left
@@ -153,7 +153,7 @@ __device__ __forceinline__ float bf16_part(float v, int part) {
   return part == 0 ? hi : part == 1 ? mid : r - mid;
 }
 // `scratch` bytes of launch_gemm_prefill for a quantised matrix
-size_t gemm_prefill_scratch_bytes(const LinearW& W, size_t rows);
+size_t gemm_prefill_scratch_bytes(const LinearW& W, const GemvCall& c, size_t rows);
 // block_per_row: one workgroup per row, row in registers -- for the few rows of a decode step (default: one wave
 // per row, the prefill's kernel; the two add the squares in different orders)
 // act = MI_F32: float32 rows and weights with the run-time logical rounding `rnd` (PagedKVCache mode)

@@ -167,7 +167,7 @@ int mi_op_gemm_codes(const mi_op_linear* w, const mi_op_gemv_args* a, int iters,
   size_t cap = 0;
   auto done = [&](int rc) { hipFree(ws); hipFree(scratch); hipFree(xs); return rc; };
   if (c.M < 4096) { cap = (size_t)128 << 20; if (hipMalloc(&ws, cap) != hipSuccess) return done(fail(MI_ERR_RUNTIME, "mi_op_gemm_codes: workspace")); }
-  if (hipMalloc(&scratch, gemm_prefill_scratch_bytes(W, (size_t)c.M)) != hipSuccess) return done(fail(MI_ERR_RUNTIME, "mi_op_gemm_codes: scratch"));
+  if (hipMalloc(&scratch, gemm_prefill_scratch_bytes(W, c, (size_t)c.M)) != hipSuccess) return done(fail(MI_ERR_RUNTIME, "mi_op_gemm_codes: scratch"));
   int rc = MI_OK;
   if (c.act == MI_F32) {                               // float32 activations: three bf16 terms (layer 0's rounded call: one)
     const int terms = c.rnd == RND_BF16 ? 1 : 3;

@@ -203,7 +203,8 @@ __global__ __launch_bounds__(256) void codes16_kernel(const uint8_t* src, T* cod
 int codes16_bias_cols(int K) { return (CODES16_TERMS * (K / 64) + 63) / 64 * 64; }
 size_t codes16_bytes(int N, int K) { return (size_t)N * ((size_t)K * 2 + (size_t)codes16_bias_cols(K) * 2 + (size_t)(K / 64) * 4); }
 
-size_t codes16_kept_bytes(int N, int K) { return codes16_bytes(N, K) + (size_t)N * codes16_bias_cols(K) * 2; }
+// (float32 rows, whose biases are last, are multiplied by bf16 models' codes alone)
+size_t codes16_kept_bytes(const LinearW& W) { return codes16_bytes(W.N, W.K) + (wk_scale_dtype(W.wk) == WK_BF16 ? (size_t)W.N * codes16_bias_cols(W.K) * 2 : 0); }
 
 // side_only: biases and scales without the codes
 static int codes16_into(const LinearW& src, void* codes, uint16_t* wb, float* sc, hipStream_t st, bool big_first, bool side_only) {
@@ -228,9 +229,10 @@ int launch_codes16(const LinearW& src, void* dst, hipStream_t st, bool big_first
 
 int launch_codes16_kept(const LinearW& src, void* dst, hipStream_t st, Codes16& out) {
   char* d = (char*)dst;
-  uint16_t* wb[2] = {(uint16_t*)(d + (size_t)src.N * src.K * 2), (uint16_t*)(d + codes16_bytes(src.N, src.K))};
+  const bool both = wk_scale_dtype(src.wk) == WK_BF16;
+  uint16_t* wb[2] = {(uint16_t*)(d + (size_t)src.N * src.K * 2), both ? (uint16_t*)(d + codes16_bytes(src.N, src.K)) : nullptr};
   float* sc = (float*)(d + (size_t)src.N * (src.K + codes16_bias_cols(src.K)) * 2);
-  for (int f32 = 0; f32 < 2; ++f32) MI_TRY(codes16_into(src, d, wb[f32], sc, st, f32 == 0, f32 == 1));
+  for (int f32 = 0; f32 < 1 + both; ++f32) MI_TRY(codes16_into(src, d, wb[f32], sc, st, f32 == 0, f32 == 1));
   out.codes = d; out.bias[0] = wb[0]; out.bias[1] = wb[1]; out.scales = sc;
   return MI_OK;
 }
@@ -239,7 +241,7 @@ Codes16 codes16_rows(const Codes16& c, int n0, int K) {
   Codes16 r = c;
   if (c.codes == nullptr) return r;
   r.codes = (const char*)c.codes + (size_t)n0 * K * 2;
-  for (int f32 = 0; f32 < 2; ++f32) r.bias[f32] = (const char*)c.bias[f32] + (size_t)n0 * codes16_bias_cols(K) * 2;
+  for (int f32 = 0; f32 < 2; ++f32) r.bias[f32] = c.bias[f32] != nullptr ? (const char*)c.bias[f32] + (size_t)n0 * codes16_bias_cols(K) * 2 : nullptr;
   r.scales = c.scales + (size_t)n0 * (K / 64);
   return r;
 }

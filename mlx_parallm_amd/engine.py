@@ -634,6 +634,10 @@ class Engine:
     def set_option(self, key: str, value: int) -> None:
         L.check(L.lib().mi_engine_set_option(self._h, key.encode(), int(value)))
 
+    def codes_bytes(self) -> int:
+        """Device memory of the copies that prefills of int4 / int8 models multiply (set_option("prefill_codes_copy", 0) gives it back)."""
+        return int(L.lib().mi_engine_codes_bytes(self._h))
+
     def sync(self) -> None:
         L.check(L.lib().mi_engine_sync(self._h))
 

@@ -111,14 +111,16 @@ class ContinuousScheduler:
         self.chunks = 0
 
     def _default_blocks(self, eng, block_tokens: int, kv_dtype: str) -> int:
-        """Arena size: every slot at full length if that fits in 80 % of the device memory that is free now, else what
-        fits (requests then wait for blocks instead of for slots: _fits)."""
+        """Arena size: every slot at full length if that fits in 80 % of the device memory that the weights leave free, else what
+        fits (requests then wait for blocks instead of for slots: _fits).  The engine's copies for prefills are no reason for a smaller
+        one: at most an eighth of that memory, they fit beside it."""
         per_row = (eng.max_positions + block_tokens - 1) // block_tokens
         full = self.max_slots * per_row + 1
         try:
             import torch
 
             free, _total = torch.cuda.mem_get_info(eng.device)
+            free += eng.codes_bytes()
             block_bytes = eng.kv_block_bytes(block_tokens, kv_dtype)
             return int(max(2 * per_row + 1, min(full, int(0.8 * free) // block_bytes)))
         except Exception:            # (no torch / no device query: the full size, and the allocation says if it is too much)

@@ -234,7 +234,8 @@ def test_the_last_piece_of_wide_logits_is_no_other_kernel(kv):
 @pytest.mark.parametrize("kv_dtype", ["model", "float32"])
 def test_kept_codes_and_codes_per_call_give_the_same_bits(bits, act, kv_dtype):
     """The copy that an engine makes of its quantised weights and the one made in front of a product hold the same: prompts' logits, and the logits of every position
-    in pieces of 32768 columns, with and without it (float32 caches: the other order of the biases)."""
+    in pieces of 32768 columns, with and without it (float32 caches: the other order of the biases).  1500 rows: q|k|v, gate|up, down and the logits run on the codes.
+    The copies take what codes_bytes says, are given back and made again; memory asked for in earnest comes before them; set in time, the option makes none."""
     from mlx_parallm_amd.engine import Engine, SampleArgs
 
     H, F, V = 1024, 2816, 33024
@@ -248,32 +249,61 @@ def test_kept_codes_and_codes_per_call_give_the_same_bits(bits, act, kv_dtype):
         scale = 2.0 / (2 ** bits - 1) / k ** 0.5
         e.set_tensor(name + ".scales", (scale * (1.0 + torch.rand((n, k // 64), generator=g, device="cuda"))).to(dt))
         e.set_tensor(name + ".biases", (-1.5 / k ** 0.5 * (1.0 + 0.3 * torch.randn((n, k // 64), generator=g, device="cuda"))).to(dt))
-    e = Engine(cfg, device=0, max_positions=1024, act_dtype=act)
-    put(e, "model.embed_tokens", V, H)
-    put(e, "lm_head", V, H)
-    for i in range(2):
-        p = f"model.layers.{i}."
-        for n, rows, cols in (("self_attn.q_proj", H, H), ("self_attn.k_proj", H, H), ("self_attn.v_proj", H, H), ("self_attn.o_proj", H, H), ("mlp.gate_proj", F, H),
-                              ("mlp.up_proj", F, H), ("mlp.down_proj", H, F)):
-            put(e, p + n, rows, cols)
-        for n in ("input_layernorm", "post_attention_layernorm"):
-            e.set_tensor(p + n + ".weight", torch.ones(H, device="cuda", dtype=dt))
-    e.set_tensor("model.norm.weight", torch.ones(H, device="cuda", dtype=dt))
-    e.finalize()
-    toks = np.random.default_rng(3).integers(0, V, (2, 450)).astype(np.int32)
-    kv = e.new_kv(2, capacity=512, kv_dtype=kv_dtype)
-    out = []
-    for kept in (1, 0):
-        e.set_option("prefill_codes_copy", kept)
+
+    def engine(kept):
+        e = Engine(cfg, device=0, max_positions=1024, act_dtype=act)
+        if not kept:
+            e.set_option("prefill_codes_copy", 0)
+        g.manual_seed(bits)
+        put(e, "model.embed_tokens", V, H)
+        put(e, "lm_head", V, H)
+        for i in range(2):
+            p = f"model.layers.{i}."
+            for n, rows, cols in (("self_attn.q_proj", H, H), ("self_attn.k_proj", H, H), ("self_attn.v_proj", H, H), ("self_attn.o_proj", H, H), ("mlp.gate_proj", F, H),
+                                  ("mlp.up_proj", F, H), ("mlp.down_proj", H, F)):
+                put(e, p + n, rows, cols)
+            for n in ("input_layernorm", "post_attention_layernorm"):
+                e.set_tensor(p + n + ".weight", torch.ones(H, device="cuda", dtype=dt))
+        e.set_tensor("model.norm.weight", torch.ones(H, device="cuda", dtype=dt))
+        e.finalize()
+        return e
+    toks = np.random.default_rng(3).integers(0, V, (3, 500)).astype(np.int32)
+
+    def results(e, kv):
         kv.reset()
         logits = np.asarray(e.forward(toks, kv)).copy()
         kv.reset()
         r = e.score_tokens(kv, toks, toks, SampleArgs(top_logprobs=3))
-        out.append((logits, np.asarray(r["logprobs"]).copy(), np.asarray(r["top_logprobs"]).copy()))
+        return logits, np.asarray(r["logprobs"]).copy(), np.asarray(r["top_logprobs"]).copy()
+
+    def bias_columns(k):                                         # (six products of a group's sum and its bias, whole K tiles)
+        return -(-6 * (k // 64) // 64) * 64
+    linears = [(V, H)] + [(3 * H, H), (H, H), (2 * F, H), (H, F)] * 2
+    want = sum(n * (2 * k + k // 64 * 4 + 2 * bias_columns(k) * (2 if act == "bfloat16" else 1)) for n, k in linears)
+    e = engine(True)
+    kv, out = e.new_kv(3, capacity=512, kv_dtype=kv_dtype), []
+    assert e.codes_bytes() == want
+    out.append(results(e, kv))
+    e.sync()
+    free = torch.cuda.mem_get_info()[0]
+    e.set_option("prefill_codes_copy", 0)
+    assert e.codes_bytes() == 0 and torch.cuda.mem_get_info()[0] - free >= 0.9 * want
+    out.append(results(e, kv))
+    e.set_option("prefill_codes_copy", 1)
+    assert e.codes_bytes() == want
+    with pytest.raises(RuntimeError, match="out of device memory"):
+        e.new_paged_kv(2, block_tokens=64, n_blocks=1 << 25, max_tokens_per_row=512, kv_dtype=kv_dtype)       # (17 TB)
+    assert e.codes_bytes() == 0
+    out.append(results(e, kv))
+    e.close()
+    e = engine(False)
+    assert e.codes_bytes() == 0
+    out.append(results(e, e.new_kv(3, capacity=512, kv_dtype=kv_dtype)))
     e.close()
     assert np.all(np.isfinite(out[0][0]))
-    for a, b in zip(*out):
-        assert np.array_equal(a, b)
+    for other in out[1:]:
+        for a, b in zip(out[0], other):
+            assert np.array_equal(a, b)
 
 
 @pytest.mark.parametrize("act", ["bfloat16", "float16"])

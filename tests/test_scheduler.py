@@ -37,6 +37,21 @@ def parts(tiny):
     return FakeModel(tiny, max_pos=2048), load_tokenizer(tiny)
 
 
+def test_the_default_arena_does_not_shrink_by_the_engines_copies(monkeypatch):
+    """80 % of what the weights leave free, with and without copies of 3 of 40 GB beside them; never more than every slot at full length."""
+    import types
+
+    import torch
+
+    def blocks(free, copies, slots=64):
+        eng = types.SimpleNamespace(max_positions=8192, device=0, kv_block_bytes=lambda tokens, dtype: 8 << 20, codes_bytes=lambda: copies)
+        monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device: (free - copies, 288 << 30))
+        return ContinuousScheduler._default_blocks(types.SimpleNamespace(max_slots=slots), eng, 64, "model")
+
+    assert blocks(40 << 30, 3 << 30) == blocks(40 << 30, 0) == int(0.8 * (40 << 30)) // (8 << 20)
+    assert blocks(280 << 30, 30 << 30) == 64 * 128 + 1
+
+
 def _alone(tiny, ids, n, eos):
     """The oracle's greedy continuation of one sequence on its own: (token ids without EOS, finish reason)."""
     ref = ref_generate.load(tiny, max_pos=2048)
