@@ -428,7 +428,7 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
   // ones: logits, the rounded call of layer 0, and gate|up up to 64 rows (28672 x 4096, 64 rows: 103 us against 116; 34816 x 5120 162 / 230; 96 rows
   // 154 / 117 and 243 / 244; the plain linears are ahead on the tile GEMM from 33 rows: 6144 x 4096 64 rows 38 / 31)
   auto tile_pays = [&]() {
-    if (quant) return gemm_prefill_quant_route(f.W, c, rows) != 0;
+    if (quant) return gemm_prefill_quant_route(f.W, c, rows, false) != 0;
     if (c.rnd != RND_NONE || c.epi == EPI_STORE_F32) return gemm_prefill_pays(false, c.kx > 0, c.rnd != RND_NONE, rows);
     return c.epi != EPI_SWIGLU || rows > 64;
   };

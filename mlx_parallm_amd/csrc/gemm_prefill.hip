@@ -1821,20 +1821,22 @@ static bool codes_plan(const LinearW& W, const GemvCall& c, size_t rows, int ldx
 
 // Float32 rows against a quantised matrix: the tile GEMM, or 32 rows per launch of the streaming kernel?  us of both, fitted to 16 shapes of int4 and int8:
 // a launch of the streaming kernel 11 + 0.30 per 2^20 weights + 0.5 per 1024 columns (6144 x 4096 20, 28672 x 4096 42 int4 and 45 int8, 2048 x 6400 20, 5120 x
-// 17408 54 and 57); the codes' copy 0.65 (none where one is kept), a round of workgroups 1.35 per K tile, the slices' reduce.  At 40 to 1365 rows of these the choice costs 0.2 % on
-// average over the better side, 12 % at most (28672 x 4096 SwiGLU: codes / streaming 192 rows 352 / 272, 256 rows 357 / 363, 512 rows 414 / 725; 6144 x 4096 96
-// rows 70 / 62, 129 rows 71 / 103; all int8), and int8, which the streaming kernel had at every size, is nowhere slower than there.
-static bool gemm_prefill_pays_codes(const LinearW& W, const GemvCall& c, size_t rows, int terms, size_t splitk_cap) {
+// 17408 54 and 57); the codes' copy 0.65, a round of workgroups 1.35 per K tile, the reduce of split256's slices.  own_copy: the call makes the copy of the codes.  The engine's calls
+// leave it out of the price whether or not they have one that is kept: the kernels differ in their last bits, and a prompt's are not to depend on the memory that was free at load time.
+// tail_plan's slices are not priced, so a SwiGLU stays on the streaming kernel for longer than it should.  Kernel times of both at 96 to 512 rows, 18 shapes of int4 and int8: with kept
+// codes the choice is never behind where it takes the codes and 7 % behind the better side on average (streaming / codes: 12800 x 2048 SwiGLU 224 rows 170 / 69, 256 rows 194 / 69,
+// taken; 28672 x 4096 SwiGLU 160 rows 226 / 210, 192 rows 271 / 214, taken; 34816 x 5120 SwiGLU 160 rows 378 / 292; 6144 x 4096 96 rows 65 / 65, 129 rows 108 / 67, both taken); with a
+// copy per call 4 % (6144 x 4096 96 rows 65 / 81, 4096 x 14336 129 rows 188 / 200, both taken).
+static bool gemm_prefill_pays_codes(const LinearW& W, const GemvCall& c, size_t rows, int terms, bool own_copy, size_t splitk_cap) {
   GemmParams p{};
   long blocks = 0;
   if (!codes_plan(W, c, rows, terms * W.K, terms, splitk_cap > 0, splitk_cap, p, blocks))
     return (c.rnd == RND_NONE && c.epi != EPI_STORE_F32) || gemm_prefill_pays(true, false, c.rnd != RND_NONE, rows);
-  // (the slices as they were when this was fitted; those of a last round alone, tail_plan, are no slower)
-  const int ks = c.epi != EPI_SWIGLU && splitk_cap > 0 && W.N % 4 == 0 ? split256(blocks, (p.ka + p.kb) / BK, rows * W.N * sizeof(float), splitk_cap) : 1;
+  const int ks = p.mb == 0 ? p.ksplit : 1;
   const int ncu = gemv_cu_count(), tiles = ((p.ka + p.kb) / BK + ks - 1) / ks;
   const double mw = (double)W.N * W.K / (1 << 20), rounds = (double)((blocks * ks + ncu - 1) / ncu);
   const double reduce = ks > 1 ? 2e-6 * ks * rows * W.N : 0.0;
-  return 12.0 + (W.codes.codes != nullptr ? 0.0 : 0.65 * mw) + 1.35 * rounds * tiles + reduce < (double)((rows + 31) / 32) * (11.0 + 0.30 * mw + 0.5 * W.K / 1024);
+  return 12.0 + (own_copy ? 0.65 * mw : 0.0) + 1.35 * rounds * tiles + reduce < (double)((rows + 31) / 32) * (11.0 + 0.30 * mw + 0.5 * W.K / 1024);
 }
 
 bool gemm_prefill_on_codes(const LinearW& W, const GemvCall& c, size_t rows) {
@@ -1844,12 +1846,12 @@ bool gemm_prefill_on_codes(const LinearW& W, const GemvCall& c, size_t rows) {
   return codes_plan(W, c, rows, c.act == MI_F32 ? terms * W.K : c.ldx, terms, false, 0, p, blocks);
 }
 
-int gemm_prefill_quant_route(const LinearW& W, const GemvCall& c, size_t rows) {
+int gemm_prefill_quant_route(const LinearW& W, const GemvCall& c, size_t rows, bool own_copy) {
   if (!gemm_prefill_supported(W, c, rows)) return 0;
   const bool x32 = c.act == MI_F32;
   const int terms = x32 && c.rnd != RND_BF16 ? 3 : 1;
   const size_t cap = rows < 4096 ? (size_t)128 << 20 : 0;                       // (of the engine's workspace for slices)
-  if (x32 && rows > 32 && gemm_skinny_supported(W, c, 32) && !gemm_prefill_pays_codes(W, c, rows, terms, cap)) return 0;
+  if (x32 && rows > 32 && gemm_skinny_supported(W, c, 32) && !gemm_prefill_pays_codes(W, c, rows, terms, own_copy, cap)) return 0;
   return gemm_prefill_on_codes(W, c, rows) ? 2 : 1;
 }
 

@@ -101,8 +101,8 @@ bool gemm_prefill_supported(const LinearW& W, const GemvCall& c, size_t rows);
 bool gemm_prefill_pays(bool codes, bool hilo, bool rounded, size_t rows);
 // can this call of split rows leave its SwiGLU as [hi | lo] rows (GemvCall::split_out)?  The 256 x 256 LDS-DMA tile alone does
 bool gemm_prefill_split_out(const LinearW& W, const GemvCall& c, size_t rows);
-// any prefill call on a quantised matrix: 2 = the tile GEMM on its codes, 1 = on its [hi | lo] copy, 0 = not the tile GEMM
-int gemm_prefill_quant_route(const LinearW& W, const GemvCall& c, size_t rows);
+// any prefill call on a quantised matrix: 2 = the tile GEMM on its codes, 1 = on its [hi | lo] copy, 0 = not the tile GEMM.  own_copy: priced with a copy of the codes
+int gemm_prefill_quant_route(const LinearW& W, const GemvCall& c, size_t rows, bool own_copy);
 bool gemm_prefill_on_codes(const LinearW& W, const GemvCall& c, size_t rows);     // .. once it is the tile GEMM
 // splitk_ws / splitk_cap: float32 workspace for the K-split form of the 128 x 128 tile (few hundred rows against a narrow
 // matrix); null = never split

@@ -197,7 +197,7 @@ int mi_op_gemm_quant_route(const mi_op_linear* w, const mi_op_gemv_args* a) {
   const LinearW W = to_linear(w);
   const GemvCall c = to_call(a);
   if (!wk_is_quant(W.wk)) return fail(MI_ERR_INVALID, "mi_op_gemm_quant_route: int4 / int8 weights");
-  return gemm_prefill_quant_route(W, c, (size_t)c.M);
+  return gemm_prefill_quant_route(W, c, (size_t)c.M, true);
 }
 
 int mi_op_gemv_reg(const mi_op_linear* w, const mi_op_gemv_args* a) {

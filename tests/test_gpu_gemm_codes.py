@@ -306,6 +306,36 @@ def test_kept_codes_and_codes_per_call_give_the_same_bits(bits, act, kv_dtype):
             assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("rows", [256, 97])
+def test_float32_prompts_take_one_route_with_and_without_kept_codes(rows):
+    """The streaming kernel and the codes differ in their last bits: which of them a prompt takes is no matter of the memory that was free at load time (gate|up at 256 rows
+    and the logits of 97 positions lie where the copy's price would decide)."""
+    from mlx_parallm_amd.engine import Engine
+
+    H, F, V = 2048, 6400, 32000
+    cfg = dict(model_type="llama", hidden_size=H, num_hidden_layers=1, num_attention_heads=16, num_key_value_heads=4, head_dim=128, intermediate_size=F, vocab_size=V,
+               rms_norm_eps=1e-5, rope_theta=10000.0, tie_word_embeddings=False, max_position_embeddings=512, quantization={"bits": 4, "group_size": 64})
+    out = []
+    for kept in (1, 0):
+        e = Engine(cfg, device=0, max_positions=512, act_dtype="bfloat16")
+        e.set_option("prefill_codes_copy", kept)
+        g = torch.Generator(device="cuda").manual_seed(1)
+        p = "model.layers.0."
+        for name, n, k in (("model.embed_tokens", V, H), ("lm_head", V, H), (p + "self_attn.q_proj", H, H), (p + "self_attn.k_proj", 512, H), (p + "self_attn.v_proj", 512, H),
+                           (p + "self_attn.o_proj", H, H), (p + "mlp.gate_proj", F, H), (p + "mlp.up_proj", F, H), (p + "mlp.down_proj", H, F)):
+            e.set_tensor(name + ".weight", torch.randint(-2 ** 31, 2 ** 31 - 1, (n, k // 8), generator=g, device="cuda", dtype=torch.int32))
+            e.set_tensor(name + ".scales", (2.0 / 15 / k ** 0.5 * (1.0 + torch.rand((n, k // 64), generator=g, device="cuda"))).bfloat16())
+            e.set_tensor(name + ".biases", (-1.5 / k ** 0.5 * (1.0 + 0.3 * torch.randn((n, k // 64), generator=g, device="cuda"))).bfloat16())
+        for n in (p + "input_layernorm", p + "post_attention_layernorm", "model.norm"):
+            e.set_tensor(n + ".weight", torch.ones(H, device="cuda", dtype=torch.bfloat16))
+        e.finalize()
+        assert (e.codes_bytes() > 0) == bool(kept)
+        toks = np.random.default_rng(3).integers(0, V, (1, rows)).astype(np.int32)
+        out.append(np.array(e.forward(toks, e.new_kv(1, capacity=300, kv_dtype="float32"), all_positions=True)))
+        e.close()
+    assert np.all(np.isfinite(out[0])) and np.array_equal(out[0], out[1])
+
+
 @pytest.mark.parametrize("act", ["bfloat16", "float16"])
 @pytest.mark.parametrize("bits,M,N,K,epi", [
     (4, 700, 2 * 11520, 1024, "swiglu"),     # 270 tiles: one round, and 15 in K slices
