@@ -478,10 +478,15 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
     // kernel is chosen for all of them: a last piece of few columns is no reason for the [hi | lo] copy
     c.codes = norm_sums || (quant && gemm_prefill_on_codes(f.W, c, rows));
     const int ncol = (wk_is_quant(f.W.wk) && c.epi == EPI_STORE_F32) ? std::min(f.W.N, 32768) : f.W.N;
+    // (before the scratch is sized: where the kept codes go for this, the scratch has to hold this call's)
+    if (rows < 4096 && e->gk_ws == nullptr) {     // K-split partial tiles of the tile GEMMs (one prompt of a few hundred to a few thousand rows)
+      e->gk_cap = (size_t)128 << 20;
+      if (dev_malloc(e, &e->gk_ws, e->gk_cap) != hipSuccess) e->gk_cap = 0;
+    }
     void* scratch = nullptr;
     if (wk_is_quant(f.W.wk)) {               // the GEMM multiplies by 16-bit codes, or a [hi | lo] 16-bit copy, made on the fly
       for (;;) {
-        LinearW part = f.W;
+        LinearW part = f.W;                    // (with the copy that is kept now: no allocation may stand between this loop and the launches below)
         part.N = ncol;
         const size_t need = gemm_prefill_scratch_bytes(part, c, rows);
         if (need <= e->deq_cap) break;
@@ -492,10 +497,6 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
         e->deq_cap = need;
       }
       scratch = e->deq_scratch;
-    }
-    if (rows < 4096 && e->gk_ws == nullptr) {     // K-split partial tiles of the tile GEMMs (one prompt of a few hundred to a few thousand rows)
-      e->gk_cap = (size_t)128 << 20;
-      if (dev_malloc(e, &e->gk_ws, e->gk_cap) != hipSuccess) e->gk_cap = 0;
     }
     for (int n0 = 0; n0 < f.W.N; n0 += ncol) {
       LinearW part = f.W;

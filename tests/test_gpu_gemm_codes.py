@@ -306,6 +306,45 @@ def test_kept_codes_and_codes_per_call_give_the_same_bits(bits, act, kv_dtype):
             assert np.array_equal(a, b)
 
 
+def test_the_kept_codes_go_for_the_slices_workspace_of_the_same_call():
+    """A prompt's workspace for slices of K (128 MiB, of its first call below 4096 rows) does not fit beside the copies: they go in the middle of that call, which then makes
+    its own copy in a scratch of that size.  The same logits as with room for all."""
+    from mlx_parallm_amd.engine import Engine
+
+    H, F, V = 1024, 2816, 65792
+    cfg = dict(model_type="llama", hidden_size=H, num_hidden_layers=1, num_attention_heads=8, num_key_value_heads=8, head_dim=128, intermediate_size=F, vocab_size=V,
+               rms_norm_eps=1e-5, rope_theta=10000.0, tie_word_embeddings=False, max_position_embeddings=2048, quantization={"bits": 4, "group_size": 64})
+    p, rng, out, MiB = "model.layers.0.", np.random.default_rng(3), [], 1 << 20
+    long, short = rng.integers(0, V, (3, 1400)).astype(np.int32), rng.integers(0, V, (3, 500)).astype(np.int32)
+    for full in (False, True):
+        e = Engine(cfg, device=0, max_positions=2048, act_dtype="bfloat16")
+        g = torch.Generator(device="cuda").manual_seed(1)
+        for name, n, k in (("model.embed_tokens", V, H), ("lm_head", V, H), (p + "self_attn.q_proj", H, H), (p + "self_attn.k_proj", H, H), (p + "self_attn.v_proj", H, H),
+                           (p + "self_attn.o_proj", H, H), (p + "mlp.gate_proj", F, H), (p + "mlp.up_proj", F, H), (p + "mlp.down_proj", H, F)):
+            e.set_tensor(name + ".weight", torch.randint(-2 ** 31, 2 ** 31 - 1, (n, k // 8), generator=g, device="cuda", dtype=torch.int32))
+            e.set_tensor(name + ".scales", (2.0 / 15 / k ** 0.5 * (1.0 + torch.rand((n, k // 64), generator=g, device="cuda"))).bfloat16())
+            e.set_tensor(name + ".biases", (-1.5 / k ** 0.5 * (1.0 + 0.3 * torch.randn((n, k // 64), generator=g, device="cuda"))).bfloat16())
+        for n in (p + "input_layernorm", p + "post_attention_layernorm", "model.norm"):
+            e.set_tensor(n + ".weight", torch.ones(H, device="cuda", dtype=torch.bfloat16))
+        e.finalize()
+        kv = e.new_kv(3, capacity=1408)
+        e.forward(long, kv)                                      # (4200 rows: everything but that workspace)
+        kv.reset()
+        e.sync()
+        torch.cuda.empty_cache()
+        held = []
+        while full and len(held) < 4 and torch.cuda.mem_get_info()[0] > 120 * MiB:      # (what is free is told to within a few parts in a thousand)
+            held.append(torch.empty(torch.cuda.mem_get_info()[0] - 108 * MiB, dtype=torch.uint8, device="cuda"))
+        assert not full or 64 * MiB < torch.cuda.mem_get_info()[0] < 128 * MiB
+        assert e.codes_bytes() > 128 * MiB
+        out.append(np.array(e.forward(short, kv)))
+        assert (e.codes_bytes() == 0) == full
+        e.close()
+        del held
+        torch.cuda.empty_cache()
+    assert np.all(np.isfinite(out[0])) and np.array_equal(out[0], out[1])
+
+
 @pytest.mark.parametrize("rows", [256, 97])
 def test_float32_prompts_take_one_route_with_and_without_kept_codes(rows):
     """The streaming kernel and the codes differ in their last bits: which of them a prompt takes is no matter of the memory that was free at load time (gate|up at 256 rows
