@@ -180,7 +180,7 @@ int ensure_workspace(mi_engine* e, size_t rows, size_t logit_rows, int B) {
   if (rows > e->d_tokens_cap) {
     MI_HIP(hipStreamSynchronize(e->stream));
     hipFree(e->d_tokens);
-    MI_HIP(hipMalloc(&e->d_tokens, rows * sizeof(int32_t)));
+    MI_HIP(dev_malloc(e, &e->d_tokens, rows * sizeof(int32_t)));
     e->d_tokens_cap = rows;
   }
   if (B > e->maxB) {
@@ -188,13 +188,13 @@ int ensure_workspace(mi_engine* e, size_t rows, size_t logit_rows, int B) {
     hipFree(e->d_next); hipFree(e->d_rowstats); hipFree(e->d_uniforms);      // (d_logprob / d_prob0 live in d_next's block)
     hipFree(e->d_topk_ids); hipFree(e->d_topk_lp);
     // tokens | logprobs | row-0 probabilities of a step in ONE block: one device-to-host copy per step instead of three
-    MI_HIP(hipMalloc(&e->d_next, (size_t)3 * B * sizeof(int32_t)));
+    MI_HIP(dev_malloc(e, &e->d_next, (size_t)3 * B * sizeof(int32_t)));
     e->d_logprob = (float*)(e->d_next + B);
     e->d_prob0 = (float*)(e->d_next + 2 * B);
-    MI_HIP(hipMalloc(&e->d_rowstats, 2 * B * sizeof(float)));
-    MI_HIP(hipMalloc(&e->d_uniforms, B * sizeof(float)));
-    MI_HIP(hipMalloc(&e->d_topk_ids, (size_t)B * MI_MAX_TOP_LOGPROBS * sizeof(int32_t)));
-    MI_HIP(hipMalloc(&e->d_topk_lp, (size_t)B * MI_MAX_TOP_LOGPROBS * sizeof(float)));
+    MI_HIP(dev_malloc(e, &e->d_rowstats, 2 * B * sizeof(float)));
+    MI_HIP(dev_malloc(e, &e->d_uniforms, B * sizeof(float)));
+    MI_HIP(dev_malloc(e, &e->d_topk_ids, (size_t)B * MI_MAX_TOP_LOGPROBS * sizeof(int32_t)));
+    MI_HIP(dev_malloc(e, &e->d_topk_lp, (size_t)B * MI_MAX_TOP_LOGPROBS * sizeof(float)));
     for (auto& s : e->slots) {
       hipHostFree(s.tokens); hipHostFree(s.topk_ids); hipHostFree(s.topk_lp);       // (logprob / prob0 live in tokens' block)
       MI_HIP(hipHostMalloc(&s.tokens, (size_t)3 * B * sizeof(int32_t)));
@@ -336,7 +336,7 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
           if (groups > e->sk_ctr_cap) {
             hipFree(e->sk_ctr); e->sk_ctr = nullptr; e->sk_ctr_cap = 0;
             const int cap = std::max(groups, 4096);
-            MI_HIP(hipMalloc(&e->sk_ctr, (size_t)cap * sizeof(unsigned)));
+            MI_HIP(dev_malloc(e, &e->sk_ctr, (size_t)cap * sizeof(unsigned)));
             MI_HIP(hipMemsetAsync(e->sk_ctr, 0, (size_t)cap * sizeof(unsigned), e->stream));
             e->sk_ctr_cap = cap;
           }
@@ -402,7 +402,7 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
     const int leave_ld = (c.act != MI_F32 && c.epi == EPI_RESID && !c.out32) ? gemm_skinny_handover_ld(f.W, c, rows) : 0;
     const bool produce = e->opt_norm_handover && leave_ld > 0 && tgroups <= 64 && c.ldo == f.W.N;
     if (produce) {
-      if (!e->d_sq) MI_HIP(hipMalloc(&e->d_sq, (size_t)4096 * 16 * sizeof(float)));     // (64 tile groups x <= 128 rows fit eight times)
+      if (!e->d_sq) MI_HIP(dev_malloc(e, &e->d_sq, (size_t)4096 * 16 * sizeof(float)));     // (64 tile groups x <= 128 rows fit eight times)
       c.sq_out = e->d_sq;
     }
     if (need > e->sk_ws_cap || groups > e->sk_ctr_cap) {
@@ -415,7 +415,7 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
       if (groups > e->sk_ctr_cap) {
         hipFree(e->sk_ctr); e->sk_ctr = nullptr; e->sk_ctr_cap = 0;
         const int cap = std::max(groups, 4096);
-        MI_HIP(hipMalloc(&e->sk_ctr, (size_t)cap * sizeof(unsigned)));
+        MI_HIP(dev_malloc(e, &e->sk_ctr, (size_t)cap * sizeof(unsigned)));
         MI_HIP(hipMemsetAsync(e->sk_ctr, 0, (size_t)cap * sizeof(unsigned), e->stream));
         e->sk_ctr_cap = cap;
       }
@@ -550,7 +550,7 @@ int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, Gemv
       if (groups > e->sk_ctr_cap) {
         hipFree(e->sk_ctr); e->sk_ctr = nullptr; e->sk_ctr_cap = 0;
         const int cap = std::max(groups, 4096);
-        MI_HIP(hipMalloc(&e->sk_ctr, (size_t)cap * sizeof(unsigned)));
+        MI_HIP(dev_malloc(e, &e->sk_ctr, (size_t)cap * sizeof(unsigned)));
         MI_HIP(hipMemsetAsync(e->sk_ctr, 0, (size_t)cap * sizeof(unsigned), e->stream));
         e->sk_ctr_cap = cap;
       }
@@ -622,8 +622,8 @@ bool can_pair(mi_engine* e, const FusedLinear& fa, GemvCall a, const FusedLinear
 
 int ensure_seam(mi_engine* e) {          // arrival counter + error flag of the in-launch seams
   if (e->d_seam_counter == nullptr) {
-    MI_HIP(hipMalloc(&e->d_seam_counter, sizeof(unsigned)));
-    MI_HIP(hipMalloc(&e->d_seam_error, sizeof(int)));
+    MI_HIP(dev_malloc(e, &e->d_seam_counter, sizeof(unsigned)));
+    MI_HIP(dev_malloc(e, &e->d_seam_error, sizeof(int)));
     MI_HIP(hipMemsetAsync(e->d_seam_counter, 0, sizeof(unsigned), e->stream));
     MI_HIP(hipMemsetAsync(e->d_seam_error, 0, sizeof(int), e->stream));
     MI_HIP(hipHostMalloc(&e->h_seam_err, (NSLOT + 1) * sizeof(int)));
@@ -788,14 +788,14 @@ int split_prefill(mi_engine* e, AttnCall& ac, int max_keys) {
   if (need > e->ap_part_cap) {
     MI_HIP(hipStreamSynchronize(e->stream));
     hipFree(e->ap_part); e->ap_part = nullptr; e->ap_part_cap = 0;
-    MI_HIP(hipMalloc(&e->ap_part, need * sizeof(float)));
+    MI_HIP(dev_malloc(e, &e->ap_part, need * sizeof(float)));
     e->ap_part_cap = need;
   }
   if (ctr > e->ap_ctr_cap) {
     MI_HIP(hipStreamSynchronize(e->stream));
     hipFree(e->ap_ctr); e->ap_ctr = nullptr; e->ap_ctr_cap = 0;
     const size_t cap = std::max<size_t>(ctr, 256);       // (at most one tile per CU where the keys are split)
-    MI_HIP(hipMalloc(&e->ap_ctr, cap * sizeof(int)));
+    MI_HIP(dev_malloc(e, &e->ap_ctr, cap * sizeof(int)));
     MI_HIP(hipMemsetAsync(e->ap_ctr, 0, cap * sizeof(int), e->stream));
     e->ap_ctr_cap = cap;
   }
@@ -834,7 +834,7 @@ int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool wan
       return fail(MI_ERR_INVALID, "forward: KV capacity / max_positions exceeded (call mi_kv_reserve)");
   const int32_t* d_rows = nullptr;
   if (rows) {
-    if (!kv->d_rows) MI_HIP(hipMalloc(&kv->d_rows, kv->B * sizeof(int32_t)));
+    if (!kv->d_rows) MI_HIP(dev_malloc(e, &kv->d_rows, kv->B * sizeof(int32_t)));
     MI_HIP(hipMemcpyAsync(kv->d_rows, rows, B * sizeof(int32_t), hipMemcpyHostToDevice, st));
     d_rows = kv->d_rows;
   }
@@ -853,7 +853,7 @@ int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool wan
     if (kv->partial == nullptr || kv->partial_splits < nsplit) {
       MI_HIP(hipStreamSynchronize(st));
       hipFree(kv->partial);
-      MI_HIP(hipMalloc(&kv->partial, (size_t)kv->B * Hq * 16 * (D + 2) * sizeof(float)));
+      MI_HIP(dev_malloc(e, &kv->partial, (size_t)kv->B * Hq * 16 * (D + 2) * sizeof(float)));
       kv->partial_splits = 16;
     }
     (void)need;
@@ -984,7 +984,7 @@ int forward_mixed(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t* l
   // weight-streaming kernel for short calls, the K-split 128 x 128 tile for a few hundred rows, plain tiles above).
   e->cur_L = R == (size_t)nd ? 1 : 2;
   e->sq_valid = false;
-  if (!kv->d_rows) MI_HIP(hipMalloc(&kv->d_rows, kv->B * sizeof(int32_t)));
+  if (!kv->d_rows) MI_HIP(dev_malloc(e, &kv->d_rows, kv->B * sizeof(int32_t)));
   MI_HIP(hipMemcpyAsync(kv->d_rows, rows, n * sizeof(int32_t), hipMemcpyHostToDevice, st));
   for (int i = 0; i < n; ++i) MI_TRY(kv_ensure_blocks(kv, rows[i], kv->h_off[rows[i]] + lens[i]));
   MI_TRY(kv_upload_table(kv, st));
@@ -999,7 +999,7 @@ int forward_mixed(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t* l
   if (nsplit > 1 && (kv->partial == nullptr || kv->partial_splits < nsplit)) {
     MI_HIP(hipStreamSynchronize(st));
     hipFree(kv->partial);
-    MI_HIP(hipMalloc(&kv->partial, (size_t)kv->B * Hq * 16 * (D + 2) * sizeof(float)));
+    MI_HIP(dev_malloc(e, &kv->partial, (size_t)kv->B * Hq * 16 * (D + 2) * sizeof(float)));
     kv->partial_splits = 16;
   }
   for (int li = 0; li < d.num_layers; ++li) {
@@ -1060,7 +1060,7 @@ int forward_mixed(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t* l
   if (n_out > 0) {                               // hidden states of the wanted positions -> compact rows -> head
     std::vector<int32_t> idx;
     for (int i = 0; i < n; ++i) if (want[i]) idx.push_back((int32_t)(tok0[i] + lens[i] - 1));
-    if (!e->d_gather) MI_HIP(hipMalloc(&e->d_gather, 4096 * sizeof(int32_t)));
+    if (!e->d_gather) MI_HIP(dev_malloc(e, &e->d_gather, 4096 * sizeof(int32_t)));
     if (idx.size() > 4096) return fail(MI_ERR_INVALID, "mixed step: too many sampled rows");
     MI_HIP(hipMemcpyAsync(e->d_gather, idx.data(), idx.size() * sizeof(int32_t), hipMemcpyHostToDevice, st));
     MI_TRY(launch_gather_rows(e->h, (size_t)H * es, e->d_gather, (int)idx.size(), e->xn, st));
@@ -1111,7 +1111,7 @@ int run_sample(mi_engine* e, int B, const mi_sample_params* sp, const int32_t* f
   hipStream_t st = e->stream;
   if (sp->n_logit_bias > 0) {
     if (sp->n_logit_bias > 4096) return fail(MI_ERR_INVALID, "too many logit_bias entries");
-    if (!e->d_bias_ids) { MI_HIP(hipMalloc(&e->d_bias_ids, 4096 * sizeof(int32_t))); MI_HIP(hipMalloc(&e->d_bias_vals, 4096 * sizeof(float))); }
+    if (!e->d_bias_ids) { MI_HIP(dev_malloc(e, &e->d_bias_ids, 4096 * sizeof(int32_t))); MI_HIP(dev_malloc(e, &e->d_bias_vals, 4096 * sizeof(float))); }
     MI_HIP(hipMemcpyAsync(e->d_bias_ids, sp->logit_bias_ids, sp->n_logit_bias * sizeof(int32_t), hipMemcpyHostToDevice, st));
     MI_HIP(hipMemcpyAsync(e->d_bias_vals, sp->logit_bias_values, sp->n_logit_bias * sizeof(float), hipMemcpyHostToDevice, st));
   }
@@ -1121,7 +1121,7 @@ int run_sample(mi_engine* e, int B, const mi_sample_params* sp, const int32_t* f
     if ((size_t)B > e->d_rowpar_cap) {
       MI_HIP(hipStreamSynchronize(st));
       hipFree(e->d_rowpar);
-      MI_HIP(hipMalloc(&e->d_rowpar, 2 * (size_t)B * sizeof(float)));
+      MI_HIP(dev_malloc(e, &e->d_rowpar, 2 * (size_t)B * sizeof(float)));
       e->d_rowpar_cap = B;
     }
     MI_HIP(hipMemcpyAsync(e->d_rowpar, sp->row_temperature, B * sizeof(float), hipMemcpyHostToDevice, st));
@@ -1293,8 +1293,8 @@ int mi_engine_set_lora(mi_engine* e, int layer, const char* proj, const void* A,
   MI_HIP(hipStreamSynchronize(e->stream));
   hipFree(f->lora_a[slot]); hipFree(f->lora_b[slot]);
   f->lora_a[slot] = f->lora_b[slot] = nullptr;
-  MI_HIP(hipMalloc(&f->lora_a[slot], (size_t)K * rank * sizeof(float)));
-  MI_HIP(hipMalloc(&f->lora_b[slot], (size_t)rank * n * sizeof(float)));
+  MI_HIP(dev_malloc(e, &f->lora_a[slot], (size_t)K * rank * sizeof(float)));
+  MI_HIP(dev_malloc(e, &f->lora_b[slot], (size_t)rank * n * sizeof(float)));
   MI_TRY(copy_in(f->lora_a[slot], A, (size_t)K * rank * sizeof(float), on_device, e->stream));
   MI_TRY(copy_in(f->lora_b[slot], B, (size_t)rank * n * sizeof(float), on_device, e->stream));
   f->W.lora_a[slot] = f->lora_a[slot]; f->W.lora_b[slot] = f->lora_b[slot];
@@ -1619,7 +1619,7 @@ int mi_score_tokens(mi_engine* e, mi_kv* kv, const int32_t* tokens, const int32_
   if (R > e->d_forced_cap) {
     MI_HIP(hipStreamSynchronize(st));
     hipFree(e->d_forced);
-    MI_HIP(hipMalloc(&e->d_forced, R * sizeof(int32_t)));
+    MI_HIP(dev_malloc(e, &e->d_forced, R * sizeof(int32_t)));
     e->d_forced_cap = R;
   }
   MI_TRY(upload_tokens(e, tokens, B, L));

@@ -306,9 +306,10 @@ def test_kept_codes_and_codes_per_call_give_the_same_bits(bits, act, kv_dtype):
             assert np.array_equal(a, b)
 
 
-def test_the_kept_codes_go_for_the_slices_workspace_of_the_same_call():
-    """A prompt's workspace for slices of K (128 MiB, of its first call below 4096 rows) does not fit beside the copies: they go in the middle of that call, which then makes
-    its own copy in a scratch of that size.  The same logits as with room for all."""
+@pytest.mark.parametrize("what", ["slices", "splits"])
+def test_the_kept_codes_go_for_a_workspace_in_the_middle_of_a_call(what):
+    """A workspace does not fit beside the copies: they go in the middle of the call that asks for it.  slices: a prompt's, for slices of K (128 MiB, of the first call below 4096
+    rows), and the call then makes its own copy of the codes in a scratch of that size; splits: the decode attention's, for 2048 slots.  The same logits as with room for all."""
     from mlx_parallm_amd.engine import Engine
 
     H, F, V = 1024, 2816, 65792
@@ -327,9 +328,13 @@ def test_the_kept_codes_go_for_the_slices_workspace_of_the_same_call():
         for n in (p + "input_layernorm", p + "post_attention_layernorm", "model.norm"):
             e.set_tensor(n + ".weight", torch.ones(H, device="cuda", dtype=torch.bfloat16))
         e.finalize()
-        kv = e.new_kv(3, capacity=1408)
-        e.forward(long, kv)                                      # (4200 rows: everything but that workspace)
-        kv.reset()
+        if what == "slices":
+            kv = e.new_kv(3, capacity=1408)
+            e.forward(long, kv)                                  # (4200 rows: everything but that workspace)
+            kv.reset()
+        else:
+            kv = e.new_paged_kv(2048, block_tokens=64, n_blocks=64, max_tokens_per_row=1536)
+            e.forward_segments(kv, [7], [long[0]], want=[1399])
         e.sync()
         torch.cuda.empty_cache()
         held = []
@@ -337,7 +342,7 @@ def test_the_kept_codes_go_for_the_slices_workspace_of_the_same_call():
             held.append(torch.empty(torch.cuda.mem_get_info()[0] - 108 * MiB, dtype=torch.uint8, device="cuda"))
         assert not full or 64 * MiB < torch.cuda.mem_get_info()[0] < 128 * MiB
         assert e.codes_bytes() > 128 * MiB
-        out.append(np.array(e.forward(short, kv)))
+        out.append(np.array(e.forward(short, kv) if what == "slices" else e.forward_segments(kv, [7], [short[0, :1]], want=[0])))
         assert (e.codes_bytes() == 0) == full
         e.close()
         del held
