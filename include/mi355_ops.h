@@ -101,7 +101,7 @@ int mi_op_gemm_prefill(const mi_op_linear* w, const mi_op_gemv_args* a, int iter
 int mi_op_gemm_codes(const mi_op_linear* w, const mi_op_gemv_args* a, int iters, float* avg_ms);
 /* what a prefill call of a->M rows on tile-major int4 / int8 weights runs on: 2 the tile GEMM on their codes, 1 the tile GEMM on their [hi | lo] copy, 0
  * another kernel (float32 activations: 32 rows per launch of the streaming one); a negative error code.  No device needed; no pointer is read.
- * For calls that make their copy of the codes, as mi_op_gemm_codes does; an engine's float32 rows take the codes from fewer rows on, as its copies are kept. */
+ * For calls that make their copy of the codes, as mi_op_gemm_codes does; an engine's float32 rows are priced without that copy and take the codes from fewer rows on. */
 int mi_op_gemm_quant_route(const mi_op_linear* w, const mi_op_gemv_args* a);
 /* gemv_reg.hip on its own: the decode linears of at most 8 rows on tile-major weights -- int4 / int8 (group 64) with scales of the
  * activations' type (plain / float32 / residual / SwiGLU epilogues, the last with the norm), dense 16-bit ones with activations of

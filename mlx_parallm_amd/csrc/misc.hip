@@ -494,7 +494,7 @@ __global__ __launch_bounds__(ST) void sample_kernel(SampleCall c) {
   float lp_scale = 1.0f, lp_lse = lse - mx;
   if (c.lp_temp && temperature > 0.f) {
     lp_scale = 1.0f / temperature;
-    float st = se;                               // T = 1: the sum of the pass above, term for term (no second walk of the row)
+    float st = se;                               // T = 1: the sum of the walk above (no second one)
     if (lp_scale != 1.0f) {                      // (uniform)
       st = 0.f;
       for_row(lg, V, [&](float l, int) { st += __expf((l - mx) * lp_scale); });
