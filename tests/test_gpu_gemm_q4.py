@@ -123,3 +123,23 @@ def test_norm_in_front_by_pieces_of_the_row(act, M, K):
     gemm_skinny(ol, xd, M, act, epi=L.EPI_STORE, out=out, ldo=48, norm_w=nwd, eps=1e-5, ksplit=q4_force(rows=1))
     assert np.all(host(out)[M:] == 7.0)
     _assert_close(host(out)[:M], round_to(matmul_nt(ref_model.rms_norm(x, act, nw, act, 1e-5)[0], w), act), act)
+
+
+@pytest.mark.parametrize("K,narrow", [(384, False), (512, True)])
+def test_where_the_narrow_kernel_begins_without_a_norm(K, narrow):
+    """By the bits: of half a million results the two kernels round some hundred differently."""
+    act, M, N = "bfloat16", 128, 4096
+    keep = [torch.randint(-2 ** 31, 2 ** 31 - 1, (N, K // 8), device="cuda", dtype=torch.int32), (0.01 + 0.01 * torch.rand((N, K // 64), device="cuda")).to(torch.bfloat16),
+            (-0.1 * torch.rand((N, K // 64), device="cuda")).to(torch.bfloat16)]
+    ol = op_linear("q4_bf16", N, K, *keep)
+    assert to_tiled(ol, keep)
+    x = torch.randn((M, K), device="cuda").to(torch.bfloat16)
+
+    def bits(ksplit):
+        out = torch.zeros((M, N), dtype=torch.bfloat16, device="cuda")
+        used = gemm_skinny(ol, x, M, act, epi=L.EPI_STORE, out=out, ldo=N, ksplit=ksplit)[0]
+        return host(out), used
+    chosen, used = bits(0)
+    rows, streaming = bits(q4_force(rows=1))[0], bits(used)[0]
+    assert not np.array_equal(rows, streaming)
+    assert np.array_equal(chosen, rows if narrow else streaming)
