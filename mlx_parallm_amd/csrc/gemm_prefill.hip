@@ -1766,15 +1766,20 @@ size_t gemm_prefill_scratch_bytes(const LinearW& W, const GemvCall& c, size_t ro
   return std::max(dequant_hilo_bytes(W.N, W.K), codes16_bytes(W.N, W.K) + sums);
 }
 
-// us of a launch over `blocks` tiles of `nk` K tiles in rounds of one workgroup per CU, those from `tail` on as `ks` slices: a round 10 + 2 per K tile (float32 rows, whose three walks
-// find W and x in the caches: 1.35), what joins the slices 3 + their 256 KiB each at 4.9 TB/s (fitted: 6144 x 4096, 700 rows, 7 slices 66 + 23, 4096 x 14336 with 5 94 + 15,
-// 28672 x 4096 SwiGLU, unsplit, 277)
-static double tail_us(long blocks, long tail, int nk, int ks, double tile_us, int ncu) {
-  const auto rounds = [&](long n) { return (double)((n + ncu - 1) / ncu); };
-  const double full = rounds(tail) * (10.0 + tile_us * nk);
-  if (tail == blocks) return full;
-  const long t = blocks - tail;
-  return full + rounds(t * ks) * (10.0 + tile_us * ((nk + ks - 1) / ks)) + 3.0 + t * ks * 0.262144 / 4.9;
+// us of a launch over `blocks` tiles of `nk` K tiles in rounds of one workgroup per CU, those from `tail` on as `ks` slices.  16-bit rows: a full round 10 + 2 per K tile; one that leaves
+// CUs idle has the power that they do not draw, 0.72 to 0.92 of that per K tile; what joins the slices 3 + 0.09 each (writing 256 KiB at the end of the loop, and reading them).  Prompts of
+// one document through six layers, int4, us a layer that slices give, by this and measured: 48 tiles (3072 x 4096, 300 rows) 56 / 52, 72 tiles 44 / 41, 120 26 / 24, 88 32 / 32, 336 (14336 x
+// 4096, 700 rows) 52 / 35, 272 (17408 x 5120, 512 rows) 96 / 88, 88 of 35 K tiles (5632 x 2048) 6 / 9; none by this: 144 tiles -10, 132 -6, 408 -8, 680 -8 (they were sliced while every
+// round counted as a full one).  Float32 rows: 1.35 per K tile, as their three walks find W and x in the caches, and 256 KiB at 4.9 TB/s.
+static double tail_us(long blocks, long tail, int nk, int ks, bool x3, int ncu) {
+  const auto rounds = [&](long n, int tiles) {
+    const long part = n % ncu;
+    const double tile = x3 ? 1.35 : 2.0;
+    return (double)(n / ncu) * (10.0 + tile * tiles) + (part > 0 ? 10.0 + tile * tiles * (x3 ? 1.0 : 0.72 + 0.2 * part / ncu) : 0.0);
+  };
+  if (tail == blocks) return rounds(blocks, nk);
+  const long slices = (blocks - tail) * ks;
+  return rounds(tail, nk) + rounds(slices, (nk + ks - 1) / ks) + 3.0 + slices * (x3 ? 0.262144 / 4.9 : 0.09);
 }
 
 // K slices for the tiles of a last, partly filled round (all of them where there is only that round) of a call that split256 leaves whole: the cheapest by the line above, at least
@@ -1785,12 +1790,11 @@ static double tail_us(long blocks, long tail, int nk, int ks, double tile_us, in
 // 28672 x 4096, 64 rows 1.008, 12800 x 2048, 300 rows 1.02, 6144 x 1024, 1024 rows 1.03; three to eight slices 0.78 to 1.00 over 4 shapes and 7 row counts).
 static void tail_plan(long mb, long blocks, int nk, bool x3, size_t cap, GemmParams& p) {
   const int ncu = gemv_cu_count();
-  const double tile_us = x3 ? 1.35 : 2.0;
-  double best = tail_us(blocks, blocks, nk, 1, tile_us, ncu) - (x3 ? 10.0 : 5.0);       // (what the line is sure of)
+  double best = tail_us(blocks, blocks, nk, 1, x3, ncu) - (x3 ? 10.0 : 5.0);       // (what the line is sure of)
   for (const long tail : {blocks / ncu * ncu / mb * mb, 0L}) {
     for (int ks = x3 ? 3 : 2; ks <= 8 && nk / ks >= 8 && (size_t)(blocks - tail) * ks * (BM2 * BN2 * 4) <= cap; ++ks) {
       if (tail == blocks) break;
-      const double t = tail_us(blocks, tail, nk, ks, tile_us, ncu);
+      const double t = tail_us(blocks, tail, nk, ks, x3, ncu);
       if (t < best) { best = t; p.mb = (int)mb; p.tail = (int)tail; p.ksplit = ks; }
     }
   }
