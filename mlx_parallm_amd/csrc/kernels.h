@@ -26,6 +26,7 @@ struct LinearW {
   const float* lora_b[2] = {nullptr, nullptr};
   int lora_row0[2] = {0, 0}, lora_n[2] = {0, 0}, lora_rank[2] = {0, 0};
   float lora_scale[2] = {0.f, 0.f};
+  bool centred = false;        // int4 on float32 rows: the streaming kernel's form with centred codes (a matrix that was the generic kernel's before its K was padded)
   Codes16 codes;               // quantised matrices: a copy of the codes that the prefill GEMM multiplies, if one is kept
 };
 

@@ -421,3 +421,34 @@ def test_q4_default_plan_on_wide_matrices(act, kind, M):
     out = torch.zeros((M, N), dtype=torch.float32, device="cuda")
     gemm_skinny(ol, xd, M, act, epi=L.EPI_STORE_F32, out=out, ldo=N)
     _assert_close(host(out), round_to(matmul_nt(x, wdense), act), act)
+
+
+@pytest.mark.parametrize("kind", ["q4_f16", "q8_f16"])
+@pytest.mark.parametrize("M,N,K,ksplit", [(1, 80, 128, 1), (8, 256, 4608, 0), (16, 144, 384, 3), (27, 256, 1024, 2)])
+@pytest.mark.parametrize("rnd", [L.RND_NONE, L.RND_F16])
+def test_float32_activations_on_quantised_f16_weights(kind, M, N, K, ksplit, rnd):
+    """A quantised float16 model with float32 caches: exact bf16 codes, float16 scales, x in three bf16 terms.  Against the float64 product: K roundings
+    of 2^-24 of a partial sum, which is some K^-1/2 of the sum of the absolute products, add up to K^1/2 of them, so 2^-24 of that sum; times four."""
+    rng = np.random.default_rng(M * N + K)
+    ol, wdense, keep = _weight(kind, N, K, rng)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    if rnd:
+        x = round_to(x, "float16")
+    xd = dev(x, "float32")
+    want = x.astype(np.float64) @ wdense.astype(np.float64).T
+    tol = 4.0 * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(wdense).astype(np.float64).T) + (2.0 ** -11 * np.abs(want) if rnd else 0.0)
+    out = torch.full((M + 1, N), 7.0, dtype=torch.float32, device="cuda")
+    gemm_skinny(ol, xd, M, "float32", epi=L.EPI_STORE, out=out, ldo=N, ksplit=ksplit, rnd=rnd)
+    got = host(out).astype(np.float64)
+    assert np.all(got[M:] == 7.0) and np.all(np.abs(got[:M] - want) <= tol), np.abs((got[:M] - want) / tol).max()
+    h = rng.standard_normal((M, N)).astype(np.float32)
+    hd = dev(h, "float32")
+    gemm_skinny(ol, xd, M, "float32", epi=L.EPI_RESID, resid=hd, ldo=N, ksplit=ksplit)
+    assert np.all(np.abs(host(hd) - (h + want)) <= tol + 2.0 ** -23 * (np.abs(h) + np.abs(want)))
+    if N % 32 == 0:
+        I = N // 2
+        g, u = want[:, :I], want[:, I:]
+        out = torch.zeros((M, I), dtype=torch.float32, device="cuda")
+        gemm_skinny(ol, xd, M, "float32", epi=L.EPI_SWIGLU, out=out, ldo=I, pair_offset=I, ksplit=1)
+        w2 = g / (1.0 + np.exp(-g)) * u                       # (the unit's slope in g is at most 1.1, times u)
+        assert np.all(np.abs(host(out) - w2) <= 1.1 * (np.abs(u) * tol[:, :I] + np.abs(g) * tol[:, I:]) + 2.0 ** -21 * np.abs(w2) + 1e-7)
