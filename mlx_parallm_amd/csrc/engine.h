@@ -18,6 +18,7 @@ struct FusedLinear {
   int parts = 0;                 // bit mask of sub-tensors seen (weight / scales / biases per part)
   int n_parts = 1;
   int part_rows[3] = {0, 0, 0};
+  int part_pad = 0, k_pad = 0;   // zero rows behind every part, zero columns behind K (mi_engine::ff)
   bool quant = false;
   int dense_dtype = -1, scale_dtype = -1;
   size_t w_bytes = 0, s_bytes = 0;
@@ -135,6 +136,10 @@ struct mi_engine {
   FusedLinear embed, lm_head;
   void* final_norm = nullptr; void* final_norm32 = nullptr;
   bool finalized = false;
+  // Columns of the feed-forward's activations: intermediate_size, of int4 models (groups of 64) the next multiple of 128, a block of the tile-major
+  // layout -- zero rows of gate and up, zero columns of down.  The matrix-core kernels take every width then: 5120 x 14656 was left to the generic
+  // kernel, 8 rows a pass over the matrix (seven layers, four mixed steps of 31 + 64 rows: 47.2 ms, 7.5 now; one of 3 rows at 2600 tokens, 3072 x 11072: 8.8, 5.7).
+  int ff = 0;
   float* cos_tab = nullptr; float* sin_tab = nullptr;
   // workspace
   size_t ws_rows = 0; size_t ws_logit_rows = 0;

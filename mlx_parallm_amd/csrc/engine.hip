@@ -50,7 +50,21 @@ int set_linear(mi_engine* e, FusedLinear& f, int part, int K, int kind, const vo
   if (ndim != 2) return fail(MI_ERR_INVALID, name + ": expected a 2-D tensor");
   const int rows = f.part_rows[part];
   int total = 0, row0 = 0;
-  for (int i = 0; i < f.n_parts; ++i) { if (i < part) row0 += f.part_rows[i]; total += f.part_rows[i]; }
+  for (int i = 0; i < f.n_parts; ++i) { if (i < part) row0 += f.part_rows[i] + f.part_pad; total += f.part_rows[i] + f.part_pad; }
+  // rows of `bytes` into the matrix, whose rows are `pad` longer
+  auto put = [&](void*& dst, size_t& had, size_t bytes, size_t pad) -> int {
+    const size_t ld = bytes + pad;
+    if (dst == nullptr) {
+      had = ld * total;
+      MI_HIP(hipMalloc(&dst, had));
+      if (f.part_pad > 0 || pad > 0) MI_HIP(hipMemsetAsync(dst, 0, had, e->stream));
+    }
+    char* to = (char*)dst + (size_t)row0 * ld;
+    if (pad == 0) return copy_in(to, data, bytes * rows, on_device, e->stream);
+    MI_HIP(hipMemcpy2DAsync(to, ld, data, bytes, bytes, rows, on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, e->stream));
+    MI_HIP(hipStreamSynchronize(e->stream));
+    return MI_OK;
+  };
   if (shape[0] != rows) return fail(MI_ERR_INVALID, name + ": wrong number of rows");
   if (kind == 0) {
     const bool packed = dtype == MI_U32;
@@ -60,12 +74,8 @@ int set_linear(mi_engine* e, FusedLinear& f, int part, int K, int kind, const vo
     if (!packed && dtype != d.act_dtype)
       return fail(MI_ERR_UNSUPPORTED, name + ": dense weight dtype differs from the model dtype");
     if (f.w != nullptr && f.quant != packed) return fail(MI_ERR_UNSUPPORTED, name + ": fused parts mix dense and quantised weights");
-    const size_t row_bytes = (size_t)cols * dtype_size(dtype);
-    if (f.w == nullptr) {
-      f.quant = packed; f.dense_dtype = packed ? -1 : dtype; f.w_bytes = row_bytes * total;
-      MI_HIP(hipMalloc(&f.w, f.w_bytes));
-    }
-    MI_TRY(copy_in((char*)f.w + (size_t)row0 * row_bytes, data, row_bytes * rows, on_device, e->stream));
+    if (f.w == nullptr) { f.quant = packed; f.dense_dtype = packed ? -1 : dtype; }
+    MI_TRY(put(f.w, f.w_bytes, (size_t)cols * dtype_size(dtype), packed ? (size_t)f.k_pad * d.quant_bits / 8 : f.k_pad * dtype_size(dtype)));
     f.seen_w[part] = 1;
   } else {
     if (d.quant_bits == 0) return fail(MI_ERR_INVALID, name + ": scales/biases but desc.quant_bits == 0");
@@ -75,10 +85,7 @@ int set_linear(mi_engine* e, FusedLinear& f, int part, int K, int kind, const vo
     if (dtype != MI_F32 && dtype != MI_BF16 && dtype != MI_F16) return fail(MI_ERR_INVALID, name + ": bad dtype");
     if (f.scale_dtype >= 0 && f.scale_dtype != dtype) return fail(MI_ERR_UNSUPPORTED, name + ": mixed scale dtypes");
     f.scale_dtype = dtype;
-    const size_t row_bytes = (size_t)cols * dtype_size(dtype);
-    void*& dst = kind == 1 ? f.scales : f.biases;
-    if (dst == nullptr) { f.s_bytes = row_bytes * total; MI_HIP(hipMalloc(&dst, f.s_bytes)); }
-    MI_TRY(copy_in((char*)dst + (size_t)row0 * row_bytes, data, row_bytes * rows, on_device, e->stream));
+    MI_TRY(put(kind == 1 ? f.scales : f.biases, f.s_bytes, (size_t)cols * dtype_size(dtype), f.k_pad / d.quant_group_size * dtype_size(dtype)));
     (kind == 1 ? f.seen_s : f.seen_b)[part] = 1;
   }
   return MI_OK;
@@ -95,7 +102,7 @@ int set_vector(mi_engine* e, void*& dst, int n, const void* data, const int64_t*
 int finalize_linear(mi_engine* e, FusedLinear& f, int K, const std::string& name) {
   int total = 0;
   for (int i = 0; i < f.n_parts; ++i) {
-    total += f.part_rows[i];
+    total += f.part_rows[i] + f.part_pad;
     if (!f.seen_w[i]) return fail(MI_ERR_NOTFOUND, name + ": weight not set");
     if (f.quant && (!f.seen_s[i] || !f.seen_b[i])) return fail(MI_ERR_NOTFOUND, name + ": scales/biases not set");
   }
@@ -103,7 +110,7 @@ int finalize_linear(mi_engine* e, FusedLinear& f, int K, const std::string& name
     return fail(MI_ERR_UNSUPPORTED, name + ": scale dtype differs from the model dtype");
   f.W.wk = kind_of(f, e->d.quant_bits);
   f.W.w = f.w; f.W.scales = f.scales; f.W.biases = f.biases;
-  f.W.N = total; f.W.K = K; f.W.group = e->d.quant_group_size > 0 ? e->d.quant_group_size : 64;
+  f.W.N = total; f.W.K = K + f.k_pad; f.W.centred = f.k_pad > 0 && f.quant; f.W.group = e->d.quant_group_size > 0 ? e->d.quant_group_size : 64;
   // "repack weights": tile-major layout for the matrices the streaming kernels read (repack.hip)
   if (e->opt_tile_weights && tiled_supported(f.W.wk, f.W.N, f.W.K, f.W.group)) {
     void* dst = nullptr;
@@ -165,7 +172,7 @@ int ensure_workspace(mi_engine* e, size_t rows, size_t logit_rows, int B) {
     MI_HIP(dev_malloc(e, &e->qkv, rows * nqkv * es));
     MI_HIP(dev_malloc(e, &e->q, rows * (size_t)d.num_heads * d.head_dim * es));
     MI_HIP(dev_malloc(e, &e->attn, rows * (size_t)d.num_heads * d.head_dim * es));
-    MI_HIP(dev_malloc(e, &e->act, rows * (size_t)d.intermediate_size * es));
+    MI_HIP(dev_malloc(e, &e->act, rows * (size_t)e->ff * es));
     MI_HIP(dev_malloc(e, &e->lora_t, rows * 2 * 64 * sizeof(float)));
     hipFree(e->xn);
     MI_HIP(dev_malloc(e, &e->xn, rows * (size_t)d.hidden_size * es));
@@ -822,7 +829,7 @@ int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool wan
   const int act = quirk ? MI_F32 : d.act_dtype;
   const size_t es = dtype_size(act);
   const int rndT = quirk ? (d.act_dtype == MI_BF16 ? RND_BF16 : RND_F16) : RND_NONE;
-  const int H = d.hidden_size, D = d.head_dim, Hq = d.num_heads, Hkv = d.num_kv_heads, I = d.intermediate_size;
+  const int H = d.hidden_size, D = d.head_dim, Hq = d.num_heads, Hkv = d.num_kv_heads, I = e->ff;
   const int nqkv = (Hq + 2 * Hkv) * D;
   hipStream_t st = e->stream;
   e->cur_L = L;
@@ -967,7 +974,7 @@ int forward_mixed(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t* l
   const int act = quirk ? MI_F32 : d.act_dtype;
   const size_t es = dtype_size(act);
   const int rndT = quirk ? (d.act_dtype == MI_BF16 ? RND_BF16 : RND_F16) : RND_NONE;
-  const int H = d.hidden_size, D = d.head_dim, Hq = d.num_heads, Hkv = d.num_kv_heads, I = d.intermediate_size;
+  const int H = d.hidden_size, D = d.head_dim, Hq = d.num_heads, Hkv = d.num_kv_heads, I = e->ff;
   const int nqkv = (Hq + 2 * Hkv) * D;
   hipStream_t st = e->stream;
   int nd = 0;                                    // decode rows: the leading segments of length 1
@@ -1178,11 +1185,14 @@ int mi_engine_create(const mi_model_desc* desc, int device, mi_engine** out) {
   if (hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) != hipSuccess) { delete e; return fail(MI_ERR_RUNTIME, "hipStreamCreate failed"); }
   e->layers.resize(d.num_layers);
   const int D = d.head_dim;
+  const bool pad = d.quant_bits == 4 && d.quant_group_size == 64 && d.act_dtype != MI_F32 && d.intermediate_size % 128 == 64;
+  e->ff = d.intermediate_size + (pad ? 64 : 0);
   for (auto& l : e->layers) {
     l.qkv.n_parts = 3; l.qkv.part_rows[0] = d.num_heads * D; l.qkv.part_rows[1] = d.num_kv_heads * D; l.qkv.part_rows[2] = d.num_kv_heads * D;
     l.o.n_parts = 1; l.o.part_rows[0] = d.hidden_size;
     l.gate_up.n_parts = 2; l.gate_up.part_rows[0] = d.intermediate_size; l.gate_up.part_rows[1] = d.intermediate_size;
     l.down.n_parts = 1; l.down.part_rows[0] = d.hidden_size;
+    l.gate_up.part_pad = l.down.k_pad = e->ff - d.intermediate_size;
   }
   e->embed.n_parts = 1; e->embed.part_rows[0] = d.vocab_size;
   e->lm_head.n_parts = 1; e->lm_head.part_rows[0] = d.vocab_size;
@@ -1293,7 +1303,8 @@ int mi_engine_set_lora(mi_engine* e, int layer, const char* proj, const void* A,
   MI_HIP(hipStreamSynchronize(e->stream));
   hipFree(f->lora_a[slot]); hipFree(f->lora_b[slot]);
   f->lora_a[slot] = f->lora_b[slot] = nullptr;
-  MI_HIP(dev_malloc(e, &f->lora_a[slot], (size_t)K * rank * sizeof(float)));
+  MI_HIP(dev_malloc(e, &f->lora_a[slot], (size_t)(K + f->k_pad) * rank * sizeof(float)));
+  if (f->k_pad > 0) MI_HIP(hipMemsetAsync(f->lora_a[slot] + (size_t)K * rank, 0, (size_t)f->k_pad * rank * sizeof(float), e->stream));
   MI_HIP(dev_malloc(e, &f->lora_b[slot], (size_t)rank * n * sizeof(float)));
   MI_TRY(copy_in(f->lora_a[slot], A, (size_t)K * rank * sizeof(float), on_device, e->stream));
   MI_TRY(copy_in(f->lora_b[slot], B, (size_t)rank * n * sizeof(float), on_device, e->stream));
@@ -1323,7 +1334,7 @@ int mi_engine_finalize(mi_engine* e) {
     MI_TRY(make_f32_copy(e, l.q_norm, d.head_dim, &l.q_norm32));
     MI_TRY(make_f32_copy(e, l.k_norm, d.head_dim, &l.k_norm32));
     // persistent second copies, while mem_get_info still tells a scheduler the truth about what is left for its KV arena
-    (void)ensure_gu8(e, l.gate_up, d.intermediate_size);
+    (void)ensure_gu8(e, l.gate_up, e->ff);
     if (d.act_dtype == MI_F16) { (void)ensure_hilo(e, l.qkv); (void)ensure_hilo(e, l.o); (void)ensure_hilo(e, l.gate_up); (void)ensure_hilo(e, l.down); }
   }
   MI_TRY(finalize_linear(e, e->embed, H, "model.embed_tokens"));

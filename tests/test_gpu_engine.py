@@ -1166,3 +1166,65 @@ def test_scheduler_soak_random_arrivals_prefixes_and_cancels(tiny_dirs):
     # every row released: the only blocks not free are the ones the prefix cache keeps (and those are evictable)
     assert stats["free_blocks"] + stats["cached_blocks"] == stats["usable_blocks"], stats
     model.engine.close()
+
+
+@pytest.mark.parametrize("dtype,kvd", [("bfloat16", "model"), ("float16", "model"), ("bfloat16", "float32")])
+@pytest.mark.parametrize("ff,dense_down", [(192, False), (320, False), (64, False), (192, True)])
+def test_int4_feed_forward_widths_between_blocks_of_the_tile_major_layout(dtype, kvd, ff, dense_down):
+    """A width that is an odd multiple of 64 runs as the next multiple of 128: the same bits as a model whose checkpoint has the zero rows and columns
+    itself, with an adapter on the padded matrix, on the kernels of 3, 24 and 300 rows.  (Float32 rows: the padded matrix is multiplied with centred codes.
+    Their sums and the others are 1e-6 of their 2-norm apart in each of two layers; five deviations for the largest of 1e4 logits, twice for the layers and the head behind.)"""
+    import torch
+
+    from mlx_parallm_amd.engine import Engine
+
+    H, V, heads, hd, rank = 256, 512, 4, 64, 3
+    tdt = getattr(torch, dtype)
+
+    def build(width):
+        cfg = dict(model_type="llama", hidden_size=H, num_hidden_layers=2, num_attention_heads=heads, num_key_value_heads=2, head_dim=hd, intermediate_size=width,
+                   vocab_size=V, rms_norm_eps=1e-5, rope_theta=10000.0, tie_word_embeddings=True, max_position_embeddings=512, quantization={"bits": 4, "group_size": 64})
+        rng = np.random.default_rng(ff)
+        e = Engine(cfg, device=0, max_positions=512, act_dtype=dtype)
+
+        def put(name, n, k, rows=0, cols=0):      # rows, cols: zeros behind the first `ff`
+            sc = rng.uniform(0.5, 1.5, (n, k // 64)).astype(np.float32) * 0.4 / np.sqrt(k)
+            a = {"weight": rng.integers(0, 1 << 32, (n, k // 8), dtype=np.uint32), "scales": sc, "biases": -7.5 * sc * rng.uniform(0.9, 1.1, sc.shape).astype(np.float32)}
+            if dense_down and name.endswith("down_proj"):
+                a = {"weight": (rng.standard_normal((n, k)) / np.sqrt(k)).astype(np.float32)}
+            for part, v in a.items():
+                more = cols // (8 if v.dtype == np.uint32 else 64 if "scales" in a else 1)
+                v = np.pad(v, ((0, rows), (0, more)))
+                e.set_tensor(name + "." + part, v if v.dtype == np.uint32 else torch.from_numpy(v).to(tdt).cuda())
+        one = torch.ones(H, dtype=tdt).cuda()
+        put("model.embed_tokens", V, H)
+        for i in range(2):
+            p = f"model.layers.{i}."
+            for n, rows in (("q_proj", heads * hd), ("k_proj", 2 * hd), ("v_proj", 2 * hd)):
+                put(p + "self_attn." + n, rows, H)
+            put(p + "self_attn.o_proj", H, heads * hd)
+            put(p + "mlp.gate_proj", ff, H, rows=width - ff)
+            put(p + "mlp.up_proj", ff, H, rows=width - ff)
+            put(p + "mlp.down_proj", H, ff, cols=width - ff)
+            e.set_tensor(p + "input_layernorm.weight", one)
+            e.set_tensor(p + "post_attention_layernorm.weight", one)
+        e.set_tensor("model.norm.weight", one)
+        e.finalize()
+        a, b = (rng.standard_normal((ff, rank)) / np.sqrt(ff)).astype(np.float32), rng.standard_normal((rank, H)).astype(np.float32)
+        return e, torch.from_numpy(np.pad(a, ((0, width - ff), (0, 0)))).cuda(), torch.from_numpy(b).cuda()
+    (e0, a0, b0), (e1, a1, b1) = build(ff), build(ff + 64)
+    rng = np.random.default_rng(1)
+    for B, Lt in ((3, 5), (24, 1), (5, 60)):
+        toks = rng.integers(0, V, (B, Lt)).astype(np.int32)
+        for lora in (False, True):
+            out = []
+            for e, a, b in ((e0, a0, b0), (e1, a1, b1)):
+                if lora:
+                    e.set_lora(1, "mlp.down_proj", a, b, 0.5)
+                kv = e.new_kv(B, capacity=Lt + 8, kv_dtype=kvd)
+                out.append(np.stack([e.forward(toks, kv), e.forward(toks[:, :1], kv)]))
+                kv.close()
+            far = 0.0 if kvd == "model" or dense_down else 1e-5 * np.abs(out[1]).max()
+            assert np.isfinite(out[0]).all() and np.abs(out[0] - out[1]).max() <= far, (B, Lt, lora, np.abs(out[0] - out[1]).max(), far)
+    e0.close()
+    e1.close()
