@@ -157,6 +157,7 @@ struct mi_engine {
   float* d_logprob = nullptr; float* d_prob0 = nullptr; float* d_rowstats = nullptr; float* d_uniforms = nullptr;
   int32_t* d_topk_ids = nullptr; float* d_topk_lp = nullptr;
   int32_t* d_bias_ids = nullptr; float* d_bias_vals = nullptr;
+  void* d_sample = nullptr;       // workspace of the sampler [min(maxB, SAMPLE_SPLIT_ROWS)]
   int maxB = 0;
   int max_lora_rank = 0;
   Slot slots[NSLOT];

@@ -199,6 +199,10 @@ int ensure_workspace(mi_engine* e, size_t rows, size_t logit_rows, int B) {
     e->d_logprob = (float*)(e->d_next + B);
     e->d_prob0 = (float*)(e->d_next + 2 * B);
     MI_HIP(dev_malloc(e, &e->d_rowstats, 2 * B * sizeof(float)));
+    if (e->d_sample == nullptr || e->maxB < SAMPLE_SPLIT_ROWS) {
+      hipFree(e->d_sample);
+      MI_HIP(dev_malloc(e, &e->d_sample, sample_ws_bytes(B)));
+    }
     MI_HIP(dev_malloc(e, &e->d_uniforms, B * sizeof(float)));
     MI_HIP(dev_malloc(e, &e->d_topk_ids, (size_t)B * MI_MAX_TOP_LOGPROBS * sizeof(int32_t)));
     MI_HIP(dev_malloc(e, &e->d_topk_lp, (size_t)B * MI_MAX_TOP_LOGPROBS * sizeof(float)));
@@ -1123,7 +1127,9 @@ int run_sample(mi_engine* e, int B, const mi_sample_params* sp, const int32_t* f
     MI_HIP(hipMemcpyAsync(e->d_bias_vals, sp->logit_bias_values, sp->n_logit_bias * sizeof(float), hipMemcpyHostToDevice, st));
   }
   if (sp->uniforms && !forced) MI_HIP(hipMemcpyAsync(e->d_uniforms, sp->uniforms, B * sizeof(float), hipMemcpyHostToDevice, st));
-  const bool per_row = sp->row_temperature != nullptr && sp->row_top_p != nullptr && !forced;
+  bool per_row = sp->row_temperature != nullptr && sp->row_top_p != nullptr && !forced;
+  const bool drawn = per_row ? std::any_of(sp->row_temperature, sp->row_temperature + B, [](float t) { return t != 0.f; }) : sp->temperature != 0.f;
+  per_row = per_row && drawn;                                    // (rows that are all greedy: a greedy call)
   if (per_row) {
     if ((size_t)B > e->d_rowpar_cap) {
       MI_HIP(hipStreamSynchronize(st));
@@ -1137,7 +1143,7 @@ int run_sample(mi_engine* e, int B, const mi_sample_params* sp, const int32_t* f
   Prof pr(e, "sample");
   SampleCall sc{};
   sc.logits = e->logits; sc.B = B; sc.V = e->d.vocab_size; sc.rnd = RND_NONE;
-  sc.temperature = sp->temperature; sc.top_p = sp->top_p;
+  sc.temperature = drawn || forced ? sp->temperature : 0.f; sc.top_p = sp->top_p;
   sc.n_bias = sp->n_logit_bias; sc.bias_ids = e->d_bias_ids; sc.bias_vals = e->d_bias_vals;
   sc.forced = forced;
   sc.uniforms = (sp->uniforms && !forced) ? e->d_uniforms : nullptr; sc.seed = sp->seed; sc.step = sp->stream_position >= 0 ? (uint64_t)sp->stream_position : e->step_counter++;
@@ -1146,7 +1152,7 @@ int run_sample(mi_engine* e, int B, const mi_sample_params* sp, const int32_t* f
   sc.row_temp = per_row ? e->d_rowpar : nullptr;
   sc.row_top_p = per_row ? e->d_rowpar + B : nullptr;
   sc.tokens_out = e->d_next; sc.logprob_out = e->d_logprob; sc.prob_row0_out = forced ? nullptr : e->d_prob0;
-  sc.topk_ids = e->d_topk_ids; sc.topk_logprobs = e->d_topk_lp; sc.row_stats = e->d_rowstats;
+  sc.topk_ids = e->d_topk_ids; sc.topk_logprobs = e->d_topk_lp; sc.row_stats = e->d_rowstats; sc.ws = e->d_sample;
   return launch_sample(sc, st);
 }
 
@@ -1216,7 +1222,7 @@ void mi_engine_destroy(mi_engine* e) {
   hipFree(e->h); hipFree(e->qkv); hipFree(e->q); hipFree(e->attn); hipFree(e->act); hipFree(e->logits); hipFree(e->lora_t); hipFree(e->d_forced); hipFree(e->d_gather);
   hipFree(e->d_seam_counter); hipFree(e->d_seam_error); hipHostFree(e->h_seam_err); hipFree(e->d_rowpar); hipFree(e->deq_scratch);
   hipFree(e->sk_ws); hipFree(e->sk_ctr); hipFree(e->d_sq); hipFree(e->ap_part); hipFree(e->ap_ctr);
-  hipFree(e->d_tokens); hipFree(e->d_next); hipFree(e->d_rowstats);
+  hipFree(e->d_tokens); hipFree(e->d_next); hipFree(e->d_rowstats); hipFree(e->d_sample);
   hipFree(e->d_uniforms); hipFree(e->d_topk_ids); hipFree(e->d_topk_lp); hipFree(e->d_bias_ids); hipFree(e->d_bias_vals);
   for (auto& s : e->slots) {
     hipHostFree(s.tokens); hipHostFree(s.topk_ids); hipHostFree(s.topk_lp);

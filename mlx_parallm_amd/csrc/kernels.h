@@ -373,7 +373,12 @@ struct SampleCall {
   int32_t* topk_ids;         // device [B][top_logprobs]
   float* topk_logprobs;
   float* row_stats;          // device [B][2] scratch: (max, logsumexp)
+  void* ws = nullptr;        // sample_ws_bytes(B), or null: one workgroup per row
 };
+// The kernels with several workgroups a row: draws of up to SAMPLE_SPLIT_ROWS rows of SAMPLE_SPLIT_VOCAB logits and more; up to 64 rows without one, the
+// arg-max alone from SAMPLE_SPLIT_GREEDY logits on (the figures: misc.hip)
+constexpr int SAMPLE_PARTS = 8, SAMPLE_SPLIT_ROWS = 512, SAMPLE_SPLIT_VOCAB = 16384, SAMPLE_SPLIT_GREEDY = 65536;
+size_t sample_ws_bytes(int B);
 int launch_sample(const SampleCall& c, hipStream_t st);
 
 int launch_advance_offsets(int32_t* offsets, const int32_t* rows, int B, int L, hipStream_t st);

@@ -324,8 +324,10 @@ int mi_op_sample(float* logits, int B, int V, float temperature, float top_p, co
   sc.uniforms = uniforms; sc.seed = 0; sc.step = 0; sc.top_logprobs = top_logprobs; sc.lp_temp = 0;
   sc.tokens_out = tokens_out; sc.logprob_out = logprob_out; sc.prob_row0_out = prob_row0_out;
   sc.topk_ids = topk_ids; sc.topk_logprobs = topk_logprobs; sc.row_stats = row_stats;
-  MI_TRY(launch_sample(sc, nullptr));
-  return finish();
+  MI_HIP(hipMalloc(&sc.ws, sample_ws_bytes(B)));
+  const int rc = launch_sample(sc, nullptr), rc2 = finish();
+  hipFree(sc.ws);
+  return rc != MI_OK ? rc : rc2;
 }
 
 }  // extern "C"

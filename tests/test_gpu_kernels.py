@@ -719,3 +719,42 @@ def test_sampler_edges_within_derived_bound(V, std, bf, temp, top_p):
     toks, _lp, _p0, _, _ = _run_sampler(np.stack(rows), temp, top_p, np.asarray(us))
     bad = [(i, us[i], int(toks[i]), wants[i]) for i in range(len(us)) if int(toks[i]) != wants[i]]
     assert not bad, bad[:5]
+
+
+def _sampler_rows(V, rng):
+    """Rows of logits where the parts of a row could disagree with one walk of it: ties, signed zeros, infinities, NaN, more equal values than fit a list."""
+    rows = [rng.standard_normal(V).astype(np.float32) * s for s in (0.3, 1.5, 6.0, 40.0)]
+    rows += [torch.from_numpy(r).to(torch.bfloat16).float().numpy() for r in rows[:3]]
+    rows.append(np.zeros(V, np.float32))
+    rows.append(np.where(np.arange(V) % 2 == 0, 0.0, -0.0).astype(np.float32))
+    rows.append(np.where(np.arange(V) % 97 == 5, 2.0, rng.standard_normal(V) - 20).astype(np.float32))
+    peak = rng.standard_normal(V).astype(np.float32)
+    peak[V - 3] = 60.0
+    rows.append(peak)
+    masked = np.full(V, -np.inf, np.float32)
+    masked[[3, V // 2, V - 1]] = [1.0, 1.0, 0.5]
+    rows += [masked, np.full(V, -np.inf, np.float32), np.full(V, np.finfo(np.float32).min, np.float32)]
+    for bad in (np.inf, np.nan):
+        r = rng.standard_normal(V).astype(np.float32)
+        r[V // 3] = bad
+        rows.append(r)
+    return np.stack(rows)
+
+
+@pytest.mark.parametrize("V", [16384, 16396, 32000, 50304, 151936])
+@pytest.mark.parametrize("temp,top_p", [(0.0, 1.0), (1.0, 1.0), (0.7, 0.9), (1.0, 0.05), (3.0, 0.999), (1e-3, 0.5), (-1.0, 0.9)])
+def test_sampler_over_several_workgroups_equals_one(V, temp, top_p):
+    """The kernels that split a row draw the ids of the one that does not: it serves calls of more rows, so the same rows are drawn behind 512 others."""
+    rng = np.random.default_rng(V)
+    rows = _sampler_rows(V, rng)
+    n = len(rows)
+    for u in (0.0, 0.37, 1.0 - 2.0 ** -24):
+        uu = np.concatenate([[u], rng.random(n - 1)]).astype(np.float32)
+        got = _run_sampler(rows, temp, top_p, uu, k=5)
+        one = _run_sampler(np.concatenate([rows, np.tile(rows[:1], (513 - n, 1))]), temp, top_p, np.concatenate([uu, np.zeros(513 - n, np.float32)]), k=5)
+        for g, o in zip((got[0], got[3]), (one[0][:n], one[3][:n])):
+            assert np.array_equal(g, o)
+        for g, o in ((got[1], one[1][:n]), (got[2], one[2][:n]), (got[4], one[4][:n])):       # sums of V terms in another order
+            np.testing.assert_allclose(g, o, rtol=1e-5, atol=2e-6)
+        shifted = _run_sampler(np.roll(rows, 1, 0), temp, top_p, np.roll(uu, 1), k=5)          # a row's ids do not depend on where it stands
+        assert np.array_equal(np.roll(shifted[0], -1), got[0])
