@@ -252,6 +252,7 @@ struct mi_engine {
   int scan_ld = 0, gate_ld = 0;
   int32_t* d_gather_list = nullptr; size_t d_gather_list_cap = 0;   // wanted positions, their normed rows
   void* head_x = nullptr; size_t head_x_cap = 0;
+  float* side_part = nullptr; size_t side_part_cap = 0;       // launch_gemv_side: the slices' sums, then the gate's shares
   float* resid_out = nullptr; int64_t resid_cap = 0;          // mi_debug_residual
 };
 

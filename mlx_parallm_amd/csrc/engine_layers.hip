@@ -877,7 +877,7 @@ void layers_free(mi_engine* e) {
   for (auto& t : e->rot_tabs) hipFree(t.p);
   for (void* p : {e->tok_embed, e->side_embed, e->pair_embed, e->low, e->qc, e->qfull, (void*)e->light_ws, (void*)e->light_ctr, (void*)e->dl_q, (void*)e->d_freq, (void*)e->x32, e->hn, e->proj, e->cat, (void*)e->scan32, (void*)e->gate32,
                   e->lq, (void*)e->lat_part, e->lat_m, e->lat_x, e->lat_kv, (void*)e->dl_w, (void*)e->dl_p, (void*)e->dl_k, (void*)e->dl_f, (void*)e->d_meta, (void*)e->d_gather_list, e->head_x,
-                  (void*)e->y32, e->v_first, (void*)e->moe_ids, (void*)e->moe_wts, e->moe_mid, e->moe_out, (void*)e->moe_plan, (void*)e->moe_counts, (void*)e->gqa_part, (void*)e->gqa_ctr}) hipFree(p);
+                  (void*)e->y32, e->v_first, (void*)e->moe_ids, (void*)e->moe_wts, e->moe_mid, e->moe_out, (void*)e->side_part, (void*)e->moe_plan, (void*)e->moe_counts, (void*)e->gqa_part, (void*)e->gqa_ctr}) hipFree(p);
 }
 
 // element offsets of the arenas (latents, keys, values) for `tokens` token places, byte offsets of the recurrent state for kv->B rows
@@ -1071,7 +1071,19 @@ int forward_segments(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t
     }
     GemvCall co; co.x = e->cat; co.ldx = l.n_cat; co.act = act; co.epi = EPI_RESID; co.out32 = 1; co.resid = e->x32; co.ldo = e->wp;
     if (post || pre || both) { co.epi = EPI_STORE; co.resid = nullptr; co.out = e->y32; }
-    MI_TRY(gemv_rows(e, l.out.f, co, R, es, sizeof(float), "gemv_out"));
+    SideNormCall sn{R, tok, e->side_embed, d.num_layers * d.side_dim, li * d.side_dim, d.vocab_size, l.side_gate, l.side_proj_t, l.side_proj_p,
+                    l.side_norm.p, d.rms_norm_eps, d.side_dim, d.hidden_size, e->wp, norm_of(ri + 1), e->x32, e->hn, act};
+    const int slices = post || pre || both || !e->opt_skinny_gemm || e->opt_force_v1 ? 0 : gemv_side_slices(l.out.f.W, act, d.side_dim, R);
+    const bool joined = slices > 0 && side_join_supported(sn, slices, l.out.N / 16);
+    if (joined) {                              // a decode step's rows: two launches that share the gate's work
+      const size_t sums = (size_t)slices * R * e->wp, shares = (size_t)slices * (l.out.N / 16) * R * 64;
+      MI_TRY(grow(e, (void**)&e->side_part, &e->side_part_cap, (sums + shares) * sizeof(float)));
+      { Prof pr(e, "gemv_out");
+        MI_TRY(launch_gemv_side(l.out.f.W, SideOutCall{e->cat, l.n_cat, R, e->x32, e->wp, l.side_gate, d.side_dim, e->side_part, e->side_part + sums, act}, st)); }
+      Prof pr(e, "side");
+      MI_TRY(launch_side_join(sn, e->side_part, e->side_part + sums, slices, l.out.N / 16, st));
+    } else
+      MI_TRY(gemv_rows(e, l.out.f, co, R, es, sizeof(float), "gemv_out"));
     // gate | up with the unit in the epilogue, down: y32
     auto dense_ff = [&]() -> int {
       GemvCall cg; cg.x = e->hn; cg.ldx = e->wp; cg.act = act; cg.epi = EPI_SWIGLU; cg.out = e->cat; cg.ldo = l.ffp; cg.pair_offset = l.ffp; cg.glu = l.glu;
@@ -1114,10 +1126,8 @@ int forward_segments(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t
         q = 1;
       }
       MI_TRY(stream_norm(l, q, in_of(ri + 1), norm_of(ri + 1), ri + 1 == n_runs));
-    } else { Prof pr(e, "side");
-      SideNormCall c{R, tok, e->side_embed, d.num_layers * d.side_dim, li * d.side_dim, d.vocab_size, l.side_gate, l.side_proj_t, l.side_proj_p,
-                     l.side_norm.p, d.rms_norm_eps, d.side_dim, d.hidden_size, e->wp, norm_of(ri + 1), e->x32, e->hn, act};
-      MI_TRY(launch_side_norm(c, st)); }
+    } else if (!joined) { Prof pr(e, "side");
+      MI_TRY(launch_side_norm(sn, st)); }
     if (e->resid_out != nullptr) {
       const float* x = e->x32;
       if (e->streams > 1) { MI_TRY(launch_stream_sum(e->x32, e->streams, R, e->wp, e->y32, st)); x = e->y32; }

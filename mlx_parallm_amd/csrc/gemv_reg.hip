@@ -463,6 +463,64 @@ __global__ __launch_bounds__(512, 2) void gemv_dense_kernel(const RegParams p) {
   do_tile(tile, std::false_type{});
 }
 
+// The output linear of a layer with a token input (layer_rows.hip: side_join_kernel reads what this leaves), 16-bit weights and rows.  A tile and a slice of K per workgroup,
+// so that a width of 2048 (128 tiles) fills the card: part[s][m][n] = the slice's sums, with the residual in slice 0; and of those 16 columns each gate output's share,
+// z[s tiles + tile][m][j] = sum_n gate[j][n] part[s][m][n], so that no workgroup of what follows reads the gate's matrix.
+// 4 rows, 2048 x 10240 bf16, us in a decode step: gemv_mfma.hip 15.6 and the gate, projection and norms of a row in one workgroup 12.2; here 10.3 and 9.3 (a layer 53 -> 46).
+struct SideParams {
+  const void* x; int ldx; int M;
+  const void* w; int nblk, ks;
+  const float* resid; int ld;
+  const void* gate; int dim;
+  float* part; float* z;
+};
+template <typename AT, int KW, bool FULL>             // (KW, FULL: as gemv_reg_kernel, of a slice)
+__global__ __launch_bounds__(512, 2) void gemv_side_kernel(const SideParams p) {
+  constexpr int NW = 8, NP = KW / 32, NQ = NP / 2;
+  __shared__ __attribute__((aligned(16))) float tl[NW * 256];
+  __shared__ __attribute__((aligned(16))) float xs[8][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c16 = lane & 15, g = lane >> 4;
+  const int tile = blockIdx.x, s = blockIdx.y, sn = p.nblk / p.ks;                     // (slices of whole pairs: the host)
+  const int q0 = s * sn + wave * sn / NW, nq = (wave + 1) * sn / NW - wave * sn / NW;
+  auto pair_at = [&](int q) { return q0 + min(q, max(nq - 1, 0)); };                   // (past the last: the last one again, unused)
+  u32x4 wb[NP], xf[NQ], gw[2];
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+    wb[i] = __builtin_nontemporal_load((const u32x4*)((const char*)p.w + ((size_t)tile * p.nblk * 2 + pair_at(i >> 1) * 2 + (i & 1)) * 1024 + lane * 16));
+  const AT* xr = (const AT*)p.x + (size_t)min(c16 & 7, p.M - 1) * p.ldx + (c16 >> 3) * 32 + g * 8;
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) xf[q] = *(const u32x4*)(xr + pair_at(q) * 64);
+  const AT* gr = (const AT*)p.gate + (size_t)min(lane, p.dim - 1) * p.ld + tile * 16;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) gw[h] = *(const u32x4*)(gr + 8 * h);
+  const int m = min(tid >> 4, p.M - 1), n = tile * 16 + (tid & 15);
+  const float r0 = p.resid[(size_t)m * p.ld + n];
+  __builtin_amdgcn_sched_barrier(0);
+  f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+    if (FULL || i < 2 * nq) acc[i & 1] = mfma16<AT>((i & 1) ? ror8(xf[i >> 1]) : xf[i >> 1], wb[i], acc[i & 1]);      // (uniform)
+  *(f32x4*)&tl[wave * 256 + lane * 4] = acc[0] + acc[1];
+  __syncthreads();
+  if (tid < 128) {
+    const float y = sum_waves(tl + (((tid >> 6) * 16 + (tid & 15)) * 4 + ((tid >> 4) & 3))) + (s == 0 ? r0 : 0.f);
+    xs[tid >> 4][tid & 15] = y;
+    if ((tid >> 4) < p.M) p.part[((size_t)s * p.M + (tid >> 4)) * p.ld + n] = y;
+  }
+  __syncthreads();
+  if (wave < p.M && lane < p.dim) {                   // row `wave`, gate output `lane`
+    float z = 0.f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x2 e = unpack2<AT>(gw[h][j]);
+        z = fmaf(e.x, xs[wave][8 * h + 2 * j], fmaf(e.y, xs[wave][8 * h + 2 * j + 1], z));
+      }
+    p.z[(((size_t)s * gridDim.x + tile) * p.M + wave) * 64 + lane] = z;
+  }
+}
+
 int quant_bits(const LinearW& W, int act) {           // 4 / 8: codes with scales of the activation type, 0: neither
   if (((W.wk == WK_Q4_BF16 && act == MI_BF16) || (W.wk == WK_Q4_F16 && act == MI_F16)) && W.group == 64) return 4;
   if (((W.wk == WK_Q8_BF16 && act == MI_BF16) || (W.wk == WK_Q8_F16 && act == MI_F16)) && W.group == 64) return 8;
@@ -579,6 +637,30 @@ int launch_gemv_dense(const LinearW& W, const GemvCall& c, size_t rows, hipStrea
   const bool gu = c.epi == EPI_SWIGLU_GU8;
   if (c.act == MI_F32) return launch_dense<bf16, true>(p, gu, st);
   return c.act == MI_BF16 ? launch_dense<bf16, false>(p, gu, st) : launch_dense<f16, false>(p, gu, st);
+}
+
+// Slices of K: as many as the card has room for beside the tiles, of the same whole pairs of blocks each, and no more than a wave's registers hold.  0: not this kernel
+int gemv_side_slices(const LinearW& W, int act, int dim, size_t rows) {
+  const bool dense = (W.wk == WK_BF16 && act == MI_BF16) || (W.wk == WK_F16 && act == MI_F16);
+  if (!dense || W.layout != 1 || rows < 1 || rows > 8 || dim < 1 || dim > 64 || W.K % 64 != 0 || W.N % 16 != 0 || W.lora_b[0] != nullptr || W.lora_b[1] != nullptr) return 0;
+  const int nblk = W.K / 64, tiles = W.N / 16;
+  for (int ks = std::max(1, std::min(4, gemv_cu_count() / tiles)); ks <= 4; ++ks)
+    if (nblk % ks == 0 && nblk / ks >= 8 && nblk / ks * 64 <= REG_K) return ks;
+  return 0;
+}
+
+int launch_gemv_side(const LinearW& W, const SideOutCall& c, hipStream_t st) {
+  const int ks = gemv_side_slices(W, c.act, c.dim, c.rows);
+  if (ks == 0 || c.ldx % 8 != 0 || c.ld % 8 != 0 || c.ld < W.N || ((uintptr_t)c.x | (uintptr_t)c.gate) % 16 != 0) return fail(MI_ERR_UNSUPPORTED, "gemv_side: shape / dtype not supported");
+  SideParams p{c.x, c.ldx, c.rows, W.w, W.K / 64, ks, c.resid, c.ld, c.gate, c.dim, c.part, c.z};
+  const dim3 grid(W.N / 16, ks);
+  auto go = [&](auto kern) -> int {
+    hipLaunchKernelGGL(kern, grid, dim3(512), 0, st, p);
+    MI_HIP(hipGetLastError());
+    return MI_OK;
+  };
+  if (c.act == MI_BF16) return by_share(p.nblk / ks, 64, [&](auto kw, auto full) { return go(gemv_side_kernel<bf16, kw.value, full.value>); });
+  return by_share(p.nblk / ks, 64, [&](auto kw, auto full) { return go(gemv_side_kernel<f16, kw.value, full.value>); });
 }
 
 }  // namespace mi

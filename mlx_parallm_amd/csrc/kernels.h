@@ -169,6 +169,18 @@ int launch_gemv_reg(const LinearW& W, const GemvCall& c, size_t rows, hipStream_
 bool gemv_dense_supported(const LinearW& W, const GemvCall& c, size_t rows);
 int launch_gemv_dense(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st);
 
+// The output linear of a layer with a token input, at most 8 rows (gemv_reg.hip: gemv_side_kernel); launch_side_join follows it
+struct SideOutCall {
+  const void* x; int ldx; int rows;
+  const float* resid; int ld;    // [rows][ld], read
+  const void* gate; int dim;     // [dim][ld]
+  float* part;                   // [slices][rows][ld]
+  float* z;                      // [slices][N / 16][rows][64]
+  int act;
+};
+int gemv_side_slices(const LinearW& W, int act, int dim, size_t rows);
+int launch_gemv_side(const LinearW& W, const SideOutCall& c, hipStream_t st);
+
 // 9..64 rows, int8 weights 1..64 (decode steps of larger batches): weight-streaming split-K GEMM (gemm_skinny.hip).
 // c.pro must be PRO_NONE; `ws` >= gemm_skinny_ws_bytes(), `ctr` >= gemm_skinny_groups() words that are zero between
 // launches (the kernel leaves them zero); ksplit = 0 lets the cost model choose.

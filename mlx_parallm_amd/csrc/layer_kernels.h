@@ -64,6 +64,9 @@ struct SideNormCall {
 };
 bool side_mfma_supported(int act, int dim, int ld);
 int launch_side_norm(const SideNormCall& c, hipStream_t st);
+// the same behind launch_gemv_side: the residual as its slices' sums, the gate's outputs as the tiles' shares (c.gate is not read)
+bool side_join_supported(const SideNormCall& c, int slices, int tiles);
+int launch_side_join(const SideNormCall& c, const float* part, const float* z, int slices, int tiles, hipStream_t st);
 
 // off[row of each segment] += its length; prev (or null): the row's last token
 int launch_advance_segments(const SegTables& t, int32_t* off, const int32_t* tokens, int32_t* prev, hipStream_t st);

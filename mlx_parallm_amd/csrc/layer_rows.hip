@@ -371,6 +371,103 @@ int side_norm_at(const SideNormCall& c, hipStream_t st) {
   return MI_OK;
 }
 
+// A row behind gemv_side_kernel.  What is left to read is the projection, 256 KiB at 2048 x 64 and all of it under way from the start (JG outputs of the gate x 8 columns
+// a thread), the tiles' shares of the gate and the slices' sums.  One CU's loads bound it still (50 to 60 GB/s).
+// NG groups of JG gate outputs, 1024 / NG threads for a row of 8192 / NG columns
+template <typename T, int NG>
+__global__ __launch_bounds__(1024) void side_join_kernel(SideNormCall c, const float* part, const float* z, int slices, int parts) {
+  constexpr int NT = 1024, TG = NT / NG, JG = 64 / NG, NW = NT / 64, NC = 8 / NG;      // NC: columns a thread ends up with
+  constexpr int MAXS = 4, MAXZ = 4;
+  __shared__ __attribute__((aligned(16))) float ys[NG][TG * 8];
+  __shared__ __attribute__((aligned(16))) float zs[NW][64];
+  __shared__ float gs[64], red[2][NW];
+  const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // the gate's shares: 16 threads a part
+  const float4* z4 = (const float4*)(z + (size_t)r * 64) + (tid & 15);
+  float4 zv[MAXZ];
+#pragma unroll
+  for (int i = 0; i < MAXZ; ++i) zv[i] = z4[(size_t)min((tid >> 4) + i * (NT / 16), parts - 1) * c.rows * 16];
+  const int col = tid * NC, colc = min(col, c.ld - NC);
+  float xv[MAXS][NC], sw[NC], nw[NC];
+#pragma unroll
+  for (int s = 0; s < MAXS; ++s)
+#pragma unroll
+    for (int i = 0; i < NC; ++i) xv[s][i] = part[((size_t)min(s, slices - 1) * c.rows + r) * c.ld + colc + i];
+  const int tok = min(max(c.tokens[r], 0), c.vocab - 1);
+  const float tab = to_f32(((const T*)c.table)[(size_t)tok * c.table_ld + c.slice + min(lane, c.dim - 1)]);
+  const int jg = tid / TG, cb = min(tid % TG * 8, c.ld - 8);
+  uint4 pw[JG];
+#pragma unroll
+  for (int j = 0; j < JG; ++j) pw[j] = *(const uint4*)((const T*)c.proj_t + (size_t)min(jg * JG + j, c.dim - 1) * c.ld + cb);
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int k = min(colc + i, c.width - 1);
+    sw[i] = c.side_w[k]; nw[i] = c.norm.w[k * c.norm.stride];
+  }
+  float zz[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < MAXZ; ++i)
+    if ((tid >> 4) + i * (NT / 16) < parts) { zz[0] += zv[i].x; zz[1] += zv[i].y; zz[2] += zv[i].z; zz[3] += zv[i].w; }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) { zz[j] += __shfl_xor(zz[j], 16, 64); zz[j] += __shfl_xor(zz[j], 32, 64); }
+  if (lane < 16) *(float4*)&zs[wave][lane * 4] = float4{zz[0], zz[1], zz[2], zz[3]};
+  __syncthreads();
+  if (tid < 64) {
+    float s = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) s += zs[w][tid];
+    gs[tid] = tid < c.dim ? gelu_tanh_f(s) * tab : 0.f;
+  }
+  __syncthreads();
+  float y8[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) y8[i] = 0.f;
+#pragma unroll
+  for (int j = 0; j < JG; ++j) {
+    const float g = gs[jg * JG + j];
+    const T* e = (const T*)&pw[j];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) y8[i] = fmaf(to_f32(e[i]), g, y8[i]);
+  }
+  *(float4*)&ys[jg][tid % TG * 8] = float4{y8[0], y8[1], y8[2], y8[3]};
+  *(float4*)&ys[jg][tid % TG * 8 + 4] = float4{y8[4], y8[5], y8[6], y8[7]};
+  __syncthreads();
+  auto row_sum = [&](float v, int which) {
+    v = wave_sum(v);
+    if (lane == 0) red[which][wave] = v;
+    __syncthreads();
+    float t = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) t += red[which][w];
+    return t;
+  };
+  float y[NC], ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    y[i] = 0.f;
+#pragma unroll
+    for (int k = 0; k < NG; ++k) y[i] += ys[k][col + i];
+    ss += col + i < c.width ? y[i] * y[i] : 0.f;
+  }
+  const float rs = 1.0f / sqrtf(row_sum(ss, 0) / (float)c.width + c.side_eps);
+  ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    float x = xv[0][i];
+#pragma unroll
+    for (int s = 1; s < MAXS; ++s) x += s < slices ? xv[s][i] : 0.f;
+    y[i] = col + i < c.width ? x + y[i] * rs * sw[i] : 0.f;
+    ss += y[i] * y[i];
+  }
+  const float rn = 1.0f / sqrtf(row_sum(ss, 1) / (float)c.width + c.norm.eps);
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    if (col + i >= c.ld) break;
+    if (col + i < c.width) c.x[(size_t)r * c.ld + col + i] = y[i];
+    ((T*)c.h)[(size_t)r * c.ld + col + i] = from_f32<T>(col + i < c.width ? y[i] * rn * nw[i] : 0.f);
+  }
+}
+
 // ---- norm of a sublayer's output, residual update, operand of what follows: one workgroup per row ------------------------
 template <typename T>
 __device__ __forceinline__ f32x4 load4v(const T* p) {
@@ -676,6 +773,23 @@ int launch_embed_pos(const EmbedPosCall& c, hipStream_t st) {
 }
 
 bool side_mfma_supported(int act, int dim, int ld) { return act != MI_F32 && dim >= 1 && dim <= 128 && ld <= 4096; }
+
+// rows of at most 2048 columns: a thread's share of the projection fits its registers
+bool side_join_supported(const SideNormCall& c, int slices, int tiles) {
+  return (c.act == MI_BF16 || c.act == MI_F16) && c.dim >= 1 && c.dim <= 64 && c.ld % 8 == 0 && c.ld <= 2048 && c.norm.w != nullptr && slices >= 1 && slices <= 4 &&
+         slices * tiles <= 256 && (uintptr_t)c.proj_t % 16 == 0;
+}
+
+int launch_side_join(const SideNormCall& c, const float* part, const float* z, int slices, int tiles, hipStream_t st) {
+  if (!side_join_supported(c, slices, tiles)) return fail(MI_ERR_UNSUPPORTED, "side_join: shape / dtype not supported");
+  const dim3 grid(c.rows), block(1024);
+#define GO(T, NG) hipLaunchKernelGGL((side_join_kernel<T, NG>), grid, block, 0, st, c, part, z, slices, slices * tiles)
+  if (c.ld > 1024) { if (c.act == MI_BF16) GO(bf16, 4); else GO(f16, 4); }
+  else { if (c.act == MI_BF16) GO(bf16, 8); else GO(f16, 8); }
+#undef GO
+  MI_HIP(hipGetLastError());
+  return MI_OK;
+}
 
 int launch_side_norm(const SideNormCall& c, hipStream_t st) {
   if (c.ld % 8 != 0) return fail(MI_ERR_INVALID, "side_norm: row stride must be a multiple of 8");

@@ -370,3 +370,26 @@ def test_server_program_completes_and_streams(tmp_path, scheduler):
 
     cfg = config(72, build_byte_tokenizer(tmp_path), [delta(4, 2, 20, 24, 3, 80), latent(3, 16, 24, 40, 0.4, 72), latent(2, 24, 16, 40, 0.3, 0, 1)], 8)
     serve_and_compare(tmp_path, scheduler, R, cfg, greedy)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("width,ff,side", [(1000, 4096, 20), (1024, 4096, 64), (2048, 8192, 64), (2032, 1536, 1), (512, 512, 33)])
+def test_token_input_of_few_rows_over_many_workgroups(bank, dtype, width, ff, side):
+    """Up to 8 rows: the output linear in slices of K with the gate's shares, the rest of the layer's end in one launch a row.  Slices that fill the waves'
+    registers and others, rows narrower than their stride, one gate output to the most; the residual stream of both layers and the logits."""
+    cfg = config(width, 96, [latent(2, 64, 64, 64, 0.125, ff), delta(2, 1, 64, 64, 4, ff)], side)
+    cfg, w, m = bank(f"side_{width}_{side}", dtype, cfg=cfg)
+    for n in (1, 3, 8):
+        reqs = [tokens(cfg, 4, 7 * n + i) for i in range(n)]
+        kv = m.engine.new_kv(n, capacity=16, kv_dtype="model")
+        m.engine.forward(np.stack([t[:3] for t in reqs]), kv)
+        cap = m.engine.capture_residual(n)
+        got = m.engine.forward(np.stack([t[3:] for t in reqs]), kv)
+        m.engine.capture_residual(0)
+        kv.close()
+        for i, t in enumerate(reqs):
+            layers = []
+            want = R.forward(cfg, w, t, layers)
+            assert err(got[i:i + 1], want[-1:]).max() < TOL[dtype], (n, i)
+            for g, x in zip(cap, layers):
+                assert np.sqrt(((g[i] - x[-1]) ** 2).mean()) < TOL[dtype] / 2 * np.sqrt((x * x).mean())
