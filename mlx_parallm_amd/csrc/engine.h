@@ -200,6 +200,10 @@ struct mi_engine {
   float* ap_part = nullptr; size_t ap_part_cap = 0;       // prefill attention with split keys: the slices' partial results ..
   int* ap_ctr = nullptr; size_t ap_ctr_cap = 0;           // .. and arrival tickets (zero between launches)
   void* gk_ws = nullptr; size_t gk_cap = 0;   // float32 partial tiles of the K-split 128 x 128 tile GEMM
+  // decode steps of a small model in one launch (stack_small.hip); null: not such a model
+  void* small_buf = nullptr; uint32_t* small_words = nullptr; float2* small_scales = nullptr; float* small_norms = nullptr;
+  int small_kind = 0;
+  bool opt_small_stack = true;
   // ---- layer-list models (engine_layers.hip)
   bool layered = false;
   std::vector<ListLayer> list;

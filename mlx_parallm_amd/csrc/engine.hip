@@ -817,6 +817,39 @@ int split_prefill(mi_engine* e, AttnCall& ac, int max_keys) {
 // the model forward for B*L tokens already in e->d_tokens; logits of the requested rows end
 // up in e->logits (float32, [B][V] or [B*L][V]).
 // `rows` (host, B distinct cache rows) = the call covers that subset of kv's rows, batch entry b <-> rows[b]
+// The layers of a small model as stack_small.hip reads them: made behind the last weight, where every matrix fits the kernel's registers
+int make_small_stack(mi_engine* e) {
+  const mi_model_desc& d = e->d;
+  if (e->layered || d.arch != MI_ARCH_LLAMA || !small_stack_shape(d.hidden_size, d.num_heads, d.num_kv_heads, d.head_dim, e->ff)) return MI_OK;
+  if (!attention_decode_supported(AttnShape{1, 1, d.num_heads, d.num_kv_heads, d.head_dim, MI_F32, MI_F32, RND_NONE, 0, nullptr})) return MI_OK;      // (refused by the prompt's kernels)
+  const LinearW& w0 = e->layers[0].qkv.W;
+  size_t words = 0, scales = 0;
+  for (LayerW& l : e->layers)
+    for (FusedLinear* f : {&l.qkv, &l.o, &l.gate_up, &l.down}) {
+      if (!small_stack_fits(f->W, f == &l.qkv || f == &l.gate_up) || small_stack_kind(f->W) != small_stack_kind(w0) || f->W.group != w0.group) return MI_OK;
+      words += small_stack_words(small_stack_kind(w0), f == &l.qkv || f == &l.gate_up); scales += small_stack_scales(small_stack_kind(w0));
+    }
+  const size_t norms = (size_t)2 * d.num_layers * d.hidden_size;
+  if (hipMalloc(&e->small_buf, words * 4 + scales * 8 + norms * 4) != hipSuccess) { (void)hipGetLastError(); e->small_buf = nullptr; return MI_OK; }
+  e->small_words = (uint32_t*)e->small_buf; e->small_scales = (float2*)(e->small_words + words); e->small_norms = (float*)(e->small_scales + scales);
+  e->small_kind = small_stack_kind(w0);
+  uint32_t* w = e->small_words; float2* sb = e->small_scales; float* nw = e->small_norms;
+  for (LayerW& l : e->layers) {
+    for (FusedLinear* f : {&l.qkv, &l.o, &l.gate_up, &l.down}) {
+      const bool big = f == &l.qkv || f == &l.gate_up;
+      MI_TRY(launch_small_pack(f->W, big, w, sb, e->stream));
+      w += small_stack_words(e->small_kind, big); sb += small_stack_scales(e->small_kind);
+    }
+    for (const void* n : {l.in_norm, l.post_norm}) { MI_TRY(launch_convert(n, d.act_dtype, nw, MI_F32, d.hidden_size, e->stream)); nw += d.hidden_size; }
+  }
+  return MI_OK;
+}
+bool small_stack_takes(const mi_engine* e, const mi_kv* kv, int act, int B, int L, const int32_t* rows) {
+  if (e->small_buf == nullptr || !e->opt_small_stack || e->opt_force_v1 || !e->opt_fused_attn || !e->prof_name.empty() || L != 1 || act != MI_F32 || kv->dtype != MI_F32) return false;
+  for (int b = 0; b < B; ++b) if (kv->h_off[rows ? rows[b] : b] + 1 > SMALL_MAX_KEYS) return false;
+  return true;
+}
+
 int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool want_logits, const int32_t* rows = nullptr) {
   const mi_model_desc& d = e->d;
   const size_t R = (size_t)B * L;
@@ -871,7 +904,14 @@ int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool wan
   }
 
   bool qkv_done = false;     // this layer's q|k|v already ran behind the previous layer's down_proj
-  for (int li = 0; li < d.num_layers; ++li) {
+  const bool small = small_stack_takes(e, kv, act, B, L, rows);
+  if (small) {
+    SmallStackCall c{AttnShape{B, L, Hq, Hkv, D, act, kv->dtype, RND_NONE, kv->cap, d_rows}, d.num_layers, H, I, e->small_kind, e->layers[0].qkv.W.group, rndT, d.rms_norm_eps,
+                     1.0f / sqrtf((float)D), e->small_words, e->small_scales, e->small_norms, (float*)e->h, (float*)kv->k, (float*)kv->v, layer_elems, kv->d_off, e->cos_tab, e->sin_tab};
+    kv_shape(kv, c.s);
+    MI_TRY(launch_stack_small(c, st));
+  }
+  for (int li = small ? d.num_layers : 0; li < d.num_layers; ++li) {
     LayerW& lw = e->layers[li];
     const bool w32 = quirk && d.act_dtype != MI_F32;     // norm weights must match the activation storage type
     const void* in_norm = w32 ? lw.in_norm32 : lw.in_norm;
@@ -954,7 +994,7 @@ int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool wan
     if (all_pos) { c.x = e->h; c.ldx = H; MI_TRY(gemv_rows(e, head, c, R, es, sizeof(float), "gemv_head")); }
     else { c.x = (char*)e->h + (size_t)(L - 1) * H * es; c.ldx = L * H; MI_TRY(gemv_rows(e, head, c, B, es, sizeof(float), "gemv_head")); }
   }
-  MI_TRY(launch_advance_offsets(kv->d_off, d_rows, B, L, st));
+  if (!small) MI_TRY(launch_advance_offsets(kv->d_off, d_rows, B, L, st));
   for (int b = 0; b < B; ++b) kv->h_off[row_of(b)] += L;
   return MI_OK;
 }
@@ -1216,7 +1256,7 @@ void mi_engine_destroy(mi_engine* e) {
     hipFree(l.in_norm); hipFree(l.post_norm); hipFree(l.q_norm); hipFree(l.k_norm);
     hipFree(l.in_norm32); hipFree(l.post_norm32); hipFree(l.q_norm32); hipFree(l.k_norm32);
   }
-  hipFree(e->final_norm32); hipFree(e->xn); hipFree(e->xs); hipFree(e->gk_ws);
+  hipFree(e->small_buf); hipFree(e->final_norm32); hipFree(e->xn); hipFree(e->xs); hipFree(e->gk_ws);
   free_linear(e->embed); free_linear(e->lm_head);
   hipFree(e->final_norm); hipFree(e->cos_tab); hipFree(e->sin_tab);
   hipFree(e->h); hipFree(e->qkv); hipFree(e->q); hipFree(e->attn); hipFree(e->act); hipFree(e->logits); hipFree(e->lora_t); hipFree(e->d_forced); hipFree(e->d_gather);
@@ -1314,6 +1354,7 @@ int mi_engine_set_lora(mi_engine* e, int layer, const char* proj, const void* A,
   MI_HIP(dev_malloc(e, &f->lora_b[slot], (size_t)rank * n * sizeof(float)));
   MI_TRY(copy_in(f->lora_a[slot], A, (size_t)K * rank * sizeof(float), on_device, e->stream));
   MI_TRY(copy_in(f->lora_b[slot], B, (size_t)rank * n * sizeof(float), on_device, e->stream));
+  hipFree(e->small_buf); e->small_buf = nullptr;      // (no adapters there; the stream is idle)
   f->W.lora_a[slot] = f->lora_a[slot]; f->W.lora_b[slot] = f->lora_b[slot];
   f->W.lora_row0[slot] = row0; f->W.lora_n[slot] = n; f->W.lora_rank[slot] = rank; f->W.lora_scale[slot] = scale;
   return MI_OK;
@@ -1353,6 +1394,7 @@ int mi_engine_finalize(mi_engine* e) {
   MI_HIP(hipMalloc(&e->sin_tab, n * sizeof(float)));
   MI_TRY(launch_rope_tables(e->cos_tab, e->sin_tab, d.max_positions, d.head_dim, d.rope_theta, d.rope_scale, e->stream));
   make_codes_copies(e);
+  MI_TRY(make_small_stack(e));
   MI_HIP(hipStreamSynchronize(e->stream));
   e->finalized = true;
   return MI_OK;
@@ -1855,6 +1897,7 @@ int mi_engine_set_option(mi_engine* e, const char* key, int64_t value) {
   if (!e || !key) return fail(MI_ERR_INVALID, "null argument");
   const std::string k(key);
   if (k == "force_generic_gemv") { e->opt_force_v1 = value != 0; return MI_OK; }
+  if (k == "small_stack") { e->opt_small_stack = value != 0; return MI_OK; }
   if (k == "fused_decode_attention") { e->opt_fused_attn = value != 0; return MI_OK; }
   if (k == "prefill_gemm") { e->opt_prefill_gemm = value != 0; return MI_OK; }
   if (k == "skinny_gemm") { e->opt_skinny_gemm = value != 0; return MI_OK; }

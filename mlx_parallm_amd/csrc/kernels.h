@@ -364,6 +364,28 @@ int launch_attention_decode(const AttnDecodeCall& c, hipStream_t st);
 bool attention_decode_supported(const AttnShape& s);
 bool gemv_mfma_supported(const LinearW& W, const GemvCall& c);
 
+// A decode step of a small model in one launch (stack_small.hip): float32 activations and caches, no norm of queries and keys, no adapters.  Words and scales of the
+// layers, q|k|v, o, gate|up and down behind one another in each; the two norms' weights of each
+enum : int { SMALL_F32 = 0, SMALL_BF16 = 1, SMALL_F16 = 2, SMALL_CODES = 3 };
+constexpr int SMALL_MAX_KEYS = 256;     // (keys of a row, the new one included)
+struct SmallStackCall {
+  AttnShape s;                   // L = 1; rows, block table
+  int layers, H, I, kind, group, rnd0;     // rnd0: logical rounding of layer 0 up to its attention
+  float eps, scale;
+  const uint32_t* words; const float2* scales; const float* norms;
+  float* h;                      // [B][H] embeddings in, last hidden states out
+  float* kcache; float* vcache; size_t layer_elems;
+  int32_t* offsets;              // [cache row], advanced by one
+  const float* cos_tab; const float* sin_tab;
+};
+bool small_stack_fits(const LinearW& W, bool big);       // big: q|k|v, gate|up
+bool small_stack_shape(int H, int heads, int kv_heads, int D, int I);
+int small_stack_kind(const LinearW& W);
+size_t small_stack_words(int kind, bool big);
+size_t small_stack_scales(int kind);
+int launch_small_pack(const LinearW& W, bool big, uint32_t* words, float2* sb, hipStream_t st);
+int launch_stack_small(const SmallStackCall& c, hipStream_t st);
+
 struct SampleCall {
   float* logits;         // [B][V] float32 (modified in place by logit_bias)
   int B, V;

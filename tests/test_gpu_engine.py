@@ -1228,3 +1228,38 @@ def test_int4_feed_forward_widths_between_blocks_of_the_tile_major_layout(dtype,
             assert np.isfinite(out[0]).all() and np.abs(out[0] - out[1]).max() <= far, (B, Lt, lora, np.abs(out[0] - out[1]).max(), far)
     e0.close()
     e1.close()
+
+
+@pytest.mark.parametrize("dtype,bits,group", [("float32", 0, 64), ("bfloat16", 0, 64), ("float16", 0, 64), ("bfloat16", 4, 64), ("float32", 4, 32), ("float16", 8, 64)])
+@pytest.mark.parametrize("heads,kv_heads,hd,hidden,ff", [(4, 4, 16, 64, 128), (4, 2, 16, 64, 64), (2, 1, 32, 64, 128), (8, 1, 16, 64, 64)])
+def test_a_small_model_s_step_in_one_launch_equals_the_launches_it_replaces(tmp_path, dtype, bits, group, heads, kv_heads, hd, hidden, ff):
+    """Decode steps with float32 activations of models whose matrices fit one workgroup's registers: rows of unequal lengths up to the longest it takes and past
+    it (there both runs are the same kernels), both cache forms, a subset of the rows.  Float32 sums in another order; in the 16-bit models' first layer a
+    rounding may fall the other way (their tests' bound)."""
+    from mlx_parallm_amd.tiny_model import build_tiny_model
+
+    cfg = build_tiny_model(tmp_path, seed=5, vocab_size=512, dtype=dtype, quantize_model=bits > 0, q_bits=bits or 4, q_group_size=group, hidden_size=hidden, layers=3, heads=heads,
+                           kv_heads=kv_heads, intermediate_size=ff, head_dim=hd, norm_jitter=0.2, with_tokenizer=False)
+    eng = utils.load_model(str(tmp_path), max_positions=1024).engine
+    rng, longest = np.random.default_rng(3), 256
+    lens = [1, 7, 63, 64, longest - 3]
+    prompts = [rng.integers(0, 512, n).astype(np.int32) for n in lens]
+    steps = rng.integers(0, 512, (6, len(lens))).astype(np.int32)
+    outs = {}
+    for paged in (False, True):
+        for on in (1, 0):
+            eng.set_option("small_stack", on)
+            kv = eng.new_paged_kv(5, block_tokens=16, max_tokens_per_row=longest + 16, kv_dtype="float32") if paged else eng.new_kv(5, capacity=longest + 16, kv_dtype="float32")
+            for r, p in enumerate(prompts):
+                eng.forward_segments(kv, [r], [p])
+            got = [eng.forward(s[:, None], kv) for s in steps]
+            eng.step_wait(eng.step_enqueue_rows(kv, [3, 1], steps[0, [3, 1]][:, None]), 2)
+            got.append(eng.forward(steps[1][:, None], kv))
+            outs[paged, on] = np.stack(got)
+            kv.close()
+        d = np.abs(outs[paged, 1] - outs[paged, 0])
+        assert d.max() <= (2e-5 if dtype == "float32" else 4e-3) * max(1.0, np.abs(outs[paged, 0]).max()), d.max()
+        assert not np.array_equal(outs[paged, 1], outs[paged, 0])
+    assert np.array_equal(outs[True, 1], outs[False, 1])
+    eng.set_option("small_stack", 1)
+    eng.close()
