@@ -204,6 +204,7 @@ struct mi_engine {
   void* small_buf = nullptr; uint32_t* small_words = nullptr; float2* small_scales = nullptr; float* small_norms = nullptr;
   int small_kind = 0;
   bool opt_small_stack = true;
+  bool opt_mixed_attn = true;      // mixed steps: a chunk's attention in the decoding rows' launch
   // ---- layer-list models (engine_layers.hip)
   bool layered = false;
   std::vector<ListLayer> list;

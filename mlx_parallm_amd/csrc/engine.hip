@@ -1065,19 +1065,20 @@ int forward_mixed(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t* l
       MI_TRY(gemv_rows(e, lw.qkv, c, R, es, es, "gemv_qkv")); }
     void* kc = (char*)kv->k + (size_t)li * layer_elems * kes;
     void* vc = (char*)kv->v + (size_t)li * layer_elems * kes;
+    AttnDecodeCall dc{};
+    bool rows_wait = false;                      // (for a chunk whose launch they share)
     if (nd > 0) {                                // the decode rows: tokens [0, nd)
       AttnShape s{nd, 1, Hq, Hkv, D, act, kv->dtype, rnd, kv->cap, kv->d_rows};
       kv_shape(kv, s);
       if (e->opt_fused_attn && attention_decode_supported(s)) {
-        AttnDecodeCall ac{s, e->qkv, kc, vc, kv->d_off, q_norm, k_norm, d.rms_norm_eps, e->cos_tab, e->sin_tab,
-                          e->attn, 1.0f / sqrtf((float)D), RND_NONE, nsplit, kv->partial, kv->counters,
-                          e->opt_attn_mfma ? 0 : 1};
+        dc = AttnDecodeCall{s, e->qkv, kc, vc, kv->d_off, q_norm, k_norm, d.rms_norm_eps, e->cos_tab, e->sin_tab,
+                            e->attn, 1.0f / sqrtf((float)D), RND_NONE, nsplit, kv->partial, kv->counters,
+                            e->opt_attn_mfma ? 0 : 1};
         if (nd <= 32) {
-          ac.n_host_off = nd;
-          for (int b = 0; b < nd; ++b) { ac.host_row[b] = rows[b]; ac.host_off[b] = kv->h_off[rows[b]]; }
+          dc.n_host_off = nd;
+          for (int b = 0; b < nd; ++b) { dc.host_row[b] = rows[b]; dc.host_off[b] = kv->h_off[rows[b]]; }
         }
-        Prof pr(e, "attn");
-        MI_TRY(launch_attention_decode(ac, st));
+        rows_wait = true;
       } else {
         RopeAppendCall rc{s, e->qkv, e->q, kc, vc, kv->d_off, q_norm, k_norm, d.rms_norm_eps, e->cos_tab, e->sin_tab, d.max_positions};
         MI_TRY(launch_rope_append(rc, st));
@@ -1097,7 +1098,17 @@ int forward_mixed(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t* l
       AttnShape sa = s; sa.rnd = RND_NONE;
       AttnCall ac{sa, q_i, kc, vc, kv->d_off, o_i, 1.0f / sqrtf((float)D), 1, nullptr, e->opt_attn_mfma ? 0 : 1};
       MI_TRY(split_prefill(e, ac, kv->h_off[rows[i]] + lens[i]));
-      MI_TRY(launch_attention(ac, st));
+      if (rows_wait && e->opt_mixed_attn && attention_mixed_takes(dc, ac, gemv_cu_count())) {
+        Prof pr(e, "attn");
+        MI_TRY(launch_attention_mixed(dc, ac, st));
+        rows_wait = false;
+      } else {
+        MI_TRY(launch_attention(ac, st));
+      }
+    }
+    if (rows_wait) {
+      Prof pr(e, "attn");
+      MI_TRY(launch_attention_decode(dc, st));
     }
     { GemvCall co; co.x = e->attn; co.ldx = Hq * D; co.act = act; co.rnd = RND_NONE; co.epi = EPI_RESID; co.resid = e->h; co.ldo = H;
       MI_TRY(gemv_rows(e, lw.o, co, R, es, es, "gemv_o"));
@@ -1897,6 +1908,7 @@ int mi_engine_set_option(mi_engine* e, const char* key, int64_t value) {
   if (!e || !key) return fail(MI_ERR_INVALID, "null argument");
   const std::string k(key);
   if (k == "force_generic_gemv") { e->opt_force_v1 = value != 0; return MI_OK; }
+  if (k == "mixed_attention") { e->opt_mixed_attn = value != 0; return MI_OK; }
   if (k == "small_stack") { e->opt_small_stack = value != 0; return MI_OK; }
   if (k == "fused_decode_attention") { e->opt_fused_attn = value != 0; return MI_OK; }
   if (k == "prefill_gemm") { e->opt_prefill_gemm = value != 0; return MI_OK; }

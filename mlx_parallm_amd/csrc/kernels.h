@@ -362,6 +362,9 @@ struct AttnDecodeCall {
 };
 int launch_attention_decode(const AttnDecodeCall& c, hipStream_t st);
 bool attention_decode_supported(const AttnShape& s);
+// decoding rows and a chunk of another row's prompt (rotated and appended) in one launch, where that is ahead of two on ncu compute units
+bool attention_mixed_takes(const AttnDecodeCall& c, const AttnCall& p, int ncu);
+int launch_attention_mixed(const AttnDecodeCall& c, const AttnCall& p, hipStream_t st);
 bool gemv_mfma_supported(const LinearW& W, const GemvCall& c);
 
 // A decode step of a small model in one launch (stack_small.hip): float32 activations and caches, no norm of queries and keys, no adapters.  Words and scales of the

@@ -1263,3 +1263,41 @@ def test_a_small_model_s_step_in_one_launch_equals_the_launches_it_replaces(tmp_
     assert np.array_equal(outs[True, 1], outs[False, 1])
     eng.set_option("small_stack", 1)
     eng.close()
+
+
+@pytest.mark.parametrize("dtype,arch,heads,kv_heads,rows,chunks", [
+    ("bfloat16", "qwen3", 10, 2, 3, (32,)),          # 5 heads a kv head, norms of q and k
+    ("float16", "llama", 4, 1, 40, (16, 33)),        # more rows than the kernel arguments hold, the second chunk on its own
+    ("bfloat16", "llama", 8, 1, 1, (17,)), ("float16", "qwen3", 2, 1, 2, (40,)), ("bfloat16", "llama", 3, 3, 5, (200, 2))])
+def test_a_mixed_step_s_attention_in_one_launch_equals_two_launches(tmp_path, dtype, arch, heads, kv_heads, rows, chunks):
+    """Decoding rows of unequal lengths and chunks of other rows' prompts, first on empty caches, then behind cached tokens (keys in slices): the same bits with the
+    chunk's workgroups in the rows' launch."""
+    from mlx_parallm_amd.tiny_model import build_tiny_model
+
+    build_tiny_model(tmp_path, seed=9, vocab_size=512, model_type=arch, dtype=dtype, quantize_model=False, hidden_size=128, layers=2, heads=heads, kv_heads=kv_heads, head_dim=128,
+                     intermediate_size=128, norm_jitter=0.2, with_tokenizer=False)
+    eng = utils.load_model(str(tmp_path), max_positions=2048).engine
+    rng = np.random.default_rng(2)
+    n = rows + len(chunks)
+    prompts = [rng.integers(0, 512, 1 + (37 * r * r) % 600).astype(np.int32) for r in range(rows)]
+    steps = rng.integers(0, 512, (4, rows)).astype(np.int32)
+    pieces = [[rng.integers(0, 512, c).astype(np.int32) for c in chunks] for _ in range(4)]
+    outs = []
+    for on in (1, 0):
+        eng.set_option("mixed_attention", on)
+        kv = eng.new_paged_kv(n, block_tokens=16, max_tokens_per_row=2048)
+        for r, p in enumerate(prompts):
+            eng.forward_segments(kv, [r], [p])
+        got = []
+        for i in range(4):
+            toks = [steps[i, r:r + 1] for r in range(rows)] + pieces[i]
+            got.append(eng.forward_segments(kv, list(range(n)), toks, list(np.cumsum([len(t) for t in toks]) - 1)))
+            want = [1] * n
+            res = eng.step_wait(eng.step_enqueue_mixed(kv, list(range(n)), toks, want, SampleArgs(temp=0.0)), n)
+            got.append(res["logprobs"])
+        outs.append([np.array(g) for g in got])
+        kv.close()
+    for a, b in zip(*outs):
+        assert np.isfinite(a).all() and np.array_equal(a, b)
+    eng.set_option("mixed_attention", 1)
+    eng.close()
