@@ -367,6 +367,7 @@ int launch_attention(const AttnCall& c, hipStream_t st) {
   const AttnShape& s = c.s;
   if (s.Hq % s.Hkv != 0) return fail(MI_ERR_INVALID, "attention: Hq must be a multiple of Hkv");
   if (s.L > 1 && c.variant != 1 && attention_prefill_supported(s)) return launch_attention_prefill(c, st);
+  if (c.frag_mt > 0) return fail(MI_ERR_UNSUPPORTED, "attention: rows in fragment order");
   if (c.nsplit < 1 || (c.nsplit > 1 && (s.L != 1 || c.partial == nullptr)))
     return fail(MI_ERR_INVALID, "attention: bad split configuration");
   if (s.act == MI_F32 && s.kv == MI_F32) return launch_attn_d<float, float>(c, st);

@@ -929,7 +929,8 @@ __device__ __forceinline__ void attn_decode_mfma_body(const AttnDecodeCall& c, c
     }
   }
   __syncthreads();
-  T* out = (T*)c.out + (size_t)b * nq;
+  // element k of this row: (uniform)
+  auto out = [&](int k) { return (T*)c.out + (c.frag_mt > 0 ? q4_frag_elem(b, k, c.frag_mt, nq / 64) : (size_t)b * nq + k); };
   for (int idx = tid; idx < G * D; idx += NTH) {
     const int g = idx / D, d = idx % D;
     float mn = -1e30f;
@@ -944,7 +945,7 @@ __device__ __forceinline__ void attn_decode_mfma_body(const AttnDecodeCall& c, c
     }
     const int h = kh * G + g;
     if (nsplit == 1) {
-      store_out<T>(&out[(size_t)h * D + d], store_act<T>(O / L, c.rnd_out), WT);
+      store_out<T>(out(h * D + d), store_act<T>(O / L, c.rnd_out), WT);
     } else {
       float* pp = c.partial + (((size_t)b * s.Hq + h) * c.nsplit + split) * (D + 2);
       __hip_atomic_store(&pp[2 + d], O, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -968,7 +969,7 @@ __device__ __forceinline__ void attn_decode_mfma_body(const AttnDecodeCall& c, c
   for (int idx = tid; idx < G * D; idx += NTH) {
     const int g = idx / D, d = idx % D, h = kh * G + g;
     const float* pp = c.partial + ((size_t)b * s.Hq + h) * c.nsplit * (D + 2);
-    store_out<T>(&out[(size_t)h * D + d], store_act<T>(combine_splits<D>(pp, nsplit, d), c.rnd_out), WT);
+    store_out<T>(out(h * D + d), store_act<T>(combine_splits<D>(pp, nsplit, d), c.rnd_out), WT);
   }
 }
 
@@ -1193,6 +1194,7 @@ int launch_attention_decode(const AttnDecodeCall& c, hipStream_t st) {
   if (!attention_decode_supported(s)) return fail(MI_ERR_UNSUPPORTED, "attention_decode: shape / dtype not supported");
   if (c.nsplit < 1 || (c.nsplit > 1 && c.partial == nullptr))
     return fail(MI_ERR_INVALID, "attention_decode: bad split configuration");
+  if (c.frag_mt > 0 && (s.act == MI_F32 || c.variant == 1)) return fail(MI_ERR_UNSUPPORTED, "attention_decode: rows in fragment order");
   if (s.act == MI_F32) return launch_d<float>(c, st);
   if (s.act == MI_BF16) return launch_d<bf16>(c, st);
   return launch_d<f16>(c, st);

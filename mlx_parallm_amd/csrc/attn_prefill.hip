@@ -227,6 +227,11 @@ __global__ __launch_bounds__(G * 64, G >= 2 ? 2 : 1) void attn_prefill_dma_kerne
   attn_prefill_dma_body<T, D, G, PAGED, QG, SPLIT>(c, gridDim.x - 1 - blockIdx.x, blockIdx.y, gridDim.x, blockIdx.z, gridDim.z, smem);
 }
 
+bool dma_kernel() {                                    // A/B and the bit-equality test: 0 = the register-staged kernel (read per call)
+  const char* env = getenv("MI_ATTN_PREFILL_DMA");
+  return env == nullptr || atoi(env) != 0;
+}
+
 template <typename T, int D, int G>
 int launch_pg(const AttnCall& c, hipStream_t st) {
   const AttnShape& s = c.s;
@@ -234,8 +239,7 @@ int launch_pg(const AttnCall& c, hipStream_t st) {
   // measured: prefill 83.3 .. 83.8 k tok/s against 84.0 .. 84.1 k (same box, alternating runs) -- the vector ALU bounds the
   // loop, not the LDS traffic -- and 79 k once the leaner softmax below pushed it past 256 registers.
   dim3 grid((s.L + QT - 1) / QT, s.B * s.Hkv), block(G * 64);
-  const char* env = getenv("MI_ATTN_PREFILL_DMA");     // A/B and the bit-equality test: 0 = the register-staged kernel (read per call)
-  if (env == nullptr || atoi(env) != 0) {
+  if (dma_kernel()) {
     grid.z = c.nsplit;
     if (c.nsplit > 1) {
       if (s.btab) hipLaunchKernelGGL((attn_prefill_dma_kernel<T, D, G, true, 1, true>), grid, block, 0, st, c);
@@ -651,6 +655,8 @@ bool attention_prefill_supported(const AttnShape& s) {
   return s.D == 32 || s.D == 64 || s.D == 128;
 }
 
+bool attention_prefill_frag(const AttnShape& s) { return attention_prefill_supported(s) && s.act != MI_F32 && dma_kernel(); }
+
 // Slices of the keys: at most as many as fill the chip (one workgroup per CU).  The costs, fitted to launches of 1 to 16 slices at 48 shapes (rocprof;
 // head groups of 1 to 8, head_dim 32 to 128, 8 to 132 key blocks; keys cold, the chunk's own warm): a key block takes 0.85 us, on float32
 // caches 1.3 + 2 / G; the join 2 + 0.47 G us, and a slice more per slice the more tiles publish theirs at once.  The rule's pick is within 2 % of
@@ -676,6 +682,7 @@ int launch_attention_prefill(const AttnCall& c, hipStream_t st) {
   if (!attention_prefill_supported(c.s)) return fail(MI_ERR_UNSUPPORTED, "attention_prefill: shape / dtype not supported");
   if (c.nsplit < 1 || c.nsplit > PREFILL_MAX_SLICES || (c.nsplit > 1 && (c.partial == nullptr || c.counters == nullptr)))
     return fail(MI_ERR_INVALID, "attention_prefill: bad split configuration");
+  if (c.frag_mt > 0 && !attention_prefill_frag(c.s)) return fail(MI_ERR_UNSUPPORTED, "attention_prefill: rows in fragment order");
   if (c.s.act == MI_F32) return c.s.D == 128 ? launch_pd32<128>(c, st) : launch_pd32<64>(c, st);
   return c.s.act == MI_BF16 ? launch_pt<bf16>(c, st) : launch_pt<f16>(c, st);
 }

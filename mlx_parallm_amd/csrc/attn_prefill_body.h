@@ -316,6 +316,18 @@ __device__ __forceinline__ void attn_prefill_dma_body(const AttnCall& c, const i
     }
     if (t0 + QT * u + c16 < s.L) {
       const float inv = 1.0f / l;
+      if (c.frag_mt > 0) {                            // (uniform) 8 k of the output linear's x from a pair of lanes: elements j and j + 4 of them share a word
+        const int row = c.frag_row0 + b * s.L + tq[u];
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+          const u32x2 v = {pack2<T>(accO[u][dt][0] * inv, accO[u][dt][1] * inv), pack2<T>(accO[u][dt][2] * inv, accO[u][dt][3] * inv)};
+          const u32x2 w = {(uint32_t)__shfl_xor((int)v.x, 16, 64), (uint32_t)__shfl_xor((int)v.y, 16, 64)};
+          if ((g4 & 1) == 0)
+            *(u32x4*)((T*)c.out + q4_frag_elem(row, h * D + 16 * dt + 4 * g4, c.frag_mt, s.Hq * D / 64)) =
+                u32x4{(v.x & 0xffffu) | w.x << 16, v.x >> 16 | (w.x & 0xffff0000u), (v.y & 0xffffu) | w.y << 16, v.y >> 16 | (w.y & 0xffff0000u)};
+        }
+        continue;
+      }
       T* op = (T*)c.out + ((size_t)b * s.L + tq[u]) * s.Hq * D + (size_t)h * D + 4 * g4;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {

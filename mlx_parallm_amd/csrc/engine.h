@@ -204,6 +204,9 @@ struct mi_engine {
   void* small_buf = nullptr; uint32_t* small_words = nullptr; float2* small_scales = nullptr; float* small_norms = nullptr;
   int small_kind = 0;
   bool opt_small_stack = true;
+  // int4 output linears that read their x in fragment order (gemm_q4.hip): the attention leaves it there [128][heads x head_dim]
+  void* o_frag = nullptr;
+  bool opt_attn_frag = true;
   bool opt_mixed_attn = true;      // mixed steps: a chunk's attention in the decoding rows' launch
   // ---- layer-list models (engine_layers.hip)
   bool layered = false;

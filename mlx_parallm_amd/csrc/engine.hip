@@ -306,6 +306,11 @@ int gemv_rows(mi_engine* e, const FusedLinear& f0, GemvCall c, size_t rows, size
 // f: the matrix the matmul kernels stream (f0 itself, or its [hi | lo] view); f0: the linear as loaded (true K, LoRA)
 int gemv_rows_on(mi_engine* e, const FusedLinear& f, const FusedLinear& f0, GemvCall c, size_t rows, size_t es_in, size_t es_out,
                  const char* prof, bool sq_was_valid) {
+  if (c.x_frag > 0) {                         // (o_frag_mt has looked at what stands below)
+    Prof pr(e, prof);
+    c.M = (int)rows;
+    return launch_gemm_q4(f.W, c, rows, e->stream, nullptr, nullptr);
+  }
   const int KT = f0.W.K;                      // the true K: columns of x
   const size_t es_res = c.out32 ? sizeof(float) : es_in;     // element size of the residual stream
   // Which kernel for a call that is not a pure decode step (prefill, mixed step)?  Measured on Mistral-7B shapes, one prompt
@@ -789,6 +794,19 @@ int choose_nsplit(const mi_kv* kv, int B, int Hkv, int L, const int32_t* rows = 
   return ns_env > 0 ? decode_row_splits(std::min(ns_env, 16), mx) : attention_decode_splits(gemv_cu_count(), Hkv * alike, mx, kv->dtype == MI_F32);
 }
 
+// Does the attention in front of the output linear `co` of `rows` rows leave its rows as gemm_q4.hip multiplies them, instead of a preparation launch (4.8 us)?  -> the
+// row tiles a slab, 0: no.  Where gemv_rows would have that kernel prepare them; an adapter reads the rows as they are.  Whole calls, decode steps of 24 rows x 705 keys (4096 wide) 6.23 -> 6.11 ms,
+// 64 x 513 (5120) 17.19 -> 16.97, 100 x 257 11.77 -> 11.74; 31 rows and 32 tokens mixed 6.67 -> 6.57.
+int o_frag_mt(mi_engine* e, const FusedLinear& o, const GemvCall& co, size_t rows) {
+  if (!e->opt_attn_frag || !e->opt_skinny_gemm || !e->opt_attn_mfma || !e->opt_fused_attn || e->opt_force_v1 || co.act == MI_F32 || rows < 17 || rows > 128) return 0;
+  if ((e->cur_L != 1 && !e->opt_short_prefill_skinny) || o.W.lora_b[0] != nullptr || o.W.lora_b[1] != nullptr || getenv("MI_SKINNY_DECODE_MAX") != nullptr) return 0;
+  if (!gemm_skinny_supported(o.W, co, rows)) return 0;
+  const int mt = gemm_q4_frag_mt(o.W, co, rows);
+  if (mt == 0) return 0;
+  if (e->o_frag == nullptr && dev_malloc(e, &e->o_frag, (size_t)128 * o.W.K * 2) != hipSuccess) { (void)hipGetLastError(); e->o_frag = nullptr; return 0; }
+  return mt;
+}
+
 // prefill attention (L > 1): the keys split over workgroups where the query tiles alone leave the chip idle
 int split_prefill(mi_engine* e, AttnCall& ac, int max_keys) {
   ac.nsplit = 1; ac.partial = nullptr;
@@ -942,6 +960,7 @@ int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool wan
       AttnDecodeCall ac{s, e->qkv, kc, vc, kv->d_off, q_norm, k_norm, d.rms_norm_eps, e->cos_tab, e->sin_tab,
                         e->attn, 1.0f / sqrtf((float)D), RND_NONE, nsplit, kv->partial, kv->counters,
                         e->opt_attn_mfma ? 0 : 1};
+      if (const int mt = o_frag_mt(e, lw.o, co, R)) { ac.out = e->o_frag; ac.frag_mt = co.x_frag = mt; co.x = e->o_frag; }
       if (B <= 32) {
         ac.n_host_off = B;
         for (int b = 0; b < B; ++b) { ac.host_row[b] = row_of(b); ac.host_off[b] = kv->h_off[row_of(b)]; }
@@ -1053,6 +1072,11 @@ int forward_mixed(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t* l
     MI_HIP(dev_malloc(e, &kv->partial, (size_t)kv->B * Hq * 16 * (D + 2) * sizeof(float)));
     kv->partial_splits = 16;
   }
+  bool chunks_frag = true;                       // (every attention launch of the step can leave its rows in fragment order)
+  for (int i = 0; i < n; ++i) {
+    AttnShape s{i < nd ? nd : 1, lens[i], Hq, Hkv, D, act, kv->dtype, RND_NONE, kv->cap, nullptr};
+    chunks_frag = chunks_frag && (i < nd ? attention_decode_supported(s) : attention_prefill_frag(s));
+  }
   for (int li = 0; li < d.num_layers; ++li) {
     LayerW& lw = e->layers[li];
     const bool w32 = quirk && d.act_dtype != MI_F32;
@@ -1065,6 +1089,9 @@ int forward_mixed(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t* l
       MI_TRY(gemv_rows(e, lw.qkv, c, R, es, es, "gemv_qkv")); }
     void* kc = (char*)kv->k + (size_t)li * layer_elems * kes;
     void* vc = (char*)kv->v + (size_t)li * layer_elems * kes;
+    GemvCall co; co.x = e->attn; co.ldx = Hq * D; co.act = act; co.rnd = RND_NONE; co.epi = EPI_RESID; co.resid = e->h; co.ldo = H;
+    const int frag = chunks_frag ? o_frag_mt(e, lw.o, co, R) : 0;
+    if (frag > 0) { co.x = e->o_frag; co.x_frag = frag; }
     AttnDecodeCall dc{};
     bool rows_wait = false;                      // (for a chunk whose launch they share)
     if (nd > 0) {                                // the decode rows: tokens [0, nd)
@@ -1074,6 +1101,7 @@ int forward_mixed(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t* l
         dc = AttnDecodeCall{s, e->qkv, kc, vc, kv->d_off, q_norm, k_norm, d.rms_norm_eps, e->cos_tab, e->sin_tab,
                             e->attn, 1.0f / sqrtf((float)D), RND_NONE, nsplit, kv->partial, kv->counters,
                             e->opt_attn_mfma ? 0 : 1};
+        if (frag > 0) { dc.out = e->o_frag; dc.frag_mt = frag; }
         if (nd <= 32) {
           dc.n_host_off = nd;
           for (int b = 0; b < nd; ++b) { dc.host_row[b] = rows[b]; dc.host_off[b] = kv->h_off[rows[b]]; }
@@ -1097,6 +1125,7 @@ int forward_mixed(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t* l
       MI_TRY(launch_rope_append(rc, st));
       AttnShape sa = s; sa.rnd = RND_NONE;
       AttnCall ac{sa, q_i, kc, vc, kv->d_off, o_i, 1.0f / sqrtf((float)D), 1, nullptr, e->opt_attn_mfma ? 0 : 1};
+      if (frag > 0) { ac.out = e->o_frag; ac.frag_mt = frag; ac.frag_row0 = (int)tok0[i]; }
       MI_TRY(split_prefill(e, ac, kv->h_off[rows[i]] + lens[i]));
       if (rows_wait && e->opt_mixed_attn && attention_mixed_takes(dc, ac, gemv_cu_count())) {
         Prof pr(e, "attn");
@@ -1110,8 +1139,7 @@ int forward_mixed(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t* l
       Prof pr(e, "attn");
       MI_TRY(launch_attention_decode(dc, st));
     }
-    { GemvCall co; co.x = e->attn; co.ldx = Hq * D; co.act = act; co.rnd = RND_NONE; co.epi = EPI_RESID; co.resid = e->h; co.ldo = H;
-      MI_TRY(gemv_rows(e, lw.o, co, R, es, es, "gemv_o"));
+    { MI_TRY(gemv_rows(e, lw.o, co, R, es, es, "gemv_o"));
       GemvCall cg; cg.x = e->h; cg.ldx = H; cg.act = act; cg.rnd = RND_NONE; cg.pro = PRO_NORM; cg.norm_w = post_norm;
       cg.eps = d.rms_norm_eps; cg.epi = EPI_SWIGLU; cg.out = e->act; cg.ldo = I; cg.pair_offset = I;
       cg.split_out = down_takes_split(e, lw.down, act, R);
@@ -1267,7 +1295,7 @@ void mi_engine_destroy(mi_engine* e) {
     hipFree(l.in_norm); hipFree(l.post_norm); hipFree(l.q_norm); hipFree(l.k_norm);
     hipFree(l.in_norm32); hipFree(l.post_norm32); hipFree(l.q_norm32); hipFree(l.k_norm32);
   }
-  hipFree(e->small_buf); hipFree(e->final_norm32); hipFree(e->xn); hipFree(e->xs); hipFree(e->gk_ws);
+  hipFree(e->small_buf); hipFree(e->o_frag); hipFree(e->final_norm32); hipFree(e->xn); hipFree(e->xs); hipFree(e->gk_ws);
   free_linear(e->embed); free_linear(e->lm_head);
   hipFree(e->final_norm); hipFree(e->cos_tab); hipFree(e->sin_tab);
   hipFree(e->h); hipFree(e->qkv); hipFree(e->q); hipFree(e->attn); hipFree(e->act); hipFree(e->logits); hipFree(e->lora_t); hipFree(e->d_forced); hipFree(e->d_gather);
@@ -1908,6 +1936,7 @@ int mi_engine_set_option(mi_engine* e, const char* key, int64_t value) {
   if (!e || !key) return fail(MI_ERR_INVALID, "null argument");
   const std::string k(key);
   if (k == "force_generic_gemv") { e->opt_force_v1 = value != 0; return MI_OK; }
+  if (k == "attention_frag") { e->opt_attn_frag = value != 0; return MI_OK; }
   if (k == "mixed_attention") { e->opt_mixed_attn = value != 0; return MI_OK; }
   if (k == "small_stack") { e->opt_small_stack = value != 0; return MI_OK; }
   if (k == "fused_decode_attention") { e->opt_fused_attn = value != 0; return MI_OK; }

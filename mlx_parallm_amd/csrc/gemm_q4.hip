@@ -833,6 +833,11 @@ bool gemm_q4_supported(const LinearW& W, const GemvCall& c, size_t rows) {
   return (size_t)(W.N / 16) * (W.K / 128) * 1152 < ((size_t)1 << 32);          // (32-bit offsets of the LDS-DMA sources)
 }
 
+int gemm_q4_frag_mt(const LinearW& W, const GemvCall& c, size_t rows) {
+  if (c.pro != PRO_NONE || !gemm_q4_supported(W, c, rows)) return 0;
+  const Q4Plan pl = q4_plan(W, c, rows);
+  return pl.rows ? pl.mt : 0;
+}
 size_t gemm_q4_ws_bytes(const LinearW& W, const GemvCall& c, size_t rows) { return q4_plan(W, c, rows).ws_bytes; }
 int gemm_q4_ksplit(const LinearW& W, const GemvCall& c, size_t rows) { return q4_plan(W, c, rows).ksplit; }
 int gemm_q4_groups(const LinearW& W, const GemvCall& c, size_t rows) {
@@ -843,16 +848,19 @@ int gemm_q4_groups(const LinearW& W, const GemvCall& c, size_t rows) {
 int launch_gemm_q4(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st, void* ws, unsigned* ctr) {
   if (!gemm_q4_supported(W, c, rows)) return fail(MI_ERR_INVALID, "gemm_q4: unsupported call");
   const Q4Plan pl = q4_plan(W, c, rows);
-  if (ws == nullptr || (pl.ksplit > 1 && ctr == nullptr)) return fail(MI_ERR_INVALID, "gemm_q4: workspace missing");
+  if (c.x_frag > 0 && (!pl.rows || pl.mt != c.x_frag || c.pro != PRO_NONE)) return fail(MI_ERR_INVALID, "gemm_q4: x prepared for another call");
+  if (c.x_frag == 0 && (ws == nullptr || (pl.ksplit > 1 && ctr == nullptr))) return fail(MI_ERR_INVALID, "gemm_q4: workspace missing");
   void* xq = ws;
   float* sx = (float*)((char*)ws + pl.xq_bytes);
   float* sxo = (float*)((char*)sx + pl.sx_bytes);
-  const void* nw = c.pro == PRO_NORM ? c.norm_w : nullptr;
-  const dim3 grid(pl.nslab * pl.mt * 16, nw != nullptr ? 1 : (W.K + 2047) / 2048);
-  (c.act == MI_BF16 ? q4_prep_launch<bf16> : q4_prep_launch<f16>)(c, grid, (int)rows, pl.mt, W.K, nw, xq, pl.rows ? nullptr : sx, sxo, st);
-  MI_HIP(hipGetLastError());
+  if (c.x_frag == 0) {
+    const void* nw = c.pro == PRO_NORM ? c.norm_w : nullptr;
+    const dim3 grid(pl.nslab * pl.mt * 16, nw != nullptr ? 1 : (W.K + 2047) / 2048);
+    (c.act == MI_BF16 ? q4_prep_launch<bf16> : q4_prep_launch<f16>)(c, grid, (int)rows, pl.mt, W.K, nw, xq, pl.rows ? nullptr : sx, sxo, st);
+    MI_HIP(hipGetLastError());
+  }
   Q4Params p{};
-  p.xq = xq; p.sx = sx; p.sxo = sxo; p.M = (int)rows; p.G = W.K / 64; p.w = W.w;
+  p.xq = c.x_frag > 0 ? c.x : xq; p.sx = sx; p.sxo = sxo; p.M = (int)rows; p.G = W.K / 64; p.w = W.w;
   p.epi = c.epi; p.out = c.out; p.ldo = c.ldo; p.resid = c.resid; p.pair_tiles = c.epi == EPI_SWIGLU ? c.pair_offset / 16 : 0;
   p.ntu = pl.ntu; p.ntiles = pl.ntiles; p.nblk = pl.nblk; p.ksplit = pl.ksplit; p.nslab = pl.nslab; p.ngroups = pl.ngroups; p.nunits = pl.ngroups * pl.ksplit;
   p.ws = (float*)((char*)sxo + pl.sxo_bytes); p.ctr = ctr;

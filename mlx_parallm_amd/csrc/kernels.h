@@ -74,6 +74,7 @@ struct GemvCall {
   float* sq_out = nullptr;
   const float* sq_in = nullptr;
   int sq_parts = 0;
+  int x_frag = 0;                 // > 0: x holds gemm_q4_frag_mt() row tiles a slab in q4_frag_elem's order, ready to be multiplied
   void* ev_start = nullptr;       // measurement: hipEvent_t pair stamped with this kernel's own begin / end
   void* ev_stop = nullptr;        // (hipExtLaunchKernelGGL); MFMA path only
 };
@@ -203,6 +204,13 @@ int gemm_q4_groups(const LinearW& W, const GemvCall& c, size_t rows);
 int gemm_q4_ksplit(const LinearW& W, const GemvCall& c, size_t rows);
 void gemm_q4_force(int code);     // test / A-B hook: mt | ksplit << 11 for this thread's next plans, any other bit: the kernel for every width; 0 clears
 int launch_gemm_q4(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t st, void* ws, unsigned* ctr);
+int gemm_q4_frag_mt(const LinearW& W, const GemvCall& c, size_t rows);      // row tiles a slab of x for a call that takes it prepared (x_frag); 0: it does not
+// where element (row, k) of x stands in the order that q4_prep_kernel leaves it in (16-bit elements; groups = K / 64)
+__host__ __device__ inline size_t q4_frag_elem(int row, int k, int mt, int groups) {
+  const int slab = row / (16 * mt), r = row - slab * 16 * mt, d = (k >> 3) & 7, j = k & 7;
+  const size_t frag = (((size_t)slab * groups + (k >> 6)) * 2 + (d & 1)) * mt + (r >> 4);
+  return (frag * 64 + (d >> 1) * 16 + (r & 15)) * 8 + (j < 4 ? 2 * j : 2 * j - 7);
+}
 
 // tile-major weight layout (repack.hip)
 bool tiled_supported(int wk, int N, int K, int group);
@@ -304,10 +312,12 @@ struct AttnCall {
   int variant;           // 0: L > 1 goes to the MFMA prefill kernel where it applies; 1: always the VALU kernel
   int* counters = nullptr;   // nsplit > 1, L > 1: attention_prefill_tiles() arrival tickets, zero between launches
   int join_cost = 0, slice_cost = 0;   // nsplit > 1, L > 1: prefill_row_slices() (0: every row takes as many slices as it can)
+  int frag_mt = 0, frag_row0 = 0;      // > 0 (attention_prefill_frag): out is q4_frag_elem's rows frag_row0 .. of the output linear's x
 };
 int launch_attention(const AttnCall& c, hipStream_t st);
 // causal prefill attention on the matrix cores (attn_prefill.hip); launch_attention dispatches to it
 bool attention_prefill_supported(const AttnShape& s);
+bool attention_prefill_frag(const AttnShape& s);       // .. and AttnCall::frag_mt
 // over how many workgroups the keys of a call that reaches at most max_keys keys are split on ncu compute units (sets c's costs), and what
 // that needs
 int attention_prefill_slices(AttnCall& c, int max_keys, int ncu);
@@ -359,6 +369,7 @@ struct AttnDecodeCall {
   int n_host_off;          // > 0: host_off[b] = offsets[cache row of b], host_row[b] = that cache row (B <= 32)
   int host_off[32];
   int host_row[32];
+  int frag_mt;             // > 0 (16-bit caches, variant 0): row b of out stands in q4_frag_elem's order
 };
 int launch_attention_decode(const AttnDecodeCall& c, hipStream_t st);
 bool attention_decode_supported(const AttnShape& s);

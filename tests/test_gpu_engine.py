@@ -1301,3 +1301,42 @@ def test_a_mixed_step_s_attention_in_one_launch_equals_two_launches(tmp_path, dt
         assert np.isfinite(a).all() and np.array_equal(a, b)
     eng.set_option("mixed_attention", 1)
     eng.close()
+
+
+@pytest.mark.parametrize("dtype,arch,heads,kv_heads,hd", [("bfloat16", "qwen3", 5, 1, 128), ("float16", "llama", 8, 8, 64), ("bfloat16", "llama", 16, 4, 32)])
+def test_attention_that_leaves_its_rows_prepared_for_the_int4_output_linear(tmp_path, dtype, arch, heads, kv_heads, hd):
+    """Decode steps and mixed steps of 17 to 128 rows (every number of row tiles and slabs) of an int4 model: the attention's rows in the output linear's order, the
+    same bits as with its preparation launch; an adapter on the output linear of one layer keeps that one."""
+    from mlx_parallm_amd.tiny_model import build_tiny_model
+
+    build_tiny_model(tmp_path, seed=4, vocab_size=512, model_type=arch, dtype=dtype, quantize_model=True, hidden_size=256, layers=2, heads=heads, kv_heads=kv_heads, head_dim=hd,
+                     intermediate_size=256, norm_jitter=0.2, with_tokenizer=False)
+    eng = utils.load_model(str(tmp_path), max_positions=1024).engine
+    rng = np.random.default_rng(6)
+    calls = [([r], 0) for r in (17, 33, 64, 65, 97, 128)] + [([12], 16), ([30], 33), ([3], 90)]
+    plans = [(rows[0], chunk, [rng.integers(0, 512, 1 + (29 * i) % 300).astype(np.int32) for i in range(rows[0] + (chunk > 0))],
+              [rng.integers(0, 512, chunk or 1).astype(np.int32) for _ in range(2)], rng.integers(0, 512, (2, rows[0])).astype(np.int32)) for rows, chunk in calls]
+    for adapted in (False, True):
+        if adapted:
+            eng.set_lora(0, "self_attn.o_proj", rng.standard_normal((heads * hd, 4)).astype(np.float32) * 0.05, rng.standard_normal((4, 256)).astype(np.float32) * 0.05, 2.0)
+        outs = []
+        for on in (1, 0):
+            eng.set_option("attention_frag", on)
+            got = []
+            for rows, chunk, prompts, pieces, steps in plans:
+                kv = eng.new_paged_kv(len(prompts), block_tokens=16, max_tokens_per_row=512)
+                for r in range(0, len(prompts), 8):
+                    eng.forward_segments(kv, list(range(r, min(r + 8, len(prompts)))), prompts[r:r + 8])
+                for i in range(2):
+                    if chunk:
+                        toks = [steps[i, r:r + 1] for r in range(rows)] + [pieces[i]]
+                        got.append(eng.forward_segments(kv, list(range(rows + 1)), toks, list(np.cumsum([len(t) for t in toks]) - 1)))
+                        eng.step_wait(eng.step_enqueue_mixed(kv, list(range(rows + 1)), toks, [1] * (rows + 1), SampleArgs(temp=0.0)), rows + 1)
+                    else:
+                        got.append(eng.forward(steps[i][:, None], kv))
+                kv.close()
+            outs.append([np.array(g) for g in got])
+        for a, b in zip(*outs):
+            assert np.isfinite(a).all() and np.array_equal(a, b)
+    eng.set_option("attention_frag", 1)
+    eng.close()
