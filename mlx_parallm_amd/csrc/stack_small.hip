@@ -6,7 +6,7 @@
 // left is a chain of five barriers a layer and the instructions between them (one CU's): 43 us that step, the whole token 250 -> 76.  On the way, us: 14
 // barriers, a thread per number 72; five, and sizes of the split known at run time alone 61; no division in the loop 51; the split fixed 43.
 // The same arithmetic as the kernels it replaces: weights as scale * code + bias with two roundings, products and sums in float32, layer 0 up to its attention
-// rounded to the model's type (`rnd0`).  The limits (64 wide, 256 outputs of q|k|v and of gate|up, 128 columns of o and down) are the registers'; 256 keys because a
+// rounded to the model's type (`rnd0`).  Prompts: small_prompt_kernel.  The limits (64 wide, 256 outputs of q|k|v and of gate|up, 128 columns of o and down) are the registers'; 256 keys because a
 // row's keys are one workgroup's: longer ones take the launches, whose attention splits them.
 #include <type_traits>
 
@@ -106,6 +106,46 @@ struct Regs {
       }
     }
     return acc[0] + acc[1];
+  }
+  // The same for TG rows x[t][ld] a time of n: a weight is multiplied out once for all of them.  out: [n][NT]
+  static constexpr int TG = 8;
+  __device__ __forceinline__ void dots(const Part& p, const float* x, int ld, int n, float* out) const {
+    for (int t0 = 0; t0 < n; t0 += TG) {
+      float acc[TG];
+      int cnt = p.cnt, cut = p.cut, m = min(n - t0, TG);
+      asm volatile("" : "+s"(cnt), "+s"(cut), "+s"(m));
+      const float* xk = x + t0 * ld + p.w0 * PER;
+#pragma unroll
+      for (int t = 0; t < TG; ++t) acc[t] = 0.f;
+#pragma unroll
+      for (int i = 0; i < MW; ++i) {
+        if (i >= cnt) break;
+        float v[PER];
+        if constexpr (KIND == SMALL_F32) v[0] = __uint_as_float(w[i]);
+        else if constexpr (KIND == SMALL_BF16) { v[0] = bf16lo(w[i]); v[1] = bf16hi(w[i]); }
+        else if constexpr (KIND == SMALL_F16) { const f16* h = (const f16*)&w[i]; v[0] = (float)h[0]; v[1] = (float)h[1]; }
+        else {
+          const float sx = i < cut ? sb[0].x : sb[1].x, sy = i < cut ? sb[0].y : sb[1].y;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = mul_add_unfused((float)((w[i] >> (8 * j)) & 255u), sx, sy);
+        }
+#pragma unroll
+        for (int t = 0; t < TG; ++t) {
+          if (t >= m) break;
+          const float* xt = xk + t * ld + PER * i;
+          if constexpr (PER == 4) {
+            const float4 q = *(const float4*)xt;
+            acc[t] = fmaf(v[3], q.w, fmaf(v[2], q.z, fmaf(v[1], q.y, fmaf(v[0], q.x, acc[t]))));
+          } else {
+#pragma unroll
+            for (int j = 0; j < PER; ++j) acc[t] = fmaf(v[j], xt[j], acc[t]);
+          }
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < TG; ++t)
+        if (t < m) out[(t0 + t) * NT + threadIdx.x] = acc[t];
+    }
   }
 };
 // the groups' sums of column n, in their order
@@ -288,6 +328,167 @@ __global__ __launch_bounds__(NT) void stack_small_kernel(SmallStackCall c) {
   }
 }
 
+// The prompt of a small model, all layers in one launch: a workgroup a row again, PT tokens a time through all layers (their keys and values are the next ones' cache).
+// A wave owns every NW-th token (its columns over the lanes, residual, norm, rotation, gated unit) and takes whole (token, head)s of the attention; the matrices are
+// multiplied by all threads, PT rows a time.  Nine tokens of two rows, eight layers, 4-bit, with the logits: 642 us -> 220, 64 rows of them 14.3 -> 1.06 ms.
+constexpr int PT = 16;
+constexpr size_t prompt_lds() { return (size_t)(PT * (64 + 2 * NT + 256 + 2 * 128) + NT / 64 * SMALL_MAX_KEYS) * 4; }
+template <int KIND, int D, bool PAGED>
+__global__ __launch_bounds__(NT) void small_prompt_kernel(SmallStackCall c) {
+  constexpr int PER = Kind<KIND>::PER, NW = NT / 64, KG = 64 / D, OWN = PT / NW;
+  constexpr float LOG2E = 1.4426950408889634f;
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float* xn = lds;                                    // [PT][64]
+  float* p0 = xn + PT * 64;                           // [PT][NT]
+  float* p1 = p0 + PT * NT;                           // [PT][NT]
+  float* qkv = p1 + PT * NT;                          // [PT][256]
+  float* ov = qkv + PT * 256;                         // [PT][128]
+  float* act = ov + PT * 128;                         // [PT][128]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), b = blockIdx.x;
+  float* s = act + PT * 128 + wave * SMALL_MAX_KEYS;  // [SMALL_MAX_KEYS]: this wave's scores
+  const int H = c.H, Hq = c.s.Hq, Hkv = c.s.Hkv, G = Hq / Hkv, nq = Hq * D, nkv = Hkv * D, I = c.I, L = c.s.L;
+  const int kb = c.s.rows ? c.s.rows[b] : b, before = c.offsets[kb];
+  const Part pq = part_of<true>(nq + 2 * nkv, H / PER, c.group), po = part_of<false>(H, nq / PER, c.group), pg = part_of<true>(2 * I, H / PER, c.group), pd = part_of<false>(H, I / PER, c.group);
+  Regs<KIND, true> rq, rg;
+  Regs<KIND, false> ro, rd;
+  constexpr int OW = rq.WORDS, GW = OW + ro.WORDS, DW = GW + rg.WORDS, LW = DW + rd.WORDS;
+  rq.load(c.words, c.scales);
+  ro.load(c.words + OW, c.scales + 2 * NT);
+  rg.load(c.words + GW, c.scales + 4 * NT);
+  rd.load(c.words + DW, c.scales + 6 * NT);
+  const int col = min(lane, H - 1), ri = lane % (D / 2);
+  const float sc2 = c.scale * LOG2E;
+  float n1 = c.norms[col], n2 = c.norms[H + col];
+  for (int t0 = 0; t0 < L; t0 += PT) {
+    const int n = min(PT, L - t0), pos = before + t0; // pos: cached keys in front of these tokens
+    float x[OWN], cs[OWN], sn[OWN];
+#pragma unroll
+    for (int u = 0; u < OWN; ++u) {
+      const int t = min(wave + NW * u, n - 1);
+      x[u] = c.h[((size_t)b * L + t0 + t) * H + col];
+      if (lane >= H) x[u] = 0.f;
+      cs[u] = c.cos_tab[(size_t)(pos + t) * (D / 2) + ri]; sn[u] = c.sin_tab[(size_t)(pos + t) * (D / 2) + ri];
+    }
+    auto norm = [&](float nw, int rnd) {
+#pragma unroll
+      for (int u = 0; u < OWN; ++u) {
+        const int t = wave + NW * u;
+        if (t >= n) break;                            // (uniform)
+        const float rs = 1.0f / sqrtf(wave_sum(x[u] * x[u]) / (float)H + c.eps);
+        float v = x[u] * rs;
+        if (rnd != RND_NONE) v = round_rt(round_rt(v, rnd) * nw, rnd);
+        else v *= nw;
+        xn[t * 64 + lane] = v;
+      }
+    };
+    for (int l = 0; l < c.layers; ++l) {
+      const int rnd = l == 0 ? c.rnd0 : RND_NONE;
+      const int nl = l + 1 < c.layers ? l + 1 : 0;    // (behind the last one: the first again, for the next tokens)
+      const uint32_t* wn = c.words + (size_t)nl * LW;
+      const float2* sbn = c.scales + (size_t)nl * 8 * NT;
+      float* kc = c.kcache + (size_t)l * c.layer_elems;
+      float* vc = c.vcache + (size_t)l * c.layer_elems;
+      norm(n1, rnd);
+      n1 = c.norms[2 * nl * H + col];
+      lds_barrier();
+      rq.dots(pq, xn, 64, n, p0);
+      rq.load(wn, sbn);
+      lds_barrier();
+#pragma unroll
+      for (int u = 0; u < OWN; ++u) {
+        const int t = wave + NW * u;
+        if (t >= n) break;
+        const float* p = p0 + t * NT;
+        float* row = qkv + t * 256;
+        for (int e = lane; e < (Hq + Hkv) * (D / 2); e += 64) {
+          const int i = e / (D / 2) * D + ri;
+          float a = join<true>(p, i), v = join<true>(p, i + D / 2);
+          if (rnd != RND_NONE) { a = round_rt(a, rnd); v = round_rt(v, rnd); }
+          float ra = a * cs[u] - v * sn[u], rv = a * sn[u] + v * cs[u];
+          if (rnd != RND_NONE) { ra = round_rt(ra, rnd); rv = round_rt(rv, rnd); }
+          row[i] = ra; row[i + D / 2] = rv;
+          if (i >= nq) {
+            float* dst = kc + kv_elem<PAGED>(c.s, kb, (i - nq) / D, pos + t) + ri;
+            dst[0] = ra; dst[D / 2] = rv;
+          }
+        }
+        for (int e = lane; e < nkv; e += 64) {
+          const float v = round_rt(join<true>(p, nq + nkv + e), rnd);
+          row[nq + nkv + e] = v;
+          vc[kv_elem<PAGED>(c.s, kb, e / D, pos + t) + e % D] = v;
+        }
+      }
+      lds_barrier();
+      for (int pr = wave; pr < n * Hq; pr += NW) {    // token t, head h: the cached keys, then those of tokens 0 .. t
+        const int t = pr / Hq, h = pr - t * Hq, hk = h / G;
+        const float* q = qkv + t * 256 + h * D;
+        float mx = -1e30f;
+        auto score = [&](const float* k, int j) {
+          float d = 0.f;
+#pragma unroll
+          for (int e = 0; e < D / 4; ++e) {
+            const float4 a = *(const float4*)(k + 4 * e), w = *(const float4*)(q + 4 * e);
+            d = fmaf(a.w, w.w, fmaf(a.z, w.z, fmaf(a.y, w.y, fmaf(a.x, w.x, d))));
+          }
+          s[j] = d * sc2;
+          mx = fmaxf(mx, d * sc2);
+        };
+        for (int j = lane; j < pos; j += 64) score(kc + kv_elem<PAGED>(c.s, kb, hk, j), j);
+        if (lane <= t) score(qkv + lane * 256 + nq + hk * D, pos + lane);
+        mx = wave_max(mx);
+        wave_lds();
+        float sum = 0.f;
+        for (int j = lane; j <= pos + t; j += 64) { const float e = __builtin_amdgcn_exp2f(s[j] - mx); s[j] = e; sum += e; }
+        sum = wave_sum(sum);
+        wave_lds();
+        float o = 0.f;
+        for (int j = lane / D; j < pos; j += KG) o = fmaf(s[j], vc[kv_elem<PAGED>(c.s, kb, hk, j) + lane % D], o);
+        for (int j = lane / D; j <= t; j += KG) o = fmaf(s[pos + j], qkv[j * 256 + nq + nkv + hk * D + lane % D], o);
+#pragma unroll
+        for (int m = D; m < 64; m <<= 1) o += __shfl_xor(o, m, 64);
+        if (lane < D) ov[t * 128 + h * D + lane] = o / sum;
+        wave_lds();                                   // (s is written again)
+      }
+      lds_barrier();
+      ro.dots(po, ov, 128, n, p1);
+      ro.load(wn + OW, sbn + 2 * NT);
+      lds_barrier();
+      auto add = [&]() {
+#pragma unroll
+        for (int u = 0; u < OWN; ++u)
+          if (wave + NW * u < n && lane < H) x[u] += join<false>(p1 + (wave + NW * u) * NT, lane);
+      };
+      add();
+      norm(n2, RND_NONE);
+      n2 = c.norms[(2 * nl + 1) * H + col];
+      lds_barrier();
+      rg.dots(pg, xn, 64, n, p0);
+      rg.load(wn + GW, sbn + 4 * NT);
+      lds_barrier();
+#pragma unroll
+      for (int u = 0; u < OWN; ++u) {
+        const int t = wave + NW * u;
+        if (t >= n) break;
+        for (int k = lane; k < I; k += 64) {
+          const float g = join<true>(p0 + t * NT, k), up = join<true>(p0 + t * NT, I + k);
+          act[t * 128 + k] = g * (1.0f / (1.0f + expf(-g))) * up;
+        }
+      }
+      lds_barrier();
+      rd.dots(pd, act, 128, n, p1);
+      rd.load(wn + DW, sbn + 6 * NT);
+      lds_barrier();
+      add();
+    }
+#pragma unroll
+    for (int u = 0; u < OWN; ++u)
+      if (wave + NW * u < n && lane < H) c.h[((size_t)b * L + t0 + wave + NW * u) * H + lane] = x[u];
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // these keys and values are the next tokens' cache
+    __syncthreads();
+  }
+  if (tid == 0) c.offsets[kb] = before + L;           // (read at the head, in front of many barriers)
+}
+
 int per_of(int kind) { return kind == SMALL_F32 ? 1 : kind == SMALL_CODES ? 4 : 2; }
 int kind_of(const LinearW& W) { return wk_is_quant(W.wk) ? SMALL_CODES : W.wk == WK_F32 ? SMALL_F32 : W.wk == WK_BF16 ? SMALL_BF16 : SMALL_F16; }
 
@@ -313,8 +514,12 @@ int launch_small_pack(const LinearW& W, bool big, uint32_t* words, float2* sb, h
 }
 
 int launch_stack_small(const SmallStackCall& c, hipStream_t st) {
-  if (!small_stack_shape(c.H, c.s.Hq, c.s.Hkv, c.s.D, c.I) || c.s.act != MI_F32 || c.s.kv != MI_F32 || c.s.L != 1) return fail(MI_ERR_UNSUPPORTED, "stack_small: shape / dtype not supported");
-#define GO(K, DV) do { if (c.s.btab) hipLaunchKernelGGL((stack_small_kernel<K, DV, true>), dim3(c.s.B), dim3(NT), 0, st, c); \
+  if (!small_stack_shape(c.H, c.s.Hq, c.s.Hkv, c.s.D, c.I) || c.s.act != MI_F32 || c.s.kv != MI_F32 || c.s.L < 1) return fail(MI_ERR_UNSUPPORTED, "stack_small: shape / dtype not supported");
+#define GOP(K, DV, PG) do { auto kern = small_prompt_kernel<K, DV, PG>; \
+    MI_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)prompt_lds())); \
+    hipLaunchKernelGGL(kern, dim3(c.s.B), dim3(NT), prompt_lds(), st, c); } while (0)
+#define GO(K, DV) do { if (c.s.L > 1) { if (c.s.btab) GOP(K, DV, true); else GOP(K, DV, false); } \
+    else if (c.s.btab) hipLaunchKernelGGL((stack_small_kernel<K, DV, true>), dim3(c.s.B), dim3(NT), 0, st, c); \
     else hipLaunchKernelGGL((stack_small_kernel<K, DV, false>), dim3(c.s.B), dim3(NT), 0, st, c); } while (0)
 #define GOK(K) do { if (c.s.D == 16) GO(K, 16); else GO(K, 32); } while (0)
   switch (c.kind) {
@@ -326,6 +531,7 @@ int launch_stack_small(const SmallStackCall& c, hipStream_t st) {
   }
 #undef GOK
 #undef GO
+#undef GOP
   MI_HIP(hipGetLastError());
   return MI_OK;
 }

@@ -1340,3 +1340,39 @@ def test_attention_that_leaves_its_rows_prepared_for_the_int4_output_linear(tmp_
             assert np.isfinite(a).all() and np.array_equal(a, b)
     eng.set_option("attention_frag", 1)
     eng.close()
+
+
+@pytest.mark.parametrize("dtype,bits,group", [("float32", 0, 64), ("bfloat16", 0, 64), ("float16", 0, 64), ("bfloat16", 4, 64), ("float32", 4, 32), ("float16", 8, 64)])
+@pytest.mark.parametrize("heads,kv_heads,hd,hidden,ff", [(4, 4, 16, 64, 128), (4, 2, 16, 64, 64), (2, 1, 32, 64, 128), (8, 1, 16, 64, 64)])
+def test_a_small_model_s_prompt_in_one_launch_equals_the_launches_it_replaces(tmp_path, dtype, bits, group, heads, kv_heads, hd, hidden, ff):
+    """Prompts around the kernel's 16 tokens a time, on empty caches and behind cached tokens, both cache forms, a subset of the rows, a decode step behind them,
+    every position's log-probability.  Float32 sums in another order; in the 16-bit models' first layer a rounding may fall the other way (their tests' bound)."""
+    from mlx_parallm_amd.tiny_model import build_tiny_model
+
+    build_tiny_model(tmp_path, seed=5, vocab_size=512, dtype=dtype, quantize_model=bits > 0, q_bits=bits or 4, q_group_size=group, hidden_size=hidden, layers=3, heads=heads,
+                     kv_heads=kv_heads, intermediate_size=ff, head_dim=hd, norm_jitter=0.2, with_tokenizer=False)
+    eng = utils.load_model(str(tmp_path), max_positions=1024).engine
+    rng = np.random.default_rng(3)
+    outs = {}
+    calls = [[rng.integers(0, 512, (3, n)).astype(np.int32) for n in lens] for lens in ((2, 1), (9, 1, 7), (16, 16, 1), (17, 30, 1), (33, 1))]
+    targets = rng.integers(0, 512, (3, 33)).astype(np.int32)
+    for paged in (False, True):
+        for on in (1, 0):
+            eng.set_option("small_stack", on)
+            got = []
+            for parts in calls:
+                kv = eng.new_paged_kv(3, block_tokens=16, max_tokens_per_row=128, kv_dtype="float32") if paged else eng.new_kv(3, capacity=128, kv_dtype="float32")
+                got += [eng.forward(p, kv) for p in parts]
+                eng.step_wait(eng.step_enqueue_rows(kv, [2, 0], parts[0][[2, 0]]), 2)
+                got.append(eng.forward(parts[-1][:, :1], kv))
+                kv.close()
+            kv = eng.new_kv(3, capacity=128, kv_dtype="float32")
+            got.append(eng.score_tokens(kv, calls[-1][0], targets, SampleArgs())["logprobs"])
+            kv.close()
+            outs[paged, on] = got
+        for a, b in zip(outs[paged, 1], outs[paged, 0]):
+            assert np.abs(a - b).max() <= (2e-5 if dtype == "float32" else 4e-3) * max(1.0, np.abs(b).max()), np.abs(a - b).max()
+            assert a.shape == b.shape
+    assert all(np.array_equal(a, b) for a, b in zip(outs[True, 1], outs[False, 1]))
+    eng.set_option("small_stack", 1)
+    eng.close()
