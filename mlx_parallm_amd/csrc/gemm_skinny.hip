@@ -123,8 +123,8 @@ struct SkinnyParams {
 // multiplies x by the weights themselves; the codes here are centred, so that a group's sum is no larger than the one it stands for: with
 // codes from 16 to 31 the result is 4 to 10 times further from 64 bits (and a launch up to 30 % faster: int4, 28672 x 4096, 8 rows, 25 us against 34).
 // CENTRED: codes less MID, the smallest terms of x first.
-template <typename AT, int QB, int MT, bool SWIGLU, bool X32 = false, typename ST = AT, bool CENTRED = !std::is_same<ST, AT>::value>
-__global__ __launch_bounds__(SK_NW * 64, (QB == 4 || (QB == 8 && MT >= 3) || MT >= 5 || (X32 && QB == 8) || (X32 && MT == 2 && SWIGLU)) ? 2 : 4) void skinny_kernel(const SkinnyParams p) {
+template <typename AT, int QB, int MT, bool SWIGLU, bool X32, typename ST, bool CENTRED>
+__device__ __forceinline__ void skinny_body(const SkinnyParams& p) {
   constexpr bool Q4 = QB == 4, Q8 = QB == 8, QUANT = QB != 0;
   static_assert(!X32 || MT <= 2, "float32 activations: 16- and 32-row instantiations");
   using XT = typename std::conditional<X32, float, AT>::type;
@@ -885,6 +885,14 @@ __global__ __launch_bounds__(SK_NW * 64, (QB == 4 || (QB == 8 && MT >= 3) || MT 
   }
   SK_STAMP(7);
 }
+template <typename AT, int QB, int MT, bool SWIGLU, bool X32 = false>
+__global__ __launch_bounds__(SK_NW * 64, (QB == 4 || (QB == 8 && MT >= 3) || MT >= 5 || (X32 && QB == 8) || (X32 && MT == 2 && SWIGLU)) ? 2 : 4) void skinny_kernel(const SkinnyParams p) {
+  skinny_body<AT, QB, MT, SWIGLU, X32, AT, false>(p);
+}
+template <int QB, int MT, bool SWIGLU, typename ST>
+__global__ __launch_bounds__(SK_NW * 64, (QB == 4 || (QB == 8 && MT >= 3) || MT >= 5 || QB == 8 || (MT == 2 && SWIGLU)) ? 2 : 4) void skinny_centred_kernel(const SkinnyParams p) {
+  skinny_body<bf16, QB, MT, SWIGLU, true, ST, true>(p);
+}
 
 // 16-row tiles of activations per workgroup: 1, 2, 3, 4, 6 or 8 (65..96 rows -> 6, 97..128 -> 8)
 int skinny_mt(size_t rows) {
@@ -1165,16 +1173,25 @@ int launch_gemm_skinny(const LinearW& W, const GemvCall& c, size_t rows, hipStre
       MI_HIP(hipGetLastError());
       return MI_OK;
     };
-#define GO32(QBV, ST) do { \
-      if (pl.mt == 1) return sw ? launch32(skinny_kernel<bf16, QBV, 1, true, true, ST>) : launch32(skinny_kernel<bf16, QBV, 1, false, true, ST>); \
-      return sw ? launch32(skinny_kernel<bf16, QBV, 2, true, true, ST>) : launch32(skinny_kernel<bf16, QBV, 2, false, true, ST>); } while (0)
-    if (W.wk == WK_Q4_BF16 && W.centred && !sw)
-      return pl.mt == 1 ? launch32(skinny_kernel<bf16, 4, 1, false, true, bf16, true>) : launch32(skinny_kernel<bf16, 4, 2, false, true, bf16, true>);
-    if (W.wk == WK_Q4_F16) GO32(4, f16);
-    if (W.wk == WK_Q8_F16) GO32(8, f16);
-    if (qb == 4) GO32(4, bf16);
-    if (qb == 8) GO32(8, bf16);
-    GO32(0, bf16);
+#define GO32(KERN) do { \
+      if (pl.mt == 1) return sw ? launch32(KERN(1, true)) : launch32(KERN(1, false)); \
+      return sw ? launch32(KERN(2, true)) : launch32(KERN(2, false)); } while (0)
+#define PLAIN4(MT, SW) skinny_kernel<bf16, 4, MT, SW, true>
+#define PLAIN8(MT, SW) skinny_kernel<bf16, 8, MT, SW, true>
+#define PLAIN0(MT, SW) skinny_kernel<bf16, 0, MT, SW, true>
+#define HALF4(MT, SW) skinny_centred_kernel<4, MT, SW, f16>
+#define HALF8(MT, SW) skinny_centred_kernel<8, MT, SW, f16>
+    if (W.wk == WK_Q4_BF16 && W.centred && !sw) return pl.mt == 1 ? launch32(skinny_centred_kernel<4, 1, false, bf16>) : launch32(skinny_centred_kernel<4, 2, false, bf16>);
+    if (W.wk == WK_Q4_F16) GO32(HALF4);
+    if (W.wk == WK_Q8_F16) GO32(HALF8);
+    if (qb == 4) GO32(PLAIN4);
+    if (qb == 8) GO32(PLAIN8);
+    GO32(PLAIN0);
+#undef PLAIN4
+#undef PLAIN8
+#undef PLAIN0
+#undef HALF4
+#undef HALF8
 #undef GO32
   }
   return c.act == MI_BF16 ? launch_at<bf16>(p, qb, sw, pl.mt, grid, st) : launch_at<f16>(p, qb, sw, pl.mt, grid, st);
