@@ -203,6 +203,7 @@ struct mi_engine {
   // decode steps of a small model in one launch (stack_small.hip); null: not such a model
   void* small_buf = nullptr; uint32_t* small_words = nullptr; float2* small_scales = nullptr; float* small_norms = nullptr;
   int small_kind = 0;
+  bool small_mfma = false;         // the launches instead would run on the matrix cores
   bool opt_small_stack = true;
   // int4 output linears that read their x in fragment order (gemm_q4.hip): the attention leaves it there [128][heads x head_dim]
   void* o_frag = nullptr;

@@ -851,6 +851,8 @@ int make_small_stack(mi_engine* e) {
   if (hipMalloc(&e->small_buf, words * 4 + scales * 8 + norms * 4) != hipSuccess) { (void)hipGetLastError(); e->small_buf = nullptr; return MI_OK; }
   e->small_words = (uint32_t*)e->small_buf; e->small_scales = (float2*)(e->small_words + words); e->small_norms = (float*)(e->small_scales + scales);
   e->small_kind = small_stack_kind(w0);
+  GemvCall prompt; prompt.act = MI_F32; prompt.M = 16; prompt.ldx = d.hidden_size;
+  e->small_mfma = gemm_skinny_supported(w0, prompt, 16);
   uint32_t* w = e->small_words; float2* sb = e->small_scales; float* nw = e->small_norms;
   for (LayerW& l : e->layers) {
     for (FusedLinear* f : {&l.qkv, &l.o, &l.gate_up, &l.down}) {
@@ -862,12 +864,15 @@ int make_small_stack(mi_engine* e) {
   }
   return MI_OK;
 }
-// Prompts: one workgroup a row, so what decides is the chain of one row against the launches, eight rows of the call each.  us by launches / here, eight layers, 4-bit: one row of 2 / 16 / 64 / 128 /
-// 200 tokens 247 / 123, 514 / 290, 1807 / 1130, 3273 / 2695, 4920 / 5004, two rows 296 / 136, 908 / 303, 3264 / 1137, 6184 / 2701, 9479 / 5052; float32 weights one row 227 / 231, 512 / 482,
-// 1702 / 1851, 3287 / 4129, two rows 270 / 240, 926 / 501, 3292 / 1870, 6457 / 4156.  So a prompt alone up to 16 tokens, on codes up to 128, and several of any length.
+// Prompts: one workgroup a row, so what decides is the chain of one row, 16 tokens a time, against the launches: eight rows of the call each where only the generic kernels take the
+// matrices, on the matrix cores else (bf16 weights, int8).  us by launches / here, eight layers, prompts of 2 / 16 / 32 / 64 / 200 tokens:
+//   4-bit   one row 244 / 117, 514 / 232, 905 / 439, 1802 / 904, 4926 / 4386   two rows 281 / 126, 908 / 244, 1809 / 453, 3269 / 925, 9501 / 4387   (float16 weights and scales alike)
+//   float32 one row 230 / 144, 516 / 325, 915 / 622, 1702 / 1262, 5074 / 5396  two rows 272 / 165, 925 / 341, 1711 / 629, 3297 / 1261, 10017 / 5427
+//   bf16    one row 256 / 145, 273 / 264, 335 / 473, 662 / 967                 two rows 280 / 162, 342 / 286, 668 / 502, 643 / 991, 690 / 4581; 32 rows 989 / 478, 993 / 605, 1036 / 817, 1135 / 1305
+//   int8    one row 279 / 130, 292 / 249, 365 / 448, 621 / 913                 two rows 307 / 144, 377 / 256, 632 / 465, 1097 / 937, 911 / 4380; 8 rows 921 / 535 at 32, 961 / 1001 at 64
 bool small_stack_takes(const mi_engine* e, const mi_kv* kv, int act, int B, int L, const int32_t* rows) {
   if (e->small_buf == nullptr || !e->opt_small_stack || e->opt_force_v1 || !e->opt_fused_attn || !e->prof_name.empty() || act != MI_F32 || kv->dtype != MI_F32) return false;
-  if (B == 1 && L > (e->small_kind == SMALL_CODES ? 128 : 16)) return false;
+  if (L > (e->small_mfma ? (B == 1 ? 16 : 32) : B == 1 ? 128 : SMALL_MAX_KEYS)) return false;
   for (int b = 0; b < B; ++b) if (kv->h_off[rows ? rows[b] : b] + L > SMALL_MAX_KEYS) return false;
   return true;
 }

@@ -89,7 +89,7 @@ struct Regs {
     const float* xk = x + p.w0 * PER;
 #pragma unroll
     for (int i = 0; i < MW; ++i) {
-      if (i >= cnt) break;                            // (uniform)
+      if (i < cnt) {                                  // (uniform; a break keeps longer loops rolled, the words in scratch)
       float& a = acc[i & 1];
       if constexpr (KIND == SMALL_F32) a = fmaf(__uint_as_float(w[i]), xk[i], a);
       else if constexpr (KIND == SMALL_BF16) a = fmaf(bf16hi(w[i]), xk[2 * i + 1], fmaf(bf16lo(w[i]), xk[2 * i], a));
@@ -104,22 +104,23 @@ struct Regs {
         a = fmaf(mul_add_unfused((float)((w[i] >> 16) & 255u), sx, sy), xv.z, a);
         a = fmaf(mul_add_unfused((float)(w[i] >> 24), sx, sy), xv.w, a);
       }
+      }
     }
     return acc[0] + acc[1];
   }
-  // The same for TG rows x[t][ld] a time of n: a weight is multiplied out once for all of them.  out: [n][NT]
-  static constexpr int TG = 8;
-  __device__ __forceinline__ void dots(const Part& p, const float* x, int ld, int n, float* out) const {
-    for (int t0 = 0; t0 < n; t0 += TG) {
-      float acc[TG];
-      int cnt = p.cnt, cut = p.cut, m = min(n - t0, TG);
-      asm volatile("" : "+s"(cnt), "+s"(cut), "+s"(m));
-      const float* xk = x + t0 * ld + p.w0 * PER;
+  // The same for n rows x[t][LD], eight or four a time: a weight is multiplied out once for all of them.  Rows behind the n-th are read (the arrays have PT of
+  // them) and their sums dropped: a condition per row and word costs more.  out: [n][NT]
+  template <int M, int LD>
+  __device__ __forceinline__ void some(const Part& p, const float* x, int m, float* out) const {
+    float acc[M];
+    int cnt = p.cnt, cut = p.cut;
+    asm volatile("" : "+s"(cnt), "+s"(cut));
+    const float* xk = x + p.w0 * PER;
 #pragma unroll
-      for (int t = 0; t < TG; ++t) acc[t] = 0.f;
+    for (int t = 0; t < M; ++t) acc[t] = 0.f;
 #pragma unroll
-      for (int i = 0; i < MW; ++i) {
-        if (i >= cnt) break;
+    for (int i = 0; i < MW; ++i) {
+      if (i < cnt) {
         float v[PER];
         if constexpr (KIND == SMALL_F32) v[0] = __uint_as_float(w[i]);
         else if constexpr (KIND == SMALL_BF16) { v[0] = bf16lo(w[i]); v[1] = bf16hi(w[i]); }
@@ -130,9 +131,8 @@ struct Regs {
           for (int j = 0; j < 4; ++j) v[j] = mul_add_unfused((float)((w[i] >> (8 * j)) & 255u), sx, sy);
         }
 #pragma unroll
-        for (int t = 0; t < TG; ++t) {
-          if (t >= m) break;
-          const float* xt = xk + t * ld + PER * i;
+        for (int t = 0; t < M; ++t) {
+          const float* xt = xk + t * LD + PER * i;
           if constexpr (PER == 4) {
             const float4 q = *(const float4*)xt;
             acc[t] = fmaf(v[3], q.w, fmaf(v[2], q.z, fmaf(v[1], q.y, fmaf(v[0], q.x, acc[t]))));
@@ -142,9 +142,16 @@ struct Regs {
           }
         }
       }
+    }
 #pragma unroll
-      for (int t = 0; t < TG; ++t)
-        if (t < m) out[(t0 + t) * NT + threadIdx.x] = acc[t];
+    for (int t = 0; t < M; ++t)
+      if (t < m) out[t * NT + threadIdx.x] = acc[t];
+  }
+  template <int LD>
+  __device__ __forceinline__ void dots(const Part& p, const float* x, int n, float* out) const {
+    for (int t = 0; t < n; t += 8) {
+      if (n - t > 4) some<8, LD>(p, x + t * LD, n - t, out + t * NT);
+      else some<4, LD>(p, x + t * LD, n - t, out + t * NT);
     }
   }
 };
@@ -175,7 +182,8 @@ __device__ __forceinline__ void lds_barrier() {
 // stands only between a matrix's partial sums (two buffers in turn) and what joins them, and behind the heads.  A wave has whole heads: keys over its lanes.
 template <int KIND, int D, bool PAGED>
 __global__ __launch_bounds__(NT) void stack_small_kernel(SmallStackCall c) {
-  constexpr int PER = Kind<KIND>::PER, NW = NT / 64, NV = 8, KG = 64 / D;
+  constexpr bool AHEAD = KIND != SMALL_F32 || D == 16;           // a layer's cached keys and values asked for at its start (float32 words leave no registers for heads of 32)
+  constexpr int PER = Kind<KIND>::PER, NW = NT / 64, NV = AHEAD ? 8 : 0, KG = 64 / D;
   constexpr float LOG2E = 1.4426950408889634f;
   __shared__ __attribute__((aligned(16))) float xn[64], p0[NT], p1[NT], qk[256], vn[128], ov[128], act[128];
   __shared__ float sc[NW][SMALL_MAX_KEYS];
@@ -216,8 +224,8 @@ __global__ __launch_bounds__(NT) void stack_small_kernel(SmallStackCall c) {
     // cached keys and values of this wave's first head: key `lane`, value column lane % D of keys lane / D + KG i
     const int last = max(pos - 1, 0);
     float4 kr[D / 4];
-    float vr[NV];
-    {
+    float vr[NV + 1];
+    if constexpr (AHEAD) {
       const float4* src = (const float4*)(kc + kv_elem<PAGED>(c.s, kb, h0, min(lane, last)));
 #pragma unroll
       for (int e = 0; e < D / 4; ++e) kr[e] = src[e];
@@ -261,7 +269,7 @@ __global__ __launch_bounds__(NT) void stack_small_kernel(SmallStackCall c) {
       };
       for (int j = lane; j <= pos; j += 64) {
         float d;
-        if (h == wave && j < 64) d = dot_key(kr);     // (uniform: h and the trip)
+        if (AHEAD && h == wave && j < 64) d = dot_key(kr);       // (uniform: h and the trip)
         else {
           float4 k[D / 4];
           const float4* src = (const float4*)(kc + kv_elem<PAGED>(c.s, kb, hk, min(j, last)));
@@ -285,7 +293,7 @@ __global__ __launch_bounds__(NT) void stack_small_kernel(SmallStackCall c) {
       wave_lds();
       float o = 0.f;
       const float v1 = vn[hk * D + lane % D];
-      if (h == wave) {
+      if (AHEAD && h == wave) {
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
           const int j = lane / D + KG * i;
@@ -330,7 +338,7 @@ __global__ __launch_bounds__(NT) void stack_small_kernel(SmallStackCall c) {
 
 // The prompt of a small model, all layers in one launch: a workgroup a row again, PT tokens a time through all layers (their keys and values are the next ones' cache).
 // A wave owns every NW-th token (its columns over the lanes, residual, norm, rotation, gated unit) and takes whole (token, head)s of the attention; the matrices are
-// multiplied by all threads, PT rows a time.  Nine tokens of two rows, eight layers, 4-bit, with the logits: 642 us -> 220, 64 rows of them 14.3 -> 1.06 ms.
+// multiplied by all threads, PT rows a time.  Nine tokens of two rows, eight layers, 4-bit, with the logits: 643 us -> 196, 32 rows of them 7.3 -> 0.6 ms.
 constexpr int PT = 16;
 constexpr size_t prompt_lds() { return (size_t)(PT * (64 + 2 * NT + 256 + 2 * 128) + NT / 64 * SMALL_MAX_KEYS) * 4; }
 template <int KIND, int D, bool PAGED>
@@ -391,7 +399,7 @@ __global__ __launch_bounds__(NT) void small_prompt_kernel(SmallStackCall c) {
       norm(n1, rnd);
       n1 = c.norms[2 * nl * H + col];
       lds_barrier();
-      rq.dots(pq, xn, 64, n, p0);
+      rq.template dots<64>(pq, xn, n, p0);
       rq.load(wn, sbn);
       lds_barrier();
 #pragma unroll
@@ -450,7 +458,7 @@ __global__ __launch_bounds__(NT) void small_prompt_kernel(SmallStackCall c) {
         wave_lds();                                   // (s is written again)
       }
       lds_barrier();
-      ro.dots(po, ov, 128, n, p1);
+      ro.template dots<128>(po, ov, n, p1);
       ro.load(wn + OW, sbn + 2 * NT);
       lds_barrier();
       auto add = [&]() {
@@ -462,7 +470,7 @@ __global__ __launch_bounds__(NT) void small_prompt_kernel(SmallStackCall c) {
       norm(n2, RND_NONE);
       n2 = c.norms[(2 * nl + 1) * H + col];
       lds_barrier();
-      rg.dots(pg, xn, 64, n, p0);
+      rg.template dots<64>(pg, xn, n, p0);
       rg.load(wn + GW, sbn + 4 * NT);
       lds_barrier();
 #pragma unroll
@@ -475,7 +483,7 @@ __global__ __launch_bounds__(NT) void small_prompt_kernel(SmallStackCall c) {
         }
       }
       lds_barrier();
-      rd.dots(pd, act, 128, n, p1);
+      rd.template dots<128>(pd, act, n, p1);
       rd.load(wn + DW, sbn + 6 * NT);
       lds_barrier();
       add();
