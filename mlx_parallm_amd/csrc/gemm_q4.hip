@@ -5,7 +5,7 @@
 // What bounds this size is the arithmetic around the weights: per 16 columns, 64 k and 64 rows 8 matrix instructions (128 cycles), 16 unpacking
 // and 16 scaling instructions (128 cycles), and they overlap only in part.  So:
 //   * a workgroup is 8 waves = 2 column halves x 4 K lanes, one workgroup per CU: every SIMD has two waves with the same work.  A wave carries
-//     TN = 5 column tiles (SwiGLU: the same 5 gate or up tiles), so that a fragment of x that it reads from LDS feeds 5 tiles, and every 4th
+//     TN = 4 or 5 column tiles (SwiGLU: the same gate or up tiles), so that a fragment of x that it reads from LDS feeds as many tiles, and every 4th
 //     block of 128 k.  Nothing but x is shared, between the two halves.
 //   * x and weights come by LDS-DMA: no staging registers, no loads in inline asm that the compiler could mistake for done.  x is prepared once
 //     per launch (q4_prep_kernel): fragment order, nibble order, RMSNorm, sums per group.  A wave's weights of block i + 1 arrive while block i
@@ -35,13 +35,10 @@ namespace {
 
 using namespace gemv;
 
-// Five tiles: the most whose accumulators and biases fit 256 registers, and for wide matrices the fewest rounds of workgroups (34816 x 5120 SwiGLU 218
-// workgroups, four tiles 272: two rounds).  Where both fit one round, four are faster, 180 against 224 of 256 CUs at 28672 x 4096: us at 32 / 64 / 128 rows,
-// five and four tiles, 28672 x 4096 26.6 / 34.6 / 63.6 and 24.9 / 30.4 / 54.0, 34816 x 5120 32.5 / 40.6 / 74.2 and 50.1 / 63.2 / 92.9, 151936 x 5120 138 /
-// 174 / 308 and 138 / 183 / 340, 16384 x 4096 22.9 / 30.7 / 35.0 and 21.4 / 27.7 / 31.3, 19200 x 3072 21.2 / 28.5 / 30.4 and 19.9 / 25.5 / 45.7.  A choice
-// per call has not been built.
-constexpr int TN = 5, TW = 2, KW = 4, NW = TW * KW, RT = 2;       // (RT: column tiles of a workgroup of q4_rows_kernel)
-constexpr int W_SLOT = TN * (1024 + 128);                       // codes of five tiles, then their scales | biases (64 + 64 bytes)
+// Five column tiles a wave: the most whose accumulators and biases fit 256 registers, and for wide matrices the fewest rounds of workgroups (34816 x 5120 SwiGLU 218
+// workgroups, four tiles 272: two rounds).  Where four take no more rounds a workgroup has less to do (28672 x 4096: 224 of 256 CUs instead of 180): q4_tiles.
+constexpr int TW = 2, KW = 4, NW = TW * KW, RT = 2;       // (RT: column tiles of a workgroup of q4_rows_kernel)
+constexpr int w_slot(int tn) { return tn * (1024 + 128); }       // codes of the tiles, then their scales | biases (64 + 64 bytes)
 constexpr int Q4_LDS = 160 * 1024;
 
 struct Q4Params {
@@ -170,8 +167,9 @@ typedef __attribute__((address_space(3))) unsigned char lds_byte;
 template <typename T> using lds_ptr = __attribute__((address_space(3))) const T*;
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-template <typename AT, int MT, bool SWIGLU>
+template <typename AT, int MT, bool SWIGLU, int TN>
 __global__ __launch_bounds__(512, 2) void q4_kernel(const Q4Params p) {
+  constexpr int W_SLOT = w_slot(TN);
   constexpr int MB = 16 * MT, X_HALF = MT * 1024, X_BUF = KW * 2 * X_HALF, X_DMAS = MT, W_DMAS = TN + 1;
   constexpr bool OFFS = std::is_same<AT, bf16>::value;          // (f16: the codes are unpacked without an offset)
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -727,10 +725,10 @@ __global__ __launch_bounds__(512, 2) void q4_rows_kernel(const Q4Params p) {
   }
 }
 
-struct Q4Plan { bool rows; int mt, nslab, ksplit, ntu, ntiles, ngroups, nblk; size_t xq_bytes, sx_bytes, sxo_bytes, ws_bytes; };
+struct Q4Plan { bool rows; int tn, mt, nslab, ksplit, ntu, ntiles, ngroups, nblk; size_t xq_bytes, sx_bytes, sxo_bytes, ws_bytes; };
 
 thread_local int q4_force_mt = 0, q4_force_ks = 0;               // test hook: row tiles per workgroup, K slices (0: the plan's own)
-thread_local int q4_force_rows = 0;
+thread_local int q4_force_rows = 0, q4_force_tn = 0;
 thread_local bool q4_forced = false;                             // .. and whatever the width
 
 // Narrow matrices: q4_rows_kernel or gemm_skinny.hip?  us, both with their preparation but without the norm launch of 4.7 that q4_prep_kernel saves, warm weights,
@@ -747,13 +745,27 @@ bool q4_rows_ahead(const LinearW& W, const GemvCall& c, size_t rows) {
 }
 bool q4_rows(const LinearW& W, const GemvCall& c) { return q4_force_rows > 0 || (!q4_forced && W.N / 16 < GEMM_Q4_MIN_TILES); }
 
+// Column tiles a wave where K is not split (a column's sum is the same whatever it shares a wave with): four where their rounds of workgroups, each some 7/8 of one of five
+// tiles, cost less.  us at 32 / 64 / 128 rows, five and four tiles: SwiGLU 28672 x 4096 25.5 / 32.5 / 61.5 and 23.3 / 28.6 / 52.4, 16384 x 4096 23.1 / 32.2 / 33.6 and
+// 20.7 / 27.8 / 29.9, 44032 x 4096 46.8 / 61.4 / 91.7 and 40.2 / 51.8 / 79.2, logits 32000 x 4096 26.1 / 34.8 / 64.7 and 24.7 / 31.8 / 58.5, 128256 x 4096 100 / 136 / 228.5 and
+// 92 / 124 / 227.1; a round more: SwiGLU 34816 x 5120 30.0 / 39.1 / 74.7 and 47.3 / 60.9 / 90.5, 19200 x 3072 at 128 rows 28.5 and 43.7, logits 151936 x 5120 128 / 169 / 309 and
+// 135 / 174 / 323, 50304 x 3072 at 128 rows 81.3 and 90.5.
+int q4_tiles(long groups4, long groups5) {
+  if (q4_force_tn == 4 || q4_force_tn == 5) return q4_force_tn;
+  const long cus = gemv_cu_count(), r4 = (groups4 + cus - 1) / cus, r5 = (groups5 + cus - 1) / cus;
+  return 7 * r4 < 8 * r5 ? 4 : 5;
+}
+
 Q4Plan q4_plan(const LinearW& W, const GemvCall& c, size_t rows) {
   Q4Plan pl{};
   const bool sw = c.epi == EPI_SWIGLU;
   pl.ntiles = W.N / 16;
   pl.ntu = sw ? c.pair_offset / 16 : pl.ntiles;
   pl.nblk = W.K / 128;
-  pl.ngroups = sw ? (pl.ntu + TN - 1) / TN : (pl.ntiles + TW * TN - 1) / (TW * TN);
+  constexpr int TN = 5;
+  const auto groups_of = [&](int tn) { return sw ? (pl.ntu + tn - 1) / tn : (pl.ntiles + TW * tn - 1) / (TW * tn); };
+  pl.tn = TN;
+  pl.ngroups = groups_of(TN);
   const int tiles = (int)((rows + 15) / 16);
   pl.nslab = (tiles + 3) / 4;
   pl.mt = std::max(2, (tiles + pl.nslab - 1) / pl.nslab);
@@ -768,6 +780,7 @@ Q4Plan q4_plan(const LinearW& W, const GemvCall& c, size_t rows) {
     if (ks > 1) t += 2.0 + 2.0 * ks * (double)pl.ngroups * TW * TN * pl.nslab * pl.mt * 1024 / 4.0e6;
     if (q4_force_ks > 0 ? ks == std::min(q4_force_ks, pl.nblk) : t < best) { best = t; pl.ksplit = ks; }
   }
+  if (!pl.rows && pl.ksplit == 1 && q4_tiles(groups_of(4) * pl.nslab, pl.ngroups * pl.nslab) == 4) { pl.tn = 4; pl.ngroups = groups_of(4); }
   const size_t G = W.K / 64;
   pl.xq_bytes = (size_t)pl.nslab * G * 2 * pl.mt * 1024;
   pl.sx_bytes = pl.rows ? 0 : (pl.nslab * G * 16 * pl.mt * sizeof(float) + 255) & ~(size_t)255;
@@ -776,9 +789,9 @@ Q4Plan q4_plan(const LinearW& W, const GemvCall& c, size_t rows) {
   return pl;
 }
 
-template <typename AT, int MT, bool SW>
+template <typename AT, int MT, bool SW, int TN>
 int q4_launch_k(const Q4Params& p, int grid, hipStream_t st) {
-  auto kern = q4_kernel<AT, MT, SW>;
+  auto kern = q4_kernel<AT, MT, SW, TN>;
   static std::atomic<bool> attr_done[64];
   int dev = 0;
   MI_HIP(hipGetDevice(&dev));
@@ -791,12 +804,12 @@ int q4_launch_k(const Q4Params& p, int grid, hipStream_t st) {
   return MI_OK;
 }
 
-template <typename AT>
+template <typename AT, int TN>
 int q4_launch_at(const Q4Params& p, int mt, bool sw, int grid, hipStream_t st) {
   switch (mt) {
-    case 2: return sw ? q4_launch_k<AT, 2, true>(p, grid, st) : q4_launch_k<AT, 2, false>(p, grid, st);
-    case 3: return sw ? q4_launch_k<AT, 3, true>(p, grid, st) : q4_launch_k<AT, 3, false>(p, grid, st);
-    case 4: return sw ? q4_launch_k<AT, 4, true>(p, grid, st) : q4_launch_k<AT, 4, false>(p, grid, st);
+    case 2: return sw ? q4_launch_k<AT, 2, true, TN>(p, grid, st) : q4_launch_k<AT, 2, false, TN>(p, grid, st);
+    case 3: return sw ? q4_launch_k<AT, 3, true, TN>(p, grid, st) : q4_launch_k<AT, 3, false, TN>(p, grid, st);
+    case 4: return sw ? q4_launch_k<AT, 4, true, TN>(p, grid, st) : q4_launch_k<AT, 4, false, TN>(p, grid, st);
   }
   return fail(MI_ERR_INVALID, "gemm_q4: 2..4 row tiles per workgroup");
 }
@@ -816,8 +829,8 @@ int q4_rows_launch(const Q4Params& p, int mt, bool sw, int grid, hipStream_t st)
 
 }  // namespace
 
-// test hook: row tiles | .. << 3 | .. << 7 | K slices << 11 (the fields between are q4_kernel's fixed shape) | q4_rows_kernel << 15; 0 clears
-void gemm_q4_force(int code) { q4_force_mt = code & 7; q4_force_ks = (code >> 11) & 15; q4_force_rows = (code >> 15) & 1; q4_forced = code != 0; }
+// test hook: row tiles | .. << 3 | column tiles a wave << 7 (K not split; the field between is q4_kernel's fixed shape) | K slices << 11 | q4_rows_kernel << 15; 0 clears
+void gemm_q4_force(int code) { q4_force_mt = code & 7; q4_force_tn = (code >> 7) & 15; q4_force_ks = (code >> 11) & 15; q4_force_rows = (code >> 15) & 1; q4_forced = code != 0; }
 
 // The wide matrices, and the narrow ones of q4_rows_ahead.  Wide: us, 64 rows (32 rows), against gemm_skinny.hip's K over workgroups; with the preparation pass, which replaces a norm launch of
 // 4.7 us in front of gate|up and the logits: 34816 x 5120 SwiGLU 42 (31) against 71 (40), 28672 x 4096 33 (25) against 40 (25), 151936 x 5120
@@ -877,7 +890,9 @@ int launch_gemm_q4(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t
     return c.act == MI_BF16 ? q4_rows_launch<bf16>(p, pl.mt, c.epi == EPI_SWIGLU, grid, st) : q4_rows_launch<f16>(p, pl.mt, c.epi == EPI_SWIGLU, grid, st);
   }
   const int blocks = pl.nslab > 1 ? (p.nunits + 7) / 8 * 8 * pl.nslab : p.nunits;
-  return c.act == MI_BF16 ? q4_launch_at<bf16>(p, pl.mt, c.epi == EPI_SWIGLU, blocks, st) : q4_launch_at<f16>(p, pl.mt, c.epi == EPI_SWIGLU, blocks, st);
+  const bool sw = c.epi == EPI_SWIGLU;
+  if (pl.tn == 4) return c.act == MI_BF16 ? q4_launch_at<bf16, 4>(p, pl.mt, sw, blocks, st) : q4_launch_at<f16, 4>(p, pl.mt, sw, blocks, st);
+  return c.act == MI_BF16 ? q4_launch_at<bf16, 5>(p, pl.mt, sw, blocks, st) : q4_launch_at<f16, 5>(p, pl.mt, sw, blocks, st);
 }
 
 }  // namespace mi

@@ -100,10 +100,10 @@ def close_frac(got: np.ndarray, want: np.ndarray, dtype: str, atol: float = 0.0)
     return float(np.mean(np.abs(got - want) > tol))
 
 
-def q4_force(mt=0, ksplit=0, rows=0) -> int:
+def q4_force(mt=0, ksplit=0, rows=0, tn=0) -> int:
     """`ksplit` argument of gemm_skinny() that forces gemm_q4.hip and its plan (include/mi355_ops.h): row tiles per workgroup, K slices over
-    workgroups; 0 = the cost model's choice; rows = 1: the kernel for narrow matrices."""
-    return -(mt | ksplit << 11 | rows << 15)
+    workgroups; 0 = the cost model's choice; rows = 1: the kernel for narrow matrices; tn: column tiles a wave where K is not split."""
+    return -(mt | tn << 7 | ksplit << 11 | rows << 15)
 
 
 def gemm_skinny(ol: L.OpLinear, x, M, act, *, epi=0, out=None, ldo=0, resid=None, pair_offset=0, ksplit=0, iters=0, ldx=None,

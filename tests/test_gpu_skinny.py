@@ -165,6 +165,26 @@ def test_q4_norm_prologue_and_epilogues(act, kind, mt, ks):
         assert np.all(host(out)[M] == 7.0)
 
 
+@pytest.mark.parametrize("act,kind", [("bfloat16", "q4_bf16"), ("float16", "q4_f16")])
+@pytest.mark.parametrize("mt", [2, 3, 4])
+def test_q4_four_and_five_column_tiles_a_wave_make_the_same_bits(act, kind, mt):
+    """Both against the oracle, with column tiles that fill no group of either."""
+    for M, N, K in [(16 * mt - 5, 16 * 11, 640), (16 * mt, 16 * 46, 1152), (32 * mt - 1, 16 * 40, 128 * 35)]:
+        ol, wdense, keep = _weight(kind, N, K, RNG_Q4)
+        x = round_to(RNG_Q4.standard_normal((M, K)).astype(np.float32), act)
+        xd, I = dev(x, act), 16 * (N // 32)
+        outs = {}
+        for tn in (4, 5):
+            out, sw = torch.full((M + 1, N), 7.0, dtype=xd.dtype, device="cuda"), torch.full((M + 1, I), 7.0, dtype=xd.dtype, device="cuda")
+            gemm_skinny(ol, xd, M, act, epi=L.EPI_STORE, out=out, ldo=N, ksplit=q4_force(mt, 1, tn=tn))
+            if N == 2 * I:
+                gemm_skinny(ol, xd, M, act, epi=L.EPI_SWIGLU, out=sw, ldo=I, pair_offset=I, ksplit=q4_force(mt, 1, tn=tn))
+            outs[tn] = host(out), host(sw)
+        for a, b in zip(outs[4], outs[5]):
+            assert np.array_equal(a, b) and np.all(a[M] == 7.0)
+        _assert_close(outs[4][0][:M], round_to(matmul_nt(x, wdense), act), act)
+
+
 def test_rows_agree_with_the_16_row_kernel():
     """The same rows through gemv_mfma.hip (<= 16 rows per launch): equal up to the rounding of differently ordered
     float32 sums."""
