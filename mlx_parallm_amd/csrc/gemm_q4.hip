@@ -736,12 +736,13 @@ thread_local bool q4_forced = false;                             // .. and whate
 // 16 / 24, 19 / 29; 8192 x 8192 15 / 22, 21 / 30, 38 / 45; 4096 x 10240 15 / 19, 22 / 29, 26 / 35; 4096 x 12288 17 / 22, 25 / 29, 29 / 38.  More than one round of workgroups: 5120 x 10240
 // at 65 rows 36 / 33, 128 43 / 41; with a norm (to be added to the other side) or a SwiGLU 10240 x 5120 16 / 17, 25 / 25, 36 / 45; 10240 x 8192 22 / 22, 35 / 34, 51 / 59; 16128 x 8192
 // 23 / 27, 36 / 44, 68 / 72; 16128 x 4096 15 / 18, 23 / 28, 41 / 38 (four rounds: behind by less than the norm); SwiGLU 14336 x 4096 15 / 19, 22 / 30, 39 / 41, 16128 x 8192 23 / 28, 36 / 43, 67 / 68.
-// A longer K: 4096 x 14336 26 / 23, 41 / 33, 43 / 45; 5120 x 17408 32 / 28, 50 / 40, 87 / 62.  So: K up to 8192 (to 12288 it would still be the faster one), and one round of workgroups,
-// or any number where a norm launch goes with the other kernel.  A short K without a norm: the preparation is a launch of its own, 256 x 128 5.5 / 4.9, 6.0 / 5.4, 6.1 / 5.4;
+// A longer K, one round: 4096 x 10240 15 / 19, 22 / 28, 27 / 35; 3072 x 11008 16 / 19, 24 / 27, 26 / 33; 4096 x 14336 20 / 22, 29 / 33, 35 / 43; 5120 x 17408 22 / 26, 34 / 40, in two rounds at
+// 128 rows 67 / 62.  So: one round of workgroups whatever K, and up to K = 8192 any number where a norm launch goes with the other kernel. A short K without a norm: the preparation is a launch of its own, 256 x 128 5.5 / 4.9, 6.0 / 5.4, 6.1 / 5.4;
 // 512 x 256 5.8 / 5.7, 6.2 / 5.8, 6.3 / 5.8; 1024 x 512 6.0 / 6.5, 6.6 / 6.6, 6.7 / 6.7.  So from K = 512.
 bool q4_rows_ahead(const LinearW& W, const GemvCall& c, size_t rows) {
   const long units = c.epi == EPI_SWIGLU ? c.pair_offset / 16 : (W.N / 16 + RT - 1) / RT, slabs = (long)((rows + 63) / 64);
-  return W.K <= 8192 && (c.pro == PRO_NORM || W.K >= 512) && (c.pro == PRO_NORM || c.epi == EPI_SWIGLU || units * slabs <= gemv_cu_count());
+  const bool one = units * slabs <= gemv_cu_count();
+  return (W.K <= 8192 || one) && (c.pro == PRO_NORM || (W.K >= 512 && (c.epi == EPI_SWIGLU || one)));
 }
 bool q4_rows(const LinearW& W, const GemvCall& c) { return q4_force_rows > 0 || (!q4_forced && W.N / 16 < GEMM_Q4_MIN_TILES); }
 

@@ -185,6 +185,21 @@ def test_q4_four_and_five_column_tiles_a_wave_make_the_same_bits(act, kind, mt):
         _assert_close(outs[4][0][:M], round_to(matmul_nt(x, wdense), act), act)
 
 
+@pytest.mark.parametrize("act,kind", [("bfloat16", "q4_bf16"), ("float16", "q4_f16")])
+@pytest.mark.parametrize("M", [17, 61, 128])
+def test_q4_narrow_matrices_of_a_long_k_match_oracle(act, kind, M):
+    """The down projections' form: a residual behind K blocks that do and do not divide by the eight waves, an odd number of column tiles."""
+    for N, K in ((80, 128 * 67), (144, 128 * 136)):
+        ol, wdense, keep = _weight(kind, N, K, RNG_Q4)
+        x = round_to(RNG_Q4.standard_normal((M, K)).astype(np.float32) * 0.5, act)
+        h = round_to(RNG_Q4.standard_normal((M + 1, N)).astype(np.float32), act)
+        xd, hd = dev(x, act), dev(h, act)
+        used, _ = gemm_skinny(ol, xd, M, act, epi=L.EPI_RESID, resid=hd, ldo=N)
+        assert used == 1                                          # (q4_rows_kernel: the other one cuts such a K)
+        _assert_close(host(hd)[:M], round_to(h[:M] + round_to(matmul_nt(x, wdense), act), act), act, scale=4.0)
+        assert np.array_equal(host(hd)[M], h[M])
+
+
 def test_rows_agree_with_the_16_row_kernel():
     """The same rows through gemv_mfma.hip (<= 16 rows per launch): equal up to the rounding of differently ordered
     float32 sums."""
