@@ -794,17 +794,30 @@ int choose_nsplit(const mi_kv* kv, int B, int Hkv, int L, const int32_t* rows = 
   return ns_env > 0 ? decode_row_splits(std::min(ns_env, 16), mx) : attention_decode_splits(gemv_cu_count(), Hkv * alike, mx, kv->dtype == MI_F32);
 }
 
-// Does the attention in front of the output linear `co` of `rows` rows leave its rows as gemm_q4.hip multiplies them, instead of a preparation launch (4.8 us)?  -> the
-// row tiles a slab, 0: no.  Where gemv_rows would have that kernel prepare them; an adapter reads the rows as they are.  Whole calls, decode steps of 24 rows x 705 keys (4096 wide) 6.23 -> 6.11 ms,
-// 64 x 513 (5120) 17.19 -> 16.97, 100 x 257 11.77 -> 11.74; 31 rows and 32 tokens mixed 6.67 -> 6.57.
+// Does a linear of `rows` rows take its x from the launch in front as gemm_q4.hip multiplies it, instead of by a preparation launch (4.8 us)?  -> the row tiles a slab, 0: no.
+// Where gemv_rows would have that kernel prepare it; an adapter reads the rows as they are.
+int frag_mt(const mi_engine* e, const FusedLinear& f, const GemvCall& c, size_t rows) {
+  if (!e->opt_attn_frag || !e->opt_skinny_gemm || e->opt_force_v1 || c.act == MI_F32 || rows < 17 || rows > 128) return 0;
+  if ((e->cur_L != 1 && !e->opt_short_prefill_skinny) || f.W.lora_b[0] != nullptr || f.W.lora_b[1] != nullptr || getenv("MI_SKINNY_DECODE_MAX") != nullptr) return 0;
+  return gemm_skinny_supported(f.W, c, rows) ? gemm_q4_frag_mt(f.W, c, rows) : 0;
+}
+bool frag_buffer(mi_engine* e, void** p, int K) {
+  if (*p == nullptr && dev_malloc(e, p, (size_t)128 * K * 2) != hipSuccess) { (void)hipGetLastError(); *p = nullptr; }
+  return *p != nullptr;
+}
+// The attention in front of the output linear `co`.  Whole calls, decode steps of 24 rows x 705 keys (4096 wide) 6.23 -> 6.11 ms, 64 x 513 (5120) 17.19 -> 16.97, 100 x 257 11.77 -> 11.74;
+// 31 rows and 32 tokens mixed 6.67 -> 6.57.
 int o_frag_mt(mi_engine* e, const FusedLinear& o, const GemvCall& co, size_t rows) {
-  if (!e->opt_attn_frag || !e->opt_skinny_gemm || !e->opt_attn_mfma || !e->opt_fused_attn || e->opt_force_v1 || co.act == MI_F32 || rows < 17 || rows > 128) return 0;
-  if ((e->cur_L != 1 && !e->opt_short_prefill_skinny) || o.W.lora_b[0] != nullptr || o.W.lora_b[1] != nullptr || getenv("MI_SKINNY_DECODE_MAX") != nullptr) return 0;
-  if (!gemm_skinny_supported(o.W, co, rows)) return 0;
-  const int mt = gemm_q4_frag_mt(o.W, co, rows);
-  if (mt == 0) return 0;
-  if (e->o_frag == nullptr && dev_malloc(e, &e->o_frag, (size_t)128 * o.W.K * 2) != hipSuccess) { (void)hipGetLastError(); e->o_frag = nullptr; return 0; }
-  return mt;
+  const int mt = e->opt_attn_mfma && e->opt_fused_attn ? frag_mt(e, o, co, rows) : 0;
+  return mt > 0 && frag_buffer(e, &e->o_frag, o.W.K) ? mt : 0;
+}
+// gate|up in front of the down projection `cd`: the same kernel's SwiGLU.  With the output linear's, 24 x 705 5.90 -> 5.63 ms, 64 x 513 17.12 -> 16.70, 100 x 257 (4096) 9.52 -> 9.28, mixed 6.62 -> 6.50.
+void act_frag(mi_engine* e, const LayerW& lw, GemvCall& cg, GemvCall& cd, size_t rows) {
+  const int mt = frag_mt(e, lw.down, cd, rows);
+  if (mt == 0 || lw.gate_up.W.lora_b[0] != nullptr || lw.gate_up.W.lora_b[1] != nullptr || !gemm_skinny_supported(lw.gate_up.W, cg, rows) || !gemm_q4_supported(lw.gate_up.W, cg, rows)) return;
+  if (!frag_buffer(e, &e->act_frag, lw.down.W.K)) return;
+  cg.out = e->act_frag; cg.out_frag = mt;
+  cd.x = e->act_frag; cd.x_frag = mt;
 }
 
 // prefill attention (L > 1): the keys split over workgroups where the query tiles alone leave the chip idle
@@ -992,11 +1005,13 @@ int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool wan
         }
         MI_TRY(launch_attention(ac, st)); }
     }
+    GemvCall cdn; cdn.x = e->act; cdn.ldx = I; cdn.act = act; cdn.rnd = RND_NONE; cdn.epi = EPI_RESID; cdn.resid = e->h; cdn.ldo = H;
     {
       // post_attention_layernorm + gate|up + SwiGLU (llama.py:189,165)
       GemvCall cg; cg.x = e->h; cg.ldx = H; cg.act = act; cg.rnd = RND_NONE; cg.pro = PRO_NORM; cg.norm_w = post_norm;
       cg.eps = d.rms_norm_eps; cg.epi = EPI_SWIGLU; cg.out = e->act; cg.ldo = I; cg.pair_offset = I;
       cg.split_out = down_takes_split(e, lw.down, act, R);
+      act_frag(e, lw, cg, cdn, R);
       if ((e->opt_fused_pairs & 1) && can_pair(e, lw.o, co, lw.gate_up, cg, R)) {
         MI_TRY(gemv_pair(e, lw.o, co, lw.gate_up, cg, R, "gemv_o_gate_up"));
       } else {
@@ -1005,7 +1020,7 @@ int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool wan
       }
     }
     {  // down_proj + residual (llama.py:165,190); with the next layer's q|k|v behind it in the same launch
-      GemvCall c; c.x = e->act; c.ldx = I; c.act = act; c.rnd = RND_NONE; c.epi = EPI_RESID; c.resid = e->h; c.ldo = H; c.x_split = e->act_split;
+      GemvCall& c = cdn; c.x_split = e->act_split;
       if ((e->opt_fused_pairs & 2) && li + 1 < d.num_layers &&
           can_pair(e, lw.down, c, e->layers[li + 1].qkv, qkv_call(li + 1), R)) {
         MI_TRY(gemv_pair(e, lw.down, c, e->layers[li + 1].qkv, qkv_call(li + 1), R, "gemv_down_qkv"));
@@ -1152,8 +1167,10 @@ int forward_mixed(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t* l
       GemvCall cg; cg.x = e->h; cg.ldx = H; cg.act = act; cg.rnd = RND_NONE; cg.pro = PRO_NORM; cg.norm_w = post_norm;
       cg.eps = d.rms_norm_eps; cg.epi = EPI_SWIGLU; cg.out = e->act; cg.ldo = I; cg.pair_offset = I;
       cg.split_out = down_takes_split(e, lw.down, act, R);
+      GemvCall c; c.x = e->act; c.ldx = I; c.act = act; c.rnd = RND_NONE; c.epi = EPI_RESID; c.resid = e->h; c.ldo = H;
+      act_frag(e, lw, cg, c, R);
       MI_TRY(gemv_rows(e, lw.gate_up, cg, R, es, es, "gemv_gate_up"));
-      GemvCall c; c.x = e->act; c.ldx = I; c.act = act; c.rnd = RND_NONE; c.epi = EPI_RESID; c.resid = e->h; c.ldo = H; c.x_split = e->act_split;
+      c.x_split = e->act_split;
       MI_TRY(gemv_rows(e, lw.down, c, R, es, es, "gemv_down")); }
   }
   if (n_out > 0) {                               // hidden states of the wanted positions -> compact rows -> head
@@ -1304,7 +1321,7 @@ void mi_engine_destroy(mi_engine* e) {
     hipFree(l.in_norm); hipFree(l.post_norm); hipFree(l.q_norm); hipFree(l.k_norm);
     hipFree(l.in_norm32); hipFree(l.post_norm32); hipFree(l.q_norm32); hipFree(l.k_norm32);
   }
-  hipFree(e->small_buf); hipFree(e->o_frag); hipFree(e->final_norm32); hipFree(e->xn); hipFree(e->xs); hipFree(e->gk_ws);
+  hipFree(e->small_buf); hipFree(e->o_frag); hipFree(e->act_frag); hipFree(e->final_norm32); hipFree(e->xn); hipFree(e->xs); hipFree(e->gk_ws);
   free_linear(e->embed); free_linear(e->lm_head);
   hipFree(e->final_norm); hipFree(e->cos_tab); hipFree(e->sin_tab);
   hipFree(e->h); hipFree(e->qkv); hipFree(e->q); hipFree(e->attn); hipFree(e->act); hipFree(e->logits); hipFree(e->lora_t); hipFree(e->d_forced); hipFree(e->d_gather);

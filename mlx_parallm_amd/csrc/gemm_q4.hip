@@ -46,6 +46,7 @@ struct Q4Params {
   int M, G;
   const void* w;
   int epi; void* out; int ldo; void* resid; int pair_tiles;
+  int out_frag;                                                 // SwiGLU: out in q4_frag_elem's order
   int ntu, ntiles;                                              // column tiles of a half of the matrix (SwiGLU: gate tiles), of all of it
   int wgs;                                                      // (q4_rows_kernel: without those that only load)
   int nblk, ksplit, nslab, ngroups, nunits;                              // K / 128; units = tile groups x ksplit
@@ -55,6 +56,10 @@ struct Q4Params {
   int lora_row0_0, lora_n_0, lora_rank_0; float lora_scale_0;
   int lora_row0_1, lora_n_1, lora_rank_1; float lora_scale_1;
 };
+
+__device__ __forceinline__ size_t swiglu_at(const Q4Params& p, int row, int n) {       // (uniform)
+  return p.out_frag > 0 ? q4_frag_elem(row, n, p.out_frag, p.ntu / 4) : (size_t)row * p.ldo + n;
+}
 
 // One workgroup per row (rows padded to whole slabs with zeros) and gridDim.y pieces of K (one with a norm: it needs the whole row).  The 8 k of dword d
 // of a group (k = 64 grp + 8 d ..) are what lane group d >> 1 multiplies in step d & 1, in unpack_q4's order.
@@ -498,7 +503,7 @@ __global__ __launch_bounds__(512, 2) void q4_kernel(const Q4Params p) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = row0 + m * 16 + g * 4 + r;
-        if (row < p.M) out[(size_t)row * p.ldo + n] = silu16<AT>(gt[r], up[r]);
+        if (row < p.M) out[swiglu_at(p, row, n)] = silu16<AT>(gt[r], up[r]);
       }
     } else {
       const f32x4 v = tot[k][0];
@@ -705,7 +710,7 @@ __global__ __launch_bounds__(512, 2) void q4_rows_kernel(const Q4Params p) {
     const float v = r == 0 ? y[0].x : r == 1 ? y[0].y : r == 2 ? y[0].z : y[0].w;
     if constexpr (SWIGLU) {
       const float up = r == 0 ? y[1].x : r == 1 ? y[1].y : r == 2 ? y[1].z : y[1].w;
-      out[(size_t)row * p.ldo + n] = silu16<AT>(v, up);
+      out[swiglu_at(p, row, n)] = silu16<AT>(v, up);
     } else {
       float z = (float)(AT)v;
       if (p.lora_t != nullptr) {
@@ -876,6 +881,8 @@ int launch_gemm_q4(const LinearW& W, const GemvCall& c, size_t rows, hipStream_t
   Q4Params p{};
   p.xq = c.x_frag > 0 ? c.x : xq; p.sx = sx; p.sxo = sxo; p.M = (int)rows; p.G = W.K / 64; p.w = W.w;
   p.epi = c.epi; p.out = c.out; p.ldo = c.ldo; p.resid = c.resid; p.pair_tiles = c.epi == EPI_SWIGLU ? c.pair_offset / 16 : 0;
+  if (c.out_frag > 0 && (c.epi != EPI_SWIGLU || c.out_frag != pl.mt || pl.ntu % 8 != 0)) return fail(MI_ERR_INVALID, "gemm_q4: fragment order for another call");
+  p.out_frag = c.out_frag;
   p.ntu = pl.ntu; p.ntiles = pl.ntiles; p.nblk = pl.nblk; p.ksplit = pl.ksplit; p.nslab = pl.nslab; p.ngroups = pl.ngroups; p.nunits = pl.ngroups * pl.ksplit;
   p.ws = (float*)((char*)sxo + pl.sxo_bytes); p.ctr = ctr;
   p.lora_t = c.lora_t; p.lora_t_ld = c.lora_t_ld;

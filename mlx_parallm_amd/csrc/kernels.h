@@ -74,6 +74,7 @@ struct GemvCall {
   float* sq_out = nullptr;
   const float* sq_in = nullptr;
   int sq_parts = 0;
+  int out_frag = 0;               // > 0 (EPI_SWIGLU of gemm_q4.hip): out takes row tiles a slab in that order, as the next linear's x
   int x_frag = 0;                 // > 0: x holds gemm_q4_frag_mt() row tiles a slab in q4_frag_elem's order, ready to be multiplied
   void* ev_start = nullptr;       // measurement: hipEvent_t pair stamped with this kernel's own begin / end
   void* ev_stop = nullptr;        // (hipExtLaunchKernelGGL); MFMA path only

@@ -1304,13 +1304,13 @@ def test_a_mixed_step_s_attention_in_one_launch_equals_two_launches(tmp_path, dt
 
 
 @pytest.mark.parametrize("dtype,arch,heads,kv_heads,hd", [("bfloat16", "qwen3", 5, 1, 128), ("float16", "llama", 8, 8, 64), ("bfloat16", "llama", 16, 4, 32)])
-def test_attention_that_leaves_its_rows_prepared_for_the_int4_output_linear(tmp_path, dtype, arch, heads, kv_heads, hd):
-    """Decode steps and mixed steps of 17 to 128 rows (every number of row tiles and slabs) of an int4 model: the attention's rows in the output linear's order, the
-    same bits as with its preparation launch; an adapter on the output linear of one layer keeps that one."""
+def test_rows_that_a_launch_leaves_prepared_for_the_next_int4_linear(tmp_path, dtype, arch, heads, kv_heads, hd):
+    """Decode steps and mixed steps of 17 to 128 rows (every number of row tiles and slabs) of an int4 model: the attention's rows in the output linear's order
+    and the gated unit's in the down projection's, the same bits as with their preparation launches; an adapter on the output linear of one layer keeps that one."""
     from mlx_parallm_amd.tiny_model import build_tiny_model
 
     build_tiny_model(tmp_path, seed=4, vocab_size=512, model_type=arch, dtype=dtype, quantize_model=True, hidden_size=256, layers=2, heads=heads, kv_heads=kv_heads, head_dim=hd,
-                     intermediate_size=256, norm_jitter=0.2, with_tokenizer=False)
+                     intermediate_size=640, norm_jitter=0.2, with_tokenizer=False)
     eng = utils.load_model(str(tmp_path), max_positions=1024).engine
     rng = np.random.default_rng(6)
     calls = [([r], 0) for r in (17, 33, 64, 65, 97, 128)] + [([12], 16), ([30], 33), ([3], 90)]
