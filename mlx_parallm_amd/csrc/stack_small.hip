@@ -502,8 +502,9 @@ int kind_of(const LinearW& W) { return wk_is_quant(W.wk) ? SMALL_CODES : W.wk ==
 
 }  // namespace
 
-// does a matrix fit the threads' registers?
+// does a matrix fit the threads' registers?  (Adapters are the launches': the kernels have no second product, and one may be set before the weights are complete)
 bool small_stack_fits(const LinearW& W, bool big) {
+  if (W.lora_b[0] != nullptr || W.lora_b[1] != nullptr) return false;
   const int kind = kind_of(W), per = per_of(kind);
   return W.N <= (big ? 256 : 64) && W.K <= (big ? 64 : 128) && W.K % per == 0 && (kind != SMALL_CODES || (W.group % 32 == 0 && W.K % W.group == 0));
 }

@@ -1376,3 +1376,34 @@ def test_a_small_model_s_prompt_in_one_launch_equals_the_launches_it_replaces(tm
     assert all(np.array_equal(a, b) for a, b in zip(outs[True, 1], outs[False, 1]))
     eng.set_option("small_stack", 1)
     eng.close()
+
+
+@pytest.mark.parametrize("proj", ["self_attn.q_proj", "self_attn.v_proj", "self_attn.o_proj", "mlp.down_proj"])
+def test_an_adapter_set_before_the_weights_are_complete_is_in_a_small_model_s_steps(tmp_path, proj):
+    """Before or after finalize: the same adapter, the same bits, of prompts and decode steps that the small models' kernels would take without one."""
+    from safetensors.torch import load_file
+
+    from mlx_parallm_amd.engine import Engine
+    from mlx_parallm_amd.tiny_model import build_tiny_model
+
+    cfg = build_tiny_model(tmp_path, seed=5, vocab_size=512, dtype="bfloat16", quantize_model=True, q_bits=4, q_group_size=64, hidden_size=64, layers=3, heads=4, kv_heads=4,
+                           intermediate_size=128, head_dim=16, norm_jitter=0.2, with_tokenizer=False)
+    weights = load_file(str(next(tmp_path.glob("*.safetensors"))))
+    rng = np.random.default_rng(8)
+    k, n = {"mlp.down_proj": (128, 64)}.get(proj, (64, 64))
+    a, b = rng.standard_normal((k, 4)).astype(np.float32) * 0.3, rng.standard_normal((4, n)).astype(np.float32) * 0.3
+    toks = rng.integers(0, 512, (2, 9)).astype(np.int32)
+    outs = []
+    for when in ("before", "after", "never"):
+        eng = Engine(cfg, device=0, max_positions=256, act_dtype="bfloat16")
+        eng.load_tensors(weights.items())
+        if when == "before":
+            eng.set_lora(1, proj, a, b, 2.0)
+        eng.finalize()
+        if when == "after":
+            eng.set_lora(1, proj, a, b, 2.0)
+        kv = eng.new_kv(2, capacity=64, kv_dtype="float32")
+        outs.append([eng.forward(toks, kv), eng.forward(toks[:, :1], kv)])
+        eng.close()
+    for before, after, never in zip(*outs):
+        assert np.array_equal(before, after) and not np.array_equal(before, never)
