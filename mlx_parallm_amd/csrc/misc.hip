@@ -1010,6 +1010,7 @@ size_t sample_ws_bytes(int B) {
 }
 
 int launch_sample(const SampleCall& c, hipStream_t st) {
+  if (c.B < 1) return fail(MI_ERR_INVALID, "sample: no rows");
   if (c.top_logprobs < 0 || c.top_logprobs > MI_MAX_TOP_LOGPROBS) return fail(MI_ERR_INVALID, "sample: top_logprobs out of range");
   const bool draws = c.forced == nullptr && (c.row_temp != nullptr || c.temperature != 0.f);
   if (c.ws != nullptr && c.V >= (draws || c.top_logprobs > 0 ? SAMPLE_SPLIT_VOCAB : SAMPLE_SPLIT_GREEDY) &&

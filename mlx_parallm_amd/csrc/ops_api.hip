@@ -318,6 +318,7 @@ int mi_op_sample(float* logits, int B, int V, float temperature, float top_p, co
                  int top_logprobs, int32_t* tokens_out, float* logprob_out, float* prob_row0_out,
                  int32_t* topk_ids, float* topk_logprobs, float* row_stats) {
   if (!logits || !tokens_out || !row_stats) return fail(MI_ERR_INVALID, "null argument");
+  if (B < 1) return fail(MI_ERR_INVALID, "mi_op_sample: no rows");
   MI_TRY(ready());
   SampleCall sc{};
   sc.logits = logits; sc.B = B; sc.V = V; sc.rnd = RND_NONE; sc.temperature = temperature; sc.top_p = top_p;

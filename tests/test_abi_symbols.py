@@ -51,6 +51,18 @@ def test_no_cpu_backend_fails_loudly():
     assert _lib.lib().mi_op_gemv(C.byref(ol), C.byref(a)) == -4          # MI_ERR_RUNTIME, not a silent fallback
 
 
+@pytest.mark.parametrize("rows", [0, -1])
+@pytest.mark.parametrize("vocab", [512, 32000])
+def test_sampling_of_no_rows_is_refused(rows, vocab):
+    """Before anything is launched or divided by their number."""
+    from mlx_parallm_amd import _lib
+
+    some = (C.c_float * 4)()                              # (never read)
+    p = C.cast(some, C.c_void_p)
+    assert _lib.lib().mi_op_sample(p, rows, vocab, 1.0, 0.9, p, 0, p, p, p, p, p, p) == -1          # MI_ERR_INVALID
+    assert b"no rows" in _lib.lib().mi_last_error()
+
+
 def test_product_never_imports_the_oracle():
     for py in (ROOT / "mlx_parallm_amd").rglob("*.py"):
         text = py.read_text()
