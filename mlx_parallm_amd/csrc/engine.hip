@@ -845,9 +845,6 @@ int split_prefill(mi_engine* e, AttnCall& ac, int max_keys) {
   return MI_OK;
 }
 
-// the model forward for B*L tokens already in e->d_tokens; logits of the requested rows end
-// up in e->logits (float32, [B][V] or [B*L][V]).
-// `rows` (host, B distinct cache rows) = the call covers that subset of kv's rows, batch entry b <-> rows[b]
 // The layers of a small model as stack_small.hip reads them: made behind the last weight, where every matrix fits the kernel's registers
 int make_small_stack(mi_engine* e) {
   const mi_model_desc& d = e->d;
@@ -883,13 +880,16 @@ int make_small_stack(mi_engine* e) {
 //   float32 one row 230 / 144, 516 / 325, 915 / 622, 1702 / 1262, 5074 / 5396  two rows 272 / 165, 925 / 341, 1711 / 629, 3297 / 1261, 10017 / 5427
 //   bf16    one row 256 / 145, 273 / 264, 335 / 473, 662 / 967                 two rows 280 / 162, 342 / 286, 668 / 502, 643 / 991, 690 / 4581; 32 rows 989 / 478, 993 / 605, 1036 / 817, 1135 / 1305
 //   int8    one row 279 / 130, 292 / 249, 365 / 448, 621 / 913                 two rows 307 / 144, 377 / 256, 632 / 465, 1097 / 937, 911 / 4380; 8 rows 921 / 535 at 32, 961 / 1001 at 64
-bool small_stack_takes(const mi_engine* e, const mi_kv* kv, int act, int B, int L, const int32_t* rows) {
-  if (e->small_buf == nullptr || !e->opt_small_stack || e->opt_force_v1 || !e->opt_fused_attn || !e->prof_name.empty() || act != MI_F32 || kv->dtype != MI_F32) return false;
-  if (L > (e->small_mfma ? (B == 1 ? 16 : 32) : B == 1 ? 128 : SMALL_MAX_KEYS)) return false;
-  for (int b = 0; b < B; ++b) if (kv->h_off[rows ? rows[b] : b] + L > SMALL_MAX_KEYS) return false;
-  return true;
+// -> the most cached keys that a row may have to be theirs; -1: none is.  A matter of the call's shape, so that a row's bits depend on its own keys and on nothing of its neighbours'
+int small_stack_keys(const mi_engine* e, const mi_kv* kv, int act, int B, int L) {
+  if (e->small_buf == nullptr || !e->opt_small_stack || e->opt_force_v1 || !e->opt_fused_attn || !e->prof_name.empty() || act != MI_F32 || kv->dtype != MI_F32) return -1;
+  if (L > (e->small_mfma ? (B == 1 ? 16 : 32) : B == 1 ? 128 : SMALL_MAX_KEYS)) return -1;
+  return SMALL_MAX_KEYS - L;
 }
 
+// the model forward for B*L tokens already in e->d_tokens; logits of the requested rows end
+// up in e->logits (float32, [B][V] or [B*L][V]).
+// `rows` (host, B distinct cache rows) = the call covers that subset of kv's rows, batch entry b <-> rows[b]
 int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool want_logits, const int32_t* rows = nullptr) {
   const mi_model_desc& d = e->d;
   const size_t R = (size_t)B * L;
@@ -944,13 +944,18 @@ int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool wan
   }
 
   bool qkv_done = false;     // this layer's q|k|v already ran behind the previous layer's down_proj
-  const bool small = small_stack_takes(e, kv, act, B, L, rows);
-  if (small) {
+  const int small_keys = small_stack_keys(e, kv, act, B, L);
+  int n_small = 0;
+  for (int b = 0; b < B; ++b) n_small += kv->h_off[row_of(b)] <= small_keys;
+  const bool small = n_small == B;
+  auto small_stack = [&](const void* x) -> int {
     SmallStackCall c{AttnShape{B, L, Hq, Hkv, D, act, kv->dtype, RND_NONE, kv->cap, d_rows}, d.num_layers, H, I, e->small_kind, e->layers[0].qkv.W.group, rndT, d.rms_norm_eps,
-                     1.0f / sqrtf((float)D), e->small_words, e->small_scales, e->small_norms, (float*)e->h, (float*)kv->k, (float*)kv->v, layer_elems, kv->d_off, e->cos_tab, e->sin_tab};
+                     1.0f / sqrtf((float)D), e->small_words, e->small_scales, e->small_norms, (const float*)x, (float*)e->h, (float*)kv->k, (float*)kv->v, layer_elems, kv->d_off,
+                     e->cos_tab, e->sin_tab, small ? SMALL_MAX_KEYS : small_keys, small};
     kv_shape(kv, c.s);
-    MI_TRY(launch_stack_small(c, st));
-  }
+    return launch_stack_small(c, st);
+  };
+  if (small) MI_TRY(small_stack(e->h));
   for (int li = small ? d.num_layers : 0; li < d.num_layers; ++li) {
     LayerW& lw = e->layers[li];
     const bool w32 = quirk && d.act_dtype != MI_F32;     // norm weights must match the activation storage type
@@ -1029,6 +1034,13 @@ int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool wan
         MI_TRY(gemv_rows(e, lw.down, c, R, es, es, "gemv_down"));
       }
     }
+  }
+  // Rows on both sides of that line: the launches have run for all of them (their kernels go by the number of rows), and what they left of the shorter rows -- hidden states and
+  // the new tokens' keys and values -- is written again
+  if (n_small > 0 && !small) {
+    EmbedCall ec{e->tok_src ? e->tok_src : e->d_tokens, (int)R, act, rndT, e->xn};
+    MI_TRY(launch_embed(e->embed.W, ec, st));
+    MI_TRY(small_stack(e->xn));
   }
   if (want_logits) {  // final norm + lm_head / tied embedding (llama.py:231,249-252)
     const FusedLinear& head = d.tie_word_embeddings ? e->embed : e->lm_head;

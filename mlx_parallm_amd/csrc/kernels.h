@@ -379,19 +379,22 @@ bool attention_mixed_takes(const AttnDecodeCall& c, const AttnCall& p, int ncu);
 int launch_attention_mixed(const AttnDecodeCall& c, const AttnCall& p, hipStream_t st);
 bool gemv_mfma_supported(const LinearW& W, const GemvCall& c);
 
-// A decode step of a small model in one launch (stack_small.hip): float32 activations and caches, no norm of queries and keys, no adapters.  Words and scales of the
-// layers, q|k|v, o, gate|up and down behind one another in each; the two norms' weights of each
+// A decode step or a prompt of a small model in one launch (stack_small.hip): float32 activations and caches, no norm of queries and keys, no adapters.  Words and scales of
+// the layers, q|k|v, o, gate|up and down behind one another in each; the two norms' weights of each
 enum : int { SMALL_F32 = 0, SMALL_BF16 = 1, SMALL_F16 = 2, SMALL_CODES = 3 };
-constexpr int SMALL_MAX_KEYS = 256;     // (keys of a row, the new one included)
+constexpr int SMALL_MAX_KEYS = 256;     // (keys of a row, the new ones included)
 struct SmallStackCall {
-  AttnShape s;                   // L = 1; rows, block table
+  AttnShape s;                   // L tokens of every row; rows, block table
   int layers, H, I, kind, group, rnd0;     // rnd0: logical rounding of layer 0 up to its attention
   float eps, scale;
   const uint32_t* words; const float2* scales; const float* norms;
-  float* h;                      // [B][H] embeddings in, last hidden states out
+  const float* x;                // [B L][H] embeddings
+  float* h;                      // [B L][H] last hidden states (x and h may be one)
   float* kcache; float* vcache; size_t layer_elems;
-  int32_t* offsets;              // [cache row], advanced by one
+  int32_t* offsets;              // [cache row]
   const float* cos_tab; const float* sin_tab;
+  int upto;                      // rows behind more cached keys than this are left alone (SMALL_MAX_KEYS: there are none)
+  bool advance;                  // offsets += L
 };
 bool small_stack_fits(const LinearW& W, bool big);       // big: q|k|v, gate|up
 bool small_stack_shape(int H, int heads, int kv_heads, int D, int I);

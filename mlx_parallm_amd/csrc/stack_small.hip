@@ -190,6 +190,7 @@ __global__ __launch_bounds__(NT) void stack_small_kernel(SmallStackCall c) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), b = blockIdx.x;
   const int H = c.H, Hq = c.s.Hq, Hkv = c.s.Hkv, G = Hq / Hkv, nq = Hq * D, nkv = Hkv * D, I = c.I;
   const int kb = c.s.rows ? c.s.rows[b] : b, pos = c.offsets[kb];
+  if (c.upto < SMALL_MAX_KEYS && pos > c.upto) return;          // (uniform)
   const Part pq = part_of<true>(nq + 2 * nkv, H / PER, c.group), po = part_of<false>(H, nq / PER, c.group), pg = part_of<true>(2 * I, H / PER, c.group), pd = part_of<false>(H, I / PER, c.group);
   Regs<KIND, true> rq, rg;
   Regs<KIND, false> ro, rd;
@@ -199,7 +200,7 @@ __global__ __launch_bounds__(NT) void stack_small_kernel(SmallStackCall c) {
   rg.load(c.words + GW, c.scales + 4 * NT);
   rd.load(c.words + DW, c.scales + 6 * NT);
   const int col = min(lane, H - 1);
-  float x = lane < H ? c.h[(size_t)b * H + lane] : 0.f;         // a lane per column of the row
+  float x = lane < H ? c.x[(size_t)b * H + lane] : 0.f;         // a lane per column of the row
   const int ri = lane % (D / 2);                      // a lane's rotation: the same for every 64 / (D / 2) heads
   const float cs = c.cos_tab[(size_t)pos * (D / 2) + ri], sn = c.sin_tab[(size_t)pos * (D / 2) + ri];
   const float sc2 = c.scale * LOG2E;
@@ -332,7 +333,7 @@ __global__ __launch_bounds__(NT) void stack_small_kernel(SmallStackCall c) {
   }
   if (wave == 0) {
     if (lane < H) c.h[(size_t)b * H + lane] = x;
-    if (lane == 0) c.offsets[kb] = pos + 1;           // (nobody else reads it in this step)
+    if (lane == 0 && c.advance) c.offsets[kb] = pos + 1;      // (nobody else reads it in this step)
   }
 }
 
@@ -356,6 +357,7 @@ __global__ __launch_bounds__(NT) void small_prompt_kernel(SmallStackCall c) {
   float* s = act + PT * 128 + wave * SMALL_MAX_KEYS;  // [SMALL_MAX_KEYS]: this wave's scores
   const int H = c.H, Hq = c.s.Hq, Hkv = c.s.Hkv, G = Hq / Hkv, nq = Hq * D, nkv = Hkv * D, I = c.I, L = c.s.L;
   const int kb = c.s.rows ? c.s.rows[b] : b, before = c.offsets[kb];
+  if (c.upto < SMALL_MAX_KEYS && before > c.upto) return;       // (uniform)
   const Part pq = part_of<true>(nq + 2 * nkv, H / PER, c.group), po = part_of<false>(H, nq / PER, c.group), pg = part_of<true>(2 * I, H / PER, c.group), pd = part_of<false>(H, I / PER, c.group);
   Regs<KIND, true> rq, rg;
   Regs<KIND, false> ro, rd;
@@ -373,7 +375,7 @@ __global__ __launch_bounds__(NT) void small_prompt_kernel(SmallStackCall c) {
 #pragma unroll
     for (int u = 0; u < OWN; ++u) {
       const int t = min(wave + NW * u, n - 1);
-      x[u] = c.h[((size_t)b * L + t0 + t) * H + col];
+      x[u] = c.x[((size_t)b * L + t0 + t) * H + col];
       if (lane >= H) x[u] = 0.f;
       cs[u] = c.cos_tab[(size_t)(pos + t) * (D / 2) + ri]; sn[u] = c.sin_tab[(size_t)(pos + t) * (D / 2) + ri];
     }
@@ -494,7 +496,7 @@ __global__ __launch_bounds__(NT) void small_prompt_kernel(SmallStackCall c) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // these keys and values are the next tokens' cache
     __syncthreads();
   }
-  if (tid == 0) c.offsets[kb] = before + L;           // (read at the head, in front of many barriers)
+  if (tid == 0 && c.advance) c.offsets[kb] = before + L;           // (read at the head, in front of many barriers)
 }
 
 int per_of(int kind) { return kind == SMALL_F32 ? 1 : kind == SMALL_CODES ? 4 : 2; }
