@@ -880,7 +880,7 @@ int make_small_stack(mi_engine* e) {
 //   float32 one row 230 / 144, 516 / 325, 915 / 622, 1702 / 1262, 5074 / 5396  two rows 272 / 165, 925 / 341, 1711 / 629, 3297 / 1261, 10017 / 5427
 //   bf16    one row 256 / 145, 273 / 264, 335 / 473, 662 / 967                 two rows 280 / 162, 342 / 286, 668 / 502, 643 / 991, 690 / 4581; 32 rows 989 / 478, 993 / 605, 1036 / 817, 1135 / 1305
 //   int8    one row 279 / 130, 292 / 249, 365 / 448, 621 / 913                 two rows 307 / 144, 377 / 256, 632 / 465, 1097 / 937, 911 / 4380; 8 rows 921 / 535 at 32, 961 / 1001 at 64
-// -> the most cached keys that a row may have to be theirs; -1: none is.  A matter of the call's shape, so that a row's bits depend on its own keys and on nothing of its neighbours'
+// -> the most cached keys that a row may have to be theirs; -1: none is.  A matter of the call's shape, so that a prompt's bits depend on its own keys and on nothing of its neighbours'
 int small_stack_keys(const mi_engine* e, const mi_kv* kv, int act, int B, int L) {
   if (e->small_buf == nullptr || !e->opt_small_stack || e->opt_force_v1 || !e->opt_fused_attn || !e->prof_name.empty() || act != MI_F32 || kv->dtype != MI_F32) return -1;
   if (L > (e->small_mfma ? (B == 1 ? 16 : 32) : B == 1 ? 128 : SMALL_MAX_KEYS)) return -1;
@@ -947,6 +947,7 @@ int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool wan
   const int small_keys = small_stack_keys(e, kv, act, B, L);
   int n_small = 0;
   for (int b = 0; b < B; ++b) n_small += kv->h_off[row_of(b)] <= small_keys;
+  if (L == 1 && n_small < B) n_small = 0;      // (decode steps: all rows or none.  The launches' attention of heads this small splits every row by the longest's keys; both kernels: 348 us for 244)
   const bool small = n_small == B;
   auto small_stack = [&](const void* x) -> int {
     SmallStackCall c{AttnShape{B, L, Hq, Hkv, D, act, kv->dtype, RND_NONE, kv->cap, d_rows}, d.num_layers, H, I, e->small_kind, e->layers[0].qkv.W.group, rndT, d.rms_norm_eps,
@@ -1035,7 +1036,7 @@ int forward_device(mi_engine* e, mi_kv* kv, int B, int L, bool all_pos, bool wan
       }
     }
   }
-  // Rows on both sides of that line: the launches have run for all of them (their kernels go by the number of rows), and what they left of the shorter rows -- hidden states and
+  // A prompt's rows on both sides of that line: the launches have run for all of them (their kernels go by the number of rows), and what they left of the shorter rows -- hidden states and
   // the new tokens' keys and values -- is written again
   if (n_small > 0 && !small) {
     EmbedCall ec{e->tok_src ? e->tok_src : e->d_tokens, (int)R, act, rndT, e->xn};
