@@ -874,17 +874,27 @@ int make_small_stack(mi_engine* e) {
   }
   return MI_OK;
 }
-// Prompts: one workgroup a row, so what decides is the chain of one row, 16 tokens a time, against the launches: eight rows of the call each where only the generic kernels take the
-// matrices, on the matrix cores else (bf16 weights, int8).  us by launches / here, eight layers, prompts of 2 / 16 / 32 / 64 / 200 tokens:
-//   4-bit   one row 244 / 117, 514 / 232, 905 / 439, 1802 / 904, 4926 / 4386   two rows 281 / 126, 908 / 244, 1809 / 453, 3269 / 925, 9501 / 4387   (float16 weights and scales alike)
-//   float32 one row 230 / 144, 516 / 325, 915 / 622, 1702 / 1262, 5074 / 5396  two rows 272 / 165, 925 / 341, 1711 / 629, 3297 / 1261, 10017 / 5427
-//   bf16    one row 256 / 145, 273 / 264, 335 / 473, 662 / 967                 two rows 280 / 162, 342 / 286, 668 / 502, 643 / 991, 690 / 4581; 32 rows 989 / 478, 993 / 605, 1036 / 817, 1135 / 1305
-//   int8    one row 279 / 130, 292 / 249, 365 / 448, 621 / 913                 two rows 307 / 144, 377 / 256, 632 / 465, 1097 / 937, 911 / 4380; 8 rows 921 / 535 at 32, 961 / 1001 at 64
+// Prompts: one workgroup a row, so what decides is the chain of one row, 16 tokens a time and every token over all of the row's keys, against the launches: eight rows of the call
+// each where only the generic kernels take the matrices, 32 on the matrix cores else (bf16 weights, int8); cached keys cost those next to nothing.  us a call by launches / here,
+// eight layers, four heads of 16, prompts of 2 / 16 / 32 / 64 / 96 tokens on empty caches, then 2 / 8 / 16 / 32 behind 128 keys:
+//   4-bit   one row 218 / 93, 485 / 211, 875 / 409, 1775 / 852, 2501 / 1454; 356 / 124, 340 / 247, 545 / 431, 886 / 867   two rows .., 868 / 208, 1765 / 409, 3210 / 854; 32 behind 192 1784 / 1117
+//   float32 one row 199 / 111, 471 / 293, 865 / 573, 1647 / 1184, 2448 / 1948; 441 / 142, 339 / 291, 624 / 519, 1025 / 1044   two rows .., 866 / 292, 1641 / 572, 3212 / 1185; 1721 / 1289
+//   bf16    one row 216 / 96, 232 / 217; 244 / 177, 272 / 306, 282 / 510   two rows 222 / 96, 288 / 218, 609 / 425; 260 / 175, 288 / 306, 335 / 507, 628 / 967   32 rows .., 605 / 225, 644 / 431; 637 / 517, 702 / 999
+//   int8    one row 251 / 92, 262 / 209; 323 / 175, 335 / 298, 322 / 494   two rows 266 / 95, 339 / 212, 591 / 410; 310 / 176, 296 / 305, 351 / 488, 604 / 928   32 rows .., 841 / 217, 884 / 418; 875 / 498, 945 / 954
+// So small_prompt_keys prices both: here what a token and the start take, and 0.12 us a token and key (of 64 columns of heads; and three tokens' worth of every cached key, for its first
+// read), the launches 25 us a token or, on the matrix cores, by the number of rows.  Eight heads of 16, 4-bit, 128 tokens behind 32 keys 3114 / 3739: the launches'.
+// A decode step is ahead at every number of keys (behind 240 287 / 213).
 // -> the most cached keys that a row may have to be theirs; -1: none is.  A matter of the call's shape, so that a prompt's bits depend on its own keys and on nothing of its neighbours'
+int small_prompt_keys(bool mfma, int kind, int width, int B, int L) {            // in units of 0.12 us; width: heads x head_dim
+  const int w = std::max(width, 64), R = B * L;
+  const int launches = !mfma ? (R < 8 ? 1600 + 85 * R : 700 + 208 * R) : R < 8 ? 1900 : R <= 16 ? 2080 : R <= 32 ? 2330 : 4600;
+  const int token = kind == SMALL_CODES || mfma ? 45 : 87;
+  return std::max(-1, (launches - 620 - token * L - (25 * L + L * L / 2) * w / 64) * 64 / (w * (L + 3)));
+}
 int small_stack_keys(const mi_engine* e, const mi_kv* kv, int act, int B, int L) {
   if (e->small_buf == nullptr || !e->opt_small_stack || e->opt_force_v1 || !e->opt_fused_attn || !e->prof_name.empty() || act != MI_F32 || kv->dtype != MI_F32) return -1;
   if (L > (e->small_mfma ? (B == 1 ? 16 : 32) : B == 1 ? 128 : SMALL_MAX_KEYS)) return -1;
-  return SMALL_MAX_KEYS - L;
+  return L == 1 ? SMALL_MAX_KEYS - 1 : std::min(SMALL_MAX_KEYS - L, small_prompt_keys(e->small_mfma, e->small_kind, e->d.num_heads * e->d.head_dim, B, L));
 }
 
 // the model forward for B*L tokens already in e->d_tokens; logits of the requested rows end

@@ -1450,3 +1450,42 @@ def test_a_small_model_s_row_does_not_depend_on_its_neighbours_keys(tmp_path, dt
                 for m, a in zip(mixed, alike):
                     assert np.isfinite(m).all() and np.array_equal(m[i], a[i]), (lens, i)
     eng.close()
+
+
+@pytest.mark.parametrize("dtype,bits,takes,leaves", [
+    ("bfloat16", 4, ((1, 100, 8), (1, 64, 64), (1, 0, 128), (2, 192, 64), (3, 0, 250), (1, 255, 1)), ((1, 200, 16), (1, 128, 96), (1, 100, 128), (1, 0, 129), (2, 200, 57), (1, 256, 1))),
+    ("float32", 0, ((1, 64, 8), (1, 64, 32), (1, 0, 128), (2, 190, 32), (3, 156, 100)), ((1, 192, 16), (1, 128, 64), (1, 64, 96), (2, 192, 65))),
+    ("bfloat16", 0, ((1, 64, 8), (1, 0, 16), (2, 20, 16), (3, 128, 16), (8, 20, 32), (1, 255, 1)), ((1, 128, 8), (1, 32, 16), (2, 64, 32), (8, 160, 16), (2, 0, 33), (1, 0, 17)))])
+@pytest.mark.parametrize("paged", [False, True])
+def test_which_prompts_of_a_small_model_its_kernel_takes(tmp_path, dtype, bits, takes, leaves, paged):
+    """By rows of the call, cached keys and tokens: what it takes differs from the launches in some last bits, what it leaves (longer behind more keys than it is ahead, or past
+    the keys it holds) does not.  Up to the last key, and the numbers of cached keys unequal as well."""
+    from mlx_parallm_amd.tiny_model import build_tiny_model
+
+    build_tiny_model(tmp_path, seed=5, vocab_size=512, dtype=dtype, quantize_model=bits > 0, q_bits=4, q_group_size=64, hidden_size=64, layers=3, heads=4, kv_heads=4,
+                     intermediate_size=128, head_dim=16, norm_jitter=0.2, with_tokenizer=False)
+    eng = utils.load_model(str(tmp_path), max_positions=1024).engine
+    rng = np.random.default_rng(4)
+
+    def both(befores, n):
+        out, B = [], len(befores)
+        toks = [rng.integers(0, 512, k).astype(np.int32) for k in befores] + [rng.integers(0, 512, (B, n)).astype(np.int32)]
+        for on in (1, 0):
+            eng.set_option("small_stack", on)
+            kv = eng.new_paged_kv(B, block_tokens=16, max_tokens_per_row=400, kv_dtype="float32") if paged else eng.new_kv(B, capacity=400, kv_dtype="float32")
+            for r in range(B):
+                if befores[r]:
+                    eng.forward_segments(kv, [r], [toks[r]])
+            out.append([eng.forward(toks[B], kv), eng.forward(toks[B][:, :1], kv) if max(befores) + n < 256 else None])
+            kv.close()
+        eng.set_option("small_stack", 1)
+        for a, b in zip(*out):
+            assert (a is None and b is None) or np.abs(a - b).max() <= (2e-5 if dtype == "float32" else 4e-3) * max(1.0, np.abs(b).max())
+        return [not np.array_equal(a, b) for a, b in zip(out[0][0], out[1][0])]
+    for B, before, n in takes:
+        assert all(both([before] * B, n)), (B, before, n)
+    for B, before, n in leaves:
+        assert not any(both([before] * B, n)), (B, before, n)
+    if bits == 4:
+        assert both([200, 0, 130], 56) == [True, True, True] and both([201, 0, 130], 56) == [False, True, True]
+    eng.close()
