@@ -559,25 +559,23 @@ __global__ __launch_bounds__(ST) void sample_kernel(SampleCall c) {
 // One workgroup per row leaves the card idle at a decode step's few rows and is bound by its own walks of the row, four to eight of them in a draw, each a
 // chain of loads, LDS atomics and barriers.  Here up to SG workgroups take a row's parts, in two launches (greedy, forced) or three:
 //   sample_parts:  maximum and sum of exp of every part, the best element of every 16 threads' share
-//   sample_masses: masses of every part in SNB bins of (max - l) / T in [0, 28): beyond, a mass is 0
+//   sample_masses: masses of every part in SNB bins of (max - l) / T from 0 to where the row's elements end, at most 28: beyond, a mass is 0
 //   sample_draw:   the bins hold the cut of the nucleus and the pick in known bins; their elements are collected, the last workgroup of the row to arrive
 //                  sorts them (key, id) and finds both, exactly: the integer masses add up to the same whatever the order.  One more workgroup does the
 //                  most likely tokens.  Probabilities of row 0 are made here: no launch of their own.
-// A row with NaN or +inf, a temperature that is no positive number, or more than SCAP elements in those bins (nearly equal logits) is drawn by
-// draw_row.  us, one workgroup per row / here: 8 rows of 32000 logits top-p with 5 log-probabilities 70 / 35, temperature alone 44 / 30, greedy with 5 23 / 19;
+// A row with NaN or +inf, a temperature that is no positive number, or more than SCAP elements in those bins (thousands of equal logits) is drawn by
+// draw_row, the launches in front for nothing (8 rows of 128256 210 us, 172 by one workgroup a row).  us, one workgroup per row / here: 8 rows of 32000 logits top-p with 5 log-probabilities 70 / 35, temperature alone 44 / 30, greedy with 5 23 / 19;
 // 128256 logits 176 / 57, 128 / 41, 32 / 22, greedy 20 / 15; 64 rows of 128256 194 / 70, greedy 20.5 / 18.8; 512 rows top-p 454 / 306; 256 rows of 16384 56 / 59.
 // Greedy without them: 32000 logits 11 / 11, 64 rows of 50304 13.0 / 14.5, 128 rows of 128256 21 / 24.  What is left of a draw is its chain: three launches,
 // the sum of the bins (3 us), the list through memory (4), the sort (3 to 6).
 constexpr int SG = SAMPLE_PARTS, SNB = 2048, SCAP = 4096, SW = ST / 64, SLABS = ST / 16;
 struct SampleRow {
-  float pmax[SG], psum[SG], psum_t[SG];
+  float pmax[SG], psum[SG], psum_t[SG], scale;
   int pidx[SG], odd[SG];
   unsigned listed, arrived;
   alignas(16) unsigned long long list[SCAP];         // order key << 32 | ~id: descending order is the candidates' order
   ArgMax slab[SG * SLABS];
 };
-// 73 bins a unit: 128256 logits of deviation 1.3 have some 600 elements in a bin at the cut
-__device__ __forceinline__ int mass_bin(float l, float mx, float inv_t) { return (int)fminf((mx - l) * inv_t * (SNB / 28.0f), SNB - 1); }
 // part g of a row: float4 pieces [first, last)
 __device__ __forceinline__ int part_at(int V, int g, int np) { return (int)((long)(V >> 2) * g / np); }
 template <class F>
@@ -615,6 +613,15 @@ __device__ __forceinline__ RowHead row_head(const SampleRow* w, int np) {
   h.lse = a.v + __logf(h.se);
   return h;
 }
+
+// Bins per unit of max - l.  Any number is right -- what lies beyond is in the last bin --, as long as both kernels use the same.  The range: three times the distance from the maximum to
+// the logarithm of the mean exp(l): all of a bell (that distance is 4.5 deviations less half a square).  28 T of every row, 73 bins a unit, left 600 elements of 128256 of deviation 1.3 in a bin
+// at the cut, and of rows that T makes flat more than a list takes: deviation 1, top-p, 8 rows at T = 1 / 5 / 20 67 / 201 / 203 us (one workgroup a row 169 / 172 / 173), 47 at all three now.
+__device__ __forceinline__ float bin_scale(const RowHead& h, int V, float inv_t) {
+  const float range = 3.0f * inv_t * (__logf((float)V) - (h.lse - h.mx));
+  return inv_t * SNB * __builtin_amdgcn_rcpf(fminf(fmaxf(range, 1e-30f), 28.0f));
+}
+__device__ __forceinline__ int mass_bin(float l, float mx, float scale) { return (int)fminf((mx - l) * scale, SNB - 1); }
 
 __global__ __launch_bounds__(ST) void sample_parts_kernel(SampleCall c, SampleRow* ws) {
   __shared__ ArgMax sh_am[SW];
@@ -655,7 +662,8 @@ __global__ __launch_bounds__(ST) void sample_masses_kernel(SampleCall c, SampleR
   if (!(temperature > 0.f)) return;
   const int np = gridDim.x;
   const RowHead h = row_head(w, np);
-  const float inv_t = 1.0f / temperature;
+  const float inv_t = 1.0f / temperature, scale = bin_scale(h, V, inv_t);
+  if (g == 0 && threadIdx.x == 0) w->scale = scale;
   for (int i = threadIdx.x; i < SNB; i += ST) m[i] = 0;
   __syncthreads();
   float st = 0.f;
@@ -664,7 +672,7 @@ __global__ __launch_bounds__(ST) void sample_masses_kernel(SampleCall c, SampleR
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const unsigned long long each = mass_fx(v[j], h.mx, inv_t);
-      if (each > 0 && !h.odd) atomicAdd(&m[mass_bin(v[j], h.mx, inv_t)], each);
+      if (each > 0 && !h.odd) atomicAdd(&m[mass_bin(v[j], h.mx, scale)], each);
       if (c.lp_temp) st += __expf((v[j] - h.mx) * inv_t);
     }
   });
@@ -727,7 +735,7 @@ __device__ __forceinline__ void sort_desc(unsigned long long (&a)[E], int n, uns
     }
 }
 
-struct DrawPlan { unsigned long long tgt, cut_above, pick_above; int cut, p0, p1; bool nucleus; float u, inv_t, mx; };
+struct DrawPlan { unsigned long long tgt, cut_above, pick_above; int cut, p0, p1; bool nucleus; float u, inv_t, mx, scale; };
 
 // The pick among the row's n collected words
 template <int E>
@@ -753,7 +761,7 @@ __device__ int pick_listed(const SampleRow* w, int n, const DrawPlan& d, unsigne
     const uint32_t k = (uint32_t)(a[e] >> 32);
     const float l = __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
     m[e] = i < n ? mass_fx(l, d.mx, d.inv_t) : 0ull;
-    bin[e] = i < n ? mass_bin(l, d.mx, d.inv_t) : -1;
+    bin[e] = i < n ? mass_bin(l, d.mx, d.scale) : -1;
   }
   unsigned long long kept = d.tgt;               // (no nucleus: everything, and tgt is the whole mass)
   if (d.nucleus) {
@@ -891,7 +899,7 @@ __global__ __launch_bounds__(ST) void sample_draw_kernel(SampleCall c, SampleRow
       token = draw_row(lg, V, mx, inv_t, top_p, u, h.best, sh_d);
     } else {
       DrawPlan d;
-      d.u = u; d.inv_t = inv_t; d.mx = mx;
+      d.u = u; d.inv_t = inv_t; d.mx = mx; d.scale = w->scale;
       d.nucleus = top_p > 0.f && top_p < 1.f;
       unsigned long long lower = 0, own = 0;     // (two bins a thread)
 #pragma unroll
@@ -927,7 +935,7 @@ __global__ __launch_bounds__(ST) void sample_draw_kernel(SampleCall c, SampleRow
         const float v[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const int bin = mass_bin(v[j], mx, inv_t);
+          const int bin = mass_bin(v[j], mx, d.scale);
           if ((bin >= d.p0 && bin <= d.p1) || bin == d.cut) {
             const unsigned i = atomicAdd(count, 1u);
             if (i < SCAP) sh.buf[i] = ((unsigned long long)order_key(v[j]) << 32) | (0xffffffffu - (uint32_t)(at + j));

@@ -758,3 +758,25 @@ def test_sampler_over_several_workgroups_equals_one(V, temp, top_p):
             np.testing.assert_allclose(g, o, rtol=1e-5, atol=2e-6)
         shifted = _run_sampler(np.roll(rows, 1, 0), temp, top_p, np.roll(uu, 1), k=5)          # a row's ids do not depend on where it stands
         assert np.array_equal(np.roll(shifted[0], -1), got[0])
+
+
+@pytest.mark.parametrize("V", [16384, 50304, 128256])
+@pytest.mark.parametrize("temp", [0.2, 5.0, 20.0, 1e4, 1e30, 3e38])
+@pytest.mark.parametrize("top_p", [1.0, 0.9, 0.999])
+def test_sampler_over_several_workgroups_on_rows_that_the_temperature_makes_flat(V, temp, top_p):
+    """The bins span the elements that have a mass, so a flat row's cut and pick lie among few: masked elements far down or at -inf, one element above the rest, equal ones."""
+    rng = np.random.default_rng(V)
+    plain = rng.standard_normal((3, V)).astype(np.float32)
+    rows = [plain[0], plain[0] * 1e-4 + 7.0, plain[1]]
+    for low in (-100.0, -1e9, float(np.finfo(np.float32).min), -np.inf):
+        rows.append(np.where(rng.random(V) < 0.3, np.float32(low), plain[2]))
+    rows.append(np.where(np.arange(V) < V // 2, np.float32(-1e9), plain[2]))      # whole parts of the row
+    top = plain[1].copy()
+    top[V // 5] = 90.0
+    rows += [top, np.full(V, 3.0, np.float32), np.where(np.arange(V) % 3 == 0, np.float32(1.0), np.float32(1.0 + 2.0 ** -23))]
+    rows, n = np.stack(rows), len(rows)
+    for u in (0.0, 0.6, 1.0 - 2.0 ** -24):
+        uu = np.concatenate([[u], rng.random(n - 1)]).astype(np.float32)
+        got = _run_sampler(rows, temp, top_p, uu)
+        one = _run_sampler(np.concatenate([rows, np.tile(rows[:1], (513 - n, 1))]), temp, top_p, np.concatenate([uu, np.zeros(513 - n, np.float32)]))
+        assert np.array_equal(got[0], one[0][:n]), (temp, top_p, u)
