@@ -427,9 +427,13 @@ struct SampleCall {
   float* row_stats;          // device [B][2] scratch: (max, logsumexp)
   void* ws = nullptr;        // sample_ws_bytes(B), or null: one workgroup per row
 };
-// The kernels with several workgroups a row: draws of up to SAMPLE_SPLIT_ROWS rows of SAMPLE_SPLIT_VOCAB logits and more; up to 64 rows without one, the
-// arg-max alone from SAMPLE_SPLIT_GREEDY logits on (the figures: misc.hip)
-constexpr int SAMPLE_PARTS = 8, SAMPLE_SPLIT_ROWS = 512, SAMPLE_SPLIT_VOCAB = 16384, SAMPLE_SPLIT_GREEDY = 65536;
+// The kernels with several workgroups a row, given a workspace (sample_splits): draws of up to SAMPLE_SPLIT_ROWS rows (SAMPLE_SPLIT_ROWS_NARROW below SAMPLE_SPLIT_WIDE logits) of
+// SAMPLE_SPLIT_VOCAB logits and more; up to SAMPLE_SPLIT_ROWS_GREEDY rows without one, the arg-max alone from SAMPLE_SPLIT_GREEDY logits on (the figures: misc.hip).  A vocabulary of
+// whole float4s.
+constexpr int SAMPLE_PARTS = 8, SAMPLE_SPLIT_VOCAB = 16384, SAMPLE_SPLIT_WIDE = 24576, SAMPLE_SPLIT_GREEDY = 65536;
+constexpr int SAMPLE_SPLIT_ROWS = 512, SAMPLE_SPLIT_ROWS_NARROW = 128, SAMPLE_SPLIT_ROWS_GREEDY = 64;
+constexpr int SAMPLE_WGS = 256;        // parts of all rows, or one a row: a round of the card's compute units (what the workspace holds, too)
+bool sample_splits(const SampleCall& c);
 size_t sample_ws_bytes(int B);
 int launch_sample(const SampleCall& c, hipStream_t st);
 

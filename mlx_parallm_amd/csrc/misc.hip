@@ -1010,24 +1010,29 @@ int launch_embed(const LinearW& W, const EmbedCall& c, hipStream_t st) {
   return fail(MI_ERR_INVALID, "embed: bad activation dtype");
 }
 
-// rows' words, then the bins of their parts: no more parts than 256 or one a row
+// rows' words, then the bins of their parts: no more parts than SAMPLE_WGS or one a row
 static_assert(sizeof(SampleRow) % 16 == 0, "the bins are read 16 bytes at a time");
 size_t sample_ws_bytes(int B) {
   const size_t rows = std::min(B, SAMPLE_SPLIT_ROWS);
-  return rows * sizeof(SampleRow) + std::max<size_t>(256, rows) * SNB * sizeof(unsigned long long);
+  return rows * sizeof(SampleRow) + std::max<size_t>(SAMPLE_WGS, rows) * SNB * sizeof(unsigned long long);
+}
+
+static bool sample_draws(const SampleCall& c) { return c.forced == nullptr && (c.row_temp != nullptr || c.temperature != 0.f); }
+bool sample_splits(const SampleCall& c) {
+  const bool draws = sample_draws(c);
+  return c.V >= (draws || c.top_logprobs > 0 ? SAMPLE_SPLIT_VOCAB : SAMPLE_SPLIT_GREEDY) &&
+         c.B <= (!draws ? SAMPLE_SPLIT_ROWS_GREEDY : c.V < SAMPLE_SPLIT_WIDE ? SAMPLE_SPLIT_ROWS_NARROW : SAMPLE_SPLIT_ROWS) && row_vec(c.logits, c.V);
 }
 
 int launch_sample(const SampleCall& c, hipStream_t st) {
   if (c.B < 1) return fail(MI_ERR_INVALID, "sample: no rows");
   if (c.top_logprobs < 0 || c.top_logprobs > MI_MAX_TOP_LOGPROBS) return fail(MI_ERR_INVALID, "sample: top_logprobs out of range");
-  const bool draws = c.forced == nullptr && (c.row_temp != nullptr || c.temperature != 0.f);
-  if (c.ws != nullptr && c.V >= (draws || c.top_logprobs > 0 ? SAMPLE_SPLIT_VOCAB : SAMPLE_SPLIT_GREEDY) &&
-      c.B <= (!draws ? 64 : c.V < 24576 ? 128 : SAMPLE_SPLIT_ROWS) && row_vec(c.logits, c.V)) {
+  if (c.ws != nullptr && sample_splits(c)) {
+    const bool draws = sample_draws(c);
     SampleRow* ws = (SampleRow*)c.ws;
     unsigned long long* hist = (unsigned long long*)(ws + c.B);
     const bool scaled = c.lp_temp && (c.row_temp != nullptr || (c.temperature > 0.f && c.temperature != 1.f));
-    // as many parts as a round of the card's 256 compute units has workgroups for
-    const int np = std::max(1, std::min(SG, 256 / c.B - (c.top_logprobs > 0))), nwg = draws ? np : 1;
+    const int np = std::max(1, std::min(SG, SAMPLE_WGS / c.B - (c.top_logprobs > 0))), nwg = draws ? np : 1;
     hipLaunchKernelGGL(sample_parts_kernel, dim3(np, c.B), dim3(ST), 0, st, c, ws);
     MI_HIP(hipGetLastError());
     if (draws || scaled) hipLaunchKernelGGL(sample_masses_kernel, dim3(np, c.B), dim3(ST), 0, st, c, ws, hist);

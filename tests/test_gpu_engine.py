@@ -1489,3 +1489,74 @@ def test_which_prompts_of_a_small_model_its_kernel_takes(tmp_path, dtype, bits, 
     if bits == 4:
         assert both([200, 0, 130], 56) == [True, True, True] and both([201, 0, 130], 56) == [False, True, True]
     eng.close()
+
+
+@pytest.mark.parametrize("vocab", [16384, 16396, 32000, 65540])
+def test_an_engine_s_sampler_over_several_workgroups(tmp_path, vocab):
+    """Every argument of a step on vocabularies whose rows several workgroups take, against one workgroup per row (more rows than the others serve) and float64: biases up to the
+    parts' edges, log-probabilities at temperature, rows with a temperature of their own next to greedy ones, given tokens and none."""
+    from mlx_parallm_amd.tiny_model import build_tiny_model
+    from tests.test_gpu_kernels import _run_sampler
+
+    build_tiny_model(tmp_path, seed=3, vocab_size=vocab, dtype="bfloat16", quantize_model=False, hidden_size=64, layers=1, heads=4, kv_heads=4, intermediate_size=128, head_dim=16,
+                     with_tokenizer=False)
+    eng = utils.load_model(str(tmp_path), max_positions=128).engine
+    rng = np.random.default_rng(vocab)
+    B = 6
+    toks = rng.integers(0, vocab, (B, 1)).astype(np.int32)
+    kv = eng.new_kv(B, capacity=64, kv_dtype="model")
+    logits = eng.forward(toks, kv)
+    edges = [4 * ((vocab // 4) * g // 8) for g in range(9)]
+    bias = {int(i): float(v) for i, v in zip(sorted({e + d for e in edges for d in (-1, 0) if 0 <= e + d < vocab}), rng.standard_normal(18) * 3)}
+
+    def biased(b):
+        lg = logits.copy()
+        for i, v in (b or {}).items():
+            lg[:, i] += np.float32(v)
+        return lg
+
+    def log_softmax(x):
+        x = x.astype(np.float64)
+        return x - x.max(-1, keepdims=True) - np.log(np.exp(x - x.max(-1, keepdims=True)).sum(-1, keepdims=True))
+
+    def check(got, lg, temps, top_ps, u, k, at_temperature):
+        for b in range(B):
+            pad = np.concatenate([lg[b:b + 1], np.tile(lg[:1], (512, 1))])
+            want = _run_sampler(pad, float(temps[b]), float(top_ps[b]), np.concatenate([u[b:b + 1], np.zeros(512, np.float32)]))[0][0]
+            assert got["tokens"].reshape(-1)[b] == want, b
+            scale = np.float32(1.0) / np.float32(temps[b]) if at_temperature and temps[b] > 0 else 1.0
+            lp = log_softmax(lg[b].astype(np.float64) * scale)
+            np.testing.assert_allclose(got["logprobs"].reshape(-1)[b], lp[want], rtol=1e-5, atol=1e-5)
+            if k:
+                order = np.lexsort((np.arange(vocab), -lg[b]))[:k]
+                assert np.array_equal(got["top_ids"].reshape(B, k)[b], order)
+                np.testing.assert_allclose(got["top_logprobs"].reshape(B, k)[b], lp[order], rtol=1e-5, atol=1e-5)
+    u = rng.random(B).astype(np.float32)
+    for temp, top_p in ((0.0, 1.0), (0.7, 0.9), (1.0, 1.0), (6.0, 0.95)):
+        for k in (0, 5):
+            for b in (None, bias):
+                for at_temperature in (False, True):
+                    kv.reset()
+                    args = SampleArgs(temp=temp, top_p=top_p, uniforms=u, logit_bias=b, top_logprobs=k, logprobs_at_temperature=at_temperature)
+                    check(eng.decode_sample(kv, toks, args), biased(b), [temp] * B, [top_p] * B, u, k, at_temperature)
+    temps, top_ps = np.array([0.0, 0.7, 1.0, 0.0, 5.0, 0.3], np.float32), np.array([1.0, 0.9, 1.0, 0.5, 0.99, 0.2], np.float32)
+    for t, p in ((temps, top_ps), (temps * 0.0, top_ps)):
+        for k in (0, 5):
+            for at_temperature in (False, True):
+                kv.reset()
+                args = SampleArgs(uniforms=u, logit_bias=bias, top_logprobs=k, logprobs_at_temperature=at_temperature)
+                args.set_row_params(t, p)
+                check(eng.decode_sample(kv, toks, args), biased(bias), t, p, u, k, at_temperature)
+    targets = rng.integers(0, vocab, (B, 1)).astype(np.int32)
+    targets[2], targets[4] = -1, edges[3]
+    for temp in (0.0, 0.7, 1.0):
+        for k in (0, 5):
+            kv.reset()
+            got = eng.score_tokens(kv, toks, targets, SampleArgs(temp=temp, logit_bias=bias, top_logprobs=k, logprobs_at_temperature=True))
+            lp = log_softmax(biased(bias).astype(np.float64) * (np.float32(1.0) / np.float32(temp) if temp else 1.0))
+            want = np.where(targets[:, 0] < 0, 0.0, lp[np.arange(B), np.maximum(targets[:, 0], 0)])
+            np.testing.assert_allclose(got["logprobs"].reshape(-1), want, rtol=1e-5, atol=1e-5)
+            if k:
+                np.testing.assert_allclose(got["top_logprobs"].reshape(B, k), -np.sort(-lp, -1)[:, :k], rtol=1e-5, atol=1e-5)
+    kv.close()
+    eng.close()
