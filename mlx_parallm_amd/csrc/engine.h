@@ -208,6 +208,7 @@ struct mi_engine {
   // int4 output linears that read their x in fragment order (gemm_q4.hip): the attention leaves it there [128][heads x head_dim]
   void* o_frag = nullptr;
   void* act_frag = nullptr;        // .. and the gated unit's for the down projection [128][ff]
+  bool frag_failed = false;
   bool opt_attn_frag = true;
   bool opt_mixed_attn = true;      // mixed steps: a chunk's attention in the decoding rows' launch
   // ---- layer-list models (engine_layers.hip)

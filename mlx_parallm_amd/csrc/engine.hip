@@ -199,9 +199,9 @@ int ensure_workspace(mi_engine* e, size_t rows, size_t logit_rows, int B) {
     e->d_logprob = (float*)(e->d_next + B);
     e->d_prob0 = (float*)(e->d_next + 2 * B);
     MI_HIP(dev_malloc(e, &e->d_rowstats, 2 * B * sizeof(float)));
-    if (e->d_sample == nullptr || e->maxB < SAMPLE_SPLIT_ROWS) {
-      hipFree(e->d_sample);
-      MI_HIP(dev_malloc(e, &e->d_sample, sample_ws_bytes(B)));
+    if (d.vocab_size >= SAMPLE_SPLIT_VOCAB && (e->d_sample == nullptr || e->maxB < SAMPLE_SPLIT_ROWS)) {      // (without it one workgroup draws a row)
+      hipFree(e->d_sample); e->d_sample = nullptr;
+      if (hipMalloc(&e->d_sample, sample_ws_bytes(B)) != hipSuccess) { (void)hipGetLastError(); e->d_sample = nullptr; }
     }
     MI_HIP(dev_malloc(e, &e->d_uniforms, B * sizeof(float)));
     MI_HIP(dev_malloc(e, &e->d_topk_ids, (size_t)B * MI_MAX_TOP_LOGPROBS * sizeof(int32_t)));
@@ -801,8 +801,9 @@ int frag_mt(const mi_engine* e, const FusedLinear& f, const GemvCall& c, size_t 
   if ((e->cur_L != 1 && !e->opt_short_prefill_skinny) || f.W.lora_b[0] != nullptr || f.W.lora_b[1] != nullptr || getenv("MI_SKINNY_DECODE_MAX") != nullptr) return 0;
   return gemm_skinny_supported(f.W, c, rows) ? gemm_q4_frag_mt(f.W, c, rows) : 0;
 }
+// (Worth a launch a layer, not the kept codes: memory for it is asked for once, and nothing goes for it)
 bool frag_buffer(mi_engine* e, void** p, int K) {
-  if (*p == nullptr && dev_malloc(e, p, (size_t)128 * K * 2) != hipSuccess) { (void)hipGetLastError(); *p = nullptr; }
+  if (*p == nullptr && !e->frag_failed && hipMalloc(p, (size_t)128 * K * 2) != hipSuccess) { (void)hipGetLastError(); *p = nullptr; e->frag_failed = true; }
   return *p != nullptr;
 }
 // The attention in front of the output linear `co`.  Whole calls, decode steps of 24 rows x 705 keys (4096 wide) 6.23 -> 6.11 ms, 64 x 513 (5120) 17.19 -> 16.97, 100 x 257 11.77 -> 11.74;

@@ -1074,10 +1074,10 @@ int forward_segments(mi_engine* e, mi_kv* kv, const int32_t* rows, const int32_t
     SideNormCall sn{R, tok, e->side_embed, d.num_layers * d.side_dim, li * d.side_dim, d.vocab_size, l.side_gate, l.side_proj_t, l.side_proj_p,
                     l.side_norm.p, d.rms_norm_eps, d.side_dim, d.hidden_size, e->wp, norm_of(ri + 1), e->x32, e->hn, act};
     const int slices = post || pre || both || !e->opt_skinny_gemm || e->opt_force_v1 ? 0 : gemv_side_slices(l.out.f.W, act, d.side_dim, R);
-    const bool joined = slices > 0 && side_join_supported(sn, slices, l.out.N / 16);
+    const size_t sums = (size_t)slices * R * e->wp, shares = (size_t)slices * (l.out.N / 16) * R * 64;
+    bool joined = slices > 0 && side_join_supported(sn, slices, l.out.N / 16);
+    if (joined && grow(e, (void**)&e->side_part, &e->side_part_cap, (sums + shares) * sizeof(float)) != MI_OK) { (void)hipGetLastError(); joined = false; }
     if (joined) {                              // a decode step's rows: two launches that share the gate's work
-      const size_t sums = (size_t)slices * R * e->wp, shares = (size_t)slices * (l.out.N / 16) * R * 64;
-      MI_TRY(grow(e, (void**)&e->side_part, &e->side_part_cap, (sums + shares) * sizeof(float)));
       { Prof pr(e, "gemv_out");
         MI_TRY(launch_gemv_side(l.out.f.W, SideOutCall{e->cat, l.n_cat, R, e->x32, e->wp, l.side_gate, d.side_dim, e->side_part, e->side_part + sums, act}, st)); }
       Prof pr(e, "side");
