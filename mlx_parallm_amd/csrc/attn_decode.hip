@@ -1172,11 +1172,11 @@ int attention_decode_splits(int ncu, int groups, int keys, bool f32) {
   return pick;
 }
 
-// The paged 16-bit caches with head_dim 128 have the kernel (the server's).  A workgroup of it has a CU to itself, so a chunk of many tiles stays a launch of its own,
+// The paged 16-bit caches with head_dim 128 have the kernel (the server's), where a chunk's own launch would be the LDS-DMA kernel (attention_prefill_frag).  A workgroup of it has a CU to itself, so a chunk of many tiles stays a launch of its own,
 // three workgroups a CU.
 bool attention_mixed_takes(const AttnDecodeCall& c, const AttnCall& p, int ncu) {
   const AttnShape& s = c.s;
-  return attention_decode_supported(s) && attention_prefill_supported(p.s) && s.act != MI_F32 && p.s.act == s.act && s.D == 128 && p.s.D == 128 && p.s.Hq == s.Hq && p.s.Hkv == s.Hkv &&
+  return attention_decode_supported(s) && attention_prefill_frag(p.s) && p.s.act == s.act && s.D == 128 && p.s.D == 128 && p.s.Hq == s.Hq && p.s.Hkv == s.Hkv &&
          p.s.B == 1 && s.btab != nullptr && p.s.btab != nullptr && c.variant == 0 && p.variant == 0 && (c.q_norm_w != nullptr) == (c.k_norm_w != nullptr) &&
          2 * attention_prefill_tiles(p.s) * p.nsplit <= ncu;
 }

@@ -1303,6 +1303,32 @@ def test_a_mixed_step_s_attention_in_one_launch_equals_two_launches(tmp_path, dt
     eng.close()
 
 
+def test_the_switch_of_the_prefill_kernels_reaches_mixed_steps(tmp_path, monkeypatch):
+    """MI_ATTN_PREFILL_DMA=0: a chunk behind cached keys takes the register-staged kernel, which does not slice keys, in a mixed step's attention as in a launch of its own."""
+    from mlx_parallm_amd.tiny_model import build_tiny_model
+
+    build_tiny_model(tmp_path, seed=9, vocab_size=512, dtype="bfloat16", quantize_model=False, hidden_size=128, layers=2, heads=5, kv_heads=1, head_dim=128, intermediate_size=128,
+                     norm_jitter=0.2, with_tokenizer=False)
+    eng = utils.load_model(str(tmp_path), max_positions=2048).engine
+    rng = np.random.default_rng(2)
+    prompts, chunk = [rng.integers(0, 512, n).astype(np.int32) for n in (50, 900, 700)], rng.integers(0, 512, 32).astype(np.int32)
+
+    def step(dma, together):
+        monkeypatch.setenv("MI_ATTN_PREFILL_DMA", dma)
+        eng.set_option("mixed_attention", together)
+        kv = eng.new_paged_kv(3, block_tokens=16, max_tokens_per_row=2048)
+        for r, p in enumerate(prompts):
+            eng.forward_segments(kv, [r], [p])
+        out = eng.forward_segments(kv, [0, 1, 2], [chunk[:1], chunk[1:2], chunk], [0, 1, 33])
+        kv.close()
+        return out
+    staged = step("0", 0)
+    assert not np.array_equal(staged[2], step("1", 0)[2])        # (keys in slices: another order of sums)
+    assert np.array_equal(step("0", 1), staged) and np.array_equal(step("1", 1), step("1", 0))
+    eng.set_option("mixed_attention", 1)
+    eng.close()
+
+
 @pytest.mark.parametrize("dtype,arch,heads,kv_heads,hd", [("bfloat16", "qwen3", 5, 1, 128), ("float16", "llama", 8, 8, 64), ("bfloat16", "llama", 16, 4, 32)])
 def test_rows_that_a_launch_leaves_prepared_for_the_next_int4_linear(tmp_path, dtype, arch, heads, kv_heads, hd):
     """Decode steps and mixed steps of 17 to 128 rows (every number of row tiles and slabs) of an int4 model: the attention's rows in the output linear's order
