@@ -1004,7 +1004,8 @@ int launch_mixed_g(const AttnDecodeCall& c, const AttnCall& p, hipStream_t st) {
   auto kern = attn_mixed_kernel<T, D, G, NORM>;
   constexpr size_t lds = std::max(attn_mfma_lds_bytes<G, D, 2, 8>(), prefill::attn_prefill_dma_lds<D>());
   const int tiles = (p.s.L + prefill::QT - 1) / prefill::QT, chunk_wgs = attention_prefill_tiles(p.s) * p.nsplit;
-  MI_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  static std::atomic<bool> granted[64];
+  MI_TRY(grant_lds((const void*)kern, lds, granted));
   hipLaunchKernelGGL(kern, dim3(chunk_wgs + c.nsplit * c.s.B * c.s.Hkv), dim3(512), lds, st, c, p, tiles, chunk_wgs);
   MI_HIP(hipGetLastError());
   return MI_OK;

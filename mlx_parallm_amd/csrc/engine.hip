@@ -797,8 +797,9 @@ int choose_nsplit(const mi_kv* kv, int B, int Hkv, int L, const int32_t* rows = 
 // Does a linear of `rows` rows take its x from the launch in front as gemm_q4.hip multiplies it, instead of by a preparation launch (4.8 us)?  -> the row tiles a slab, 0: no.
 // Where gemv_rows would have that kernel prepare it; an adapter reads the rows as they are.
 int frag_mt(const mi_engine* e, const FusedLinear& f, const GemvCall& c, size_t rows) {
-  if (!e->opt_attn_frag || !e->opt_skinny_gemm || e->opt_force_v1 || c.act == MI_F32 || rows < 17 || rows > 128) return 0;
-  if ((e->cur_L != 1 && !e->opt_short_prefill_skinny) || f.W.lora_b[0] != nullptr || f.W.lora_b[1] != nullptr || getenv("MI_SKINNY_DECODE_MAX") != nullptr) return 0;
+  static const bool limited = getenv("MI_SKINNY_DECODE_MAX") != nullptr;       // A/B (gemv_rows_on)
+  if (!e->opt_attn_frag || !e->opt_skinny_gemm || e->opt_force_v1 || c.act == MI_F32 || rows < 17 || rows > 128 || limited) return 0;
+  if ((e->cur_L != 1 && !e->opt_short_prefill_skinny) || f.W.lora_b[0] != nullptr || f.W.lora_b[1] != nullptr) return 0;
   return gemm_skinny_supported(f.W, c, rows) ? gemm_q4_frag_mt(f.W, c, rows) : 0;
 }
 // (Worth a launch a layer, not the kept codes: memory for it is asked for once, and nothing goes for it)

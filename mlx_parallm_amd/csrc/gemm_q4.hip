@@ -21,7 +21,6 @@
 #include <hip/hip_ext.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <type_traits>
 
@@ -798,13 +797,8 @@ Q4Plan q4_plan(const LinearW& W, const GemvCall& c, size_t rows) {
 template <typename AT, int MT, bool SW, int TN>
 int q4_launch_k(const Q4Params& p, int grid, hipStream_t st) {
   auto kern = q4_kernel<AT, MT, SW, TN>;
-  static std::atomic<bool> attr_done[64];
-  int dev = 0;
-  MI_HIP(hipGetDevice(&dev));
-  if (dev < 0 || dev >= 64 || !attr_done[dev].load(std::memory_order_acquire)) {
-    MI_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Q4_LDS));
-    if (dev >= 0 && dev < 64) attr_done[dev].store(true, std::memory_order_release);
-  }
+  static std::atomic<bool> granted[64];
+  MI_TRY(grant_lds((const void*)kern, Q4_LDS, granted));
   hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * 64), Q4_LDS, st, p);
   MI_HIP(hipGetLastError());
   return MI_OK;

@@ -1,8 +1,22 @@
 // kernels.h -- host-side launch interface of the HIP kernels (internal to the library).
 #pragma once
+#include <atomic>
+
 #include "common.h"
 
 namespace mi {
+
+// More than 64 KiB of LDS for a kernel, granted once: to the kernel object of the CURRENT device (one engine per GPU may live in one process: server --devices), and several
+// scheduler threads launch concurrently, so `done` is that kernel's own, a flag per device, set after the call
+inline int grant_lds(const void* kern, size_t bytes, std::atomic<bool> (&done)[64]) {
+  int dev = 0;
+  MI_HIP(hipGetDevice(&dev));
+  const bool known = dev >= 0 && dev < 64;
+  if (known && done[dev].load(std::memory_order_acquire)) return MI_OK;
+  MI_HIP(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+  if (known) done[dev].store(true, std::memory_order_release);
+  return MI_OK;
+}
 
 // The operands of the prefill GEMM on codes (repack.hip): the codes as 16-bit integers, the biases (of 16-bit rows: the largest parts first, of float32 rows: last), the scales
 struct Codes16 {

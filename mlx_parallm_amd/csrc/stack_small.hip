@@ -527,7 +527,8 @@ int launch_small_pack(const LinearW& W, bool big, uint32_t* words, float2* sb, h
 int launch_stack_small(const SmallStackCall& c, hipStream_t st) {
   if (!small_stack_shape(c.H, c.s.Hq, c.s.Hkv, c.s.D, c.I) || c.s.act != MI_F32 || c.s.kv != MI_F32 || c.s.L < 1) return fail(MI_ERR_UNSUPPORTED, "stack_small: shape / dtype not supported");
 #define GOP(K, DV, PG) do { auto kern = small_prompt_kernel<K, DV, PG>; \
-    MI_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)prompt_lds())); \
+    static std::atomic<bool> granted[64]; \
+    MI_TRY(grant_lds((const void*)kern, prompt_lds(), granted)); \
     hipLaunchKernelGGL(kern, dim3(c.s.B), dim3(NT), prompt_lds(), st, c); } while (0)
 #define GO(K, DV) do { if (c.s.L > 1) { if (c.s.btab) GOP(K, DV, true); else GOP(K, DV, false); } \
     else if (c.s.btab) hipLaunchKernelGGL((stack_small_kernel<K, DV, true>), dim3(c.s.B), dim3(NT), 0, st, c); \
