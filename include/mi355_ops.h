@@ -140,6 +140,12 @@ int mi_op_attention_decode(const mi_op_attn_shape* s, const void* qkv, void* kca
 /* splits that a decode step's attention is launched with: `groups` (rows x kv heads) whose rows have `keys` cached keys of kv_dtype, on
  * ncu compute units (no device needed) */
 int mi_op_attention_decode_splits(int ncu, int groups, int keys, int kv_dtype);
+/* row tiles a slab in which an int4 linear of a->M rows (17..128) takes its x as the launch in front of it left it, in the order that it multiplies; 0: it prepares x itself, or is
+ * another kernel's (no device needed) */
+int mi_op_gemm_q4_prepared(const mi_op_linear* w, const mi_op_gemv_args* a);
+/* 1: decoding rows (L == 1) and a chunk of another row's prompt (B == 1), its keys in `slices` workgroups, share one attention launch on paged caches and ncu compute units (no device
+ * needed) */
+int mi_op_attention_mixed(const mi_op_attn_shape* rows, const mi_op_attn_shape* chunk, int slices, int ncu);
 /* 1: logits (rounded = 0) or layer 0's rounded q|k|v (1) of `rows` rows of float32 activations go to the tile GEMM, 0: 32 rows at a time to the
  * streaming kernel.  codes: int4 weights too small for the tile GEMM on codes (the others: mi_op_gemm_quant_route), hilo: an
  * f16 matrix through its [hi | lo] copy (no device needed) */

@@ -161,6 +161,8 @@ SIGNATURES = {
     "mi_op_attention_decode": (C.c_int, [C.POINTER(OpAttnShape), _P, _P, _P, _P, _P, _P, C.c_float, _P, _P, _P, C.c_float,
                                          C.c_int, C.c_int, _P, _P, C.c_int, C.c_int, C.POINTER(C.c_float)]),
     "mi_op_attention_decode_splits": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int]),
+    "mi_op_gemm_q4_prepared": (C.c_int, [C.POINTER(OpLinear), C.POINTER(OpGemvArgs)]),
+    "mi_op_attention_mixed": (C.c_int, [C.POINTER(OpAttnShape), C.POINTER(OpAttnShape), C.c_int, C.c_int]),
     "mi_op_gemm_prefill_pays": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int]),
     "mi_op_sample": (C.c_int, [_P, C.c_int, C.c_int, C.c_float, C.c_float, _P, C.c_int, _P, _P, _P, _P, _P, _P]),
 }

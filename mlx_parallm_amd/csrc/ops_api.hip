@@ -310,6 +310,23 @@ int mi_op_attention_decode_splits(int ncu, int groups, int keys, int kv_dtype) {
   return attention_decode_splits(ncu, groups, keys, kv_dtype == MI_F32);
 }
 
+int mi_op_gemm_q4_prepared(const mi_op_linear* w, const mi_op_gemv_args* a) {
+  if (!w || !a || a->M < 1) return fail(MI_ERR_INVALID, "mi_op_gemm_q4_prepared: arguments");
+  const LinearW W = to_linear(w);
+  const GemvCall c = to_call(a);
+  return gemm_skinny_supported(W, c, (size_t)c.M) ? gemm_q4_frag_mt(W, c, (size_t)c.M) : 0;
+}
+
+int mi_op_attention_mixed(const mi_op_attn_shape* rows, const mi_op_attn_shape* chunk, int slices, int ncu) {
+  if (!rows || !chunk || slices < 1 || ncu < 1) return fail(MI_ERR_INVALID, "mi_op_attention_mixed: arguments");
+  static const int32_t table = 0;
+  AttnDecodeCall c{};
+  c.s = to_shape(rows); c.s.btab = &table;
+  AttnCall p{};
+  p.s = to_shape(chunk); p.s.btab = &table; p.nsplit = slices;
+  return attention_mixed_takes(c, p, ncu) ? 1 : 0;
+}
+
 int mi_op_gemm_prefill_pays(int codes, int hilo, int rounded, int rows) {
   return rows > 0 && gemm_prefill_pays(codes != 0, hilo != 0, rounded != 0, (size_t)rows) ? 1 : 0;
 }

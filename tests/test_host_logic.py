@@ -459,3 +459,46 @@ def test_prefill_attention_slices(f32):
         got = [slices(B, L_, k, Hq, Hkv) for k in range(L_, 8192, 7)]
         assert got == sorted(got) and 1 <= got[0] and got[-1] <= 16
         assert all(n == 1 or 2 * n <= (k + 31) // 32 for n, k in zip(got, range(L_, 8192, 7)))
+
+
+def test_which_int4_linears_take_their_rows_prepared():
+    """The shapes of test_gpu_engine.py's test of prepared rows are such linears at every number of rows there (each of its row tiles a slab), and where the rule ends: rows, short K
+    without a norm, more than one round of workgroups behind a long K, a norm of its own."""
+    import ctypes as C
+
+    from mlx_parallm_amd import _lib as L
+
+    def prepared(rows, N, K, act="bfloat16", epi=L.EPI_RESID, pro=0):
+        ol, a = L.OpLinear(), L.OpGemvArgs()
+        ol.wk, ol.N, ol.K, ol.group, ol.layout = L.WK["q4_bf16" if act == "bfloat16" else "q4_f16"], N, K, 64, 1
+        a.M, a.act, a.ldx, a.ldo, a.epi, a.pro = rows, L.MI_BF16 if act == "bfloat16" else L.MI_F16, K, N, epi, pro
+        return L.lib().mi_op_gemm_q4_prepared(C.byref(ol), C.byref(a))
+
+    for act, K in (("bfloat16", 640), ("float16", 512), ("bfloat16", 512)):
+        assert [prepared(n, 256, K, act) for n in (17, 33, 64, 65, 97, 128)] == [2, 3, 4, 3, 4, 4]
+        assert all(prepared(n, 256, K, act) > 0 for n in (12 + 16, 30 + 33, 3 + 90))
+    assert all(prepared(n, 256, 640) > 0 for n in (17, 28, 33, 63, 64, 65, 93, 97, 128))          # the down projection there
+    assert prepared(16, 256, 640) == prepared(129, 256, 640) == prepared(64, 256, 384) == prepared(64, 256, 640, pro=L.PRO_NORM) == 0
+    assert prepared(64, 4096, 14336) == 4 and prepared(64, 5120, 17408) == 4 and prepared(100, 5120, 17408) == 0
+
+
+def test_which_chunks_share_the_attention_launch_of_a_mixed_step():
+    """The first chunks of test_gpu_engine.py's mixed steps do at the numbers of keys there (its second one of two has a launch of its own), a chunk of many tiles and other caches do not."""
+    import ctypes as C
+
+    from mlx_parallm_amd import _lib as L
+
+    def shape(B, n, heads, kv_heads, hd=128, act=L.MI_BF16, kv=None):
+        s = L.OpAttnShape()
+        s.B, s.L, s.Hq, s.Hkv, s.D, s.act, s.kv, s.rnd, s.cap = B, n, heads, kv_heads, hd, act, act if kv is None else kv, 0, 4096
+        return s
+
+    def shared(rows, chunk, heads, kv_heads, keys, **kw):
+        r, c = shape(rows, 1, heads, kv_heads, **kw), shape(1, chunk, heads, kv_heads, **kw)
+        return L.lib().mi_op_attention_mixed(C.byref(r), C.byref(c), max(1, L.lib().mi_op_attention_prefill_slices(C.byref(c), keys, 256)), 256)
+
+    for rows, chunk, heads, kv_heads, act in ((3, 32, 10, 2, L.MI_BF16), (40, 16, 4, 1, L.MI_F16), (1, 17, 8, 1, L.MI_BF16), (2, 40, 2, 1, L.MI_F16)):
+        assert all(shared(rows, chunk, heads, kv_heads, chunk * k, act=act) == 1 for k in (1, 2, 3, 4)), (rows, chunk)
+    assert [shared(5, 200, 3, 3, k) for k in (200, 800)] == [1, 0]          # (39 tiles; in slices more workgroups than half of the compute units)
+    assert shared(31, 32, 40, 8, 672) == 1 and shared(31, 512, 40, 8, 1152) == 0
+    assert shared(3, 32, 8, 2, 64, act=L.MI_F32) == shared(3, 32, 8, 2, 64, hd=64) == shared(3, 32, 6, 2, 64) == shared(3, 1, 8, 2, 64) == 0
