@@ -1522,7 +1522,7 @@ def test_an_engine_s_sampler_over_several_workgroups(tmp_path, vocab):
     """Every argument of a step on vocabularies whose rows several workgroups take, against one workgroup per row (more rows than the others serve) and float64: biases up to the
     parts' edges, log-probabilities at temperature, rows with a temperature of their own next to greedy ones, given tokens and none."""
     from mlx_parallm_amd.tiny_model import build_tiny_model
-    from tests.test_gpu_kernels import _run_sampler
+    from test_gpu_kernels import _run_sampler
 
     build_tiny_model(tmp_path, seed=3, vocab_size=vocab, dtype="bfloat16", quantize_model=False, hidden_size=64, layers=1, heads=4, kv_heads=4, intermediate_size=128, head_dim=16,
                      with_tokenizer=False)
@@ -1585,4 +1585,84 @@ def test_an_engine_s_sampler_over_several_workgroups(tmp_path, vocab):
             if k:
                 np.testing.assert_allclose(got["top_logprobs"].reshape(B, k), -np.sort(-lp, -1)[:, :k], rtol=1e-5, atol=1e-5)
     kv.close()
+    eng.close()
+
+
+@pytest.mark.parametrize("dtype,bits,group", [("float32", 0, 64), ("bfloat16", 0, 64), ("float16", 0, 64), ("bfloat16", 4, 64), ("float32", 4, 32), ("float16", 8, 64)])
+@pytest.mark.parametrize("heads,kv_heads,hd,ff", [(4, 2, 16, 128), (2, 1, 32, 64)])
+def test_a_small_model_s_kernels_against_exact_sums(tmp_path, dtype, bits, group, heads, kv_heads, hd, ff):
+    """A prompt of two tokens and two decode steps in one launch each, against the oracle, whose sums are exact.  In the 16-bit models' first layer a rounding falls the other way in one
+    token of ten at most (400 values of 11 bits, sums off by 1e-7), so the better rows are as close as float32 sums are; without the rounding of q|k|v -- planted in the oracle -- no row is."""
+    from mlx_parallm_amd.tiny_model import build_tiny_model
+
+    cfg = build_tiny_model(tmp_path, seed=5, vocab_size=512, dtype=dtype, quantize_model=bits > 0, q_bits=bits or 4, q_group_size=group, hidden_size=64, layers=3, heads=heads,
+                           kv_heads=kv_heads, intermediate_size=ff, head_dim=hd, norm_jitter=0.2, with_tokenizer=False)
+    eng = utils.load_model(str(tmp_path), max_positions=64).engine
+    rng, B = np.random.default_rng(3), 16
+    toks = rng.integers(0, cfg["vocab_size"], (B, 4)).astype(np.int32)
+
+    def oracle(planted):
+        ref = ref_generate.load(str(tmp_path), max_pos=64)
+        for p in "qkv" if planted else "":
+            ref.w[f"model.layers.0.self_attn.{p}_proj"].dtype = "float32"
+        cache = ref.make_cache(B, paged=True)
+        return [ref(toks[:, a:b], cache=cache)[:, -1] for a, b in ((0, 2), (2, 3), (3, 4))]
+    kv = eng.new_kv(B, capacity=32, kv_dtype="float32")
+    got = [eng.forward(toks[:, a:b], kv) for a, b in ((0, 2), (2, 3), (3, 4))]
+    eng.set_option("small_stack", 0)
+    kv.reset()
+    assert not np.array_equal(got[0], eng.forward(toks[:, :2], kv)) and not np.array_equal(got[1], eng.forward(toks[:, 2:3], kv))
+    eng.close()
+
+    def off(want):
+        return [np.sort(np.linalg.norm(g - w, axis=-1) / np.linalg.norm(w, axis=-1)) for g, w in zip(got, want)]
+    for d in off(oracle(False)):
+        assert d[B // 4] <= 1e-5 and (dtype != "float32" or d[-1] <= 1e-5) and d[-1] <= 2e-2, d
+    if dtype != "float32":
+        for d in off(oracle(True)):
+            assert d[0] > 3e-5 and d[B // 4] > 1e-4, d
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float16"])
+@pytest.mark.parametrize("paged", [False, True])
+def test_a_small_model_s_caches_with_infinities_and_what_they_leave_behind(tmp_path, dtype, paged):
+    """A token whose keys and values are no numbers: the launches' finite outputs are finite and their others are not, the rows next to it keep their bits, and so does what is cached
+    later in its place."""
+    from safetensors.torch import load_file
+
+    from mlx_parallm_amd.engine import Engine
+    from mlx_parallm_amd.tiny_model import build_tiny_model
+
+    cfg = build_tiny_model(tmp_path, seed=5, vocab_size=512, dtype=dtype, quantize_model=False, hidden_size=64, layers=3, heads=4, kv_heads=4, intermediate_size=128, head_dim=16,
+                           tie_word_embeddings=False, norm_jitter=0.2, with_tokenizer=False)
+    weights = load_file(str(next(tmp_path.glob("*.safetensors"))))
+    weights["model.embed_tokens.weight"][7] = float("inf")
+    eng = Engine(cfg, device=0, max_positions=256, act_dtype=dtype)
+    eng.load_tensors(weights.items())
+    eng.finalize()
+    rng = np.random.default_rng(3)
+    good = rng.integers(8, 512, (3, 20)).astype(np.int32)
+    bad = good.copy()
+    bad[1, 5] = 7
+
+    def cache():
+        return eng.new_paged_kv(3, block_tokens=16, n_blocks=8, max_tokens_per_row=32, kv_dtype="float32") if paged else eng.new_kv(3, capacity=32, kv_dtype="float32")
+    clean, outs = cache(), []
+    want = [eng.forward(good[:, :18], clean), eng.forward(good[:, 18:19], clean), eng.forward(good[:, 19:], clean)]
+    clean.close()
+    for on in (1, 0):
+        eng.set_option("small_stack", on)
+        kv = cache()
+        outs.append([eng.forward(bad[:, :18], kv), eng.forward(bad[:, 18:19], kv)])
+        if on:
+            for r in range(3):
+                kv.reset_row(r)
+            order = [1, 2, 0]                        # (every row in another's place, or on another's blocks)
+            again = [eng.forward(good[order, :18], kv), eng.forward(good[order, 18:19], kv), eng.forward(good[order, 19:], kv)]
+            for a, w in zip(again, want):
+                assert np.isfinite(a).all() and np.array_equal(a, w[order])
+        kv.close()
+    for a, b, w in zip(*outs, want):
+        assert np.array_equal(np.isfinite(a), np.isfinite(b)) and not np.isfinite(a[1]).any()
+        assert np.array_equal(a[[0, 2]], w[[0, 2]])
     eng.close()
