@@ -889,7 +889,7 @@ __global__ __launch_bounds__(SK_NW * 64, (QB == 4 || (QB == 8 && MT >= 3) || MT 
   skinny_body<AT, QB, MT, SWIGLU, X32, AT, false>(p);
 }
 template <int QB, int MT, bool SWIGLU, typename ST>
-__global__ __launch_bounds__(SK_NW * 64, (QB == 4 || (QB == 8 && MT >= 3) || MT >= 5 || QB == 8 || (MT == 2 && SWIGLU)) ? 2 : 4) void skinny_centred_kernel(const SkinnyParams p) {
+__global__ __launch_bounds__(SK_NW * 64, 2) void skinny_centred_kernel(const SkinnyParams p) {
   skinny_body<bf16, QB, MT, SWIGLU, true, ST, true>(p);
 }
 

@@ -1,4 +1,4 @@
-// stack_small.hip -- a decode step of a small model, all layers in ONE launch (float32 activations: float32 models, and the float32-cache mode).
+// stack_small.hip -- a decode step or a prompt of a small model, all layers in ONE launch (float32 activations: float32 models, and the float32-cache mode).
 //
 // A model of some 10^4 weights a layer has nothing to stream: its step is the launches, six a layer of 3 to 5 us each (64 wide, eight layers, 4-bit:
 // 200 us a token).  A row needs no other row, so one workgroup walks all layers of its row: every matrix is spread over the 512 threads, in registers, and a thread
@@ -6,7 +6,8 @@
 // left is a chain of five barriers a layer and the instructions between them (one CU's): 43 us that step, the whole token 250 -> 76.  On the way, us: 14
 // barriers, a thread per number 72; five, and sizes of the split known at run time alone 61; no division in the loop 51; the split fixed 43.
 // The same arithmetic as the kernels it replaces: weights as scale * code + bias with two roundings, products and sums in float32, layer 0 up to its attention
-// rounded to the model's type (`rnd0`).  Prompts: small_prompt_kernel.  The limits (64 wide, 256 outputs of q|k|v and of gate|up, 128 columns of o and down) are the registers'; 256 keys because a
+// rounded to the model's type (`rnd0`).  Prompts: small_prompt_kernel.  The limits (64 wide, 256 outputs of q|k|v and of gate|up, 128 columns of o and down) are
+// those at which a layer's float32 weights fill the threads' registers (222 to 240 of 256); codes take 84, and no model of codes alone that is wider has been tried.  256 keys because a
 // row's keys are one workgroup's: longer ones take the launches, whose attention splits them.
 #include <type_traits>
 
