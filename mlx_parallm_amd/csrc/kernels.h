@@ -407,8 +407,8 @@ struct SmallStackCall {
   float* kcache; float* vcache; size_t layer_elems;
   int32_t* offsets;              // [cache row]
   const float* cos_tab; const float* sin_tab;
-  int upto;                      // rows behind more cached keys than this are left alone (SMALL_MAX_KEYS: there are none)
-  bool advance;                  // offsets += L
+  int upto;                      // prompts: rows behind more cached keys than this are left alone (SMALL_MAX_KEYS: there are none)
+  bool advance;                  // prompts: offsets += L (a decode step advances every row)
 };
 bool small_stack_fits(const LinearW& W, bool big);       // big: q|k|v, gate|up
 bool small_stack_shape(int H, int heads, int kv_heads, int D, int I);

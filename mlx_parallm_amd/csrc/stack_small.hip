@@ -191,7 +191,6 @@ __global__ __launch_bounds__(NT) void stack_small_kernel(SmallStackCall c) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), b = blockIdx.x;
   const int H = c.H, Hq = c.s.Hq, Hkv = c.s.Hkv, G = Hq / Hkv, nq = Hq * D, nkv = Hkv * D, I = c.I;
   const int kb = c.s.rows ? c.s.rows[b] : b, pos = c.offsets[kb];
-  if (c.upto < SMALL_MAX_KEYS && pos > c.upto) return;          // (uniform)
   const Part pq = part_of<true>(nq + 2 * nkv, H / PER, c.group), po = part_of<false>(H, nq / PER, c.group), pg = part_of<true>(2 * I, H / PER, c.group), pd = part_of<false>(H, I / PER, c.group);
   Regs<KIND, true> rq, rg;
   Regs<KIND, false> ro, rd;
@@ -334,7 +333,7 @@ __global__ __launch_bounds__(NT) void stack_small_kernel(SmallStackCall c) {
   }
   if (wave == 0) {
     if (lane < H) c.h[(size_t)b * H + lane] = x;
-    if (lane == 0 && c.advance) c.offsets[kb] = pos + 1;      // (nobody else reads it in this step)
+    if (lane == 0) c.offsets[kb] = pos + 1;           // (nobody else reads it in this step)
   }
 }
 
