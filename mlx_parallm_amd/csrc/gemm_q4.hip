@@ -741,12 +741,15 @@ thread_local bool q4_forced = false;                             // .. and whate
 // at 65 rows 36 / 33, 128 43 / 41; with a norm (to be added to the other side) or a SwiGLU 10240 x 5120 16 / 17, 25 / 25, 36 / 45; 10240 x 8192 22 / 22, 35 / 34, 51 / 59; 16128 x 8192
 // 23 / 27, 36 / 44, 68 / 72; 16128 x 4096 15 / 18, 23 / 28, 41 / 38 (four rounds: behind by less than the norm); SwiGLU 14336 x 4096 15 / 19, 22 / 30, 39 / 41, 16128 x 8192 23 / 28, 36 / 43, 67 / 68.
 // A longer K, one round: 4096 x 10240 15 / 19, 22 / 28, 27 / 35; 3072 x 11008 16 / 19, 24 / 27, 26 / 33; 4096 x 14336 20 / 22, 29 / 33, 35 / 43; 5120 x 17408 22 / 26, 34 / 40, in two rounds at
-// 128 rows 67 / 62.  So: one round of workgroups whatever K, and up to K = 8192 any number where a norm launch goes with the other kernel. A short K without a norm: the preparation is a launch of its own, 256 x 128 5.5 / 4.9, 6.0 / 5.4, 6.1 / 5.4;
+// 128 rows 67 / 62.  Few columns behind a long K leave CUs idle, which the other kernel splits K over (us at 17 / 64 / 128 rows; where the launch in front
+// leaves x prepared the first is 4.8 less): 4096 x 22016 27 / 25, 40 / 38, 46 / 57, x 28672 33 / 29, 51 / 43, 58 / 68; 3072 x 17408 22 / 21, 33 / 31, 35 / 41, x 22016 26 / 23, 40 / 35, 43 / 49; 2048 x 10240 15 / 17, 22 / 23, 24 / 28,
+// x 17408 21 / 20, 32 / 29, 35 / 34, x 22016 26 / 22, 40 / 32, 42 / 38; 1024 x 8704 13 / 15, 20 / 18, 21 / 24, x 17408 22 / 19, 33 / 22, 35 / 29.
+// So: one round of workgroups up to K = 20480 or 6 N, and up to K = 8192 any number where a norm launch goes with the other kernel. A short K without a norm: the preparation is a launch of its own, 256 x 128 5.5 / 4.9, 6.0 / 5.4, 6.1 / 5.4;
 // 512 x 256 5.8 / 5.7, 6.2 / 5.8, 6.3 / 5.8; 1024 x 512 6.0 / 6.5, 6.6 / 6.6, 6.7 / 6.7.  So from K = 512.
 bool q4_rows_ahead(const LinearW& W, const GemvCall& c, size_t rows) {
   const long units = c.epi == EPI_SWIGLU ? c.pair_offset / 16 : (W.N / 16 + RT - 1) / RT, slabs = (long)((rows + 63) / 64);
   const bool one = units * slabs <= gemv_cu_count();
-  return (W.K <= 8192 || one) && (c.pro == PRO_NORM || (W.K >= 512 && (c.epi == EPI_SWIGLU || one)));
+  return (W.K <= 8192 || (one && W.K <= std::max(20480, 6 * W.N))) && (c.pro == PRO_NORM || (W.K >= 512 && (c.epi == EPI_SWIGLU || one)));
 }
 bool q4_rows(const LinearW& W, const GemvCall& c) { return q4_force_rows > 0 || (!q4_forced && W.N / 16 < GEMM_Q4_MIN_TILES); }
 

@@ -463,7 +463,7 @@ def test_prefill_attention_slices(f32):
 
 def test_which_int4_linears_take_their_rows_prepared():
     """The shapes of test_gpu_engine.py's test of prepared rows are such linears at every number of rows there (each of its row tiles a slab), and where the rule ends: rows, short K
-    without a norm, more than one round of workgroups behind a long K, a norm of its own."""
+    without a norm, more than one round of workgroups behind a long K, few columns behind a long K, a norm of its own."""
     import ctypes as C
 
     from mlx_parallm_amd import _lib as L
@@ -480,6 +480,7 @@ def test_which_int4_linears_take_their_rows_prepared():
     assert all(prepared(n, 256, 640) > 0 for n in (17, 28, 33, 63, 64, 65, 93, 97, 128))          # the down projection there
     assert prepared(16, 256, 640) == prepared(129, 256, 640) == prepared(64, 256, 384) == prepared(64, 256, 640, pro=L.PRO_NORM) == 0
     assert prepared(64, 4096, 14336) == 4 and prepared(64, 5120, 17408) == 4 and prepared(100, 5120, 17408) == 0
+    assert prepared(64, 2048, 20480) == 4 and prepared(64, 4096, 24576) == 4 and prepared(64, 2048, 20608) == prepared(17, 3072, 24576) == prepared(17, 4096, 24704) == 0
 
 
 def test_which_chunks_share_the_attention_launch_of_a_mixed_step():
