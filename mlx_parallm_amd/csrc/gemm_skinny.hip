@@ -1021,6 +1021,24 @@ static int skinny_min_rows() {
   return v;
 }
 
+// Small matrices that are centred here, up to 8 rows of float32 activations: the generic kernel (gemv_v1.hip) is one launch of 4 us with the norm in it, this one staging, three images of x and a
+// join.  us, generic / this one, int4 (int8 within 5 %), at 1 / 2 / 4 / 8 rows:
+//   no norm    512 x 512 4.3 / 7.2, 4.2 / 7.5, 3.9 / 7.8, 4.7 / 7.8; 256 x 768 5.8 / 7.2, 7.1 / 7.3, 7.6 / 7.6, 10.8 / 7.6; 1024 x 1024 5.8 / 7.4, 7.3 / 7.5, 7.8 / 8.0, 11.1 / 7.9;
+//              512 x 1536 6.7 / 8.0, 8.5 / 8.2; 2048 x 2048 8.2 / 9.4, 9.8 / 9.7; 1024 x 3072 10.0 / 9.6
+//   norm       768 x 128 5.1 / 4.8, 5.0 / 5.1, 6.5 / 5.7, 9.9 / 5.8; 1536 x 256 5.4 / 6.2, 5.4 / 6.5, 7.2 / 7.1, 11.0 / 7.1; 3072 x 512 5.7 / 8.5, 5.8 / 8.8, 7.9 / 9.5, 13.1 / 9.4;
+//              6144 x 1024 6.9 / 9.7, 10.0 / 10.0, 12.2 / 10.7; 4096 x 2048 9.6 / 9.1, 13.8 / 9.2; many columns of a short K 32000 x 128 6.4 / 4.9, 32000 x 512 11.0 / 6.8.  (A rounded
+//              call's norm is a launch of its own here, 4.8 more)
+// A float16 model's decode step, float32 caches, four layers, us: generic for all / this one for all / by this rule 512 wide 177 / 229 / 175 at one row, 219 / 248 / 209 at four; 1024 wide at one row
+// 227 / 246 / 217, at two 281 / 250 / 250; 128 wide 155 / 188 / 155, eight rows 213 / 206 / 187.
+bool gemm_skinny_behind(const LinearW& W, const GemvCall& c, size_t rows) {
+  const bool centred = W.wk == WK_Q4_F16 || W.wk == WK_Q8_F16 || (W.centred && c.epi != EPI_SWIGLU);
+  if (c.act != MI_F32 || !centred || rows > 8) return false;
+  const long size = (long)W.N * W.K;
+  const bool norm = c.pro == PRO_NORM;
+  if (W.K <= 512) return size <= (1l << 21) && (!norm || rows <= (W.K > 256 || c.rnd != RND_NONE ? 4u : 2u));
+  return size <= (1l << 23) && (norm ? W.K <= 1024 && rows == 1 : W.K <= 2048 && rows <= (W.K <= 1024 ? 4u : 1u));
+}
+
 bool gemm_skinny_supported(const LinearW& W, const GemvCall& c, size_t rows) {
   if (c.act == MI_F32 && (c.glu.kind != GLU_SILU || c.silu_cols > 0)) return false;
   if (c.force_v1 || W.layout != 1) return false;

@@ -201,6 +201,7 @@ int launch_gemv_side(const LinearW& W, const SideOutCall& c, hipStream_t st);
 // c.pro must be PRO_NONE; `ws` >= gemm_skinny_ws_bytes(), `ctr` >= gemm_skinny_groups() words that are zero between
 // launches (the kernel leaves them zero); ksplit = 0 lets the cost model choose.
 bool gemm_skinny_supported(const LinearW& W, const GemvCall& c, size_t rows);
+bool gemm_skinny_behind(const LinearW& W, const GemvCall& c, size_t rows);     // .. but the generic kernel is ahead of it
 size_t gemm_skinny_ws_bytes(const LinearW& W, const GemvCall& c, size_t rows);
 int gemm_skinny_groups(const LinearW& W, const GemvCall& c, size_t rows);
 int gemm_skinny_ksplit(const LinearW& W, const GemvCall& c, size_t rows);

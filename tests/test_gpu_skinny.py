@@ -487,3 +487,30 @@ def test_float32_activations_on_quantised_f16_weights(kind, M, N, K, ksplit, rnd
         gemm_skinny(ol, xd, M, "float32", epi=L.EPI_SWIGLU, out=out, ldo=I, pair_offset=I, ksplit=1)
         w2 = g / (1.0 + np.exp(-g)) * u                       # (the unit's slope in g is at most 1.1, times u)
         assert np.all(np.abs(host(out) - w2) <= 1.1 * (np.abs(u) * tol[:, :I] + np.abs(g) * tol[:, I:]) + 2.0 ** -21 * np.abs(w2) + 1e-7)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_small_quantised_f16_models_with_float32_caches_stay_on_the_generic_kernel(tmp_path, bits):
+    """Linears of 512 columns, at most 4 rows: the same bits with the streaming kernel switched off, in decode steps and prompts of as many rows.  Above, and wider ones, differ."""
+    from mlx_parallm_amd import utils
+    from mlx_parallm_amd.tiny_model import build_tiny_model
+
+    outs = {}
+    for hidden, ff in ((512, 512), (2048, 2048)):
+        d = tmp_path / str(hidden)
+        d.mkdir()
+        build_tiny_model(d, seed=5, vocab_size=512, dtype="float16", quantize_model=True, q_bits=bits, q_group_size=64, hidden_size=hidden, layers=2, heads=8, kv_heads=4, head_dim=64,
+                         intermediate_size=ff, with_tokenizer=False)
+        eng = utils.load_model(str(d), max_positions=64).engine
+        rng = np.random.default_rng(3)
+        for B, n in ((1, 1), (2, 1), (4, 1), (1, 3), (8, 1)):
+            toks = rng.integers(0, 512, (B, n)).astype(np.int32)
+            for on in (1, 0):
+                eng.set_option("skinny_gemm", on)
+                kv = eng.new_kv(B, capacity=32, kv_dtype="float32")
+                outs[hidden, B, n, on] = eng.forward(toks, kv)
+                kv.close()
+            a, b = outs[hidden, B, n, 1], outs[hidden, B, n, 0]
+            assert np.abs(a - b).max() <= 4e-3 * max(1.0, np.abs(b).max())      # (16-bit roundings of layer 0 that fall the other way)
+            assert np.array_equal(a, b) == (hidden == 512 and B * n <= 4), (hidden, B, n)
+        eng.close()
