@@ -885,7 +885,6 @@ int make_small_stack(mi_engine* e) {
 //   int8    one row 251 / 92, 262 / 209; 323 / 175, 335 / 298, 322 / 494   two rows 266 / 95, 339 / 212, 591 / 410; 310 / 176, 296 / 305, 351 / 488, 604 / 928   32 rows .., 841 / 217, 884 / 418; 875 / 498, 945 / 954
 // So small_prompt_keys prices both: here what a token and the start take, and 0.12 us a token and key (of 64 columns of heads; and three tokens' worth of every cached key, for its first
 // read), the launches 25 us a token or, on the matrix cores, by the number of rows.  Eight heads of 16, 4-bit, 128 tokens behind 32 keys 3114 / 3739: the launches'.
-// A decode step is ahead at every number of keys (behind 240 287 / 213).
 // -> the most cached keys that a row may have to be theirs; -1: none is.  A matter of the call's shape, so that a prompt's bits depend on its own keys and on nothing of its neighbours'
 int small_prompt_keys(bool mfma, int kind, int width, int B, int L) {            // in units of 0.12 us; width: heads x head_dim
   const int w = std::max(width, 64), R = B * L;
@@ -893,10 +892,19 @@ int small_prompt_keys(bool mfma, int kind, int width, int B, int L) {           
   const int token = kind == SMALL_CODES || mfma ? 45 : 87;
   return std::max(-1, (launches - 620 - token * L - (25 * L + L * L / 2) * w / 64) * 64 / (w * (L + 3)));
 }
+// A decode step is ahead at every number of keys (behind 240 287 / 213), unless its rows are several rounds of workgroups and the matrix cores would take them all at once: us by launches /
+// here, eight layers of bf16, 600 rows behind 1, 100 and 250 keys 763 / 229, 817 / 421, 871 / 847 (heads of 16), 720 / 234, 743 / 540, 799 / 1380 (two of 32, so two of the eight waves have
+// keys); 300 rows of these behind 250 673 / 701.  So (0.1 us a layer): 80 us by the launches, 5.4 and 0.1 a key of 16 columns a round here.
+int small_decode_keys(bool mfma, int D, int B) {
+  if (!mfma) return SMALL_MAX_KEYS - 1;
+  const int cus = gemv_cu_count(), rounds = (B + cus - 1) / cus;
+  return std::max(-1, (800 / rounds - 54) * 16 / D);
+}
 int small_stack_keys(const mi_engine* e, const mi_kv* kv, int act, int B, int L) {
   if (e->small_buf == nullptr || !e->opt_small_stack || e->opt_force_v1 || !e->opt_fused_attn || !e->prof_name.empty() || act != MI_F32 || kv->dtype != MI_F32) return -1;
   if (L > (e->small_mfma ? (B == 1 ? 16 : 32) : B == 1 ? 128 : SMALL_MAX_KEYS)) return -1;
-  return L == 1 ? SMALL_MAX_KEYS - 1 : std::min(SMALL_MAX_KEYS - L, small_prompt_keys(e->small_mfma, e->small_kind, e->d.num_heads * e->d.head_dim, B, L));
+  if (L == 1) return std::min(SMALL_MAX_KEYS - 1, small_decode_keys(e->small_mfma, e->d.head_dim, B));
+  return std::min(SMALL_MAX_KEYS - L, small_prompt_keys(e->small_mfma, e->small_kind, e->d.num_heads * e->d.head_dim, B, L));
 }
 
 // the model forward for B*L tokens already in e->d_tokens; logits of the requested rows end

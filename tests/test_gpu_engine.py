@@ -1666,3 +1666,26 @@ def test_a_small_model_s_caches_with_infinities_and_what_they_leave_behind(tmp_p
         assert np.array_equal(np.isfinite(a), np.isfinite(b)) and not np.isfinite(a[1]).any()
         assert np.array_equal(a[[0, 2]], w[[0, 2]])
     eng.close()
+
+
+def test_decode_steps_of_more_rows_than_compute_units_on_a_small_model(tmp_path):
+    """Several rounds of the small models' kernel behind many keys are the launches', whose matrix cores take all rows at once; behind few keys, and one round, the kernel's."""
+    from mlx_parallm_amd.tiny_model import build_tiny_model
+
+    build_tiny_model(tmp_path, seed=5, vocab_size=512, dtype="bfloat16", quantize_model=False, hidden_size=64, layers=2, heads=2, kv_heads=1, head_dim=32, intermediate_size=64,
+                     norm_jitter=0.2, with_tokenizer=False)
+    eng = utils.load_model(str(tmp_path), max_positions=300).engine
+    rng = np.random.default_rng(4)
+    for rows, keys, kernel in ((520, 90, True), (520, 140, False), (64, 240, True)):
+        toks = rng.integers(0, 512, (rows, keys + 1)).astype(np.int32)
+        kv, out = eng.new_kv(rows, capacity=256, kv_dtype="float32"), []
+        for on in (0, 1):
+            kv.reset()
+            eng.set_option("small_stack", 0)
+            eng.forward(toks[:, :keys], kv)
+            eng.set_option("small_stack", on)
+            out.append(eng.forward(toks[:, keys:], kv))
+        kv.close()
+        assert np.abs(out[0] - out[1]).max() <= 4e-3 * max(1.0, np.abs(out[0]).max())
+        assert np.array_equal(*out) != kernel, (rows, keys)
+    eng.close()
